@@ -173,7 +173,7 @@ int ConfigModel::open(std::unique_ptr<ConfigModel> e, const Safetensors& file, c
   if (int rc2 = e->zeroed((void**)&e->rows, kLogitRows * 4)) return rc2;
   if (int rc2 = e->zeroed(&e->head_in, kLogitRows * e->ld * e->unit())) return rc2;
   if (int rc2 = e->zeroed((void**)&e->logits, kLogitRows * e->vocab * 4)) return rc2;
-  if (int rc2 = e->zeroed((void**)&e->best, 8)) return rc2;
+  if (int rc2 = e->zeroed((void**)&e->best, 8 * dense_candidates(e->vocab))) return rc2;
   if (int rc2 = launch_fill_zero(e->d_token, 4, e->stream)) return rc2;
   AWQ_HIP_TRY(hipStreamSynchronize(e->stream));
   e->finalized = true;
@@ -221,7 +221,7 @@ int ConfigModel::enqueue_step(StepKind kind, int64_t) {
     if (int rc = run_pass(true, nullptr, 1, pos)) return rc;
   if (kind == STEP_PROMPT) return AWQ_OK;
   if (int rc = logits_of(stream_of(true), nullptr, 1, true)) return rc;
-  return launch_take_best(best, d_token, d_out, d_state, kind == STEP_GENERATE ? 1 : 0, stream);
+  return launch_take_best(best, dense_candidates(vocab), d_token, d_out, d_state, kind == STEP_GENERATE ? 1 : 0, stream);
 }
 
 int64_t ConfigModel::prompt_pass_tokens(int64_t, int64_t rest) const {

@@ -68,7 +68,8 @@ enum DenseOut {
   DENSE_STORE = 0,     // y in the activations' type, or float where the segment says so
   DENSE_RESIDUAL = 1,  // y is float: y = (y + sum) + addend (addend: same shape, may be null)
   DENSE_F32 = 2,       // y is float
-  DENSE_ARGMAX = 3,    // one token: y is float, and *best becomes the largest (value, -row) candidate
+  DENSE_ARGMAX = 3,    // one token, one segment: y is float, and best[i] becomes the largest (value, -row) candidate of rows
+                       // 16 i .. + 15 (0: none), for i < dense_candidates(rows)
 };
 // A run of tokens that one weight block of several is applied to: rows first .. first + count - 1 of the list.
 struct DenseTile {
@@ -83,7 +84,7 @@ struct DenseArgs {
   int32_t start[kDenseSegments] = {};  // the segments' first rows (launch_dense)
   DenseSegment seg[kDenseSegments];
   const float* addend = nullptr;
-  unsigned long long* best = nullptr;  // DENSE_ARGMAX: zero between launches
+  unsigned long long* best = nullptr;  // DENSE_ARGMAX
   // one token, DENSE_RESIDUAL: the first gate_k inputs of segment 0 are not read from x but formed in the launch, the RMS
   // norm of o over gate_n values times w times sigmoid(g), zeros behind them (dense_gate_fused says where it can be)
   const float* gate_o = nullptr;
@@ -107,6 +108,9 @@ struct DenseArgs {
   int32_t max_tiles = 0, tile_tokens = 64, list_div = 1;
 };
 inline int64_t dense_glu_rows(int64_t n) { return round_up(n, 8) * 2; }
+// A slot per 16 rows and no common maximum: 32,768 rows of 1,024 inputs with a maximum per row in one word took 381 us in
+// binary32 (now 29), with a look at the word ahead of each workgroup's 24 us in bfloat16 (now 12).
+inline int64_t dense_candidates(int64_t rows) { return round_up(rows, kDenseRowAlign) / 16; }
 int64_t dense_weight_bytes(int64_t rows_padded, int64_t k_padded, bool f32);
 // src [rows][cols] bfloat16 or float, row major on the device, into rows row0.., inputs col0.. of a block (col0 a
 // multiple of 8); the rest of the block is left as it is (zero it first)
@@ -149,8 +153,8 @@ int launch_norm_conv(const NormConvArgs& a, bool f32, hipStream_t st);
 int launch_gated_norm(const float* o, int64_t ldo, const void* g, int64_t ldg, const float* w, void* y, int64_t ldy,
                       int64_t n, int64_t M, float eps, bool f32, hipStream_t st);
 int launch_add_rows(float* x, const float* y, int64_t n, hipStream_t st);  // x += y
-// the best candidate becomes the token; `state` moves on to the next position (epoch + epoch_step)
-int launch_take_best(unsigned long long* best, int32_t* out_token, int32_t* out_array, StepState* state,
+// the best of n candidates becomes the token; `state` moves on to the next position (epoch + epoch_step)
+int launch_take_best(const unsigned long long* best, int64_t n, int32_t* out_token, int32_t* out_array, StepState* state,
                      int32_t epoch_step, hipStream_t st);
 
 // --- attention over a sliding window (window_attention.hip) --------------------------------------------------

@@ -312,12 +312,25 @@ __global__ __launch_bounds__(256) void gated_norm_kernel(const float* __restrict
   for (int i = tid; i < n; i += 256) y[i] = (T)(o[i] * inv * w[i] * (1.0f / (1.0f + expf(-(float)g[i]))));
 }
 
-__global__ void take_best_kernel(unsigned long long* best, int32_t* out_token, int32_t* out_array, StepState* state,
-                                 int32_t epoch_step) {
-  if (threadIdx.x != 0) return;
-  const int32_t tok = (int32_t)(0xffffffffu - (uint32_t)(*best & 0xffffffffull));
-  *out_token = tok;
+__global__ __launch_bounds__(1024) void take_best_kernel(const unsigned long long* best, int n, int32_t* out_token,
+                                                         int32_t* out_array, StepState* state, int32_t epoch_step) {
+  __shared__ unsigned long long part[16];
+  const int tid = threadIdx.x;
   StepState s = *state;
+  unsigned long long b = 0ull;
+  for (int i = tid; i < n; i += 1024) b = best[i] > b ? best[i] : b;
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) {
+    const unsigned long long o = __shfl_xor(b, off, 64);
+    b = o > b ? o : b;
+  }
+  if ((tid & 63) == 0) part[tid >> 6] = b;
+  __syncthreads();
+  if (tid != 0) return;
+#pragma unroll
+  for (int v = 1; v < 16; ++v) b = part[v] > b ? part[v] : b;
+  const int32_t tok = (int32_t)(0xffffffffu - (uint32_t)(b & 0xffffffffull));
+  *out_token = tok;
   if (out_array) out_array[s.out_index] = tok;
   s.pos += 1;
   s.len_lo = s.pos;
@@ -326,7 +339,6 @@ __global__ void take_best_kernel(unsigned long long* best, int32_t* out_token, i
   s.out_index += 1;
   s.epoch += epoch_step;
   *state = s;
-  *best = 0ull;
 }
 
 unsigned grid_for(int64_t n) { return (unsigned)std::max<int64_t>(1, std::min<int64_t>((n + 255) / 256, 65536)); }
@@ -415,10 +427,10 @@ int launch_add_rows(float* x, const float* y, int64_t n, hipStream_t st) {
   return AWQ_OK;
 }
 
-int launch_take_best(unsigned long long* best, int32_t* out_token, int32_t* out_array, StepState* state,
+int launch_take_best(const unsigned long long* best, int64_t n, int32_t* out_token, int32_t* out_array, StepState* state,
                      int32_t epoch_step, hipStream_t st) {
-  AWQ_REQUIRE(best && out_token && state, "bad arguments");
-  hipLaunchKernelGGL(take_best_kernel, dim3(1), dim3(64), 0, st, best, out_token, out_array, state, epoch_step);
+  AWQ_REQUIRE(best && n >= 1 && n < (1 << 30) && out_token && state, "bad arguments");
+  hipLaunchKernelGGL(take_best_kernel, dim3(1), dim3(1024), 0, st, best, (int)n, out_token, out_array, state, epoch_step);
   AWQ_HIP_TRY(hipGetLastError());
   return AWQ_OK;
 }
