@@ -163,11 +163,10 @@ int ConfigModel::open(std::unique_ptr<ConfigModel> e, const Safetensors& file, c
   if (rc) return rc;
   awq_note_load_seconds(std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count());
 
-  if (!e->f32) {  // for products that are cut along k
-    constexpr int64_t kDenseWorkspace = 32ll << 20;
-    e->dense_ws_floats = std::min<int64_t>(kDenseWorkspace, 4 * e->pass_tokens * round_up(e->width, kDenseRowAlign));
-    if (int rc2 = e->dev_alloc((void**)&e->dense_ws, e->dense_ws_floats * 4)) return rc2;
-  }
+  // for products that are cut along k
+  constexpr int64_t kDenseWorkspace = 32ll << 20;
+  e->dense_ws_floats = std::min<int64_t>(kDenseWorkspace, 4 * e->pass_tokens * round_up(e->width, kDenseRowAlign));
+  if (int rc2 = e->dev_alloc((void**)&e->dense_ws, e->dense_ws_floats * 4)) return rc2;
   if (int rc2 = e->make_buffers()) return rc2;
   if (int rc2 = e->zeroed((void**)&e->tokens, e->pass_tokens * 4)) return rc2;
   if (int rc2 = e->zeroed((void**)&e->rows, kLogitRows * 4)) return rc2;

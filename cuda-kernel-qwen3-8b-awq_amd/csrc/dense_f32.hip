@@ -95,72 +95,110 @@ __global__ __launch_bounds__(256) void dense_one_f32_kernel(DenseArgs a) {
 }
 
 // --- many tokens ---------------------------------------------------------------------------------------------
-// 64 rows x 64 tokens per workgroup, 4 x 4 per thread, through LDS.  A thread's rows are two of an eight and the same two of
-// the eight behind it: a gate and its up row meet.
-template <int OUT, bool LISTED = false>
-__global__ __launch_bounds__(256) void dense_many_f32_kernel(DenseArgs a) {
-  __shared__ float ws[16][68], xs[16][68];
-  const int tid = threadIdx.x;
-  const int row0 = blockIdx.x * 64;
-  const int64_t tok0 = LISTED ? 0 : (int64_t)blockIdx.y * 64;
-  const DenseSegment& s = segment_of(a, row0);
-  if (row0 >= a.seg[a.n_seg - 1].row0 + a.seg[a.n_seg - 1].rows) return;
-  int64_t group = blockIdx.z, n_tok = a.M;
+// On v_mfma_f32_32x32x2_f32: a workgroup of four wavefronts takes 64 rows and 32 TW C tokens, steps of 32 inputs.  Two
+// wavefronts share the rows, TW the tokens (C accumulators each) and KW the inputs of a step, whose sums meet in LDS.
+// Weights and tokens go through LDS, 128 bytes per row and step, the eight 16-byte pieces of row r at positions c ^ (r & 7),
+// requested a step ahead into registers.  Lane (n, kh) reads piece 2 j + kh of row n of both operands, and instruction e
+// multiplies element e of the two: the inputs of a step are met in another order on both sides alike.
+// Up to about 50 tokens bound by the weights' bytes (2 operations per token and 4 bytes against 134 TFLOP/s and 5.1 TB/s),
+// beyond by the matrix cores.  Where the tiles do not fill the device, k is cut over `cuts` workgroups and a second launch
+// adds their sums, as in bfloat16.  333 tokens: 1,024 rows of 4,096 inputs 46 + 7 us (the sums' launch), 7,168 of 1,024 64 + 15,
+// 32,768 of 1,024 at 128 tokens 82 (104 TFLOP/s); 4 x 4 sums per thread without matrix cores took 273, 155 and 191.
+template <int TW, int KW, int C, int OUT, bool LISTED = false>
+__global__ __launch_bounds__(256) void dense_many_f32_kernel(DenseArgs a, int row_tiles, int tok_tiles, int cuts) {
+  static_assert(TW * KW == 2, "four wavefronts, two of them share the rows");
+  constexpr int TOK = 32 * TW * C, NL = (64 + TOK) / 32;  // pieces per thread and step
+  __shared__ __attribute__((aligned(16))) float tiles[2][(64 + TOK) * 32];
+  const int total = row_tiles * tok_tiles * cuts;
+  // workgroups whose indices agree modulo 8 share a die: each die walks its own run of row tiles
+  const int per = (total + 7) >> 3;
+  const int work = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+  if (work >= total) return;
+  const int rc = work / tok_tiles, tile = work - rc * tok_tiles, tt0 = LISTED ? 0 : tile * TOK;
+  const int rt = rc / cuts, cut = rc - rt * cuts;
+  int64_t group = blockIdx.y;
+  int n_tok = (int)min((int64_t)1 << 30, a.M);
   const int32_t* list = nullptr;
   if constexpr (LISTED) {
-    const DenseTile run = a.tiles[blockIdx.y];
+    const DenseTile run = a.tiles[tile];
     if (run.count == 0) return;
     group = run.group;
     n_tok = run.count;
     list = a.list + run.first;
   }
-  const int lr = tid >> 2, lk = (tid & 3) * 4;
-  const float* w = reinterpret_cast<const float*>(a.w) + group * a.w_batch + (int64_t)(row0 + lr) * a.k + lk;
-  int64_t tok = min(tok0 + lr, n_tok - 1);
-  if constexpr (LISTED) tok = list[tok] / a.list_div;
-  const float* x = reinterpret_cast<const float*>(s.x) + blockIdx.z * a.x_batch + tok * s.ldx + lk;
-  const int tc = (tid >> 4) * 4;
-  int tr[4];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 31, kh = lane >> 5;
+  const int rw = wave & 1, tw = TW == 2 ? wave >> 1 : 0, kw = KW == 2 ? wave >> 1 : 0;
+  const DenseSegment& s = segment_of(a, rt * 64);
+  if (rt * 64 >= a.seg[a.n_seg - 1].row0 + a.seg[a.n_seg - 1].rows) return;  // padding
+  const int all_steps = (int)(a.k >> 5);
+  const int first_step = (int)((int64_t)all_steps * cut / cuts);
+  const int steps = (int)((int64_t)all_steps * (cut + 1) / cuts) - first_step;
+
+  // this thread's pieces of a step: place tid % 8 of rows tid / 8 + 32 i, the first two of them weights
+  const float* src[NL];
+  const int lr = tid >> 3, at = (tid & 7) << 2;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) tr[i] = 16 * ((tid & 15) >> 2) + 2 * (tid & 3) + (i & 1) + 8 * (i >> 1);
-  float acc[4][4] = {};
-  for (int k0 = 0; k0 < (int)a.k; k0 += 16) {
-    const f32x4_t wv = *reinterpret_cast<const f32x4_t*>(w + k0);
-    f32x4_t xv;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) xv[j] = x[k0 + j];
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < 4; ++j) ws[lk + j][lr] = wv[j], xs[lk + j][lr] = xv[j];
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < 16; ++k)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_fmaf(ws[k][tr[i]], xs[k][tc + j], acc[i][j]);
-  }
-  const int64_t y0 = blockIdx.z * a.y_batch;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    if (tok0 + tc + j >= n_tok) continue;
-    int64_t t = tok0 + tc + j;
-    if constexpr (LISTED) t = list[t];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const DenseSegment& out = segment_of(a, row0 + tr[i]);
-      const int row = row0 + tr[i] - out.row0;
-      if (row >= out.rows) continue;
-      if constexpr (OUT == DENSE_STORE) {
-        if (out.act == DENSE_GLU) {
-          const int r = (row >> 4) * 8 + (row & 7);
-          if (i < 2 && r < out.glu_rows) store_one<float>(out, y0, t, r, glu<true>(acc[i][j], acc[i | 2][j]));
-          continue;
-        }
-      }
-      finish_one<float, OUT>(a, out, t, row, acc[i][j], y0);
+  for (int i = 0; i < NL; ++i) {
+    if (i < 2) {
+      src[i] = reinterpret_cast<const float*>(a.w) + group * a.w_batch + (int64_t)(rt * 64 + lr + 32 * i) * a.k;
+    } else {
+      int64_t tok = min(tt0 + lr + 32 * (i - 2), n_tok - 1);
+      if constexpr (LISTED) tok = list[tok] / a.list_div;
+      src[i] = reinterpret_cast<const float*>(s.x) + blockIdx.y * a.x_batch + tok * s.ldx;
     }
+    src[i] += first_step * 32 + at;
   }
+  const int place = lr * 32 + (((tid & 7) ^ (lr & 7)) << 2);
+  f32x4_t next[NL];
+  auto request = [&](int step) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NL; ++i) next[i] = *reinterpret_cast<const f32x4u_t*>(src[i] + step * 32);
+  };
+  auto keep = [&](float* to) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < NL; ++i) *reinterpret_cast<f32x4_t*>(to + i * 1024 + place) = next[i];
+  };
+  f32x16_t acc[C];
+#pragma unroll
+  for (int t = 0; t < C; ++t)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[t][i] = 0.0f;
+  request(0);
+  keep(tiles[0]);
+  __syncthreads();
+  for (int st = 0; st < steps; ++st) {
+    if (st + 1 < steps) request(st + 1);
+    const float* const now = tiles[st & 1];
+#pragma unroll
+    for (int jj = 0; jj < 4 / KW; ++jj) {
+      const int piece = ((2 * (jj + kw * 2) + kh) ^ (n & 7)) << 2;
+      const f32x4_t wv = *reinterpret_cast<const f32x4_t*>(now + (rw * 32 + n) * 32 + piece);
+      f32x4_t xv[C];
+#pragma unroll
+      for (int t = 0; t < C; ++t) xv[t] = *reinterpret_cast<const f32x4_t*>(now + (64 + (tw * C + t) * 32 + n) * 32 + piece);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int t = 0; t < C; ++t) acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(wv[e], xv[t][e], acc[t], 0, 0, 0);
+    }
+    if (st + 1 < steps) keep(tiles[(st + 1) & 1]);  // its readers passed the barrier behind the step before
+    __syncthreads();
+  }
+  if constexpr (KW == 2) {
+    float* const other = tiles[0] + rw * 1024;
+    if (kw == 1) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) other[i * 64 + lane] = acc[0][i];
+    }
+    __syncthreads();
+    if (kw == 1) return;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[0][i] += other[i * 64 + lane];
+    wave_sync();
+  }
+  store_block_rows<float, OUT, LISTED>(a, tiles[0] + wave * 1024, acc, rt * 64 + rw * 32, tt0 + tw * C * 32, n_tok, list, row_tiles * 64,
+                                       cut);
 }
 
 template <int OUT>
@@ -178,10 +216,42 @@ int launch_one(const DenseArgs& a, int64_t rows, hipStream_t st) {
   return AWQ_OK;
 }
 
+// tokens of a workgroup's tile: 128 unless the last tile would be mostly padding
+int tile_of(int64_t M) {
+  if (M <= 32) return 32;
+  return M > 64 && round_up(M, 128) * 5 <= round_up(M, 64) * 6 ? 128 : 64;
+}
+
+template <int OUT, bool LISTED>
+int launch_tiles(const DenseArgs& a, int64_t rows, int tile, int tok_tiles, int cuts, hipStream_t st) {
+  const int row_tiles = (int)(rows / 64);
+  const dim3 grid((unsigned)(((int64_t)row_tiles * tok_tiles * cuts + 7) / 8 * 8), (unsigned)a.batch);
+  if (tile == 32)
+    hipLaunchKernelGGL((dense_many_f32_kernel<1, 2, 1, OUT, LISTED>), grid, dim3(256), 0, st, a, row_tiles, tok_tiles, cuts);
+  else if (tile == 64)
+    hipLaunchKernelGGL((dense_many_f32_kernel<2, 1, 1, OUT, LISTED>), grid, dim3(256), 0, st, a, row_tiles, tok_tiles, cuts);
+  else
+    hipLaunchKernelGGL((dense_many_f32_kernel<2, 1, 2, OUT, LISTED>), grid, dim3(256), 0, st, a, row_tiles, tok_tiles, cuts);
+  AWQ_HIP_TRY(hipGetLastError());
+  return AWQ_OK;
+}
+
 template <int OUT>
 int launch_many(const DenseArgs& a, int64_t rows, hipStream_t st) {
-  hipLaunchKernelGGL(dense_many_f32_kernel<OUT>, dim3((unsigned)(rows / 64), (unsigned)((a.M + 63) / 64), (unsigned)a.batch),
-                     dim3(256), 0, st, a);
+  const int tile = tile_of(a.M);
+  const int64_t tok_tiles = (a.M + tile - 1) / tile, tiles = rows / 64 * tok_tiles;
+  AWQ_REQUIRE(tiles < (1ll << 28), "too large");
+  // two workgroups per compute unit, at least four steps each (48 tokens, 1,024 x 3,072: sixteen tiles alone took 209 us, cut in
+  // eight 7 + 5)
+  int64_t cuts = 1;
+  if (a.workspace && a.batch == 1 && a.M <= 65535 && tiles < 384) {
+    cuts = std::min<int64_t>((512 + tiles / 2) / tiles, (a.k >> 5) / 4);
+    cuts = std::max<int64_t>(1, std::min<int64_t>(cuts, a.workspace_floats / (a.M * rows)));
+  }
+  if (cuts == 1) return launch_tiles<OUT, false>(a, rows, tile, (int)tok_tiles, 1, st);
+  if (int rc = launch_tiles<DENSE_PART, false>(a, rows, tile, (int)tok_tiles, (int)cuts, st)) return rc;
+  hipLaunchKernelGGL((dense_parts_kernel<float, OUT>), dim3((unsigned)((rows / 4 + 255) / 256), (unsigned)a.M), dim3(256), 0, st, a,
+                     (int)rows, (int)cuts);
   AWQ_HIP_TRY(hipGetLastError());
   return AWQ_OK;
 }
@@ -198,12 +268,7 @@ int launch_dense_one_f32(const DenseArgs& a, int64_t rows, hipStream_t st) {
 }
 
 int launch_dense_many_f32(const DenseArgs& a, int64_t rows, hipStream_t st) {
-  if (a.tiles) {
-    hipLaunchKernelGGL((dense_many_f32_kernel<DENSE_STORE, true>), dim3((unsigned)(rows / 64), (unsigned)a.max_tiles), dim3(256), 0,
-                       st, a);
-    AWQ_HIP_TRY(hipGetLastError());
-    return AWQ_OK;
-  }
+  if (a.tiles) return launch_tiles<DENSE_STORE, true>(a, rows, a.tile_tokens <= 32 ? 32 : 64, a.max_tiles, 1, st);
   switch (a.out) {
     case DENSE_STORE: return launch_many<DENSE_STORE>(a, rows, st);
     case DENSE_RESIDUAL: return launch_many<DENSE_RESIDUAL>(a, rows, st);

@@ -96,6 +96,37 @@ def test_dense_two_segments(awq, lib, dev, f32, tokens, shape):
     assert km.rms_error(dev.host(y), va[:, :k] @ wa.T) < 2e-5
 
 
+@pytest.mark.parametrize("tokens", [1, 2, 31, 32, 33, 64, 65, 96, 127, 129, 193])
+@pytest.mark.parametrize("rows,k", [(1, 64), (70, 320), (257, 1088), (8200, 256)])
+def test_binary32_products_at_the_edges_of_tiles(awq, lib, dev, tokens, rows, k):
+    """every tile of tokens, shares of k down to one, inputs and outputs that are not aligned to 16 bytes.  A sum of k products
+    in binary32 is off by about sqrt(k) roundings of 2^-24 of its size"""
+    print("binary32", tokens, rows, k, flush=True)
+    rng = np.random.default_rng(rows + tokens)
+    padded = (rows + 255) // 256 * 256
+    block = dev.torch.zeros(padded * k, dtype=dev.torch.float32, device="cuda")
+    w = (rng.standard_normal((rows, k)) / k ** 0.5).astype(np.float32)
+    d = dev.f(w)
+    awq.check(lib.awq_dense_pack(d.data_ptr(), 1, rows, k, block.data_ptr(), k, 0, 0, 1, dev.stream))
+    x = rng.standard_normal((tokens, k)).astype(np.float32)
+    want = x.astype(np.float64) @ w.T.astype(np.float64)
+    ws = dev.empty((1 << 22,), True)
+    for off in (0, 1):
+        xd, y = dev.empty((tokens * k + 1,), True), dev.empty((tokens * rows + 5,), True)
+        xd[off:off + tokens * k] = dev.f(x).reshape(-1)
+        for floats in (ws.numel(), 0):
+            y.fill_(float("nan"))
+            a = awq.AwqDenseArgs()
+            a.w, a.k, a.tokens, a.n_segments, a.out = block.data_ptr(), k, tokens, 1, awq.DENSE_F32
+            a.segment[0] = awq.AwqDenseSegment(xd.data_ptr() + 4 * off, y.data_ptr() + 4 * off, k, rows, 0, rows, 0, 0, 0, 0)
+            a.workspace, a.workspace_floats = (ws.data_ptr() if floats else None), floats
+            awq.check(lib.awq_dense(ctypes.byref(a), 1, dev.stream))
+            got = dev.host(y)
+            assert np.isnan(got[:off]).all() and np.isnan(got[off + tokens * rows:]).all()
+            got = got[off:off + tokens * rows].reshape(tokens, rows)
+            assert np.abs(got - want).max() < 8 * k ** 0.5 * 2.0 ** -24
+
+
 def test_xielu_near_zero_and_far_out(awq, lib, dev):
     """the negative branch cancels near zero: small arguments keep their relative accuracy"""
     z = np.concatenate([-np.geomspace(1e-6, 60, 200), np.geomspace(1e-6, 60, 56)]).astype(np.float32)
