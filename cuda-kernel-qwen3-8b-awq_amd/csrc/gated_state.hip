@@ -112,6 +112,8 @@ __global__ __launch_bounds__(HEAD ? 1024 : 256) void gated_step_kernel(GatedStat
 // Operands, lane (n, j) = (lane % 16, lane / 16), step i: an accumulator holds rows 4 j + i of column n, and used as an
 // operand it is just that for an order of the summed index of 4 j + i.
 //     A^T[s][t] = K Q^T,  O^T[c][t] = R^T Q^T + V^T (A^T, s <= t),  R[d][c] += K^T V
+// HEAD: one decay per head (linear attention in binary32); the logarithm stands in the place of every channel's.  333
+// tokens, 8 heads of 128: 30 us, token by token 395 (bound by a token's trip through a wavefront, 1.2 us each).
 // Where a channel of a block decays by more than 2^-kSafe the factors could leave the range of binary32: such a block goes
 // token by token, in the same accumulators.
 constexpr int kBlock = 16;
@@ -133,8 +135,9 @@ constexpr int chunk_lds() {
 }
 
 // EVEN: dim is even, two channels make one load; keys: there are keys beside the decays
-template <typename T, int D, bool EVEN, bool keys>
+template <typename T, int D, bool EVEN, bool keys, bool HEAD>
 __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
+  static_assert(keys || !HEAD, "a head's decay leaves no keys");
   constexpr int B = chunk_blocks<D>(), C = B * kBlock, S4 = D + 4, VS = kValueStride;
   constexpr int NT = D / 64;                  // tiles of 16 state rows per wavefront
   constexpr int kHalf = kBlock / 2;
@@ -151,7 +154,8 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
   const T* const q = reinterpret_cast<const T*>(a.q) + (int64_t)head * a.dim;
   const T* const k = keys ? reinterpret_cast<const T*>(a.k) + (int64_t)head * a.dim : q;
   const T* const v = reinterpret_cast<const T*>(a.v) + (int64_t)head * a.vdim + c0;
-  const float* const g = a.g + (int64_t)head * a.dim;
+  const float* const g = HEAD ? a.head_decay : a.g + (int64_t)head * a.dim;
+  const float of_head = HEAD ? a.head_decay[head] : 0.0f;
   if (tid < 3 * B) unsafe[tid / B][tid % B] = 0;
   __syncthreads();
 
@@ -174,7 +178,8 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
 #pragma unroll
       for (int t = 0; t < kHalf; ++t) {
         const int64_t tok = min(at + t0 + t, M - 1);
-        gr[t] = two(g + tok * a.ldg + dc);
+        if constexpr (HEAD) gr[t] = f32x2_t{of_head, of_head};
+        else gr[t] = two(g + tok * a.ldg + dc);
         qr[t] = two(q + tok * a.ldp + dc);
         if constexpr (keys) kr[t] = two(k + tok * a.ldp + dc);
       }
@@ -321,7 +326,7 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
               const int r = row0 + 16 * i + j4 + e;
               if (r >= a.dim) continue;
               float decay, key;
-              decay_and_key(g[tok * a.ldg + r], keys, keys ? (float)k[tok * a.ldp + r] : 0.0f, decay, key);
+              decay_and_key(HEAD ? of_head : g[tok * a.ldg + r], keys, keys ? (float)k[tok * a.ldp + r] : 0.0f, decay, key);
               s[i][e] = __builtin_fmaf(key, value, decay * s[i][e]);
               out = __builtin_fmaf(s[i][e], (float)q[tok * a.ldp + r] * a.q_scale, out);
             }
@@ -346,15 +351,15 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
     }
 }
 
-template <typename T, int D, bool EVEN, bool KEYS>
+template <typename T, int D, bool EVEN, bool KEYS, bool HEAD = false>
 int launch_chunk_form(const GatedStateArgs& a, hipStream_t st) {
   static bool raised = false;  // more LDS than the default limit of a launch
   if (!raised) {
-    AWQ_HIP_TRY(hipFuncSetAttribute((const void*)gated_chunk_kernel<T, D, EVEN, KEYS>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    AWQ_HIP_TRY(hipFuncSetAttribute((const void*)gated_chunk_kernel<T, D, EVEN, KEYS, HEAD>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     chunk_lds<D>()));
     raised = true;
   }
-  hipLaunchKernelGGL((gated_chunk_kernel<T, D, EVEN, KEYS>), dim3((unsigned)a.heads, (unsigned)((a.vdim + 15) / 16)), dim3(512),
+  hipLaunchKernelGGL((gated_chunk_kernel<T, D, EVEN, KEYS, HEAD>), dim3((unsigned)a.heads, (unsigned)((a.vdim + 15) / 16)), dim3(512),
                      chunk_lds<D>(), st, a);
   AWQ_HIP_TRY(hipGetLastError());
   return AWQ_OK;
@@ -363,6 +368,8 @@ template <typename T, int D>
 int launch_chunks(const GatedStateArgs& a, hipStream_t st) {
   const uintptr_t parts = (uintptr_t)a.q | (uintptr_t)a.k;  // two values of T, two floats
   const bool even = a.dim % 2 == 0 && a.ldp % 2 == 0 && a.ldg % 2 == 0 && parts % (2 * sizeof(T)) == 0 && (uintptr_t)a.g % 8 == 0;
+  if constexpr (sizeof(T) == 4)
+    if (a.head_decay) return even ? launch_chunk_form<T, D, true, true, true>(a, st) : launch_chunk_form<T, D, false, true, true>(a, st);
   if (a.k) return even ? launch_chunk_form<T, D, true, true>(a, st) : launch_chunk_form<T, D, false, true>(a, st);
   return even ? launch_chunk_form<T, D, true, false>(a, st) : launch_chunk_form<T, D, false, false>(a, st);
 }
@@ -402,6 +409,26 @@ int launch(const GatedStateArgs& a, hipStream_t st) {
 }
 
 }  // namespace
+
+int launch_linear_chunks_f32(const LinearAttnArgs& u, hipStream_t st) {
+  const float* p = reinterpret_cast<const float*>(u.proj);
+  const int64_t keys = (int64_t)u.heads * u.dim;
+  GatedStateArgs a;
+  a.q = p;
+  a.k = p + keys;
+  a.v = p + 2 * keys;
+  a.ldp = u.ldp;
+  a.head_decay = u.log2_decay;
+  a.heads = u.heads;
+  a.dim = u.dim;
+  a.vdim = u.vdim;
+  a.state = u.state;
+  a.o = u.o;
+  a.M = u.M;
+  a.pos = u.pos;
+  if (a.dim <= 64) return launch_chunks<float, 64>(a, st);
+  return a.dim <= 128 ? launch_chunks<float, 128>(a, st) : launch_chunks<float, 256>(a, st);
+}
 
 int launch_gated_state(const GatedStateArgs& a, bool f32, hipStream_t st) {
   AWQ_REQUIRE(a.q && a.v && a.g && a.state && (a.o || a.ctx) && a.M >= 1 && a.M < (1 << 30), "bad arguments");

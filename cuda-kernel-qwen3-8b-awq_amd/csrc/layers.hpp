@@ -212,6 +212,8 @@ struct LinearAttnArgs {
 };
 int64_t linear_state_floats(int32_t heads, int32_t dim, int32_t vdim);
 int launch_linear_attention(const LinearAttnArgs& a, bool f32, hipStream_t st);
+// its binary32 form for many tokens (gated_state.hip): dim <= 256, log2_decay set
+int launch_linear_chunks_f32(const LinearAttnArgs& a, hipStream_t st);
 
 // --- linear attention whose state decays per channel (gated_state.hip) -----------------------------------------
 // Per head S <- diag(decay_t) S + k_t v_t^T, o_t = S^T (q_scale q_t); the decay of a token is one number per row of S.
@@ -223,6 +225,7 @@ struct GatedStateArgs {
   // which then are the keys as well
   const float* g = nullptr;
   int64_t ldg = 0;
+  const float* head_decay = nullptr;  // [heads] binary logarithms, instead of g (launch_linear_chunks_f32)
   int32_t heads = 0, dim = 0, vdim = 0;
   float q_scale = 1.0f;
   float* state = nullptr;

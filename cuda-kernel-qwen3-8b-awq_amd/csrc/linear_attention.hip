@@ -4,7 +4,7 @@
 namespace {
 
 // The recurrence token by token: a wavefront holds kCols columns of the state, lane l the rows l, l + 64, ...
-// of each.  Used for single tokens and for the binary32 form; the state never leaves the registers inside a pass.
+// of each.  Used for few tokens and for decays of zero; the state never leaves the registers inside a pass.
 constexpr int kCols = 4;
 
 template <typename T, int DPL>
@@ -390,8 +390,9 @@ int launch_linear_attention(const LinearAttnArgs& a, bool f32, hipStream_t st) {
   AWQ_REQUIRE(a.heads >= 1 && a.dim >= 1 && a.vdim >= 1 && a.vdim <= 65536 && a.ldp % 8 == 0 &&
                   a.ldp >= (int64_t)a.heads * (2 * a.dim + a.vdim),
               "bad shape");
-  if (f32) return launch_step<float>(a, st);
-  if (a.log2_decay && a.M >= kChunkFrom && a.M < (1 << 30) && a.dim <= 256) {
+  const bool chunks = a.log2_decay && a.M >= kChunkFrom && a.M < (1 << 30) && a.dim <= 256;
+  if (f32) return chunks ? launch_linear_chunks_f32(a, st) : launch_step<float>(a, st);
+  if (chunks) {
     const bool whole = ((a.dim | a.vdim) & 7) == 0;
     if (a.dim <= 64) return whole ? launch_chunks<64, true>(a, st) : launch_chunks<64, false>(a, st);
     if (a.dim <= 128) return whole ? launch_chunks<128, true>(a, st) : launch_chunks<128, false>(a, st);

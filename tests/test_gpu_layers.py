@@ -243,6 +243,33 @@ def test_linear_attention(awq, lib, dev, f32, heads, dim, vdim):
             assert np.abs(s[h] - S[h]).max() <= 3e-5 * np.abs(S[h]).max(), (sizes, h)
 
 
+@pytest.mark.parametrize("heads,dim,vdim", [(3, 63, 5), (4, 64, 40), (2, 128, 16), (2, 130, 33), (1, 256, 72)])
+@pytest.mark.parametrize("sizes", [[16], [129, 1, 2], [130, 31], [15, 17, 300]], ids=str)
+def test_linear_attention_in_binary32_portions(awq, lib, dev, heads, dim, vdim, sizes):
+    """chunks beside single tokens on one state; decays that leave the range of a block's factors; odd widths"""
+    print("linear attention, binary32", heads, dim, vdim, sizes, flush=True)
+    rng = np.random.default_rng(dim + sizes[0])
+    T, n = 332, heads * (2 * dim + vdim)
+    ldp = (n + 7) // 8 * 8
+    proj, pv = dev.act(np.pad(rng.standard_normal((T, n)) * 0.5 + 0.2, ((0, 0), (0, ldp - n))), True)
+    q, k = (pv[:, i * heads * dim:(i + 1) * heads * dim].reshape(T, heads, dim) for i in (0, 1))
+    v = pv[:, 2 * heads * dim:n].reshape(T, heads, vdim)
+    decay = np.array([0.999, 1e-6, 0.9, 1.0][:heads], np.float32)
+    want, S = plain.linear_attention(q, k, v, decay.astype(np.float64))
+    d_decay, d_lg = dev.f(decay), dev.f(np.log2(decay.astype(np.float64)))
+    state = dev.empty((heads, vdim, (dim + 63) // 64 * 64), True)
+    o, at, i = dev.empty((T, heads * vdim), True), 0, 0
+    while at < T:
+        m = min(sizes[i % len(sizes)], T - at)
+        awq.check(lib.awq_linear_attention(proj[at:].data_ptr(), ldp, heads, dim, vdim, d_decay.data_ptr(), d_lg.data_ptr(),
+                                           state.data_ptr(), o[at:].data_ptr(), m, at, 1, dev.stream))
+        at, i = at + m, i + 1
+    got, s = dev.host(o).reshape(T, heads, vdim), dev.host(state)[:, :, :dim].transpose(0, 2, 1)
+    for h in range(heads):  # sums of up to 332 x 256 products in binary32, as in the test above
+        assert km.rms_error(got[:, h], want[:, h]) < 3e-5
+        assert np.abs(s[h] - S[h]).max() <= 3e-5 * np.abs(S[h]).max()
+
+
 def attend(awq, lib, dev, f32, proj, heads, kv, dim, vdim, window, scale, eps, temp, sizes, T, slots, max_pos):
     """the attention of T tokens in portions; proj: the tensor with all tokens' projections (kept as it is)"""
     kr, vr = lib.awq_window_row(dim), lib.awq_window_row(vdim)
