@@ -172,6 +172,7 @@ int ConfigModel::open(std::unique_ptr<ConfigModel> e, const Safetensors& file, c
   if (int rc2 = e->zeroed((void**)&e->rows, kLogitRows * 4)) return rc2;
   if (int rc2 = e->zeroed(&e->head_in, kLogitRows * e->ld * e->unit())) return rc2;
   if (int rc2 = e->zeroed((void**)&e->logits, kLogitRows * e->vocab * 4)) return rc2;
+  if (int rc2 = e->to_host.create()) return rc2;
   if (int rc2 = e->zeroed((void**)&e->best, 8 * dense_candidates(e->vocab))) return rc2;
   if (int rc2 = launch_fill_zero(e->d_token, 4, e->stream)) return rc2;
   AWQ_HIP_TRY(hipStreamSynchronize(e->stream));
@@ -243,14 +244,27 @@ int ConfigModel::enqueue_prompt_pass(const int32_t* ids, int64_t pos0, int64_t M
 }
 
 int ConfigModel::read_rows_logits(bool batched, const int32_t* which, int32_t n, float* host_dst) {
-  for (int64_t at = 0; at < n; at += kLogitRows) {
-    const int64_t k = std::min<int64_t>(kLogitRows, n - at);
-    if (batched) AWQ_HIP_TRY(hipMemcpyAsync(rows, which + at, (size_t)k * 4, hipMemcpyHostToDevice, stream));
-    if (int rc = logits_of(stream_of(!batched), batched ? rows : nullptr, k, false)) return rc;
-    AWQ_HIP_TRY(hipMemcpyAsync(host_dst + at * vocab, logits, (size_t)(k * vocab) * 4, hipMemcpyDeviceToHost, stream));
-    AWQ_HIP_TRY(hipStreamSynchronize(stream));
-  }
-  return AWQ_OK;
+  const bool ring = (int64_t)n * vocab * 4 >= HostRing::kFrom;
+  const auto all = [&]() -> int {
+    for (int64_t at = 0; at < n; at += kLogitRows) {
+      const int64_t k = std::min<int64_t>(kLogitRows, n - at);
+      if (batched) AWQ_HIP_TRY(hipMemcpyAsync(rows, which + at, (size_t)k * 4, hipMemcpyHostToDevice, stream));
+      if (int rc = logits_of(stream_of(!batched), batched ? rows : nullptr, k, false)) return rc;
+      if (ring) {
+        if (int rc = to_host.push(host_dst + at * vocab, logits, k * vocab * 4, stream)) return rc;
+      } else {
+        AWQ_HIP_TRY(hipMemcpyAsync(host_dst + at * vocab, logits, (size_t)(k * vocab) * 4, hipMemcpyDeviceToHost, stream));
+      }
+    }
+    return AWQ_OK;
+  };
+  if (ring) to_host.begin(device);
+  int rc = all();
+  const int rc2 = ring ? to_host.end() : AWQ_OK;
+  rc = rc ? rc : rc2;
+  const hipError_t drained = hipStreamSynchronize(stream);  // `which` is the caller's
+  if (rc == AWQ_OK) AWQ_HIP_TRY(drained);
+  return rc;
 }
 
 int ConfigModel::read_logits_f32(float* host_dst) {

@@ -54,6 +54,7 @@ struct ConfigModel : awq_engine {
   int32_t* rows = nullptr;  // which rows' logits are asked for
   void* head_in = nullptr;  // [kLogitRows][ld]
   float* logits = nullptr;  // [kLogitRows][vocab]
+  HostRing to_host;
   unsigned long long* best = nullptr;
   float* dense_ws = nullptr;
   int64_t dense_ws_floats = 0;

@@ -105,6 +105,104 @@ awq_engine::~awq_engine() {
 extern "C" void awq_destroy(awq_engine* e) { delete e; }
 
 // ---------------------------------------------------------------------------
+// results to the host
+// ---------------------------------------------------------------------------
+int HostRing::create() {
+  AWQ_HIP_TRY(hipHostMalloc((void**)&pinned, (size_t)(kSlots * kPiece), hipHostMallocDefault));
+  for (hipEvent_t& e : arrived) AWQ_HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  return AWQ_OK;
+}
+
+HostRing::~HostRing() {
+  for (hipEvent_t e : arrived)
+    if (e) (void)hipEventDestroy(e);
+  if (pinned) (void)hipHostFree(pinned);
+}
+
+void HostRing::copy_out(const Piece& p) {
+  const bool ok = hipEventSynchronize(arrived[p.slot]) == hipSuccess;
+  if (ok) memcpy(p.dst, pinned + p.slot * kPiece, (size_t)p.bytes);
+  std::lock_guard<std::mutex> hold(lock);
+  busy[p.slot] = false;
+  failed = failed || !ok;
+  changed.notify_all();
+}
+
+void HostRing::work(int device) {
+  (void)hipSetDevice(device);
+  for (;;) {
+    Piece p;
+    {
+      std::unique_lock<std::mutex> hold(lock);
+      changed.wait(hold, [&] { return closing || !pieces.empty(); });
+      if (pieces.empty()) return;
+      p = pieces.front();
+      pieces.pop_front();
+    }
+    copy_out(p);
+  }
+}
+
+void HostRing::begin(int device) {
+  closing = failed = false;
+  try {
+    for (int i = 0; i < kThreads; ++i) threads.emplace_back([this, device] { work(device); });
+  } catch (const std::exception&) {
+    // fewer threads, or none: the caller's thread copies
+  }
+}
+
+int HostRing::push(void* host_dst, const void* device_src, int64_t bytes, hipStream_t st) {
+  for (int64_t at = 0, n = 0; at < bytes; at += n) {
+    // pieces end where a page of the host's memory does: two threads in one fresh page of 2 MB would both clear it
+    n = std::min(bytes - at, kPiece - (int64_t)((uintptr_t)host_dst + (uintptr_t)at) % kPiece);
+    Piece p{0, (char*)host_dst + at, n};
+    {
+      std::unique_lock<std::mutex> hold(lock);
+      changed.wait(hold, [&] {
+        for (int i = 0; i < kSlots; ++i)
+          if (!busy[i]) {
+            p.slot = i;
+            return true;
+          }
+        return false;
+      });
+      busy[p.slot] = true;
+    }
+    hipError_t err = hipMemcpyAsync(pinned + p.slot * kPiece, (const char*)device_src + at, (size_t)p.bytes, hipMemcpyDeviceToHost, st);
+    if (err == hipSuccess) err = hipEventRecord(arrived[p.slot], st);
+    if (err != hipSuccess) {
+      std::lock_guard<std::mutex> hold(lock);
+      busy[p.slot] = false;
+      AWQ_HIP_TRY(err);
+    }
+    if (threads.empty()) {
+      copy_out(p);
+      continue;
+    }
+    std::lock_guard<std::mutex> hold(lock);
+    pieces.push_back(p);
+    changed.notify_all();
+  }
+  return AWQ_OK;
+}
+
+int HostRing::end() {
+  {
+    std::lock_guard<std::mutex> hold(lock);
+    closing = true;
+    changed.notify_all();
+  }
+  for (std::thread& t : threads) t.join();
+  threads.clear();
+  if (failed) {
+    awq_set_error("copying results to the host failed");
+    return AWQ_ERR_HIP;
+  }
+  return AWQ_OK;
+}
+
+// ---------------------------------------------------------------------------
 // steps
 // ---------------------------------------------------------------------------
 namespace {

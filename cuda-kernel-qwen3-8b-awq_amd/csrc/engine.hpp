@@ -1,7 +1,11 @@
 // Host-side engine declarations: the state and the step driver every model shares (engine.cpp), what a model
 // supplies to it, and the registry by which a model folder finds its class.
 #pragma once
+#include <condition_variable>
+#include <deque>
+#include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "common.hpp"
@@ -11,6 +15,39 @@ enum StepKind {
   STEP_PROMPT = 0,    // the state's token goes through the layers
   STEP_GENERATE = 1,  // ... and the next token is sampled; the step leaves the next one's state on the device
   STEP_SAMPLE = 2,    // no position: the next token is sampled from the hidden state as it stands
+};
+
+// Large results on their way to pageable host memory: the device copies pieces into a ring of pinned ones, threads copy these
+// out (and take the page faults of fresh memory, most of the time of such a copy) while the next are on their way.  Ring and
+// events are the engine's; the threads end with the request.
+class HostRing {
+ public:
+  static constexpr int kSlots = 8, kThreads = 4;
+  static constexpr int64_t kPiece = 2 << 20;
+  static constexpr int64_t kFrom = 4 << 20;  // smaller results go as one pageable copy
+  int create();
+  ~HostRing();
+  // a request: begin, any number of pushes in stream order, end (which waits for all of it); `end` after a failure too
+  void begin(int device);
+  int push(void* host_dst, const void* device_src, int64_t bytes, hipStream_t st);
+  int end();
+
+ private:
+  struct Piece {
+    int slot;
+    char* dst;
+    int64_t bytes;
+  };
+  void work(int device);
+  void copy_out(const Piece& p);
+  char* pinned = nullptr;
+  hipEvent_t arrived[kSlots] = {};
+  bool busy[kSlots] = {};
+  std::mutex lock;
+  std::condition_variable changed;
+  std::deque<Piece> pieces;
+  bool closing = false, failed = false;
+  std::vector<std::thread> threads;
 };
 
 // One engine: the sequence, its step state on the device and the captured steps are the driver's (engine.cpp);

@@ -209,3 +209,21 @@ def test_command_line_and_trace_runner(awq, torch_gpu, tmp_path):
         assert not (out / "1.f32").exists()
         assert km.rms_error(read(2), za[[5]]) < LIMIT[dtype]
         assert km.rms_error(read(3), zb[[1]]) < LIMIT[dtype]
+
+
+def test_many_logits_come_out_as_few_do(awq, torch_gpu, tmp_path):
+    """more than 4 MB of logits pass through pinned pieces on several threads: the bits are those of requests for fewer rows,
+    whether or not a group of rows or the whole fills its last piece; into fresh memory each time"""
+    cfg = km.model(64, 2051, [km.attention(2, 1, 32, 32, 40, ff=96)])
+    km.write(str(tmp_path), cfg, km.weights(cfg, 3))
+    eng = awq.open_model(str(tmp_path), dtype="bfloat16", max_positions=1300)
+    tokens = [(7 * i + 1) % 2051 for i in range(1300)]
+
+    def logits(want):
+        eng.reset()
+        return eng.forward(tokens, want)
+    few = np.concatenate([logits(range(at, min(at + 128, 1300))) for at in range(0, 1300, 128)])  # 1 MB each
+    for n in (512, 640, 1300):
+        many = logits(range(n))
+        assert many.nbytes >= 4 << 20 and np.array_equal(many, few[:n]), n
+    eng.close()
