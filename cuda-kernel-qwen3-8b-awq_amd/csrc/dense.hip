@@ -1,6 +1,8 @@
 // Dense products of bfloat16 weights with one token or many, packing of weights, the launch of any product (layers.hpp).
 #include "dense_device.hpp"
 
+#include <type_traits>
+
 namespace {
 // --- one token, bfloat16 -----------------------------------------------------------------------------------
 // A workgroup owns 16 rows and all of k, its wavefronts a run of k each; a load of a wavefront is four pieces of 256
@@ -110,6 +112,102 @@ __global__ __launch_bounds__(NW * 64) void dense_one_kernel(DenseArgs a) {
       b = o > b ? o : b;
     }
     if (tid == 0) a.best[blockIdx.x] = b;
+  }
+}
+
+// --- few tokens, bfloat16 ----------------------------------------------------------------------------------
+// The one-token kernel with NT tiles of 16 tokens in the columns of v_mfma_f32_16x16x32_bf16: bound by the weights' bytes and by
+// the tokens, which every workgroup reads out of its die's L2 (NT tiles beside R of weights).  A workgroup owns 16 R rows
+// and all of k, so that nothing is left for a second launch to add.  9 tokens: 7,168 x 1,024 4.9 us, 4,096 x 4,096 8.0, 28,672 x
+// 4,096 42.7 (5.5 TB/s); as tiles of 64 tokens with k cut over workgroups and a second launch 12.3, 18.8 and 58.5.
+template <int NW, int NT, int R, int OUT, bool LISTED>
+__global__ __launch_bounds__(NW * 64) void dense_few_kernel(DenseArgs a) {
+  constexpr int PS = 20;  // floats per token of a wavefront's sums
+  __shared__ __attribute__((aligned(16))) float part[NW * R * NT * 16 * PS];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int row0 = blockIdx.x * 16 * R;
+  const DenseSegment& s = segment_of(a, row0);
+  const int local = row0 - s.row0;
+  if (local >= s.rows) return;  // padding
+  int64_t group = blockIdx.y;
+  int n_tok = (int)a.M;
+  const int32_t* list = nullptr;
+  if constexpr (LISTED) {
+    const DenseTile run = a.tiles[blockIdx.y];
+    if (run.count == 0) return;
+    group = run.group;
+    n_tok = run.count;
+    list = a.list + run.first;
+  }
+  const int steps = (int)(a.k >> 5);
+  const int per = (steps + NW - 1) / NW;
+  const int s0 = min(wave * per, steps), s1 = min(s0 + per, steps);
+  const int r = lane & 15, c = lane >> 4;
+  const bf16x8_t* w = reinterpret_cast<const bf16x8_t*>(reinterpret_cast<const bf16_t*>(a.w) + group * a.w_batch) +
+                      ((int64_t)(row0 >> 5) * (a.k >> 4) + (c >> 1)) * 64 + 32 * (c & 1) + (row0 & 16) + r;
+  const bf16x8_t* x[NT];  // (rows 16 .. 31 of a block of weights are 16 pieces behind rows 0 .. 15)
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    int64_t tok = min(16 * t + r, n_tok - 1);
+    if constexpr (LISTED) tok = list[tok] / a.list_div;
+    x[t] = reinterpret_cast<const bf16x8_t*>(reinterpret_cast<const bf16_t*>(s.x) + (LISTED ? 0 : blockIdx.y * a.x_batch) + tok * s.ldx) + c;
+  }
+  f32x4_t acc[R][NT];
+#pragma unroll
+  for (int b = 0; b < R; ++b)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[b][t] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  constexpr int U = R * NT == 1 ? 8 : 4;
+  int i = s0;
+  for (; i + U <= s1; i += U) {
+    bf16x8_t wv[U][R], xv[U][NT];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int b = 0; b < R; ++b) wv[u][b] = __builtin_nontemporal_load(w + (int64_t)(i + u) * 128 + 16 * b);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int t = 0; t < NT; ++t) xv[u][t] = x[t][(i + u) * 4];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int b = 0; b < R; ++b) acc[b][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[u][b], xv[u][t], acc[b][t], 0, 0, 0);
+  }
+  for (; i < s1; ++i) {
+#pragma unroll
+    for (int b = 0; b < R; ++b) {
+      const bf16x8_t wv = __builtin_nontemporal_load(w + (int64_t)i * 128 + 16 * b);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[b][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv, x[t][i * 4], acc[b][t], 0, 0, 0);
+    }
+  }
+  // acc[b][t][j]: row 16 b + 4 c + j of token 16 t + r
+#pragma unroll
+  for (int b = 0; b < R; ++b)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) *reinterpret_cast<f32x4_t*>(part + (((wave * R + b) * NT + t) * 16 + r) * PS + 4 * c) = acc[b][t];
+  __syncthreads();
+  const int64_t y0 = blockIdx.y * a.y_batch;
+  for (int at = tid; at < R * NT * 256; at += NW * 64) {
+    const int b = at / (NT * 256), token = (at >> 4) % (NT * 16), row = at & 15;
+    const int here = local + 16 * b;
+    float sum = 0.0f;
+#pragma unroll
+    for (int v = 0; v < NW; ++v) sum += part[((v * R + b) * NT * 16 + token) * PS + row];
+    int64_t tok = token;
+    if constexpr (LISTED) tok = list[min(token, n_tok - 1)];
+    if constexpr (OUT == DENSE_STORE) {
+      if (s.act == DENSE_GLU) {
+        const float up = __shfl_down(sum, 8, 16);
+        if (token < n_tok && row < 8 && here / 2 + row < s.glu_rows)
+          store_one<bf16_t>(s, LISTED ? 0 : y0, tok, here / 2 + row, glu<false>(sum, up));
+        continue;
+      }
+    }
+    if (token < n_tok && here + row < s.rows) finish_one<bf16_t, OUT>(a, s, tok, here + row, sum, LISTED ? 0 : y0);
   }
 }
 
@@ -243,6 +341,8 @@ __global__ __launch_bounds__(256) void dense_pack_kernel(const S* __restrict__ s
   }
 }
 
+constexpr int kFewTokens = 32;
+
 template <int OUT>
 int launch_one(const DenseArgs& a, int64_t rows, hipStream_t st) {
   const dim3 g((unsigned)(rows / 16), (unsigned)a.batch);
@@ -263,8 +363,36 @@ int launch_one(const DenseArgs& a, int64_t rows, hipStream_t st) {
   return AWQ_OK;
 }
 
+// up to 32 tokens, or tiles of as many
+template <int OUT, bool LISTED>
+int launch_few(const DenseArgs& a, int64_t rows, int tokens, int blocks, hipStream_t st) {
+  // 32 rows per workgroup read the tokens half as often, 16 make twice the workgroups: 8,192 x 1,024 at 9 tokens 6.9 against 5.2 us,
+  // 16,384 x 4,096 at 16 tokens 25.4 against 32.0, at 32 tokens 32.3 against 46.7
+  const bool pairs = rows * blocks >= (tokens <= 16 ? 16384 : 8192);
+  const dim3 g((unsigned)(rows / (pairs ? 32 : 16)), (unsigned)blocks);
+  const auto launch = [&](auto waves) {
+    constexpr int NW = decltype(waves)::value;
+    const dim3 t(NW * 64);
+    if (tokens <= 16) {
+      if (pairs) hipLaunchKernelGGL((dense_few_kernel<NW, 1, 2, OUT, LISTED>), g, t, 0, st, a);
+      else hipLaunchKernelGGL((dense_few_kernel<NW, 1, 1, OUT, LISTED>), g, t, 0, st, a);
+    } else {
+      if (pairs) hipLaunchKernelGGL((dense_few_kernel<NW, 2, 2, OUT, LISTED>), g, t, 0, st, a);
+      else hipLaunchKernelGGL((dense_few_kernel<NW, 2, 1, OUT, LISTED>), g, t, 0, st, a);
+    }
+  };
+  if (a.k > 8192) launch(std::integral_constant<int, 16>{});
+  else if (a.k > 1024) launch(std::integral_constant<int, 8>{});
+  else launch(std::integral_constant<int, 4>{});
+  AWQ_HIP_TRY(hipGetLastError());
+  return AWQ_OK;
+}
+
 template <int OUT>
 int launch_many(const DenseArgs& a, int64_t rows, hipStream_t st) {
+  // (25 to 32 tokens on few long rows read the tokens more than the weights: 4,096 x 12,288 37 us, below 33)
+  if (a.M <= 24 || (a.M <= kFewTokens && (rows >= 8192 || a.k <= 8192)))
+    return launch_few<OUT, false>(a, rows, (int)a.M, a.batch, st);
   const int row_tiles = (int)(rows / 256);
   // few weights (few rows or a short k) are read again for less: tiles of 64 tokens where those of 128 are few
   const bool small = (row_tiles <= 4 || a.k <= 512) && row_tiles * ((a.M + 127) / 128) <= 256;
@@ -297,6 +425,7 @@ int launch_many(const DenseArgs& a, int64_t rows, hipStream_t st) {
 
 // tokens with weight blocks of their own
 int launch_listed(const DenseArgs& a, int64_t rows, hipStream_t st) {
+  if (a.tile_tokens <= kFewTokens) return launch_few<DENSE_STORE, true>(a, rows, a.tile_tokens, a.max_tiles, st);
   const int row_tiles = (int)(rows / 256);
   const unsigned grid = (unsigned)(((int64_t)row_tiles * a.max_tiles + 7) / 8 * 8);
   if (a.tile_tokens <= 64)

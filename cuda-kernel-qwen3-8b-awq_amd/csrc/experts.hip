@@ -151,7 +151,19 @@ int32_t route_max_tiles(int64_t M, int32_t top, int32_t experts, int32_t tile_to
   return (int32_t)std::max<int64_t>(1, std::min<int64_t>(pairs, pairs / tile_tokens + std::min<int64_t>(experts, pairs)));
 }
 
-int32_t route_tile_tokens(int64_t M, int32_t top, int32_t outputs, bool f32) { return !f32 && M * top >= 128ll * outputs ? 128 : 64; }
+// (an expert's run of a few entries goes through the products of few tokens)
+int32_t route_tile_tokens(int64_t M, int32_t top, int32_t outputs, bool f32) {
+  const int64_t pairs = M * top;
+  if (pairs <= 8ll * outputs) return f32 ? 32 : 16;
+  if (pairs <= 20ll * outputs) return 32;
+  return !f32 && pairs >= 128ll * outputs ? 128 : 64;
+}
+
+int32_t route_tiles_room(int64_t M, int32_t top, int32_t experts, int32_t outputs) {
+  const auto upto = [&](int64_t per) { return std::max<int64_t>(1, std::min(M, per * outputs / top)); };
+  return std::max(route_max_tiles(M, top, experts, 64),
+                  std::max(route_max_tiles(upto(8), top, experts, 16), route_max_tiles(upto(20), top, experts, 32)));
+}
 
 int launch_route(const RouteArgs& a, hipStream_t st) {
   AWQ_REQUIRE(a.logits && a.ids && a.weights && a.M >= 1, "bad arguments");

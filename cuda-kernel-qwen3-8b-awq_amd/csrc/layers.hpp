@@ -308,8 +308,10 @@ struct RouteArgs {
   DenseTile* tiles = nullptr;     // [route_max_tiles]
   int32_t* list = nullptr;        // [M * top]
 };
-// tokens of a tile: 64, or 128 where an expert has as many on average and the products have tiles of that size
+// tokens of a tile: 64, 128 where an expert has as many on average and the products have tiles of that size, 16 or 32
+// where it has few
 int32_t route_tile_tokens(int64_t M, int32_t top, int32_t outputs, bool f32);
+int32_t route_tiles_room(int64_t M, int32_t top, int32_t experts, int32_t outputs);  // for passes of up to M tokens
 int32_t route_max_tiles(int64_t M, int32_t top, int32_t experts, int32_t tile_tokens);
 int launch_route(const RouteArgs& a, hipStream_t st);
 

@@ -488,7 +488,7 @@ int TudasunEngine::make_activations(Buffers* b, int64_t n) {
       router = std::max<int64_t>(router, s.outputs());
       pairs = std::max<int64_t>(pairs, (int64_t)s.top * width);
       top = std::max<int64_t>(top, s.top);
-      tiles = std::max<int64_t>(tiles, route_max_tiles(n, s.top, s.experts, 64));
+      tiles = std::max<int64_t>(tiles, route_tiles_room(n, s.top, s.experts, s.outputs()));
     }
   }
   // every buffer starts as zeros: what pads a product's inputs meets zero weights, and has to be finite

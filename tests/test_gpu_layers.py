@@ -127,6 +127,29 @@ def test_binary32_products_at_the_edges_of_tiles(awq, lib, dev, tokens, rows, k)
             assert np.abs(got - want).max() < 8 * k ** 0.5 * 2.0 ** -24
 
 
+@pytest.mark.parametrize("tokens", [2, 15, 16, 17, 24, 25, 31, 32])
+@pytest.mark.parametrize("rows,k", [(1, 64), (47, 320), (300, 1088), (264, 8256), (8200, 192), (16400, 64)])
+def test_products_of_few_tokens(awq, lib, dev, tokens, rows, k):
+    """one and two tiles of 16 tokens, 16 and 32 rows per workgroup, 4, 8 and 16 wavefronts, rests of k.  The operands are
+    exact: a sum of k products in binary32 is off by about sqrt(k) roundings of 2^-24 of its size"""
+    print("few tokens", tokens, rows, k, flush=True)
+    rng = np.random.default_rng(rows + tokens)
+    block = dev.torch.zeros((rows + 255) // 256 * 256 * k, dtype=dev.torch.bfloat16, device="cuda")
+    w, wv = dev.act(rng.standard_normal((rows, k)) / k ** 0.5, False)
+    awq.check(lib.awq_dense_pack(w.data_ptr(), 0, rows, k, block.data_ptr(), k, 0, 0, 0, dev.stream))
+    x, xv = dev.act(rng.standard_normal((tokens, k)), False)
+    ws = dev.empty((1 << 20,), True)
+    y = dev.empty((tokens + 1, rows), True)
+    a = awq.AwqDenseArgs()
+    a.w, a.k, a.tokens, a.n_segments, a.out = block.data_ptr(), k, tokens, 1, awq.DENSE_F32
+    a.segment[0] = awq.AwqDenseSegment(x.data_ptr(), y.data_ptr(), k, rows, 0, rows, 0, 0, 0, 0)
+    a.workspace, a.workspace_floats = ws.data_ptr(), ws.numel()
+    awq.check(lib.awq_dense(ctypes.byref(a), 0, dev.stream))
+    got = dev.host(y)
+    assert np.isnan(got[tokens]).all()
+    assert np.abs(got[:tokens] - xv @ wv.T).max() < 8 * k ** 0.5 * 2.0 ** -24
+
+
 def test_xielu_near_zero_and_far_out(awq, lib, dev):
     """the negative branch cancels near zero: small arguments keep their relative accuracy"""
     z = np.concatenate([-np.geomspace(1e-6, 60, 200), np.geomspace(1e-6, 60, 56)]).astype(np.float32)
