@@ -1,6 +1,8 @@
 // Dense products of bfloat16 weights with one token or many, packing of weights, the launch of any product (layers.hpp).
 #include "dense_device.hpp"
 
+#include <math.h>
+
 #include <type_traits>
 
 namespace {
@@ -215,14 +217,18 @@ __global__ __launch_bounds__(NW * 64) void dense_few_kernel(DenseArgs a) {
 // A workgroup of four wavefronts takes 256 rows and 32 TT tokens: 64 rows per wavefront as 2 x TT accumulators of
 // v_mfma_f32_32x32x16_bf16.  The weights go from memory into registers in operand order, every byte once per
 // workgroup; the tokens go through LDS (global_load_lds_dwordx4, 128 bytes per token and step of 64 inputs, the
-// eight 16-byte pieces of row r at positions c ^ (r & 7)).  Both are requested a step ahead.  Where the tiles do not
+// eight 16-byte pieces of row r at positions c ^ (r & 7)).  Both are requested two steps ahead.  Where the tiles do not
 // fill the device, k is cut over `cuts` workgroups whose sums go to the workspace, [cut][token][row]; a second launch
-// adds them in order.
+// adds them in order.  At 2,048 tokens bound by the matrix cores: 28,672 x 4,096 434 us, 1.11 PFLOP/s (requested a step ahead, with
+// a wait for everything on its way at each barrier, 474); at few by the trips to memory (33 tokens, 4,096 x 4,096: 17.8,
+// was 19.9).
 // LISTED: the tokens come from runs of a list, each with a weight block of its own.
 template <int TT, int OUT, bool LISTED = false>
 __global__ __launch_bounds__(256, 2) void dense_many_kernel(DenseArgs a, int row_tiles, int tok_tiles, int cuts) {
-  __shared__ __attribute__((aligned(16))) bf16_t tile0[2 * 32 * TT * 64];
-  bf16_t* const tile1 = tile0 + 32 * TT * 64;
+  // three arrays, so that the compiler can tell which reads a request on its way may touch
+  __shared__ __attribute__((aligned(16))) bf16_t tile0[32 * TT * 64];
+  __shared__ __attribute__((aligned(16))) bf16_t tile1[32 * TT * 64];
+  __shared__ __attribute__((aligned(16))) bf16_t tile2[32 * TT * 64];
   const int total = row_tiles * tok_tiles * cuts;
   // workgroups whose indices agree modulo 8 share a die: each die walks its own run of row tiles
   const int per = (total + 7) >> 3;
@@ -258,18 +264,21 @@ __global__ __launch_bounds__(256, 2) void dense_many_kernel(DenseArgs a, int row
     src[i] = reinterpret_cast<const bf16_t*>(s.x) + blockIdx.y * a.x_batch + tok * s.ldx + first_step * 64 +
              (((lane & 7) ^ (row & 7)) << 3);
   }
+  const bf16_t* const x_first = reinterpret_cast<const bf16_t*>(s.x);
   auto request = [&](bf16_t* tile, int step) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < TT; ++i)
-      __builtin_amdgcn_global_load_lds((gptr_t)(src[i] + step * 64), (lptr_t)(tile + (wave * TT + i) * 8 * 64), 16, 0, 0);
+    for (int i = 0; i < TT; ++i) {
+      const bf16_t* from = step < steps ? src[i] + step * 64 : x_first;
+      __builtin_amdgcn_global_load_lds((gptr_t)from, (lptr_t)(tile + (wave * TT + i) * 8 * 64), 16, 0, 0);
+    }
   };
   const bf16x8_t* wp = reinterpret_cast<const bf16x8_t*>(reinterpret_cast<const bf16_t*>(a.w) + group * a.w_batch) +
-                       ((int64_t)(rt * 8 + wave * 2) * k16 + first_step * 4) * 64 + lane;
-  auto weights = [&](bf16x8_t (&wv)[2][4], int step) __attribute__((always_inline)) {
+                       ((int64_t)(rt * 8 + wave * 2) * k16 + first_step * 4) * 64;
+  auto weights = [&](bf16x8_t (&wv)[2][4], int step, int j) __attribute__((always_inline)) {
+    const int at = step < steps ? lane : 0;
+    step = min(step, steps - 1);
 #pragma unroll
-    for (int b = 0; b < 2; ++b)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) wv[b][j] = wp[(b * k16 + step * 4 + j) * 64];
+    for (int b = 0; b < 2; ++b) wv[b][j] = wp[(b * k16 + step * 4 + j) * 64 + at];
   };
   f32x16_t acc[2][TT];
 #pragma unroll
@@ -278,41 +287,90 @@ __global__ __launch_bounds__(256, 2) void dense_many_kernel(DenseArgs a, int row
     for (int t = 0; t < TT; ++t)
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[b][t][i] = 0.0f;
-  auto multiply = [&](const bf16_t* tile, const bf16x8_t (&wv)[2][4]) __attribute__((always_inline)) {
+  auto read_x = [&](const bf16_t* tile, int j, bf16x8_t (&xv)[TT]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      bf16x8_t xv[TT];
-#pragma unroll
-      for (int t = 0; t < TT; ++t)
-        xv[t] = *reinterpret_cast<const bf16x8_t*>(tile + (32 * t + n) * 64 + (((2 * j + kh) ^ (n & 7)) << 3));
-#pragma unroll
-      for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int t = 0; t < TT; ++t) acc[b][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv[b][j], xv[t], acc[b][t], 0, 0, 0);
-    }
+    for (int t = 0; t < TT; ++t) xv[t] = *reinterpret_cast<const bf16x8_t*>(tile + (32 * t + n) * 64 + (((2 * j + kh) ^ (n & 7)) << 3));
   };
-  bf16x8_t w0[2][4], w1[2][4];
-  request(tile0, 0);
-  weights(w0, 0);
-  for (int st = 0; st < steps; st += 2) {
-    __syncthreads();  // tile0 has arrived, tile1's readers are done
-    if (st + 1 < steps) {
-      request(tile1, st + 1);
-      weights(w1, st + 1);
+  auto multiply = [&](const bf16x8_t (&wv)[2][4], int j, const bf16x8_t (&xv)[TT]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) acc[b][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv[b][j], xv[t], acc[b][t], 0, 0, 0);
+  };
+  // The order in which a slice of a step (16 of its inputs) is issued: the next slice's reads between the first products, the
+  // weights of two steps on behind them.
+  auto spread = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int t = 0; t < TT; ++t) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
     }
-    multiply(tile0, w0);
+    __builtin_amdgcn_sched_group_barrier(0x008, TT, 0);
+    __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);
+  };
+  // Step st multiplies tile st % 3 and set st % 2 of the weights.  Both were requested two steps ago, so that a trip to memory
+  // has two steps of products to hide behind: at the wait the 8 + TT requests of the step between may still be on their
+  // way.  A slice's weights are requested into the registers that the slice has just used.  Past the end every lane
+  // requests the same piece, which is not used: the number of requests on their way is that of any other step.
+  bf16x8_t w0[2][4], w1[2][4];
+  auto step = [&](const bf16_t* now, bf16x8_t (&w)[2][4], bf16_t* later, int st) __attribute__((always_inline)) {
+    __builtin_amdgcn_s_waitcnt(0x0f70 | (8 + TT));  // vmcnt(8 + TT)
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();  // this step's tile is whole, the readers of the tile ahead of it are done
+    asm volatile("" ::: "memory");
+    request(later, st + 2);
+    bf16x8_t xa[TT], xb[TT];
+    read_x(now, 0, xa);
+    __builtin_amdgcn_sched_barrier(0);
+    read_x(now, 1, xb);
+    multiply(w, 0, xa);
+    weights(w, st + 2, 0);
+    spread();
+    read_x(now, 2, xa);
+    multiply(w, 1, xb);
+    weights(w, st + 2, 1);
+    spread();
+    read_x(now, 3, xb);
+    multiply(w, 2, xa);
+    weights(w, st + 2, 2);
+    spread();
+    multiply(w, 3, xb);
+    weights(w, st + 2, 3);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  request(tile0, 0);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) weights(w0, 0, j);
+  __builtin_amdgcn_sched_barrier(0);
+  request(tile1, 1);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) weights(w1, 1, j);
+  int st = 0;
+  for (; st + 6 <= steps; st += 6) {
+    step(tile0, w0, tile2, st);
+    step(tile1, w1, tile0, st + 1);
+    step(tile2, w0, tile1, st + 2);
+    step(tile0, w1, tile2, st + 3);
+    step(tile1, w0, tile0, st + 4);
+    step(tile2, w1, tile1, st + 5);
+  }
+  if (st < steps) {
+    step(tile0, w0, tile2, st);
     if (st + 1 < steps) {
-      __syncthreads();
+      step(tile1, w1, tile0, st + 1);
       if (st + 2 < steps) {
-        request(tile0, st + 2);
-        weights(w0, st + 2);
+        step(tile2, w0, tile1, st + 2);
+        if (st + 3 < steps) {
+          step(tile0, w1, tile2, st + 3);
+          if (st + 4 < steps) step(tile1, w0, tile0, st + 4);
+        }
       }
-      multiply(tile1, w1);
     }
   }
   const int row_w = rt * 256 + wave * 64;
-  float* const turn = reinterpret_cast<float*>(tile0) + wave * 1024;
-  __syncthreads();  // the last step's readers are done
+  float* const turn = reinterpret_cast<float*>(TT == 4 ? tile0 : (wave < 2 ? tile0 : tile1)) + (TT == 4 ? wave : wave & 1) * 1024;
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): no request is on its way into the tiles any more
+  __syncthreads();                     // the last step's readers are done
 #pragma unroll
   for (int b = 0; b < 2; ++b)
     store_block_rows<bf16_t, OUT, LISTED>(a, turn, acc[b], row_w + 32 * b, tt0, n_tok, list, row_tiles * 256, cut);
@@ -388,23 +446,46 @@ int launch_few(const DenseArgs& a, int64_t rows, int tokens, int blocks, hipStre
   return AWQ_OK;
 }
 
+// The time of a product of many tokens in us, but for what all forms of it share: what a choice between tiles of 64 and 128
+// tokens and numbers of shares of k needs.  The rates are fitted to 1,204 timings (ten shapes from 256 x 4,096 to 28,672 x 4,096,
+// 40 to 2,048 tokens, 1 to 16 shares, weights from memory; with 8.5 us added 5 % off in the mean square): a step of a
+// workgroup that has its compute unit to itself waits for memory, the longer the more weights are on their way; a second
+// workgroup on the unit adds its products; 5.4 TB/s of weights, 16 TB/s out of the L2s; the sums of the shares are written and
+// read at 5.7 TB/s.  The form it picks takes 1.9 % longer on average than the fastest of those timed (256 workgroups whatever
+// the size, tiles of 64 up to 256 tokens: 10 %, up to 79 %; 512 workgroups, as it was: 20 to 50 % at 129 to 512 tokens).
+float many_time(const DenseArgs& a, int64_t rows, bool wide, int64_t cuts) {
+  const int64_t row_tiles = rows / 256, tile = wide ? 128 : 64, tok_tiles = (a.M + tile - 1) / tile;
+  const float groups = (float)(row_tiles * tok_tiles * cuts * a.batch), steps = (float)(((a.k >> 6) + cuts - 1) / cuts);
+  const float wait = (wide ? 0.49f : 0.28f) + 0.05f * sqrtf((float)std::min<int64_t>(256, row_tiles * cuts * a.batch));
+  const float per_unit = ceilf(groups / 256.0f);
+  float t = steps * wait * ceilf(groups / 512.0f);
+  if (per_unit > 1.0f) t = std::max(t, steps * per_unit * (wide ? 0.87f : 0.56f));
+  t = std::max(t, (float)rows * (float)a.k * (float)a.batch * 2.0f / 5.4e6f);
+  t = std::max(t, groups * steps * (float)(32768 + tile * 128) / 16e6f);
+  if (cuts > 1) t += 1.5f + (float)cuts * (float)a.M * (float)rows * 8.0f / 5.7e6f;
+  return t;
+}
+
 template <int OUT>
 int launch_many(const DenseArgs& a, int64_t rows, hipStream_t st) {
-  // (25 to 32 tokens on few long rows read the tokens more than the weights: 4,096 x 12,288 37 us, below 33)
-  if (a.M <= 24 || (a.M <= kFewTokens && (rows >= 8192 || a.k <= 8192)))
+  // (21 to 32 tokens on few long rows read the tokens more than the weights: 4,096 x 12,288 at 32 37 us, below 32; 2,048 x 8,192 at 25
+  // 20.4, below 18.8)
+  if (a.M <= 20 || (a.M <= kFewTokens && (rows >= 8192 || a.k <= 4096)))
     return launch_few<OUT, false>(a, rows, (int)a.M, a.batch, st);
   const int row_tiles = (int)(rows / 256);
-  // few weights (few rows or a short k) are read again for less: tiles of 64 tokens where those of 128 are few
-  const bool small = (row_tiles <= 4 || a.k <= 512) && row_tiles * ((a.M + 127) / 128) <= 256;
-  const bool wide = a.M > 64 && !small;
+  int64_t most = 1;  // shares of k: at least four steps each
+  if (a.workspace && a.batch == 1 && a.M <= 65535)
+    most = std::max<int64_t>(1, std::min(std::min<int64_t>(16, a.k >> 8), a.workspace_floats / (a.M * rows)));
+  bool wide = false;
+  int64_t cuts = 1;
+  float best = HUGE_VALF;
+  for (int w = 0; w < 2; ++w)
+    for (int64_t c = 1; c <= most; ++c) {
+      const float t = many_time(a, rows, w != 0, c);
+      if (t < best) best = t, wide = w != 0, cuts = c;
+    }
   const int64_t tok_tiles = wide ? (a.M + 127) / 128 : (a.M + 63) / 64;
   const int64_t tiles = row_tiles * tok_tiles;
-  // two workgroups per compute unit, at least eight steps each (four in a small product)
-  int64_t cuts = 1;
-  if (a.workspace && a.batch == 1 && a.M <= 65535 && tiles < 384) {
-    cuts = std::min<int64_t>((512 + tiles / 2) / tiles, (a.k >> 6) / (small ? 4 : 8));
-    cuts = std::max<int64_t>(1, std::min<int64_t>(cuts, a.workspace_floats / (a.M * rows)));
-  }
   const dim3 grid((unsigned)((tiles * cuts + 7) / 8 * 8), (unsigned)a.batch);
   if (cuts > 1) {
     if (wide)

@@ -150,6 +150,31 @@ def test_products_of_few_tokens(awq, lib, dev, tokens, rows, k):
     assert np.abs(got[:tokens] - xv @ wv.T).max() < 8 * k ** 0.5 * 2.0 ** -24
 
 
+@pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 6, 7, 8, 9, 12, 13, 37])
+@pytest.mark.parametrize("tokens", [33, 129, 700])
+def test_products_of_every_number_of_steps(awq, lib, dev, tokens, steps):
+    """the products of many tokens go six steps of 64 inputs at a time and end anywhere; with and without shares of k.  The
+    operands are exact: a sum of k products in binary32 is off by about sqrt(k) roundings of 2^-24 of its size"""
+    rows, k = 300, 64 * steps
+    print("steps", tokens, steps, flush=True)
+    rng = np.random.default_rng(steps + tokens)
+    block = dev.torch.zeros(512 * k, dtype=dev.torch.bfloat16, device="cuda")
+    w, wv = dev.act(rng.standard_normal((rows, k)) / k ** 0.5, False)
+    awq.check(lib.awq_dense_pack(w.data_ptr(), 0, rows, k, block.data_ptr(), k, 0, 0, 0, dev.stream))
+    x, xv = dev.act(rng.standard_normal((tokens, k)), False)
+    ws = dev.empty((1 << 22,), True)
+    for floats in (ws.numel(), 0):
+        y = dev.empty((tokens + 1, rows), True)
+        a = awq.AwqDenseArgs()
+        a.w, a.k, a.tokens, a.n_segments, a.out = block.data_ptr(), k, tokens, 1, awq.DENSE_F32
+        a.segment[0] = awq.AwqDenseSegment(x.data_ptr(), y.data_ptr(), k, rows, 0, rows, 0, 0, 0, 0)
+        a.workspace, a.workspace_floats = (ws.data_ptr() if floats else None), floats
+        awq.check(lib.awq_dense(ctypes.byref(a), 0, dev.stream))
+        got = dev.host(y)
+        assert np.isnan(got[tokens]).all()
+        assert np.abs(got[:tokens] - xv @ wv.T).max() < 8 * k ** 0.5 * 2.0 ** -24
+
+
 def test_xielu_near_zero_and_far_out(awq, lib, dev):
     """the negative branch cancels near zero: small arguments keep their relative accuracy"""
     z = np.concatenate([-np.geomspace(1e-6, 60, 200), np.geomspace(1e-6, 60, 56)]).astype(np.float32)
