@@ -360,8 +360,9 @@ int launch_chunks(const LinearAttnArgs& a, hipStream_t st) {
   return AWQ_OK;
 }
 
-// below this many tokens the token-by-token form is as fast
-constexpr int kChunkFrom = 16;
+// tokens from which on a chunk is the faster form: 8 or 32 heads of 128, 5.3 us from 2 tokens on (binary32: 5.0), token by token
+// 5.6 at 2, 16.7 at 9 (binary32: 4.6, 5.6 at 3, 11.6)
+constexpr int kChunkFrom = 2, kChunkFromF32 = 3;
 
 template <typename T>
 int launch_step(const LinearAttnArgs& a, hipStream_t st) {
@@ -390,7 +391,7 @@ int launch_linear_attention(const LinearAttnArgs& a, bool f32, hipStream_t st) {
   AWQ_REQUIRE(a.heads >= 1 && a.dim >= 1 && a.vdim >= 1 && a.vdim <= 65536 && a.ldp % 8 == 0 &&
                   a.ldp >= (int64_t)a.heads * (2 * a.dim + a.vdim),
               "bad shape");
-  const bool chunks = a.log2_decay && a.M >= kChunkFrom && a.M < (1 << 30) && a.dim <= 256;
+  const bool chunks = a.log2_decay && a.M >= (f32 ? kChunkFromF32 : kChunkFrom) && a.M < (1 << 30) && a.dim <= 256;
   if (f32) return chunks ? launch_linear_chunks_f32(a, st) : launch_step<float>(a, st);
   if (chunks) {
     const bool whole = ((a.dim | a.vdim) & 7) == 0;
