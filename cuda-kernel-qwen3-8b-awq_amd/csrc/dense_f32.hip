@@ -1,6 +1,8 @@
 // Dense products of binary32 weights with one token or many (layers.hpp).
 #include "dense_device.hpp"
 
+#include <math.h>
+
 namespace {
 
 // --- one token -----------------------------------------------------------------------------------------------
@@ -102,8 +104,8 @@ __global__ __launch_bounds__(256) void dense_one_f32_kernel(DenseArgs a) {
 // multiplies element e of the two: the inputs of a step are met in another order on both sides alike.
 // Up to about 50 tokens bound by the weights' bytes (2 operations per token and 4 bytes against 134 TFLOP/s and 5.1 TB/s),
 // beyond by the matrix cores.  Where the tiles do not fill the device, k is cut over `cuts` workgroups and a second launch
-// adds their sums, as in bfloat16.  333 tokens: 1,024 rows of 4,096 inputs 46 + 7 us (the sums' launch), 7,168 of 1,024 64 + 15,
-// 32,768 of 1,024 at 128 tokens 82 (104 TFLOP/s); 4 x 4 sums per thread without matrix cores took 273, 155 and 191.
+// adds their sums, as in bfloat16.  333 tokens, sums added: 1,024 rows of 4,096 inputs 39 us, 7,168 of 1,024 57, 32,768 of 1,024
+// 212 (106 TFLOP/s); 4 x 4 sums per thread without matrix cores took 270, 135 and 482.  20 tokens on 1,024 x 4,096: 18, was 273.
 template <int TW, int KW, int C, int OUT, bool LISTED = false>
 __global__ __launch_bounds__(256) void dense_many_f32_kernel(DenseArgs a, int row_tiles, int tok_tiles, int cuts) {
   static_assert(TW * KW == 2, "four wavefronts, two of them share the rows");
@@ -216,10 +218,19 @@ int launch_one(const DenseArgs& a, int64_t rows, hipStream_t st) {
   return AWQ_OK;
 }
 
-// tokens of a workgroup's tile: 128 unless the last tile would be mostly padding
-int tile_of(int64_t M) {
-  if (M <= 32) return 32;
-  return M > 64 && round_up(M, 128) * 5 <= round_up(M, 64) * 6 ? 128 : 64;
+// The time of a product of many tokens in us, but for what all forms of it share, for the choice between tiles of 32, 64 and 128
+// tokens and shares of k: a step of a workgroup that has its compute unit to itself, the steps of several on one, weights
+// at 4.6 TB/s, the shares' sums written and read at 6.8 TB/s.  Fitted to 1,190 timings (eight shapes from 256 x 1,536 to 32,768
+// x 1,024, 3 to 512 tokens, 1 to 16 shares; 5 % off in the mean square with 7.3 us added).  The form it picks takes 2.9 % longer
+// on average than the fastest timed; two workgroups per compute unit whatever the size, as it was, 7.4 %, up to 30 %.
+float many_time(const DenseArgs& a, int64_t rows, int tile, int64_t cuts) {
+  const float alone = tile == 32 ? 0.52f : tile == 64 ? 0.65f : 1.18f, beside = tile == 32 ? 0.32f : tile == 64 ? 0.56f : 1.05f;
+  const float steps = (float)(((a.k >> 5) + cuts - 1) / cuts);
+  const float per_unit = ceilf((float)(rows / 64 * ((a.M + tile - 1) / tile) * cuts * a.batch) / 256.0f);
+  float t = std::max(steps * alone, (float)rows * (float)a.k * (float)a.batch * 4.0f / 4.6e6f);
+  if (per_unit > 1.0f) t = std::max(t, steps * beside * per_unit);
+  if (cuts > 1) t += 2.3f + (float)cuts * (float)a.M * (float)rows * 8.0f / 6.8e6f;
+  return t;
 }
 
 template <int OUT, bool LISTED>
@@ -238,16 +249,19 @@ int launch_tiles(const DenseArgs& a, int64_t rows, int tile, int tok_tiles, int 
 
 template <int OUT>
 int launch_many(const DenseArgs& a, int64_t rows, hipStream_t st) {
-  const int tile = tile_of(a.M);
-  const int64_t tok_tiles = (a.M + tile - 1) / tile, tiles = rows / 64 * tok_tiles;
-  AWQ_REQUIRE(tiles < (1ll << 28), "too large");
-  // two workgroups per compute unit, at least four steps each (48 tokens, 1,024 x 3,072: sixteen tiles alone took 209 us, cut in
-  // eight 7 + 5)
+  int64_t most = 1;  // shares of k: at least four steps each
+  if (a.workspace && a.batch == 1 && a.M <= 65535)
+    most = std::max<int64_t>(1, std::min(std::min<int64_t>(16, a.k >> 7), a.workspace_floats / (a.M * rows)));
+  int tile = 32;
   int64_t cuts = 1;
-  if (a.workspace && a.batch == 1 && a.M <= 65535 && tiles < 384) {
-    cuts = std::min<int64_t>((512 + tiles / 2) / tiles, (a.k >> 5) / 4);
-    cuts = std::max<int64_t>(1, std::min<int64_t>(cuts, a.workspace_floats / (a.M * rows)));
-  }
+  float best = HUGE_VALF;
+  for (int t = 32; t <= 128; t *= 2)
+    for (int64_t c = 1; c <= most; ++c) {
+      const float time = many_time(a, rows, t, c);
+      if (time < best) best = time, tile = t, cuts = c;
+    }
+  const int64_t tok_tiles = (a.M + tile - 1) / tile, tiles = rows / 64 * tok_tiles;
+  AWQ_REQUIRE(tiles < (1ll << 26), "too large");
   if (cuts == 1) return launch_tiles<OUT, false>(a, rows, tile, (int)tok_tiles, 1, st);
   if (int rc = launch_tiles<DENSE_PART, false>(a, rows, tile, (int)tok_tiles, (int)cuts, st)) return rc;
   hipLaunchKernelGGL((dense_parts_kernel<float, OUT>), dim3((unsigned)((rows / 4 + 255) / 256), (unsigned)a.M), dim3(256), 0, st, a,
