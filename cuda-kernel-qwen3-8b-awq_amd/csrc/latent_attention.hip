@@ -1,6 +1,6 @@
 // Attention over a shared latent (layers.hpp): keys and values of all heads are linear images of one cached vector per
 // position, beside a rotated key part that the heads share; softmax with a learned score that has no key.
-#include "layers.hpp"
+#include "query_attention.hpp"
 
 namespace {
 
@@ -144,62 +144,40 @@ __global__ __launch_bounds__(256) void latent_query_one_kernel(LatentAttnArgs a,
 }
 
 // --- in the latent space, a query at a time --------------------------------------------------------------------
-// A workgroup per (head, token), a thread per key, blocks of 256 keys with a running maximum.  Any sizes; the binary32
-// form.  `kv_in`: padded inputs of the value product.
-constexpr int kMaxColsPerThread = 4;
-template <typename T>
+// A few queries of a head per workgroup (query_attention.hpp).  Any sizes; the binary32 form.  `kv_in`: padded inputs of the value
+// product.
+constexpr int kMaxCols = 1024;
+template <typename T, int QN>
 __global__ __launch_bounds__(256) void latent_query_kernel(LatentAttnArgs a, int kv_in) {
-  extern __shared__ float lds[];
-  const int row = a.l.row(), rank = a.l.rank;
-  float* q = lds;            // [row]
-  float* p = lds + row;      // [256]
-  float* red = p + 256;      // [4]
-  const int h = blockIdx.x, t = blockIdx.y, tid = threadIdx.x;
-  const int pos = a.pos.position() + t;
-  const T* const ql = reinterpret_cast<const T*>(a.ql) + ((int64_t)t * a.heads + h) * row;
-  for (int d = tid; d < row; d += 256) q[d] = (float)ql[d];
-  const T* const cache = reinterpret_cast<const T*>(a.cache);
-  float m = a.sink ? a.sink[h] : -INFINITY, l = a.sink ? 1.0f : 0.0f, acc[kMaxColsPerThread] = {};
-  __syncthreads();
-  for (int k0 = 0; k0 <= pos; k0 += 256) {
-    const int key = k0 + tid;
-    float s = -INFINITY;
-    if (key <= pos) {
-      const T* kr = cache + (int64_t)key * row;
-      float dot = 0.0f;
-      for (int d = 0; d < row; ++d) dot = __builtin_fmaf(q[d], (float)kr[d], dot);
-      s = dot * a.scale;
-    }
-    float mx = s;
+  extern __shared__ __attribute__((aligned(16))) float lds[];  // query_lds(row, QN)
+  const int row = a.l.row(), rank = a.l.rank, M = (int)a.M;
+  const int h = blockIdx.x, t0 = blockIdx.y * QN, tid = threadIdx.x;
+  const int pos0 = a.pos.position();
+  int pos[QN];
+  float m[QN], l[QN];
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-    if ((tid & 63) == 0) red[tid >> 6] = mx;
-    __syncthreads();
-    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    const float m_new = fmaxf(m, mx), alpha = expf(m - m_new), e = expf(s - m_new);
-    p[tid] = e;
-    const float sum = wave_sum(e);
-    __syncthreads();
-    if ((tid & 63) == 0) red[tid >> 6] = sum;
-    __syncthreads();
-    l = l * alpha + ((red[0] + red[1]) + (red[2] + red[3]));
-    m = m_new;
-    const int n = min(256, pos + 1 - k0);
-#pragma unroll
-    for (int c = 0; c < kMaxColsPerThread; ++c) {
-      const int col = c * 256 + tid;
-      if (col < rank) {
-        float v = acc[c] * alpha;
-        for (int j = 0; j < n; ++j) v = __builtin_fmaf(p[j], (float)cache[(int64_t)(k0 + j) * row + col], v);
-        acc[c] = v;
-      }
-    }
-    __syncthreads();
+  for (int i = 0; i < QN; ++i) {
+    const int t = min(t0 + i, M - 1);
+    const T* const ql = reinterpret_cast<const T*>(a.ql) + ((int64_t)t * a.heads + h) * row;
+    for (int d = tid; d < row; d += 256) lds[i * row + d] = (float)ql[d];
+    pos[i] = pos0 + t;
+    m[i] = a.sink ? a.sink[h] : -INFINITY;
+    l[i] = a.sink ? 1.0f : 0.0f;
   }
-  T* out = reinterpret_cast<T*>(a.ol) + ((int64_t)t * a.heads + h) * kv_in;
+  const T* const cache = reinterpret_cast<const T*>(a.cache);
+  const auto key_row = [&](int key) { return cache + (int64_t)key * row; };
+  attend_queries<T, QN>(
+      lds, row, rank, 0, pos[QN - 1], key_row, key_row,
+      [&](int i, int key, float dot) { return key <= pos[i] ? dot * a.scale : -INFINITY; }, m, l,
+      [&](int i, int col, q4_t sum, float total) {
+        if (t0 + i >= M) return;
+        T* const out = reinterpret_cast<T*>(a.ol) + ((int64_t)(t0 + i) * a.heads + h) * kv_in + col;
 #pragma unroll
-  for (int c = 0; c < kMaxColsPerThread; ++c)
-    if (c * 256 + tid < kv_in) out[c * 256 + tid] = (T)(c * 256 + tid < rank ? acc[c] / l : 0.0f);
+        for (int e = 0; e < 4; ++e)
+          if (col + e < rank) out[e] = (T)(sum[e] / total);
+      });
+  for (int i = 0; i < QN && t0 + i < M; ++i)  // what pads the value product's inputs
+    for (int d = rank + tid; d < kv_in; d += 256) reinterpret_cast<T*>(a.ol)[((int64_t)(t0 + i) * a.heads + h) * kv_in + d] = (T)0.0f;
 }
 
 // --- in the latent space, on the matrix cores ------------------------------------------------------------------
@@ -728,7 +706,7 @@ int launch_latent_pack(const LatentAttnArgs& a, const void* uk, const void* uv, 
 
 int launch_latent_attention(const LatentAttnArgs& a, bool f32, hipStream_t st) {
   AWQ_REQUIRE(a.q && a.freq && a.cache && a.w_uk && a.w_uv && a.ctx && a.qa && a.ql && a.ol && (!a.down || a.norm), "bad arguments");
-  AWQ_REQUIRE(a.heads >= 1 && a.heads <= 65535 && a.dim >= 1 && a.vdim >= 1 && a.l.rank >= 1 && a.l.rank <= 256 * kMaxColsPerThread &&
+  AWQ_REQUIRE(a.heads >= 1 && a.heads <= 65535 && a.dim >= 1 && a.vdim >= 1 && a.l.rank >= 1 && a.l.rank <= kMaxCols &&
                   a.l.rot >= 2 && a.l.rot % 2 == 0 && a.l.rot <= 1024,
               "bad shape");
   AWQ_REQUIRE(a.M >= 1 && a.M <= 65535 && a.M * a.heads < (1ll << 30) && a.ldq >= (int64_t)a.heads * (a.dim + a.l.rot) &&
@@ -783,10 +761,13 @@ int launch_latent_attention(const LatentAttnArgs& a, bool f32, hipStream_t st) {
     }
     hipLaunchKernelGGL(latent_combine_kernel, dim3((unsigned)(a.M * a.heads)), dim3(256), 0, st, a, parts, (int)v_inputs(a));
   } else {
-    const size_t lds = (size_t)(a.l.row() + 256 + 4) * 4;
-    const dim3 g((unsigned)a.heads, (unsigned)a.M);
-    if (f32) hipLaunchKernelGGL(latent_query_kernel<float>, g, dim3(256), lds, st, a, (int)v_inputs(a));
-    else hipLaunchKernelGGL(latent_query_kernel<bf16_t>, g, dim3(256), lds, st, a, (int)v_inputs(a));
+    const int row = a.l.row(), kv_in = (int)v_inputs(a);
+    const bool few = a.M < 4 || query_lds(row, 4) > 65536;
+    const dim3 g((unsigned)a.heads, (unsigned)(few ? a.M : (a.M + 3) / 4));
+    if (f32 && few) hipLaunchKernelGGL((latent_query_kernel<float, 1>), g, dim3(256), query_lds(row, 1), st, a, kv_in);
+    else if (f32) hipLaunchKernelGGL((latent_query_kernel<float, 4>), g, dim3(256), query_lds(row, 4), st, a, kv_in);
+    else if (few) hipLaunchKernelGGL((latent_query_kernel<bf16_t, 1>), g, dim3(256), query_lds(row, 1), st, a, kv_in);
+    else hipLaunchKernelGGL((latent_query_kernel<bf16_t, 4>), g, dim3(256), query_lds(row, 4), st, a, kv_in);
   }
   AWQ_HIP_TRY(hipGetLastError());
   return heads_product(a, a.w_uv, latent_uv_block(a), v_inputs(a), a.ol, a.ctx, a.ldc, a.vdim, a.vdim, f32, st);

@@ -1,5 +1,5 @@
 // Attention over a sliding window with a distance bias (layers.hpp).
-#include "layers.hpp"
+#include "query_attention.hpp"
 
 namespace {
 
@@ -74,66 +74,41 @@ __global__ __launch_bounds__(256) void window_append8_kernel(WindowAttnArgs a, i
   }
 }
 
-// A query at a time: a workgroup per (token, head), a thread per key, blocks of 256 keys with a running maximum.
-// Any sizes; the binary32 form and what the tiled kernel has no instance for.
-constexpr int kMaxColsPerThread = 4;
-template <typename T>
+// A few queries of a head at a time (query_attention.hpp); the binary32 form and what the tiled kernel has no instance for.
+constexpr int kMaxCols = 1024;
+template <typename T, int QN>
 __global__ __launch_bounds__(256) void window_query_kernel(WindowAttnArgs a) {
-  extern __shared__ float lds[];
-  float* q = lds;              // [dim]
-  float* p = lds + a.dim;      // [256]
-  float* red = p + 256;        // [4]
-  const int h = blockIdx.x, t = blockIdx.y, tid = threadIdx.x;
+  extern __shared__ __attribute__((aligned(16))) float lds[];  // query_lds(kl.row, QN)
+  const int h = blockIdx.x, t0 = blockIdx.y * QN, tid = threadIdx.x, row = a.kl.row, M = (int)a.M;
   const int g = h / (a.heads / a.kv_heads);
-  const int pos = a.pos.position() + t;
-  const T* qrow = reinterpret_cast<const T*>(a.proj) + (int64_t)t * a.ldp + (int64_t)h * a.dim;
-  for (int d = tid; d < a.dim; d += 256) q[d] = (float)qrow[d];
-  const float mul = a.scale * temperature(a, pos), slope = a.slope[h];
-  const int lo = a.window > 0 ? max(0, pos - a.window + 1) : 0;
-  float m = -INFINITY, l = 0.0f, acc[kMaxColsPerThread] = {};
-  __syncthreads();
-  for (int k0 = lo; k0 <= pos; k0 += 256) {
-    const int key = k0 + tid;
-    float s = -INFINITY;
-    if (key <= pos) {
-      const T* kr = reinterpret_cast<const T*>(a.k_cache) + ring_row(a.kl, g, key % a.kl.slots);
-      float dot = 0.0f;
-      for (int d = 0; d < a.dim; ++d) dot = __builtin_fmaf(q[d], (float)kr[d], dot);
-      s = dot * mul - slope * (float)(pos - key);
-    }
-    float mx = s;
+  const int pos0 = a.pos.position();
+  const float slope = a.slope[h];
+  int pos[QN], lo[QN];
+  float mul[QN], m[QN], l[QN];
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
-    if ((tid & 63) == 0) red[tid >> 6] = mx;
-    __syncthreads();
-    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-    const float m_new = fmaxf(m, mx), alpha = expf(m - m_new), e = expf(s - m_new);
-    p[tid] = e;
-    float sum = e;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
-    __syncthreads();
-    if ((tid & 63) == 0) red[tid >> 6] = sum;
-    __syncthreads();
-    l = l * alpha + ((red[0] + red[1]) + (red[2] + red[3]));
-    m = m_new;
-    const int n = min(256, pos + 1 - k0);
-#pragma unroll
-    for (int c = 0; c < kMaxColsPerThread; ++c) {
-      const int col = c * 256 + tid;
-      if (col < a.vdim) {
-        float v = acc[c] * alpha;
-        for (int j = 0; j < n; ++j)
-          v = __builtin_fmaf(p[j], (float)reinterpret_cast<const T*>(a.v_cache)[ring_row(a.vl, g, (k0 + j) % a.vl.slots) + col], v);
-        acc[c] = v;
-      }
-    }
-    __syncthreads();
+  for (int i = 0; i < QN; ++i) {
+    const int t = min(t0 + i, M - 1);
+    const T* const q = reinterpret_cast<const T*>(a.proj) + (int64_t)t * a.ldp + (int64_t)h * a.dim;
+    for (int d = tid; d < row; d += 256) lds[i * row + d] = d < a.dim ? (float)q[d] : 0.0f;
+    pos[i] = pos0 + t;
+    lo[i] = a.window > 0 ? max(0, pos[i] - a.window + 1) : 0;
+    mul[i] = a.scale * temperature(a, pos[i]);
+    m[i] = -INFINITY;
+    l[i] = 0.0f;
   }
-  T* out = reinterpret_cast<T*>(a.ctx) + (int64_t)t * a.ldc + (int64_t)h * a.vdim;
+  const T* const kc = reinterpret_cast<const T*>(a.k_cache);
+  const T* const vc = reinterpret_cast<const T*>(a.v_cache);
+  attend_queries<T, QN>(
+      lds, row, a.vdim, lo[0], pos[QN - 1], [&](int key) { return kc + ring_row(a.kl, g, key % a.kl.slots); },
+      [&](int key) { return vc + ring_row(a.vl, g, key % a.vl.slots); },
+      [&](int i, int key, float dot) { return key >= lo[i] && key <= pos[i] ? dot * mul[i] - slope * (float)(pos[i] - key) : -INFINITY; }, m, l,
+      [&](int i, int col, q4_t sum, float total) {
+        if (t0 + i >= M) return;
+        T* const out = reinterpret_cast<T*>(a.ctx) + (int64_t)(t0 + i) * a.ldc + (int64_t)h * a.vdim + col;
 #pragma unroll
-  for (int c = 0; c < kMaxColsPerThread; ++c)
-    if (c * 256 + tid < a.vdim) out[c * 256 + tid] = (T)(acc[c] / l);
+        for (int e = 0; e < 4; ++e)
+          if (col + e < a.vdim) out[e] = (T)(sum[e] / total);
+      });
 }
 
 // One token.  blockIdx.x: kv head and up to R of its query heads, blockIdx.y: 64 of the visible keys.  The rows a
@@ -573,8 +548,10 @@ int launch_append(const WindowAttnArgs& a, hipStream_t st) {
 
 template <typename T>
 int launch_queries(const WindowAttnArgs& a, hipStream_t st) {
-  hipLaunchKernelGGL(window_query_kernel<T>, dim3((unsigned)a.heads, (unsigned)a.M), dim3(256),
-                     (size_t)(a.dim + 256 + 4) * sizeof(float), st, a);
+  if (a.M >= 4)
+    hipLaunchKernelGGL((window_query_kernel<T, 4>), dim3((unsigned)a.heads, (unsigned)((a.M + 3) / 4)), dim3(256), query_lds(a.kl.row, 4), st, a);
+  else
+    hipLaunchKernelGGL((window_query_kernel<T, 1>), dim3((unsigned)a.heads, (unsigned)a.M), dim3(256), query_lds(a.kl.row, 1), st, a);
   AWQ_HIP_TRY(hipGetLastError());
   return AWQ_OK;
 }
@@ -591,7 +568,7 @@ int64_t window_parts_floats(int32_t heads, int32_t vdim, int64_t window, int64_t
 int launch_window_attention(const WindowAttnArgs& a, bool f32, hipStream_t st) {
   AWQ_REQUIRE(a.proj && a.k_cache && a.v_cache && a.ctx && a.slope && a.M >= 1 && a.M <= 65535, "bad arguments");
   AWQ_REQUIRE(a.heads >= 1 && a.kv_heads >= 1 && a.heads % a.kv_heads == 0, "heads must be a multiple of kv_heads");
-  AWQ_REQUIRE(a.dim >= 1 && a.dim <= 1024 && a.vdim >= 1 && a.vdim <= 256 * kMaxColsPerThread, "head sizes must be at most 1024");
+  AWQ_REQUIRE(a.dim >= 1 && a.dim <= 1024 && a.vdim >= 1 && a.vdim <= kMaxCols, "head sizes must be at most 1024");
   AWQ_REQUIRE(a.kl.slots > 0 && a.kl.slots % 64 == 0 && a.vl.slots == a.kl.slots && a.kl.row == window_row_padded(a.dim) &&
                   a.vl.row == window_row_padded(a.vdim) && a.ldp % 8 == 0 && a.ldc % 8 == 0,
               "bad cache layout");
