@@ -22,11 +22,8 @@ __global__ __launch_bounds__(NW * 64) void dense_one_kernel(DenseArgs a) {
   const DenseSegment& s = segment_of(a, row0);
   const int local = row0 - s.row0;
   if (local >= s.rows) return;  // padding
-  int group = blockIdx.y;
-  if (a.ids) {
-    group = a.ids[blockIdx.y];
-    if (group >= a.n_groups) return;
-  }
+  const int group = block_of_product(a);
+  if (group < 0) return;
   const int steps = (int)(a.k >> 5);  // even: k is a multiple of 64
   const int per = (steps + NW - 1) / NW;
   const int s0 = min(wave * per, steps), s1 = min(s0 + per, steps);
@@ -565,6 +562,7 @@ int launch_dense(const DenseArgs& args, bool f32, hipStream_t st) {
   AWQ_REQUIRE(a.batch >= 1 && a.batch <= 65535 && (a.batch == 1 || (a.out == DENSE_STORE && a.w_batch % 8 == 0 && a.x_batch % 8 == 0)),
               "bad batch");
   AWQ_REQUIRE(!a.ids || (a.M == 1 && a.n_groups >= 0), "weight blocks by number take one token");
+  AWQ_REQUIRE(a.fixed == 0 || (a.ids && a.fixed > 0 && a.fixed <= a.batch), "bad number of fixed weight blocks");
   if (a.tiles) {
     AWQ_REQUIRE(a.out == DENSE_STORE && a.list && a.list_div >= 1 && a.batch == 1 && a.max_tiles >= 1 && a.max_tiles <= 65535 &&
                     a.tile_tokens >= 1 && a.tile_tokens <= (f32 ? 64 : 128),

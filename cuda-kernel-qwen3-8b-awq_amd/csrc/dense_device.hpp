@@ -105,6 +105,15 @@ __device__ __forceinline__ const DenseSegment& segment_of(const DenseArgs& a, in
   return a.seg[i];
 }
 
+// the weight block of this workgroup's product (one token), or -1: it is left out
+__device__ __forceinline__ int block_of_product(const DenseArgs& a) {
+  const int b = blockIdx.y, by_number = a.batch - a.fixed;
+  if (!a.ids) return b;
+  if (b >= by_number) return a.n_groups + b - by_number;
+  const int group = a.ids[b];
+  return group < a.n_groups ? group : -1;
+}
+
 // one output of one token (DENSE_STORE), `y0` elements into the segment's output
 template <typename T>
 __device__ __forceinline__ void store_one(const DenseSegment& s, int64_t y0, int64_t t, int row, float v) {

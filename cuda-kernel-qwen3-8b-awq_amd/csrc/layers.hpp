@@ -101,6 +101,7 @@ struct DenseArgs {
   int64_t w_batch = 0, x_batch = 0, y_batch = 0;
   const int32_t* ids = nullptr;
   int32_t n_groups = 0;
+  int32_t fixed = 0;  // with ids: the last `fixed` products take the blocks n_groups, n_groups + 1, ..
   // Many tokens, each with weight blocks of its own (DENSE_STORE): `tiles` (device, max_tiles of them, count 0 behind the
   // last) name runs of `list`; entry p of the list reads input row p / list_div and writes output row p.
   const DenseTile* tiles = nullptr;

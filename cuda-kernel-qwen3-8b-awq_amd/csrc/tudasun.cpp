@@ -254,6 +254,7 @@ struct LayerDev {
   void *w_down = nullptr, *w_shared_down = nullptr, *w_gate_up = nullptr, *w_expert_down = nullptr;
   const float *act = nullptr, *correction = nullptr;
   int64_t ff_k = 0, shared_k = 0, gate_up_block = 0, expert_down_block = 0;
+  bool shared_last = false;
   // token input
   void *w_side_gate = nullptr, *w_side_proj = nullptr;
   const float* side_norm = nullptr;
@@ -430,14 +431,22 @@ int TudasunEngine::load_layer(Loader& ldr, int i) {
         mid.push_back({f + "shared.up", 0, PACK_UP, true});
         mid.push_back({f + "shared.sg", 1});
         L.shared_k = round_up(s.shared_ff, kDenseKAlign);
-        if (int rc = load_out(ldr, f + "shared.down", W, L.shared_k, &L.w_shared_down)) return rc;
+        if (L.shared_k != L.ff_k)
+          if (int rc = load_out(ldr, f + "shared.down", W, L.shared_k, &L.w_shared_down)) return rc;
       }
       if (int rc = ldr.vector(f + "correction", &L.correction)) return rc;
       const int64_t gu_rows = round_up(dense_glu_rows(s.ff), kDenseRowAlign), down_rows = round_up(W, kDenseRowAlign);
       L.gate_up_block = gu_rows * ld;
       L.expert_down_block = down_rows * L.ff_k;
       if (int rc = ldr.block(&L.w_gate_up, s.experts * gu_rows, ld)) return rc;
-      if (int rc = ldr.block(&L.w_expert_down, s.experts * down_rows, L.ff_k)) return rc;
+      // the shared expert's matrix is a block behind the experts' where its inputs are as many: one token then meets them all in
+      // one launch
+      L.shared_last = s.shared_ff > 0 && L.shared_k == L.ff_k;
+      if (int rc = ldr.block(&L.w_expert_down, (s.experts + (L.shared_last ? 1 : 0)) * down_rows, L.ff_k)) return rc;
+      if (L.shared_last) {
+        L.w_shared_down = (char*)L.w_expert_down + dense_weight_bytes(s.experts * down_rows, L.ff_k, f32);
+        if (int rc = ldr.matrix(f + "shared.down", L.w_expert_down, L.ff_k, s.experts * down_rows, 0)) return rc;
+      }
       for (int e = 0; e < s.experts; ++e) {
         const std::string x = f + "e" + std::to_string(e) + ".";
         if (int rc = ldr.matrix(x + "gate", L.w_gate_up, ld, e * gu_rows, 0, PACK_GATE)) return rc;
@@ -483,10 +492,10 @@ int TudasunEngine::make_activations(Buffers* b, int64_t n) {
     }
     if (s.mlp == MLP_DENSE) mid = std::max(mid, L.ff_k);
     if (s.mlp == MLP_EXPERTS) {
-      mid = std::max(mid, s.top * L.ff_k);
+      mid = std::max(mid, (s.top + (L.shared_last ? 1 : 0)) * L.ff_k);
       shared_mid = std::max(shared_mid, L.shared_k);
       router = std::max<int64_t>(router, s.outputs());
-      pairs = std::max<int64_t>(pairs, (int64_t)s.top * width);
+      pairs = std::max<int64_t>(pairs, (int64_t)(s.top + (L.shared_last ? 1 : 0)) * width);
       top = std::max<int64_t>(top, s.top);
       tiles = std::max<int64_t>(tiles, route_tiles_room(n, s.top, s.experts, s.outputs()));
     }
@@ -672,6 +681,10 @@ int TudasunEngine::dense_feed_forward(int i, Buffers& b, int64_t M) {
 int TudasunEngine::routed_feed_forward(int i, Buffers& b, int64_t M, JoinArgs* end) {
   const LayerSpec& s = spec.layers[i];
   const LayerDev& L = layers[i];
+  // one token: the shared expert is the choice behind the last
+  const bool beside = M == 1 && L.shared_last && s.experts;
+  void* const shared_mid = beside ? (char*)b.mid + s.top * L.ff_k * unit() : b.shared_mid;
+  float* const shared_y = beside ? b.pairs + (int64_t)s.top * width : b.y;
   {
     DenseArgs a = product(L.mid.w, ld, M);
     DenseSegment& g = segment(&a, b.h, ld, b.gate, ldg, L.mid.at[0], width);
@@ -679,7 +692,7 @@ int TudasunEngine::routed_feed_forward(int i, Buffers& b, int64_t M, JoinArgs* e
     g.bias = L.rg2_b;
     segment(&a, b.h, ld, b.router, s.outputs(), L.mid.at[1], s.outputs()).y_f32 = 1;
     if (s.shared_ff) {
-      DenseSegment& m = segment(&a, b.h, ld, b.shared_mid, L.shared_k, L.mid.at[2], dense_glu_rows(s.shared_ff));
+      DenseSegment& m = segment(&a, b.h, ld, shared_mid, L.shared_k, L.mid.at[2], dense_glu_rows(s.shared_ff));
       m.act = DENSE_GLU;
       m.glu_rows = s.shared_ff;
       segment(&a, b.h, ld, b.shared_gate, 1, L.mid.at[3], 1).y_f32 = 1;
@@ -732,15 +745,16 @@ int TudasunEngine::routed_feed_forward(int i, Buffers& b, int64_t M, JoinArgs* e
     DenseArgs down = product(L.w_expert_down, L.ff_k, M);
     segment(&down, b.mid, L.ff_k, b.pairs, width, 0, width).y_f32 = 1;
     choose(&down, L.expert_down_block, L.ff_k, width, 0);
+    if (beside) down.batch += 1, down.fixed = 1;
     if (int rc = launch_dense(down, f32, stream)) return rc;
   }
-  if (s.shared_ff) {
+  if (s.shared_ff && !beside) {
     DenseArgs a = product(L.w_shared_down, L.shared_k, M);
     a.out = DENSE_F32;
     segment(&a, b.shared_mid, L.shared_k, b.y, width, 0, width);
     if (int rc = launch_dense(a, f32, stream)) return rc;
   }
-  end->y = s.shared_ff ? b.y : nullptr;
+  end->y = s.shared_ff ? shared_y : nullptr;
   end->y_gate = s.shared_ff ? b.shared_gate : nullptr;
   end->pairs = b.pairs;
   end->ids = b.ids;
