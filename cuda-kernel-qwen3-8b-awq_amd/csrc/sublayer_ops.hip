@@ -136,6 +136,73 @@ __global__ __launch_bounds__(1024) void join_kernel(JoinArgs a) {
   }
 }
 
+// The same where a row is a workgroup's threads times V at most and a token has at most kJoinTop choices, which then wait in
+// registers.  Bound by trips to memory: the form above makes three, one behind the other, and one more for each choice; here
+// everything is requested at once (an identity output's row of `pairs` too, which is then not used).  Tudasun of width 4,096,
+// 64 tokens one by one with 12 launches each: 38.6 -> 37.8 ms; width 1,024 in binary32, 24 tokens: 7.73 -> 7.50.
+constexpr int kJoinTop = 8;
+template <typename T, int V>
+__global__ __launch_bounds__(1024) void join_row_kernel(JoinArgs a) {
+  __shared__ float sums[2][16];
+  const int tid = threadIdx.x, W = (int)a.width, c = tid * V;
+  const int64_t t = blockIdx.x;
+  const bool mine = c < W;
+  float v[V] = {}, g[V] = {}, r[V] = {}, w_post[V] = {}, w_next[V] = {}, h[V] = {}, u[kJoinTop][V], w[kJoinTop];
+  int ids[kJoinTop];
+  if (mine) {
+    if (a.y) read<float, V>(a.y + t * W + c, v);
+    if (a.gate) read<T, V>(reinterpret_cast<const T*>(a.gate) + t * a.ldg + c, g);
+    read<float, V>(a.x + t * W + c, r);
+    read<float, V>(a.w_post + c, w_post);
+    if (a.w_next) read<float, V>(a.w_next + c, w_next);
+    if (a.top > 0) read<T, V>(reinterpret_cast<const T*>(a.h) + t * a.ldh + c, h);
+  }
+#pragma unroll
+  for (int j = 0; j < kJoinTop; ++j)
+    if (j < a.top) {
+      ids[j] = a.ids[t * a.top + j];
+      w[j] = a.weights[t * a.top + j];
+      if (mine) read<float, V>(a.pairs + (t * a.top + j) * W + c, u[j]);
+    }
+  const float y_mul = a.y_gate ? 1.0f / (1.0f + expf(-a.y_gate[t])) : 1.0f;
+  float sq = 0.0f;
+  if (mine) {
+    if (a.y) {
+#pragma unroll
+      for (int i = 0; i < V; ++i) v[i] *= y_mul;
+    }
+#pragma unroll
+    for (int j = 0; j < kJoinTop; ++j)
+      if (j < a.top) {
+#pragma unroll
+        for (int i = 0; i < V; ++i) v[i] = __builtin_fmaf(w[j], ids[j] < a.experts ? u[j][i] : h[i], v[i]);
+      }
+    if (a.gate) {
+#pragma unroll
+      for (int i = 0; i < V; ++i) v[i] *= g[i];
+    }
+#pragma unroll
+    for (int i = 0; i < V; ++i) sq = __builtin_fmaf(v[i], v[i], sq);
+  }
+  const float inv = 1.0f / sqrtf(group_sum(sq, sums[0]) / (float)W + a.eps);
+  sq = 0.0f;
+  if (mine) {
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      r[i] = r[i] + v[i] * inv * w_post[i];
+      sq = __builtin_fmaf(r[i], r[i], sq);
+    }
+    write<float, V>(a.x + t * W + c, r);
+  }
+  if (!a.out) return;
+  if (a.w_next) {
+    const float next = 1.0f / sqrtf(group_sum(sq, sums[1]) / (float)W + a.eps);
+#pragma unroll
+    for (int i = 0; i < V; ++i) r[i] = r[i] * next * w_next[i];
+  }
+  if (mine) write<T, V>(reinterpret_cast<T*>(a.out) + t * a.ldo + c, r);
+}
+
 template <typename T, int V>
 __global__ __launch_bounds__(1024) void polynorm_kernel(T* z, int64_t ld, int n, const float* __restrict__ abce, float eps) {
   __shared__ float sums[3][16];
@@ -215,7 +282,9 @@ int join(const JoinArgs& a, hipStream_t st) {
   const dim3 g((unsigned)a.M);
   const int64_t items = a.width / (quads ? 4 : 1);
   const dim3 b((unsigned)std::min<int64_t>(a.M < 512 ? 1024 : 256, round_up(items, 64)));
-  if (quads) hipLaunchKernelGGL((join_kernel<T, 4>), g, b, lds, st, a);
+  // by measurement above wherever the registers hold a row; wider rows, more choices and odd widths keep the general form
+  if (quads && items <= (int64_t)b.x && a.top <= kJoinTop) hipLaunchKernelGGL((join_row_kernel<T, 4>), g, b, 0, st, a);
+  else if (quads) hipLaunchKernelGGL((join_kernel<T, 4>), g, b, lds, st, a);
   else hipLaunchKernelGGL((join_kernel<T, 1>), g, b, lds, st, a);
   AWQ_HIP_TRY(hipGetLastError());
   return AWQ_OK;

@@ -537,6 +537,35 @@ def test_the_end_of_a_sublayer(awq, lib, dev, f32, width):
 
 
 @pytest.mark.parametrize("f32", FORMATS, ids=["bf16", "f32"])
+@pytest.mark.parametrize("width, top", [(1020, 8), (1028, 9), (4096, 1), (4096, 8), (4100, 8)])
+def test_the_end_of_a_sublayer_at_the_bounds_of_its_forms(awq, lib, dev, f32, width, top):
+    """Rows and choices that registers hold and do not, without identity outputs; binary32 sums of top + 1 values: the
+    tolerance is that of the test above, whose values are of the same size."""
+    rng = np.random.default_rng(width + top)
+    for T in (1, 3, 512):
+        if T == 512 and width > 1028:
+            continue
+        x, y = rng.standard_normal((2, T, width)).astype(np.float32)
+        w1 = (1 + 0.3 * rng.standard_normal(width)).astype(np.float32)
+        pairs = rng.standard_normal((T, top, width)).astype(np.float32)
+        weights = rng.random((T, top)).astype(np.float32)
+        d = {n: dev.f(v) for n, v in dict(x=x, y=y, w1=w1, pairs=pairs.reshape(T * top, width), weights=weights).items()}
+        ids = dev.torch.zeros((T, top), dtype=dev.torch.int32).cuda()
+        h, _ = dev.act(np.full((T, up(width, 8)), np.nan), f32)   # not used
+        out = dev.empty((T, width), f32)
+        a = awq.AwqJoinArgs()
+        a.x, a.n_tokens, a.width, a.eps, a.y, a.w_post = d["x"].data_ptr(), T, width, 1e-3, d["y"].data_ptr(), d["w1"].data_ptr()
+        a.pairs, a.ids, a.weights, a.top, a.experts = d["pairs"].data_ptr(), ids.data_ptr(), d["weights"].data_ptr(), top, 4
+        a.h, a.ldh, a.w_next, a.out, a.ldo = h.data_ptr(), h.shape[1], d["w1"].data_ptr(), out.data_ptr(), width
+        awq.check(lib.awq_join(ctypes.byref(a), f32, dev.stream))
+        s = y + (weights[..., None].astype(np.float64) * pairs).sum(1)
+        want = x + plain.rms(s, 1e-3) * w1
+        assert np.abs(dev.host(d["x"]) - want).max() < 2e-5
+        want = plain.rms(want, 1e-3) * w1
+        assert np.all(np.abs(dev.host(out) - want) <= (3e-5 if f32 else 0.004 * np.abs(want) + 1e-3))
+
+
+@pytest.mark.parametrize("f32", FORMATS, ids=["bf16", "f32"])
 @pytest.mark.parametrize("n", [3, 64, 333, 12288])
 def test_polynorm(awq, lib, dev, f32, n):
     rng = np.random.default_rng(n)
