@@ -48,6 +48,7 @@ struct GemmParams {
   int32_t nr, n_tiles;  // rows split: 256-row blocks, tiles = row blocks x 128-token blocks (row block fastest)
   int32_t* sk_head;     // rows split with handed-over sums: status word at [0], "give up now" at [1], counters at [16 + workgroup]
   float* sk_part;       // and one tile of FP32 sums per workgroup
+  GemmNorm* norm;       // host: may be done by the launch that adds partial sums
 };
 
 // exact-erf GeLU (Inference.cu:274-277) for the many-token kernels, whose sums are not bit-identical
@@ -1208,6 +1209,72 @@ __global__ __launch_bounds__(256) void reduce_parts_kernel(GemmParams p) {
   with_epilogue(p, [&](auto E) { store_out<decltype(E)::value, true>(p, (int)(at / p.m), (int)(at % p.m), v); });
 }
 
+// The same for residual sums whose RMS norm the next launch wants: a workgroup per token, which holds the row.  Bound by the
+// trip of the partial sums through memory, so everything is requested at once: 40 tokens of 4,096 with k in four parts 4.8 us
+// (eight wavefronts; with four, two pieces one behind the other, no faster than the two launches of 5.0 and 4.6 before).
+constexpr int kNormRow = 8192;
+__global__ __launch_bounds__(512) void reduce_norm_kernel(GemmParams p, const half_t* __restrict__ gamma, half_t* __restrict__ out,
+                                                          float eps) {
+  __shared__ float wsum[8];
+  constexpr int kKeep = kNormRow / 4096;
+  const int tid = threadIdx.x, chunks = p.m >> 3;
+  const int64_t total = (int64_t)p.M * p.m, row = (int64_t)blockIdx.x * p.m;
+  half8_t held[kKeep], gv[kKeep];
+  float acc = 0.0f;
+#pragma unroll
+  for (int c = 0; c < kKeep; ++c) {
+    const int at = tid + c * 512;
+    if (at < chunks) {
+      const float* part = p.part + row + at * 8;
+      const half8_t r = *reinterpret_cast<const half8_t*>(p.res + row + at * 8);
+      gv[c] = reinterpret_cast<const half8_t*>(gamma)[at];
+      float4_t a[4], b[4];  // kz is 2 or 4
+#pragma unroll
+      for (int z = 0; z < 4; ++z)
+        if (z < p.kz) {
+          a[z] = *reinterpret_cast<const float4_t*>(part + z * total);
+          b[z] = *reinterpret_cast<const float4_t*>(part + z * total + 4);
+        }
+#pragma unroll
+      for (int z = 1; z < 4; ++z)
+        if (z < p.kz) a[0] += a[z], b[0] += b[z];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        held[c][e] = r[e] + (half_t)(e < 4 ? a[0][e & 3] : b[0][e & 3]);
+        acc = __builtin_fmaf((float)held[c][e], (float)held[c][e], acc);
+      }
+      *reinterpret_cast<half8_t*>(p.y + row + at * 8) = held[c];
+    }
+  }
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+  if ((tid & 63) == 0) wsum[tid >> 6] = acc;
+  __syncthreads();
+  float all = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) all += wsum[i];
+  const half_t sc = (half_t)awq_rsqrtf(all / (float)p.m + eps);
+  const half8_t sc8 = half8_t{sc, sc, sc, sc, sc, sc, sc, sc};
+#pragma unroll
+  for (int c = 0; c < kKeep; ++c) {
+    const int at = tid + c * 512;
+    if (at < chunks) *reinterpret_cast<half8_t*>(out + row + at * 8) = (held[c] * sc8) * gv[c];
+  }
+}
+
+// the sums of a product whose k was cut
+void launch_reduce(const GemmParams& p, hipStream_t st) {
+  const int64_t total = (int64_t)p.M * p.m;
+  const auto at16 = [](const void* a) { return ((uintptr_t)a & 15) == 0; };
+  if (p.norm && p.epilogue == EPI_RESIDUAL && p.m <= kNormRow && p.kz <= 4 && at16(p.part) && at16(p.res) && at16(p.y) &&
+      at16(p.norm->gamma) && at16(p.norm->out)) {
+    hipLaunchKernelGGL(reduce_norm_kernel, dim3((unsigned)p.M), dim3(512), 0, st, p, p.norm->gamma, p.norm->out, p.norm->eps);
+    p.norm->done = true;
+    return;
+  }
+  hipLaunchKernelGGL(reduce_parts_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, p);
+}
+
 // tokens per workgroup of the k-split shape: 32, 64 or 128
 // tokens per workgroup of the k-split shape, in units of 32: 32, 64 or 128 by the token count; fewer
 // when a matrix with few rows and short k would otherwise get under 128 workgroups (4096 x 4096 at
@@ -1252,10 +1319,7 @@ int launch_wide(const GemmParams& p, bool zint, int n_wgs, hipStream_t st) {
     }
   }
   hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, p);
-  if (KSPLIT && p.kz > 1) {
-    const int64_t total = (int64_t)p.M * p.m;
-    hipLaunchKernelGGL(reduce_parts_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, p);
-  }
+  if (KSPLIT && p.kz > 1) launch_reduce(p, st);
   return AWQ_OK;
 }
 
@@ -1355,10 +1419,7 @@ int launch_shared32(const GemmParams& p, bool zint, hipStream_t st) {
     }
   }
   hipLaunchKernelGGL(kern, dim3((unsigned)(p.m / 64), (unsigned)p.kz), dim3(512), lds, st, p);
-  if (p.kz > 1) {
-    const int64_t total = (int64_t)p.M * p.m;
-    hipLaunchKernelGGL(reduce_parts_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, p);
-  }
+  if (p.kz > 1) launch_reduce(p, st);
   return AWQ_OK;
 }
 
@@ -1427,7 +1488,7 @@ int64_t gemm_workspace_bytes(int64_t m, int64_t k, int64_t M) {
 
 int launch_gemm(const void* wq, const half_t* scale, const half_t* zp, int64_t m, int64_t k, const half_t* x,
                 half_t* y, int64_t M, int zp_integral, int epilogue, const half_t* res, void* workspace,
-                int64_t workspace_bytes, hipStream_t st) {
+                int64_t workspace_bytes, hipStream_t st, GemmNorm* norm) {
   AWQ_REQUIRE(epilogue == EPI_STORE || epilogue == EPI_GELU || (epilogue == EPI_RESIDUAL && res),
               "epilogue must be store, GeLU or residual (with res)");
   AWQ_REQUIRE(m > 0 && m % 128 == 0 && k > 0 && k % 128 == 0, "m and k must be positive multiples of 128");
@@ -1455,6 +1516,7 @@ int launch_gemm(const void* wq, const half_t* scale, const half_t* zp, int64_t m
   p.nr = p.n_tiles = 0;
   p.sk_head = nullptr;
   p.sk_part = nullptr;
+  p.norm = norm;
   if (shared32_kcut_takes(m, k, M) && workspace && kSkHeaderBytes + 4 * M * m * 4 <= workspace_bytes) {
     p.kz = 4;
     p.part = (float*)((char*)workspace + kSkHeaderBytes);

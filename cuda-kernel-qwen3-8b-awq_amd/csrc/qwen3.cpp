@@ -888,19 +888,21 @@ int ensure_prefill_buffers(Qwen3Engine* e) {
 }
 
 int gemm_of(Qwen3Engine* e, const DevLinear& t, const half_t* x, half_t* y, int64_t M, int epilogue = EPI_STORE,
-            const half_t* res = nullptr) {
+            const half_t* res = nullptr, GemmNorm* norm = nullptr) {
   return launch_gemm(t.stream_order, t.scale, t.zp, t.m, t.k, x, y, M, t.zp_integral, epilogue, res, e->pb.gemm_ws,
-                     kGemmWsBytes, e->stream);
+                     kGemmWsBytes, e->stream, norm);
 }
 
 // runOneLayer, Inference.cu:1029-1230, for M prompt positions pos0.. at once.
 // Layer 0 reads current_seq_len_ before the prompt loop updates it (:1118, :1331).
-int enqueue_layer_batch(Qwen3Engine* e, int l, int64_t pos0, int64_t M) {
+// *normed: b.norm already holds this layer's first norm; then the next layer's.
+int enqueue_layer_batch(Qwen3Engine* e, int l, int64_t pos0, int64_t M, bool* normed) {
   LayerDev& L = e->layers[l];
   hipStream_t st = e->stream;
   const int64_t H = e->cfg.hidden;
   auto& b = e->pb;
-  if (int rc = launch_rmsnorm_batch(b.hidden, L.gamma, b.norm, H, M, e->cfg.eps, st)) return rc;  // :1040
+  if (!*normed)
+    if (int rc = launch_rmsnorm_batch(b.hidden, L.gamma, b.norm, H, M, e->cfg.eps, st)) return rc;  // :1040
   if (int rc = gemm_of(e, L.wqkv, b.norm, b.qkv, M)) return rc;                                    // :1052
   // (with the fused launch on, the appended rows also go into its second copy of the caches)
   if (int rc = launch_rope_kv_append_batch(b.qkv, e->cos_t, e->sin_t, b.q, L.kcache, L.vcache, e->n_heads,
@@ -913,10 +915,16 @@ int enqueue_layer_batch(Qwen3Engine* e, int l, int64_t pos0, int64_t M) {
                                         st))
     return rc;  // :1110
   // :1128 Wo product, :1149 residual add in its epilogue
-  if (int rc = gemm_of(e, L.wo, b.ctx, b.hidden, M, EPI_RESIDUAL, b.hidden)) return rc;
-  if (int rc = launch_rmsnorm_batch(b.hidden, L.gamma, b.norm, H, M, e->cfg.eps, st)) return rc;  // :1163
+  GemmNorm norm{L.gamma, b.norm, e->cfg.eps, false};
+  if (int rc = gemm_of(e, L.wo, b.ctx, b.hidden, M, EPI_RESIDUAL, b.hidden, &norm)) return rc;
+  if (!norm.done)
+    if (int rc = launch_rmsnorm_batch(b.hidden, L.gamma, b.norm, H, M, e->cfg.eps, st)) return rc;  // :1163
   if (int rc = gemm_of(e, L.w1, b.norm, b.mid, M, EPI_GELU)) return rc;  // :1176, :1196
-  return gemm_of(e, L.w2, b.mid, b.hidden, M, EPI_RESIDUAL, b.hidden);   // :1201, :1221
+  const bool last = l + 1 == e->cfg.n_layers;
+  GemmNorm next{last ? nullptr : e->layers[l + 1].gamma, b.norm, e->cfg.eps, false};
+  const int rc = gemm_of(e, L.w2, b.mid, b.hidden, M, EPI_RESIDUAL, b.hidden, last ? nullptr : &next);  // :1201, :1221
+  *normed = next.done;
+  return rc;
 }
 
 }  // namespace
@@ -943,8 +951,9 @@ int Qwen3Engine::enqueue_prompt_pass(const int32_t* tokens, int64_t pos0, int64_
   if (int rc = launch_embed_batch(e->embed.packed, e->embed.scale, e->embed.zp, H, e->cfg.vocab, e->pb.tokens, M,
                                   e->pb.hidden, e->stream))
     return rc;
+  bool normed = false;
   for (int l = 0; l < e->cfg.n_layers; ++l)
-    if (int rc = enqueue_layer_batch(e, l, pos0, M)) return rc;
+    if (int rc = enqueue_layer_batch(e, l, pos0, M, &normed)) return rc;
   // the state the generation loop starts from (:1357): the last position's output
   AWQ_HIP_TRY(hipMemcpyAsync(e->hidden, e->pb.hidden + (M - 1) * H, (size_t)H * 2, hipMemcpyDeviceToDevice,
                              e->stream));

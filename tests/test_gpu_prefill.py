@@ -92,6 +92,25 @@ def test_small_model_batched_prompt_matches_sequential(awq, oracle, torch_gpu, s
     oracle.awqo_model_destroy(model)
 
 
+@pytest.mark.parametrize("hidden,inter", [(1024, 2048), (4096, 2048), (8192, 2048)])
+def test_sums_of_a_cut_product_normed_by_their_launch(awq, oracle, torch_gpu, hidden, inter):
+    """Rows of fewer pieces than threads, of one for each, and of the most that registers hold."""
+    cfg = awq.make_config(n_layers=2, hidden=hidden, inter=inter, vocab=1024, max_pos=64)
+    model = make_oracle_model(oracle, cfg)
+    eng = awq.QWen3AWQInfer.empty(cfg)
+    fill_pair(awq, oracle, cfg, 78, engine=eng, model=model, profile=awq.SYNTH_BALANCED)
+    for n in (5, 33):
+        prompt = np.random.default_rng(n).integers(0, cfg.vocab, n).tolist()
+        eng.reset()
+        eng.prefill(prompt)
+        want = as_f32(eng.read_hidden()).copy()
+        eng.reset()
+        eng.prefill(prompt, batched=True)
+        assert close(as_f32(eng.read_hidden()), want), n
+    eng.close()
+    oracle.awqo_model_destroy(model)
+
+
 def test_batched_prompt_in_pieces_equals_one_call(awq, oracle, torch_gpu):
     """Positions, attended lengths and cache rows must not depend on how the prompt is cut into
     calls.  The pieces are long enough (more than 32 tokens) for the same product kernel to serve
