@@ -14,8 +14,8 @@ __device__ __forceinline__ void decay_and_key(float g, bool keys, float k, float
 }
 
 // The recurrence token by token: a wavefront holds kCols columns of the state, lane l the rows l, l + 64, ... of each.
-// HEAD: one token, a workgroup per head; the head's norm and gate are formed behind the recurrence in the same launch.
-// Otherwise a workgroup takes 4 kCols columns.
+// Used for one token.  HEAD: a workgroup per head; the head's norm and gate are formed behind the recurrence in the same
+// launch.  Otherwise a workgroup takes 4 kCols columns.
 template <typename T, int DPL, bool HEAD, int kCols>
 __global__ __launch_bounds__(HEAD ? 1024 : 256) void gated_step_kernel(GatedStateArgs a) {
   extern __shared__ float row[];  // HEAD: [vdim]
@@ -99,6 +99,137 @@ __global__ __launch_bounds__(HEAD ? 1024 : 256) void gated_step_kernel(GatedStat
   }
 }
 
+// The same for several tokens: fewer than the chunked form takes, wider heads, linear attention with few tokens or a decay of
+// zero (HEAD: one decay per head).  A token's sums are those of a pass of its own, bit for bit.  Bound, token by token, by the
+// trip of a token's inputs through memory and by the exchanges that end its sums, so the inputs of G tokens are requested
+// together and left in LDS for the four wavefronts (a decay is formed once instead of four times), and sixteen sums are ended
+// at a time.  8 heads of 128, 9 tokens: decays per head 4.1 us, per channel 4.5 (a token after the other 11.7 to 17.4; the chunked
+// form 4.9 to 5.2, at 2 to 40 times the error); 15 tokens 4.2 and 4.6.  Two columns per wavefront: four took 4.9 and 5.3.
+template <int DPL>
+constexpr int few_tokens() { return DPL <= 4 ? 16 : 8; }  // 48 KB of LDS at most
+template <int DPL>
+constexpr int few_cols() { return DPL <= 4 ? 2 : 4; }
+
+// x of lane ^ 1, 2, 4 or 8
+template <int OFF>
+__device__ __forceinline__ float other_lane(float x) {
+  const int v = __float_as_int(x);
+  if constexpr (OFF == 4) return __int_as_float(__builtin_amdgcn_ds_swizzle(v, (4 << 10) | 31));
+  constexpr int kControl = OFF == 1 ? 0xb1 : OFF == 2 ? 0x4e : 0x128;  // quad_perm 1 0 3 2, quad_perm 2 3 0 1, row_ror:8
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, v, kControl, 0xf, 0xf, true));
+}
+
+// Sixteen sums over all lanes, number lane / 4 in x[0]: at each of the first four exchanges a lane hands over the half of its
+// sums that it does not end with.  Each is added up as by an exchange of it at every distance from 32 to 1, bit for bit.
+__device__ __forceinline__ void sixteen_sums(float (&x)[16], int lane) {
+  typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const u32x2_t p = __builtin_amdgcn_permlane32_swap(__float_as_uint(x[i]), __float_as_uint(x[i + 8]), false, false);
+    x[i] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const u32x2_t p = __builtin_amdgcn_permlane16_swap(__float_as_uint(x[i]), __float_as_uint(x[i + 4]), false, false);
+    x[i] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const float low = x[i], high = x[i + 2];
+    x[i] = (lane & 8 ? high : low) + other_lane<8>(lane & 8 ? low : high);
+  }
+  const float low = x[0], high = x[1];
+  x[0] = (lane & 4 ? high : low) + other_lane<4>(lane & 4 ? low : high);
+  x[0] += other_lane<2>(x[0]);
+  x[0] += other_lane<1>(x[0]);
+}
+
+template <typename T, int DPL, bool HEAD>
+__global__ __launch_bounds__(256) void gated_few_kernel(GatedStateArgs a) {
+  constexpr int kCols = few_cols<DPL>(), J = 16 / kCols;  // J tokens a step
+  constexpr int G = few_tokens<DPL>(), D = DPL * 64, N = G * DPL / 4;  // N pieces of 64 channels of a token per wavefront
+  __shared__ float qs[G * D], ks[G * D], ds[HEAD ? 1 : G * D];
+  const int head = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col0 = (blockIdx.y * 4 + wave) * kCols, nc = min(kCols, a.vdim - col0);
+  const T* const q = reinterpret_cast<const T*>(a.q) + (int64_t)head * a.dim;
+  const bool keys = HEAD || a.k != nullptr, fresh = a.pos.position() == 0;
+  const T* const k = keys ? reinterpret_cast<const T*>(a.k) + (int64_t)head * a.dim : q;
+  const T* const v = reinterpret_cast<const T*>(a.v) + (int64_t)head * a.vdim;
+  const float* const g = HEAD ? a.head_decay : a.g + (int64_t)head * a.dim;
+  const float of_head = HEAD ? a.head_decay[head] : 0.0f;
+  float* const o = a.o + (int64_t)head * a.vdim + col0;
+  const int64_t ldo = (int64_t)a.heads * a.vdim;
+  float* const state = a.state + ((int64_t)head * a.vdim + col0) * D;
+  float s[kCols][DPL];
+#pragma unroll
+  for (int c = 0; c < kCols; ++c)
+#pragma unroll
+    for (int i = 0; i < DPL; ++i) s[c][i] = fresh || c >= nc ? 0.0f : state[c * D + i * 64 + lane];
+  for (int64_t t0 = 0; t0 < a.M; t0 += G) {
+    const int n = (int)min((int64_t)G, a.M - t0);
+    T qr[N], kr[N], vr;
+    float gr[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {  // (behind the last token and channel: read again, not kept)
+      const int piece = i * 4 + wave, d = min(piece % DPL * 64 + lane, a.dim - 1);
+      const int64_t t = t0 + min(piece / DPL, n - 1);
+      qr[i] = q[t * a.ldp + d];
+      kr[i] = k[t * a.ldp + d];
+      if constexpr (!HEAD) gr[i] = g[t * a.ldg + d];
+    }
+    // lane kCols t + c: column c of token t
+    vr = v[(t0 + min(lane / kCols, n - 1)) * a.ldp + min(col0 + lane % kCols, a.vdim - 1)];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int piece = i * 4 + wave, at = piece * 64 + lane;
+      const bool there = piece % DPL * 64 + lane < a.dim;
+      float decay = 0.0f, key;
+      if constexpr (HEAD) key = (float)kr[i];
+      else decay_and_key(gr[i], keys, (float)kr[i], decay, key);
+      qs[at] = there ? (float)qr[i] * a.q_scale : 0.0f;
+      ks[at] = there ? key : 0.0f;
+      if constexpr (!HEAD) ds[at] = there ? decay : 0.0f;
+    }
+    __syncthreads();
+    const float value = lane % kCols < nc ? (float)vr : 0.0f;
+    for (int tj = 0; tj < n; tj += J) {
+      float qv[J][DPL], kv[J][DPL], dv[J][DPL], out[16];
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+#pragma unroll
+        for (int i = 0; i < DPL; ++i) {
+          const int at = (tj + j) * D + i * 64 + lane;
+          qv[j][i] = qs[at];
+          kv[j][i] = ks[at];
+          dv[j][i] = HEAD ? of_head : ds[at];
+        }
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+#pragma unroll
+        for (int c = 0; c < kCols; ++c) {
+          float& sum = out[j * kCols + c];
+          sum = 0.0f;
+          if (tj + j >= n) continue;
+          const float vv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(value), (tj + j) * kCols + c));
+#pragma unroll
+          for (int i = 0; i < DPL; ++i) {
+            s[c][i] = __builtin_fmaf(kv[j][i], vv, dv[j][i] * s[c][i]);
+            sum = __builtin_fmaf(s[c][i], qv[j][i], sum);
+          }
+        }
+      sixteen_sums(out, lane);
+      const int t = tj + (lane >> 2) / kCols, c = (lane >> 2) % kCols;
+      if ((lane & 3) == 0 && t < n && c < nc) o[(t0 + t) * ldo + c] = out[0];
+    }
+    if (t0 + G < a.M) __syncthreads();  // the group is read
+  }
+#pragma unroll
+  for (int c = 0; c < kCols; ++c)
+    if (c < nc)
+#pragma unroll
+      for (int i = 0; i < DPL; ++i) state[c * D + i * 64 + lane] = s[c][i];
+}
+
 // Many tokens on the binary32 matrix instruction (v_mfma_f32_16x16x4_f32), C tokens (a chunk) after the other in blocks
 // of 16.  Inside a block, with L_t the sum of the logarithms of the decays up to and with token t (a number per
 // channel), T that of all 16, S the state ahead of the block and
@@ -154,8 +285,8 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
   const T* const q = reinterpret_cast<const T*>(a.q) + (int64_t)head * a.dim;
   const T* const k = keys ? reinterpret_cast<const T*>(a.k) + (int64_t)head * a.dim : q;
   const T* const v = reinterpret_cast<const T*>(a.v) + (int64_t)head * a.vdim + c0;
-  const float* const g = HEAD ? a.head_decay : a.g + (int64_t)head * a.dim;
-  const float of_head = HEAD ? a.head_decay[head] : 0.0f;
+  const float* const g = HEAD ? a.head_log2 : a.g + (int64_t)head * a.dim;
+  const float of_head = HEAD ? a.head_log2[head] : 0.0f;
   if (tid < 3 * B) unsafe[tid / B][tid % B] = 0;
   __syncthreads();
 
@@ -369,7 +500,7 @@ int launch_chunks(const GatedStateArgs& a, hipStream_t st) {
   const uintptr_t parts = (uintptr_t)a.q | (uintptr_t)a.k;  // two values of T, two floats
   const bool even = a.dim % 2 == 0 && a.ldp % 2 == 0 && a.ldg % 2 == 0 && parts % (2 * sizeof(T)) == 0 && (uintptr_t)a.g % 8 == 0;
   if constexpr (sizeof(T) == 4)
-    if (a.head_decay) return even ? launch_chunk_form<T, D, true, true, true>(a, st) : launch_chunk_form<T, D, false, true, true>(a, st);
+    if (a.head_log2) return even ? launch_chunk_form<T, D, true, true, true>(a, st) : launch_chunk_form<T, D, false, true, true>(a, st);
   if (a.k) return even ? launch_chunk_form<T, D, true, true>(a, st) : launch_chunk_form<T, D, false, true>(a, st);
   return even ? launch_chunk_form<T, D, true, false>(a, st) : launch_chunk_form<T, D, false, false>(a, st);
 }
@@ -377,24 +508,20 @@ int launch_chunks(const GatedStateArgs& a, hipStream_t st) {
 template <typename T, int DPL>
 void launch_steps(const GatedStateArgs& a, hipStream_t st) {
   constexpr int kHeadCols = DPL <= 4 ? 8 : 4, kCols = 4;
+  const auto groups = [&](int cols) { return dim3((unsigned)a.heads, (unsigned)((a.vdim + 4 * cols - 1) / (4 * cols))); };
   if (a.ctx)
     hipLaunchKernelGGL((gated_step_kernel<T, DPL, true, kHeadCols>), dim3((unsigned)a.heads),
                        dim3((unsigned)std::min<int64_t>(1024, (a.vdim + kHeadCols - 1) / kHeadCols * 64)), (size_t)a.vdim * 4, st, a);
+  else if (a.head_decay)
+    hipLaunchKernelGGL((gated_few_kernel<T, DPL, true>), groups(few_cols<DPL>()), dim3(256), 0, st, a);
+  else if (a.M == 1)
+    hipLaunchKernelGGL((gated_step_kernel<T, DPL, false, kCols>), groups(kCols), dim3(256), 0, st, a);
   else
-    hipLaunchKernelGGL((gated_step_kernel<T, DPL, false, kCols>),
-                       dim3((unsigned)a.heads, (unsigned)((a.vdim + 4 * kCols - 1) / (4 * kCols))), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((gated_few_kernel<T, DPL, false>), groups(few_cols<DPL>()), dim3(256), 0, st, a);
 }
 
-// tokens from which on a chunk is the faster form: 8 or 32 heads of 128, 5.0 to 5.4 us from 2 tokens on, token by token 5.7 at
-// 2, 17.4 at 9 (binary32: 5.3, 15.4)
-constexpr int kChunkFrom = 2;
-
 template <typename T>
-int launch(const GatedStateArgs& a, hipStream_t st) {
-  if (a.M >= kChunkFrom && a.dim <= 256) {
-    if (a.dim <= 64) return launch_chunks<T, 64>(a, st);
-    return a.dim <= 128 ? launch_chunks<T, 128>(a, st) : launch_chunks<T, 256>(a, st);
-  }
+int launch_any_steps(const GatedStateArgs& a, hipStream_t st) {
   switch ((a.dim + 63) / 64) {
     case 1: launch_steps<T, 1>(a, st); break;
     case 2: launch_steps<T, 2>(a, st); break;
@@ -409,17 +536,27 @@ int launch(const GatedStateArgs& a, hipStream_t st) {
   return AWQ_OK;
 }
 
-}  // namespace
+// Tokens from which on a chunk is used, 5.0 us for one.  Its factors are exponentials of sums of logarithms, further off than the
+// decays themselves: without keys the state behind 9 tokens 1.2e-7, token by token 4.7e-8.
+constexpr int kChunkFrom = 16;
 
-int launch_linear_chunks_f32(const LinearAttnArgs& u, hipStream_t st) {
-  const float* p = reinterpret_cast<const float*>(u.proj);
+template <typename T>
+int launch(const GatedStateArgs& a, hipStream_t st) {
+  if (a.M < kChunkFrom || a.dim > 256) return launch_any_steps<T>(a, st);
+  if (a.dim <= 64) return launch_chunks<T, 64>(a, st);
+  return a.dim <= 128 ? launch_chunks<T, 128>(a, st) : launch_chunks<T, 256>(a, st);
+}
+
+// linear attention's arguments, but for the decay
+template <typename T>
+GatedStateArgs of_linear(const LinearAttnArgs& u) {
+  const T* p = reinterpret_cast<const T*>(u.proj);
   const int64_t keys = (int64_t)u.heads * u.dim;
   GatedStateArgs a;
   a.q = p;
   a.k = p + keys;
   a.v = p + 2 * keys;
   a.ldp = u.ldp;
-  a.head_decay = u.log2_decay;
   a.heads = u.heads;
   a.dim = u.dim;
   a.vdim = u.vdim;
@@ -427,6 +564,20 @@ int launch_linear_chunks_f32(const LinearAttnArgs& u, hipStream_t st) {
   a.o = u.o;
   a.M = u.M;
   a.pos = u.pos;
+  return a;
+}
+
+}  // namespace
+
+int launch_linear_few(const LinearAttnArgs& u, bool f32, hipStream_t st) {
+  GatedStateArgs a = f32 ? of_linear<float>(u) : of_linear<bf16_t>(u);
+  a.head_decay = u.decay;
+  return f32 ? launch_any_steps<float>(a, st) : launch_any_steps<bf16_t>(a, st);
+}
+
+int launch_linear_chunks_f32(const LinearAttnArgs& u, hipStream_t st) {
+  GatedStateArgs a = of_linear<float>(u);
+  a.head_log2 = u.log2_decay;
   if (a.dim <= 64) return launch_chunks<float, 64>(a, st);
   return a.dim <= 128 ? launch_chunks<float, 128>(a, st) : launch_chunks<float, 256>(a, st);
 }

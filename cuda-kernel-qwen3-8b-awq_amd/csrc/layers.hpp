@@ -213,7 +213,8 @@ struct LinearAttnArgs {
 };
 int64_t linear_state_floats(int32_t heads, int32_t dim, int32_t vdim);
 int launch_linear_attention(const LinearAttnArgs& a, bool f32, hipStream_t st);
-// its binary32 form for many tokens (gated_state.hip): dim <= 256, log2_decay set
+// its form for several tokens, token by token (gated_state.hip), and in binary32 for many: dim <= 256, log2_decay set
+int launch_linear_few(const LinearAttnArgs& a, bool f32, hipStream_t st);
 int launch_linear_chunks_f32(const LinearAttnArgs& a, hipStream_t st);
 
 // --- linear attention whose state decays per channel (gated_state.hip) -----------------------------------------
@@ -226,7 +227,8 @@ struct GatedStateArgs {
   // which then are the keys as well
   const float* g = nullptr;
   int64_t ldg = 0;
-  const float* head_decay = nullptr;  // [heads] binary logarithms, instead of g (launch_linear_chunks_f32)
+  // linear attention, [heads], instead of g: the decays (few tokens) or their binary logarithms (chunks)
+  const float *head_decay = nullptr, *head_log2 = nullptr;
   int32_t heads = 0, dim = 0, vdim = 0;
   float q_scale = 1.0f;
   float* state = nullptr;

@@ -4,7 +4,7 @@
 namespace {
 
 // The recurrence token by token: a wavefront holds kCols columns of the state, lane l the rows l, l + 64, ...
-// of each.  Used for few tokens and for decays of zero; the state never leaves the registers inside a pass.
+// of each.  Used for one token (launch_linear_few takes several the same way).
 constexpr int kCols = 4;
 
 template <typename T, int DPL>
@@ -360,9 +360,9 @@ int launch_chunks(const LinearAttnArgs& a, hipStream_t st) {
   return AWQ_OK;
 }
 
-// tokens from which on a chunk is the faster form: 8 or 32 heads of 128, 5.3 us from 2 tokens on (binary32: 5.0), token by token
-// 5.6 at 2, 16.7 at 9 (binary32: 4.6, 5.6 at 3, 11.6)
-constexpr int kChunkFrom = 2, kChunkFromF32 = 3;
+// Tokens from which on a chunk is used.  In bfloat16 its weights (k . q) decay^n are two terms of 8 bits: outputs 2.5e-6 off, by
+// the recurrence 6e-8 (3.5 to 4.2 us for 2 to 15 tokens, a chunk 5.2).
+constexpr int kChunkFrom = 16;
 
 template <typename T>
 int launch_step(const LinearAttnArgs& a, hipStream_t st) {
@@ -375,8 +375,7 @@ int launch_step(const LinearAttnArgs& a, hipStream_t st) {
     case 5: hipLaunchKernelGGL((linear_step_kernel<T, 5>), g, dim3(256), 0, st, a); break;
     case 6: hipLaunchKernelGGL((linear_step_kernel<T, 6>), g, dim3(256), 0, st, a); break;
     case 7: hipLaunchKernelGGL((linear_step_kernel<T, 7>), g, dim3(256), 0, st, a); break;
-    case 8: hipLaunchKernelGGL((linear_step_kernel<T, 8>), g, dim3(256), 0, st, a); break;
-    default: awq_set_error("launch_linear_attention: dim must be at most 512"); return AWQ_ERR_ARG;
+    default: hipLaunchKernelGGL((linear_step_kernel<T, 8>), g, dim3(256), 0, st, a); break;
   }
   AWQ_HIP_TRY(hipGetLastError());
   return AWQ_OK;
@@ -391,7 +390,9 @@ int launch_linear_attention(const LinearAttnArgs& a, bool f32, hipStream_t st) {
   AWQ_REQUIRE(a.heads >= 1 && a.dim >= 1 && a.vdim >= 1 && a.vdim <= 65536 && a.ldp % 8 == 0 &&
                   a.ldp >= (int64_t)a.heads * (2 * a.dim + a.vdim),
               "bad shape");
-  const bool chunks = a.log2_decay && a.M >= (f32 ? kChunkFromF32 : kChunkFrom) && a.M < (1 << 30) && a.dim <= 256;
+  AWQ_REQUIRE(a.dim <= 512, "dim must be at most 512");
+  const bool chunks = a.log2_decay && a.M >= kChunkFrom && a.M < (1 << 30) && a.dim <= 256;
+  if (a.M > 1 && !chunks) return launch_linear_few(a, f32, st);
   if (f32) return chunks ? launch_linear_chunks_f32(a, st) : launch_step<float>(a, st);
   if (chunks) {
     const bool whole = ((a.dim | a.vdim) & 7) == 0;

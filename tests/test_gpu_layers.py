@@ -291,6 +291,40 @@ def test_linear_attention(awq, lib, dev, f32, heads, dim, vdim):
             assert np.abs(s[h] - S[h]).max() <= 3e-5 * np.abs(S[h]).max(), (sizes, h)
 
 
+@pytest.mark.parametrize("f32", FORMATS, ids=["bf16", "f32"])
+@pytest.mark.parametrize("heads,dim,vdim", [(3, 9, 5), (4, 64, 40), (2, 130, 33), (1, 256, 72), (2, 300, 16), (1, 512, 17)])
+def test_several_tokens_of_linear_attention_are_those_of_single_ones(awq, lib, dev, f32, heads, dim, vdim):
+    """few tokens at a time, and any number where a decay of zero or a wide head leaves no chunks: the same bits.  A value that
+    is infinite reaches its own column from its own token on and nothing else"""
+    print("linear attention, several tokens", heads, dim, vdim, f32, flush=True)
+    rng = np.random.default_rng(dim)
+    T, at, n = 47, 20, heads * (2 * dim + vdim)
+    x = np.pad(rng.standard_normal((T, n)) * 0.5 + 0.2, ((0, 0), (0, -n % 8)))
+    x[at, 2 * heads * dim + 1] = np.inf
+    proj, _ = dev.act(x, f32)
+    decay = np.array([0.999, 0.3, 0.9, 1e-6][:heads], np.float32)
+    d_lg = dev.f(np.log2(decay.astype(np.float64)))
+
+    def run(sizes, decay, lg):
+        state, o = dev.empty((heads, vdim, (dim + 63) // 64 * 64), True), dev.empty((T, heads * vdim), True)
+        d_decay = dev.f(decay)
+        t = i = 0
+        while t < T:
+            m = min(sizes[i % len(sizes)], T - t)
+            awq.check(lib.awq_linear_attention(proj[t:].data_ptr(), proj.shape[1], heads, dim, vdim, d_decay.data_ptr(), lg, state.data_ptr(),
+                                               o[t:].data_ptr(), m, t, f32, dev.stream))
+            t, i = t + m, i + 1
+        return dev.host(o), dev.host(state)
+    for zero in (False, True):
+        d, lg = (np.where(decay < 0.1, 0, decay).astype(np.float32), None) if zero else (decay, d_lg.data_ptr())
+        want = run([1], d, lg)
+        column = np.arange(heads * vdim) == 1
+        assert np.isfinite(want[0][:at]).all() and np.isfinite(want[0][:, ~column]).all() and not np.isfinite(want[0][at:, 1]).any()
+        for sizes in ([2], [3, 1, 15], [15], [9, 4]) + (([40], [47]) if zero or dim > 256 else ()):
+            got = run(sizes, d, lg)
+            assert np.array_equal(got[0], want[0], equal_nan=True) and np.array_equal(got[1], want[1], equal_nan=True), sizes
+
+
 @pytest.mark.parametrize("heads,dim,vdim", [(3, 63, 5), (4, 64, 40), (2, 128, 16), (2, 130, 33), (1, 256, 72)])
 @pytest.mark.parametrize("sizes", [[16], [129, 1, 2], [130, 31], [15, 17, 300]], ids=str)
 def test_linear_attention_in_binary32_portions(awq, lib, dev, heads, dim, vdim, sizes):

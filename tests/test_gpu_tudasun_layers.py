@@ -309,6 +309,37 @@ def test_gated_state(awq, lib, dev, f32, keys, heads, dim, vdim):
 
 
 @pytest.mark.parametrize("f32", FORMATS, ids=["bf16", "f32"])
+@pytest.mark.parametrize("keys", [True, False], ids=["keys", "no keys"])
+@pytest.mark.parametrize("heads,dim,vdim", [(3, 9, 5), (4, 64, 40), (2, 130, 33), (2, 256, 72), (2, 300, 16), (1, 512, 17)])
+def test_several_tokens_of_a_state_are_those_of_single_ones(awq, lib, dev, f32, keys, heads, dim, vdim):
+    """few tokens at a time, and any number where a wide head leaves no chunks: the same bits.  An infinite value reaches its own
+    column from its own token on and nothing else"""
+    print("gated state, several tokens", heads, dim, vdim, f32, keys, flush=True)
+    rng = np.random.default_rng(dim)
+    T, at, hd = 47, 20, heads * dim
+    q, k, v, rate = state_inputs(rng, T, heads, dim, vdim, True)
+    v[at, 0, 1] = np.inf
+    x = np.concatenate([y.reshape(T, -1) for y in (q, k, v)], axis=1)
+    proj, _ = dev.act(np.pad(x, ((0, 0), (0, -x.shape[1] % 8))), f32)
+    d_g = dev.f((-rate if keys else 1.0 - 2.0 ** -rate).reshape(T, hd))
+
+    def run(sizes):
+        state, o = dev.empty((heads, vdim, up(dim, 64)), True), dev.empty((T, heads * vdim), True)
+        for t, m in portions(T, sizes):
+            base, unit = proj[t:].data_ptr(), proj.element_size()
+            a = awq.AwqGatedStateArgs(base, base + hd * unit if keys else None, base + 2 * hd * unit, d_g[t:].data_ptr(), proj.shape[1], hd,
+                                      heads, dim, vdim, 0.3, state.data_ptr(), o[t:].data_ptr(), m, t)
+            awq.check(lib.awq_gated_state(ctypes.byref(a), f32, dev.stream))
+        return dev.host(o), dev.host(state)
+    want = run([1])
+    column = np.arange(heads * vdim) == 1
+    assert np.isfinite(want[0][:at]).all() and np.isfinite(want[0][:, ~column]).all() and not np.isfinite(want[0][at:, 1]).any()
+    for sizes in ([2], [3, 1, 15], [15], [9, 4]) + (([40], [47]) if dim > 256 else ()):
+        got = run(sizes)
+        assert np.array_equal(got[0], want[0], equal_nan=True) and np.array_equal(got[1], want[1], equal_nan=True), sizes
+
+
+@pytest.mark.parametrize("f32", FORMATS, ids=["bf16", "f32"])
 def test_a_key_far_back_in_a_state(awq, lib, dev, f32):
     """one token writes a marked row, hundreds of tokens later a query reads just that row"""
     T, dim, vdim, far = 420, 64, 32, 37
