@@ -243,8 +243,12 @@ __global__ __launch_bounds__(256) void gated_few_kernel(GatedStateArgs a) {
 // Operands, lane (n, j) = (lane % 16, lane / 16), step i: an accumulator holds rows 4 j + i of column n, and used as an
 // operand it is just that for an order of the summed index of 4 j + i.
 //     A^T[s][t] = K Q^T,  O^T[c][t] = R^T Q^T + V^T (A^T, s <= t),  R[d][c] += K^T V
-// HEAD: one decay per head (linear attention in binary32); the logarithm stands in the place of every channel's.  333
-// tokens, 8 heads of 128: 30 us, token by token 395 (bound by a token's trip through a wavefront, 1.2 us each).
+// HEAD: one decay per head (linear attention in binary32).  Its powers are factors of whole sums then,
+//     o_t = decay^(t+1) S^T q_t + sum over s <= t of decay^(t-s) (q_t . k_s) v_s,
+//     S <- decay^n S + sum over s < n of k_s decay^(n-1-s) v_s    (n tokens in the block),
+// rounded once from 64 bits; the state's, which every block meets again, is a sum of two numbers.  333 tokens, 8 heads of 128:
+// 22 us, a token after the other 395; outputs 7.8e-8 off, by the recurrence 8.4e-8 (exponentials of the logarithm as factors
+// of q and k: 29 us, 1.8e-7).
 // Where a channel of a block decays by more than 2^-kSafe the factors could leave the range of binary32: such a block goes
 // token by token, in the same accumulators.
 constexpr int kBlock = 16;
@@ -285,8 +289,17 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
   const T* const q = reinterpret_cast<const T*>(a.q) + (int64_t)head * a.dim;
   const T* const k = keys ? reinterpret_cast<const T*>(a.k) + (int64_t)head * a.dim : q;
   const T* const v = reinterpret_cast<const T*>(a.v) + (int64_t)head * a.vdim + c0;
-  const float* const g = HEAD ? a.head_log2 : a.g + (int64_t)head * a.dim;
-  const float of_head = HEAD ? a.head_log2[head] : 0.0f;
+  const float* const g = HEAD ? a.head_decay : a.g + (int64_t)head * a.dim;
+  const float of_head = HEAD ? a.head_decay[head] : 0.0f;
+  __shared__ float power[HEAD ? kBlock + 1 : 1], power_rest[HEAD ? kBlock + 1 : 1];  // of the decay: their sum is the n-th
+  if constexpr (HEAD) {
+    if (tid <= kBlock) {
+      double x = 1.0;
+      for (int i = 0; i < tid; ++i) x *= (double)of_head;
+      power[tid] = (float)x;
+      power_rest[tid] = (float)(x - (double)(float)x);
+    }
+  }
   if (tid < 3 * B) unsafe[tid / B][tid % B] = 0;
   __syncthreads();
 
@@ -309,8 +322,7 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
 #pragma unroll
       for (int t = 0; t < kHalf; ++t) {
         const int64_t tok = min(at + t0 + t, M - 1);
-        if constexpr (HEAD) gr[t] = f32x2_t{of_head, of_head};
-        else gr[t] = two(g + tok * a.ldg + dc);
+        if constexpr (!HEAD) gr[t] = two(g + tok * a.ldg + dc);
         qr[t] = two(q + tok * a.ldp + dc);
         if constexpr (keys) kr[t] = two(k + tok * a.ldp + dc);
       }
@@ -319,6 +331,28 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
     };
     auto form = [&](int chunk) __attribute__((always_inline)) {
       const int at = chunk * C + t0, par = chunk & 1;
+      float* const qs = qs2 + (par * C + t0) * S4 + d;
+      float* const ks = ks2 + (par * C + t0) * S4 + d;
+      auto values = [&]() __attribute__((always_inline)) {  // (behind the last token and column: they meet keys of zero, or are not stored)
+#pragma unroll
+        for (int i = 0; i < B; ++i) vs2[(par * C + i * 16 + (p >> 4)) * VS + (p & 15)] = (float)vr[i];
+      };
+      if constexpr (HEAD) {
+#pragma unroll
+        for (int t = 0; t < kHalf; ++t) {
+          f32x2_t qv, kv;
+#pragma unroll
+          for (int e = 0; e < 2; ++e) {
+            const bool there = has[e] && at + t < M;
+            qv[e] = there ? (float)qr[t][e] * a.q_scale : 0.0f;
+            kv[e] = there ? (float)kr[t][e] : 0.0f;
+          }
+          *reinterpret_cast<f32x2_t*>(qs + t * S4) = qv;
+          *reinterpret_cast<f32x2_t*>(ks + t * S4) = kv;
+        }
+        values();
+        return;
+      }
       f32x2_t L[kHalf];
       float sum[2] = {0.0f, 0.0f};
 #pragma unroll
@@ -339,8 +373,6 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
         ahead[e] = half ? other : 0.0f;
       }
       if (half == 0 && fminf(mid[0], mid[1]) < -0.5f * kSafe) unsafe[chunk % 3][blk] = 1;
-      float* const qs = qs2 + (par * C + t0) * S4 + d;
-      float* const ks = ks2 + (par * C + t0) * S4 + d;
 #pragma unroll
       for (int t = 0; t < kHalf; ++t) {
         f32x2_t qv, kv;
@@ -357,9 +389,7 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
       if (half == 0)
         *reinterpret_cast<f32x2_t*>(ts2 + (par * B + blk) * D + d) =
             f32x2_t{__builtin_amdgcn_exp2f(mid[0]), __builtin_amdgcn_exp2f(mid[1])};
-#pragma unroll
-      for (int i = 0; i < B; ++i)  // (behind the last token and column: values that meet keys of zero, or are not stored)
-        vs2[(par * C + i * 16 + (p >> 4)) * VS + (p & 15)] = (float)vr[i];
+      values();
     };
     auto store = [&](int chunk) __attribute__((always_inline)) {
       if (p >= C * 4) return;
@@ -405,6 +435,15 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
     s[i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     if (!fresh && d < dimp && n < nv) s[i] = *reinterpret_cast<const f32x4_t*>(state + d);
   }
+  // HEAD: a power that is no number, or leaves the range where a product with it is as exact as others, is not used
+  const bool whole = !HEAD || (power[kBlock] > 0x1p-100f && power[kBlock] < 0x1p100f);
+  float state_power = 0.0f, state_power_rest = 0.0f, out_power = 0.0f, out_power_rest = 0.0f, back[4] = {}, to_end[4] = {};
+  if constexpr (HEAD) {
+    state_power = power[kBlock], state_power_rest = power_rest[kBlock];
+    out_power = power[n + 1], out_power_rest = power_rest[n + 1];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) back[i] = power[max(n - j4 - i, 0)], to_end[i] = power[kBlock - 1 - j4 - i];
+  }
   __syncthreads();
   for (int chunk = 0; chunk < chunks; ++chunk) {
     const int par = chunk & 1;
@@ -419,32 +458,78 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
       float vv[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) vv[i] = vs[(b * kBlock + j4 + i) * VS + n];
-      if (unsafe[chunk % 3][b] == 0) {
-        f32x4_t w = {0.0f, 0.0f, 0.0f, 0.0f}, f[NT];
+      if (unsafe[chunk % 3][b] == 0 && whole) {
+        if constexpr (HEAD) {
+          const int here = min(kBlock, M - chunk * C - b * kBlock);  // tokens of the block
+          if (here > 0) {
+            f32x4_t w[2 * NT], ot[2 * NT];  // an accumulator per 8 rows: the sums over rows are short chains, added in pairs
 #pragma unroll
-        for (int i = 0; i < NT; ++i) {
-          f[i] = *reinterpret_cast<const f32x4_t*>(ts + b * D + row0 + 16 * i + j4);
+            for (int i = 0; i < 2 * NT; ++i) w[i] = ot[i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-          for (int e = 0; e < 4; ++e) s[i][e] *= f[i][e];
-          const f32x4_t qv = *reinterpret_cast<const f32x4_t*>(qs + (b * kBlock + n) * S4 + row0 + 16 * i + j4);
-          const f32x4_t kv = *reinterpret_cast<const f32x4_t*>(ks + (b * kBlock + n) * S4 + row0 + 16 * i + j4);
+            for (int i = 0; i < NT; ++i) {
+              const f32x4_t qv = *reinterpret_cast<const f32x4_t*>(qs + (b * kBlock + n) * S4 + row0 + 16 * i + j4);
+              const f32x4_t kv = *reinterpret_cast<const f32x4_t*>(ks + (b * kBlock + n) * S4 + row0 + 16 * i + j4);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            w = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[e], qv[e], w, 0, 0, 0);
-            o = __builtin_amdgcn_mfma_f32_16x16x4f32(s[i][e], qv[e], o, 0, 0, 0);
+              for (int e = 0; e < 4; ++e) {
+                const int j = 2 * i + (e & 1);
+                w[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[e], qv[e], w[j], 0, 0, 0);
+                ot[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(s[i][e], qv[e], ot[j], 0, 0, 0);
+              }
+            }
+            float f = state_power, f_rest = state_power_rest, later[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) later[e] = to_end[e] * vv[e];
+            if (here < kBlock) {  // the last block
+              f = power[here];
+              f_rest = power_rest[here];
+#pragma unroll
+              for (int e = 0; e < 4; ++e) later[e] = j4 + e < here ? power[max(here - 1 - j4 - e, 0)] * vv[e] : 0.0f;
+            }
+#pragma unroll
+            for (int i = 0; i < NT; ++i) {
+#pragma unroll
+              for (int e = 0; e < 4; ++e) s[i][e] = __builtin_fmaf(s[i][e], f, s[i][e] * f_rest);
+#pragma unroll
+              for (int e = 0; e < 4; ++e)
+                s[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(ks[(b * kBlock + j4 + e) * S4 + row0 + 16 * i + n], later[e], s[i], 0, 0, 0);
+            }
+#pragma unroll
+            for (int half = NT; half > 0; half >>= 1)
+#pragma unroll
+              for (int i = 0; i < half; ++i) w[i] = w[i] + w[i + half], ot[i] = ot[i] + ot[i + half];
+            // w[0][i]: key token j4 + i, query token n
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[i] = __builtin_fmaf(ot[0][i], out_power, ot[0][i] * out_power_rest);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[i], j4 + i <= n ? w[0][i] * back[i] : 0.0f, o, 0, 0, 0);
           }
+        } else {
+          f32x4_t w = {0.0f, 0.0f, 0.0f, 0.0f}, f[NT];
+#pragma unroll
+          for (int i = 0; i < NT; ++i) {
+            f[i] = *reinterpret_cast<const f32x4_t*>(ts + b * D + row0 + 16 * i + j4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[i][e] *= f[i][e];
+            const f32x4_t qv = *reinterpret_cast<const f32x4_t*>(qs + (b * kBlock + n) * S4 + row0 + 16 * i + j4);
+            const f32x4_t kv = *reinterpret_cast<const f32x4_t*>(ks + (b * kBlock + n) * S4 + row0 + 16 * i + j4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              w = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[e], qv[e], w, 0, 0, 0);
+              o = __builtin_amdgcn_mfma_f32_16x16x4f32(s[i][e], qv[e], o, 0, 0, 0);
+            }
+          }
+#pragma unroll
+          for (int i = 0; i < NT; ++i) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              s[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(ks[(b * kBlock + j4 + e) * S4 + row0 + 16 * i + n], vv[e], s[i], 0, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[i][e] *= f[i][e];
+          }
+          // w[i]: key token j4 + i, query token n
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[i], j4 + i <= n ? w[i] : 0.0f, o, 0, 0, 0);
         }
-#pragma unroll
-        for (int i = 0; i < NT; ++i) {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            s[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(ks[(b * kBlock + j4 + e) * S4 + row0 + 16 * i + n], vv[e], s[i], 0, 0, 0);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) s[i][e] *= f[i][e];
-        }
-        // w[i]: key token j4 + i, query token n
-#pragma unroll
-        for (int i = 0; i < 4; ++i) o = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[i], j4 + i <= n ? w[i] : 0.0f, o, 0, 0, 0);
       } else {
         for (int t = 0; t < kBlock && chunk * C + b * kBlock + t < M; ++t) {
           const int64_t tok = chunk * C + b * kBlock + t;
@@ -456,8 +541,9 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
             for (int e = 0; e < 4; ++e) {
               const int r = row0 + 16 * i + j4 + e;
               if (r >= a.dim) continue;
-              float decay, key;
-              decay_and_key(HEAD ? of_head : g[tok * a.ldg + r], keys, keys ? (float)k[tok * a.ldp + r] : 0.0f, decay, key);
+              float decay = of_head, key;
+              if constexpr (HEAD) key = (float)k[tok * a.ldp + r];
+              else decay_and_key(g[tok * a.ldg + r], keys, keys ? (float)k[tok * a.ldp + r] : 0.0f, decay, key);
               s[i][e] = __builtin_fmaf(key, value, decay * s[i][e]);
               out = __builtin_fmaf(s[i][e], (float)q[tok * a.ldp + r] * a.q_scale, out);
             }
@@ -500,7 +586,7 @@ int launch_chunks(const GatedStateArgs& a, hipStream_t st) {
   const uintptr_t parts = (uintptr_t)a.q | (uintptr_t)a.k;  // two values of T, two floats
   const bool even = a.dim % 2 == 0 && a.ldp % 2 == 0 && a.ldg % 2 == 0 && parts % (2 * sizeof(T)) == 0 && (uintptr_t)a.g % 8 == 0;
   if constexpr (sizeof(T) == 4)
-    if (a.head_log2) return even ? launch_chunk_form<T, D, true, true, true>(a, st) : launch_chunk_form<T, D, false, true, true>(a, st);
+    if (a.head_decay) return even ? launch_chunk_form<T, D, true, true, true>(a, st) : launch_chunk_form<T, D, false, true, true>(a, st);
   if (a.k) return even ? launch_chunk_form<T, D, true, true>(a, st) : launch_chunk_form<T, D, false, true>(a, st);
   return even ? launch_chunk_form<T, D, true, false>(a, st) : launch_chunk_form<T, D, false, false>(a, st);
 }
@@ -577,7 +663,7 @@ int launch_linear_few(const LinearAttnArgs& u, bool f32, hipStream_t st) {
 
 int launch_linear_chunks_f32(const LinearAttnArgs& u, hipStream_t st) {
   GatedStateArgs a = of_linear<float>(u);
-  a.head_log2 = u.log2_decay;
+  a.head_decay = u.decay;
   if (a.dim <= 64) return launch_chunks<float, 64>(a, st);
   return a.dim <= 128 ? launch_chunks<float, 128>(a, st) : launch_chunks<float, 256>(a, st);
 }

@@ -227,8 +227,7 @@ struct GatedStateArgs {
   // which then are the keys as well
   const float* g = nullptr;
   int64_t ldg = 0;
-  // linear attention, [heads], instead of g: the decays (few tokens) or their binary logarithms (chunks)
-  const float *head_decay = nullptr, *head_log2 = nullptr;
+  const float* head_decay = nullptr;  // linear attention, [heads], instead of g: the decays
   int32_t heads = 0, dim = 0, vdim = 0;
   float q_scale = 1.0f;
   float* state = nullptr;

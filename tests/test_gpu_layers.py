@@ -352,6 +352,33 @@ def test_linear_attention_in_binary32_portions(awq, lib, dev, heads, dim, vdim, 
         assert np.abs(s[h] - S[h]).max() <= 3e-5 * np.abs(S[h]).max()
 
 
+@pytest.mark.parametrize("heads,dim,vdim", [(8, 128, 128), (8, 64, 40), (8, 256, 72)])
+@pytest.mark.parametrize("f32,T,sizes", [(0, 60, [15]), (0, 60, [2]), (0, 60, [9, 1]), (1, 60, [15]), (1, 333, [333]), (1, 333, [40, 1])], ids=str)
+def test_roundings_of_linear_attention(awq, lib, dev, f32, T, sizes, heads, dim, vdim):
+    """Every form that carries binary32 is as close to 64 bits as the recurrence in binary32.  An output rounds its last sum, the
+    products it adds and the state's decay by 2^-25 each in the mean, and a state that remembers n tokens has been rounded n
+    times, the older ones decayed: 4 x 2^-25 for an output, sqrt(n) x 2^-25 for a state, n = 256 at most here."""
+    rng = np.random.default_rng(dim + T)
+    n = heads * (2 * dim + vdim)
+    proj, pv = dev.act(plain.silu(rng.standard_normal((T, n))), f32)
+    q, k = (pv[:, i * heads * dim:(i + 1) * heads * dim].reshape(T, heads, dim) for i in (0, 1))
+    v = pv[:, 2 * heads * dim:n].reshape(T, heads, vdim)
+    decay = (1.0 - 2.0 ** (-1.0 - 7.0 * np.arange(heads) / heads)).astype(np.float32)
+    want, S = plain.linear_attention(q, k, v, decay.astype(np.float64))
+    d_decay, d_lg = dev.f(decay), dev.f(np.log2(decay.astype(np.float64)))
+    state, o, at, i = dev.empty((heads, vdim, (dim + 63) // 64 * 64), True), dev.empty((T, heads * vdim), True), 0, 0
+    while at < T:
+        m = min(sizes[i % len(sizes)], T - at)
+        awq.check(lib.awq_linear_attention(proj[at:].data_ptr(), n, heads, dim, vdim, d_decay.data_ptr(), d_lg.data_ptr(), state.data_ptr(),
+                                           o[at:].data_ptr(), m, at, f32, dev.stream))
+        at, i = at + m, i + 1
+    got, s = dev.host(o).reshape(T, heads, vdim), dev.host(state)[:, :, :dim].transpose(0, 2, 1)
+    off = lambda x, y: np.linalg.norm(x - y) / np.linalg.norm(y)
+    worst = max(off(got[:, h], want[:, h]) for h in range(heads)), max(off(s[h], S[h]) for h in range(heads))
+    print("roundings", dim, f32, T, sizes, "%.1e %.1e" % worst, flush=True)
+    assert worst[0] < 4 * 2.0 ** -25 and worst[1] < min(T, 256) ** 0.5 * 2.0 ** -25
+
+
 def attend(awq, lib, dev, f32, proj, heads, kv, dim, vdim, window, scale, eps, temp, sizes, T, slots, max_pos):
     """the attention of T tokens in portions; proj: the tensor with all tokens' projections (kept as it is)"""
     kr, vr = lib.awq_window_row(dim), lib.awq_window_row(vdim)
