@@ -247,10 +247,11 @@ __global__ __launch_bounds__(256) void gated_few_kernel(GatedStateArgs a) {
 //     o_t = decay^(t+1) S^T q_t + sum over s <= t of decay^(t-s) (q_t . k_s) v_s,
 //     S <- decay^n S + sum over s < n of k_s decay^(n-1-s) v_s    (n tokens in the block),
 // rounded once from 64 bits; the state's, which every block meets again, is a sum of two numbers.  333 tokens, 8 heads of 128:
-// 22 us, a token after the other 395; outputs 7.8e-8 off, by the recurrence 8.4e-8 (exponentials of the logarithm as factors
+// 23 us, a token after the other 395; outputs 7.8e-8 off, by the recurrence 8.4e-8 (exponentials of the logarithm as factors
 // of q and k: 29 us, 1.8e-7).
 // Where a channel of a block decays by more than 2^-kSafe the factors could leave the range of binary32: such a block goes
-// token by token, in the same accumulators.
+// token by token, in the same accumulators.  So does a block with a value that is infinite or NaN, which the weights of zero
+// that stand for s > t would bring to the tokens ahead of it.
 constexpr int kBlock = 16;
 constexpr float kSafe = 200.0f;
 constexpr int kValueStride = 20;
@@ -335,7 +336,11 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
       float* const ks = ks2 + (par * C + t0) * S4 + d;
       auto values = [&]() __attribute__((always_inline)) {  // (behind the last token and column: they meet keys of zero, or are not stored)
 #pragma unroll
-        for (int i = 0; i < B; ++i) vs2[(par * C + i * 16 + (p >> 4)) * VS + (p & 15)] = (float)vr[i];
+        for (int i = 0; i < B; ++i) {
+          const float x = (float)vr[i];
+          vs2[(par * C + i * 16 + (p >> 4)) * VS + (p & 15)] = x;
+          if (!(fabsf(x) < INFINITY)) unsafe[chunk % 3][i] = 1;
+        }
       };
       if constexpr (HEAD) {
 #pragma unroll
@@ -435,8 +440,16 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
     s[i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     if (!fresh && d < dimp && n < nv) s[i] = *reinterpret_cast<const f32x4_t*>(state + d);
   }
-  // HEAD: a power that is no number, or leaves the range where a product with it is as exact as others, is not used
-  const bool whole = !HEAD || (power[kBlock] > 0x1p-100f && power[kBlock] < 0x1p100f);
+  // HEAD: a power that is no number, or leaves the range where a product with it is as exact as others, is not used; nor is any
+  // for a state that is not finite (the power's second number may be 0)
+  bool whole = !HEAD || (power[kBlock] > 0x1p-100f && power[kBlock] < 0x1p100f);
+  if constexpr (HEAD) {
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) whole = whole && fabsf(s[i][e]) < INFINITY;
+    whole = __all(whole);
+  }
   float state_power = 0.0f, state_power_rest = 0.0f, out_power = 0.0f, out_power_rest = 0.0f, back[4] = {}, to_end[4] = {};
   if constexpr (HEAD) {
     state_power = power[kBlock], state_power_rest = power_rest[kBlock];
@@ -531,6 +544,7 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
           for (int i = 0; i < 4; ++i) o = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[i], j4 + i <= n ? w[i] : 0.0f, o, 0, 0, 0);
         }
       } else {
+        if constexpr (HEAD) whole = false;
         for (int t = 0; t < kBlock && chunk * C + b * kBlock + t < M; ++t) {
           const int64_t tok = chunk * C + b * kBlock + t;
           const float value = vs[(b * kBlock + t) * VS + n];

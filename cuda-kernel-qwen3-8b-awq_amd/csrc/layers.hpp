@@ -199,7 +199,8 @@ int launch_window_attention(const WindowAttnArgs& a, bool f32, hipStream_t st);
 
 // --- linear attention with a decaying state (linear_attention.hip) -------------------------------------------
 // per head S <- decay S + k v^T, o = S^T q; state [heads][vdim][round_up(dim, 64)] float (S transposed), zero ahead of
-// position 0
+// position 0.  A value that is infinite or NaN leaves the tokens ahead of its own as they are, but for bfloat16 passes of 16
+// tokens on (dim up to 256), where it reaches its column of the 128 tokens that are formed together.
 struct LinearAttnArgs {
   const void* proj = nullptr;  // [M][ldp]: heads * dim of q, heads * dim of k, heads * vdim of v
   int64_t ldp = 0;

@@ -323,6 +323,13 @@ def test_several_tokens_of_linear_attention_are_those_of_single_ones(awq, lib, d
         for sizes in ([2], [3, 1, 15], [15], [9, 4]) + (([40], [47]) if zero or dim > 256 else ()):
             got = run(sizes, d, lg)
             assert np.array_equal(got[0], want[0], equal_nan=True) and np.array_equal(got[1], want[1], equal_nan=True), sizes
+        if f32 and not zero:  # the chunks: inside a block, behind it, in the next pass
+            for sizes in ([47], [16, 31], [30, 1]):
+                got = run(sizes, d, lg)
+                for x, y in ((got[0], want[0]), (got[1][:, :, :dim], want[1][:, :, :dim])):
+                    fine = np.isfinite(y)
+                    assert np.array_equal(np.isfinite(x), fine), sizes
+                    assert np.abs(x[fine] - y[fine]).max() < 1e-5 * np.abs(y[fine]).max(), sizes
 
 
 @pytest.mark.parametrize("heads,dim,vdim", [(3, 63, 5), (4, 64, 40), (2, 128, 16), (2, 130, 33), (1, 256, 72)])

@@ -337,6 +337,12 @@ def test_several_tokens_of_a_state_are_those_of_single_ones(awq, lib, dev, f32, 
     for sizes in ([2], [3, 1, 15], [15], [9, 4]) + (([40], [47]) if dim > 256 else ()):
         got = run(sizes)
         assert np.array_equal(got[0], want[0], equal_nan=True) and np.array_equal(got[1], want[1], equal_nan=True), sizes
+    for sizes in ([47], [16, 31], [30, 1]):  # the chunks: inside a block, behind it, in the next pass
+        got = run(sizes)
+        for x, y in ((got[0], want[0]), (got[1][:, :, :dim], want[1][:, :, :dim])):
+            fine = np.isfinite(y)
+            assert np.array_equal(np.isfinite(x), fine), sizes
+            assert np.abs(x[fine] - y[fine]).max() < 2e-5 * np.abs(y[fine]).max(), sizes
 
 
 @pytest.mark.parametrize("f32", FORMATS, ids=["bf16", "f32"])
