@@ -153,7 +153,7 @@ __global__ __launch_bounds__(256) void latent_query_kernel(LatentAttnArgs a, int
   const int row = a.l.row(), rank = a.l.rank, M = (int)a.M;
   const int h = blockIdx.x, t0 = blockIdx.y * QN, tid = threadIdx.x;
   const int pos0 = a.pos.position();
-  int pos[QN];
+  int first[QN] = {}, pos[QN];
   float m[QN], l[QN];
 #pragma unroll
   for (int i = 0; i < QN; ++i) {
@@ -167,8 +167,7 @@ __global__ __launch_bounds__(256) void latent_query_kernel(LatentAttnArgs a, int
   const T* const cache = reinterpret_cast<const T*>(a.cache);
   const auto key_row = [&](int key) { return cache + (int64_t)key * row; };
   attend_queries<T, QN>(
-      lds, row, rank, 0, pos[QN - 1], key_row, key_row,
-      [&](int i, int key, float dot) { return key <= pos[i] ? dot * a.scale : -INFINITY; }, m, l,
+      lds, row, rank, first, pos, key_row, key_row, [&](int i, int key, float dot) { return dot * a.scale; }, m, l,
       [&](int i, int col, q4_t sum, float total) {
         if (t0 + i >= M) return;
         T* const out = reinterpret_cast<T*>(a.ol) + ((int64_t)(t0 + i) * a.heads + h) * kv_in + col;

@@ -194,7 +194,8 @@ struct WindowAttnArgs {
 };
 int32_t window_row_padded(int32_t dim);
 int64_t window_parts_floats(int32_t heads, int32_t vdim, int64_t window, int64_t max_pos);
-// normalise q and k, append k and v, attend
+// Normalise q and k, append k and v, attend.  A value that is infinite or NaN leaves the positions that do not see it as they are;
+// not so in bfloat16 tiles of 64 queries (heads of up to 256), where a value meets queries of its tile with weight zero.
 int launch_window_attention(const WindowAttnArgs& a, bool f32, hipStream_t st);
 
 // --- linear attention with a decaying state (linear_attention.hip) -------------------------------------------

@@ -14,18 +14,19 @@ struct Four {
 
 inline size_t query_lds(int row, int queries) { return sizeof(float) * (size_t)(queries * (row + 256 + 4 + 1024)); }
 
-// A workgroup of 256 threads takes QN queries next to each other, `q` [QN][row] in LDS, and the keys first .. last in blocks of
-// 256 with a running maximum.  Scores: sixteen lanes per key, four values each, so that a row is read in whole lines and
+// A workgroup of 256 threads takes QN queries next to each other, `q` [QN][row] in LDS, query i the keys lo[i] .. hi[i] (both
+// ascending in i), in blocks of 256 with a running maximum.  Scores: sixteen lanes per key, four values each, so that a row is read in whole lines and
 // by all queries at once; softmax: a thread per key; values: a thread per four columns and share of the block's keys.
-// key_row(key), value_row(key): rows (row and cols values, row a multiple of 4); score(i, key, dot): query i's score, -infinity
-// for a key that it does not see (it sees one of the first block).  m, l: where a query's maximum and sum start; they
-// and the columns come out through store(i, column, four sums, l), for columns below `cols`.
+// key_row(key), value_row(key): rows (row and cols values, row a multiple of 4); score(i, key, dot): query i's score of a key that
+// it sees (one of the first block among them).  m, l: where a query's maximum and sum start; they and the columns come out
+// through store(i, column, four sums, l), for columns below `cols`.  A row that a query does not see is not in its
+// sums, whatever the row holds.
 // Bound by the reads out of the L2 and, for few queries, by the trips to it.  8 heads of 128, 333 queries, binary32: 39 us (one query of
-// 8 heads against 60 latents of 576: 9.8); 108 (19) with a
-// thread per key and query that read its row value by value.
+// 8 heads against 60 latents of 576: 9.8); 108 (19) with a thread per key and query that read its row value by value.
+// (The few keys that only some of the queries see have loops of their own: 0.2 us.)
 template <typename T, int QN, typename K, typename V, typename S, typename O>
-__device__ __forceinline__ void attend_queries(float* lds, int row, int cols, int first, int last, K key_row, V value_row, S score,
-                                               float (&m)[QN], float (&l)[QN], O store) {
+__device__ __forceinline__ void attend_queries(float* lds, int row, int cols, const int (&lo)[QN], const int (&hi)[QN], K key_row,
+                                               V value_row, S score, float (&m)[QN], float (&l)[QN], O store) {
   typedef typename Four<T>::type four_t;
   float* const q = lds;               // [QN][row]
   float* const p = q + QN * row;      // [QN][256]
@@ -37,8 +38,8 @@ __device__ __forceinline__ void attend_queries(float* lds, int row, int cols, in
 #pragma unroll
   for (int i = 0; i < QN; ++i) acc[i] = q4_t{0.0f, 0.0f, 0.0f, 0.0f};
   __syncthreads();  // q is written
-  for (int k0 = first; k0 <= last; k0 += 256) {
-    const int n = min(256, last + 1 - k0);
+  for (int k0 = lo[0]; k0 <= hi[QN - 1]; k0 += 256) {
+    const int n = min(256, hi[QN - 1] + 1 - k0);
     for (int j0 = 0; j0 < n; j0 += 64) {  // four keys of a group at a time: j0 + 16 u + group
       float dot[4][QN] = {};
       const T* rows[4];
@@ -72,7 +73,8 @@ __device__ __forceinline__ void attend_queries(float* lds, int row, int cols, in
     float alpha[QN];
 #pragma unroll
     for (int i = 0; i < QN; ++i) {
-      const float s = tid < n ? score(i, k0 + tid, p[i * 256 + tid]) : -INFINITY;
+      const int key = k0 + tid;
+      const float s = key >= lo[i] && key <= hi[i] ? score(i, key, p[i * 256 + tid]) : -INFINITY;
       float mx = s;
 #pragma unroll
       for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
@@ -103,8 +105,7 @@ __device__ __forceinline__ void attend_queries(float* lds, int row, int cols, in
       acc[i] = acc[i] * alpha[i];
     }
     if (share < shares) {
-#pragma unroll 4
-      for (int j = share; j < n; j += shares) {
+      auto add = [&](int j, bool all) __attribute__((always_inline)) {
         const T* const at = value_row(k0 + j) + 4 * quad;
         float v[4];
         if (4 * quad + 3 < cols) {
@@ -117,11 +118,21 @@ __device__ __forceinline__ void attend_queries(float* lds, int row, int cols, in
         }
 #pragma unroll
         for (int i = 0; i < QN; ++i) {
+          if (!all && (k0 + j < lo[i] || k0 + j > hi[i])) continue;
           const float w = p[i * 256 + j];
 #pragma unroll
           for (int e = 0; e < 4; ++e) acc[i][e] = __builtin_fmaf(w, v[e], acc[i][e]);
         }
-      }
+      };
+      // the keys ahead of the last query's first and behind the first query's last are not seen by all
+      const int from = min(lo[QN - 1] - k0, n), to = min(hi[0] + 1 - k0, n);
+      int j = share;
+      if constexpr (QN > 1)
+        for (; j < from; j += shares) add(j, false);
+#pragma unroll 4
+      for (; j < (QN > 1 ? to : n); j += shares) add(j, true);
+      if constexpr (QN > 1)
+        for (; j < n; j += shares) add(j, false);
     }
     __syncthreads();  // the block's weights are read
   }

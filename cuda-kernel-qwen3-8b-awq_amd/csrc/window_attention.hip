@@ -99,9 +99,9 @@ __global__ __launch_bounds__(256) void window_query_kernel(WindowAttnArgs a) {
   const T* const kc = reinterpret_cast<const T*>(a.k_cache);
   const T* const vc = reinterpret_cast<const T*>(a.v_cache);
   attend_queries<T, QN>(
-      lds, row, a.vdim, lo[0], pos[QN - 1], [&](int key) { return kc + ring_row(a.kl, g, key % a.kl.slots); },
+      lds, row, a.vdim, lo, pos, [&](int key) { return kc + ring_row(a.kl, g, key % a.kl.slots); },
       [&](int key) { return vc + ring_row(a.vl, g, key % a.vl.slots); },
-      [&](int i, int key, float dot) { return key >= lo[i] && key <= pos[i] ? dot * mul[i] - slope * (float)(pos[i] - key) : -INFINITY; }, m, l,
+      [&](int i, int key, float dot) { return dot * mul[i] - slope * (float)(pos[i] - key); }, m, l,
       [&](int i, int col, q4_t sum, float total) {
         if (t0 + i >= M) return;
         T* const out = reinterpret_cast<T*>(a.ctx) + (int64_t)(t0 + i) * a.ldc + (int64_t)h * a.vdim + col;

@@ -434,6 +434,28 @@ def test_window_attention(awq, lib, dev, f32, shape, window):
         assert km.rms_error(got, want) < (3e-5 if f32 else 0.01), sizes
 
 
+@pytest.mark.parametrize("f32,shape", [(1, (4, 2, 64, 64)), (1, (6, 1, 20, 12)), (1, (2, 1, 300, 72)), (0, (2, 1, 300, 72))], ids=str)
+@pytest.mark.parametrize("window", [0, 1, 2, 5, 250])
+def test_values_that_a_query_does_not_see(awq, lib, dev, f32, shape, window):
+    """several queries share a reading of the rows; a row that some of them do not see may hold anything"""
+    heads, kv, dim, vdim = shape
+    print("rows not seen", shape, window, f32, flush=True)
+    rng = np.random.default_rng(window)
+    T, n = 300, heads * dim + kv * (dim + vdim)
+    x = np.pad(rng.standard_normal((T, n)), ((0, 0), (0, -n % 8)))
+    args = lambda p, sizes: attend(awq, lib, dev, f32, dev.act(p, f32)[0], heads, kv, dim, vdim, window, dim ** -0.5, 1e-6, (0.0, 1.0), sizes,
+                                   T, ((window or T) - 1 + max(sizes) + 63) // 64 * 64, T)
+    for sizes in ([T], [64, 7, 4]):
+        want = args(x, sizes)
+        assert np.isfinite(want).all()
+        for at in (0, 5, 130, 256, 258):
+            y = x.copy()
+            y[at, (heads + kv) * dim:n] = np.nan if at & 1 else np.inf
+            got = args(y, sizes)
+            sees = (np.arange(T) >= at) & (np.arange(T) < (at + window if window else T))
+            assert np.array_equal(got[~sees], want[~sees]) and not np.isfinite(got[sees]).any(), (at, sizes)
+
+
 @pytest.mark.parametrize("f32", FORMATS, ids=["bf16", "f32"])
 @pytest.mark.parametrize("window", [1, 2, 31, 32, 33, 64, 65, 96, 128, 160])
 def test_window_edges(awq, lib, dev, f32, window):

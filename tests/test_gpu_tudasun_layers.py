@@ -492,6 +492,26 @@ def test_latent_attention(awq, lib, dev, f32, shape):
         assert km.rms_error(got, want) < (3e-5 if f32 else 0.03), sizes
 
 
+@pytest.mark.parametrize("shape", [(3, 20, 6, 12, 37), (2, 64, 32, 64, 128)], ids=str)
+def test_latents_that_a_query_does_not_see(awq, lib, dev, shape):
+    """several queries share a reading of the rows in binary32; the rows behind a query's own may hold anything"""
+    heads, dim, rot, vdim, rank = shape
+    print("latents not seen", shape, flush=True)
+    rng = np.random.default_rng(rank)
+    T = 300
+    q, down = rng.standard_normal((T, heads * (dim + rot))), rng.standard_normal((T, rank + rot)).astype(np.float32)
+    uk, uv = (km.bf16(rng.standard_normal((heads * n, rank)) / rank ** 0.5) for n in (dim, vdim))
+    layer = Latent(awq, lib, dev, True, heads, dim, rot, vdim, rank, uk, uv, np.ones(rank), None, (dim + rot) ** -0.5, 1e-6, 1e4, T, T)
+    run = lambda d, sizes: np.concatenate([layer.run(q[at:at + n], d[at:at + n], at) for at, n in portions(T, sizes)])
+    for sizes in ([T], [64, 7, 4]):
+        want = run(down, sizes)
+        for at in (1, 5, 130, 256, 258):
+            d = down.copy()
+            d[at, :rank] = np.nan
+            got = run(d, sizes)
+            assert np.isfinite(want).all() and np.array_equal(got[:at], want[:at]) and not np.isfinite(got[at:]).any(), (at, sizes)
+
+
 @pytest.mark.parametrize("f32", FORMATS, ids=["bf16", "f32"])
 @pytest.mark.parametrize("shape", [(2, 64, 32, 64, 128), (3, 20, 6, 12, 37)], ids=str)
 def test_a_key_far_back_and_the_sink(awq, lib, dev, f32, shape):
