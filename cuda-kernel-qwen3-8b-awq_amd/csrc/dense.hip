@@ -308,7 +308,9 @@ __global__ __launch_bounds__(256, 2) void dense_many_kernel(DenseArgs a, int row
   // Step st multiplies tile st % 3 and set st % 2 of the weights.  Both were requested two steps ago, so that a trip to memory
   // has two steps of products to hide behind: at the wait the 8 + TT requests of the step between may still be on their
   // way.  A slice's weights are requested into the registers that the slice has just used.  Past the end every lane
-  // requests the same piece, which is not used: the number of requests on their way is that of any other step.
+  // requests the same piece, which is not used.  The compiler need not keep the weights' requests of those steps: at the
+  // wait ahead of a last step the youngest 8 + TT are then TT past the end and the 8 for that step's own weights, whose
+  // use waits for them.  That leaves no request to spare, and needs a step's tokens to be requested ahead of its weights.
   bf16x8_t w0[2][4], w1[2][4];
   auto step = [&](const bf16_t* now, bf16x8_t (&w)[2][4], bf16_t* later, int st) __attribute__((always_inline)) {
     __builtin_amdgcn_s_waitcnt(0x0f70 | (8 + TT));  // vmcnt(8 + TT)
@@ -481,6 +483,11 @@ int launch_many(const DenseArgs& a, int64_t rows, hipStream_t st) {
       const float t = many_time(a, rows, w != 0, c);
       if (t < best) best = t, wide = w != 0, cuts = c;
     }
+  // With few steps most of the time is the end of a tile, which the estimate leaves out and which is twice as long for 128 tokens:
+  // at up to 512 inputs tiles of 64 are the faster ones wherever all of them are on the device at once (38 of 38 timed,
+  // by 4 to 32 %: 4,096 x 256 at 2,048 tokens 15.6 us against 18.1, 2,048 x 256 11.5 against 16.6).  Where they are not, or k is
+  // longer, it goes either way and the estimate decides.
+  if (wide && cuts == 1 && a.k <= 512 && row_tiles * ((a.M + 63) / 64) * a.batch <= 512) wide = false;
   const int64_t tok_tiles = wide ? (a.M + 127) / 128 : (a.M + 63) / 64;
   const int64_t tiles = row_tiles * tok_tiles;
   const dim3 grid((unsigned)((tiles * cuts + 7) / 8 * 8), (unsigned)a.batch);

@@ -175,6 +175,26 @@ def test_products_of_every_number_of_steps(awq, lib, dev, tokens, steps):
         assert np.abs(got[:tokens] - xv @ wv.T).max() < 8 * k ** 0.5 * 2.0 ** -24
 
 
+@pytest.mark.parametrize("k", [64, 320, 512, 576])
+@pytest.mark.parametrize("rows,tokens", [(2000, 2001), (8200, 1030)])
+def test_products_of_few_inputs_and_many_tokens(awq, lib, dev, rows, tokens, k):
+    """either side of the rule by which few inputs go in small tiles: inputs up to 512, tiles on the device at once or not"""
+    print("few inputs", rows, tokens, k, flush=True)
+    rng = np.random.default_rng(k + rows)
+    block = dev.torch.zeros((rows + 255) // 256 * 256 * k, dtype=dev.torch.bfloat16, device="cuda")
+    w, wv = dev.act(rng.standard_normal((rows, k)) / k ** 0.5, False)
+    awq.check(lib.awq_dense_pack(w.data_ptr(), 0, rows, k, block.data_ptr(), k, 0, 0, 0, dev.stream))
+    x, xv = dev.act(rng.standard_normal((tokens, k)), False)
+    y = dev.empty((tokens + 1, rows), True)
+    a = awq.AwqDenseArgs()
+    a.w, a.k, a.tokens, a.n_segments, a.out = block.data_ptr(), k, tokens, 1, awq.DENSE_F32
+    a.segment[0] = awq.AwqDenseSegment(x.data_ptr(), y.data_ptr(), k, rows, 0, rows, 0, 0, 0, 0)
+    awq.check(lib.awq_dense(ctypes.byref(a), 0, dev.stream))
+    got = dev.host(y)
+    assert np.isnan(got[tokens]).all()
+    assert np.abs(got[:tokens] - xv @ wv.T).max() < 8 * k ** 0.5 * 2.0 ** -24   # as in the test above
+
+
 def test_xielu_near_zero_and_far_out(awq, lib, dev):
     """the negative branch cancels near zero: small arguments keep their relative accuracy"""
     z = np.concatenate([-np.geomspace(1e-6, 60, 200), np.geomspace(1e-6, 60, 56)]).astype(np.float32)
