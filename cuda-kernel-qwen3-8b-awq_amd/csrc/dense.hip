@@ -420,12 +420,22 @@ int launch_one(const DenseArgs& a, int64_t rows, hipStream_t st) {
   return AWQ_OK;
 }
 
+// 32 rows per workgroup read the tokens half as often, 16 make twice the workgroups: 8,192 x 1,024 at 9 tokens 6.9 against 5.2 us,
+// 16,384 x 4,096 at 16 tokens 25.4 against 32.0, at 32 tokens 32.3 against 46.7
+bool few_pairs(int64_t rows, int64_t tokens, int64_t blocks) { return rows * blocks >= (tokens <= 16 ? 16384 : 8192); }
+
+// The time of such a launch in us, without its first 1.5: what the workgroups of a compute unit take in, at the rates at which
+// one does for one and for two tiles of tokens, or the weights out of memory.
+float few_time(const DenseArgs& a, int64_t rows) {
+  const int64_t R = few_pairs(rows, a.M, a.batch) ? 32 : 16, per_unit = (rows / R * a.batch + 255) / 256;
+  return std::max((float)per_unit * (float)((R + a.M) * a.k) * 2.0f / (a.M <= 16 ? 36e3f : 28e3f),
+                  (float)rows * (float)a.k * (float)a.batch * 2.0f / 5.4e6f);
+}
+
 // up to 32 tokens, or tiles of as many
 template <int OUT, bool LISTED>
 int launch_few(const DenseArgs& a, int64_t rows, int tokens, int blocks, hipStream_t st) {
-  // 32 rows per workgroup read the tokens half as often, 16 make twice the workgroups: 8,192 x 1,024 at 9 tokens 6.9 against 5.2 us,
-  // 16,384 x 4,096 at 16 tokens 25.4 against 32.0, at 32 tokens 32.3 against 46.7
-  const bool pairs = rows * blocks >= (tokens <= 16 ? 16384 : 8192);
+  const bool pairs = few_pairs(rows, tokens, blocks);
   const dim3 g((unsigned)(rows / (pairs ? 32 : 16)), (unsigned)blocks);
   const auto launch = [&](auto waves) {
     constexpr int NW = decltype(waves)::value;
@@ -467,10 +477,14 @@ float many_time(const DenseArgs& a, int64_t rows, bool wide, int64_t cuts) {
 
 template <int OUT>
 int launch_many(const DenseArgs& a, int64_t rows, hipStream_t st) {
-  // (21 to 32 tokens on few long rows read the tokens more than the weights: 4,096 x 12,288 at 32 37 us, below 32; 2,048 x 8,192 at 25
-  // 20.4, below 18.8)
-  if (a.M <= 20 || (a.M <= kFewTokens && (rows >= 8192 || a.k <= 4096)))
-    return launch_few<OUT, false>(a, rows, (int)a.M, a.batch, st);
+  // A product of few tokens goes the way whose time is estimated to be the shorter; what the other way's estimate leaves out is 9.5 us
+  // more.  Workgroups that leave compute units idle and long rows, which read the tokens more than the weights, are against
+  // the few-token kernel: 6,144 x 12,288 at 20 tokens 54 us, below 36; 28,672 x 4,096 at 32 59 and 51.  Of 888 timings (14 x 9
+  // shapes from 256 x 512 to 28,672 x 4,096, 2 to 32 tokens, both ways) the choice is 0.1 % off on average and 12 % at most; with
+  // up to 20 tokens always there, and up to 32 from 8,192 rows or to 4,096 inputs, 2.3 and 67 %.
+  constexpr float kManyMore = 9.5f;
+  const float few = a.M <= kFewTokens ? few_time(a, rows) : HUGE_VALF;
+  if (few < kManyMore) return launch_few<OUT, false>(a, rows, (int)a.M, a.batch, st);
   const int row_tiles = (int)(rows / 256);
   int64_t most = 1;  // shares of k: at least four steps each
   if (a.workspace && a.batch == 1 && a.M <= 65535)
@@ -483,8 +497,9 @@ int launch_many(const DenseArgs& a, int64_t rows, hipStream_t st) {
       const float t = many_time(a, rows, w != 0, c);
       if (t < best) best = t, wide = w != 0, cuts = c;
     }
+  if (few < best + kManyMore) return launch_few<OUT, false>(a, rows, (int)a.M, a.batch, st);
   // With few steps most of the time is the end of a tile, which the estimate leaves out and which is twice as long for 128 tokens:
-  // at up to 512 inputs tiles of 64 are the faster ones wherever all of them are on the device at once (38 of 38 timed,
+  // at up to 512 inputs tiles of 64 are the faster ones wherever all of them are on the device at once (36 of 36 timed,
   // by 4 to 32 %: 4,096 x 256 at 2,048 tokens 15.6 us against 18.1, 2,048 x 256 11.5 against 16.6).  Where they are not, or k is
   // longer, it goes either way and the estimate decides.
   if (wide && cuts == 1 && a.k <= 512 && row_tiles * ((a.M + 63) / 64) * a.batch <= 512) wide = false;
