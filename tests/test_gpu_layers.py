@@ -97,9 +97,10 @@ def test_dense_two_segments(awq, lib, dev, f32, tokens, shape):
 
 
 @pytest.mark.parametrize("tokens", [1, 2, 31, 32, 33, 64, 65, 96, 127, 129, 193])
-@pytest.mark.parametrize("rows,k", [(1, 64), (70, 320), (257, 1088), (8200, 256)])
+@pytest.mark.parametrize("rows,k", [(1, 64), (70, 320), (257, 1088), (300, 1856), (8200, 256), (16401, 448)])
 def test_binary32_products_at_the_edges_of_tiles(awq, lib, dev, tokens, rows, k):
-    """every tile of tokens, shares of k down to one, inputs and outputs that are not aligned to 16 bytes.  A sum of k products
+    """every tile of tokens, shares of k down to one, one, two and four rows per wavefront for one token, inputs and outputs that are
+    not aligned to 16 bytes.  A sum of k products
     in binary32 is off by about sqrt(k) roundings of 2^-24 of its size"""
     print("binary32", tokens, rows, k, flush=True)
     rng = np.random.default_rng(rows + tokens)

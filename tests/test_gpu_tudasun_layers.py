@@ -154,6 +154,38 @@ def test_batches(products, awq, dev, tokens):
                 assert np.isnan(got[i]).all()
 
 
+@pytest.mark.parametrize("n", [1, 2, 6])
+def test_gated_products_of_one_token_by_number(products, awq, dev, n):
+    """gate and up rows that one wavefront holds, two pairs of them where there are many rows, with blocks that are left out"""
+    f32 = products.f32
+    rng = np.random.default_rng(n)
+    blocks, ff, k = 4, 1501, 192
+    rp = up(2 * up(ff, 8), 256)
+    block = products.block(blocks * rp, k)
+    gate, upw = ([products.matrix(rng, ff, k, 1.5) for _ in range(blocks)] for _ in range(2))
+    for i in range(blocks):
+        products.pack(gate[i], block, k, i * rp, 1)
+        products.pack(upw[i], block, k, i * rp, 2)
+    ids = [3, 0, 9, 2, 0, 1][:n]
+    d_ids = dev.torch.tensor(ids, dtype=dev.torch.int32).cuda()
+    x, xv = dev.act(rng.standard_normal((n, k)), f32)
+    y = dev.empty((n, ff + 3), f32)
+    a = awq.AwqDenseArgs()
+    a.w, a.k, a.tokens, a.n_segments, a.out = block.data_ptr(), k, 1, 1, awq.DENSE_STORE
+    a.segment[0] = awq.AwqDenseSegment(x.data_ptr(), y.data_ptr(), k, ff, 0, 2 * up(ff, 8), awq.ACT_GLU)
+    a.segment[0].glu_rows = ff
+    a.batch, a.w_batch, a.x_batch, a.y_batch, a.ids, a.n_groups = n, rp * k, k, ff + 3, d_ids.data_ptr(), blocks
+    products.run(a)
+    got = dev.host(y)
+    assert np.isnan(got[:, ff:]).all()
+    for i, e in enumerate(ids):
+        if e >= blocks:
+            assert np.isnan(got[i]).all()
+        else:
+            want = plain.silu(xv[i] @ gate[e].T) * (xv[i] @ upw[e].T)
+            assert np.abs(got[i, :ff] - want).max() < limit(f32) * max(1.0, np.abs(want).max())
+
+
 def route_inputs(rng, tokens, outputs):
     return 2 * rng.standard_normal((tokens, outputs)).astype(np.float32), (0.3 * rng.standard_normal(outputs) - 0.5).astype(np.float32)
 
