@@ -134,10 +134,11 @@ void HostRing::work(int device) {
     Piece p;
     {
       std::unique_lock<std::mutex> hold(lock);
-      changed.wait(hold, [&] { return closing || !pieces.empty(); });
-      if (pieces.empty()) return;
-      p = pieces.front();
-      pieces.pop_front();
+      changed.wait(hold, [&] { return closing || n_pieces > 0; });
+      if (n_pieces == 0) return;
+      p = pieces[first_piece];
+      first_piece = (first_piece + 1) % kSlots;
+      --n_pieces;
     }
     copy_out(p);
   }
@@ -181,7 +182,7 @@ int HostRing::push(void* host_dst, const void* device_src, int64_t bytes, hipStr
       continue;
     }
     std::lock_guard<std::mutex> hold(lock);
-    pieces.push_back(p);
+    pieces[(first_piece + n_pieces++) % kSlots] = p;
     changed.notify_all();
   }
   return AWQ_OK;

@@ -2,7 +2,6 @@
 // supplies to it, and the registry by which a model folder finds its class.
 #pragma once
 #include <condition_variable>
-#include <deque>
 #include <mutex>
 #include <string>
 #include <thread>
@@ -18,8 +17,9 @@ enum StepKind {
 };
 
 // Large results on their way to pageable host memory: the device copies pieces into a ring of pinned ones, threads copy these
-// out (and take the page faults of fresh memory, most of the time of such a copy) while the next are on their way.  Ring and
-// events are the engine's; the threads end with the request.
+// out (and take the page faults of fresh memory, most of the time of such a copy) while the next are on their way.  Ring (16 MB,
+// pinned when the engine is made) and events are the engine's; the threads end with the request.  Nothing here throws:
+// a request of a C entry runs through it.
 class HostRing {
  public:
   static constexpr int kSlots = 8, kThreads = 4;
@@ -45,7 +45,8 @@ class HostRing {
   bool busy[kSlots] = {};
   std::mutex lock;
   std::condition_variable changed;
-  std::deque<Piece> pieces;
+  Piece pieces[kSlots];  // a ring: a piece has a slot, so there are never more
+  int first_piece = 0, n_pieces = 0;
   bool closing = false, failed = false;
   std::vector<std::thread> threads;
 };
