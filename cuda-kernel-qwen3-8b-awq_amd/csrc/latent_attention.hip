@@ -761,7 +761,7 @@ int launch_latent_attention(const LatentAttnArgs& a, bool f32, hipStream_t st) {
     hipLaunchKernelGGL(latent_combine_kernel, dim3((unsigned)(a.M * a.heads)), dim3(256), 0, st, a, parts, (int)v_inputs(a));
   } else {
     const int row = a.l.row(), kv_in = (int)v_inputs(a);
-    const bool few = a.M < 4 || query_lds(row, 4) > 65536;
+    const bool few = a.M < 4;  // (four queries of the longest row, 1,024 of each part, are 53 KB of LDS)
     const dim3 g((unsigned)a.heads, (unsigned)(few ? a.M : (a.M + 3) / 4));
     if (f32 && few) hipLaunchKernelGGL((latent_query_kernel<float, 1>), g, dim3(256), query_lds(row, 1), st, a, kv_in);
     else if (f32) hipLaunchKernelGGL((latent_query_kernel<float, 4>), g, dim3(256), query_lds(row, 4), st, a, kv_in);
