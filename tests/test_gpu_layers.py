@@ -151,6 +151,52 @@ def test_products_of_few_tokens(awq, lib, dev, tokens, rows, k):
     assert np.abs(got[:tokens] - xv @ wv.T).max() < 8 * k ** 0.5 * 2.0 ** -24
 
 
+@pytest.mark.parametrize("tokens", [2, 16, 17, 20, 32])
+@pytest.mark.parametrize("k", [192, 1088, 8256])
+def test_few_tokens_on_many_rows(awq, lib, dev, tokens, k):
+    """32 rows per workgroup with 4, 8 and 16 wavefronts, for every kind of output: gated pairs, biases, another type, a residual.
+    17,152 padded rows: the few-token kernel up to 8,256 inputs and 20 tokens at least, by its estimate against the other one."""
+    torch = dev.torch
+    print("few tokens, many rows", tokens, k, flush=True)
+    rows0, glu, plain_rows, sig = [0, 16032, 16320], 8009, 261, 300   # at multiples of 32
+    total = 17152
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(tokens + k)
+    block = torch.zeros(total * k, dtype=torch.bfloat16, device="cuda")
+    w = {n: (torch.randn(r, k, generator=gen, device="cuda") / k ** 0.5).bfloat16() for n, r in
+         (("gate", glu), ("up", glu), ("plain", plain_rows), ("sig", sig))}
+    for n, r0, form in (("gate", 0, 1), ("up", 0, 2), ("plain", rows0[1], 0), ("sig", rows0[2], 0)):
+        awq.check(lib.awq_dense_pack_form(w[n].data_ptr(), 0, w[n].shape[0], k, block.data_ptr(), k, r0, 0, form, 0, dev.stream))
+    x = torch.randn(tokens, k, generator=gen, device="cuda").bfloat16()
+    z = {n: (x.double() @ v.double().t()).cpu().numpy() for n, v in w.items()}
+    y = {n: dev.empty((tokens + 1, r + 3), n == "plain") for n, r in (("glu", glu), ("plain", plain_rows), ("sig", sig))}
+    bias = torch.randn(sig, generator=gen, device="cuda")
+    a = awq.AwqDenseArgs()
+    a.w, a.k, a.tokens, a.n_segments, a.out = block.data_ptr(), k, tokens, 3, awq.DENSE_STORE
+    for i, (n, rows, act) in enumerate((("glu", 16032, awq.ACT_GLU), ("plain", plain_rows, awq.ACT_NONE), ("sig", sig, awq.ACT_SIGMOID))):
+        a.segment[i] = awq.AwqDenseSegment(x.data_ptr(), y[n].data_ptr(), k, y[n].shape[1], rows0[i], rows, act)
+    a.segment[0].glu_rows, a.segment[1].y_f32, a.segment[2].bias = glu, 1, bias.data_ptr()
+    awq.check(lib.awq_dense(ctypes.byref(a), 0, dev.stream))
+    want = {"glu": plain.silu(z["gate"]) * z["up"], "plain": z["plain"], "sig": plain.sigmoid(z["sig"] + bias.double().cpu().numpy())}
+    exact = 8 * k ** 0.5 * 2.0 ** -24  # a sum of k exact products in binary32; a result in bfloat16 is off by 2^-9 of its size more
+    for n, v in want.items():
+        got = dev.host(y[n])
+        assert np.isnan(got[tokens]).all() and np.isnan(got[:, v.shape[1]:]).all(), n
+        off = np.abs(got[:tokens, :v.shape[1]] - v)
+        assert np.all(off <= 4 * exact * (1 + np.abs(v)) + (0 if n == "plain" else 2.0 ** -8 * np.abs(v))), n
+    # the same rows as a residual: gate and up rows lie in eights
+    r = dev.f(np.zeros((tokens, 16032)))
+    r.normal_(generator=gen)
+    before = dev.host(r)
+    a.n_segments, a.out = 1, awq.DENSE_RESIDUAL
+    a.segment[0] = awq.AwqDenseSegment(x.data_ptr(), r.data_ptr(), k, 16032, 0, 16032)
+    awq.check(lib.awq_dense(ctypes.byref(a), 0, dev.stream))
+    sums = np.zeros((tokens, 16032))
+    at = np.arange(glu) // 8 * 16 + np.arange(glu) % 8
+    sums[:, at], sums[:, at + 8] = z["gate"], z["up"]
+    assert np.abs(dev.host(r) - (before + sums)).max() < exact + 8 * 2.0 ** -24   # and the residual's own rounding
+
+
 @pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 6, 7, 8, 9, 12, 13, 37])
 @pytest.mark.parametrize("tokens", [33, 129, 700])
 def test_products_of_every_number_of_steps(awq, lib, dev, tokens, steps):

@@ -96,10 +96,15 @@ def test_small_model_batched_prompt_matches_sequential(awq, oracle, torch_gpu, s
 def test_sums_of_a_cut_product_normed_by_their_launch(awq, oracle, torch_gpu, hidden, inter):
     """Rows of fewer pieces than threads, of one for each, and of the most that registers hold."""
     cfg = awq.make_config(n_layers=2, hidden=hidden, inter=inter, vocab=1024, max_pos=64)
+    # a product with its sums in parts, for which alone the launch is there, among those of the passes below
+    lib = awq.load_library()
+    cut = [n for n in (5, 16, 33) for k in (hidden, inter)
+           if lib.awq_gemm_plan(hidden, k, n, 1) == 1 and lib.awq_gemm_workspace_bytes(hidden, k, n) > 0]
+    assert cut, "no product of these sizes is cut along k any more"
     model = make_oracle_model(oracle, cfg)
     eng = awq.QWen3AWQInfer.empty(cfg)
     fill_pair(awq, oracle, cfg, 78, engine=eng, model=model, profile=awq.SYNTH_BALANCED)
-    for n in (5, 33):
+    for n in (5, 16, 33):
         prompt = np.random.default_rng(n).integers(0, cfg.vocab, n).tolist()
         eng.reset()
         eng.prefill(prompt)

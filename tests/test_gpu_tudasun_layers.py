@@ -201,7 +201,7 @@ def test_router(awq, lib, dev, outputs, experts, top, groups, keep, corrected):
     print("router", outputs, experts, top, groups, keep, flush=True)
     rng = np.random.default_rng(outputs)
     t = dev.torch
-    for tokens, size in ((1, 64), (2, 64), (67, 64), (500, 128), (1500, 64)):
+    for tokens, size in ((1, 64), (2, 64), (67, 64), (500, 128), (1500, 64), (3, 16), (67, 16), (40, 32), (301, 32)):
         z, corr = route_inputs(rng, tokens, outputs)
         ld = outputs + 3
         d_z, d_c = dev.f(np.pad(z, ((0, 0), (0, 3)), constant_values=50.0)), dev.f(corr)
@@ -235,18 +235,29 @@ def test_router(awq, lib, dev, outputs, experts, top, groups, keep, corrected):
 @pytest.mark.parametrize("tokens", [2, 40, 300, 700])
 def test_products_of_token_lists(products, awq, lib, dev, tokens):
     """a gated product that reads a token per entry and one that reads an entry's own row"""
+    token_lists(products, awq, lib, dev, tokens, 128 if tokens == 700 and not products.f32 else 64, 72, 45)
+
+
+@pytest.mark.parametrize("size", [16, 32])
+@pytest.mark.parametrize("tokens,width,ff", [(2, 72, 45), (13, 72, 45), (40, 72, 45), (64, 1100, 700), (61, 600, 1300)])
+def test_products_of_lists_in_small_tiles(products, awq, lib, dev, size, tokens, width, ff):
+    """tiles of 16 and 32 entries, full and ragged; bfloat16: 16 and, where rows times tiles are many (18 tiles of 1,536 and 1,280
+    rows, 12 of 2,816 and 768), 32 rows per workgroup, with four and eight wavefronts"""
+    token_lists(products, awq, lib, dev, tokens, 32 if products.f32 else size, width, ff)
+
+
+def token_lists(products, awq, lib, dev, tokens, size, width, ff):
     f32, t = products.f32, dev.torch
-    print("lists", tokens, f32, flush=True)
+    print("lists", tokens, size, width, ff, f32, flush=True)
     rng = np.random.default_rng(tokens)
-    experts, outputs, top, width, ff = 6, 8, 3, 72, 45
-    size = 128 if tokens == 700 and not f32 else 64
-    wk, fk, gu_rows = up(width, 64), up(ff, 64), 256
+    experts, outputs, top = 6, 8, 3
+    wk, fk, gu_rows, out_rows = up(width, 64), up(ff, 64), up(2 * up(ff, 8), 256), up(width, 256)
     gate, upw, down = ([products.matrix(rng, r, c, 1.5) for _ in range(experts)] for r, c in ((ff, width), (ff, width), (width, ff)))
-    w_in, w_out = products.block(experts * gu_rows, wk), products.block(experts * 256, fk)
+    w_in, w_out = products.block(experts * gu_rows, wk), products.block(experts * out_rows, fk)
     for e in range(experts):
         products.pack(gate[e], w_in, wk, e * gu_rows, 1)
         products.pack(upw[e], w_in, wk, e * gu_rows, 2)
-        products.pack(down[e], w_out, fk, e * 256)
+        products.pack(down[e], w_out, fk, e * out_rows)
     x, xv = dev.act(np.pad(rng.standard_normal((tokens, width)), ((0, 0), (0, wk - width))), f32)
     z, corr = route_inputs(rng, tokens, outputs)
     d_z, d_c = dev.f(z), dev.f(corr)
@@ -266,7 +277,7 @@ def test_products_of_token_lists(products, awq, lib, dev, tokens):
     b.w, b.k, b.tokens, b.n_segments, b.out = w_out.data_ptr(), fk, tokens, 1, awq.DENSE_STORE
     b.segment[0] = awq.AwqDenseSegment(mid.data_ptr(), y.data_ptr(), fk, width, 0, width)
     b.segment[0].y_f32 = 1
-    b.w_batch, b.tiles, b.list, b.max_tiles, b.tile_tokens, b.list_div = 256 * fk, tiles.data_ptr(), lst.data_ptr(), n_tiles, size, 1
+    b.w_batch, b.tiles, b.list, b.max_tiles, b.tile_tokens, b.list_div = out_rows * fk, tiles.data_ptr(), lst.data_ptr(), n_tiles, size, 1
     products.run(b)
     got, chosen = dev.host(y), ids.cpu().numpy().reshape(-1)
     scale = 0.0
