@@ -660,6 +660,21 @@ int heads_product(const LatentAttnArgs& a, const void* w, int64_t w_batch, int64
   return launch_dense(d, f32, st);
 }
 
+template <typename T, int QN>
+void launch_query_kernel(const LatentAttnArgs& a, hipStream_t st) {  // (four queries of the longest row, 1,024 of each part, are 53 KB of LDS)
+  hipLaunchKernelGGL((latent_query_kernel<T, QN>), dim3((unsigned)a.heads, (unsigned)((a.M + QN - 1) / QN)), dim3(256),
+                     query_lds(a.l.row(), QN), st, a, (int)v_inputs(a));
+}
+
+template <typename T>
+void launch_queries(const LatentAttnArgs& a, hipStream_t st) {
+  switch (queries_together(a.heads, a.M)) {
+    case 1: launch_query_kernel<T, 1>(a, st); break;
+    case 2: launch_query_kernel<T, 2>(a, st); break;
+    default: launch_query_kernel<T, 4>(a, st); break;
+  }
+}
+
 }  // namespace
 
 int64_t latent_uk_block(const LatentAttnArgs& a) { return round_up(a.l.rank, kDenseRowAlign) * q_inputs(a); }
@@ -759,14 +774,10 @@ int launch_latent_attention(const LatentAttnArgs& a, bool f32, hipStream_t st) {
       return AWQ_OK;
     }
     hipLaunchKernelGGL(latent_combine_kernel, dim3((unsigned)(a.M * a.heads)), dim3(256), 0, st, a, parts, (int)v_inputs(a));
+  } else if (f32) {
+    launch_queries<float>(a, st);
   } else {
-    const int row = a.l.row(), kv_in = (int)v_inputs(a);
-    const bool few = a.M < 4;  // (four queries of the longest row, 1,024 of each part, are 53 KB of LDS)
-    const dim3 g((unsigned)a.heads, (unsigned)(few ? a.M : (a.M + 3) / 4));
-    if (f32 && few) hipLaunchKernelGGL((latent_query_kernel<float, 1>), g, dim3(256), query_lds(row, 1), st, a, kv_in);
-    else if (f32) hipLaunchKernelGGL((latent_query_kernel<float, 4>), g, dim3(256), query_lds(row, 4), st, a, kv_in);
-    else if (few) hipLaunchKernelGGL((latent_query_kernel<bf16_t, 1>), g, dim3(256), query_lds(row, 1), st, a, kv_in);
-    else hipLaunchKernelGGL((latent_query_kernel<bf16_t, 4>), g, dim3(256), query_lds(row, 4), st, a, kv_in);
+    launch_queries<bf16_t>(a, st);
   }
   AWQ_HIP_TRY(hipGetLastError());
   return heads_product(a, a.w_uv, latent_uv_block(a), v_inputs(a), a.ol, a.ctx, a.ldc, a.vdim, a.vdim, f32, st);

@@ -12,18 +12,30 @@ struct Four {
   typedef T type __attribute__((ext_vector_type(4), aligned(sizeof(T))));
 };
 
+// Queries that share a workgroup.  A workgroup's time grows with them (one, two and four: 9, 11 and 15 us for 4 queries against their own
+// keys, 122, 143 and 218 for 64 queries of 8 heads of 128 behind 3,000), so they share one only where single ones would be
+// several per compute unit, and then for the rows that are read once: 200 queries of 8 heads of 128 behind 3,000 259, 213 and
+// 247 us, of 32 heads 850, 630 and 560.  The lines lie between what was slower and what was faster there at 0, 60, 400 and 3,000 keys
+// ahead of 2 to 512 queries (heads of 64 to 512, latents of 160 to 1,064).  Without a window a query's sums are the same in all three.
+inline int queries_together(int64_t heads, int64_t queries) {
+  const int64_t alone = heads * queries;  // workgroups
+  return alone <= 1024 ? 1 : alone <= 2560 ? 2 : 4;
+}
+
 inline size_t query_lds(int row, int queries) { return sizeof(float) * (size_t)(queries * (row + 256 + 4 + 1024)); }
 
 // A workgroup of 256 threads takes QN queries next to each other, `q` [QN][row] in LDS, query i the keys lo[i] .. hi[i] (both
 // ascending in i), in blocks of 256 with a running maximum.  Scores: sixteen lanes per key, four values each, so that a row is read in whole lines and
 // by all queries at once; softmax: a thread per key; values: a thread per four columns and share of the block's keys.
-// key_row(key), value_row(key): rows (row and cols values, row a multiple of 4); score(i, key, dot): query i's score of a key that
+// key_row(key), value_row(key): rows (row and cols values, row a multiple of 4; the columns behind
+// the last to the next multiple of 4 are read too); score(i, key, dot): query i's score of a key that
 // it sees (one of the first block among them).  m, l: where a query's maximum and sum start; they and the columns come out
 // through store(i, column, four sums, l), for columns below `cols`.  A row that a query does not see is not in its
 // sums, whatever the row holds.
-// Bound by the reads out of the L2 and, for few queries, by the trips to it.  8 heads of 128, 333 queries, binary32: 39 us (one query of
-// 8 heads against 60 latents of 576: 9.8); 108 (19) with a thread per key and query that read its row value by value.
-// (The few keys that only some of the queries see have loops of their own: 0.2 us.)
+// Bound by the reads out of the L2 and, for few queries, by the trips to it.  8 heads of 128, binary32: 333 queries 42 us (a thread per
+// key and query that read its row value by value: 103), 16 queries 9.4 (11.5) and behind 3,000 keys 102 (361).  One query of
+// 8 heads against 3,001 latents of 1,064 in bfloat16: 505 (735; 815 while the loop over value rows had a branch for the last columns
+// in it, which waits for each row).  (The few keys that only some of the queries see have loops of their own: 0.2 us.)
 template <typename T, int QN, typename K, typename V, typename S, typename O>
 __device__ __forceinline__ void attend_queries(float* lds, int row, int cols, const int (&lo)[QN], const int (&hi)[QN], K key_row,
                                                V value_row, S score, float (&m)[QN], float (&l)[QN], O store) {
@@ -106,22 +118,14 @@ __device__ __forceinline__ void attend_queries(float* lds, int row, int cols, co
     }
     if (share < shares) {
       auto add = [&](int j, bool all) __attribute__((always_inline)) {
-        const T* const at = value_row(k0 + j) + 4 * quad;
-        float v[4];
-        if (4 * quad + 3 < cols) {
-          const four_t v4 = *reinterpret_cast<const four_t*>(at);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = (float)v4[e];
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = 4 * quad + e < cols ? (float)at[e] : 0.0f;
-        }
+        // (columns behind the last, which are there, are not stored: a branch for them would wait for each key's row)
+        const four_t v = *reinterpret_cast<const four_t*>(value_row(k0 + j) + 4 * quad);
 #pragma unroll
         for (int i = 0; i < QN; ++i) {
           if (!all && (k0 + j < lo[i] || k0 + j > hi[i])) continue;
           const float w = p[i * 256 + j];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) acc[i][e] = __builtin_fmaf(w, v[e], acc[i][e]);
+          for (int e = 0; e < 4; ++e) acc[i][e] = __builtin_fmaf(w, (float)v[e], acc[i][e]);
         }
       };
       // the keys ahead of the last query's first and behind the first query's last are not seen by all
@@ -140,8 +144,10 @@ __device__ __forceinline__ void attend_queries(float* lds, int row, int cols, co
 #pragma unroll
     for (int i = 0; i < QN; ++i) *reinterpret_cast<q4_t*>(part + (tid * QN + i) * 4) = acc[i];
     __syncthreads();
+    const int used = min(shares, hi[QN - 1] + 1 - lo[0]);  // shares that had a key
     if (share == 0)
-      for (int o = 1; o < shares; ++o)
+#pragma unroll 4
+      for (int o = 1; o < used; ++o)
 #pragma unroll
         for (int i = 0; i < QN; ++i) acc[i] = acc[i] + *reinterpret_cast<const q4_t*>(part + ((o * quads + quad) * QN + i) * 4);
   }

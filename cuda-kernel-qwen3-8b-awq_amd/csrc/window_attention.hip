@@ -546,12 +546,19 @@ int launch_append(const WindowAttnArgs& a, hipStream_t st) {
   return AWQ_OK;
 }
 
+template <typename T, int QN>
+void launch_query_kernel(const WindowAttnArgs& a, hipStream_t st) {
+  hipLaunchKernelGGL((window_query_kernel<T, QN>), dim3((unsigned)a.heads, (unsigned)((a.M + QN - 1) / QN)), dim3(256), query_lds(a.kl.row, QN),
+                     st, a);
+}
+
 template <typename T>
 int launch_queries(const WindowAttnArgs& a, hipStream_t st) {
-  if (a.M >= 4)
-    hipLaunchKernelGGL((window_query_kernel<T, 4>), dim3((unsigned)a.heads, (unsigned)((a.M + 3) / 4)), dim3(256), query_lds(a.kl.row, 4), st, a);
-  else
-    hipLaunchKernelGGL((window_query_kernel<T, 1>), dim3((unsigned)a.heads, (unsigned)a.M), dim3(256), query_lds(a.kl.row, 1), st, a);
+  switch (queries_together(a.heads, a.M)) {
+    case 1: launch_query_kernel<T, 1>(a, st); break;
+    case 2: launch_query_kernel<T, 2>(a, st); break;
+    default: launch_query_kernel<T, 4>(a, st); break;
+  }
   AWQ_HIP_TRY(hipGetLastError());
   return AWQ_OK;
 }

@@ -501,10 +501,12 @@ def test_window_attention(awq, lib, dev, f32, shape, window):
         assert km.rms_error(got, want) < (3e-5 if f32 else 0.01), sizes
 
 
-@pytest.mark.parametrize("f32,shape", [(1, (4, 2, 64, 64)), (1, (6, 1, 20, 12)), (1, (2, 1, 300, 72)), (0, (2, 1, 300, 72))], ids=str)
+@pytest.mark.parametrize("f32,shape", [(1, (4, 2, 64, 64)), (1, (6, 1, 20, 12)), (1, (2, 1, 300, 72)), (0, (2, 1, 300, 72)),
+                                       (1, (10, 2, 64, 36)), (0, (10, 1, 300, 72)), (0, (6, 1, 300, 72))], ids=str)
 @pytest.mark.parametrize("window", [0, 1, 2, 5, 250])
 def test_values_that_a_query_does_not_see(awq, lib, dev, f32, shape, window):
-    """several queries share a reading of the rows; a row that some of them do not see may hold anything"""
+    """several queries share a reading of the rows, two or four where there are many; a row that some of them do not see may hold
+    anything.  Without a window their bits are those of queries that share none"""
     heads, kv, dim, vdim = shape
     print("rows not seen", shape, window, f32, flush=True)
     rng = np.random.default_rng(window)
@@ -514,7 +516,7 @@ def test_values_that_a_query_does_not_see(awq, lib, dev, f32, shape, window):
                                    T, ((window or T) - 1 + max(sizes) + 63) // 64 * 64, T)
     for sizes in ([T], [64, 7, 4]):
         want = args(x, sizes)
-        assert np.isfinite(want).all()
+        assert np.isfinite(want).all() and (window or np.array_equal(want, args(x, [2, 70, 3])))
         for at in (0, 5, 130, 256, 258):
             y = x.copy()
             y[at, (heads + kv) * dim:n] = np.nan if at & 1 else np.inf

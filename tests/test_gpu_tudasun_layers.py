@@ -496,7 +496,7 @@ def portions(T, sizes):
 
 
 LATENTS = [(3, 20, 6, 12, 37), (4, 64, 32, 64, 128), (40, 16, 16, 24, 64), (2, 128, 64, 128, 512), (1, 72, 2, 40, 300), (2, 8, 8, 256, 200),
-           (2, 192, 64, 64, 96), (1, 100, 30, 20, 700)]
+           (2, 192, 64, 64, 96), (1, 100, 30, 20, 700), (8, 12, 30, 20, 700)]
 
 
 @pytest.mark.parametrize("f32", FORMATS, ids=["bf16", "f32"])
@@ -535,7 +535,7 @@ def test_latent_attention(awq, lib, dev, f32, shape):
         assert km.rms_error(got, want) < (3e-5 if f32 else 0.03), sizes
 
 
-@pytest.mark.parametrize("shape", [(3, 20, 6, 12, 37), (2, 64, 32, 64, 128)], ids=str)
+@pytest.mark.parametrize("shape", [(3, 20, 6, 12, 37), (5, 20, 6, 12, 37), (2, 64, 32, 64, 128), (9, 64, 32, 64, 128)], ids=str)
 def test_latents_that_a_query_does_not_see(awq, lib, dev, shape):
     """several queries share a reading of the rows in binary32; the rows behind a query's own may hold anything"""
     heads, dim, rot, vdim, rank = shape
