@@ -22,7 +22,7 @@ __device__ __forceinline__ void best_of_wave(float& v, int& i) {
 
 // Up to 64 outputs, a lane each: an output's place in the order is the number of outputs ahead of it, counted with every lane's
 // value read in turn, where the form below finds one output after the other with a reduction of its own.  The choice and
-// the bits of the weights are those of the form below.  One token, 16 outputs: 7.6 us below.
+// the bits of the weights are those of the form below.  One token, four of 16 outputs: 3.6 us, 6.1 below.
 __global__ __launch_bounds__(256) void route_few_kernel(RouteArgs a) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), E = a.outputs;
   const int64_t t = (int64_t)blockIdx.x * 4 + wave;
@@ -228,7 +228,11 @@ int launch_route(const RouteArgs& a, hipStream_t st) {
               "bad groups");
   AWQ_REQUIRE(a.M * a.top < (1 << 30) && a.tile_tokens >= 1, "too many tokens");
   const size_t lds = sizeof(float) * (2 * a.outputs + a.groups);
-  if (a.outputs <= 64)
+  // A step per output (two with groups) against one per choice: 4,000 tokens of 64 outputs, one choice 13.0 us and 10.7 below, four
+  // 21.4 and 22.2; in four groups, four choices of 40 24.9 and 23.7, of 24
+  // 21.4 and 23.5.  The lines lie where 1 to 4,000 tokens, 4 to 64 outputs and 1 to 8 choices took as long either way.
+  const int64_t few = 8 + (a.groups > 0 ? 8 : 16) * (int64_t)a.top;
+  if (a.outputs <= 64 && a.outputs <= few)
     hipLaunchKernelGGL(route_few_kernel, dim3((unsigned)((a.M + 3) / 4)), dim3(256), 0, st, a);
   else if (a.outputs <= 1024)
     hipLaunchKernelGGL(route_kernel<4>, dim3((unsigned)((a.M + 3) / 4)), dim3(256), 4 * lds, st, a);

@@ -191,7 +191,8 @@ def route_inputs(rng, tokens, outputs):
 
 
 ROUTERS = [(8, 8, 2, 0, 0), (10, 8, 4, 2, 1), (12, 9, 3, 4, 2), (6, 6, 6, 0, 0), (70, 64, 5, 7, 3), (300, 290, 8, 10, 4), (4, 0, 2, 2, 1),
-           (9, 5, 1, 9, 2)]
+           (9, 5, 1, 9, 2),
+           (40, 40, 2, 0, 0), (41, 41, 2, 0, 0), (64, 64, 4, 0, 0), (24, 22, 2, 4, 2), (28, 28, 2, 4, 2), (64, 60, 7, 4, 2)]
 
 
 @pytest.mark.parametrize("outputs,experts,top,groups,keep", ROUTERS)
