@@ -456,33 +456,34 @@ int launch_few(const DenseArgs& a, int64_t rows, int tokens, int blocks, hipStre
 }
 
 // The time of a product of many tokens in us, but for what all forms of it share: what a choice between tiles of 64 and 128
-// tokens and numbers of shares of k needs.  The rates are fitted to 1,204 timings (ten shapes from 256 x 4,096 to 28,672 x 4,096,
-// 40 to 2,048 tokens, 1 to 16 shares, weights from memory; with 8.5 us added 5 % off in the mean square): a step of a
-// workgroup that has its compute unit to itself waits for memory, the longer the more weights are on their way; a second
-// workgroup on the unit adds its products; 5.4 TB/s of weights, 16 TB/s out of the L2s; the sums of the shares are written and
-// read at 5.7 TB/s.  The form it picks takes 1.9 % longer on average than the fastest of those timed (256 workgroups whatever
-// the size, tiles of 64 up to 256 tokens: 10 %, up to 79 %; 512 workgroups, as it was: 20 to 50 % at 129 to 512 tokens).
+// tokens and numbers of shares of k needs.  A step of a workgroup that has its compute unit to itself waits for memory, the
+// longer the more weights are on their way; a second workgroup on the unit adds its products; weights out of memory; tokens out
+// of the L2s; the end of a tile; the shares' sums, written, read and added one after the other.  The numbers are fitted for the
+// choice, not for the time, to 27,100 timings (152 shapes from 256 x 64 to 32,768 x 4,096 and 8,192 x 16,384, 2 to 2,048 tokens, both
+// tiles, 1 to 16 shares, weights from memory).  From 33 tokens on the form it picks takes 1.0 % longer on average than the fastest
+// timed, 20 % at most, and 11 % at most than tiles of 128 from 65 tokens on and 512 workgroups whatever the size; without the end of
+// a tile and the time per share 2.4, 28 and 18 % (2,048 x 4,096 at 64 tokens 18.7 us, now 15.4).
 float many_time(const DenseArgs& a, int64_t rows, bool wide, int64_t cuts) {
   const int64_t row_tiles = rows / 256, tile = wide ? 128 : 64, tok_tiles = (a.M + tile - 1) / tile;
   const float groups = (float)(row_tiles * tok_tiles * cuts * a.batch), steps = (float)(((a.k >> 6) + cuts - 1) / cuts);
-  const float wait = (wide ? 0.49f : 0.28f) + 0.05f * sqrtf((float)std::min<int64_t>(256, row_tiles * cuts * a.batch));
+  const float wait = (wide ? 0.47f : 0.332f) + 0.048f * sqrtf((float)std::min<int64_t>(256, row_tiles * cuts * a.batch));
   const float per_unit = ceilf(groups / 256.0f);
   float t = steps * wait * ceilf(groups / 512.0f);
-  if (per_unit > 1.0f) t = std::max(t, steps * per_unit * (wide ? 0.87f : 0.56f));
-  t = std::max(t, (float)rows * (float)a.k * (float)a.batch * 2.0f / 5.4e6f);
-  t = std::max(t, groups * steps * (float)(32768 + tile * 128) / 16e6f);
-  if (cuts > 1) t += 1.5f + (float)cuts * (float)a.M * (float)rows * 8.0f / 5.7e6f;
+  if (per_unit > 1.0f) t = std::max(t, steps * per_unit * (wide ? 0.78f : 0.76f));
+  t = std::max(t, (float)rows * (float)a.k * (float)a.batch * 2.0f / 5.86e6f);
+  t = std::max(t, groups * steps * (float)(32768 + tile * 128) / 25e6f) + per_unit * (wide ? 2.04f : 0.9f);
+  if (cuts > 1) t += 0.11f + (float)cuts * (0.325f + (float)a.M * (float)rows * 8.0f / 4.55e6f);
   return t;
 }
 
 template <int OUT>
 int launch_many(const DenseArgs& a, int64_t rows, hipStream_t st) {
-  // A product of few tokens goes the way whose time is estimated to be the shorter; what the other way's estimate leaves out is 9.5 us
+  // A product of few tokens goes the way whose time is estimated to be the shorter; what the other way's estimate leaves out is 8.9 us
   // more.  Workgroups that leave compute units idle and long rows, which read the tokens more than the weights, are against
-  // the few-token kernel: 6,144 x 12,288 at 20 tokens 54 us, below 36; 28,672 x 4,096 at 32 59 and 51.  Of 888 timings (14 x 9
-  // shapes from 256 x 512 to 28,672 x 4,096, 2 to 32 tokens, both ways) the choice is 0.1 % off on average and 12 % at most; with
-  // up to 20 tokens always there, and up to 32 from 8,192 rows or to 4,096 inputs, 2.3 and 67 %.
-  constexpr float kManyMore = 9.5f;
+  // the few-token kernel: 6,144 x 12,288 at 20 tokens 54 us, below 36; 28,672 x 4,096 at 32 59 and 51.  Of 480 products (48
+  // shapes from 256 x 512 to 28,672 x 12,288, 2 to 32 tokens, both ways timed) the choice is 0.2 % off on average and 9 % at most;
+  // with up to 20 tokens always there, and up to 32 from 8,192 rows or to 4,096 inputs, 2.3 and 67 %.
+  constexpr float kManyMore = 8.9f;
   const float few = a.M <= kFewTokens ? few_time(a, rows) : HUGE_VALF;
   if (few < kManyMore) return launch_few<OUT, false>(a, rows, (int)a.M, a.batch, st);
   const int row_tiles = (int)(rows / 256);
@@ -498,7 +499,7 @@ int launch_many(const DenseArgs& a, int64_t rows, hipStream_t st) {
       if (t < best) best = t, wide = w != 0, cuts = c;
     }
   if (few < best + kManyMore) return launch_few<OUT, false>(a, rows, (int)a.M, a.batch, st);
-  // With few steps most of the time is the end of a tile, which the estimate leaves out and which is twice as long for 128 tokens:
+  // With few steps most of the time is the end of a tile, for which the estimate has one number of each size of tile:
   // at up to 512 inputs tiles of 64 are the faster ones wherever all of them are on the device at once (36 of 36 timed,
   // by 4 to 32 %: 4,096 x 256 at 2,048 tokens 15.6 us against 18.1, 2,048 x 256 11.5 against 16.6).  Where they are not, or k is
   // longer, it goes either way and the estimate decides.
