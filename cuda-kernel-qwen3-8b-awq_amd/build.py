@@ -27,7 +27,7 @@ CONFIG_MODEL_SOURCES = ["config_model.cpp", "kugilix.cpp", "tudasun.cpp", "dense
                         "window_attention.hip", "linear_attention.hip", "latent_attention.hip", "gated_state.hip",
                         "experts.hip"]
 # the int4 model of the raw weight directory and the entry points for single kernels
-INT4_SOURCES = ["gemv.hip", "gemm.hip", "prefill.hip", "attention.hip", "fused.hip", "qkv_attn.hip", "qwen3.cpp",
+INT4_SOURCES = ["gemv.hip", "gemm.hip", "prefill.hip", "canon_prompt.hip", "attention.hip", "fused.hip", "qkv_attn.hip", "qwen3.cpp",
                 "kernel_api.cpp", "layer_api.cpp", "synth.cpp"]
 
 # -ffp-contract=off: every fma in the sources is written out; a contracted

@@ -208,6 +208,38 @@ int launch_rope_kv_append_batch(const half_t* qkv, const half_t* cos_t, const ha
                                 half_t* kc, half_t* vc, int n_heads, int64_t max_pos, KvLayout kv, int64_t pos0,
                                 int64_t M, hipStream_t st, half_t* k_parts = nullptr, half_t* v_parts = nullptr,
                                 int parts_pos = 0);
+// Prompt positions together with the arithmetic of the one-token step (canon_prompt.hip), kCanonFrom (two take 1.8 ms one after
+// the other and 2.4 together, three 2.6 and 2.4) to kCanonTokens of them, up to position kCanonPositions.  Tokens in block fixed point, padded to a multiple of 16: the integers in the matrix
+// instruction's operand order, and each block's power of two and sum.
+constexpr int64_t kCanonFrom = 3;
+constexpr int64_t kCanonTokens = 128;
+constexpr int64_t kCanonPositions = 2048;  // four queries' scores in LDS
+inline int64_t round16(int64_t v) { return (v + 15) / 16 * 16; }
+struct CanonTokens {
+  half_t* op = nullptr;  // [tokens][k]
+  float* c = nullptr;    // [tokens][k / 32]
+  float* s = nullptr;
+};
+struct CanonQkv {
+  const half_t *cos_t = nullptr, *sin_t = nullptr;
+  half_t *q_out = nullptr, *k_cache = nullptr, *v_cache = nullptr, *k_parts = nullptr, *v_parts = nullptr;
+  int32_t parts_pos = 0, pos0 = 0;
+  KvLayout kv = {0, 0, 0};
+};
+enum CanonOut {
+  CANON_PARTS = 0,  // binary32 sums [canon_prompt_parts][M][m], for launch_canon_norm
+  CANON_GELU = 1,   // GeLU, in block fixed point
+  CANON_QKV = 2,    // rotary, q and the caches
+};
+bool canon_prompt_supported(int64_t hidden, int64_t inter);
+int canon_prompt_parts(int64_t m, int64_t k);
+int launch_canon_norm(const float* part, int parts, half_t* hidden, const half_t* gamma, float eps, CanonTokens out, int64_t M,
+                      hipStream_t st);
+// zp_small: the zero-points are integers 0 .. 16
+int launch_canon_product(const void* wq, const half_t* scale, const half_t* zp, bool zp_small, int64_t m, int64_t k, CanonTokens x,
+                         int64_t M, int out, float* part, CanonTokens y, const CanonQkv& qkv, hipStream_t st);
+int launch_canon_attention(const half_t* q, const half_t* kc, const half_t* vc, KvLayout kv, int n_heads, int64_t pos0, int64_t M,
+                           int use_len_hi, CanonTokens out, hipStream_t st);
 int launch_residual(const half_t* a, const half_t* b, half_t* out, int64_t n, hipStream_t st);
 int launch_gelu(half_t* x, int64_t n, hipStream_t st);
 int64_t argmax_workspace_bytes(int64_t n);

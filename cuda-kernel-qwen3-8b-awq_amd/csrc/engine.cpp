@@ -383,8 +383,19 @@ extern "C" int awq_reset(awq_engine* e) {
 extern "C" int awq_prefill(awq_engine* e, const int32_t* prompt_ids, int32_t n_prompt) {
   AWQ_REQUIRE(e != nullptr && n_prompt >= 0 && (n_prompt == 0 || prompt_ids), "bad arguments");
   if (int rc = check_prompt(e, prompt_ids, n_prompt, "awq_prefill")) return rc;
-  for (int32_t i = 0; i < n_prompt; ++i)
-    if (int rc = prompt_step(e, prompt_ids[i])) return rc;
+  for (int64_t off = 0, M = 0; off < n_prompt; off += M) {
+    const int64_t pos0 = e->n_positions;
+    M = e->exact_pass_tokens(pos0, n_prompt - off);
+    if (M > 0) {
+      if (int rc = e->enqueue_exact_pass(prompt_ids + off, pos0, M)) return rc;
+      AWQ_HIP_TRY(hipStreamSynchronize(e->stream));  // the token ids were read from the caller's buffer
+      e->current_seq_len = (int)(pos0 + M - 1);
+      e->n_positions = (int)(pos0 + M);
+    } else {
+      M = 1;
+      if (int rc = prompt_step(e, prompt_ids[off])) return rc;
+    }
+  }
   AWQ_HIP_TRY(hipStreamSynchronize(e->stream));
   return e->check_steps();
 }

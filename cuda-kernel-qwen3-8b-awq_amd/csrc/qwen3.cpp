@@ -124,6 +124,7 @@ struct DevLinear {
   half_t* zp = nullptr;
   int64_t m = 0, k = 0;
   int zp_integral = 0;
+  bool zp_small = false;  // integers 0 .. 16
   bool have[3] = {false, false, false};
   bool reordered = false;  // stream_order already holds the reordered copy (the directory loader does it on the fly)
 };
@@ -160,6 +161,13 @@ struct Qwen3Engine final : awq_engine {
     void* gemm_ws = nullptr;  // partial sums of products whose k is cut over workgroups
     int64_t chunk = 0;
   } pb;
+  // of the prompt pass with the one-token steps' arithmetic (canon_prompt.hip): what the products read, q, partial sums
+  struct {
+    CanonTokens x, mid;
+    half_t *hidden = nullptr, *q = nullptr;
+    float* part = nullptr;
+    int32_t* tokens = nullptr;
+  } pc;
   // Wo and W1 of a layer as one launch (fused.hip): the hidden state between them as tagged words, and the word
   // through which a wait that gave up reports
   bool fused = false;
@@ -191,6 +199,8 @@ struct Qwen3Engine final : awq_engine {
   int64_t prompt_pass_tokens(int64_t done, int64_t rest) const override;
   int enqueue_prompt_pass(const int32_t* tokens, int64_t pos0, int64_t M) override;
   int check_prompt_pass() override;
+  int64_t exact_pass_tokens(int64_t done, int64_t rest) const override;
+  int enqueue_exact_pass(const int32_t* tokens, int64_t pos0, int64_t M) override;
   int read_rows_logits(bool batched, const int32_t* rows, int32_t n, float* host_dst) override;
   int read_logits_f32(float* host_dst) override;
   int read_hidden_f32(float* host_dst) override;
@@ -247,6 +257,12 @@ int alloc_linear(Qwen3Engine* e, DevLinear& t, int kind, bool with_packed = true
   return AWQ_OK;
 }
 
+
+void note_zero_points(DevLinear* t, const uint16_t* zp, int64_t n) {
+  t->zp_integral = awq_zp_all_integral(zp, n);
+  t->zp_small = t->zp_integral != 0;
+  for (int64_t i = 0; i < n; ++i) t->zp_small = t->zp_small && (zp[i] & 0x7fff) <= 0x4c00;  // 16
+}
 
 // one fused-linear launch on the engine's stream
 LinearArgs linear_args(Qwen3Engine* e, const DevLinear& t, const half_t* x, half_t* y) {
@@ -497,7 +513,7 @@ extern "C" int awq_upload(awq_engine* handle, int layer, int kind, int part, con
   AWQ_REQUIRE(t != nullptr, "layer out of range");
   void* dst = part == AWQ_P_PACKED ? (void*)t->packed : part == AWQ_P_SCALE ? (void*)t->scale : (void*)t->zp;
   AWQ_HIP_TRY(hipMemcpy(dst, host_src, (size_t)bytes, hipMemcpyHostToDevice));
-  if (part == AWQ_P_ZP) t->zp_integral = awq_zp_all_integral((const uint16_t*)host_src, bytes / 2);
+  if (part == AWQ_P_ZP) note_zero_points(t, (const uint16_t*)host_src, bytes / 2);
   t->have[part] = true;
   return AWQ_OK;
 }
@@ -672,7 +688,7 @@ extern "C" int awq_create(const char* weight_dir, const awq_config* cfg_in, awq_
         t = find_linear(e, wf.layer, wf.kind);
         if (wf.part == AWQ_P_PACKED && wf.kind != AWQ_T_EMBED) t->packed = (uint8_t*)dstage[n_staged++ & 1];
         dst = wf.part == AWQ_P_PACKED ? (void*)t->packed : wf.part == AWQ_P_SCALE ? (void*)t->scale : (void*)t->zp;
-        if (wf.part == AWQ_P_ZP) t->zp_integral = awq_zp_all_integral((const uint16_t*)s.host, wf.bytes / 2);
+        if (wf.part == AWQ_P_ZP) note_zero_points(t, (const uint16_t*)s.host, wf.bytes / 2);
         t->have[wf.part] = true;
       }
       if (hipMemcpyAsync(dst, s.host, (size_t)wf.bytes, hipMemcpyHostToDevice, e->stream) != hipSuccess ||
@@ -958,6 +974,72 @@ int Qwen3Engine::enqueue_prompt_pass(const int32_t* tokens, int64_t pos0, int64_
   AWQ_HIP_TRY(hipMemcpyAsync(e->hidden, e->pb.hidden + (M - 1) * H, (size_t)H * 2, hipMemcpyDeviceToDevice,
                              e->stream));
   return AWQ_OK;
+}
+
+namespace {
+int alloc_canon_tokens(Qwen3Engine* e, CanonTokens& t, int64_t k) {
+  if (int rc = e->dev_alloc((void**)&t.op, kCanonTokens * k * 2)) return rc;
+  if (int rc = e->dev_alloc((void**)&t.c, kCanonTokens * k / 8)) return rc;
+  return e->dev_alloc((void**)&t.s, kCanonTokens * k / 8);
+}
+
+int ensure_canon_buffers(Qwen3Engine* e) {
+  if (e->pc.tokens) return AWQ_OK;
+  const int64_t H = e->cfg.hidden, I = e->cfg.inter, parts = std::max(canon_prompt_parts(H, H), canon_prompt_parts(H, I));
+  if (int rc = alloc_canon_tokens(e, e->pc.x, H)) return rc;
+  if (int rc = alloc_canon_tokens(e, e->pc.mid, I)) return rc;
+  if (int rc = e->dev_alloc((void**)&e->pc.hidden, kCanonTokens * H * 2)) return rc;
+  if (int rc = e->dev_alloc((void**)&e->pc.q, kCanonTokens * H * 2)) return rc;
+  if (int rc = e->dev_alloc((void**)&e->pc.part, parts * kCanonTokens * H * 4)) return rc;
+  return e->dev_alloc((void**)&e->pc.tokens, kCanonTokens * 4);
+}
+
+int canon_product(Qwen3Engine* e, const DevLinear& t, const CanonTokens& x, int64_t M, int out, const CanonTokens& y = {},
+                  const CanonQkv& qkv = {}) {
+  return launch_canon_product(t.stream_order, t.scale, t.zp, t.zp_small, t.m, t.k, x, M, out, e->pc.part, y, qkv, e->stream);
+}
+
+// The layers of M prompt positions pos0 .., `hidden` in and out, every launch with the one-token steps' arithmetic.
+int enqueue_canon_layers(Qwen3Engine* e, half_t* hidden, int64_t pos0, int64_t M) {
+  auto& b = e->pc;
+  const int64_t H = e->cfg.hidden, I = e->cfg.inter;
+  const KvLayout kv = kv_blocked(e->n_heads);
+  for (int l = 0; l < e->cfg.n_layers; ++l) {
+    LayerDev& L = e->layers[l];
+    // :1040 (and the layer before's :1201-1227)
+    if (int rc = launch_canon_norm(b.part, l ? canon_prompt_parts(H, I) : 0, hidden, L.gamma, e->cfg.eps, b.x, M, e->stream)) return rc;
+    CanonQkv qkv;  // (with the fused launch on, the appended rows also go into its second copy of the caches)
+    qkv.cos_t = e->cos_t, qkv.sin_t = e->sin_t, qkv.q_out = b.q, qkv.k_cache = L.kcache, qkv.v_cache = L.vcache;
+    if (e->fused_qkv) qkv.k_parts = L.kparts, qkv.v_parts = L.vparts, qkv.parts_pos = e->parts_pos;
+    qkv.pos0 = (int32_t)pos0, qkv.kv = kv;
+    if (int rc = canon_product(e, L.wqkv, b.x, M, CANON_QKV, {}, qkv)) return rc;                             // :1052-1103
+    if (int rc = launch_canon_attention(b.q, L.kcache, L.vcache, kv, e->n_heads, pos0, M, l >= 1, b.x, e->stream)) return rc;  // :1110
+    if (int rc = canon_product(e, L.wo, b.x, M, CANON_PARTS)) return rc;                                      // :1128
+    if (int rc = launch_canon_norm(b.part, canon_prompt_parts(H, H), hidden, L.gamma, e->cfg.eps, b.x, M, e->stream)) return rc;  // :1149-1163
+    if (int rc = canon_product(e, L.w1, b.x, M, CANON_GELU, b.mid)) return rc;                                // :1176-1196
+    if (int rc = canon_product(e, L.w2, b.mid, M, CANON_PARTS)) return rc;                                    // :1201
+  }
+  return launch_canon_norm(b.part, canon_prompt_parts(H, I), hidden, nullptr, e->cfg.eps, b.x, M, e->stream);  // :1227
+}
+}  // namespace
+
+int64_t Qwen3Engine::exact_pass_tokens(int64_t done, int64_t rest) const {
+  const int64_t room = std::min(rest, kCanonPositions - done);
+  if (room < kCanonFrom || !canon_prompt_supported(cfg.hidden, cfg.inter)) return 0;
+  const int64_t passes = (room + kCanonTokens - 1) / kCanonTokens;
+  return std::min(room, round16((room + passes - 1) / passes));
+}
+
+int Qwen3Engine::enqueue_exact_pass(const int32_t* tokens, int64_t pos0, int64_t M) {
+  Qwen3Engine* e = this;
+  if (int rc = ensure_canon_buffers(e)) return rc;
+  const int64_t H = e->cfg.hidden;
+  AWQ_HIP_TRY(hipMemcpyAsync(e->pc.tokens, tokens, (size_t)M * 4, hipMemcpyHostToDevice, e->stream));
+  if (int rc = launch_embed_batch(e->embed.packed, e->embed.scale, e->embed.zp, H, e->cfg.vocab, e->pc.tokens, M, e->pc.hidden, e->stream))
+    return rc;
+  if (int rc = enqueue_canon_layers(e, e->pc.hidden, pos0, M)) return rc;
+  // the state the generation loop starts from (:1357): the last position's output
+  return launch_copy(e->pc.hidden + (M - 1) * H, e->hidden, H * 2, e->stream);
 }
 
 int Qwen3Engine::check_prompt_pass() {

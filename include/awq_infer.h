@@ -132,8 +132,8 @@ int awq_decode(awq_engine* e, int32_t n_steps, int32_t* out_ids);
  * positions the sequential loop gives it.  Leaves the same state as awq_prefill
  * up to rounding: the products are summed in a different order, so K/V and the
  * hidden state agree to binary16 rounding noise, not bit for bit.
- * awq_set_prefill_mode(e, 1) makes awq_generate use it; the default (0) is the
- * token-by-token loop. */
+ * awq_set_prefill_mode(e, 1) makes awq_generate use it; the default (0) is
+ * awq_prefill, which leaves the bits of the token-by-token loop. */
 int awq_prefill_batched(awq_engine* e, const int32_t* prompt_ids, int32_t n_prompt);
 int awq_set_prefill_mode(awq_engine* e, int batched);
 /* Test hook, no counterpart in the reference: some of the batched pass's

@@ -335,3 +335,44 @@ def test_handed_over_sums_give_up_path(awq, lib, oracle, torch_gpu):
     assert np.array_equal(np.ctypeslib.as_array(eng.read_hidden()), hid)
     assert eng.decode(4) == tok
     eng.close()
+
+
+# Widths at which awq_prefill takes several positions together with the one-token steps' arithmetic.  k of the second
+# MLP matrix: one and three runs of 128 blocks.  Zero-points: integers within 16 (products of q - z), beyond, and not
+# integers (the general block value).
+@pytest.mark.parametrize("inter,zero,fused", [(4096, None, True), (12288, None, True), (12288, 17.0, True), (4096, 6.5, False)])
+def test_prompt_positions_together_have_the_bits_of_single_steps(awq, oracle, torch_gpu, inter, zero, fused):
+    """Portions of every count of token tiles with full and ragged last tiles, against one token a call (a single
+    position is always a step of its own): the state after the portion and what is generated from its cache rows."""
+    cfg = awq.make_config(n_layers=2, hidden=4096, inter=inter, vocab=1024, max_pos=512)
+    model = make_oracle_model(oracle, cfg)
+
+    def mutate(layer, kind, part, p, count):
+        if zero is not None and part == awq.P_ZP and kind != awq.T_GAMMA:
+            a = np.ctypeslib.as_array((ctypes.c_uint16 * count).from_address(ctypes.cast(p, ctypes.c_void_p).value))
+            a[::3] = np.float16(zero).view(np.uint16)
+
+    eng = awq.QWen3AWQInfer.empty(cfg)
+    fill_pair(awq, oracle, cfg, 31, engine=eng, model=model, profile=awq.SYNTH_BALANCED, mutate=mutate)
+    oracle.awqo_model_destroy(model)
+    if not fused:
+        eng.set_fused_mode(0)
+    rng = np.random.default_rng(inter)
+
+    def after(portions):
+        eng.reset()
+        for ids in portions:
+            eng.prefill(ids)
+        hidden = np.ctypeslib.as_array(eng.read_hidden()).copy()
+        ids = eng.decode(2)
+        return hidden, ids, np.ctypeslib.as_array(eng.read_logits()).copy()
+
+    for cuts in ([2], [3], [5], [16], [17], [31], [48], [64], [65], [96], [128], [97, 1, 34], [130], [300]):
+        portions = [rng.integers(0, cfg.vocab, n).tolist() for n in cuts]
+        print("portions", cuts, flush=True)
+        one = after([[t] for ids in portions for t in ids])
+        got = after(portions)
+        assert np.isfinite(one[0].view(np.float16)).all() and one[0].any()
+        assert np.array_equal(got[0], one[0]), cuts
+        assert got[1] == one[1] and np.array_equal(got[2], one[2]), cuts
+    eng.close()
