@@ -7,44 +7,50 @@
 
 namespace {
 // --- one token, bfloat16 -----------------------------------------------------------------------------------
-// A workgroup owns 16 rows and all of k, its wavefronts a run of k each; a load of a wavefront is four pieces of 256
-// contiguous bytes of the block.  v_mfma_f32_16x16x32_bf16 with the token in every column: the matrix unit does the
-// additions, and nothing but loads stands between the wavefront and memory.
+// A workgroup owns RW rows and all of k, its wavefronts a run of k each; a load of a wavefront is pieces of 16 RW contiguous
+// bytes of the block.  v_mfma_f32_16x16x32_bf16 with the token in the columns: the matrix unit does the additions, and nothing
+// but loads stands between the wavefront and memory.  With RW = 8 the 16 rows of the instruction are 8 rows at two steps of 32
+// inputs next to each other, and a column holds the inputs of the step whose rows it meets.
+// Eight steps of a wavefront are requested at once, and what is left of its run as well: one by one 1,536 rows of 1,536 inputs took
+// 5.7 us, now 4.0, 1,152 of 1,152 4.9 and 3.6.  Requesting the next eight ahead of these products cost more in wavefronts per unit
+// (81 registers instead of 62) than it gained: 28,672 x 4,096 40 -> 44 us.
 // GATED: the first gate_k inputs are formed here, RMS norm of o times w times sigmoid(g) (token_ops.hip has it as a
 // launch of its own for many tokens): every workgroup normalises for itself while its first weights are on their way.
-template <int NW, int OUT, bool GATED>
+template <int NW, int OUT, bool GATED, int RW>
 __global__ __launch_bounds__(NW * 64) void dense_one_kernel(DenseArgs a) {
+  constexpr int SP = 16 / RW;  // steps of an instruction
   extern __shared__ __attribute__((aligned(16))) bf16_t gated[];  // [gate_k]
   __shared__ float part[NW][16];
   __shared__ float squares[NW];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int row0 = blockIdx.x * 16;
+  const int row0 = blockIdx.x * RW;
   const DenseSegment& s = segment_of(a, row0);
   const int local = row0 - s.row0;
   if (local >= s.rows) return;  // padding
   const int group = block_of_product(a);
   if (group < 0) return;
   const int steps = (int)(a.k >> 5);  // even: k is a multiple of 64
-  const int per = (steps + NW - 1) / NW;
-  const int s0 = min(wave * per, steps), s1 = min(s0 + per, steps);
-  const int r = lane & 15, c = lane >> 4;
+  const int per = ((steps + SP - 1) / SP + NW - 1) / NW;
+  const int s0 = min(wave * per * SP, steps), s1 = min(s0 + per * SP, steps);
+  const int r = lane & 15, c = lane >> 4, sub = r / RW;
   // piece of (row, 8-wide chunk c of step i): block (row / 32, 2 i + c / 2), lane 32 (c % 2) + row % 32
   const bf16x8_t* w = reinterpret_cast<const bf16x8_t*>(reinterpret_cast<const bf16_t*>(a.w) + group * a.w_batch) +
-                      ((int64_t)(row0 >> 5) * (a.k >> 4) + (c >> 1)) * 64 + 32 * (c & 1) + (row0 & 16) + r;
-  const bf16x8_t* x = reinterpret_cast<const bf16x8_t*>(reinterpret_cast<const bf16_t*>(s.x) + blockIdx.y * a.x_batch) + c;
+                      ((int64_t)(row0 >> 5) * (a.k >> 4) + (c >> 1) + 2 * sub) * 64 + 32 * (c & 1) + (row0 & (32 - RW)) + r % RW;
+  const bf16x8_t* x = reinterpret_cast<const bf16x8_t*>(reinterpret_cast<const bf16_t*>(s.x) + blockIdx.y * a.x_batch) + c + 4 * sub;
   f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
   constexpr int U = 8;
-  bf16x8_t wv[U], xv[U];
+  constexpr int US = U * SP;
+  bf16x8_t wv[U];
   auto weights = [&](int i) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < U; ++u) wv[u] = __builtin_nontemporal_load(w + (int64_t)(i + u) * 128);
+    for (int u = 0; u < U; ++u) wv[u] = __builtin_nontemporal_load(w + (int64_t)(i + u * SP) * 128);
   };
   auto input = [&](int i) __attribute__((always_inline)) {
-    if (GATED && i * 32 < a.gate_k) return reinterpret_cast<const bf16x8_t*>(gated)[i * 4 + c];
+    if (GATED && (i + sub) * 32 < a.gate_k) return reinterpret_cast<const bf16x8_t*>(gated)[(i + sub) * 4 + c];
     return x[i * 4];
   };
   int i = s0;
-  if (i + U <= s1) weights(i);
+  if (i + US <= s1) weights(i);
   if constexpr (GATED) {
     constexpr int NT = NW * 64;
     const bf16_t* gate = reinterpret_cast<const bf16_t*>(a.gate_g);
@@ -74,27 +80,50 @@ __global__ __launch_bounds__(NW * 64) void dense_one_kernel(DenseArgs a) {
     }
     __syncthreads();
   }
-  for (; i + U <= s1; i += U) {
+  for (; i + US <= s1; i += US) {
     if (i != s0) weights(i);
+    bf16x8_t xv[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) xv[u] = input(i + u);
+    for (int u = 0; u < U; ++u) xv[u] = input(i + u * SP);
 #pragma unroll
     for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[u], xv[u], acc, 0, 0, 0);
   }
-  for (; i < s1; ++i)
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_nontemporal_load(w + (int64_t)i * 128), input(i), acc, 0, 0, 0);
-  if (r == 0) {
+  // the rest together as well: steps past the run's end request its last again and count as zeros
+  auto rest = [&](auto count) __attribute__((always_inline)) {
+    constexpr int N = decltype(count)::value;
+    bf16x8_t xv[N];
+#pragma unroll
+    for (int u = 0; u < N; ++u) wv[u] = __builtin_nontemporal_load(w + (int64_t)(min(i + u * SP + sub, s1 - 1) - sub) * 128);
+#pragma unroll
+    for (int u = 0; u < N; ++u) xv[u] = input(min(i + u * SP + sub, s1 - 1) - sub);
+#pragma unroll
+    for (int u = 0; u < N; ++u) {
+      if (i + u * SP + sub >= s1)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) wv[u][e] = xv[u][e] = (bf16_t)0.0f;
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[u], xv[u], acc, 0, 0, 0);
+    }
+  };
+  if (s1 - i > US / 2) rest(std::integral_constant<int, U>{});
+  else if (i < s1) rest(std::integral_constant<int, U / 2>{});
+  // lane (c, r): rows 4 c .. + 3 of the instruction against column r, which is theirs where r / RW is 4 c / RW
+  if (r == 4 * c / RW * RW) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) part[wave][4 * c + j] = acc[j];
   }
   __syncthreads();
-  if (tid >= 16) return;
+  if (tid >= RW) return;
   float sum = 0.0f;
 #pragma unroll
-  for (int v = 0; v < NW; ++v) sum += part[v][tid];
+  for (int v = 0; v < NW; ++v) {
+    float one = part[v][tid];
+#pragma unroll
+    for (int j = 1; j < SP; ++j) one += part[v][j * RW + tid];
+    sum += one;
+  }
   const int row = local + tid;
   const int64_t y0 = blockIdx.y * a.y_batch;
-  if constexpr (OUT == DENSE_STORE) {
+  if constexpr (OUT == DENSE_STORE && RW == 16) {
     if (s.act == DENSE_GLU) {
       const float up = __shfl_down(sum, 8, 16);
       if (tid < 8 && local / 2 + tid < s.glu_rows) store_one<bf16_t>(s, y0, 0, local / 2 + tid, glu<false>(sum, up));
@@ -400,24 +429,36 @@ __global__ __launch_bounds__(256) void dense_pack_kernel(const S* __restrict__ s
 
 constexpr int kFewTokens = 32;
 
-template <int OUT>
-int launch_one(const DenseArgs& a, int64_t rows, hipStream_t st) {
-  const dim3 g((unsigned)(rows / 16), (unsigned)a.batch);
-  if constexpr (OUT == DENSE_RESIDUAL) {
-    if (a.gate_o) {
-      const size_t lds = (size_t)a.gate_k * 2;
-      if (a.k > 8192) hipLaunchKernelGGL((dense_one_kernel<16, OUT, true>), g, dim3(1024), lds, st, a);
-      else if (a.k > 1024) hipLaunchKernelGGL((dense_one_kernel<8, OUT, true>), g, dim3(512), lds, st, a);
-      else hipLaunchKernelGGL((dense_one_kernel<4, OUT, true>), g, dim3(256), lds, st, a);
-      AWQ_HIP_TRY(hipGetLastError());
-      return AWQ_OK;
-    }
+template <int OUT, bool GATED, int RW>
+void launch_one_rows(const DenseArgs& a, int64_t rows, size_t lds, hipStream_t st) {
+  const dim3 g((unsigned)(rows / RW), (unsigned)a.batch);
+  if (a.k > 8192) hipLaunchKernelGGL((dense_one_kernel<16, OUT, GATED, RW>), g, dim3(1024), lds, st, a);
+  else if (a.k > 1024) hipLaunchKernelGGL((dense_one_kernel<8, OUT, GATED, RW>), g, dim3(512), lds, st, a);
+  else hipLaunchKernelGGL((dense_one_kernel<4, OUT, GATED, RW>), g, dim3(256), lds, st, a);
+}
+
+template <int OUT, bool GATED>
+int launch_one_as(const DenseArgs& a, int64_t rows, hipStream_t st) {
+  const size_t lds = GATED ? (size_t)a.gate_k * 2 : 0;
+  // Up to 2,048 rows 16 of them a workgroup leave half of the compute units or more without one, and a unit takes in no more than
+  // about 30 KB a us.  8 rows against 16: 1,024 x 4,096 4.8 and 6.1 us, 1,536 x 6,144 6.7 and 8.9, 2,048 x 8,192 9.6 and 11.8, 1,024 x
+  // 16,384 12.2 and 17.8; from 2,304 rows on 16 are faster (2,304 x 9,216 13.9 against 15.3, 3,072 x 3,072 6.4 against 7.7), and with
+  // up to 1,024 inputs neither is (3.5).  Both rows of a gated pair, and the rows of a candidate, are in one workgroup of 16.
+  bool eight = OUT != DENSE_ARGMAX && a.k > 1024 && rows * a.batch <= 2048;
+  for (int i = 0; i < a.n_seg; ++i) eight = eight && a.seg[i].act != DENSE_GLU;
+  if constexpr (OUT != DENSE_ARGMAX) {
+    if (eight) launch_one_rows<OUT, GATED, 8>(a, rows, lds, st);
   }
-  if (a.k > 8192) hipLaunchKernelGGL((dense_one_kernel<16, OUT, false>), g, dim3(1024), 0, st, a);
-  else if (a.k > 1024) hipLaunchKernelGGL((dense_one_kernel<8, OUT, false>), g, dim3(512), 0, st, a);
-  else hipLaunchKernelGGL((dense_one_kernel<4, OUT, false>), g, dim3(256), 0, st, a);
+  if (!eight) launch_one_rows<OUT, GATED, 16>(a, rows, lds, st);
   AWQ_HIP_TRY(hipGetLastError());
   return AWQ_OK;
+}
+
+template <int OUT>
+int launch_one(const DenseArgs& a, int64_t rows, hipStream_t st) {
+  if constexpr (OUT == DENSE_RESIDUAL)
+    if (a.gate_o) return launch_one_as<OUT, true>(a, rows, st);
+  return launch_one_as<OUT, false>(a, rows, st);
 }
 
 // 32 rows per workgroup read the tokens half as often, 16 make twice the workgroups: 8,192 x 1,024 at 9 tokens 6.9 against 5.2 us,

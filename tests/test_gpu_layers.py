@@ -128,6 +128,27 @@ def test_binary32_products_at_the_edges_of_tiles(awq, lib, dev, tokens, rows, k)
             assert np.abs(got - want).max() < 8 * k ** 0.5 * 2.0 ** -24
 
 
+@pytest.mark.parametrize("k", [64, 192, 1024, 1088, 1152, 2048, 2112, 4160, 8192, 8256, 12352])
+@pytest.mark.parametrize("rows", [1, 9, 1000, 2048, 2049])
+def test_products_of_one_token(awq, lib, dev, rows, k):
+    """8 and 16 rows per workgroup, 4, 8 and 16 wavefronts, runs of whole turns and every kind of rest, wavefronts without a
+    step.  The operands are exact: a sum of k products in binary32 is off by about sqrt(k) roundings of 2^-24 of its size"""
+    print("one token", rows, k, flush=True)
+    rng = np.random.default_rng(rows + k)
+    block = dev.torch.zeros((rows + 255) // 256 * 256 * k, dtype=dev.torch.bfloat16, device="cuda")
+    w, wv = dev.act(rng.standard_normal((rows, k)) / k ** 0.5, False)
+    awq.check(lib.awq_dense_pack(w.data_ptr(), 0, rows, k, block.data_ptr(), k, 0, 0, 0, dev.stream))
+    x, xv = dev.act(rng.standard_normal((1, k)), False)
+    y = dev.empty((2, rows), True)
+    a = awq.AwqDenseArgs()
+    a.w, a.k, a.tokens, a.n_segments, a.out = block.data_ptr(), k, 1, 1, awq.DENSE_F32
+    a.segment[0] = awq.AwqDenseSegment(x.data_ptr(), y.data_ptr(), k, rows, 0, rows, 0, 0, 0, 0)
+    awq.check(lib.awq_dense(ctypes.byref(a), 0, dev.stream))
+    got = dev.host(y)
+    assert np.isnan(got[1]).all()
+    assert np.abs(got[0] - (xv @ wv.T)[0]).max() < 8 * k ** 0.5 * 2.0 ** -24
+
+
 @pytest.mark.parametrize("tokens", [2, 15, 16, 17, 24, 25, 31, 32])
 @pytest.mark.parametrize("rows,k", [(1, 64), (47, 320), (300, 1088), (264, 8256), (8200, 192), (16400, 64)])
 def test_products_of_few_tokens(awq, lib, dev, tokens, rows, k):
