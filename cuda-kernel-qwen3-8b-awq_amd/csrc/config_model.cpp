@@ -193,7 +193,9 @@ int ConfigModel::logits_of(const float* x, const int32_t* which, int64_t n, bool
   a.w1 = final_norm;
   a.out1 = head_in;
   a.ld = ld;
-  if (int rc = launch_norm_conv(a, f32, stream)) return rc;
+  const bool fused = sample && dense_norm_fused(a, f32);
+  if (!fused)
+    if (int rc = launch_norm_conv(a, f32, stream)) return rc;
   DenseArgs d;
   d.w = head;
   d.k = ld;
@@ -211,7 +213,7 @@ int ConfigModel::logits_of(const float* x, const int32_t* which, int64_t n, bool
     d.seg[0].act = DENSE_SOFTCAP;
     d.seg[0].act_pos = softcap;
   }
-  return launch_dense(d, f32, stream);
+  return launch_dense(d, f32, stream, fused ? &a : nullptr);
 }
 
 int ConfigModel::enqueue_step(StepKind kind, int64_t) {

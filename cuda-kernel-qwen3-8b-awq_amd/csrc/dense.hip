@@ -1,5 +1,6 @@
 // Dense products of bfloat16 weights with one token or many, packing of weights, the launch of any product (layers.hpp).
 #include "dense_device.hpp"
+#include "lane_sums.hpp"
 
 #include <math.h>
 
@@ -14,12 +15,99 @@ namespace {
 // Eight steps of a wavefront are requested at once, and what is left of its run as well: one by one 1,536 rows of 1,536 inputs took
 // 5.7 us, now 4.0, 1,152 of 1,152 4.9 and 3.6.  Requesting the next eight ahead of these products cost more in wavefronts per unit
 // (81 registers instead of 62) than it gained: 28,672 x 4,096 40 -> 44 us.
-// GATED: the first gate_k inputs are formed here, RMS norm of o times w times sigmoid(g) (token_ops.hip has it as a
+// IN_GATED: the first gate_k inputs are formed here, RMS norm of o times w times sigmoid(g) (token_ops.hip has it as a
 // launch of its own for many tokens): every workgroup normalises for itself while its first weights are on their way.
-template <int NW, int OUT, bool GATED, int RW>
-__global__ __launch_bounds__(NW * 64) void dense_one_kernel(DenseArgs a) {
+// IN_NORMED: all inputs are formed here, the grouped norms and the convolution of NormConvArgs (norm_conv4_kernel in token_ops.hip),
+// the first norm's for segment 0, the second's for segment 1.  A launch between two products costs 3.5 to 4 us whatever it does, the
+// norms in every workgroup about two: Kugilix's q, k, v and W_up at width 1,024 8.8 us with the launch ahead, now 6.6; with the row
+// requested behind the weights, and the statistic through LDS, 7.4 (a compute unit's requests are served in order).
+constexpr int kFusedTaps = 4;
+enum OneInput { IN_READ, IN_GATED, IN_NORMED };
+
+// A group of the norm is a wavefront's, at most four channels a lane.  Everything is requested ahead of the statistic and in two
+// parts, so that the first of the weights can go between them; the inputs ahead of the pass for both parities, since which one it
+// is comes out of memory too.
+template <int NW, int TAPS>
+struct NormedInput {
+  static constexpr int BACK = TAPS > 0 ? TAPS - 1 : 0, KN = TAPS > 0 ? TAPS : 1, HN = BACK > 0 ? BACK : 1;
+  const NormConvArgs& a;
+  const bool conv;
+  const float* const w;
+  const int part, lane, wave;
+  int pos = 0, par = 0;
+  f32x4_t x, wv, taps[KN], past[2][HN];
+  __device__ __forceinline__ NormedInput(const NormConvArgs& n, bool second)
+      : a(n), conv(TAPS > 0 && !second), w(second ? n.w2 : n.w1), part((int)n.width / n.groups), lane(threadIdx.x & 63),
+        wave(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) {}
+  __device__ __forceinline__ bool mine(int g) const { return g < a.groups && 4 * lane < part; }
+  __device__ __forceinline__ void request_row(int g) {
+    x = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    if (mine(g)) x = *reinterpret_cast<const f32x4_t*>(a.x + g * part + 4 * lane);
+    if (conv) pos = a.pos.position(), par = a.pos.parity();
+  }
+  __device__ __forceinline__ void request_constants(int g) {
+    if (!mine(g)) return;
+    const int c = g * part + 4 * lane;
+    wv = *reinterpret_cast<const f32x4_t*>(w + c);
+    if (conv) {
+#pragma unroll
+      for (int i = 0; i < TAPS; ++i) taps[i] = *reinterpret_cast<const f32x4_t*>(a.conv + (int64_t)c * TAPS + 4 * i);
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int j = 0; j < BACK; ++j) past[p][j] = *reinterpret_cast<const f32x4_t*>(a.state[p] + (int64_t)j * a.width + c);
+    }
+  }
+  __device__ __forceinline__ void finish(int g, bool keeps, bf16_t* in) {
+    float sq = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) sq = __builtin_fmaf(x[e], x[e], sq);
+    const float inv = 1.0f / sqrtf(lanes::sum(sq) / (float)part + a.eps);
+    if (!mine(g)) return;
+    const int c = g * part + 4 * lane;
+    const f32x4_t h = x * inv * wv;
+    f32x4_t y = h;
+    if (conv) {
+      f32x4_t before[HN];
+#pragma unroll
+      for (int j = 0; j < BACK; ++j) {
+        before[j] = par ? past[1][j] : past[0][j];
+        if (pos - BACK + j < 0) before[j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {  // four channels of TAPS taps each, contiguous
+        auto tap = [&](int j) { return taps[(e * TAPS + j) >> 2][(e * TAPS + j) & 3]; };
+#pragma unroll
+        for (int j = 0; j < BACK; ++j) y[e] = __builtin_fmaf(tap(j), before[j][e], y[e]);
+        y[e] = __builtin_fmaf(tap(BACK), h[e], y[e]);
+      }
+      if (keeps) {
+        float* const after = a.state[par ^ 1] + c;
+#pragma unroll
+        for (int j = 0; j + 1 < BACK; ++j) *reinterpret_cast<f32x4_t*>(after + (int64_t)j * a.width) = before[j + 1];
+        *reinterpret_cast<f32x4_t*>(after + (int64_t)(BACK - 1) * a.width) = h;
+      }
+    }
+    bf16x4_t o;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = (bf16_t)y[e];
+    *reinterpret_cast<bf16x4_t*>(in + c) = o;
+  }
+  __device__ __forceinline__ void rest(bool keeps, int k, bf16_t* in) {
+    for (int g = wave + NW; g < a.groups; g += NW) {
+      request_row(g);
+      request_constants(g);
+      finish(g, keeps, in);
+    }
+    for (int c = (int)a.width + (int)threadIdx.x; c < k; c += NW * 64) in[c] = (bf16_t)0.0f;
+    __syncthreads();
+  }
+};
+
+template <int NW, int OUT, int IN, int RW, int TAPS = 0>
+__global__ __launch_bounds__(NW * 64) void dense_one_kernel(DenseArgs a, std::conditional_t<IN == IN_NORMED, NormConvArgs, std::false_type> norm) {
   constexpr int SP = 16 / RW;  // steps of an instruction
-  extern __shared__ __attribute__((aligned(16))) bf16_t gated[];  // [gate_k]
+  extern __shared__ __attribute__((aligned(16))) bf16_t formed[];  // the inputs that are formed here
   __shared__ float part[NW][16];
   __shared__ float squares[NW];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -38,7 +126,7 @@ __global__ __launch_bounds__(NW * 64) void dense_one_kernel(DenseArgs a) {
                       ((int64_t)(row0 >> 5) * (a.k >> 4) + (c >> 1) + 2 * sub) * 64 + 32 * (c & 1) + (row0 & (32 - RW)) + r % RW;
   const bf16x8_t* x = reinterpret_cast<const bf16x8_t*>(reinterpret_cast<const bf16_t*>(s.x) + blockIdx.y * a.x_batch) + c + 4 * sub;
   f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-  constexpr int U = 8;
+  constexpr int U = IN == IN_NORMED ? 4 : 8;
   constexpr int US = U * SP;
   bf16x8_t wv[U];
   auto weights = [&](int i) __attribute__((always_inline)) {
@@ -46,12 +134,24 @@ __global__ __launch_bounds__(NW * 64) void dense_one_kernel(DenseArgs a) {
     for (int u = 0; u < U; ++u) wv[u] = __builtin_nontemporal_load(w + (int64_t)(i + u * SP) * 128);
   };
   auto input = [&](int i) __attribute__((always_inline)) {
-    if (GATED && (i + sub) * 32 < a.gate_k) return reinterpret_cast<const bf16x8_t*>(gated)[(i + sub) * 4 + c];
+    if (IN == IN_NORMED || (IN == IN_GATED && (i + sub) * 32 < a.gate_k)) return reinterpret_cast<const bf16x8_t*>(formed)[(i + sub) * 4 + c];
     return x[i * 4];
   };
   int i = s0;
-  if (i + US <= s1) weights(i);
-  if constexpr (GATED) {
+  if constexpr (IN == IN_NORMED) {
+    NormedInput<NW, TAPS> in(norm, a.n_seg > 1 && row0 >= a.start[1]);
+    in.request_row(in.wave);
+    __builtin_amdgcn_sched_barrier(0);
+    in.request_constants(in.wave);
+    __builtin_amdgcn_sched_barrier(0);
+    if (i + US <= s1) weights(i);
+    __builtin_amdgcn_sched_barrier(0);
+    in.finish(in.wave, blockIdx.x == 0, formed);
+    in.rest(blockIdx.x == 0, (int)a.k, formed);
+  } else {
+    if (i + US <= s1) weights(i);
+  }
+  if constexpr (IN == IN_GATED) {
     constexpr int NT = NW * 64;
     const bf16_t* gate = reinterpret_cast<const bf16_t*>(a.gate_g);
     float sq = 0.0f;
@@ -76,7 +176,7 @@ __global__ __launch_bounds__(NW * 64) void dense_one_kernel(DenseArgs a) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) y[e] = (bf16_t)(o[e] * inv * gw[e] * sigmoid_exact((float)g[e]));
       }
-      *reinterpret_cast<bf16x4_t*>(gated + j) = y;
+      *reinterpret_cast<bf16x4_t*>(formed + j) = y;
     }
     __syncthreads();
   }
@@ -429,17 +529,18 @@ __global__ __launch_bounds__(256) void dense_pack_kernel(const S* __restrict__ s
 
 constexpr int kFewTokens = 32;
 
-template <int OUT, bool GATED, int RW>
+template <int OUT, int IN, int RW>
 void launch_one_rows(const DenseArgs& a, int64_t rows, size_t lds, hipStream_t st) {
   const dim3 g((unsigned)(rows / RW), (unsigned)a.batch);
-  if (a.k > 8192) hipLaunchKernelGGL((dense_one_kernel<16, OUT, GATED, RW>), g, dim3(1024), lds, st, a);
-  else if (a.k > 1024) hipLaunchKernelGGL((dense_one_kernel<8, OUT, GATED, RW>), g, dim3(512), lds, st, a);
-  else hipLaunchKernelGGL((dense_one_kernel<4, OUT, GATED, RW>), g, dim3(256), lds, st, a);
+  const std::false_type no;
+  if (a.k > 8192) hipLaunchKernelGGL((dense_one_kernel<16, OUT, IN, RW>), g, dim3(1024), lds, st, a, no);
+  else if (a.k > 1024) hipLaunchKernelGGL((dense_one_kernel<8, OUT, IN, RW>), g, dim3(512), lds, st, a, no);
+  else hipLaunchKernelGGL((dense_one_kernel<4, OUT, IN, RW>), g, dim3(256), lds, st, a, no);
 }
 
-template <int OUT, bool GATED>
+template <int OUT, int IN>
 int launch_one_as(const DenseArgs& a, int64_t rows, hipStream_t st) {
-  const size_t lds = GATED ? (size_t)a.gate_k * 2 : 0;
+  const size_t lds = IN == IN_GATED ? (size_t)a.gate_k * 2 : 0;
   // Up to 2,048 rows 16 of them a workgroup leave half of the compute units or more without one, and a unit takes in no more than
   // about 30 KB a us.  8 rows against 16: 1,024 x 4,096 4.8 and 6.1 us, 1,536 x 6,144 6.7 and 8.9, 2,048 x 8,192 9.6 and 11.8, 1,024 x
   // 16,384 12.2 and 17.8; from 2,304 rows on 16 are faster (2,304 x 9,216 13.9 against 15.3, 3,072 x 3,072 6.4 against 7.7), and with
@@ -447,9 +548,9 @@ int launch_one_as(const DenseArgs& a, int64_t rows, hipStream_t st) {
   bool eight = OUT != DENSE_ARGMAX && a.k > 1024 && rows * a.batch <= 2048;
   for (int i = 0; i < a.n_seg; ++i) eight = eight && a.seg[i].act != DENSE_GLU;
   if constexpr (OUT != DENSE_ARGMAX) {
-    if (eight) launch_one_rows<OUT, GATED, 8>(a, rows, lds, st);
+    if (eight) launch_one_rows<OUT, IN, 8>(a, rows, lds, st);
   }
-  if (!eight) launch_one_rows<OUT, GATED, 16>(a, rows, lds, st);
+  if (!eight) launch_one_rows<OUT, IN, 16>(a, rows, lds, st);
   AWQ_HIP_TRY(hipGetLastError());
   return AWQ_OK;
 }
@@ -457,8 +558,18 @@ int launch_one_as(const DenseArgs& a, int64_t rows, hipStream_t st) {
 template <int OUT>
 int launch_one(const DenseArgs& a, int64_t rows, hipStream_t st) {
   if constexpr (OUT == DENSE_RESIDUAL)
-    if (a.gate_o) return launch_one_as<OUT, true>(a, rows, st);
-  return launch_one_as<OUT, false>(a, rows, st);
+    if (a.gate_o) return launch_one_as<OUT, IN_GATED>(a, rows, st);
+  return launch_one_as<OUT, IN_READ>(a, rows, st);
+}
+
+template <int OUT>
+int launch_one_normed(const DenseArgs& a, const NormConvArgs& n, int64_t rows, hipStream_t st) {
+  const dim3 g((unsigned)(rows / 16));
+  const size_t lds = (size_t)a.k * 2;
+  if (n.conv) hipLaunchKernelGGL((dense_one_kernel<8, OUT, IN_NORMED, 16, kFusedTaps>), g, dim3(512), lds, st, a, n);
+  else hipLaunchKernelGGL((dense_one_kernel<8, OUT, IN_NORMED, 16>), g, dim3(512), lds, st, a, n);
+  AWQ_HIP_TRY(hipGetLastError());
+  return AWQ_OK;
 }
 
 // 32 rows per workgroup read the tokens half as often, 16 make twice the workgroups: 8,192 x 1,024 at 9 tokens 6.9 against 5.2 us,
@@ -602,7 +713,15 @@ int launch_dense_pack(const void* src, bool src_f32, int64_t rows, int64_t cols,
   return AWQ_OK;
 }
 
-int launch_dense(const DenseArgs& args, bool f32, hipStream_t st) {
+// Up to 2,048 values, where every workgroup's reading of row, weights, taps and state (36 bytes a value) costs as much as the launch:
+// Kugilix, 64 tokens after 100, with it and without: width 1,280 13.5 and 14.6 ms, 1,664 15.6 and 16.1, 2,048 18.4 and 18.5.
+bool dense_norm_fused(const NormConvArgs& n, bool f32) {
+  const int64_t part = n.groups > 0 && n.width % n.groups == 0 ? n.width / n.groups : 0;
+  return !f32 && n.M == 1 && n.width <= 2048 && n.groups >= 4 && part % 4 == 0 && part > 0 && part <= 256 && !n.rows && n.ld % kDenseKAlign == 0 &&
+         (!n.conv || n.taps == kFusedTaps) && (((uintptr_t)n.x | (uintptr_t)n.w1 | (uintptr_t)n.w2 | (uintptr_t)n.conv) & 15) == 0;
+}
+
+int launch_dense(const DenseArgs& args, bool f32, hipStream_t st, const NormConvArgs* norm) {
   DenseArgs a = args;
   AWQ_REQUIRE(a.w && a.M >= 1 && a.k > 0 && a.k % kDenseKAlign == 0, "bad product");
   AWQ_REQUIRE(a.n_seg >= 1 && a.n_seg <= kDenseSegments, "too few or too many segments");
@@ -635,6 +754,12 @@ int launch_dense(const DenseArgs& args, bool f32, hipStream_t st) {
   }
   AWQ_REQUIRE(a.out >= DENSE_STORE && a.out <= DENSE_ARGMAX, "unknown output");
   AWQ_REQUIRE(a.out != DENSE_ARGMAX || (a.M == 1 && a.best), "sampling takes one token");
+  if (norm) {
+    AWQ_REQUIRE(dense_norm_fused(*norm, f32) && a.M == 1 && a.k == norm->ld && a.batch == 1 && !a.gate_o && a.n_seg <= (norm->w2 ? 2 : 1) &&
+                    (a.out == DENSE_STORE || a.out == DENSE_ARGMAX) && norm->x && norm->w1 && (!norm->conv || (norm->state[0] && norm->state[1])),
+                "the norm cannot be part of this product");
+    return a.out == DENSE_STORE ? launch_one_normed<DENSE_STORE>(a, *norm, rows, st) : launch_one_normed<DENSE_ARGMAX>(a, *norm, rows, st);
+  }
   if (f32) return a.M == 1 ? launch_dense_one_f32(a, rows, st) : launch_dense_many_f32(a, rows, st);
   switch (a.out) {
     case DENSE_STORE: return a.M == 1 ? launch_one<DENSE_STORE>(a, rows, st) : launch_many<DENSE_STORE>(a, rows, st);

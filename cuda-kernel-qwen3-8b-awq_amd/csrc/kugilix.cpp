@@ -329,25 +329,26 @@ int KugilixEngine::run_pass(bool one, const int32_t* ids, int64_t M, PassPos pos
     const LayerDev& L = layers[r.layer];
     void* const cat = b.cat[r.layer];
     char* const mid = (char*)cat + L.mixed_k * unit();
-    {
-      NormConvArgs a;
-      a.x = b.x;
-      a.M = M;
-      a.width = W;
-      a.groups = spec.groups;
-      a.eps = spec.eps;
-      a.w1 = L.norm1;
-      a.conv = L.conv;
-      a.taps = spec.taps;
-      a.state[0] = r.conv_state[0];
-      a.state[1] = r.conv_state[1];
-      a.out1 = b.h;
-      a.w2 = L.norm2;
-      a.out2 = b.n;
-      a.ld = ld;
-      a.pos = pos;
-      if (int rc = launch_norm_conv(a, f32, stream)) return rc;
-    }
+    NormConvArgs norm;
+    norm.x = b.x;
+    norm.M = M;
+    norm.width = W;
+    norm.groups = spec.groups;
+    norm.eps = spec.eps;
+    norm.w1 = L.norm1;
+    norm.conv = L.conv;
+    norm.taps = spec.taps;
+    norm.state[0] = r.conv_state[0];
+    norm.state[1] = r.conv_state[1];
+    norm.out1 = b.h;
+    norm.w2 = L.norm2;
+    norm.out2 = b.n;
+    norm.ld = ld;
+    norm.pos = pos;
+    // a single token's norms are part of the product below
+    const bool norm_fused = dense_norm_fused(norm, f32);
+    if (!norm_fused)
+      if (int rc = launch_norm_conv(norm, f32, stream)) return rc;
     {
       DenseArgs a;
       a.w = L.w_in;
@@ -378,7 +379,7 @@ int KugilixEngine::run_pass(bool one, const int32_t* ids, int64_t M, PassPos pos
         up.act_pos = L.act_pos;
         up.act_neg = L.act_neg;
       }
-      if (int rc = launch_dense(a, f32, stream)) return rc;
+      if (int rc = launch_dense(a, f32, stream, norm_fused ? &norm : nullptr)) return rc;
     }
     const char* gate = nullptr;
     bool gate_fused = false;

@@ -123,7 +123,11 @@ enum DensePack {
 };
 int launch_dense_pack(const void* src, bool src_f32, int64_t rows, int64_t cols, void* w, int64_t k_padded, int64_t row0,
                       int64_t col0, bool f32, hipStream_t st, int form = PACK_PLAIN);
-int launch_dense(const DenseArgs& a, bool f32, hipStream_t st);
+struct NormConvArgs;
+// norm (one token, where dense_norm_fused): launch_norm_conv is part of the product, out1 the input of segment 0, out2 of segment 1;
+// neither is written, and what the segments name as x is not read
+int launch_dense(const DenseArgs& a, bool f32, hipStream_t st, const NormConvArgs* norm = nullptr);
+bool dense_norm_fused(const NormConvArgs& n, bool f32);
 bool dense_gate_fused(int64_t n, int64_t k_padded, int64_t M, bool f32);
 
 // --- per-token operators (token_ops.hip) -------------------------------------------------------------------

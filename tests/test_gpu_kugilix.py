@@ -227,3 +227,26 @@ def test_many_logits_come_out_as_few_do(awq, torch_gpu, tmp_path):
         many = logits(range(n))
         assert many.nbytes >= 4 << 20 and np.array_equal(many, few[:n]), n
     eng.close()
+
+
+@pytest.mark.parametrize("width,groups", [(640, 10), (1024, 4), (168, 6), (2048, 16)])
+def test_single_tokens_whose_norms_are_part_of_the_product(awq, torch_gpu, tmp_path, width, groups):
+    """groups of 28 to 256 values, more of them than wavefronts, inputs padded behind the width; windows of two parts and a new one"""
+    cfg = km.model(width, 96, [attention_of(70), km.lightning(2, 16, 16, [0.9, 0.99], ff=64), attention_of(None)], groups=groups, taps=4)
+    w = km.weights(cfg, width)
+    km.write(str(tmp_path), cfg, w)
+    tokens = np.random.default_rng(2).integers(0, 96, 140).tolist()
+    want = plain.forward(cfg, w, tokens)
+    eng = awq.open_model(str(tmp_path), dtype="bfloat16", max_positions=200)
+    got = np.concatenate([eng.forward([t], [0]) for t in tokens])
+    assert km.rms_error(got, want) < LIMIT["bfloat16"]
+    eng.reset()
+    out = eng.generateResponse(tokens[:60], 70)   # the head's norm with it, in captured steps
+    z = plain.forward(cfg, w, tokens[:60] + out[:-1])[59:]
+    short = z.max(axis=1) - z[np.arange(len(out)), out]
+    assert short.max() <= 6 * LIMIT["bfloat16"] * np.std(z)
+    eng.close()
+
+
+def attention_of(window):
+    return km.attention(2, 1, 64, 64, window, ff=128)
