@@ -168,6 +168,7 @@ struct KugilixEngine final : ConfigModel {
   std::vector<LayerRun> runs;
   Buffers step, pass;
   float* attn_parts = nullptr;
+  int32_t* attn_done = nullptr;
 
   const char* architecture() const override { return "Kugilix"; }
   int load_layers(Loader& ldr) override;
@@ -297,7 +298,7 @@ int KugilixEngine::make_runs() {
       runs.push_back(r);
     }
   }
-  int64_t parts = 4;
+  int64_t parts = 4, heads = 1;
   for (LayerRun& r : runs) {
     const LayerSpec& s = spec.layers[r.layer];
     if (spec.taps > 1)
@@ -314,7 +315,9 @@ int KugilixEngine::make_runs() {
     if (int rc = zeroed(&r.k_cache, r.kl.elements() * unit())) return rc;
     if (int rc = zeroed(&r.v_cache, r.vl.elements() * unit())) return rc;
     parts = std::max(parts, window_parts_floats(s.heads, s.vdim, s.window, max_pos));
+    heads = std::max<int64_t>(heads, s.heads);
   }
+  if (int rc = zeroed((void**)&attn_done, heads * 4)) return rc;
   return zeroed((void**)&attn_parts, parts * 4);
 }
 
@@ -406,6 +409,7 @@ int KugilixEngine::run_pass(bool one, const int32_t* ids, int64_t M, PassPos pos
       a.M = M;
       a.pos = pos;
       a.parts = attn_parts;
+      a.done = attn_done;
       a.len_bound = (int32_t)max_pos;
       if (int rc = launch_window_attention(a, f32, stream)) return rc;
     } else {

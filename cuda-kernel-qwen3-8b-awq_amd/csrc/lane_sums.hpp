@@ -47,4 +47,33 @@ __device__ __forceinline__ float maximum(float v) {
   return over<N>(v, Max());
 }
 
+// n lanes next to each other (8, 16, 32 or 64, the same in the whole wavefront), in every lane
+__device__ __forceinline__ float sum_of(float v, int n) {
+  v = sum<8>(v);
+  if (n > 8) v += from<0x140>(v);
+  if (n > 16) {
+    float a = v, b = v;
+    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+    v = a + b;
+  }
+  if (n > 32) {
+    float a = v, b = v;
+    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+    v = a + b;
+  }
+  return v;
+}
+// the lanes n, 2 n, .. apart (n: 8, 16 or 32), in every lane
+__device__ __forceinline__ float sum_apart(float v, int n) {
+  if (n <= 8) v += from<0x128>(v);  // rotated by 8 within 16
+  float a = v, b = v;
+  if (n <= 16) {
+    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+    v = a + b;
+    a = b = v;
+  }
+  asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+  return a + b;
+}
+
 }  // namespace lanes

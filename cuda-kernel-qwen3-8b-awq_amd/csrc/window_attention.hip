@@ -1,4 +1,5 @@
 // Attention over a sliding window with a distance bias (layers.hpp).
+#include "lane_sums.hpp"
 #include "query_attention.hpp"
 
 namespace {
@@ -114,7 +115,10 @@ __global__ __launch_bounds__(256) void window_query_kernel(WindowAttnArgs a) {
 // One token.  blockIdx.x: kv head and up to R of its query heads, blockIdx.y: 64 of the visible keys.  The rows a
 // workgroup needs are requested before anything else; every lane group normalises the queries for itself, and the
 // workgroup of the newest position takes its key and value from the projections and appends them.  A wavefront's
-// lane holds the weight of one key.  With more than one part a second launch adds the parts up.
+// lane holds the weight of one key.  With more than one part the workgroup that counts itself in last adds the parts up, where
+// the caller has counters, otherwise a second launch does: that costs 4 us.  One part of 8 heads of 128: 8.2 us
+// and the second launch's 4.0, now 6.5 for both (of which the sums over lanes through LDS took 1.2); 64 tokens of Kugilix at width 1,024
+// after 960, 15 parts and four such layers: 14.5 -> 12.5 ms.
 constexpr int kPartKeys = 64;
 
 __host__ __device__ inline int window_parts(int64_t window, int64_t max_pos) {
@@ -146,6 +150,40 @@ __device__ __forceinline__ void row_piece(const T* row, int at, int n, bool alig
   }
 }
 
+// A part's results leave the die and are read past its caches: another die's workgroup may add them up in the same launch.
+__device__ __forceinline__ void put_part(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ float get_part(const float* p) {
+  return __hip_atomic_load(const_cast<float*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// One head's parts, [maximum, sum, context] each, by a workgroup of 256; red: 256 floats of LDS
+template <typename T>
+__device__ __forceinline__ void combine_parts(const WindowAttnArgs& a, int h, int n_parts, int parts, float* red) {
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int64_t ps = 2 + a.vdim;
+  const float* p = a.parts + (int64_t)h * n_parts * ps;
+  // columns, and as many runs of parts next to each other as there are threads left
+  const int cols = min(256, a.vdim), runs = 256 / cols, run = tid / cols;
+  float m = -INFINITY, l = 0.0f;
+  for (int s = lane; s < parts; s += 64) m = fmaxf(m, get_part(p + s * ps));
+  m = lanes::maximum(m);
+  for (int s = lane; s < parts; s += 64) l = __builtin_fmaf(expf(get_part(p + s * ps) - m), get_part(p + s * ps + 1), l);
+  l = lanes::sum(l);
+  for (int c = tid % cols; c < (a.vdim + cols - 1) / cols * cols; c += cols) {
+    float x = 0.0f;
+    if (run < runs && c < a.vdim)
+#pragma unroll 4
+      for (int s = run; s < parts; s += runs) x = __builtin_fmaf(expf(get_part(p + s * ps) - m), get_part(p + s * ps + 2 + c), x);
+    red[tid] = x;
+    __syncthreads();
+    if (run == 0 && c < a.vdim) {
+      for (int i = 1; i < runs; ++i) x += red[tid + i * cols];
+      reinterpret_cast<T*>(a.ctx)[(int64_t)h * a.vdim + c] = (T)(x / l);
+    }
+    __syncthreads();
+  }
+}
+
 // U: cache rows of a lane, row length / 32
 template <typename T, int R, int U>
 __global__ __launch_bounds__(256) void window_decode_kernel(WindowAttnArgs a, int chunks) {
@@ -168,35 +206,44 @@ __global__ __launch_bounds__(256) void window_decode_kernel(WindowAttnArgs a, in
   const int tpv = vw >> 3, c0 = (tid % tpv) * 8, first = tid / tpv, step = 256 / tpv, uv = vw >> 5;
   const T* const kc = reinterpret_cast<const T*>(a.k_cache);
   const T* const vc = reinterpret_cast<const T*>(a.v_cache);
+  const int slot0 = b % a.kl.slots;
+  auto slot_of = [&](int key) {  // of a key of this part
+    const int s = slot0 + key - b;
+    return s < a.kl.slots ? s : s - a.kl.slots;
+  };
   Vec8<T> kv[U], vv[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int key = b + (u * 4 + wave) * kpw + sub;
-    if (u < uk && key < pos) kv[u] = *reinterpret_cast<const Vec8<T>*>(kc + ring_row(a.kl, g, key % a.kl.slots) + d0);
+    if (u < uk && key < pos) kv[u] = *reinterpret_cast<const Vec8<T>*>(kc + ring_row(a.kl, g, slot_of(key)) + d0);
   }
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     const int key = b + u * step + first;
-    if (u < uv && key < pos) vv[u] = *reinterpret_cast<const Vec8<T>*>(vc + ring_row(a.vl, g, key % a.vl.slots) + c0);
+    if (u < uv && key < pos) vv[u] = *reinterpret_cast<const Vec8<T>*>(vc + ring_row(a.vl, g, slot_of(key)) + c0);
   }
   const T* const proj = reinterpret_cast<const T*>(a.proj);
   const bool dim8 = (a.dim & 7) == 0, vdim8 = ((a.dim | a.vdim) & 7) == 0;
-  auto normalised = [&](const T* row, float (&x)[8]) {
-    row_piece(row, d0, a.dim, dim8, x);
+  float qv[R][8], kn[8] = {}, vn[8] = {};
+#pragma unroll
+  for (int r = 0; r < R; ++r) row_piece(proj + (int64_t)(h0 + min(r, nr - 1)) * a.dim, d0, a.dim, dim8, qv[r]);
+  if (newest) {
+    row_piece(proj + (int64_t)(a.heads + g) * a.dim, d0, a.dim, dim8, kn);
+    row_piece(proj + (int64_t)(a.heads + a.kv_heads) * a.dim + (int64_t)g * a.vdim, c0, a.vdim, vdim8, vn);
+  }
+  const float mul = a.scale * temperature(a, pos);  // (while the rows are on their way)
+  auto normalise = [&](float (&x)[8]) {
     float acc = 0.0f;
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc = __builtin_fmaf(x[i], x[i], acc);
-    for (int off = lpk >> 1; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
-    const float inv = 1.0f / sqrtf(acc / (float)a.dim + a.eps);
+    const float inv = 1.0f / sqrtf(lanes::sum_of(acc, lpk) / (float)a.dim + a.eps);
 #pragma unroll
     for (int i = 0; i < 8; ++i) x[i] = (float)(T)(x[i] * inv);
   };
-  float qv[R][8], kn[8] = {}, vn[8] = {};
 #pragma unroll
-  for (int r = 0; r < R; ++r) normalised(proj + (int64_t)(h0 + min(r, nr - 1)) * a.dim, qv[r]);
+  for (int r = 0; r < R; ++r) normalise(qv[r]);
   if (newest) {
-    normalised(proj + (int64_t)(a.heads + g) * a.dim, kn);
-    row_piece(proj + (int64_t)(a.heads + a.kv_heads) * a.dim + (int64_t)g * a.vdim, c0, a.vdim, vdim8, vn);
+    normalise(kn);
     Vec8<T> out;
     if (rz == 0 && tid < lpk) {
 #pragma unroll
@@ -209,7 +256,6 @@ __global__ __launch_bounds__(256) void window_decode_kernel(WindowAttnArgs a, in
       *reinterpret_cast<Vec8<T>*>(reinterpret_cast<T*>(a.v_cache) + ring_row(a.vl, g, pos % a.vl.slots) + c0) = out;
     }
   }
-  const float mul = a.scale * temperature(a, pos);
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     if (u >= uk) break;
@@ -222,7 +268,7 @@ __global__ __launch_bounds__(256) void window_decode_kernel(WindowAttnArgs a, in
       float dot = 0.0f;
 #pragma unroll
       for (int j = 0; j < 8; ++j) dot = __builtin_fmaf(qv[r][j], x[j], dot);
-      for (int off = lpk >> 1; off > 0; off >>= 1) dot += __shfl_xor(dot, off, 64);
+      dot = lanes::sum_of(dot, lpk);
       if (d0 == 0) sc[r][i] = dot;
     }
   }
@@ -232,16 +278,10 @@ __global__ __launch_bounds__(256) void window_decode_kernel(WindowAttnArgs a, in
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     const float s = lane < nk && r < nr ? sc[r][lane] * mul - a.slope[h0 + r] * (float)(pos - b - lane) : -INFINITY;
-    float m = s;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-    const float e = r < nr ? expf(s - m) : 0.0f;
-    float l = e;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) l += __shfl_xor(l, off, 64);
+    const float m = lanes::maximum(s), e = r < nr ? expf(s - m) : 0.0f;
     p[r] = e;
     pm[r] = m;
-    pl[r] = l;
+    pl[r] = lanes::sum(e);
   }
   float acc[R][8] = {};
 #pragma unroll
@@ -263,57 +303,47 @@ __global__ __launch_bounds__(256) void window_decode_kernel(WindowAttnArgs a, in
   for (int r = 0; r < R; ++r)
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      for (int off = tpv; off < 64; off <<= 1) acc[r][j] += __shfl_xor(acc[r][j], off, 64);
+      acc[r][j] = lanes::sum_apart(acc[r][j], tpv);
       if (lane < tpv) red[(wave * R + r) * vw + c0 + j] = acc[r][j];
     }
   __syncthreads();
   const int n_parts = gridDim.y;
+  const bool alone = n_parts == 1 || (a.done && parts == 1);
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     if (r >= nr) break;
     float* const mine = a.parts + ((int64_t)(h0 + r) * n_parts + part) * (2 + a.vdim);
     for (int c = tid; c < a.vdim; c += 256) {
       const float x = (red[r * vw + c] + red[(R + r) * vw + c]) + (red[(2 * R + r) * vw + c] + red[(3 * R + r) * vw + c]);
-      if (n_parts == 1)
-        reinterpret_cast<T*>(a.ctx)[(int64_t)(h0 + r) * a.vdim + c] = (T)(x / pl[r]);
-      else
-        mine[2 + c] = x;
+      if (alone) reinterpret_cast<T*>(a.ctx)[(int64_t)(h0 + r) * a.vdim + c] = (T)(x / pl[r]);
+      else put_part(mine + 2 + c, x);
     }
-    if (n_parts > 1 && tid == 0) mine[0] = pm[r], mine[1] = pl[r];
+    if (!alone && tid == 0) put_part(mine, pm[r]), put_part(mine + 1, pl[r]);
+  }
+  if (alone || !a.done) return;
+  // the parts are out of this die when the workgroup counts itself in; the last one finds all of them
+  __shared__ int last;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (tid == 0) {
+    last = __hip_atomic_fetch_add(a.done + blockIdx.x, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
+    if (last) __hip_atomic_store(a.done + blockIdx.x, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
+  }
+  __syncthreads();
+  if (!last) return;
+  for (int r = 0; r < nr; ++r) {
+    combine_parts<T>(a, h0 + r, n_parts, parts, red);
+    __syncthreads();
   }
 }
 
-// a workgroup per head; a part is [maximum, sum, context]
+// a workgroup per head
 template <typename T>
 __global__ __launch_bounds__(256) void window_combine_kernel(WindowAttnArgs a, int n_parts) {
   __shared__ float red[256];
-  const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
   const int pos = a.pos.position();
   const int parts = ((a.window > 0 ? min(a.window, pos + 1) : pos + 1) + kPartKeys - 1) / kPartKeys;
-  const int64_t ps = 2 + a.vdim;
-  const float* p = a.parts + (int64_t)h * n_parts * ps;
-  float m = -INFINITY, l = 0.0f;
-  for (int s = lane; s < parts; s += 64) m = fmaxf(m, p[s * ps]);
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-  for (int s = lane; s < parts; s += 64) l = __builtin_fmaf(expf(p[s * ps] - m), p[s * ps + 1], l);
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) l += __shfl_xor(l, off, 64);
-  // columns, and as many runs of parts next to each other as there are threads left
-  const int cols = min(256, a.vdim), runs = 256 / cols, run = tid / cols;
-  for (int c = tid % cols; c < (a.vdim + cols - 1) / cols * cols; c += cols) {
-    float x = 0.0f;
-    if (run < runs && c < a.vdim)
-#pragma unroll 4
-      for (int s = run; s < parts; s += runs) x = __builtin_fmaf(expf(p[s * ps] - m), p[s * ps + 2 + c], x);
-    red[tid] = x;
-    __syncthreads();
-    if (run == 0 && c < a.vdim) {
-      for (int i = 1; i < runs; ++i) x += red[tid + i * cols];
-      reinterpret_cast<T*>(a.ctx)[(int64_t)h * a.vdim + c] = (T)(x / l);
-    }
-    __syncthreads();
-  }
+  combine_parts<T>(a, blockIdx.x, n_parts, parts, red);
 }
 
 template <typename T, int R>
@@ -322,13 +352,13 @@ int launch_decode_rows(const WindowAttnArgs& a, hipStream_t st) {
   const int parts = window_parts(a.window, a.len_bound);
   AWQ_REQUIRE(parts >= 1 && parts <= 65535, "too many keys");
   const dim3 g((unsigned)(a.kv_heads * chunks), (unsigned)parts);
-  const size_t lds = sizeof(float) * 4 * R * a.vl.row;
+  const size_t lds = sizeof(float) * 4 * R * a.vl.row;  // (256 floats at least)
   const int row = std::max(a.kl.row, a.vl.row);
   if (row == 64) hipLaunchKernelGGL((window_decode_kernel<T, R, 2>), g, dim3(256), lds, st, a, chunks);
   else if (row == 128) hipLaunchKernelGGL((window_decode_kernel<T, R, 4>), g, dim3(256), lds, st, a, chunks);
   else hipLaunchKernelGGL((window_decode_kernel<T, R, 8>), g, dim3(256), lds, st, a, chunks);
   AWQ_HIP_TRY(hipGetLastError());
-  if (parts > 1) {
+  if (parts > 1 && !a.done) {
     hipLaunchKernelGGL(window_combine_kernel<T>, dim3((unsigned)a.heads), dim3(256), 0, st, a, parts);
     AWQ_HIP_TRY(hipGetLastError());
   }
