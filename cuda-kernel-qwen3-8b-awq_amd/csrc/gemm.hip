@@ -570,6 +570,8 @@ __device__ __forceinline__ int sk_wg_of(int64_t q, int64_t W, int G) {
   return b;
 }
 
+constexpr int EPI_PART = -1;  // rows split: a share of k only, FP32 sums to the workspace
+
 enum WideMode { WIDE_ROWS = 0, WIDE_K = 1, WIDE_ROWS_CUT = 2 };  // rows split (a tile per workgroup), k split, rows split with work cut evenly
 
 template <bool ZINT, int MODE, int EPI, int TT>
@@ -601,6 +603,10 @@ __global__ __launch_bounds__(256, (MODE == WIDE_K && TT == 4) ? 1 : ((MODE == WI
   do {
     // this piece: steps [s_lo, s_lo + steps) of the tile
     int s_lo = 0, steps = tile_steps;
+    if (MODE == WIDE_ROWS && EPI == EPI_PART) {  // share blockIdx.y of k
+      s_lo = tile_steps * (int)blockIdx.y / p.kz;
+      steps = tile_steps * ((int)blockIdx.y + 1) / p.kz - s_lo;
+    }
     if (CUT) {
       const int64_t q0 = (int64_t)tile * S2;
       const int pb = (int)((lo > q0 ? lo : q0) - q0), pe = (int)((hi < q0 + S2 ? hi : q0 + S2) - q0);
@@ -977,10 +983,27 @@ __global__ __launch_bounds__(256, (MODE == WIDE_K && TT == 4) ? 1 : ((MODE == WI
         const int row = rg0 * 16 + a * 32 + n;
 #pragma unroll
         for (int t = 0; t < TT; ++t) {
+          // Residuals some at a time: y may be res, so that a load behind a store of the same instance waits for its own trip to
+          // memory, 64 of them one after the other for 4,096 x 4,096 at 1,000 tokens (in a prompt pass 60 us, now 53).
+          constexpr int B = EPI == EPI_RESIDUAL ? (TT == 2 ? 16 : 4) : 16;
 #pragma unroll
-          for (int i = 0; i < 16; ++i) {
-            const int tok = t0 + t * 32 + (i >> 2) * 8 + kh * 4 + (i & 3);
-            if (tok < p.M) store_out<EPI, true>(p, tok, row, acc[a][t][i] * scf);
+          for (int i0 = 0; i0 < 16; i0 += B) {
+            auto token = [&](int i) { return t0 + t * 32 + ((i0 + i) >> 2) * 8 + kh * 4 + ((i0 + i) & 3); };
+            half_t before[B];
+            if (EPI == EPI_RESIDUAL) {
+#pragma unroll
+              for (int i = 0; i < B; ++i) before[i] = p.res[(int64_t)(token(i) < p.M ? token(i) : p.M - 1) * p.m + row];
+            }
+#pragma unroll
+            for (int i = 0; i < B; ++i) {
+              const int tok = token(i);
+              if (tok < p.M) {
+                const float v = acc[a][t][i0 + i] * scf;
+                if constexpr (EPI == EPI_PART) p.part[((int64_t)blockIdx.y * p.M + tok) * p.m + row] = v;
+                else if constexpr (EPI == EPI_RESIDUAL) p.y[(int64_t)tok * p.m + row] = before[i] + (half_t)v;  // Inference.cu:1149-1155
+                else store_out<EPI, true>(p, tok, row, v);
+              }
+            }
           }
         }
       }
@@ -1228,7 +1251,7 @@ __global__ __launch_bounds__(512) void reduce_norm_kernel(GemmParams p, const ha
       const float* part = p.part + row + at * 8;
       const half8_t r = *reinterpret_cast<const half8_t*>(p.res + row + at * 8);
       gv[c] = reinterpret_cast<const half8_t*>(gamma)[at];
-      float4_t a[4], b[4];  // kz is 2 or 4
+      float4_t a[4], b[4];  // kz is 2, 3 or 4
 #pragma unroll
       for (int z = 0; z < 4; ++z)
         if (z < p.kz) {
@@ -1320,6 +1343,15 @@ int launch_wide(const GemmParams& p, bool zint, int n_wgs, hipStream_t st) {
   }
   hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, p);
   if (KSPLIT && p.kz > 1) launch_reduce(p, st);
+  return AWQ_OK;
+}
+
+// rows split, a tile of 128 tokens and a share of k per workgroup
+int launch_wide_shares(const GemmParams& p, bool zint, hipStream_t st) {
+  const dim3 grid((unsigned)p.n_tiles, (unsigned)p.kz);
+  if (zint) hipLaunchKernelGGL((gemm_wide_kernel<true, WIDE_ROWS, EPI_PART, kWideTT>), grid, dim3(256), 0, st, p);
+  else hipLaunchKernelGGL((gemm_wide_kernel<false, WIDE_ROWS, EPI_PART, kWideTT>), grid, dim3(256), 0, st, p);
+  launch_reduce(p, st);
   return AWQ_OK;
 }
 
@@ -1450,6 +1482,20 @@ static WidePlan plan_wide(int64_t m, int64_t k, int64_t M, bool has_workspace) {
   if (k <= 4096 && tiles64 >= 128) return PLAN_ROWS_64;
   const int64_t pairs = tiles * (k / AWQ_BLOCK_K / kWideNH / 2);
   return has_workspace && pairs / 4 >= kSkWgs ? PLAN_ROWS_CUT : PLAN_ROWS;
+}
+
+// Shares of k of a product whose sums a second launch adds and norms (0: none).  Long k and too few tiles: as many shares as give
+// each compute unit one workgroup, three where two units' worth are then less than full.  Rows then cost no launch for their
+// norm (5.7 us), and nothing waits for another workgroup's sums.  4,096 x 12,288 with the launch that adds, against the k-split
+// workgroups up to 512 tokens and the work cut evenly above: 384 tokens 54 us (61), 512 61 (66), 640 73 (103), 768 91 (106), 1,000
+// 104 (119), 1,152 126 (150), 1,280 132 (160); from 1,281 on (176 tiles) a tile per workgroup is faster (1,536: 166 against 152).  At
+// k = 4,096 the sums' way through memory costs more than the tiles gain (1,000 tokens 48 us with two shares, 39 without).
+static int norm_shares(int64_t m, int64_t k, int64_t M) {
+  const int64_t tiles = (m + 255) / 256 * ((M + kWideTokens - 1) / kWideTokens);
+  if (k < 8192 || m > kNormRow || tiles < 48) return 0;
+  for (int kz : {4, 3, 2})
+    if (tiles * kz <= kSkWgs) return kz;
+  return tiles * 3 <= 2 * kSkWgs ? 3 : 0;
 }
 
 // room for a header and the partial sums of a product whose work is cut over workgroups (0: never cut)
@@ -1587,6 +1633,15 @@ int launch_gemm(const void* wq, const half_t* scale, const half_t* zp, int64_t m
     const int64_t part_bytes = workspace_bytes - kSkHeaderBytes;
     const bool room = workspace && kSkWgs * (int64_t)kSkTileFloats * 4 <= part_bytes;
     const WidePlan plan = plan_wide(m, k, M, room);
+    if (const int shares = norm_shares(m, k, M); norm && shares && epilogue == EPI_RESIDUAL && workspace && (int64_t)shares * M * m * 4 <= part_bytes) {
+      p.nr = (int32_t)nr;
+      p.n_tiles = (int32_t)tiles;
+      p.kz = shares;
+      p.part = (float*)ws_part;
+      if (int rc = launch_wide_shares(p, zp_integral, st)) return rc;
+      AWQ_HIP_TRY(hipGetLastError());
+      return AWQ_OK;
+    }
     if (plan != PLAN_K) {
       AWQ_REQUIRE(tiles < (1ll << 30), "too many output tiles");
       p.nr = (int32_t)nr;
