@@ -1,5 +1,6 @@
 // Dense products of bfloat16 weights with one token or many, packing of weights, the launch of any product (layers.hpp).
 #include "dense_device.hpp"
+#include "join_device.hpp"
 #include "lane_sums.hpp"
 
 #include <math.h>
@@ -22,7 +23,24 @@ namespace {
 // norms in every workgroup about two: Kugilix's q, k, v and W_up at width 1,024 8.8 us with the launch ahead, now 6.6; with the row
 // requested behind the weights, and the statistic through LDS, 7.4 (a compute unit's requests are served in order).
 constexpr int kFusedTaps = 4;
-enum OneInput { IN_READ, IN_GATED, IN_NORMED };
+// IN_JOINED, _2: all inputs are formed here, the end of the sublayer ahead (JoinArgs, one and two turns of the workgroup's threads).
+enum OneInput { IN_READ, IN_GATED, IN_NORMED, IN_JOINED, IN_JOINED_2 };
+template <int IN>
+struct OneExtra {
+  typedef std::false_type type;
+};
+template <>
+struct OneExtra<IN_NORMED> {
+  typedef NormConvArgs type;
+};
+template <>
+struct OneExtra<IN_JOINED> {
+  typedef JoinArgs type;
+};
+template <>
+struct OneExtra<IN_JOINED_2> {
+  typedef JoinArgs type;
+};
 
 // A group of the norm is a wavefront's, at most four channels a lane.  Everything is requested ahead of the statistic and in two
 // parts, so that the first of the weights can go between them; the inputs ahead of the pass for both parities, since which one it
@@ -105,7 +123,8 @@ struct NormedInput {
 };
 
 template <int NW, int OUT, int IN, int RW, int TAPS = 0>
-__global__ __launch_bounds__(NW * 64) void dense_one_kernel(DenseArgs a, std::conditional_t<IN == IN_NORMED, NormConvArgs, std::false_type> norm) {
+__global__ __launch_bounds__(NW * 64) void dense_one_kernel(DenseArgs a, typename OneExtra<IN>::type ahead) {
+  constexpr bool JOINED = IN == IN_JOINED || IN == IN_JOINED_2;
   constexpr int SP = 16 / RW;  // steps of an instruction
   extern __shared__ __attribute__((aligned(16))) bf16_t formed[];  // the inputs that are formed here
   __shared__ float part[NW][16];
@@ -126,7 +145,7 @@ __global__ __launch_bounds__(NW * 64) void dense_one_kernel(DenseArgs a, std::co
                       ((int64_t)(row0 >> 5) * (a.k >> 4) + (c >> 1) + 2 * sub) * 64 + 32 * (c & 1) + (row0 & (32 - RW)) + r % RW;
   const bf16x8_t* x = reinterpret_cast<const bf16x8_t*>(reinterpret_cast<const bf16_t*>(s.x) + blockIdx.y * a.x_batch) + c + 4 * sub;
   f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
-  constexpr int U = IN == IN_NORMED ? 4 : 8;
+  constexpr int U = IN == IN_NORMED || JOINED ? 4 : 8;
   constexpr int US = U * SP;
   bf16x8_t wv[U];
   auto weights = [&](int i) __attribute__((always_inline)) {
@@ -134,12 +153,12 @@ __global__ __launch_bounds__(NW * 64) void dense_one_kernel(DenseArgs a, std::co
     for (int u = 0; u < U; ++u) wv[u] = __builtin_nontemporal_load(w + (int64_t)(i + u * SP) * 128);
   };
   auto input = [&](int i) __attribute__((always_inline)) {
-    if (IN == IN_NORMED || (IN == IN_GATED && (i + sub) * 32 < a.gate_k)) return reinterpret_cast<const bf16x8_t*>(formed)[(i + sub) * 4 + c];
+    if (IN == IN_NORMED || JOINED || (IN == IN_GATED && (i + sub) * 32 < a.gate_k)) return reinterpret_cast<const bf16x8_t*>(formed)[(i + sub) * 4 + c];
     return x[i * 4];
   };
   int i = s0;
   if constexpr (IN == IN_NORMED) {
-    NormedInput<NW, TAPS> in(norm, a.n_seg > 1 && row0 >= a.start[1]);
+    NormedInput<NW, TAPS> in(ahead, a.n_seg > 1 && row0 >= a.start[1]);
     in.request_row(in.wave);
     __builtin_amdgcn_sched_barrier(0);
     in.request_constants(in.wave);
@@ -148,6 +167,11 @@ __global__ __launch_bounds__(NW * 64) void dense_one_kernel(DenseArgs a, std::co
     __builtin_amdgcn_sched_barrier(0);
     in.finish(in.wave, blockIdx.x == 0, formed);
     in.rest(blockIdx.x == 0, (int)a.k, formed);
+  } else if constexpr (JOINED) {
+    __shared__ float sums[2][16];
+    joined_input<bf16_t, IN == IN_JOINED ? 1 : 2>(ahead, blockIdx.x == 0 && blockIdx.y == 0, (int)a.k, formed, sums, [&]() {
+      if (i + US <= s1) weights(i);
+    });
   } else {
     if (i + US <= s1) weights(i);
   }
@@ -529,6 +553,16 @@ __global__ __launch_bounds__(256) void dense_pack_kernel(const S* __restrict__ s
 
 constexpr int kFewTokens = 32;
 
+// Up to 2,048 rows 16 of them a workgroup leave half of the compute units or more without one, and a unit takes in no more than
+// about 30 KB a us.  8 rows against 16: 1,024 x 4,096 4.8 and 6.1 us, 1,536 x 6,144 6.7 and 8.9, 2,048 x 8,192 9.6 and 11.8, 1,024 x
+// 16,384 12.2 and 17.8; from 2,304 rows on 16 are faster (2,304 x 9,216 13.9 against 15.3, 3,072 x 3,072 6.4 against 7.7), and with
+// up to 1,024 inputs neither is (3.5).  Both rows of a gated pair, and the rows of a candidate, are in one workgroup of 16.
+bool eight_rows(const DenseArgs& a, int64_t rows) {
+  bool eight = a.k > 1024 && rows * a.batch <= 2048;
+  for (int i = 0; i < a.n_seg; ++i) eight = eight && a.seg[i].act != DENSE_GLU;
+  return eight;
+}
+
 template <int OUT, int IN, int RW>
 void launch_one_rows(const DenseArgs& a, int64_t rows, size_t lds, hipStream_t st) {
   const dim3 g((unsigned)(rows / RW), (unsigned)a.batch);
@@ -541,12 +575,7 @@ void launch_one_rows(const DenseArgs& a, int64_t rows, size_t lds, hipStream_t s
 template <int OUT, int IN>
 int launch_one_as(const DenseArgs& a, int64_t rows, hipStream_t st) {
   const size_t lds = IN == IN_GATED ? (size_t)a.gate_k * 2 : 0;
-  // Up to 2,048 rows 16 of them a workgroup leave half of the compute units or more without one, and a unit takes in no more than
-  // about 30 KB a us.  8 rows against 16: 1,024 x 4,096 4.8 and 6.1 us, 1,536 x 6,144 6.7 and 8.9, 2,048 x 8,192 9.6 and 11.8, 1,024 x
-  // 16,384 12.2 and 17.8; from 2,304 rows on 16 are faster (2,304 x 9,216 13.9 against 15.3, 3,072 x 3,072 6.4 against 7.7), and with
-  // up to 1,024 inputs neither is (3.5).  Both rows of a gated pair, and the rows of a candidate, are in one workgroup of 16.
-  bool eight = OUT != DENSE_ARGMAX && a.k > 1024 && rows * a.batch <= 2048;
-  for (int i = 0; i < a.n_seg; ++i) eight = eight && a.seg[i].act != DENSE_GLU;
+  const bool eight = OUT != DENSE_ARGMAX && eight_rows(a, rows);
   if constexpr (OUT != DENSE_ARGMAX) {
     if (eight) launch_one_rows<OUT, IN, 8>(a, rows, lds, st);
   }
@@ -568,6 +597,19 @@ int launch_one_normed(const DenseArgs& a, const NormConvArgs& n, int64_t rows, h
   const size_t lds = (size_t)a.k * 2;
   if (n.conv) hipLaunchKernelGGL((dense_one_kernel<8, OUT, IN_NORMED, 16, kFusedTaps>), g, dim3(512), lds, st, a, n);
   else hipLaunchKernelGGL((dense_one_kernel<8, OUT, IN_NORMED, 16>), g, dim3(512), lds, st, a, n);
+  AWQ_HIP_TRY(hipGetLastError());
+  return AWQ_OK;
+}
+
+int launch_one_joined(const DenseArgs& a, const JoinArgs& j, int64_t rows, hipStream_t st) {
+  const size_t lds = (size_t)a.k * 2;
+  const auto launch = [&](auto in) {
+    constexpr int IN = decltype(in)::value;
+    if (eight_rows(a, rows)) hipLaunchKernelGGL((dense_one_kernel<8, DENSE_STORE, IN, 8>), dim3((unsigned)(rows / 8)), dim3(512), lds, st, a, j);
+    else hipLaunchKernelGGL((dense_one_kernel<8, DENSE_STORE, IN, 16>), dim3((unsigned)(rows / 16)), dim3(512), lds, st, a, j);
+  };
+  if (j.width <= 2048) launch(std::integral_constant<int, IN_JOINED>{});
+  else launch(std::integral_constant<int, IN_JOINED_2>{});
   AWQ_HIP_TRY(hipGetLastError());
   return AWQ_OK;
 }
@@ -721,7 +763,17 @@ bool dense_norm_fused(const NormConvArgs& n, bool f32) {
          (!n.conv || n.taps == kFusedTaps) && (((uintptr_t)n.x | (uintptr_t)n.w1 | (uintptr_t)n.w2 | (uintptr_t)n.conv) & 15) == 0;
 }
 
-int launch_dense(const DenseArgs& args, bool f32, hipStream_t st, const NormConvArgs* norm) {
+// Every workgroup of the product reads the rows and the norms' weights, 24 bytes a value and more, and adds them up for itself: up to
+// 4,096 rows at width 4,096 (or as many values in all) that costs less than the launch.  Tudasun, 24 tokens after 48, without it, up to
+// 1 M values (the token input's products only), up to 16 M and always: width 1,024 5.97, 5.96, 5.60 and 5.73 ms, 1,536 6.95, 7.01, 6.60
+// and 6.76, 2,048 8.00, 7.98, 7.56 and 7.67, 2,816 10.4, 10.4, 10.3 and 10.9; 4,096, 64 after 128, 37.2, 37.2, 37.0 and 39.7; width
+// 1,024 in binary32 6.97, 7.08, 6.84 and 6.98.
+bool dense_join_fused(const JoinArgs& j, int64_t rows, bool f32) {
+  return j.M == 1 && j.out && j.x_out && j.x_out != j.x && (j.top == 0 || j.out != j.h) && j.top <= kJoinTop && j.width <= (f32 ? 2048 : 4096) &&
+         ((j.width | j.ldo | j.ldg | j.ldh) & 3) == 0 && j.ldo % kDenseKAlign == 0 && rows * j.width <= 16 << 20;
+}
+
+int launch_dense(const DenseArgs& args, bool f32, hipStream_t st, const NormConvArgs* norm, const JoinArgs* join) {
   DenseArgs a = args;
   AWQ_REQUIRE(a.w && a.M >= 1 && a.k > 0 && a.k % kDenseKAlign == 0, "bad product");
   AWQ_REQUIRE(a.n_seg >= 1 && a.n_seg <= kDenseSegments, "too few or too many segments");
@@ -759,6 +811,12 @@ int launch_dense(const DenseArgs& args, bool f32, hipStream_t st, const NormConv
                     (a.out == DENSE_STORE || a.out == DENSE_ARGMAX) && norm->x && norm->w1 && (!norm->conv || (norm->state[0] && norm->state[1])),
                 "the norm cannot be part of this product");
     return a.out == DENSE_STORE ? launch_one_normed<DENSE_STORE>(a, *norm, rows, st) : launch_one_normed<DENSE_ARGMAX>(a, *norm, rows, st);
+  }
+  if (join) {
+    AWQ_REQUIRE(dense_join_fused(*join, rows, f32) && a.M == 1 && a.k == join->ldo && a.batch == 1 && !a.ids && !a.gate_o && a.out == DENSE_STORE &&
+                    join->x && join->w_post && (join->y || join->top > 0),
+                "the end of the sublayer cannot be part of this product");
+    return f32 ? launch_dense_one_joined_f32(a, *join, rows, st) : launch_one_joined(a, *join, rows, st);
   }
   if (f32) return a.M == 1 ? launch_dense_one_f32(a, rows, st) : launch_dense_many_f32(a, rows, st);
   switch (a.out) {

@@ -256,4 +256,5 @@ __global__ __launch_bounds__(256) void dense_parts_kernel(DenseArgs a, int rows,
 
 // binary32 (dense_f32.hip)
 int launch_dense_one_f32(const DenseArgs& a, int64_t rows, hipStream_t st);
+int launch_dense_one_joined_f32(const DenseArgs& a, const JoinArgs& j, int64_t rows, hipStream_t st);
 int launch_dense_many_f32(const DenseArgs& a, int64_t rows, hipStream_t st);  // a.tiles: token lists

@@ -1,5 +1,6 @@
 // Dense products of binary32 weights with one token or many (layers.hpp).
 #include "dense_device.hpp"
+#include "join_device.hpp"
 
 #include <math.h>
 
@@ -13,8 +14,10 @@ namespace {
 // inputs whatever R is.  Rows of 1,024 inputs: 32,768 of them (a vocabulary's logits, R = 4) 29 us, 4.6 TB/s; four blocks of
 // 1,536 gated rows (R = 2) 6.8 us, where a wavefront that took the two rows of a pair one after the other, beside one
 // that had none, took 9.8; below 8,192 rows one each, so that 1,024 rows still make 256 workgroups.
-template <int OUT, int R>
-__global__ __launch_bounds__(256) void dense_one_f32_kernel(DenseArgs a) {
+// JQ: the input is formed here, the end of the sublayer ahead (JoinArgs, JQ turns of the workgroup's threads)
+template <int OUT, int R, int JQ = 0>
+__global__ __launch_bounds__(256) void dense_one_f32_kernel(DenseArgs a, std::conditional_t<JQ != 0, JoinArgs, std::false_type> join) {
+  extern __shared__ __attribute__((aligned(16))) float formed[];  // [k]
   __shared__ unsigned long long candidates[4];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   // rows of the wavefront: row(0), and with R = 2 row(0) + 8, with R = 4 row(0) + 1, + 8, + 9
@@ -38,6 +41,23 @@ __global__ __launch_bounds__(256) void dense_one_f32_kernel(DenseArgs a) {
   };
   constexpr int U = R == 4 ? 4 : 8;
   int at = lane;
+  if constexpr (JQ != 0) {
+    __shared__ float sums[2][16];
+    f32x4_t wv[4][R];  // the first weights, behind the request for the row
+    const bool first = at + 64 * 3 < (int)k4;
+    joined_input<float, JQ>(join, blockIdx.x == 0 && blockIdx.y == 0, (int)a.k, formed, sums, [&]() {
+      if (!first) return;
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int i = 0; i < R; ++i) wv[u][i] = __builtin_nontemporal_load(w + row_of(i) * k4 + at + 64 * u);
+    });
+    if (first) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) add(wv[u], reinterpret_cast<const f32x4_t*>(formed)[at + 64 * u]);
+      at += 64 * 4;
+    }
+  }
   auto pieces = [&](auto count) __attribute__((always_inline)) {
     constexpr int N = decltype(count)::value;
     f32x4_t wv[N][R], xv[N];
@@ -45,7 +65,8 @@ __global__ __launch_bounds__(256) void dense_one_f32_kernel(DenseArgs a) {
     for (int u = 0; u < N; ++u) {
 #pragma unroll
       for (int i = 0; i < R; ++i) wv[u][i] = __builtin_nontemporal_load(w + row_of(i) * k4 + at + 64 * u);
-      xv[u] = x[at + 64 * u];
+      if constexpr (JQ != 0) xv[u] = reinterpret_cast<const f32x4_t*>(formed)[at + 64 * u];
+      else xv[u] = x[at + 64 * u];
     }
 #pragma unroll
     for (int u = 0; u < N; ++u) add(wv[u], xv[u]);
@@ -209,12 +230,13 @@ int launch_one(const DenseArgs& a, int64_t rows, hipStream_t st) {
   bool pairs = false;
   for (int i = 0; i < a.n_seg; ++i) pairs |= a.seg[i].act == DENSE_GLU;
   const int64_t all = rows * a.batch;
+  const std::false_type no;
   if (OUT == DENSE_ARGMAX || all >= 16384)
-    hipLaunchKernelGGL((dense_one_f32_kernel<OUT, 4>), dim3((unsigned)(rows / 16), (unsigned)a.batch), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((dense_one_f32_kernel<OUT, 4>), dim3((unsigned)(rows / 16), (unsigned)a.batch), dim3(256), 0, st, a, no);
   else if (pairs || all >= 8192)
-    hipLaunchKernelGGL((dense_one_f32_kernel<OUT, 2>), dim3((unsigned)(rows / 8), (unsigned)a.batch), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((dense_one_f32_kernel<OUT, 2>), dim3((unsigned)(rows / 8), (unsigned)a.batch), dim3(256), 0, st, a, no);
   else
-    hipLaunchKernelGGL((dense_one_f32_kernel<OUT, 1>), dim3((unsigned)(rows / 4), (unsigned)a.batch), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((dense_one_f32_kernel<OUT, 1>), dim3((unsigned)(rows / 4), (unsigned)a.batch), dim3(256), 0, st, a, no);
   AWQ_HIP_TRY(hipGetLastError());
   return AWQ_OK;
 }
@@ -280,6 +302,19 @@ int launch_dense_one_f32(const DenseArgs& a, int64_t rows, hipStream_t st) {
     case DENSE_F32: return launch_one<DENSE_F32>(a, rows, st);
     default: return launch_one<DENSE_ARGMAX>(a, rows, st);
   }
+}
+
+int launch_dense_one_joined_f32(const DenseArgs& a, const JoinArgs& j, int64_t rows, hipStream_t st) {
+  const size_t lds = (size_t)a.k * 4;
+  const auto launch = [&](auto q) {
+    constexpr int Q = decltype(q)::value;
+    if (rows >= 2048) hipLaunchKernelGGL((dense_one_f32_kernel<DENSE_STORE, 4, Q>), dim3((unsigned)(rows / 16)), dim3(256), lds, st, a, j);
+    else hipLaunchKernelGGL((dense_one_f32_kernel<DENSE_STORE, 2, Q>), dim3((unsigned)(rows / 8)), dim3(256), lds, st, a, j);
+  };
+  if (j.width <= 1024) launch(std::integral_constant<int, 1>{});
+  else launch(std::integral_constant<int, 2>{});
+  AWQ_HIP_TRY(hipGetLastError());
+  return AWQ_OK;
 }
 
 int launch_dense_many_f32(const DenseArgs& a, int64_t rows, hipStream_t st) {

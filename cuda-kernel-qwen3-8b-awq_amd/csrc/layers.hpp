@@ -126,7 +126,11 @@ int launch_dense_pack(const void* src, bool src_f32, int64_t rows, int64_t cols,
 struct NormConvArgs;
 // norm (one token, where dense_norm_fused): launch_norm_conv is part of the product, out1 the input of segment 0, out2 of segment 1;
 // neither is written, and what the segments name as x is not read
-int launch_dense(const DenseArgs& a, bool f32, hipStream_t st, const NormConvArgs* norm = nullptr);
+struct JoinArgs;
+// join (one token, DENSE_STORE, where dense_join_fused says so of a product of `rows` padded rows): launch_join is part of the
+// product, its result the segments' input; x_out and out are written, x stays
+int launch_dense(const DenseArgs& a, bool f32, hipStream_t st, const NormConvArgs* norm = nullptr, const JoinArgs* join = nullptr);
+bool dense_join_fused(const JoinArgs& j, int64_t rows, bool f32);
 bool dense_norm_fused(const NormConvArgs& n, bool f32);
 bool dense_gate_fused(int64_t n, int64_t k_padded, int64_t M, bool f32);
 
@@ -332,6 +336,7 @@ int launch_embed_tokens(const void* table, const void* side_table, bool f32, con
 // What ends a sublayer: x += RMS norm(y * gate) * w_post, then out = RMS norm(x) * w_next.
 struct JoinArgs {
   float* x = nullptr;         // [M][width]
+  float* x_out = nullptr;     // where the new x goes; null: x
   int64_t M = 0, width = 0;
   float eps = 0.0f;
   const float* y = nullptr;   // [M][width], or null

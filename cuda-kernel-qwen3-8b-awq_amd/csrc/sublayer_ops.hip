@@ -1,49 +1,8 @@
 // What stands around the products of a sublayer (layers.hpp): token rows, the gated and normalised sum into the residual
 // stream with the next norm behind it, PolyNorm.
-#include "layers.hpp"
+#include "join_device.hpp"
 
 namespace {
-
-template <typename T, int V>
-struct Vec {
-  typedef T type __attribute__((ext_vector_type(V)));
-};
-template <typename T, int V>
-__device__ __forceinline__ void read(const T* p, float (&v)[V]) {
-  if constexpr (V == 1) {
-    v[0] = (float)*p;
-  } else {
-    const typename Vec<T, V>::type r = *reinterpret_cast<const typename Vec<T, V>::type*>(p);
-#pragma unroll
-    for (int i = 0; i < V; ++i) v[i] = (float)r[i];
-  }
-}
-template <typename T, int V>
-__device__ __forceinline__ void write(T* p, const float (&v)[V]) {
-  if constexpr (V == 1) {
-    *p = (T)v[0];
-  } else {
-    typename Vec<T, V>::type r;
-#pragma unroll
-    for (int i = 0; i < V; ++i) r[i] = (T)v[i];
-    *reinterpret_cast<typename Vec<T, V>::type*>(p) = r;
-  }
-}
-
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
-}
-// sum over the workgroup; `sums` has a place per wavefront and is free again behind the next barrier
-__device__ __forceinline__ float group_sum(float v, float* sums) {
-  v = wave_sum(v);
-  if ((threadIdx.x & 63) == 0) sums[threadIdx.x >> 6] = v;
-  __syncthreads();
-  float all = 0.0f;
-  for (int i = 0; i < (int)(blockDim.x >> 6); ++i) all += sums[i];
-  return all;
-}
 
 template <typename T, int V>
 __global__ __launch_bounds__(256) void embed_tokens_kernel(const T* __restrict__ table, const T* __restrict__ side_table,
@@ -77,7 +36,8 @@ __global__ __launch_bounds__(1024) void join_kernel(JoinArgs a) {
   __shared__ float sums[2][16];
   const int tid = threadIdx.x, step = blockDim.x * V, W = (int)a.width;
   const int64_t t = blockIdx.x;
-  float* const x = a.x + t * W;
+  const float* const x = a.x + t * W;
+  float* const x_out = (a.x_out ? a.x_out : a.x) + t * W;
   const float y_mul = a.y_gate ? 1.0f / (1.0f + expf(-a.y_gate[t])) : 1.0f;
   float sq = 0.0f;
   for (int c = tid * V; c < W; c += step) {
@@ -118,7 +78,7 @@ __global__ __launch_bounds__(1024) void join_kernel(JoinArgs a) {
       r[i] = r[i] + v[i] * inv * w[i];
       sq = __builtin_fmaf(r[i], r[i], sq);
     }
-    write<float, V>(x + c, r);
+    write<float, V>(x_out + c, r);
     if (a.out) write<float, V>(row + c, r);
   }
   if (!a.out) return;
@@ -137,70 +97,18 @@ __global__ __launch_bounds__(1024) void join_kernel(JoinArgs a) {
 }
 
 // The same where a row is a workgroup's threads times V at most and a token has at most kJoinTop choices, which then wait in
-// registers.  Bound by trips to memory: the form above makes three, one behind the other, and one more for each choice; here
-// everything is requested at once (an identity output's row of `pairs` too, which is then not used).  Tudasun of width 4,096,
-// 64 tokens one by one with 12 launches each: 38.6 -> 37.8 ms; width 1,024 in binary32, 24 tokens: 7.73 -> 7.50.
-constexpr int kJoinTop = 8;
+// registers (join_device.hpp): the form above makes three trips to memory, one behind the other, and one more for each choice.
+// Tudasun of width 4,096, 64 tokens one by one with 12 launches each: 38.6 -> 37.8 ms; width 1,024 in binary32, 24 tokens:
+// 7.73 -> 7.50.
 template <typename T, int V>
 __global__ __launch_bounds__(1024) void join_row_kernel(JoinArgs a) {
   __shared__ float sums[2][16];
-  const int tid = threadIdx.x, W = (int)a.width, c = tid * V;
-  const int64_t t = blockIdx.x;
-  const bool mine = c < W;
-  float v[V] = {}, g[V] = {}, r[V] = {}, w_post[V] = {}, w_next[V] = {}, h[V] = {}, u[kJoinTop][V], w[kJoinTop];
-  int ids[kJoinTop];
-  if (mine) {
-    if (a.y) read<float, V>(a.y + t * W + c, v);
-    if (a.gate) read<T, V>(reinterpret_cast<const T*>(a.gate) + t * a.ldg + c, g);
-    read<float, V>(a.x + t * W + c, r);
-    read<float, V>(a.w_post + c, w_post);
-    if (a.w_next) read<float, V>(a.w_next + c, w_next);
-    if (a.top > 0) read<T, V>(reinterpret_cast<const T*>(a.h) + t * a.ldh + c, h);
-  }
-#pragma unroll
-  for (int j = 0; j < kJoinTop; ++j)
-    if (j < a.top) {
-      ids[j] = a.ids[t * a.top + j];
-      w[j] = a.weights[t * a.top + j];
-      if (mine) read<float, V>(a.pairs + (t * a.top + j) * W + c, u[j]);
-    }
-  const float y_mul = a.y_gate ? 1.0f / (1.0f + expf(-a.y_gate[t])) : 1.0f;
-  float sq = 0.0f;
-  if (mine) {
-    if (a.y) {
-#pragma unroll
-      for (int i = 0; i < V; ++i) v[i] *= y_mul;
-    }
-#pragma unroll
-    for (int j = 0; j < kJoinTop; ++j)
-      if (j < a.top) {
-#pragma unroll
-        for (int i = 0; i < V; ++i) v[i] = __builtin_fmaf(w[j], ids[j] < a.experts ? u[j][i] : h[i], v[i]);
-      }
-    if (a.gate) {
-#pragma unroll
-      for (int i = 0; i < V; ++i) v[i] *= g[i];
-    }
-#pragma unroll
-    for (int i = 0; i < V; ++i) sq = __builtin_fmaf(v[i], v[i], sq);
-  }
-  const float inv = 1.0f / sqrtf(group_sum(sq, sums[0]) / (float)W + a.eps);
-  sq = 0.0f;
-  if (mine) {
-#pragma unroll
-    for (int i = 0; i < V; ++i) {
-      r[i] = r[i] + v[i] * inv * w_post[i];
-      sq = __builtin_fmaf(r[i], r[i], sq);
-    }
-    write<float, V>(a.x + t * W + c, r);
-  }
-  if (!a.out) return;
-  if (a.w_next) {
-    const float next = 1.0f / sqrtf(group_sum(sq, sums[1]) / (float)W + a.eps);
-#pragma unroll
-    for (int i = 0; i < V; ++i) r[i] = r[i] * next * w_next[i];
-  }
-  if (mine) write<T, V>(reinterpret_cast<T*>(a.out) + t * a.ldo + c, r);
+  JoinRow<T, V, 1> row(a, blockIdx.x, blockDim.x);
+  row.request_rows();
+  row.request_weights();
+  float* const x = (a.x_out ? a.x_out : a.x) + row.t * row.W;
+  row.finish(sums, [&](int c, const float (&r)[V]) { write<float, V>(x + c, r); });
+  if (a.out && row.column(0) < row.W) write<T, V>(reinterpret_cast<T*>(a.out) + row.t * a.ldo + row.column(0), row.r[0]);
 }
 
 template <typename T, int V>

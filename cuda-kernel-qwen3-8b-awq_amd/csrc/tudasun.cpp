@@ -234,6 +234,7 @@ TensorTable expected_tensors(const Spec& c) {
 struct InBlock {
   void* w = nullptr;
   std::vector<int32_t> at;  // first rows, in the order they were asked for
+  int64_t rows = 0;         // padded
 };
 
 struct LayerDev {
@@ -262,9 +263,9 @@ struct LayerDev {
 
 // activations of a pass of up to `tokens` tokens
 struct Buffers {
-  float *x = nullptr, *y = nullptr, *o = nullptr, *decay = nullptr, *down = nullptr, *router = nullptr, *shared_gate = nullptr,
+  float *x = nullptr, *x2 = nullptr, *y = nullptr, *o = nullptr, *decay = nullptr, *down = nullptr, *router = nullptr, *shared_gate = nullptr,
         *pairs = nullptr, *weights = nullptr;
-  void *h = nullptr, *xt = nullptr, *proj = nullptr, *gate = nullptr, *low = nullptr, *ctx = nullptr, *mid = nullptr,
+  void *h = nullptr, *xt = nullptr, *proj = nullptr, *gate = nullptr, *gate2 = nullptr, *low = nullptr, *ctx = nullptr, *mid = nullptr,
        *shared_mid = nullptr, *side = nullptr, *side_mid = nullptr;
   int32_t *ids = nullptr, *list = nullptr;
   DenseTile* tiles = nullptr;
@@ -291,6 +292,15 @@ struct TudasunEngine final : ConfigModel {
   int make_activations(Buffers* b, int64_t n_tokens);
   LatentAttnArgs latent_args(int i) const;
   int64_t side_width() const { return (int64_t)layers.size() * spec.side; }
+
+  // the end of a sublayer that is part of the product behind it
+  JoinArgs waiting;
+  bool is_waiting = false;
+  const JoinArgs* take_waiting() {
+    const JoinArgs* const j = is_waiting ? &waiting : nullptr;
+    is_waiting = false;
+    return j;
+  }
 
   // the parts of a layer
   DenseArgs product(const void* w, int64_t k, int64_t M) const;
@@ -328,6 +338,7 @@ int load_in(Loader& ldr, ConfigModel* e, const std::vector<Part>& parts, InBlock
   if (int rc = ldr.block(&b->w, round_up(rows, kDenseRowAlign), e->ld)) return rc;
   for (size_t i = 0; i < parts.size(); ++i)
     if (int rc = ldr.matrix(parts[i].name, b->w, e->ld, first[i], 0, parts[i].form)) return rc;
+  b->rows = round_up(rows, kDenseRowAlign);
   return AWQ_OK;
 }
 
@@ -506,12 +517,12 @@ int TudasunEngine::make_activations(Buffers* b, int64_t n) {
     int64_t bytes;
   };
   const int64_t u = unit();
-  const Need all[] = {{(void**)&b->x, n * width * 4}, {(void**)&b->y, n * width * 4}, {(void**)&b->o, n * o * 4},
+  const Need all[] = {{(void**)&b->x, n * width * 4}, {(void**)&b->x2, n == 1 ? width * 4 : 16}, {(void**)&b->y, n * width * 4}, {(void**)&b->o, n * o * 4},
                       {(void**)&b->decay, n * decay * 4}, {(void**)&b->down, n * down * 4}, {(void**)&b->router, n * router * 4},
                       {(void**)&b->shared_gate, n * 4}, {(void**)&b->pairs, n * pairs * 4}, {(void**)&b->weights, n * top * 4},
                       {(void**)&b->ids, n * top * 4}, {(void**)&b->list, n * top * 4},
                       {(void**)&b->tiles, tiles * (int64_t)sizeof(DenseTile)}, {&b->h, n * ld * u}, {&b->xt, n * ld * u},
-                      {&b->proj, n * proj * u}, {&b->gate, n * ldg * u}, {&b->low, n * low * u}, {&b->ctx, n * ctx * u},
+                      {&b->proj, n * proj * u}, {&b->gate, n * ldg * u}, {&b->gate2, n * ldg * u}, {&b->low, n * low * u}, {&b->ctx, n * ctx * u},
                       {&b->mid, n * mid * u}, {&b->shared_mid, n * shared_mid * u}, {&b->side, n * std::max<int64_t>(1, side_width()) * u},
                       {&b->side_mid, n * std::max<int64_t>(8, side_k) * u}};
   for (const Need& need : all)
@@ -596,7 +607,7 @@ int TudasunEngine::mix(int i, Buffers& b, int64_t M, PassPos pos) {
     DenseSegment& g = rows(b.gate, ldg, width);
     g.act = DENSE_SIGMOID;
     g.bias = L.rg1_b;
-    if (int rc = launch_dense(a, f32, stream)) return rc;
+    if (int rc = launch_dense(a, f32, stream, nullptr, take_waiting())) return rc;
   }
   if (s.type == MIX_LATENT) {
     LatentAttnArgs a = latent_args(i);
@@ -665,11 +676,11 @@ int TudasunEngine::dense_feed_forward(int i, Buffers& b, int64_t M) {
   const LayerDev& L = layers[i];
   {
     DenseArgs a = product(L.mid.w, ld, M);
-    DenseSegment& g = segment(&a, b.h, ld, b.gate, ldg, L.mid.at[0], width);
+    DenseSegment& g = segment(&a, b.h, ld, b.gate2, ldg, L.mid.at[0], width);
     g.act = DENSE_SIGMOID;
     g.bias = L.rg2_b;
     segment(&a, b.h, ld, b.mid, L.ff_k, L.mid.at[1], s.ff);
-    if (int rc = launch_dense(a, f32, stream)) return rc;
+    if (int rc = launch_dense(a, f32, stream, nullptr, take_waiting())) return rc;
   }
   if (int rc = launch_polynorm(b.mid, L.ff_k, s.ff, M, L.act, eps, f32, stream)) return rc;
   DenseArgs a = product(L.w_down, L.ff_k, M);
@@ -687,7 +698,7 @@ int TudasunEngine::routed_feed_forward(int i, Buffers& b, int64_t M, JoinArgs* e
   float* const shared_y = beside ? b.pairs + (int64_t)s.top * width : b.y;
   {
     DenseArgs a = product(L.mid.w, ld, M);
-    DenseSegment& g = segment(&a, b.h, ld, b.gate, ldg, L.mid.at[0], width);
+    DenseSegment& g = segment(&a, b.h, ld, b.gate2, ldg, L.mid.at[0], width);
     g.act = DENSE_SIGMOID;
     g.bias = L.rg2_b;
     segment(&a, b.h, ld, b.router, s.outputs(), L.mid.at[1], s.outputs()).y_f32 = 1;
@@ -697,7 +708,7 @@ int TudasunEngine::routed_feed_forward(int i, Buffers& b, int64_t M, JoinArgs* e
       m.glu_rows = s.shared_ff;
       segment(&a, b.h, ld, b.shared_gate, 1, L.mid.at[3], 1).y_f32 = 1;
     }
-    if (int rc = launch_dense(a, f32, stream)) return rc;
+    if (int rc = launch_dense(a, f32, stream, nullptr, take_waiting())) return rc;
   }
   const int32_t tile_tokens = route_tile_tokens(M, s.top, s.outputs(), f32);
   {
@@ -773,7 +784,7 @@ int TudasunEngine::token_input(int i, Buffers& b, int64_t M, JoinArgs* end) {
   g.act = DENSE_GELU;
   g.mul = (const char*)b.side + (int64_t)i * spec.side * unit();
   g.ldmul = side_width();
-  if (int rc = launch_dense(a, f32, stream)) return rc;
+  if (int rc = launch_dense(a, f32, stream, nullptr, take_waiting())) return rc;
   DenseArgs p = product(L.w_side_proj, side_k, M);
   p.out = DENSE_F32;
   segment(&p, b.side_mid, side_k, b.y, width, 0, width);
@@ -797,12 +808,29 @@ int TudasunEngine::run_pass(bool one, const int32_t* ids, int64_t M, PassPos pos
     a.ld = ld;
     if (int rc = launch_norm_conv(a, f32, stream)) return rc;
   }
+  // The stream is read from one place and written to another where the end of a sublayer is part of the product behind it, whose
+  // other workgroups still read it; the last end leaves it where it was embedded.
+  float *x = b.x, *spare = b.x2;
+  const auto end_sublayer = [&](JoinArgs& e, int64_t next_rows, bool last) -> int {
+    e.x = x;
+    e.x_out = spare;
+    if (one && !tap_on && next_rows > 0 && dense_join_fused(e, next_rows, f32)) {
+      std::swap(x, spare);
+      waiting = e;
+      is_waiting = true;
+      return AWQ_OK;
+    }
+    e.x_out = last ? b.x : x;
+    return launch_join(e, f32, stream);
+  };
+  is_waiting = false;
   for (int i = 0; i < n; ++i) {
     const LayerSpec& s = spec.layers[i];
     const LayerDev& L = layers[i];
+    const bool end = i + 1 == n;
+    const int64_t side_rows = round_up(spec.side, kDenseRowAlign);
     const auto ending = [&]() {
       JoinArgs e;
-      e.x = b.x;
       e.M = M;
       e.width = width;
       e.eps = eps;
@@ -813,10 +841,11 @@ int TudasunEngine::run_pass(bool one, const int32_t* ids, int64_t M, PassPos pos
     const auto leaves = [&](JoinArgs* e, bool token_input_next) {
       if (token_input_next) {
         e->out = b.xt;
-      } else if (i + 1 < n) {
+      } else if (!end) {
         e->w_next = layers[i + 1].norm1;
         e->out = b.h;
       }
+      return token_input_next ? side_rows : end ? 0 : layers[i + 1].in.rows;
     };
     if (int rc = mix(i, b, M, pos)) return rc;
     {
@@ -829,29 +858,30 @@ int TudasunEngine::run_pass(bool one, const int32_t* ids, int64_t M, PassPos pos
       e.gate = b.gate;
       e.ldg = ldg;
       e.w_post = L.norm1b;
+      int64_t next = L.mid.rows;
       if (s.mlp != MLP_NONE) {
         e.w_next = L.norm2;
         e.out = b.h;
       } else {
-        leaves(&e, spec.side > 0);
+        next = leaves(&e, spec.side > 0);
       }
-      if (int rc = launch_join(e, f32, stream)) return rc;
+      if (int rc = end_sublayer(e, next, end && s.mlp == MLP_NONE && !spec.side)) return rc;
     }
     if (s.mlp != MLP_NONE) {
       JoinArgs e = ending();
       e.y = b.y;
       if (int rc = s.mlp == MLP_DENSE ? dense_feed_forward(i, b, M) : routed_feed_forward(i, b, M, &e)) return rc;
-      e.gate = b.gate;
+      e.gate = b.gate2;
       e.ldg = ldg;
       e.w_post = L.norm2b;
-      leaves(&e, spec.side > 0);
-      if (int rc = launch_join(e, f32, stream)) return rc;
+      const int64_t next = leaves(&e, spec.side > 0);
+      if (int rc = end_sublayer(e, next, end && !spec.side)) return rc;
     }
     if (spec.side) {
       JoinArgs e = ending();
       if (int rc = token_input(i, b, M, &e)) return rc;
-      leaves(&e, false);
-      if (int rc = launch_join(e, f32, stream)) return rc;
+      const int64_t next = leaves(&e, false);
+      if (int rc = end_sublayer(e, next, end)) return rc;
     }
     if (tap_on)
       if (int rc = tap_layer(i, b.x, M)) return rc;
