@@ -1,4 +1,5 @@
 // Linear attention whose state decays per channel (layers.hpp): per head S <- diag(decay_t) S + k_t v_t^T, o_t = S^T q_t.
+#include "lane_sums.hpp"
 #include "layers.hpp"
 
 #include <type_traits>
@@ -14,13 +15,10 @@ __device__ __forceinline__ void decay_and_key(float g, bool keys, float k, float
 }
 
 // The recurrence token by token: a wavefront holds kCols columns of the state, lane l the rows l, l + 64, ... of each.
-// Used for one token.  HEAD: a workgroup per head; the head's norm and gate are formed behind the recurrence in the same
-// launch.  Otherwise a workgroup takes 4 kCols columns.
-template <typename T, int DPL, bool HEAD, int kCols>
-__global__ __launch_bounds__(HEAD ? 1024 : 256) void gated_step_kernel(GatedStateArgs a) {
-  extern __shared__ float row[];  // HEAD: [vdim]
-  __shared__ float sums[16];
-  const int head = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+// Used for one token.  A workgroup takes 4 kCols columns.
+template <typename T, int DPL, int kCols>
+__global__ __launch_bounds__(256) void gated_step_kernel(GatedStateArgs a) {
+  const int head = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int dimp = DPL * 64;
   const T* q = reinterpret_cast<const T*>(a.q) + (int64_t)head * a.dim;
   const T* k = reinterpret_cast<const T*>(a.k) + (int64_t)head * a.dim;
@@ -29,74 +27,48 @@ __global__ __launch_bounds__(HEAD ? 1024 : 256) void gated_step_kernel(GatedStat
   float* o = a.o + (int64_t)head * a.vdim;
   const int64_t ldo = (int64_t)a.heads * a.vdim;
   const bool keys = a.k != nullptr, fresh = a.pos.position() == 0;
-  const int first = HEAD ? wave * kCols : (blockIdx.y * 4 + wave) * kCols, step = HEAD ? waves * kCols : a.vdim;
-  for (int col0 = first; col0 < a.vdim; col0 += step) {
-    float* state = a.state + ((int64_t)head * a.vdim + col0) * dimp;
-    const int nc = min(kCols, a.vdim - col0);
-    float s[kCols][DPL];
+  const int col0 = (blockIdx.y * 4 + wave) * kCols;
+  if (col0 >= a.vdim) return;
+  float* state = a.state + ((int64_t)head * a.vdim + col0) * dimp;
+  const int nc = min(kCols, a.vdim - col0);
+  float s[kCols][DPL];
 #pragma unroll
-    for (int c = 0; c < kCols; ++c)
+  for (int c = 0; c < kCols; ++c)
 #pragma unroll
-      for (int i = 0; i < DPL; ++i) s[c][i] = fresh || c >= nc ? 0.0f : state[c * dimp + i * 64 + lane];
-    for (int64_t t = 0; t < a.M; ++t) {
-      float qv[DPL], kv[DPL], dv[DPL], out[kCols];
+    for (int i = 0; i < DPL; ++i) s[c][i] = fresh || c >= nc ? 0.0f : state[c * dimp + i * 64 + lane];
+  for (int64_t t = 0; t < a.M; ++t) {
+    float qv[DPL], kv[DPL], dv[DPL], out[kCols];
+#pragma unroll
+    for (int i = 0; i < DPL; ++i) {
+      const int d = i * 64 + lane;
+      qv[i] = kv[i] = dv[i] = 0.0f;
+      if (d < a.dim) {
+        qv[i] = (float)q[t * a.ldp + d] * a.q_scale;
+        decay_and_key(g[t * a.ldg + d], keys, keys ? (float)k[t * a.ldp + d] : 0.0f, dv[i], kv[i]);
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < kCols; ++c) {
+      const float vv = c < nc ? (float)v[t * a.ldp + col0 + c] : 0.0f;
+      out[c] = 0.0f;
 #pragma unroll
       for (int i = 0; i < DPL; ++i) {
-        const int d = i * 64 + lane;
-        qv[i] = kv[i] = dv[i] = 0.0f;
-        if (d < a.dim) {
-          qv[i] = (float)q[t * a.ldp + d] * a.q_scale;
-          decay_and_key(g[t * a.ldg + d], keys, keys ? (float)k[t * a.ldp + d] : 0.0f, dv[i], kv[i]);
-        }
-      }
-#pragma unroll
-      for (int c = 0; c < kCols; ++c) {
-        const float vv = c < nc ? (float)v[t * a.ldp + col0 + c] : 0.0f;
-        out[c] = 0.0f;
-#pragma unroll
-        for (int i = 0; i < DPL; ++i) {
-          s[c][i] = __builtin_fmaf(kv[i], vv, dv[i] * s[c][i]);
-          out[c] = __builtin_fmaf(s[c][i], qv[i], out[c]);
-        }
-      }
-#pragma unroll
-      for (int c = 0; c < kCols; ++c) {
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) out[c] += __shfl_xor(out[c], off, 64);
-        if (lane == c && c < nc) {
-          if constexpr (HEAD) row[col0 + c] = out[c];
-          else o[t * ldo + col0 + c] = out[c];
-        }
+        s[c][i] = __builtin_fmaf(kv[i], vv, dv[i] * s[c][i]);
+        out[c] = __builtin_fmaf(s[c][i], qv[i], out[c]);
       }
     }
 #pragma unroll
-    for (int c = 0; c < kCols; ++c)
-      if (c < nc)
+    for (int c = 0; c < kCols; ++c) {
 #pragma unroll
-        for (int i = 0; i < DPL; ++i) state[c * dimp + i * 64 + lane] = s[c][i];
-  }
-  if constexpr (HEAD) {
-    __syncthreads();
-    float sq = 0.0f;
-    for (int c = threadIdx.x; c < a.vdim; c += blockDim.x) sq = __builtin_fmaf(row[c], row[c], sq);
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) sq += __shfl_xor(sq, off, 64);
-    if (lane == 0) sums[wave] = sq;
-    __syncthreads();
-    float all = 0.0f;
-    for (int i = 0; i < waves; ++i) all += sums[i];
-    const float inv = 1.0f / sqrtf(all / (float)a.vdim + a.eps);
-    const T* gate = reinterpret_cast<const T*>(a.gate);
-    T* ctx = reinterpret_cast<T*>(a.ctx) + (int64_t)head * a.vdim;
-    for (int c = threadIdx.x; c < a.vdim; c += blockDim.x) {
-      float y = row[c] * inv * a.norm[c];
-      if (gate) {
-        const float z = (float)gate[(int64_t)head * a.vdim + c];
-        y *= z / (1.0f + expf(-z));
-      }
-      ctx[c] = (T)y;
+      for (int off = 32; off > 0; off >>= 1) out[c] += __shfl_xor(out[c], off, 64);
+      if (lane == c && c < nc) o[t * ldo + col0 + c] = out[c];
     }
   }
+#pragma unroll
+  for (int c = 0; c < kCols; ++c)
+    if (c < nc)
+#pragma unroll
+      for (int i = 0; i < DPL; ++i) state[c * dimp + i * 64 + lane] = s[c][i];
 }
 
 // The same for several tokens: fewer than the chunked form takes, wider heads, linear attention with few tokens or a decay of
@@ -142,6 +114,108 @@ __device__ __forceinline__ void sixteen_sums(float (&x)[16], int lane) {
   x[0] = (lane & 4 ? high : low) + other_lane<4>(lane & 4 ? low : high);
   x[0] += other_lane<2>(x[0]);
   x[0] += other_lane<1>(x[0]);
+}
+
+// One token with the head's norm and gate behind the recurrence: a workgroup per head, the recurrence as above.  Bound by the trips to
+// memory and by what a compute unit takes in and gives out (the head's state both ways), so everything is requested at once:
+// the state before the position is known (what it holds ahead of position 0 is not used), norm and gate ahead of the sums,
+// which are ended together.  32 heads of 128 5.4 us; with the state requested behind the position, and each sum
+// by itself, 8.2.
+template <int N>
+__device__ __forceinline__ void ended_sums(float (&x)[N], int lane) {  // N = 8, 4: number lane / (64 / N) in x[0], in the order of sixteen_sums
+  typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
+#pragma unroll
+  for (int i = 0; i < N / 2; ++i) {
+    const u32x2_t p = __builtin_amdgcn_permlane32_swap(__float_as_uint(x[i]), __float_as_uint(x[i + N / 2]), false, false);
+    x[i] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+  }
+#pragma unroll
+  for (int i = 0; i < N / 4; ++i) {
+    const u32x2_t p = __builtin_amdgcn_permlane16_swap(__float_as_uint(x[i]), __float_as_uint(x[i + N / 4]), false, false);
+    x[i] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+  }
+  if constexpr (N == 8) x[0] = (lane & 8 ? x[1] : x[0]) + other_lane<8>(lane & 8 ? x[0] : x[1]);
+  else x[0] += other_lane<8>(x[0]);
+  x[0] += other_lane<4>(x[0]);
+  x[0] += other_lane<2>(x[0]);
+  x[0] += other_lane<1>(x[0]);
+}
+
+template <typename T, int DPL, int kCols>
+__global__ __launch_bounds__(1024) void gated_head_kernel(GatedStateArgs a) {
+  extern __shared__ float row[];  // [vdim]
+  __shared__ float sums[16];
+  const int head = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, waves = blockDim.x >> 6;
+  const int dimp = DPL * 64;
+  const T* q = reinterpret_cast<const T*>(a.q) + (int64_t)head * a.dim;
+  const T* k = reinterpret_cast<const T*>(a.k) + (int64_t)head * a.dim;
+  const T* v = reinterpret_cast<const T*>(a.v) + (int64_t)head * a.vdim;
+  const T* gate = reinterpret_cast<const T*>(a.gate) + (int64_t)head * a.vdim;
+  const float* g = a.g + (int64_t)head * a.dim;
+  const bool keys = a.k != nullptr;
+  float qv[DPL], kv[DPL], gv[DPL], s[kCols][DPL], vv = 0.0f;
+  auto request = [&](int col0) __attribute__((always_inline)) {
+    const float* state = a.state + (int64_t)head * a.vdim * dimp;
+#pragma unroll
+    for (int c = 0; c < kCols; ++c)
+#pragma unroll
+      for (int i = 0; i < DPL; ++i) s[c][i] = state[(int64_t)min(col0 + c, a.vdim - 1) * dimp + i * 64 + lane];
+    vv = (float)v[min(col0 + lane % kCols, a.vdim - 1)];
+  };
+#pragma unroll
+  for (int i = 0; i < DPL; ++i) {
+    const int d = min(i * 64 + lane, a.dim - 1);
+    qv[i] = (float)q[d];
+    gv[i] = g[d];
+    kv[i] = keys ? (float)k[d] : 0.0f;
+  }
+  const int first = wave * kCols;
+  if (first < a.vdim) request(first);
+  const int c0 = min(tid, a.vdim - 1);
+  float norm = a.norm[c0], z = a.gate ? (float)gate[c0] : 0.0f;
+  const bool fresh = a.pos.position() == 0;
+  float dv[DPL];
+#pragma unroll
+  for (int i = 0; i < DPL; ++i) {
+    decay_and_key(gv[i], keys, kv[i], dv[i], kv[i]);
+    qv[i] *= a.q_scale;
+    if (i * 64 + lane >= a.dim) qv[i] = kv[i] = dv[i] = 0.0f;
+  }
+  for (int col0 = first; col0 < a.vdim; col0 += waves * kCols) {
+    if (col0 != first) request(col0);
+    float out[kCols];
+#pragma unroll
+    for (int c = 0; c < kCols; ++c) {
+      const float one = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(vv), c));
+      out[c] = 0.0f;
+#pragma unroll
+      for (int i = 0; i < DPL; ++i) {
+        s[c][i] = __builtin_fmaf(kv[i], one, dv[i] * (fresh ? 0.0f : s[c][i]));
+        out[c] = __builtin_fmaf(s[c][i], qv[i], out[c]);
+      }
+      if (col0 + c < a.vdim)
+#pragma unroll
+        for (int i = 0; i < DPL; ++i) a.state[((int64_t)head * a.vdim + col0 + c) * dimp + i * 64 + lane] = s[c][i];
+    }
+    ended_sums(out, lane);
+    const int c = lane / (64 / kCols);
+    if (lane % (64 / kCols) == 0 && col0 + c < a.vdim) row[col0 + c] = out[0];
+  }
+  __syncthreads();
+  float sq = 0.0f;
+  for (int c = tid; c < a.vdim; c += blockDim.x) sq = __builtin_fmaf(row[c], row[c], sq);
+  sq = lanes::sum(sq);
+  if (lane == 0) sums[wave] = sq;
+  __syncthreads();
+  const float all = lanes::sum<16>((lane & 15) < waves ? sums[lane & 15] : 0.0f);
+  const float inv = 1.0f / sqrtf(all / (float)a.vdim + a.eps);
+  T* ctx = reinterpret_cast<T*>(a.ctx) + (int64_t)head * a.vdim;
+  for (int c = tid; c < a.vdim; c += blockDim.x) {
+    if (c != tid) norm = a.norm[c], z = a.gate ? (float)gate[c] : 0.0f;
+    float y = row[c] * inv * norm;
+    if (a.gate) y *= z / (1.0f + expf(-z));
+    ctx[c] = (T)y;
+  }
 }
 
 template <typename T, int DPL, bool HEAD>
@@ -610,12 +684,12 @@ void launch_steps(const GatedStateArgs& a, hipStream_t st) {
   constexpr int kHeadCols = DPL <= 4 ? 8 : 4, kCols = 4;
   const auto groups = [&](int cols) { return dim3((unsigned)a.heads, (unsigned)((a.vdim + 4 * cols - 1) / (4 * cols))); };
   if (a.ctx)
-    hipLaunchKernelGGL((gated_step_kernel<T, DPL, true, kHeadCols>), dim3((unsigned)a.heads),
+    hipLaunchKernelGGL((gated_head_kernel<T, DPL, kHeadCols>), dim3((unsigned)a.heads),
                        dim3((unsigned)std::min<int64_t>(1024, (a.vdim + kHeadCols - 1) / kHeadCols * 64)), (size_t)a.vdim * 4, st, a);
   else if (a.head_decay)
     hipLaunchKernelGGL((gated_few_kernel<T, DPL, true>), groups(few_cols<DPL>()), dim3(256), 0, st, a);
   else if (a.M == 1)
-    hipLaunchKernelGGL((gated_step_kernel<T, DPL, false, kCols>), groups(kCols), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((gated_step_kernel<T, DPL, kCols>), groups(kCols), dim3(256), 0, st, a);
   else
     hipLaunchKernelGGL((gated_few_kernel<T, DPL, false>), groups(few_cols<DPL>()), dim3(256), 0, st, a);
 }
