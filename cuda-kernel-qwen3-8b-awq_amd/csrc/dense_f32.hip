@@ -306,10 +306,13 @@ int launch_dense_one_f32(const DenseArgs& a, int64_t rows, hipStream_t st) {
 
 int launch_dense_one_joined_f32(const DenseArgs& a, const JoinArgs& j, int64_t rows, hipStream_t st) {
   const size_t lds = (size_t)a.k * 4;
+  bool pairs = false;
+  for (int i = 0; i < a.n_seg; ++i) pairs |= a.seg[i].act == DENSE_GLU;
   const auto launch = [&](auto q) {
     constexpr int Q = decltype(q)::value;
     if (rows >= 2048) hipLaunchKernelGGL((dense_one_f32_kernel<DENSE_STORE, 4, Q>), dim3((unsigned)(rows / 16)), dim3(256), lds, st, a, j);
-    else hipLaunchKernelGGL((dense_one_f32_kernel<DENSE_STORE, 2, Q>), dim3((unsigned)(rows / 8)), dim3(256), lds, st, a, j);
+    else if (pairs) hipLaunchKernelGGL((dense_one_f32_kernel<DENSE_STORE, 2, Q>), dim3((unsigned)(rows / 8)), dim3(256), lds, st, a, j);
+    else hipLaunchKernelGGL((dense_one_f32_kernel<DENSE_STORE, 1, Q>), dim3((unsigned)(rows / 4)), dim3(256), lds, st, a, j);
   };
   if (j.width <= 1024) launch(std::integral_constant<int, 1>{});
   else launch(std::integral_constant<int, 2>{});
