@@ -364,7 +364,7 @@ __global__ __launch_bounds__(NW * 64) void dense_few_kernel(DenseArgs a) {
 }
 
 // --- many tokens, bfloat16 ---------------------------------------------------------------------------------
-// A workgroup of four wavefronts takes 256 rows and 32 TT tokens: 64 rows per wavefront as 2 x TT accumulators of
+// A workgroup of four wavefronts takes 128 RB rows and 32 TT tokens: 32 RB rows per wavefront as RB x TT accumulators of
 // v_mfma_f32_32x32x16_bf16.  The weights go from memory into registers in operand order, every byte once per
 // workgroup; the tokens go through LDS (global_load_lds_dwordx4, 128 bytes per token and step of 64 inputs, the
 // eight 16-byte pieces of row r at positions c ^ (r & 7)).  Both are requested two steps ahead.  Where the tiles do not
@@ -373,7 +373,7 @@ __global__ __launch_bounds__(NW * 64) void dense_few_kernel(DenseArgs a) {
 // a wait for everything on its way at each barrier, 474); at few by the trips to memory (33 tokens, 4,096 x 4,096: 17.8,
 // was 19.9).
 // LISTED: the tokens come from runs of a list, each with a weight block of its own.
-template <int TT, int OUT, bool LISTED = false>
+template <int TT, int RB, int OUT, bool LISTED = false>
 __global__ __launch_bounds__(256, 2) void dense_many_kernel(DenseArgs a, int row_tiles, int tok_tiles, int cuts) {
   // three arrays, so that the compiler can tell which reads a request on its way may touch
   __shared__ __attribute__((aligned(16))) bf16_t tile0[32 * TT * 64];
@@ -398,7 +398,7 @@ __global__ __launch_bounds__(256, 2) void dense_many_kernel(DenseArgs a, int row
   }
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, kh = lane >> 5;
-  const DenseSegment& s = segment_of(a, rt * 256);
+  const DenseSegment& s = segment_of(a, rt * 128 * RB);
   const int all_steps = (int)(a.k >> 6);
   const int first_step = (int)((int64_t)all_steps * cut / cuts);
   const int steps = (int)((int64_t)all_steps * (cut + 1) / cuts) - first_step;
@@ -423,16 +423,16 @@ __global__ __launch_bounds__(256, 2) void dense_many_kernel(DenseArgs a, int row
     }
   };
   const bf16x8_t* wp = reinterpret_cast<const bf16x8_t*>(reinterpret_cast<const bf16_t*>(a.w) + group * a.w_batch) +
-                       ((int64_t)(rt * 8 + wave * 2) * k16 + first_step * 4) * 64;
-  auto weights = [&](bf16x8_t (&wv)[2][4], int step, int j) __attribute__((always_inline)) {
+                       ((int64_t)(rt * 4 + wave) * RB * k16 + first_step * 4) * 64;
+  auto weights = [&](bf16x8_t (&wv)[RB][4], int step, int j) __attribute__((always_inline)) {
     const int at = step < steps ? lane : 0;
     step = min(step, steps - 1);
 #pragma unroll
-    for (int b = 0; b < 2; ++b) wv[b][j] = wp[(b * k16 + step * 4 + j) * 64 + at];
+    for (int b = 0; b < RB; ++b) wv[b][j] = wp[(b * k16 + step * 4 + j) * 64 + at];
   };
-  f32x16_t acc[2][TT];
+  f32x16_t acc[RB][TT];
 #pragma unroll
-  for (int b = 0; b < 2; ++b)
+  for (int b = 0; b < RB; ++b)
 #pragma unroll
     for (int t = 0; t < TT; ++t)
 #pragma unroll
@@ -441,11 +441,11 @@ __global__ __launch_bounds__(256, 2) void dense_many_kernel(DenseArgs a, int row
 #pragma unroll
     for (int t = 0; t < TT; ++t) xv[t] = *reinterpret_cast<const bf16x8_t*>(tile + (32 * t + n) * 64 + (((2 * j + kh) ^ (n & 7)) << 3));
   };
-  auto multiply = [&](const bf16x8_t (&wv)[2][4], int j, const bf16x8_t (&xv)[TT]) __attribute__((always_inline)) {
+  auto multiply = [&](const bf16x8_t (&wv)[RB][4], int j, const bf16x8_t (&xv)[TT]) __attribute__((always_inline)) {
 #pragma unroll
     for (int t = 0; t < TT; ++t)
 #pragma unroll
-      for (int b = 0; b < 2; ++b) acc[b][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv[b][j], xv[t], acc[b][t], 0, 0, 0);
+      for (int b = 0; b < RB; ++b) acc[b][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv[b][j], xv[t], acc[b][t], 0, 0, 0);
   };
   // The order in which a slice of a step (16 of its inputs) is issued: the next slice's reads between the first products, the
   // weights of two steps on behind them.
@@ -455,18 +455,18 @@ __global__ __launch_bounds__(256, 2) void dense_many_kernel(DenseArgs a, int row
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
     }
-    __builtin_amdgcn_sched_group_barrier(0x008, TT, 0);
-    __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);
+    if (RB == 2) __builtin_amdgcn_sched_group_barrier(0x008, TT, 0);
+    __builtin_amdgcn_sched_group_barrier(0x020, RB, 0);
   };
   // Step st multiplies tile st % 3 and set st % 2 of the weights.  Both were requested two steps ago, so that a trip to memory
-  // has two steps of products to hide behind: at the wait the 8 + TT requests of the step between may still be on their
+  // has two steps of products to hide behind: at the wait the 4 RB + TT requests of the step between may still be on their
   // way.  A slice's weights are requested into the registers that the slice has just used.  Past the end every lane
   // requests the same piece, which is not used.  The compiler need not keep the weights' requests of those steps: at the
-  // wait ahead of a last step the youngest 8 + TT are then TT past the end and the 8 for that step's own weights, whose
+  // wait ahead of a last step the youngest 4 RB + TT are then TT past the end and the 4 RB for that step's own weights, whose
   // use waits for them.  That leaves no request to spare, and needs a step's tokens to be requested ahead of its weights.
-  bf16x8_t w0[2][4], w1[2][4];
-  auto step = [&](const bf16_t* now, bf16x8_t (&w)[2][4], bf16_t* later, int st) __attribute__((always_inline)) {
-    __builtin_amdgcn_s_waitcnt(0x0f70 | (8 + TT));  // vmcnt(8 + TT)
+  bf16x8_t w0[RB][4], w1[RB][4];
+  auto step = [&](const bf16_t* now, bf16x8_t (&w)[RB][4], bf16_t* later, int st) __attribute__((always_inline)) {
+    __builtin_amdgcn_s_waitcnt(0x0f70 | (4 * RB + TT));  // vmcnt(4 RB + TT)
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();  // this step's tile is whole, the readers of the tile ahead of it are done
     asm volatile("" ::: "memory");
@@ -519,13 +519,13 @@ __global__ __launch_bounds__(256, 2) void dense_many_kernel(DenseArgs a, int row
       }
     }
   }
-  const int row_w = rt * 256 + wave * 64;
+  const int row_w = (rt * 4 + wave) * 32 * RB;
   float* const turn = reinterpret_cast<float*>(TT == 4 ? tile0 : (wave < 2 ? tile0 : tile1)) + (TT == 4 ? wave : wave & 1) * 1024;
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): no request is on its way into the tiles any more
   __syncthreads();                     // the last step's readers are done
 #pragma unroll
-  for (int b = 0; b < 2; ++b)
-    store_block_rows<bf16_t, OUT, LISTED>(a, turn, acc[b], row_w + 32 * b, tt0, n_tok, list, row_tiles * 256, cut);
+  for (int b = 0; b < RB; ++b)
+    store_block_rows<bf16_t, OUT, LISTED>(a, turn, acc[b], row_w + 32 * b, tt0, n_tok, list, row_tiles * 128 * RB, cut);
 }
 
 template <typename S>
@@ -649,70 +649,80 @@ int launch_few(const DenseArgs& a, int64_t rows, int tokens, int blocks, hipStre
   return AWQ_OK;
 }
 
-// The time of a product of many tokens in us, but for what all forms of it share: what a choice between tiles of 64 and 128
-// tokens and numbers of shares of k needs.  A step of a workgroup that has its compute unit to itself waits for memory, the
-// longer the more weights are on their way; a second workgroup on the unit adds its products; weights out of memory; tokens out
-// of the L2s; the end of a tile; the shares' sums, written, read and added one after the other.  The numbers are fitted for the
-// choice, not for the time, to 27,100 timings (152 shapes from 256 x 64 to 32,768 x 4,096 and 8,192 x 16,384, 2 to 2,048 tokens, both
-// tiles, 1 to 16 shares, weights from memory).  From 33 tokens on the form it picks takes 1.0 % longer on average than the fastest
-// timed, 20 % at most, and 11 % at most than tiles of 128 from 65 tokens on and 512 workgroups whatever the size; without the end of
-// a tile and the time per share 2.4, 28 and 18 % (2,048 x 4,096 at 64 tokens 18.7 us, now 15.4).
-float many_time(const DenseArgs& a, int64_t rows, bool wide, int64_t cuts) {
-  const int64_t row_tiles = rows / 256, tile = wide ? 128 : 64, tok_tiles = (a.M + tile - 1) / tile;
+// The forms of a product of many tokens: tiles of 256 or 128 rows and 64 or 128 tokens.  Small tiles put more workgroups on the
+// device, and three or four of them on a compute unit instead of two, so that fewer shares of k (and often no second launch) are
+// needed; large ones read less.  2,048 x 2,048 at 129 tokens 14.2 -> 11.9 us with 128 rows, 8,192 x 2,048 18.2 -> 13.2, 4,096 x 4,096
+// at 512 30.8 -> 23.4, 1,024 x 1,024 at 64 to 1,024 tokens 12 -> 8.4.
+struct ManyForm {
+  int tt, rb;         // 32 tt tokens, 128 rb rows
+  int resident;       // workgroups that the device holds
+  float wait, root;   // a step of a workgroup that has its unit to itself waits for memory, the longer the more weights are on their way
+  float step;         // a step of one of several workgroups
+  float end;          // the end of a tile
+};
+constexpr ManyForm kManyForms[4] = {{2, 2, 512, 0.388f, 0.0136f, 0.450f, 0.766f},
+                                    {2, 1, 1024, 0.219f, 0.0205f, 0.292f, 0.0f},
+                                    {4, 2, 512, 0.316f, 0.0432f, 0.596f, 2.715f},
+                                    {4, 1, 768, 0.396f, 0.0074f, 0.393f, 0.763f}};
+
+// The time of a product in us, but for what all forms of it share: what the choice of a form and of a number of shares of k needs.
+// Weights out of memory; what workgroups take in; the shares' sums, written, read and added one after the other.  The numbers are
+// fitted for the choice, not for the time, to 18,400 timings (31 shapes from 256 x 64 to 32,768 x 1,024 and 28,672 x 4,096, 33 to
+// 2,048 tokens, all forms, 1 to 16 shares, weights from memory).  The form it picks takes 0.7 % longer on average than the fastest
+// timed, 10 % at the 99th of 100 and 18 % at most; the fastest with 256 rows 16 % on average.
+float many_time(const DenseArgs& a, int64_t rows, const ManyForm& f, int64_t cuts) {
+  const int64_t row_tiles = rows / (128 * f.rb), tok_tiles = (a.M + 32 * f.tt - 1) / (32 * f.tt);
   const float groups = (float)(row_tiles * tok_tiles * cuts * a.batch), steps = (float)(((a.k >> 6) + cuts - 1) / cuts);
-  const float wait = (wide ? 0.47f : 0.332f) + 0.048f * sqrtf((float)std::min<int64_t>(256, row_tiles * cuts * a.batch));
+  const float wait = f.wait + f.root * sqrtf((float)std::min<int64_t>(256, row_tiles * cuts * a.batch));
   const float per_unit = ceilf(groups / 256.0f);
-  float t = steps * wait * ceilf(groups / 512.0f);
-  if (per_unit > 1.0f) t = std::max(t, steps * per_unit * (wide ? 0.78f : 0.76f));
-  t = std::max(t, (float)rows * (float)a.k * (float)a.batch * 2.0f / 5.86e6f);
-  t = std::max(t, groups * steps * (float)(32768 + tile * 128) / 25e6f) + per_unit * (wide ? 2.04f : 0.9f);
-  if (cuts > 1) t += 0.11f + (float)cuts * (0.325f + (float)a.M * (float)rows * 8.0f / 4.55e6f);
+  float t = steps * wait * ceilf(groups / (float)f.resident);
+  if (per_unit > 1.0f) t = std::max(t, steps * per_unit * f.step);
+  t = std::max(t, (float)rows * (float)a.k * (float)a.batch * 2.0f / 6.63e6f);
+  t = std::max(t, groups * steps * (float)(16384 * f.rb + f.tt * 4096) / 108.6e6f) + per_unit * f.end;
+  if (cuts > 1) t += 1.65f + (float)cuts * (0.244f + (float)a.M * (float)rows * 8.0f / 3.33e6f);
   return t;
+}
+
+template <int OUT, bool LISTED>
+void launch_form(const DenseArgs& a, const ManyForm& f, int64_t rows, int64_t tok_tiles, int64_t cuts, hipStream_t st) {
+  const int row_tiles = (int)(rows / (128 * f.rb));
+  const dim3 grid((unsigned)((row_tiles * tok_tiles * cuts + 7) / 8 * 8), (unsigned)a.batch), b(256);
+  if (f.tt == 2 && f.rb == 2) hipLaunchKernelGGL((dense_many_kernel<2, 2, OUT, LISTED>), grid, b, 0, st, a, row_tiles, (int)tok_tiles, (int)cuts);
+  else if (f.tt == 2) hipLaunchKernelGGL((dense_many_kernel<2, 1, OUT, LISTED>), grid, b, 0, st, a, row_tiles, (int)tok_tiles, (int)cuts);
+  else if (f.rb == 2) hipLaunchKernelGGL((dense_many_kernel<4, 2, OUT, LISTED>), grid, b, 0, st, a, row_tiles, (int)tok_tiles, (int)cuts);
+  else hipLaunchKernelGGL((dense_many_kernel<4, 1, OUT, LISTED>), grid, b, 0, st, a, row_tiles, (int)tok_tiles, (int)cuts);
 }
 
 template <int OUT>
 int launch_many(const DenseArgs& a, int64_t rows, hipStream_t st) {
-  // A product of few tokens goes the way whose time is estimated to be the shorter; what the other way's estimate leaves out is 8.9 us
+  // A product of few tokens goes the way whose time is estimated to be the shorter; what the other way's estimate leaves out is 6.5 us
   // more.  Workgroups that leave compute units idle and long rows, which read the tokens more than the weights, are against
-  // the few-token kernel: 6,144 x 12,288 at 20 tokens 54 us, below 36; 28,672 x 4,096 at 32 59 and 51.  Of 480 products (48
-  // shapes from 256 x 512 to 28,672 x 12,288, 2 to 32 tokens, both ways timed) the choice is 0.2 % off on average and 9 % at most;
-  // with up to 20 tokens always there, and up to 32 from 8,192 rows or to 4,096 inputs, 2.3 and 67 %.
-  constexpr float kManyMore = 8.9f;
+  // the few-token kernel: 6,144 x 12,288 at 20 tokens 54 us, below 36.  Of 310 products (31 shapes from 256 x 64 to 28,672 x 4,096, 2
+  // to 32 tokens, both ways timed) the choice is 0.2 % off on average and 13 % at most.
+  constexpr float kManyMore = 6.5f;
   const float few = a.M <= kFewTokens ? few_time(a, rows) : HUGE_VALF;
   if (few < kManyMore) return launch_few<OUT, false>(a, rows, (int)a.M, a.batch, st);
-  const int row_tiles = (int)(rows / 256);
   int64_t most = 1;  // shares of k: at least four steps each
   if (a.workspace && a.batch == 1 && a.M <= 65535)
     most = std::max<int64_t>(1, std::min(std::min<int64_t>(16, a.k >> 8), a.workspace_floats / (a.M * rows)));
-  bool wide = false;
+  const ManyForm* form = nullptr;
   int64_t cuts = 1;
   float best = HUGE_VALF;
-  for (int w = 0; w < 2; ++w)
+  for (const ManyForm& f : kManyForms)
     for (int64_t c = 1; c <= most; ++c) {
-      const float t = many_time(a, rows, w != 0, c);
-      if (t < best) best = t, wide = w != 0, cuts = c;
+      const float t = many_time(a, rows, f, c);
+      if (t < best) best = t, form = &f, cuts = c;
     }
+  if (!form) form = &kManyForms[2];  // (a product too long for the estimate)
   if (few < best + kManyMore) return launch_few<OUT, false>(a, rows, (int)a.M, a.batch, st);
-  // With few steps most of the time is the end of a tile, for which the estimate has one number of each size of tile:
-  // at up to 512 inputs tiles of 64 are the faster ones wherever all of them are on the device at once (36 of 36 timed,
-  // by 4 to 32 %: 4,096 x 256 at 2,048 tokens 15.6 us against 18.1, 2,048 x 256 11.5 against 16.6).  Where they are not, or k is
-  // longer, it goes either way and the estimate decides.
-  if (wide && cuts == 1 && a.k <= 512 && row_tiles * ((a.M + 63) / 64) * a.batch <= 512) wide = false;
-  const int64_t tok_tiles = wide ? (a.M + 127) / 128 : (a.M + 63) / 64;
-  const int64_t tiles = row_tiles * tok_tiles;
-  const dim3 grid((unsigned)((tiles * cuts + 7) / 8 * 8), (unsigned)a.batch);
+  const int64_t tok_tiles = (a.M + 32 * form->tt - 1) / (32 * form->tt);
   if (cuts > 1) {
-    if (wide)
-      hipLaunchKernelGGL((dense_many_kernel<4, DENSE_PART>), grid, dim3(256), 0, st, a, row_tiles, (int)tok_tiles, (int)cuts);
-    else
-      hipLaunchKernelGGL((dense_many_kernel<2, DENSE_PART>), grid, dim3(256), 0, st, a, row_tiles, (int)tok_tiles, (int)cuts);
+    launch_form<DENSE_PART, false>(a, *form, rows, tok_tiles, cuts, st);
     AWQ_HIP_TRY(hipGetLastError());
     hipLaunchKernelGGL((dense_parts_kernel<bf16_t, OUT>), dim3((unsigned)((rows / 4 + 255) / 256), (unsigned)a.M), dim3(256), 0, st, a,
                        (int)rows, (int)cuts);
-  } else if (wide) {
-    hipLaunchKernelGGL((dense_many_kernel<4, OUT>), grid, dim3(256), 0, st, a, row_tiles, (int)tok_tiles, 1);
   } else {
-    hipLaunchKernelGGL((dense_many_kernel<2, OUT>), grid, dim3(256), 0, st, a, row_tiles, (int)tok_tiles, 1);
+    launch_form<OUT, false>(a, *form, rows, tok_tiles, 1, st);
   }
   AWQ_HIP_TRY(hipGetLastError());
   return AWQ_OK;
@@ -721,12 +731,11 @@ int launch_many(const DenseArgs& a, int64_t rows, hipStream_t st) {
 // tokens with weight blocks of their own
 int launch_listed(const DenseArgs& a, int64_t rows, hipStream_t st) {
   if (a.tile_tokens <= kFewTokens) return launch_few<DENSE_STORE, true>(a, rows, a.tile_tokens, a.max_tiles, st);
-  const int row_tiles = (int)(rows / 256);
-  const unsigned grid = (unsigned)(((int64_t)row_tiles * a.max_tiles + 7) / 8 * 8);
-  if (a.tile_tokens <= 64)
-    hipLaunchKernelGGL((dense_many_kernel<2, DENSE_STORE, true>), dim3(grid), dim3(256), 0, st, a, row_tiles, a.max_tiles, 1);
-  else
-    hipLaunchKernelGGL((dense_many_kernel<4, DENSE_STORE, true>), dim3(grid), dim3(256), 0, st, a, row_tiles, a.max_tiles, 1);
+  // 128 rows where 64 tokens meet a weight block, and where 128 do and 256 rows would be at most two workgroups per compute unit, of
+  // which not all have tokens: Tudasun 2,048 at 129 tokens 1,010 -> 957 us, 1,536 at 300 (128 tokens) 888 -> 856; 4,096 at 1,024, 1,104
+  // workgroups of 256 rows, 3,436 and with 128 rows 3,608
+  const bool few_groups = rows / 256 * a.max_tiles <= 512;
+  launch_form<DENSE_STORE, true>(a, kManyForms[a.tile_tokens <= 64 ? 1 : few_groups ? 3 : 2], rows, a.max_tiles, 1, st);
   AWQ_HIP_TRY(hipGetLastError());
   return AWQ_OK;
 }

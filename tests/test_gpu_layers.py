@@ -243,6 +243,36 @@ def test_products_of_every_number_of_steps(awq, lib, dev, tokens, steps):
         assert np.abs(got[:tokens] - xv @ wv.T).max() < 8 * k ** 0.5 * 2.0 ** -24
 
 
+# tiles of 128 and 256 rows and of 64 and 128 tokens, each alone and with its k in shares (as the estimate picks them with a workspace
+# of 2^22 floats), rows and tokens that end inside a tile
+@pytest.mark.parametrize("rows,k,tokens", [(100, 64, 33), (100, 1088, 33), (12300, 512, 257), (4200, 4160, 129), (2100, 320, 1000),
+                                           (8200, 2112, 65), (4200, 320, 1500), (1000, 1088, 200), (130, 2112, 700)])
+def test_products_of_many_tokens_in_every_form(awq, lib, dev, rows, k, tokens):
+    """all three outputs; the operands are exact: a sum of k products in binary32 is off by about sqrt(k) roundings of 2^-24 of its size"""
+    print("forms", rows, k, tokens, flush=True)
+    rng = np.random.default_rng(rows + tokens)
+    block = dev.torch.zeros((rows + 255) // 256 * 256 * k, dtype=dev.torch.bfloat16, device="cuda")
+    w, wv = dev.act(rng.standard_normal((rows, k)) / k ** 0.5, False)
+    awq.check(lib.awq_dense_pack(w.data_ptr(), 0, rows, k, block.data_ptr(), k, 0, 0, 0, dev.stream))
+    x, xv = dev.act(rng.standard_normal((tokens, k)), False)
+    want = xv @ wv.T
+    ws = dev.empty((1 << 22,), True)
+    exact = 8 * k ** 0.5 * 2.0 ** -24
+    for out in (awq.DENSE_F32, awq.DENSE_RESIDUAL, awq.DENSE_STORE):
+        y = dev.empty((tokens + 1, rows), out != awq.DENSE_STORE, fill=0.5)
+        y[tokens] = float("nan")
+        a = awq.AwqDenseArgs()
+        a.w, a.k, a.tokens, a.n_segments, a.out = block.data_ptr(), k, tokens, 1, out
+        a.segment[0] = awq.AwqDenseSegment(x.data_ptr(), y.data_ptr(), k, rows, 0, rows, 0, 0, 0, 0)
+        a.workspace, a.workspace_floats = ws.data_ptr(), ws.numel()
+        awq.check(lib.awq_dense(ctypes.byref(a), 0, dev.stream))
+        got = dev.host(y)
+        assert np.isnan(got[tokens]).all()
+        off = np.abs(got[:tokens] - want - (0.5 if out == awq.DENSE_RESIDUAL else 0.0))
+        # (the residual's own rounding; a bfloat16 output has 8 bits, half a unit of the last is at most 2^-8 of its value)
+        assert (off <= exact + (2.0 ** -8 * np.abs(want) if out == awq.DENSE_STORE else 8 * 2.0 ** -24)).all()
+
+
 @pytest.mark.parametrize("k", [64, 320, 512, 576])
 @pytest.mark.parametrize("rows,tokens", [(2000, 2001), (8200, 1030)])
 def test_products_of_few_inputs_and_many_tokens(awq, lib, dev, rows, tokens, k):
