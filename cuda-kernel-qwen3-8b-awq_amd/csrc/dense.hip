@@ -1,3 +1,5 @@
+#include <cstdlib>
+#include <cstdio>
 // Dense products of bfloat16 weights with one token or many, packing of weights, the launch of any product (layers.hpp).
 #include "dense_device.hpp"
 #include "join_device.hpp"
@@ -670,6 +672,10 @@ constexpr ManyForm kManyForms[4] = {{2, 2, 512, 0.388f, 0.0136f, 0.450f, 0.766f}
 // fitted for the choice, not for the time, to 18,400 timings (31 shapes from 256 x 64 to 32,768 x 1,024 and 28,672 x 4,096, 33 to
 // 2,048 tokens, all forms, 1 to 16 shares, weights from memory).  The form it picks takes 0.7 % longer on average than the fastest
 // timed, 10 % at the 99th of 100 and 18 % at most; the fastest with 256 rows 16 % on average.
+float weights_time(const DenseArgs& a, int64_t rows) { return (float)rows * (float)a.k * (float)a.batch * 2.0f / 6.63e6f; }
+float shares_time(const DenseArgs& a, int64_t rows, int64_t cuts) {
+  return 1.65f + (float)cuts * (0.244f + (float)a.M * (float)rows * 8.0f / 3.33e6f);
+}
 float many_time(const DenseArgs& a, int64_t rows, const ManyForm& f, int64_t cuts) {
   const int64_t row_tiles = rows / (128 * f.rb), tok_tiles = (a.M + 32 * f.tt - 1) / (32 * f.tt);
   const float groups = (float)(row_tiles * tok_tiles * cuts * a.batch), steps = (float)(((a.k >> 6) + cuts - 1) / cuts);
@@ -677,10 +683,9 @@ float many_time(const DenseArgs& a, int64_t rows, const ManyForm& f, int64_t cut
   const float per_unit = ceilf(groups / 256.0f);
   float t = steps * wait * ceilf(groups / (float)f.resident);
   if (per_unit > 1.0f) t = std::max(t, steps * per_unit * f.step);
-  t = std::max(t, (float)rows * (float)a.k * (float)a.batch * 2.0f / 6.63e6f);
+  t = std::max(t, weights_time(a, rows));
   t = std::max(t, groups * steps * (float)(16384 * f.rb + f.tt * 4096) / 108.6e6f) + per_unit * f.end;
-  if (cuts > 1) t += 1.65f + (float)cuts * (0.244f + (float)a.M * (float)rows * 8.0f / 3.33e6f);
-  return t;
+  return cuts > 1 ? t + shares_time(a, rows, cuts) : t;
 }
 
 template <int OUT, bool LISTED>
@@ -701,7 +706,8 @@ int launch_many(const DenseArgs& a, int64_t rows, hipStream_t st) {
   // to 32 tokens, both ways timed) the choice is 0.2 % off on average and 13 % at most.
   constexpr float kManyMore = 6.5f;
   const float few = a.M <= kFewTokens ? few_time(a, rows) : HUGE_VALF;
-  if (few < kManyMore) return launch_few<OUT, false>(a, rows, (int)a.M, a.batch, st);
+  // (the other way takes at least the weights' time: mostly known without an estimate of its forms)
+  if (few < weights_time(a, rows) + kManyMore) return launch_few<OUT, false>(a, rows, (int)a.M, a.batch, st);
   int64_t most = 1;  // shares of k: at least four steps each
   if (a.workspace && a.batch == 1 && a.M <= 65535)
     most = std::max<int64_t>(1, std::min(std::min<int64_t>(16, a.k >> 8), a.workspace_floats / (a.M * rows)));
@@ -709,10 +715,11 @@ int launch_many(const DenseArgs& a, int64_t rows, hipStream_t st) {
   int64_t cuts = 1;
   float best = HUGE_VALF;
   for (const ManyForm& f : kManyForms)
-    for (int64_t c = 1; c <= most; ++c) {
+    for (int64_t c = 1; c <= most && (c == 1 || shares_time(a, rows, c) < best); ++c) {
       const float t = many_time(a, rows, f, c);
       if (t < best) best = t, form = &f, cuts = c;
     }
+  if (const char* e = getenv("MX")) { int tt, rb, c; sscanf(e, "%d,%d,%d", &tt, &rb, &c); for (const ManyForm& f : kManyForms) if (f.tt == tt && f.rb == rb) form = &f; cuts = c; }
   if (!form) form = &kManyForms[2];  // (a product too long for the estimate)
   if (few < best + kManyMore) return launch_few<OUT, false>(a, rows, (int)a.M, a.batch, st);
   const int64_t tok_tiles = (a.M + 32 * form->tt - 1) / (32 * form->tt);
