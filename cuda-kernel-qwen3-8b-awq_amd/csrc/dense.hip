@@ -1,5 +1,3 @@
-#include <cstdlib>
-#include <cstdio>
 // Dense products of bfloat16 weights with one token or many, packing of weights, the launch of any product (layers.hpp).
 #include "dense_device.hpp"
 #include "join_device.hpp"
@@ -719,7 +717,6 @@ int launch_many(const DenseArgs& a, int64_t rows, hipStream_t st) {
       const float t = many_time(a, rows, f, c);
       if (t < best) best = t, form = &f, cuts = c;
     }
-  if (const char* e = getenv("MX")) { int tt, rb, c; sscanf(e, "%d,%d,%d", &tt, &rb, &c); for (const ManyForm& f : kManyForms) if (f.tt == tt && f.rb == rb) form = &f; cuts = c; }
   if (!form) form = &kManyForms[2];  // (a product too long for the estimate)
   if (few < best + kManyMore) return launch_few<OUT, false>(a, rows, (int)a.M, a.batch, st);
   const int64_t tok_tiles = (a.M + 32 * form->tt - 1) / (32 * form->tt);

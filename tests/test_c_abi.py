@@ -206,3 +206,10 @@ def test_gemm_plan_for_the_model_matrices(lib):
     assert [plan(wo, M) for M in (65, 128, 193, 512)] == [K_SPLIT] * 4 and [plan(wo, M) for M in (129, 192)] == [6] * 2
     assert [plan(wo, M) for M in (576, 1024, 1280)] == [ROWS_64] * 3
     assert plan(wo, 2048) == ROWS and plan(wo, 2560) == ROWS_64 and plan(wo, 4096) == ROWS
+
+
+def test_the_library_does_not_read_the_environment(lib):
+    """what a product or a model does is settled by its arguments: no variable of the process reaches a launch"""
+    csrc = os.path.join(ROOT, "cuda-kernel-qwen3-8b-awq_amd", "csrc")
+    reads = [f for f in sorted(os.listdir(csrc)) if re.search(r"\b(secure_)?getenv\b|\benviron\b", open(os.path.join(csrc, f)).read())]
+    assert reads == []
