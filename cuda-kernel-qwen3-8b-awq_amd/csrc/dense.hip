@@ -786,6 +786,15 @@ bool dense_join_fused(const JoinArgs& j, int64_t rows, bool f32) {
          ((j.width | j.ldo | j.ldg | j.ldh) & 3) == 0 && j.ldo % kDenseKAlign == 0 && rows * j.width <= 16 << 20;
 }
 
+// every workgroup reads the operands of the end, the last of them behind the first one's outputs
+static bool writes_operand_of(const DenseArgs& a, const JoinArgs& j) {
+  const void* const operands[] = {j.x, j.y, j.y_gate, j.pairs, j.ids, j.weights, j.top > 0 ? j.h : nullptr, j.gate};
+  for (int i = 0; i < a.n_seg; ++i)
+    for (const void* p : operands)
+      if (p && p == a.seg[i].y) return true;
+  return false;
+}
+
 int launch_dense(const DenseArgs& args, bool f32, hipStream_t st, const NormConvArgs* norm, const JoinArgs* join) {
   DenseArgs a = args;
   AWQ_REQUIRE(a.w && a.M >= 1 && a.k > 0 && a.k % kDenseKAlign == 0, "bad product");
@@ -829,6 +838,7 @@ int launch_dense(const DenseArgs& args, bool f32, hipStream_t st, const NormConv
     AWQ_REQUIRE(dense_join_fused(*join, rows, f32) && a.M == 1 && a.k == join->ldo && a.batch == 1 && !a.ids && !a.gate_o && a.out == DENSE_STORE &&
                     join->x && join->w_post && (join->y || join->top > 0),
                 "the end of the sublayer cannot be part of this product");
+    AWQ_REQUIRE(!writes_operand_of(a, *join), "the product writes what the end of the sublayer in it reads");
     return f32 ? launch_dense_one_joined_f32(a, *join, rows, st) : launch_one_joined(a, *join, rows, st);
   }
   if (f32) return a.M == 1 ? launch_dense_one_f32(a, rows, st) : launch_dense_many_f32(a, rows, st);

@@ -128,7 +128,7 @@ struct NormConvArgs;
 // neither is written, and what the segments name as x is not read
 struct JoinArgs;
 // join (one token, DENSE_STORE, where dense_join_fused says so of a product of `rows` padded rows): launch_join is part of the
-// product, its result the segments' input; x_out and out are written, x stays
+// product, its result the segments' input; x_out and out are written, x stays, and no segment's y is an operand of it
 int launch_dense(const DenseArgs& a, bool f32, hipStream_t st, const NormConvArgs* norm = nullptr, const JoinArgs* join = nullptr);
 bool dense_join_fused(const JoinArgs& j, int64_t rows, bool f32);
 bool dense_norm_fused(const NormConvArgs& n, bool f32);

@@ -296,6 +296,10 @@ struct TudasunEngine final : ConfigModel {
   // the end of a sublayer that is part of the product behind it
   JoinArgs waiting;
   bool is_waiting = false;
+  // A sublayer's product writes its gate while its workgroups still read the gate of the one ahead, whose end waits in it: the
+  // sublayers of a pass, of whichever kind and layer, take turns at the two buffers.
+  void* gate_now = nullptr;
+  void* next_gate(const Buffers& b) { return gate_now = gate_now == b.gate ? b.gate2 : b.gate; }
   const JoinArgs* take_waiting() {
     const JoinArgs* const j = is_waiting ? &waiting : nullptr;
     is_waiting = false;
@@ -604,7 +608,7 @@ int TudasunEngine::mix(int i, Buffers& b, int64_t M, PassPos pos) {
       rows(b.proj, L.ldp, (int64_t)s.heads * (s.dim + s.rot));
       if (s.kv_from < 0) rows(b.down, s.rank + s.rot, s.rank + s.rot).y_f32 = 1;
     }
-    DenseSegment& g = rows(b.gate, ldg, width);
+    DenseSegment& g = rows(next_gate(b), ldg, width);
     g.act = DENSE_SIGMOID;
     g.bias = L.rg1_b;
     if (int rc = launch_dense(a, f32, stream, nullptr, take_waiting())) return rc;
@@ -676,7 +680,7 @@ int TudasunEngine::dense_feed_forward(int i, Buffers& b, int64_t M) {
   const LayerDev& L = layers[i];
   {
     DenseArgs a = product(L.mid.w, ld, M);
-    DenseSegment& g = segment(&a, b.h, ld, b.gate2, ldg, L.mid.at[0], width);
+    DenseSegment& g = segment(&a, b.h, ld, next_gate(b), ldg, L.mid.at[0], width);
     g.act = DENSE_SIGMOID;
     g.bias = L.rg2_b;
     segment(&a, b.h, ld, b.mid, L.ff_k, L.mid.at[1], s.ff);
@@ -698,7 +702,7 @@ int TudasunEngine::routed_feed_forward(int i, Buffers& b, int64_t M, JoinArgs* e
   float* const shared_y = beside ? b.pairs + (int64_t)s.top * width : b.y;
   {
     DenseArgs a = product(L.mid.w, ld, M);
-    DenseSegment& g = segment(&a, b.h, ld, b.gate2, ldg, L.mid.at[0], width);
+    DenseSegment& g = segment(&a, b.h, ld, next_gate(b), ldg, L.mid.at[0], width);
     g.act = DENSE_SIGMOID;
     g.bias = L.rg2_b;
     segment(&a, b.h, ld, b.router, s.outputs(), L.mid.at[1], s.outputs()).y_f32 = 1;
@@ -824,6 +828,7 @@ int TudasunEngine::run_pass(bool one, const int32_t* ids, int64_t M, PassPos pos
     return launch_join(e, f32, stream);
   };
   is_waiting = false;
+  gate_now = nullptr;
   for (int i = 0; i < n; ++i) {
     const LayerSpec& s = spec.layers[i];
     const LayerDev& L = layers[i];
@@ -855,7 +860,7 @@ int TudasunEngine::run_pass(bool one, const int32_t* ids, int64_t M, PassPos pos
       if (int rc = launch_dense(a, f32, stream)) return rc;
       JoinArgs e = ending();
       e.y = b.y;
-      e.gate = b.gate;
+      e.gate = gate_now;
       e.ldg = ldg;
       e.w_post = L.norm1b;
       int64_t next = L.mid.rows;
@@ -871,7 +876,7 @@ int TudasunEngine::run_pass(bool one, const int32_t* ids, int64_t M, PassPos pos
       JoinArgs e = ending();
       e.y = b.y;
       if (int rc = s.mlp == MLP_DENSE ? dense_feed_forward(i, b, M) : routed_feed_forward(i, b, M, &e)) return rc;
-      e.gate = b.gate2;
+      e.gate = gate_now;
       e.ldg = ldg;
       e.w_post = L.norm2b;
       const int64_t next = leaves(&e, spec.side > 0);

@@ -1,0 +1,69 @@
+"""What a product refuses before anything is launched (host code: the program below sees no device)."""
+import os
+import subprocess
+
+PKG = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "cuda-kernel-qwen3-8b-awq_amd")
+
+PROGRAM = r"""
+#include <stdio.h>
+
+#include "layers.hpp"
+
+int main() {
+  // places of 64 KB: none is read or written
+  auto place = [](int i) { return (void*)(((uintptr_t)i + 1) << 16); };
+  DenseArgs a;
+  a.w = place(0);
+  a.k = 256;
+  a.M = 1;
+  a.n_seg = 2;
+  for (int i = 0; i < 2; ++i) {
+    a.seg[i].x = place(1);
+    a.seg[i].ldx = 256;
+    a.seg[i].y = place(2 + i);
+    a.seg[i].ldy = 256;
+    a.seg[i].row0 = 256 * i;
+    a.seg[i].rows = 256;
+  }
+  JoinArgs j;
+  j.x = (float*)place(4);
+  j.x_out = (float*)place(5);
+  j.M = 1;
+  j.width = j.ldo = j.ldg = j.ldh = 256;
+  j.y = (const float*)place(6);
+  j.y_gate = (const float*)place(7);
+  j.pairs = (const float*)place(8);
+  j.ids = (const int32_t*)place(9);
+  j.weights = (const float*)place(10);
+  j.top = 2;
+  j.experts = 4;
+  j.h = place(11);
+  j.gate = place(12);
+  j.w_post = (const float*)place(13);
+  j.out = place(1);
+  const void* const reads[] = {j.x, j.y, j.y_gate, j.pairs, j.ids, j.weights, j.h, j.gate};
+  for (int f32 = 0; f32 < 2; ++f32) {
+    printf("%d\n", launch_dense(a, f32 != 0, nullptr, nullptr, &j));  // nothing shared: the launch alone fails here
+    for (const void* r : reads)
+      for (int i = 0; i < 2; ++i) {
+        DenseArgs b = a;
+        b.seg[i].y = const_cast<void*>(r);
+        printf("%d\n", launch_dense(b, f32 != 0, nullptr, nullptr, &j));
+      }
+  }
+}
+"""
+
+
+def test_a_product_does_not_write_what_the_sublayers_end_in_it_reads(awq, lib, tmp_path):
+    """every workgroup reads the end's operands: one that starts late would read another's outputs"""
+    src, exe = tmp_path / "args.cpp", str(tmp_path / "args")
+    src.write_text(PROGRAM)
+    subprocess.run(["/opt/rocm/bin/hipcc", "-x", "hip", "--offload-host-only", "-std=c++17", "-I" + os.path.join(PKG, "csrc"), str(src),
+                    "-o", exe, "-L" + PKG, "-lawq_infer", "-Wl,-rpath," + PKG], check=True, capture_output=True, text=True, timeout=300)
+    env = dict(os.environ, HIP_VISIBLE_DEVICES="-1", ROCR_VISIBLE_DEVICES="")
+    run = subprocess.run([exe], capture_output=True, text=True, timeout=100, env=env)
+    assert run.returncode == 0, run.stderr
+    got = [int(v) for v in run.stdout.split()]
+    bad_argument, no_device = 1, 3
+    assert got == ([no_device] + 16 * [bad_argument]) * 2

@@ -285,3 +285,29 @@ def test_single_tokens_whose_sublayers_end_in_the_next_product(awq, torch_gpu, t
     # value: far below the distance to the plain statement, which one-head layers of this size can have in bfloat16 (routers of
     # other choice among it), and so half of the limit that holds for that one
     assert km.rms_error(got, again) < LIMIT[dtype] / 2
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+@pytest.mark.parametrize("kinds", ["----", "-d--", "--e-", "d-d-"])
+def test_single_tokens_of_mixers_that_follow_each_other(awq, torch_gpu, tmp_path, kinds, dtype):
+    """layers without feed-forward ahead of others, no token input: a mixer's product forms the end of the mixer ahead, whose gate
+    it must not write.  More rows than one round of workgroups holds (1,024 of 8 wavefronts)"""
+    ff = {"-": None, "d": tm.dense(80), "e": tm.moe(3, 2, 32, identity=1, shared=64)}
+    cfg = tm.model(768, 96, [tm.gla(4, 512, 1024, 4.0, ff[kinds[0]]), tm.hgrn2(16, 128, 896, ff[kinds[1]]),
+                             tm.latent(2, 32, 8, 16, 64, mlp=ff[kinds[2]]), tm.gla(1, 16, 8, 2.0, ff[kinds[3]])])
+    w = tm.weights(cfg, 6)
+    km.write(str(tmp_path), cfg, w)
+    tokens = np.random.default_rng(4).integers(0, 96, 20).tolist()
+    want, margins = reference(cfg, w, tokens)
+    eng = awq.open_model(str(tmp_path), dtype=dtype, max_positions=64)
+    print("mixers", kinds, dtype, flush=True)
+    got = np.concatenate([eng.forward([t], [0]) for t in tokens])
+    eng.reset()
+    same = np.concatenate([eng.forward([t], [0]) for t in tokens])
+    eng.set_layer_tap(True)  # every end of a sublayer in a launch of its own
+    eng.reset()
+    again = np.concatenate([eng.forward([t], [0]) for t in tokens])
+    eng.close()
+    assert np.array_equal(got, same)
+    assert agrees(got, want, dtype, margins)
+    assert km.rms_error(got, again) < LIMIT[dtype] / 2  # (the orders of the norms' sums, as above)
