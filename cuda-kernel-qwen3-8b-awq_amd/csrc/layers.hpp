@@ -199,8 +199,10 @@ struct WindowAttnArgs {
   // one-token form: partial results of the parts a window is cut into
   float* parts = nullptr;
   int32_t len_bound = 0;  // >= positions the sequence will hold
-  int32_t* done = nullptr;  // [heads] zeros, left as zeros: the parts are added up in the same launch; null: in a second one
+  // [heads] zeros, left as zeros: the parts are added up in the same launch where window_counted_parts; null: always in a second one
+  int32_t* done = nullptr;
 };
+bool window_counted_parts(int32_t heads, int32_t kv_heads, int64_t window, int64_t max_pos);
 int32_t window_row_padded(int32_t dim);
 int64_t window_parts_floats(int32_t heads, int32_t vdim, int64_t window, int64_t max_pos);
 // Normalise q and k, append k and v, attend.  A value that is infinite or NaN leaves the positions that do not see it as they are;

@@ -115,10 +115,9 @@ __global__ __launch_bounds__(256) void window_query_kernel(WindowAttnArgs a) {
 // One token.  blockIdx.x: kv head and up to R of its query heads, blockIdx.y: 64 of the visible keys.  The rows a
 // workgroup needs are requested before anything else; every lane group normalises the queries for itself, and the
 // workgroup of the newest position takes its key and value from the projections and appends them.  A wavefront's
-// lane holds the weight of one key.  With more than one part the workgroup that counts itself in last adds the parts up, where
-// the caller has counters, otherwise a second launch does: that costs 4 us.  One part of 8 heads of 128: 8.2 us
-// and the second launch's 4.0, now 6.5 for both (of which the sums over lanes through LDS took 1.2); 64 tokens of Kugilix at width 1,024
-// after 960, 15 parts and four such layers: 14.5 -> 12.5 ms.
+// lane holds the weight of one key.  Sums over lanes go without LDS: 8 heads of 128 and one part 8.2 us with trips through it, 6.5 without.
+// Several parts are added up by a second launch, a workgroup per head, or where window_counted_parts says so by the workgroup that
+// counts itself in last.
 constexpr int kPartKeys = 64;
 
 __host__ __device__ inline int window_parts(int64_t window, int64_t max_pos) {
@@ -150,14 +149,21 @@ __device__ __forceinline__ void row_piece(const T* row, int at, int n, bool alig
   }
 }
 
-// A part's results leave the die and are read past its caches: another die's workgroup may add them up in the same launch.
-__device__ __forceinline__ void put_part(float* p, float v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+// SAME: the parts are added up in the launch that forms them.  They then leave the die as they are stored and are read past its
+// caches, since another die's workgroup may be the one that adds them.
+template <bool SAME>
+__device__ __forceinline__ void put_part(float* p, float v) {
+  if constexpr (SAME) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else *p = v;
+}
+template <bool SAME>
 __device__ __forceinline__ float get_part(const float* p) {
-  return __hip_atomic_load(const_cast<float*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if constexpr (SAME) return __hip_atomic_load(const_cast<float*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else return *p;
 }
 
 // One head's parts, [maximum, sum, context] each, by a workgroup of 256; red: 256 floats of LDS
-template <typename T>
+template <typename T, bool SAME>
 __device__ __forceinline__ void combine_parts(const WindowAttnArgs& a, int h, int n_parts, int parts, float* red) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int64_t ps = 2 + a.vdim;
@@ -165,15 +171,15 @@ __device__ __forceinline__ void combine_parts(const WindowAttnArgs& a, int h, in
   // columns, and as many runs of parts next to each other as there are threads left
   const int cols = min(256, a.vdim), runs = 256 / cols, run = tid / cols;
   float m = -INFINITY, l = 0.0f;
-  for (int s = lane; s < parts; s += 64) m = fmaxf(m, get_part(p + s * ps));
+  for (int s = lane; s < parts; s += 64) m = fmaxf(m, get_part<SAME>(p + s * ps));
   m = lanes::maximum(m);
-  for (int s = lane; s < parts; s += 64) l = __builtin_fmaf(expf(get_part(p + s * ps) - m), get_part(p + s * ps + 1), l);
+  for (int s = lane; s < parts; s += 64) l = __builtin_fmaf(expf(get_part<SAME>(p + s * ps) - m), get_part<SAME>(p + s * ps + 1), l);
   l = lanes::sum(l);
   for (int c = tid % cols; c < (a.vdim + cols - 1) / cols * cols; c += cols) {
     float x = 0.0f;
     if (run < runs && c < a.vdim)
 #pragma unroll 4
-      for (int s = run; s < parts; s += runs) x = __builtin_fmaf(expf(get_part(p + s * ps) - m), get_part(p + s * ps + 2 + c), x);
+      for (int s = run; s < parts; s += runs) x = __builtin_fmaf(expf(get_part<SAME>(p + s * ps) - m), get_part<SAME>(p + s * ps + 2 + c), x);
     red[tid] = x;
     __syncthreads();
     if (run == 0 && c < a.vdim) {
@@ -185,7 +191,7 @@ __device__ __forceinline__ void combine_parts(const WindowAttnArgs& a, int h, in
 }
 
 // U: cache rows of a lane, row length / 32
-template <typename T, int R, int U>
+template <typename T, int R, int U, bool SAME>
 __global__ __launch_bounds__(256) void window_decode_kernel(WindowAttnArgs a, int chunks) {
   extern __shared__ float red[];      // [4][R][vw]
   __shared__ float sc[R][kPartKeys];
@@ -308,7 +314,7 @@ __global__ __launch_bounds__(256) void window_decode_kernel(WindowAttnArgs a, in
     }
   __syncthreads();
   const int n_parts = gridDim.y;
-  const bool alone = n_parts == 1 || (a.done && parts == 1);
+  const bool alone = n_parts == 1 || (SAME && parts == 1);
 #pragma unroll
   for (int r = 0; r < R; ++r) {
     if (r >= nr) break;
@@ -316,24 +322,24 @@ __global__ __launch_bounds__(256) void window_decode_kernel(WindowAttnArgs a, in
     for (int c = tid; c < a.vdim; c += 256) {
       const float x = (red[r * vw + c] + red[(R + r) * vw + c]) + (red[(2 * R + r) * vw + c] + red[(3 * R + r) * vw + c]);
       if (alone) reinterpret_cast<T*>(a.ctx)[(int64_t)(h0 + r) * a.vdim + c] = (T)(x / pl[r]);
-      else put_part(mine + 2 + c, x);
+      else put_part<SAME>(mine + 2 + c, x);
     }
-    if (!alone && tid == 0) put_part(mine, pm[r]), put_part(mine + 1, pl[r]);
+    if (!alone && tid == 0) put_part<SAME>(mine, pm[r]), put_part<SAME>(mine + 1, pl[r]);
   }
-  if (alone || !a.done) return;
-  // the parts are out of this die when the workgroup counts itself in; the last one finds all of them
-  __shared__ int last;
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
-  if (tid == 0) {
-    last = __hip_atomic_fetch_add(a.done + blockIdx.x, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
-    if (last) __hip_atomic_store(a.done + blockIdx.x, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
-  }
-  __syncthreads();
-  if (!last) return;
-  for (int r = 0; r < nr; ++r) {
-    combine_parts<T>(a, h0 + r, n_parts, parts, red);
+  if constexpr (SAME) {
+    if (alone) return;
+    // the parts are out of this die when the workgroup counts itself in; the last one finds all of them
+    __shared__ int last;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
+    if (tid == 0) {
+      last = __hip_atomic_fetch_add(a.done + blockIdx.x, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
+      if (last) __hip_atomic_store(a.done + blockIdx.x, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
+    }
+    __syncthreads();
+    if (!last) return;
+    static_assert(R == 1, "heads next to each other would be added up one after the other");
+    combine_parts<T, true>(a, h0, n_parts, parts, red);
   }
 }
 
@@ -343,35 +349,37 @@ __global__ __launch_bounds__(256) void window_combine_kernel(WindowAttnArgs a, i
   __shared__ float red[256];
   const int pos = a.pos.position();
   const int parts = ((a.window > 0 ? min(a.window, pos + 1) : pos + 1) + kPartKeys - 1) / kPartKeys;
-  combine_parts<T>(a, blockIdx.x, n_parts, parts, red);
+  combine_parts<T, false>(a, blockIdx.x, n_parts, parts, red);
 }
 
-template <typename T, int R>
-int launch_decode_rows(const WindowAttnArgs& a, hipStream_t st) {
+template <typename T, int R, bool SAME>
+void launch_decode_parts(const WindowAttnArgs& a, int parts, hipStream_t st) {
   const int chunks = (a.heads / a.kv_heads + R - 1) / R;
-  const int parts = window_parts(a.window, a.len_bound);
-  AWQ_REQUIRE(parts >= 1 && parts <= 65535, "too many keys");
   const dim3 g((unsigned)(a.kv_heads * chunks), (unsigned)parts);
   const size_t lds = sizeof(float) * 4 * R * a.vl.row;  // (256 floats at least)
   const int row = std::max(a.kl.row, a.vl.row);
-  if (row == 64) hipLaunchKernelGGL((window_decode_kernel<T, R, 2>), g, dim3(256), lds, st, a, chunks);
-  else if (row == 128) hipLaunchKernelGGL((window_decode_kernel<T, R, 4>), g, dim3(256), lds, st, a, chunks);
-  else hipLaunchKernelGGL((window_decode_kernel<T, R, 8>), g, dim3(256), lds, st, a, chunks);
-  AWQ_HIP_TRY(hipGetLastError());
-  if (parts > 1 && !a.done) {
-    hipLaunchKernelGGL(window_combine_kernel<T>, dim3((unsigned)a.heads), dim3(256), 0, st, a, parts);
-    AWQ_HIP_TRY(hipGetLastError());
-  }
-  return AWQ_OK;
+  if (row == 64) hipLaunchKernelGGL((window_decode_kernel<T, R, 2, SAME>), g, dim3(256), lds, st, a, chunks);
+  else if (row == 128) hipLaunchKernelGGL((window_decode_kernel<T, R, 4, SAME>), g, dim3(256), lds, st, a, chunks);
+  else hipLaunchKernelGGL((window_decode_kernel<T, R, 8, SAME>), g, dim3(256), lds, st, a, chunks);
 }
 
 template <typename T>
 int launch_decode(const WindowAttnArgs& a, hipStream_t st) {
+  const int parts = window_parts(a.window, a.len_bound);
+  AWQ_REQUIRE(parts >= 1 && parts <= 65535, "too many keys");
   const int per = a.heads / a.kv_heads;
-  if (per == 1) return launch_decode_rows<T, 1>(a, st);
-  if (per == 2) return launch_decode_rows<T, 2>(a, st);
-  if (per <= 4) return launch_decode_rows<T, 4>(a, st);
-  return launch_decode_rows<T, 8>(a, st);
+  const bool same = a.done && window_counted_parts(a.heads, a.kv_heads, a.window, a.len_bound);
+  if (same) launch_decode_parts<T, 1, true>(a, parts, st);
+  else if (per == 1) launch_decode_parts<T, 1, false>(a, parts, st);
+  else if (per == 2) launch_decode_parts<T, 2, false>(a, parts, st);
+  else if (per <= 4) launch_decode_parts<T, 4, false>(a, parts, st);
+  else launch_decode_parts<T, 8, false>(a, parts, st);
+  AWQ_HIP_TRY(hipGetLastError());
+  if (parts > 1 && !same) {
+    hipLaunchKernelGGL(window_combine_kernel<T>, dim3((unsigned)a.heads), dim3(256), 0, st, a, parts);
+    AWQ_HIP_TRY(hipGetLastError());
+  }
+  return AWQ_OK;
 }
 
 // Many tokens, bfloat16.  128 queries of one head per workgroup, 32 per wavefront; keys and values of 32 positions at
@@ -597,6 +605,17 @@ int launch_queries(const WindowAttnArgs& a, hipStream_t st) {
 
 // the tiled and the one-token kernel have rows of 64, 128 or 256 elements; longer ones go a query at a time
 int32_t window_row_padded(int32_t dim) { return dim <= 64 ? 64 : dim <= 128 ? 128 : (int32_t)round_up(dim, 256); }
+
+// The last workgroup reads the parts past the caches and, of heads that share a kv head, one head after the other; a second launch costs
+// 2 to 4 us, reads through the caches and has a workgroup per head.  Kugilix of width 1,024, eight layers of attention without window, a
+// token at 20, 300, 1,000, 2,500 and 30,000 positions: 16 heads of 64 125, 150, 176, 228 and 1,151 us against 146, 153, 157, 173 and 506 with
+// the second launch; 8 heads of 128 132, 157, 176 and 223 against 151, 155, 168 and 180; on 4 kv heads 147, 186, 211 and 272 against 168,
+// 177, 184 and 200; on one 239, 361, 463 and 644 against 259, 274, 273 and 283.  So it is for heads with a kv head each and up to 16 parts, where
+// what the first positions gain is as much as what the last ones lose.
+bool window_counted_parts(int32_t heads, int32_t kv_heads, int64_t window, int64_t max_pos) {
+  const int parts = window_parts(window, max_pos);
+  return heads == kv_heads && parts > 1 && parts <= 16;
+}
 
 int64_t window_parts_floats(int32_t heads, int32_t vdim, int64_t window, int64_t max_pos) {
   return (int64_t)heads * window_parts(window, max_pos) * (2 + vdim);

@@ -1,9 +1,12 @@
 """numpy utilities shared by the tests: pointer plumbing, an independent numpy
 version of the seeded generator, reference packing helpers."""
 import ctypes
+import os
+import subprocess
 
 import numpy as np
 
+PKG = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "cuda-kernel-qwen3-8b-awq_amd")
 MASK64 = (1 << 64) - 1
 
 
@@ -166,3 +169,14 @@ def heavy_tailed_inputs(rng, k):
     g = rng.standard_normal(k)
     out["GeLU of N(0,1)"] = np.array([0.5 * v * (1.0 + erf(v * 0.70710678)) for v in g]).astype(np.float16)
     return out
+
+
+def host_program(tmp_path, source):
+    """the numbers that a program linked with the library prints; it sees no device, so only host code runs"""
+    src, exe = tmp_path / "program.cpp", str(tmp_path / "program")
+    src.write_text(source)
+    subprocess.run(["/opt/rocm/bin/hipcc", "-x", "hip", "--offload-host-only", "-std=c++17", "-I" + os.path.join(PKG, "csrc"), str(src),
+                    "-o", exe, "-L" + PKG, "-lawq_infer", "-Wl,-rpath," + PKG], check=True, capture_output=True, text=True, timeout=300)
+    run = subprocess.run([exe], check=True, capture_output=True, text=True, timeout=100,
+                         env=dict(os.environ, HIP_VISIBLE_DEVICES="-1", ROCR_VISIBLE_DEVICES=""))
+    return [int(v) for v in run.stdout.split()]

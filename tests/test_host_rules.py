@@ -1,8 +1,5 @@
-"""What a product refuses before anything is launched (host code: the program below sees no device)."""
-import os
-import subprocess
-
-PKG = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "cuda-kernel-qwen3-8b-awq_amd")
+"""Rules of the launchers that are host code: what a product refuses before anything is launched, and which form a call takes."""
+from helpers import host_program
 
 PROGRAM = r"""
 #include <stdio.h>
@@ -55,15 +52,16 @@ int main() {
 """
 
 
-def test_a_product_does_not_write_what_the_sublayers_end_in_it_reads(awq, lib, tmp_path):
+def test_a_product_does_not_write_what_the_sublayers_end_in_it_reads(lib, tmp_path):
     """every workgroup reads the end's operands: one that starts late would read another's outputs"""
-    src, exe = tmp_path / "args.cpp", str(tmp_path / "args")
-    src.write_text(PROGRAM)
-    subprocess.run(["/opt/rocm/bin/hipcc", "-x", "hip", "--offload-host-only", "-std=c++17", "-I" + os.path.join(PKG, "csrc"), str(src),
-                    "-o", exe, "-L" + PKG, "-lawq_infer", "-Wl,-rpath," + PKG], check=True, capture_output=True, text=True, timeout=300)
-    env = dict(os.environ, HIP_VISIBLE_DEVICES="-1", ROCR_VISIBLE_DEVICES="")
-    run = subprocess.run([exe], capture_output=True, text=True, timeout=100, env=env)
-    assert run.returncode == 0, run.stderr
-    got = [int(v) for v in run.stdout.split()]
     bad_argument, no_device = 1, 3
-    assert got == ([no_device] + 16 * [bad_argument]) * 2
+    assert host_program(tmp_path, PROGRAM) == ([no_device] + 16 * [bad_argument]) * 2
+
+
+def test_parts_of_a_window_that_their_own_launch_adds_up(lib, tmp_path):
+    """few parts of heads with a kv head each; others would be added up one after the other by a single workgroup"""
+    shapes = [(8, 8, 1024, 8192), (8, 8, 0, 1024), (8, 8, 64, 8192), (8, 8, 1025, 8192), (8, 8, 0, 8192), (8, 8, 0, 32768),
+              (8, 4, 1024, 8192), (8, 1, 128, 8192)]
+    calls = "".join('printf("%%d\\n", (int)window_counted_parts(%d, %d, %d, %d));' % s for s in shapes)
+    got = host_program(tmp_path, '#include <stdio.h>\n#include "layers.hpp"\nint main() { %s }' % calls)
+    assert got == [1, 1, 0, 0, 0, 0, 0, 0]
