@@ -769,10 +769,13 @@ int launch_dense_pack(const void* src, bool src_f32, int64_t rows, int64_t cols,
 }
 
 // Up to 2,048 values, where every workgroup's reading of row, weights, taps and state (36 bytes a value) costs as much as the launch:
-// Kugilix, 64 tokens after 100, with it and without: width 1,280 13.5 and 14.6 ms, 1,664 15.6 and 16.1, 2,048 18.4 and 18.5.
+// Kugilix, 64 tokens after 100, with it and without: width 1,280 13.5 and 14.6 ms, 1,664 15.6 and 16.1, 2,048 18.4 and 18.5.  And up to 24
+// groups: a wavefront takes every eighth, each a trip to memory behind the one ahead.  A token of four layers with it
+// and without: 24 groups of 1,536 values 114 and 116 us, 16 of 1,024 98 and 102, 20 of 640 82 and 86; 32 of 2,048 134 and 134, 32 of 1,024
+// 108 and 102, 40 of 640 94 and 86, 256 of 1,024 276 and 102.
 bool dense_norm_fused(const NormConvArgs& n, bool f32) {
   const int64_t part = n.groups > 0 && n.width % n.groups == 0 ? n.width / n.groups : 0;
-  return !f32 && n.M == 1 && n.width <= 2048 && n.groups >= 4 && part % 4 == 0 && part > 0 && part <= 256 && !n.rows && n.ld % kDenseKAlign == 0 &&
+  return !f32 && n.M == 1 && n.width <= 2048 && n.groups >= 4 && n.groups <= 24 && part % 4 == 0 && part > 0 && part <= 256 && !n.rows && n.ld % kDenseKAlign == 0 &&
          (!n.conv || n.taps == kFusedTaps) && (((uintptr_t)n.x | (uintptr_t)n.w1 | (uintptr_t)n.w2 | (uintptr_t)n.conv) & 15) == 0;
 }
 

@@ -65,3 +65,22 @@ def test_parts_of_a_window_that_their_own_launch_adds_up(lib, tmp_path):
     calls = "".join('printf("%%d\\n", (int)window_counted_parts(%d, %d, %d, %d));' % s for s in shapes)
     got = host_program(tmp_path, '#include <stdio.h>\n#include "layers.hpp"\nint main() { %s }' % calls)
     assert got == [1, 1, 0, 0, 0, 0, 0, 0]
+
+
+def test_norms_that_are_part_of_their_product(lib, tmp_path):
+    """a wavefront per group, a few turns at most: each turn waits for memory behind the one ahead"""
+    program = """
+#include <stdio.h>
+#include "layers.hpp"
+int main() {
+  for (int groups : {1, 4, 8, 16, 24, 32, 64, 256, 512}) {
+    NormConvArgs n;
+    n.M = 1;
+    n.width = groups == 24 ? 1536 : groups == 1 ? 256 : 2048 < 256 * groups ? 2048 : 256 * groups;
+    n.groups = groups;
+    n.ld = n.width;
+    printf("%d\\n", (int)dense_norm_fused(n, false));
+  }
+}
+"""
+    assert host_program(tmp_path, program) == [0, 1, 1, 1, 1, 0, 0, 0, 0]
