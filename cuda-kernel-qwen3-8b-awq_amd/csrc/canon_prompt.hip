@@ -642,6 +642,16 @@ bool canon_prompt_supported(int64_t hidden, int64_t inter) {
          awq_group_period(hidden, hidden) == 1 && awq_group_period(inter, hidden) == 1 && awq_group_period(hidden, inter) == 1;
 }
 
+// A layer of a pass of up to 16 positions against the steps it takes the place of.  A step's attention cuts the sequence over workgroups,
+// the pass's gives a workgroup four queries of a head and all their keys.  Us per layer, pass and step: at position 0 63 and 20.8 with
+// inter 4,096, 71 and 26.1 with 12,288, 73 and 32.4 with 16,384; at 1,500 of 12,288 141 and 33.0, at 2,000 170 and 36.6.  12 layers, 3
+// positions from 0, 1,000 and 2,000 on: single 940, 1,098 and 1,319 us, together 857, 1,455 and 2,039; 4: 1,236, 1,449 and 1,735
+// against 850, 1,462 and 2,051; 8 are faster together everywhere (2,000: 2,033 against 3,413).
+int64_t canon_prompt_from(int64_t inter, int64_t pos0) {
+  const float at = (float)pos0, wide = (float)inter;
+  return (int64_t)ceilf((61.0f + 0.001f * wide + 0.0495f * at) / (18.1f + 0.00065f * wide + 0.0052f * at));
+}
+
 int launch_canon_norm(const float* part, int parts, half_t* hidden, const half_t* gamma, float eps, CanonTokens out, int64_t M,
                       hipStream_t st) {
   AWQ_REQUIRE(M >= 1 && M <= kCanonTokens && parts >= 0 && parts <= 4 && (parts == 0 || part), "bad arguments");

@@ -208,10 +208,9 @@ int launch_rope_kv_append_batch(const half_t* qkv, const half_t* cos_t, const ha
                                 half_t* kc, half_t* vc, int n_heads, int64_t max_pos, KvLayout kv, int64_t pos0,
                                 int64_t M, hipStream_t st, half_t* k_parts = nullptr, half_t* v_parts = nullptr,
                                 int parts_pos = 0);
-// Prompt positions together with the arithmetic of the one-token step (canon_prompt.hip), kCanonFrom (two take 1.8 ms one after
-// the other and 2.4 together, three 2.6 and 2.4) to kCanonTokens of them, up to position kCanonPositions.  Tokens in block fixed point, padded to a multiple of 16: the integers in the matrix
+// Prompt positions together with the arithmetic of the one-token step (canon_prompt.hip), canon_prompt_from to kCanonTokens of them, up
+// to position kCanonPositions.  Tokens in block fixed point, padded to a multiple of 16: the integers in the matrix
 // instruction's operand order, and each block's power of two and sum.
-constexpr int64_t kCanonFrom = 3;
 constexpr int64_t kCanonTokens = 128;
 constexpr int64_t kCanonPositions = 2048;  // four queries' scores in LDS
 inline int64_t round16(int64_t v) { return (v + 15) / 16 * 16; }
@@ -232,6 +231,7 @@ enum CanonOut {
   CANON_QKV = 2,    // rotary, q and the caches
 };
 bool canon_prompt_supported(int64_t hidden, int64_t inter);
+int64_t canon_prompt_from(int64_t inter, int64_t pos0);  // fewest positions from pos0 on that are faster together than as single steps
 int canon_prompt_parts(int64_t m, int64_t k);
 int launch_canon_norm(const float* part, int parts, half_t* hidden, const half_t* gamma, float eps, CanonTokens out, int64_t M,
                       hipStream_t st);

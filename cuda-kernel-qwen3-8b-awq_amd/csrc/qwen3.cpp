@@ -1025,7 +1025,7 @@ int enqueue_canon_layers(Qwen3Engine* e, half_t* hidden, int64_t pos0, int64_t M
 
 int64_t Qwen3Engine::exact_pass_tokens(int64_t done, int64_t rest) const {
   const int64_t room = std::min(rest, kCanonPositions - done);
-  if (room < kCanonFrom || !canon_prompt_supported(cfg.hidden, cfg.inter)) return 0;
+  if (!canon_prompt_supported(cfg.hidden, cfg.inter) || room < canon_prompt_from(cfg.inter, done)) return 0;
   const int64_t passes = (room + kCanonTokens - 1) / kCanonTokens;
   return std::min(room, round16((room + passes - 1) / passes));
 }

@@ -84,3 +84,11 @@ int main() {
 }
 """
     assert host_program(tmp_path, program) == [0, 1, 1, 1, 1, 0, 0, 0, 0]
+
+
+def test_prompt_positions_that_go_together(lib, tmp_path):
+    """the deeper in a sequence, the more of them it takes: a step's attention is cut over workgroups, the pass's is not"""
+    calls = "".join('printf("%%d\\n", (int)canon_prompt_from(%d, %d));' % s for s in
+                    [(12288, 0), (12288, 1000), (12288, 2000), (4096, 0), (4096, 1500), (4096, 2000), (16384, 0), (16384, 1500)])
+    got = host_program(tmp_path, '#include <stdio.h>\n#include "common.hpp"\nint main() { %s }' % calls)
+    assert got == [3, 4, 5, 4, 5, 6, 3, 5]
