@@ -99,8 +99,8 @@ struct awq_engine {
   virtual int64_t prompt_pass_tokens(int64_t done, int64_t rest) const = 0;
   virtual int enqueue_prompt_pass(const int32_t* tokens, int64_t pos0, int64_t M) = 0;
   virtual int check_prompt_pass() { return AWQ_OK; }
-  // The same for awq_prefill, whose passes leave the bits of the one-token steps.
-  virtual int64_t exact_pass_tokens(int64_t, int64_t) const { return 0; }
+  // The same for awq_prefill, whose passes leave the bits of the one-token steps: 0 also where there is no memory for the pass.
+  virtual int64_t exact_pass_tokens(int64_t, int64_t) { return 0; }
   virtual int enqueue_exact_pass(const int32_t*, int64_t, int64_t) { return AWQ_ERR_STATE; }
 
   // 32-bit logits of `n` rows of the latest pass (`batched`: a prompt pass, row = token of the pass; otherwise the

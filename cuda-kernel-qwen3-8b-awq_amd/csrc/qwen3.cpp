@@ -199,7 +199,7 @@ struct Qwen3Engine final : awq_engine {
   int64_t prompt_pass_tokens(int64_t done, int64_t rest) const override;
   int enqueue_prompt_pass(const int32_t* tokens, int64_t pos0, int64_t M) override;
   int check_prompt_pass() override;
-  int64_t exact_pass_tokens(int64_t done, int64_t rest) const override;
+  int64_t exact_pass_tokens(int64_t done, int64_t rest) override;
   int enqueue_exact_pass(const int32_t* tokens, int64_t pos0, int64_t M) override;
   int read_rows_logits(bool batched, const int32_t* rows, int32_t n, float* host_dst) override;
   int read_logits_f32(float* host_dst) override;
@@ -977,21 +977,29 @@ int Qwen3Engine::enqueue_prompt_pass(const int32_t* tokens, int64_t pos0, int64_
 }
 
 namespace {
-int alloc_canon_tokens(Qwen3Engine* e, CanonTokens& t, int64_t k) {
-  if (int rc = e->dev_alloc((void**)&t.op, kCanonTokens * k * 2)) return rc;
-  if (int rc = e->dev_alloc((void**)&t.c, kCanonTokens * k / 8)) return rc;
-  return e->dev_alloc((void**)&t.s, kCanonTokens * k / 8);
-}
-
+// One allocation, so that there are all of them or none.
 int ensure_canon_buffers(Qwen3Engine* e) {
   if (e->pc.tokens) return AWQ_OK;
   const int64_t H = e->cfg.hidden, I = e->cfg.inter, parts = std::max(canon_prompt_parts(H, H), canon_prompt_parts(H, I));
-  if (int rc = alloc_canon_tokens(e, e->pc.x, H)) return rc;
-  if (int rc = alloc_canon_tokens(e, e->pc.mid, I)) return rc;
-  if (int rc = e->dev_alloc((void**)&e->pc.hidden, kCanonTokens * H * 2)) return rc;
-  if (int rc = e->dev_alloc((void**)&e->pc.q, kCanonTokens * H * 2)) return rc;
-  if (int rc = e->dev_alloc((void**)&e->pc.part, parts * kCanonTokens * H * 4)) return rc;
-  return e->dev_alloc((void**)&e->pc.tokens, kCanonTokens * 4);
+  const auto tokens = [](int64_t k) { return kCanonTokens * (k * 2 + k / 4); };
+  char* at = nullptr;
+  if (int rc = e->dev_alloc((void**)&at, tokens(H) + tokens(I) + kCanonTokens * (4 * H + parts * H * 4 + 4))) return rc;
+  const auto take = [&](auto** p, int64_t bytes) {
+    *p = reinterpret_cast<std::decay_t<decltype(*p)>>(at);
+    at += bytes;
+  };
+  const auto take_tokens = [&](CanonTokens& t, int64_t k) {
+    take(&t.op, kCanonTokens * k * 2);
+    take(&t.c, kCanonTokens * k / 8);
+    take(&t.s, kCanonTokens * k / 8);
+  };
+  take_tokens(e->pc.x, H);
+  take_tokens(e->pc.mid, I);
+  take(&e->pc.hidden, kCanonTokens * H * 2);
+  take(&e->pc.q, kCanonTokens * H * 2);
+  take(&e->pc.part, parts * kCanonTokens * H * 4);
+  take(&e->pc.tokens, kCanonTokens * 4);
+  return AWQ_OK;
 }
 
 int canon_product(Qwen3Engine* e, const DevLinear& t, const CanonTokens& x, int64_t M, int out, const CanonTokens& y = {},
@@ -1023,16 +1031,19 @@ int enqueue_canon_layers(Qwen3Engine* e, half_t* hidden, int64_t pos0, int64_t M
 }
 }  // namespace
 
-int64_t Qwen3Engine::exact_pass_tokens(int64_t done, int64_t rest) const {
+int64_t Qwen3Engine::exact_pass_tokens(int64_t done, int64_t rest) {
   const int64_t room = std::min(rest, kCanonPositions - done);
   if (!canon_prompt_supported(cfg.hidden, cfg.inter) || room < canon_prompt_from(cfg.inter, done)) return 0;
+  if (ensure_canon_buffers(this)) {  // no memory for the pass: single steps need none
+    (void)hipGetLastError();
+    return 0;
+  }
   const int64_t passes = (room + kCanonTokens - 1) / kCanonTokens;
   return std::min(room, round16((room + passes - 1) / passes));
 }
 
 int Qwen3Engine::enqueue_exact_pass(const int32_t* tokens, int64_t pos0, int64_t M) {
   Qwen3Engine* e = this;
-  if (int rc = ensure_canon_buffers(e)) return rc;
   const int64_t H = e->cfg.hidden;
   AWQ_HIP_TRY(hipMemcpyAsync(e->pc.tokens, tokens, (size_t)M * 4, hipMemcpyHostToDevice, e->stream));
   if (int rc = launch_embed_batch(e->embed.packed, e->embed.scale, e->embed.zp, H, e->cfg.vocab, e->pc.tokens, M, e->pc.hidden, e->stream))

@@ -5,11 +5,13 @@ The two prompt loops sum the products in different orders, so their states agree
 rounding noise (tolerance below), not bit for bit; greedy tokens must be identical except where the
 oracle's own top-1/top-2 logit margin is within that noise."""
 import ctypes
+import os
+import subprocess
 
 import numpy as np
 import pytest
 
-from helpers import fill_pair, make_oracle_model, ptr
+from helpers import PKG, fill_pair, make_oracle_model, ptr
 
 pytestmark = pytest.mark.gpu
 
@@ -376,3 +378,61 @@ def test_prompt_positions_together_have_the_bits_of_single_steps(awq, oracle, to
         assert np.array_equal(got[0], one[0]), cuts
         assert got[1] == one[1] and np.array_equal(got[2], one[2]), cuts
     eng.close()
+
+
+# A program whose own hipMalloc stands before the runtime's and can refuse: a prompt of 20 tokens when there is memory for the
+# pass's buffers, when there is none, and when there is some again.  It prints what each call returned and whether the state
+# after it is that of the first.
+NO_MEMORY = r"""
+#define _GNU_SOURCE
+#include <dlfcn.h>
+#include <stdint.h>
+#include <stdio.h>
+#include <stdlib.h>
+#include <string.h>
+
+#include "awq_infer.h"
+
+static int refuse;
+int hipMalloc(void** p, size_t n) {
+  static int (*real)(void**, size_t);
+  if (!real) real = (int (*)(void**, size_t))dlsym(RTLD_NEXT, "hipMalloc");
+  return refuse ? 2 : real(p, n);
+}
+
+int main(int argc, char** argv) {
+  awq_config c = {2, 4096, 4096, 1024, 64, 1, 1e-6f};
+  awq_engine* e = 0;
+  int32_t ids[20];
+  static uint16_t first[4096], hidden[4096];
+  if (awq_create(argv[1], &c, &e)) return puts(awq_last_error()), 1;
+  awq_synth_tokens(3, 5, ids, 20, 1024);
+  for (int i = 0; i < 20; ++i)
+    if (awq_prefill(e, ids + i, 1)) return puts(awq_last_error()), 1;
+  if (awq_read_hidden(e, first)) return 1;
+  for (int turn = 0; turn < 3; ++turn) {
+    refuse = turn == 0;
+    if (awq_reset(e)) return 1;
+    int rc = awq_prefill(e, ids, 20);
+    refuse = 0;
+    if (awq_read_hidden(e, hidden)) return 1;
+    printf("%d %d\n", rc, memcmp(first, hidden, sizeof first) == 0);
+  }
+  return awq_destroy(e), 0;
+}
+"""
+
+
+def test_a_prompt_for_whose_pass_there_is_no_memory(awq, lib, torch_gpu, tmp_path):
+    """single steps need no buffers of their own: they are taken instead, as before positions went together"""
+    cfg = awq.make_config(n_layers=2, hidden=4096, inter=4096, vocab=1024, max_pos=64, split_idx=1)
+    weights = str(tmp_path / "weights")
+    os.mkdir(weights)
+    awq.check(lib.awq_write_weight_dir_profile(weights.encode(), ctypes.byref(cfg), 9, awq.SYNTH_BALANCED))
+    src, exe = tmp_path / "no_memory.c", str(tmp_path / "no_memory")
+    src.write_text(NO_MEMORY)
+    subprocess.run(["gcc", "-O1", "-I" + os.path.join(os.path.dirname(PKG), "include"), str(src), "-o", exe, "-L" + PKG, "-lawq_infer",
+                    "-ldl", "-Wl,--export-dynamic,-rpath," + PKG], check=True, capture_output=True, text=True, timeout=60)
+    run = subprocess.run([exe, weights], capture_output=True, text=True, timeout=100)
+    assert run.returncode == 0, run.stdout + run.stderr
+    assert run.stdout.split() == ["0", "1"] * 3
