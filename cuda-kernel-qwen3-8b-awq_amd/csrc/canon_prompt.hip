@@ -389,8 +389,7 @@ __global__ __launch_bounds__(256) void canon_norm_kernel(const float* __restrict
 #pragma unroll
       for (int j = 0; j < E; ++j) {
         float t;
-        if constexpr (P == 1) t = v[0][j];
-        else if constexpr (P == 2) t = v[0][j] + v[1][j];
+        if constexpr (P == 2) t = v[0][j] + v[1][j];
         else if constexpr (P == 3) t = (v[0][j] + v[1][j]) + v[2][j];
         else t = (v[0][j] + v[1][j]) + (v[2][j] + v[3][j]);
         x[j] = x[j] + (half_t)t;
@@ -654,10 +653,9 @@ int64_t canon_prompt_from(int64_t inter, int64_t pos0) {
 
 int launch_canon_norm(const float* part, int parts, half_t* hidden, const half_t* gamma, float eps, CanonTokens out, int64_t M,
                       hipStream_t st) {
-  AWQ_REQUIRE(M >= 1 && M <= kCanonTokens && parts >= 0 && parts <= 4 && (parts == 0 || part), "bad arguments");
+  AWQ_REQUIRE(M >= 1 && M <= kCanonTokens && (parts == 0 || (parts >= 2 && parts <= 4 && part)), "bad arguments");
   const dim3 grid((unsigned)(gamma ? round16(M) : M)), block(256);
   if (parts == 0) hipLaunchKernelGGL((canon_norm_kernel<0>), grid, block, 0, st, part, hidden, gamma, eps, out, (int)M);
-  else if (parts == 1) hipLaunchKernelGGL((canon_norm_kernel<1>), grid, block, 0, st, part, hidden, gamma, eps, out, (int)M);
   else if (parts == 2) hipLaunchKernelGGL((canon_norm_kernel<2>), grid, block, 0, st, part, hidden, gamma, eps, out, (int)M);
   else if (parts == 3) hipLaunchKernelGGL((canon_norm_kernel<3>), grid, block, 0, st, part, hidden, gamma, eps, out, (int)M);
   else hipLaunchKernelGGL((canon_norm_kernel<4>), grid, block, 0, st, part, hidden, gamma, eps, out, (int)M);

@@ -1490,7 +1490,7 @@ static WidePlan plan_wide(int64_t m, int64_t k, int64_t M, bool has_workspace) {
 // workgroups up to 512 tokens and the work cut evenly above: 384 tokens 54 us (61), 512 61 (66), 640 73 (103), 768 91 (106), 1,000
 // 104 (119), 1,152 126 (150), 1,280 132 (160); from 1,281 on (176 tiles) a tile per workgroup is faster (1,536: 166 against 152).  At
 // k = 4,096 the sums' way through memory costs more than the tiles gain (1,000 tokens 48 us with two shares, 39 without).
-static int norm_shares(int64_t m, int64_t k, int64_t M) {
+int gemm_norm_shares(int64_t m, int64_t k, int64_t M) {
   const int64_t tiles = (m + 255) / 256 * ((M + kWideTokens - 1) / kWideTokens);
   if (k < 8192 || m > kNormRow || tiles < 48) return 0;
   for (int kz : {4, 3, 2})
@@ -1633,7 +1633,7 @@ int launch_gemm(const void* wq, const half_t* scale, const half_t* zp, int64_t m
     const int64_t part_bytes = workspace_bytes - kSkHeaderBytes;
     const bool room = workspace && kSkWgs * (int64_t)kSkTileFloats * 4 <= part_bytes;
     const WidePlan plan = plan_wide(m, k, M, room);
-    if (const int shares = norm_shares(m, k, M); norm && shares && epilogue == EPI_RESIDUAL && workspace && (int64_t)shares * M * m * 4 <= part_bytes) {
+    if (const int shares = gemm_norm_shares(m, k, M); norm && shares && epilogue == EPI_RESIDUAL && workspace && (int64_t)shares * M * m * 4 <= part_bytes) {
       p.nr = (int32_t)nr;
       p.n_tiles = (int32_t)tiles;
       p.kz = shares;

@@ -12,6 +12,7 @@ import numpy as np
 import pytest
 
 from helpers import PKG, fill_pair, make_oracle_model, ptr
+from test_host_rules import SHARES
 
 pytestmark = pytest.mark.gpu
 
@@ -339,15 +340,10 @@ def test_handed_over_sums_give_up_path(awq, lib, oracle, torch_gpu):
     eng.close()
 
 
-# Widths at which awq_prefill takes several positions together with the one-token steps' arithmetic.  k of the second
-# MLP matrix: one and three runs of 128 blocks.  Zero-points: integers within 16 (products of q - z), beyond, and not
-# integers (the general block value).
-@pytest.mark.parametrize("inter,zero,fused", [(4096, None, True), (12288, None, True), (12288, 17.0, True), (4096, 6.5, False)])
-def test_prompt_positions_together_have_the_bits_of_single_steps(awq, oracle, torch_gpu, inter, zero, fused):
-    """Portions of every count of token tiles with full and ragged last tiles, against one token a call (a single
-    position is always a step of its own): the state after the portion and what is generated from its cache rows."""
-    cfg = awq.make_config(n_layers=2, hidden=4096, inter=inter, vocab=1024, max_pos=512)
-    model = make_oracle_model(oracle, cfg)
+def engine_with_zero_points(awq, oracle, inter, max_pos, zero):
+    """two layers of width 4,096, every third zero-point of every matrix replaced unless `zero` is None"""
+    cfg = awq.make_config(n_layers=2, hidden=4096, inter=inter, vocab=1024, max_pos=max_pos)
+    model = make_oracle_model(oracle, cfg)   # only as the host buffer of the weights here
 
     def mutate(layer, kind, part, p, count):
         if zero is not None and part == awq.P_ZP and kind != awq.T_GAMMA:
@@ -357,6 +353,18 @@ def test_prompt_positions_together_have_the_bits_of_single_steps(awq, oracle, to
     eng = awq.QWen3AWQInfer.empty(cfg)
     fill_pair(awq, oracle, cfg, 31, engine=eng, model=model, profile=awq.SYNTH_BALANCED, mutate=mutate)
     oracle.awqo_model_destroy(model)
+    return eng, cfg
+
+
+# Widths at which awq_prefill takes several positions together with the one-token steps' arithmetic.  k of the second
+# MLP matrix: one to four runs of 128 blocks.  Zero-points: integers within 16 (products of q - z), beyond, and not
+# integers (the general block value).
+@pytest.mark.parametrize("inter,zero,fused", [(4096, None, True), (8192, None, True), (12288, None, True), (12288, 17.0, True),
+                                              (4096, 6.5, False), (16384, 6.5, True)])
+def test_prompt_positions_together_have_the_bits_of_single_steps(awq, oracle, torch_gpu, inter, zero, fused):
+    """Portions of every count of token tiles with full and ragged last tiles, against one token a call (a single
+    position is always a step of its own): the state after the portion and what is generated from its cache rows."""
+    eng, cfg = engine_with_zero_points(awq, oracle, inter, 512, zero)
     if not fused:
         eng.set_fused_mode(0)
     rng = np.random.default_rng(inter)
@@ -378,6 +386,59 @@ def test_prompt_positions_together_have_the_bits_of_single_steps(awq, oracle, to
         assert np.array_equal(got[0], one[0]), cuts
         assert got[1] == one[1] and np.array_equal(got[2], one[2]), cuts
     eng.close()
+
+
+@pytest.mark.parametrize("fused", [True, False])
+def test_positions_together_deep_in_a_sequence(awq, oracle, torch_gpu, fused):
+    """As above behind a prefix: where a step's attention changes its form (about 704 positions), at many chunks of 64 positions,
+    portions that end at position 2,048, pass it and start there, where positions stop going together."""
+    eng, cfg = engine_with_zero_points(awq, oracle, 12288, 2176, None)
+    if not fused:
+        eng.set_fused_mode(0)
+    rng = np.random.default_rng(3)
+    tokens = rng.integers(0, cfg.vocab, 2100).tolist()
+
+    def after(pos0, n, together):
+        eng.reset()
+        eng.prefill(tokens[:pos0], batched=True)
+        for portion in [tokens[pos0:pos0 + n]] if together else [[t] for t in tokens[pos0:pos0 + n]]:
+            eng.prefill(portion)
+        hidden = np.ctypeslib.as_array(eng.read_hidden()).copy()
+        return hidden, eng.decode(2), np.ctypeslib.as_array(eng.read_logits()).copy()
+
+    for pos0, n in ((690, 30), (1010, 48), (1500, 128), (1960, 100), (2031, 17), (2040, 20), (2048, 9)):
+        print("portion of", n, "from", pos0, flush=True)
+        one, got = after(pos0, n, False), after(pos0, n, True)
+        assert np.isfinite(one[0].view(np.float16)).all() and one[0].any()
+        assert np.array_equal(got[0], one[0]), (pos0, n)
+        assert got[1] == one[1] and np.array_equal(got[2], one[2]), (pos0, n)
+    eng.close()
+
+
+@pytest.mark.parametrize("zero", [None, 6.5])
+def test_second_matrix_in_shares_that_the_norm_adds(awq, oracle, torch_gpu, zero):
+    """Passes whose second MLP product goes in four, three and two shares of k to tiles of 128 tokens, with ragged last tiles, the
+    shares added by the launch that norms the rows for the layer behind (SHARES in test_host_rules.py): logits at places of every
+    tile against the prompt's bits of single steps."""
+    eng, cfg = engine_with_zero_points(awq, oracle, 12288, 1280, zero)
+    tokens = np.random.default_rng(12).integers(0, cfg.vocab, 1153).tolist()
+    want, last = {}, -1
+    eng.reset()
+    for p in sorted({p for n in SHARES for p in places(n)}):
+        eng.prefill(tokens[last + 1:p])
+        want[p] = eng.forward([tokens[p]], [0])[0]
+        last = p
+    for n in SHARES:
+        print("shares,", n, "tokens", flush=True)
+        eng.reset()
+        got = eng.forward(tokens[:n], places(n))
+        for p, z in zip(places(n), got):
+            assert np.isfinite(z).all() and close(want[p], z), (n, p)
+    eng.close()
+
+
+def places(n):
+    return sorted({0, 127, 128, n // 2, n // 128 * 128 - 1, n // 128 * 128, n - 1} & set(range(n)))
 
 
 # A program whose own hipMalloc stands before the runtime's and can refuse: a prompt of 20 tokens when there is memory for the

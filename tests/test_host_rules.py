@@ -1,6 +1,9 @@
 """Rules of the launchers that are host code: what a product refuses before anything is launched, and which form a call takes."""
 from helpers import host_program
 
+# tokens of a pass -> shares of k of a 4,096 x 12,288 product whose rows a norm follows
+SHARES = {385: 4, 600: 3, 1000: 2, 1153: 3}
+
 PROGRAM = r"""
 #include <stdio.h>
 
@@ -92,3 +95,10 @@ def test_prompt_positions_that_go_together(lib, tmp_path):
                     [(12288, 0), (12288, 1000), (12288, 2000), (4096, 0), (4096, 1500), (4096, 2000), (16384, 0), (16384, 1500)])
     got = host_program(tmp_path, '#include <stdio.h>\n#include "common.hpp"\nint main() { %s }' % calls)
     assert got == [3, 4, 5, 4, 5, 6, 3, 5]
+
+
+def test_shares_of_the_second_matrix(lib, tmp_path):
+    calls = [(4096, 12288, m) for m in list(SHARES) + [256, 1408]] + [(4096, 4096, 1000), (8320, 8192, 385)]
+    lines = "".join('printf("%%d\\n", gemm_norm_shares(%d, %d, %d));' % c for c in calls)
+    got = host_program(tmp_path, '#include <stdio.h>\n#include "common.hpp"\nint main() { %s }' % lines)
+    assert got == list(SHARES.values()) + [0] * 4
