@@ -660,20 +660,22 @@ struct ManyForm {
   float step;         // a step of one of several workgroups
   float end;          // the end of a tile
 };
-constexpr ManyForm kManyForms[4] = {{2, 2, 512, 0.388f, 0.0136f, 0.450f, 0.766f},
-                                    {2, 1, 1024, 0.219f, 0.0205f, 0.292f, 0.0f},
-                                    {4, 2, 512, 0.316f, 0.0432f, 0.596f, 2.715f},
-                                    {4, 1, 768, 0.396f, 0.0074f, 0.393f, 0.763f}};
+constexpr ManyForm kManyForms[4] = {{2, 2, 512, 0.4619f, 0.0118f, 0.5130f, 0.1225f},
+                                    {2, 1, 1024, 0.3175f, 0.0115f, 0.3461f, 0.001f},
+                                    {4, 2, 512, 0.6420f, 0.0f, 0.5867f, 2.6015f},
+                                    {4, 1, 768, 0.4699f, 0.0033f, 0.3965f, 1.022f}};
 
-// The time of a product in us, but for what all forms of it share: what the choice of a form and of a number of shares of k needs.
-// Weights out of memory; what workgroups take in; the shares' sums, written, read and added one after the other.  The numbers are
-// fitted for the choice, not for the time, to 18,400 timings (31 shapes from 256 x 64 to 32,768 x 1,024 and 28,672 x 4,096, 33 to
-// 2,048 tokens, all forms, 1 to 16 shares, weights from memory).  The form it picks takes 0.7 % longer on average than the fastest
-// timed, 10 % at the 99th of 100 and 18 % at most; the fastest with 256 rows 16 % on average.
-float weights_time(const DenseArgs& a, int64_t rows) { return (float)rows * (float)a.k * (float)a.batch * 2.0f / 6.63e6f; }
+float weights_time(const DenseArgs& a, int64_t rows) { return (float)rows * (float)a.k * (float)a.batch * 2.0f / 7.0415e6f; }
+// the shares' sums, written, read and added one after the other
 float shares_time(const DenseArgs& a, int64_t rows, int64_t cuts) {
-  return 1.65f + (float)cuts * (0.244f + (float)a.M * (float)rows * 8.0f / 3.33e6f);
+  return 3.4666f + (float)cuts * (0.3631f + (float)a.M * (float)rows * 8.0f / 3.9616e6f);
 }
+// The time of a product in us, but for what all forms of it share: what the choice of a form and of a number of shares of k needs.
+// The numbers are fitted for the choice, not for the time, to 32,100 timings (52 shapes from 256 x 64 to 32,768 x 1,024, 28,672 x 8,192 and
+// 4,096 x 16,384, 33 to 2,048 tokens, all forms, 1 to 16 shares, weights from memory).  The form it picks takes 0.9 % longer on
+// average than the fastest timed, 11 % at the 99th of 100; against tiles of 256 rows alone, by an estimate of their own, it is 13 %
+// faster on average (6 % beyond 4,096 inputs) and for one product in 200 slower by 5 % or more, 10 % at most.  Fitted to shapes of up to 4,096
+// inputs, most of them, it was for one in ten of the longer ones: 10,752 x 15,232 at 98 tokens 77 -> 89 us, now 75.
 float many_time(const DenseArgs& a, int64_t rows, const ManyForm& f, int64_t cuts) {
   const int64_t row_tiles = rows / (128 * f.rb), tok_tiles = (a.M + 32 * f.tt - 1) / (32 * f.tt);
   const float groups = (float)(row_tiles * tok_tiles * cuts * a.batch), steps = (float)(((a.k >> 6) + cuts - 1) / cuts);
@@ -681,8 +683,7 @@ float many_time(const DenseArgs& a, int64_t rows, const ManyForm& f, int64_t cut
   const float per_unit = ceilf(groups / 256.0f);
   float t = steps * wait * ceilf(groups / (float)f.resident);
   if (per_unit > 1.0f) t = std::max(t, steps * per_unit * f.step);
-  t = std::max(t, weights_time(a, rows));
-  t = std::max(t, groups * steps * (float)(16384 * f.rb + f.tt * 4096) / 108.6e6f) + per_unit * f.end;
+  t = std::max(t, weights_time(a, rows)) + per_unit * f.end;
   return cuts > 1 ? t + shares_time(a, rows, cuts) : t;
 }
 
@@ -698,33 +699,16 @@ void launch_form(const DenseArgs& a, const ManyForm& f, int64_t rows, int64_t to
 
 template <int OUT>
 int launch_many(const DenseArgs& a, int64_t rows, hipStream_t st) {
-  // A product of few tokens goes the way whose time is estimated to be the shorter; what the other way's estimate leaves out is 6.5 us
-  // more.  Workgroups that leave compute units idle and long rows, which read the tokens more than the weights, are against
-  // the few-token kernel: 6,144 x 12,288 at 20 tokens 54 us, below 36.  Of 310 products (31 shapes from 256 x 64 to 28,672 x 4,096, 2
-  // to 32 tokens, both ways timed) the choice is 0.2 % off on average and 13 % at most.
-  constexpr float kManyMore = 6.5f;
-  const float few = a.M <= kFewTokens ? few_time(a, rows) : HUGE_VALF;
-  // (the other way takes at least the weights' time: mostly known without an estimate of its forms)
-  if (few < weights_time(a, rows) + kManyMore) return launch_few<OUT, false>(a, rows, (int)a.M, a.batch, st);
-  int64_t most = 1;  // shares of k: at least four steps each
-  if (a.workspace && a.batch == 1 && a.M <= 65535)
-    most = std::max<int64_t>(1, std::min(std::min<int64_t>(16, a.k >> 8), a.workspace_floats / (a.M * rows)));
-  const ManyForm* form = nullptr;
-  int64_t cuts = 1;
-  float best = HUGE_VALF;
-  for (const ManyForm& f : kManyForms)
-    for (int64_t c = 1; c <= most && (c == 1 || shares_time(a, rows, c) < best); ++c) {
-      const float t = many_time(a, rows, f, c);
-      if (t < best) best = t, form = &f, cuts = c;
-    }
-  if (!form) form = &kManyForms[2];  // (a product too long for the estimate)
-  if (few < best + kManyMore) return launch_few<OUT, false>(a, rows, (int)a.M, a.batch, st);
+  const DenseForm c = dense_form(a, rows);
+  if (c.tt == 0) return launch_few<OUT, false>(a, rows, (int)a.M, a.batch, st);
+  const ManyForm* form = kManyForms;
+  while (form->tt != c.tt || form->rb != c.rb) ++form;
   const int64_t tok_tiles = (a.M + 32 * form->tt - 1) / (32 * form->tt);
-  if (cuts > 1) {
-    launch_form<DENSE_PART, false>(a, *form, rows, tok_tiles, cuts, st);
+  if (c.cuts > 1) {
+    launch_form<DENSE_PART, false>(a, *form, rows, tok_tiles, c.cuts, st);
     AWQ_HIP_TRY(hipGetLastError());
     hipLaunchKernelGGL((dense_parts_kernel<bf16_t, OUT>), dim3((unsigned)((rows / 4 + 255) / 256), (unsigned)a.M), dim3(256), 0, st, a,
-                       (int)rows, (int)cuts);
+                       (int)rows, (int)c.cuts);
   } else {
     launch_form<OUT, false>(a, *form, rows, tok_tiles, 1, st);
   }
@@ -745,6 +729,29 @@ int launch_listed(const DenseArgs& a, int64_t rows, hipStream_t st) {
 }
 
 }  // namespace
+
+// A product of few tokens goes the way whose time is estimated to be the shorter; what the other way's estimate leaves out is 5.5 us
+// more.  Workgroups that leave compute units idle and long rows, which read the tokens more than the weights, are against
+// the few-token kernel: 6,144 x 12,288 at 20 tokens 54 us, below 36.  Of 520 products (52 shapes from 256 x 64 to 28,672 x 8,192, 2
+// to 32 tokens, both ways timed) the choice is 0.5 % off on average and 16 % at most.
+DenseForm dense_form(const DenseArgs& a, int64_t rows) {
+  constexpr float kManyMore = 5.5f;
+  const float few = a.M <= kFewTokens ? few_time(a, rows) : HUGE_VALF;
+  DenseForm form;
+  // (the other way takes at least the weights' time: mostly known without an estimate of its forms)
+  if (few < weights_time(a, rows) + kManyMore) return form;
+  int64_t most = 1;  // shares of k: at least four steps each
+  if (a.workspace && a.batch == 1 && a.M <= 65535)
+    most = std::max<int64_t>(1, std::min(std::min<int64_t>(16, a.k >> 8), a.workspace_floats / (a.M * rows)));
+  float best = HUGE_VALF;
+  for (const ManyForm& f : kManyForms)
+    for (int64_t c = 1; c <= most && (c == 1 || shares_time(a, rows, c) < best); ++c) {
+      const float t = many_time(a, rows, f, c);
+      if (t < best) best = t, form = DenseForm{f.tt, f.rb, (int32_t)c};
+    }
+  if (few < best + kManyMore) return DenseForm();
+  return form.tt ? form : DenseForm{4, 2, 1};  // (a product too long for the estimate)
+}
 
 bool dense_gate_fused(int64_t n, int64_t k_padded, int64_t M, bool f32) {
   return !f32 && M == 1 && n % 4 == 0 && n > 0 && n <= k_padded && k_padded % kDenseKAlign == 0 && k_padded <= 16384;

@@ -131,6 +131,12 @@ struct JoinArgs;
 // product, its result the segments' input; x_out and out are written, x stays, and no segment's y is an operand of it
 int launch_dense(const DenseArgs& a, bool f32, hipStream_t st, const NormConvArgs* norm = nullptr, const JoinArgs* join = nullptr);
 bool dense_join_fused(const JoinArgs& j, int64_t rows, bool f32);
+// How a bfloat16 product of several tokens and `rows` padded rows goes: tiles of 32 tt tokens and 128 rb rows, k in `cuts` shares; tt 0: by
+// the kernel for few tokens
+struct DenseForm {
+  int32_t tt = 0, rb = 0, cuts = 1;
+};
+DenseForm dense_form(const DenseArgs& a, int64_t rows);
 bool dense_norm_fused(const NormConvArgs& n, bool f32);
 bool dense_gate_fused(int64_t n, int64_t k_padded, int64_t M, bool f32);
 

@@ -8,6 +8,7 @@ import pytest
 
 import kugilix_model as km
 import kugilix_plain as plain
+from test_host_rules import FORMS
 
 pytestmark = pytest.mark.gpu
 
@@ -243,10 +244,9 @@ def test_products_of_every_number_of_steps(awq, lib, dev, tokens, steps):
         assert np.abs(got[:tokens] - xv @ wv.T).max() < 8 * k ** 0.5 * 2.0 ** -24
 
 
-# tiles of 128 and 256 rows and of 64 and 128 tokens, each alone and with its k in shares (as the estimate picks them with a workspace
-# of 2^22 floats), rows and tokens that end inside a tile
-@pytest.mark.parametrize("rows,k,tokens", [(100, 64, 33), (100, 1088, 33), (12300, 512, 257), (4200, 4160, 129), (2100, 320, 1000),
-                                           (8200, 2112, 65), (4200, 320, 1500), (1000, 1088, 200), (130, 2112, 700)])
+# tiles of 128 and 256 rows and of 64 and 128 tokens, each alone and with its k in shares (test_host_rules.py has which is which), rows
+# and tokens that end inside a tile
+@pytest.mark.parametrize("rows,k,tokens", sorted(FORMS))
 def test_products_of_many_tokens_in_every_form(awq, lib, dev, rows, k, tokens):
     """all three outputs; the operands are exact: a sum of k products in binary32 is off by about sqrt(k) roundings of 2^-24 of its size"""
     print("forms", rows, k, tokens, flush=True)
@@ -256,7 +256,7 @@ def test_products_of_many_tokens_in_every_form(awq, lib, dev, rows, k, tokens):
     awq.check(lib.awq_dense_pack(w.data_ptr(), 0, rows, k, block.data_ptr(), k, 0, 0, 0, dev.stream))
     x, xv = dev.act(rng.standard_normal((tokens, k)), False)
     want = xv @ wv.T
-    ws = dev.empty((1 << 22,), True)
+    ws = dev.empty((1 << 25,), True)
     exact = 8 * k ** 0.5 * 2.0 ** -24
     for out in (awq.DENSE_F32, awq.DENSE_RESIDUAL, awq.DENSE_STORE):
         y = dev.empty((tokens + 1, rows), out != awq.DENSE_STORE, fill=0.5)
@@ -276,7 +276,7 @@ def test_products_of_many_tokens_in_every_form(awq, lib, dev, rows, k, tokens):
 @pytest.mark.parametrize("k", [64, 320, 512, 576])
 @pytest.mark.parametrize("rows,tokens", [(2000, 2001), (8200, 1030)])
 def test_products_of_few_inputs_and_many_tokens(awq, lib, dev, rows, tokens, k):
-    """either side of the rule by which few inputs go in small tiles: inputs up to 512, tiles on the device at once or not"""
+    """products whose steps are few, tiles on the device at once or not, without a workspace"""
     print("few inputs", rows, tokens, k, flush=True)
     rng = np.random.default_rng(k + rows)
     block = dev.torch.zeros((rows + 255) // 256 * 256 * k, dtype=dev.torch.bfloat16, device="cuda")

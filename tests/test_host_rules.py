@@ -3,6 +3,10 @@ from helpers import host_program
 
 # tokens of a pass -> shares of k of a 4,096 x 12,288 product whose rows a norm follows
 SHARES = {385: 4, 600: 3, 1000: 2, 1153: 3}
+# (rows, inputs, tokens) of a bfloat16 product -> 32 and 128 in a tile's tokens and rows, whether k goes in shares: every form there is
+FORMS = {(100, 64, 33): (2, 1, False), (1000, 1088, 200): (2, 1, False), (130, 2112, 700): (2, 1, True), (12300, 512, 257): (2, 2, False),
+         (4200, 4160, 129): (2, 2, True), (12300, 2112, 129): (4, 1, False), (8200, 3136, 65): (4, 1, True), (4200, 576, 1000): (4, 2, False),
+         (4200, 6208, 341): (4, 2, True)}
 
 PROGRAM = r"""
 #include <stdio.h>
@@ -102,3 +106,37 @@ def test_shares_of_the_second_matrix(lib, tmp_path):
     lines = "".join('printf("%%d\\n", gemm_norm_shares(%d, %d, %d));' % c for c in calls)
     got = host_program(tmp_path, '#include <stdio.h>\n#include "common.hpp"\nint main() { %s }' % lines)
     assert got == list(SHARES.values()) + [0] * 4
+
+
+def forms_of(tmp_path, shapes):
+    program = """
+#include <stdio.h>
+#include "layers.hpp"
+int main() {
+  const int shapes[][3] = {%s};
+  for (const auto& s : shapes) {
+    DenseArgs a;
+    a.k = s[1];
+    a.M = s[2];
+    a.workspace = (float*)16;
+    a.workspace_floats = 1 << 25;
+    const DenseForm f = dense_form(a, round_up(s[0], kDenseRowAlign));
+    printf("%%d %%d %%d\\n", f.tt, f.rb, f.cuts > 1);
+  }
+}
+""" % ", ".join("{%d, %d, %d}" % s for s in shapes)
+    got = host_program(tmp_path, program)
+    return [tuple(got[i:i + 3]) for i in range(0, len(got), 3)]
+
+
+def test_forms_of_products_of_many_tokens(lib, tmp_path):
+    assert forms_of(tmp_path, FORMS) == list(FORMS.values())
+    assert len(set(FORMS.values())) == 8
+
+
+def test_long_rows_go_in_a_form_that_is_near_the_fastest(lib, tmp_path):
+    """forms that were timed within 6 % of the fastest of all (the others took 13 to 26 % longer)"""
+    near = {(512, 12288, 2048): [(2, 2), (4, 2)], (10752, 15232, 98): [(4, 1), (4, 2)], (3584, 7168, 512): [(4, 2)], (6144, 12288, 98): [(4, 1)],
+            (2304, 14720, 512): [(4, 2)], (4096, 16384, 278): [(4, 2)], (2304, 14720, 2048): [(4, 2)], (10240, 8320, 160): [(4, 2)]}
+    for shape, form in zip(near, forms_of(tmp_path, near)):
+        assert form[:2] in near[shape] and form[2], shape
