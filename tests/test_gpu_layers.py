@@ -129,7 +129,7 @@ def test_binary32_products_at_the_edges_of_tiles(awq, lib, dev, tokens, rows, k)
             assert np.abs(got - want).max() < 8 * k ** 0.5 * 2.0 ** -24
 
 
-@pytest.mark.parametrize("k", [64, 192, 1024, 1088, 1152, 2048, 2112, 4160, 8192, 8256, 12352])
+@pytest.mark.parametrize("k", [64, 192, 320, 448, 1024, 1088, 1152, 1536, 1792, 2048, 2112, 2560, 3072, 3584, 4160, 8192, 8256, 12352])
 @pytest.mark.parametrize("rows", [1, 9, 1000, 2048, 2049])
 def test_products_of_one_token(awq, lib, dev, rows, k):
     """8 and 16 rows per workgroup, 4, 8 and 16 wavefronts, runs of whole turns and every kind of rest, wavefronts without a
