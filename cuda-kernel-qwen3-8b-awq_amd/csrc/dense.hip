@@ -674,24 +674,25 @@ struct ManyForm {
   int resident;       // workgroups that the device holds
   float wait, root;   // a step of a workgroup that has its unit to itself waits for memory, the longer the more weights are on their way
   float step;         // a step of one of several workgroups
-  float end;          // the end of a tile
+  float end;          // the end of a tile, of binary32 outputs that are not added to others
 };
-constexpr ManyForm kManyForms[4] = {{2, 2, 512, 0.4619f, 0.0118f, 0.5130f, 0.1225f},
-                                    {2, 1, 1024, 0.3175f, 0.0115f, 0.3461f, 0.001f},
-                                    {4, 2, 512, 0.6420f, 0.0f, 0.5867f, 2.6015f},
-                                    {4, 1, 768, 0.4699f, 0.0033f, 0.3965f, 1.022f}};
+constexpr ManyForm kManyForms[4] = {{2, 2, 512, 0.5296f, 0.0068f, 0.4825f, 2.9902f},
+                                    {2, 1, 1024, 0.4289f, 0.0f, 0.3366f, 0.0f},
+                                    {4, 2, 512, 0.7263f, 0.0f, 0.6619f, 4.8844f},
+                                    {4, 1, 768, 0.5590f, 0.0f, 0.4261f, 1.6886f}};
 
-float weights_time(const DenseArgs& a, int64_t rows) { return (float)rows * (float)a.k * (float)a.batch * 2.0f / 7.0415e6f; }
 // the shares' sums, written, read and added one after the other
 float shares_time(const DenseArgs& a, int64_t rows, int64_t cuts) {
-  return 3.4666f + (float)cuts * (0.3631f + (float)a.M * (float)rows * 8.0f / 3.9616e6f);
+  return 2.71f + (float)cuts * (0.3703f + (float)a.M * (float)rows * 8.0f / 2.708e6f);
 }
 // The time of a product in us, but for what all forms of it share: what the choice of a form and of a number of shares of k needs.
-// The numbers are fitted for the choice, not for the time, to 32,100 timings (52 shapes from 256 x 64 to 32,768 x 1,024, 28,672 x 8,192 and
-// 4,096 x 16,384, 33 to 2,048 tokens, all forms, 1 to 16 shares, weights from memory).  The form it picks takes 0.9 % longer on
-// average than the fastest timed, 11 % at the 99th of 100; against tiles of 256 rows alone, by an estimate of their own, it is 13 %
-// faster on average (6 % beyond 4,096 inputs) and for one product in 200 slower by 5 % or more, 10 % at most.  Fitted to shapes of up to 4,096
-// inputs, most of them, it was for one in ten of the longer ones: 10,752 x 15,232 at 98 tokens 77 -> 89 us, now 75.
+// The numbers are fitted for the choice, not for the time, to 49,600 timings (2,153 products: 111 shapes from 256 x 64 to 32,768 x 1,024,
+// 28,672 x 8,192 and 4,096 x 16,384, 33 to 2,048 tokens, all forms, 1 to 16 shares, every kind of output, weights from memory).  The form
+// it picks takes 0.7 % longer on average than the fastest timed, 11 % at the 99th of 100; against tiles of 256 rows alone, by an
+// estimate of their own, it is 13 % faster on average (21 % with up to 512 inputs, 6 % beyond 4,096) and for one product in 170 slower by 5 %
+// or more, 17 % at most.  Fitted to binary32 outputs and mostly to 1,024 to 4,096 inputs, it was for one in ten of the longer ones
+// and wherever 2,816 to 4,096 rows of 512 met 1,500 tokens or more: 10,752 x 15,232 at 98 tokens 77 -> 89 us, now 74; 3,328 x 512 at 1,500, added to
+// the stream, 19.3 -> 24.7, now 15.5.  The choice costs the host 0.1 to 1 us.
 float many_time(const DenseArgs& a, int64_t rows, const ManyForm& f, int64_t cuts) {
   const int64_t row_tiles = rows / (128 * f.rb), tok_tiles = (a.M + 32 * f.tt - 1) / (32 * f.tt);
   const float groups = (float)(row_tiles * tok_tiles * cuts * a.batch), steps = (float)(((a.k >> 6) + cuts - 1) / cuts);
@@ -699,8 +700,8 @@ float many_time(const DenseArgs& a, int64_t rows, const ManyForm& f, int64_t cut
   const float per_unit = ceilf(groups / 256.0f);
   float t = steps * wait * ceilf(groups / (float)f.resident);
   if (per_unit > 1.0f) t = std::max(t, steps * per_unit * f.step);
-  t = std::max(t, weights_time(a, rows)) + per_unit * f.end;
-  return cuts > 1 ? t + shares_time(a, rows, cuts) : t;
+  t = std::max(t, (float)rows * (float)a.k * (float)a.batch * 2.0f / 9.12e6f);
+  return cuts > 1 ? t + shares_time(a, rows, cuts) : t + per_unit * f.end * (a.out == DENSE_F32 ? 1.0f : 1.7f);
 }
 
 template <int OUT, bool LISTED>
@@ -746,16 +747,16 @@ int launch_listed(const DenseArgs& a, int64_t rows, hipStream_t st) {
 
 }  // namespace
 
-// A product of few tokens goes the way whose time is estimated to be the shorter; what the other way's estimate leaves out is 5.5 us
-// more.  Workgroups that leave compute units idle and long rows, which read the tokens more than the weights, are against
-// the few-token kernel: 6,144 x 12,288 at 20 tokens 54 us, below 36.  Of 520 products (52 shapes from 256 x 64 to 28,672 x 8,192, 2
-// to 32 tokens, both ways timed) the choice is 0.5 % off on average and 16 % at most.
+// A product of few tokens goes the way whose time is estimated to be the shorter; what the other way's estimate leaves out is 7 us
+// more, and it takes the weights' time at least.  Workgroups that leave compute units idle and long rows, which read the tokens more than the
+// weights, are against the few-token kernel: 6,144 x 12,288 at 20 tokens 54 us, below 36.  Of 520 products (52 shapes from 256 x 64 to
+// 28,672 x 8,192, 2 to 32 tokens, both ways timed) the choice is 0.6 % off on average and 16 % at most.
 DenseForm dense_form(const DenseArgs& a, int64_t rows) {
-  constexpr float kManyMore = 5.5f;
+  constexpr float kManyMore = 7.0f;
   const float few = a.M <= kFewTokens ? few_time(a, rows) : HUGE_VALF;
   DenseForm form;
-  // (the other way takes at least the weights' time: mostly known without an estimate of its forms)
-  if (few < weights_time(a, rows) + kManyMore) return form;
+  // (mostly known without an estimate of the other way's forms)
+  if (few < (float)rows * (float)a.k * (float)a.batch * 2.0f / 5.8e6f + kManyMore) return form;
   int64_t most = 1;  // shares of k: at least four steps each
   if (a.workspace && a.batch == 1 && a.M <= 65535)
     most = std::max<int64_t>(1, std::min(std::min<int64_t>(16, a.k >> 8), a.workspace_floats / (a.M * rows)));
