@@ -341,8 +341,8 @@ def main():
                           "tok_s": round(args.steps / elapsed, 1), "ms_per_step": round(1e3 * elapsed / args.steps, 4)}))
         return
 
-    # ---- the prompt pass, both ways (not part of `value`): token by token as the reference does,
-    #      and all positions through each layer together on the matrix cores ---------------------
+    # ---- the prompt pass, both ways (not part of `value`): with the bits of single tokens, as the reference's,
+    #      and batched, whose sums have another order ---------------------
     prefill_ms = {}
     for name, batched in (("batched", True), ("sequential", False)):
         for rep in range(2):                       # the first pass builds graphs / allocates buffers
@@ -351,7 +351,7 @@ def main():
             tp = time.perf_counter()
             eng.prefill(prompt.tolist(), batched=batched)   # returns after the device finished
             prefill_ms[name] = round(1000.0 * (time.perf_counter() - tp), 3)
-    log("prompt of %d tokens: %.2f ms token by token, %.2f ms batched" %
+    log("prompt of %d tokens: %.2f ms with the bits of single tokens, %.2f ms batched" %
         (args.prompt_len, prefill_ms["sequential"], prefill_ms["batched"]))
 
     # ---- timed decode: K steps after the prompt and W warm-up steps ------------------------------

@@ -341,7 +341,7 @@ class Engine:
         check(fn(self._h, _int32_array(prompt_ids), len(prompt_ids)))
 
     def set_prefill_mode(self, batched):
-        """Which prompt loop generateResponse uses (default: token by token)."""
+        """Which prompt loop generateResponse uses (default: the one that leaves the bits of single tokens)."""
         check(self._lib.awq_set_prefill_mode(self._h, 1 if batched else 0))
 
     def decode(self, n_steps):
