@@ -106,8 +106,8 @@ __device__ __forceinline__ const DenseSegment& segment_of(const DenseArgs& a, in
 }
 
 // the weight block of this workgroup's product (one token), or -1: it is left out
-__device__ __forceinline__ int block_of_product(const DenseArgs& a) {
-  const int b = blockIdx.y, by_number = a.batch - a.fixed;
+__device__ __forceinline__ int block_of_product(const DenseArgs& a, int b) {
+  const int by_number = a.batch - a.fixed;
   if (!a.ids) return b;
   if (b >= by_number) return a.n_groups + b - by_number;
   const int group = a.ids[b];

@@ -27,7 +27,7 @@ __global__ __launch_bounds__(256) void dense_one_f32_kernel(DenseArgs a, std::co
   const DenseSegment& s = segment_of(a, base);
   const int local0 = base - s.row0;
   if (local0 >= s.rows) return;
-  const int group = block_of_product(a);
+  const int group = block_of_product(a, blockIdx.y);
   if (group < 0) return;
   const f32x4u_t* x = reinterpret_cast<const f32x4u_t*>(reinterpret_cast<const float*>(s.x) + blockIdx.y * a.x_batch);
   const f32x4_t* w = reinterpret_cast<const f32x4_t*>(reinterpret_cast<const float*>(a.w) + group * a.w_batch);

@@ -78,6 +78,9 @@ struct DenseTile {
 struct DenseArgs {
   const void* w = nullptr;
   int64_t k = 0;  // padded
+  // inputs of a whole row of the weight block, where the product takes k of them (w: the block's first of them, a multiple of 64 behind
+  // its start); 0: k.  One token in bfloat16 only.
+  int64_t ldk = 0;
   int64_t M = 0;
   int32_t n_seg = 1;
   int32_t out = DENSE_STORE;
@@ -123,6 +126,10 @@ enum DensePack {
 };
 int launch_dense_pack(const void* src, bool src_f32, int64_t rows, int64_t cols, void* w, int64_t k_padded, int64_t row0,
                       int64_t col0, bool f32, hipStream_t st, int form = PACK_PLAIN);
+// The product of a token that another launch takes in (`beside` below): bfloat16, DENSE_RESIDUAL, one segment, inputs as they are in
+// memory.  It reads nothing that the launch writes, and the launch nothing of its output.  Checks it and fills in what launch_dense does;
+// a workgroup of 512 threads takes *per_group of the *rows.
+int dense_prepare_beside(DenseArgs* a, int64_t* rows, int* per_group);
 struct NormConvArgs;
 // norm (one token, where dense_norm_fused): launch_norm_conv is part of the product, out1 the input of segment 0, out2 of segment 1;
 // neither is written, and what the segments name as x is not read
@@ -213,7 +220,9 @@ int32_t window_row_padded(int32_t dim);
 int64_t window_parts_floats(int32_t heads, int32_t vdim, int64_t window, int64_t max_pos);
 // Normalise q and k, append k and v, attend.  A value that is infinite or NaN leaves the positions that do not see it as they are;
 // not so in bfloat16 tiles of 64 queries (heads of up to 256), where a value meets queries of its tile with weight zero.
-int launch_window_attention(const WindowAttnArgs& a, bool f32, hipStream_t st);
+// beside (where window_takes_product): a product in the same launch.
+int launch_window_attention(const WindowAttnArgs& a, bool f32, hipStream_t st, const DenseArgs* beside = nullptr);
+bool window_takes_product(const WindowAttnArgs& a, bool f32);
 
 // --- linear attention with a decaying state (linear_attention.hip) -------------------------------------------
 // per head S <- decay S + k v^T, o = S^T q; state [heads][vdim][round_up(dim, 64)] float (S transposed), zero ahead of
@@ -231,7 +240,9 @@ struct LinearAttnArgs {
   PassPos pos;
 };
 int64_t linear_state_floats(int32_t heads, int32_t dim, int32_t vdim);
-int launch_linear_attention(const LinearAttnArgs& a, bool f32, hipStream_t st);
+// beside (where linear_takes_product): a product in the same launch
+int launch_linear_attention(const LinearAttnArgs& a, bool f32, hipStream_t st, const DenseArgs* beside = nullptr);
+bool linear_takes_product(const LinearAttnArgs& a, bool f32);
 // its form for several tokens, token by token (gated_state.hip), and in binary32 for many: dim <= 256, log2_decay set
 int launch_linear_few(const LinearAttnArgs& a, bool f32, hipStream_t st);
 int launch_linear_chunks_f32(const LinearAttnArgs& a, hipStream_t st);

@@ -1,5 +1,5 @@
 // Linear attention with a decaying state (layers.hpp): per head S <- decay S + k v^T, o = S^T q.
-#include "layers.hpp"
+#include "dense_one_device.hpp"
 
 namespace {
 
@@ -8,9 +8,9 @@ namespace {
 constexpr int kCols = 4;
 
 template <typename T, int DPL>
-__global__ __launch_bounds__(256) void linear_step_kernel(LinearAttnArgs a) {
-  const int head = blockIdx.x, lane = threadIdx.x & 63;
-  const int col0 = (blockIdx.y * 4 + (threadIdx.x >> 6)) * kCols;
+__device__ __forceinline__ void step_columns(const LinearAttnArgs& a, const int head, const int block) {
+  const int lane = threadIdx.x & 63;
+  const int col0 = (block * 4 + (threadIdx.x >> 6)) * kCols;
   if (col0 >= a.vdim) return;
   const int dimp = DPL * 64;
   float* state = a.state + ((int64_t)head * a.vdim + col0) * dimp;
@@ -60,6 +60,24 @@ __global__ __launch_bounds__(256) void linear_step_kernel(LinearAttnArgs a) {
       for (int i = 0; i < DPL; ++i) state[c * dimp + i * 64 + lane] = s[c][i];
 }
 
+template <typename T, int DPL>
+__global__ __launch_bounds__(256) void linear_step_kernel(LinearAttnArgs a) {
+  step_columns<T, DPL>(a, blockIdx.x, blockIdx.y);
+}
+
+// The same with a product that does not wait for it in the launch (a layer's W_down beside its mixer): the first `groups` workgroups
+// take the recurrence, four of their wavefronts, the others RW rows of the product each.
+template <int DPL, int RW>
+__global__ __launch_bounds__(512) void linear_step_beside_kernel(LinearAttnArgs a, int groups, DenseArgs beside) {
+  const int block = blockIdx.x;
+  if (block >= groups) {
+    dense_one_rows<8, DENSE_RESIDUAL, IN_READ, RW>(beside, std::false_type(), block - groups, 0);
+    return;
+  }
+  if (threadIdx.x >= 256) return;
+  step_columns<bf16_t, DPL>(a, block % a.heads, block / a.heads);
+}
+
 // The same for many tokens on the matrix cores, 128 tokens (a chunk) after the other.  With t, s counted inside the
 // chunk and S the state ahead of it,
 //     o_t = decay^(t+1) S^T q_t + sum over s <= t of decay^(t-s) (k_s . q_t) v_s
@@ -75,8 +93,6 @@ __global__ __launch_bounds__(256) void linear_step_kernel(LinearAttnArgs a) {
 //     O^T[v][t] += V^T W          W's elements are already where the second operand wants them, if a 16-wide slice
 //                                 j takes s = 16 j + 8 (e / 4) + 4 kh + e % 4; V^T from LDS as [v][t]
 //     S[d][v]   += K^T V'         the same slices; K^T by the transposing LDS read
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef short short4_t __attribute__((ext_vector_type(4)));
 constexpr int kChunk = 128;
 constexpr int kVStride = kChunk + 8;  // elements per column of V^T
@@ -364,9 +380,38 @@ int launch_chunks(const LinearAttnArgs& a, hipStream_t st) {
 // the recurrence 6e-8 (3.5 to 4.2 us for 2 to 15 tokens, a chunk 5.2).
 constexpr int kChunkFrom = 16;
 
+template <int DPL>
+int launch_step_beside(const LinearAttnArgs& a, const DenseArgs& product, hipStream_t st) {
+  DenseArgs p = product;
+  int64_t rows = 0;
+  int per_group = 0;
+  if (int rc = dense_prepare_beside(&p, &rows, &per_group)) return rc;
+  const int64_t groups = (int64_t)a.heads * ((a.vdim + 4 * kCols - 1) / (4 * kCols)), blocks = groups + rows / per_group;
+  AWQ_REQUIRE(blocks < (1ll << 31), "too large");
+  const dim3 g((unsigned)blocks);
+  if (per_group == 8) hipLaunchKernelGGL((linear_step_beside_kernel<DPL, 8>), g, dim3(512), 0, st, a, (int)groups, p);
+  else hipLaunchKernelGGL((linear_step_beside_kernel<DPL, 16>), g, dim3(512), 0, st, a, (int)groups, p);
+  AWQ_HIP_TRY(hipGetLastError());
+  return AWQ_OK;
+}
+
 template <typename T>
-int launch_step(const LinearAttnArgs& a, hipStream_t st) {
+int launch_step(const LinearAttnArgs& a, hipStream_t st, const DenseArgs* beside = nullptr) {
   const dim3 g((unsigned)a.heads, (unsigned)((a.vdim + 4 * kCols - 1) / (4 * kCols)));
+  if constexpr (sizeof(T) == 2) {
+    if (beside) {
+      switch ((a.dim + 63) / 64) {
+        case 1: return launch_step_beside<1>(a, *beside, st);
+        case 2: return launch_step_beside<2>(a, *beside, st);
+        case 3: return launch_step_beside<3>(a, *beside, st);
+        case 4: return launch_step_beside<4>(a, *beside, st);
+        case 5: return launch_step_beside<5>(a, *beside, st);
+        case 6: return launch_step_beside<6>(a, *beside, st);
+        case 7: return launch_step_beside<7>(a, *beside, st);
+        default: return launch_step_beside<8>(a, *beside, st);
+      }
+    }
+  }
   switch ((a.dim + 63) / 64) {
     case 1: hipLaunchKernelGGL((linear_step_kernel<T, 1>), g, dim3(256), 0, st, a); break;
     case 2: hipLaunchKernelGGL((linear_step_kernel<T, 2>), g, dim3(256), 0, st, a); break;
@@ -385,12 +430,15 @@ int launch_step(const LinearAttnArgs& a, hipStream_t st) {
 
 int64_t linear_state_floats(int32_t heads, int32_t dim, int32_t vdim) { return (int64_t)heads * vdim * round_up(dim, 64); }
 
-int launch_linear_attention(const LinearAttnArgs& a, bool f32, hipStream_t st) {
+bool linear_takes_product(const LinearAttnArgs& a, bool f32) { return !f32 && a.M == 1; }
+
+int launch_linear_attention(const LinearAttnArgs& a, bool f32, hipStream_t st, const DenseArgs* beside) {
   AWQ_REQUIRE(a.proj && a.decay && a.state && a.o && a.M >= 1, "bad arguments");
   AWQ_REQUIRE(a.heads >= 1 && a.dim >= 1 && a.vdim >= 1 && a.vdim <= 65536 && a.ldp % 8 == 0 &&
                   a.ldp >= (int64_t)a.heads * (2 * a.dim + a.vdim),
               "bad shape");
   AWQ_REQUIRE(a.dim <= 512, "dim must be at most 512");
+  AWQ_REQUIRE(!beside || linear_takes_product(a, f32), "no product beside this attention");
   const bool chunks = a.log2_decay && a.M >= kChunkFrom && a.M < (1 << 30) && a.dim <= 256;
   if (a.M > 1 && !chunks) return launch_linear_few(a, f32, st);
   if (f32) return chunks ? launch_linear_chunks_f32(a, st) : launch_step<float>(a, st);
@@ -400,5 +448,5 @@ int launch_linear_attention(const LinearAttnArgs& a, bool f32, hipStream_t st) {
     if (a.dim <= 128) return whole ? launch_chunks<128, true>(a, st) : launch_chunks<128, false>(a, st);
     return whole ? launch_chunks<256, true>(a, st) : launch_chunks<256, false>(a, st);
   }
-  return launch_step<bf16_t>(a, st);
+  return launch_step<bf16_t>(a, st, beside);
 }

@@ -1,5 +1,5 @@
 // Attention over a sliding window with a distance bias (layers.hpp).
-#include "lane_sums.hpp"
+#include "dense_one_device.hpp"
 #include "query_attention.hpp"
 
 namespace {
@@ -192,17 +192,16 @@ __device__ __forceinline__ void combine_parts(const WindowAttnArgs& a, int h, in
 
 // U: cache rows of a lane, row length / 32
 template <typename T, int R, int U, bool SAME>
-__global__ __launch_bounds__(256) void window_decode_kernel(WindowAttnArgs a, int chunks) {
+__device__ __forceinline__ void decode_part(const WindowAttnArgs& a, const int chunks, const int block, const int part, const int n_parts) {
   extern __shared__ float red[];      // [4][R][vw]
   __shared__ float sc[R][kPartKeys];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int g = blockIdx.x / chunks, rz = (blockIdx.x - g * chunks) * R;
+  const int g = block / chunks, rz = (block - g * chunks) * R;
   const int per_group = a.heads / a.kv_heads;
   const int nr = min(R, per_group - rz), h0 = g * per_group + rz;
   const int pos = a.pos.position();
   const int lo = a.window > 0 ? max(0, pos - a.window + 1) : 0;
   const int parts = (pos + 1 - lo + kPartKeys - 1) / kPartKeys;
-  const int part = blockIdx.y;
   if (part >= parts) return;
   const int b = lo + part * kPartKeys, nk = min(kPartKeys, pos + 1 - b);
   const bool newest = part == parts - 1;
@@ -313,7 +312,6 @@ __global__ __launch_bounds__(256) void window_decode_kernel(WindowAttnArgs a, in
       if (lane < tpv) red[(wave * R + r) * vw + c0 + j] = acc[r][j];
     }
   __syncthreads();
-  const int n_parts = gridDim.y;
   const bool alone = n_parts == 1 || (SAME && parts == 1);
 #pragma unroll
   for (int r = 0; r < R; ++r) {
@@ -333,14 +331,32 @@ __global__ __launch_bounds__(256) void window_decode_kernel(WindowAttnArgs a, in
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (tid == 0) {
-      last = __hip_atomic_fetch_add(a.done + blockIdx.x, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
-      if (last) __hip_atomic_store(a.done + blockIdx.x, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
+      last = __hip_atomic_fetch_add(a.done + block, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == parts - 1;
+      if (last) __hip_atomic_store(a.done + block, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // for the next launch
     }
     __syncthreads();
     if (!last) return;
     static_assert(R == 1, "heads next to each other would be added up one after the other");
     combine_parts<T, true>(a, h0, n_parts, parts, red);
   }
+}
+
+template <typename T, int R, int U, bool SAME>
+__global__ __launch_bounds__(256) void window_decode_kernel(WindowAttnArgs a, int chunks) {
+  decode_part<T, R, U, SAME>(a, chunks, blockIdx.x, blockIdx.y, gridDim.y);
+}
+
+// The same with a product that does not wait for it in the launch (a layer's W_down beside its attention): the first
+// groups * n_parts workgroups attend, four of their wavefronts, the others take RW rows of the product each.
+template <int R, int U, bool SAME, int RW>
+__global__ __launch_bounds__(512) void window_decode_beside_kernel(WindowAttnArgs a, int chunks, int groups, int n_parts, DenseArgs beside) {
+  const int block = blockIdx.x;
+  if (block >= groups * n_parts) {
+    dense_one_rows<8, DENSE_RESIDUAL, IN_READ, RW>(beside, std::false_type(), block - groups * n_parts, 0);
+    return;
+  }
+  if (threadIdx.x >= 256) return;
+  decode_part<bf16_t, R, U, SAME>(a, chunks, block % groups, block / groups, n_parts);
 }
 
 // a workgroup per head
@@ -352,28 +368,50 @@ __global__ __launch_bounds__(256) void window_combine_kernel(WindowAttnArgs a, i
   combine_parts<T, false>(a, blockIdx.x, n_parts, parts, red);
 }
 
+template <int R, int U, bool SAME>
+int launch_decode_beside(const WindowAttnArgs& a, int chunks, int parts, size_t lds, const DenseArgs& product, hipStream_t st) {
+  DenseArgs p = product;
+  int64_t rows = 0;
+  int per_group = 0;
+  if (int rc = dense_prepare_beside(&p, &rows, &per_group)) return rc;
+  const int groups = a.kv_heads * chunks;
+  const int64_t blocks = (int64_t)groups * parts + rows / per_group;
+  AWQ_REQUIRE(blocks < (1ll << 31), "too large");
+  const dim3 g((unsigned)blocks);
+  if (per_group == 8) hipLaunchKernelGGL((window_decode_beside_kernel<R, U, SAME, 8>), g, dim3(512), lds, st, a, chunks, groups, parts, p);
+  else hipLaunchKernelGGL((window_decode_beside_kernel<R, U, SAME, 16>), g, dim3(512), lds, st, a, chunks, groups, parts, p);
+  return AWQ_OK;
+}
+
 template <typename T, int R, bool SAME>
-void launch_decode_parts(const WindowAttnArgs& a, int parts, hipStream_t st) {
+int launch_decode_parts(const WindowAttnArgs& a, int parts, const DenseArgs* beside, hipStream_t st) {
   const int chunks = (a.heads / a.kv_heads + R - 1) / R;
   const dim3 g((unsigned)(a.kv_heads * chunks), (unsigned)parts);
   const size_t lds = sizeof(float) * 4 * R * a.vl.row;  // (256 floats at least)
   const int row = std::max(a.kl.row, a.vl.row);
+  if constexpr (sizeof(T) == 2) {
+    if (beside) {
+      if (row == 64) return launch_decode_beside<R, 2, SAME>(a, chunks, parts, lds, *beside, st);
+      if (row == 128) return launch_decode_beside<R, 4, SAME>(a, chunks, parts, lds, *beside, st);
+      return launch_decode_beside<R, 8, SAME>(a, chunks, parts, lds, *beside, st);
+    }
+  }
   if (row == 64) hipLaunchKernelGGL((window_decode_kernel<T, R, 2, SAME>), g, dim3(256), lds, st, a, chunks);
   else if (row == 128) hipLaunchKernelGGL((window_decode_kernel<T, R, 4, SAME>), g, dim3(256), lds, st, a, chunks);
   else hipLaunchKernelGGL((window_decode_kernel<T, R, 8, SAME>), g, dim3(256), lds, st, a, chunks);
+  return AWQ_OK;
 }
 
 template <typename T>
-int launch_decode(const WindowAttnArgs& a, hipStream_t st) {
+int launch_decode(const WindowAttnArgs& a, hipStream_t st, const DenseArgs* beside) {
   const int parts = window_parts(a.window, a.len_bound);
   AWQ_REQUIRE(parts >= 1 && parts <= 65535, "too many keys");
   const int per = a.heads / a.kv_heads;
   const bool same = a.done && window_counted_parts(a.heads, a.kv_heads, a.window, a.len_bound);
-  if (same) launch_decode_parts<T, 1, true>(a, parts, st);
-  else if (per == 1) launch_decode_parts<T, 1, false>(a, parts, st);
-  else if (per == 2) launch_decode_parts<T, 2, false>(a, parts, st);
-  else if (per <= 4) launch_decode_parts<T, 4, false>(a, parts, st);
-  else launch_decode_parts<T, 8, false>(a, parts, st);
+  const auto launch = same ? launch_decode_parts<T, 1, true>
+                           : per == 1 ? launch_decode_parts<T, 1, false>
+                                      : per == 2 ? launch_decode_parts<T, 2, false> : per <= 4 ? launch_decode_parts<T, 4, false> : launch_decode_parts<T, 8, false>;
+  if (int rc = launch(a, parts, beside, st)) return rc;
   AWQ_HIP_TRY(hipGetLastError());
   if (parts > 1 && !same) {
     hipLaunchKernelGGL(window_combine_kernel<T>, dim3((unsigned)a.heads), dim3(256), 0, st, a, parts);
@@ -389,7 +427,6 @@ int launch_decode(const WindowAttnArgs& a, hipStream_t st) {
 // so that a query's maximum, sum and rescaling stay in a lane and its partner, and the weights a lane forms are the
 // elements it supplies to the second product (slice j: keys 16 j + 8 (e / 4) + 4 kh + e % 4; V^T by the transposing
 // LDS read).  Scores and weights are binary32; a weight enters the product as the sum of two bfloat16 terms.
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef short short4_t __attribute__((ext_vector_type(4)));
 constexpr int kTileQueries = 128, kTileKeys = 32;
 
@@ -621,19 +658,22 @@ int64_t window_parts_floats(int32_t heads, int32_t vdim, int64_t window, int64_t
   return (int64_t)heads * window_parts(window, max_pos) * (2 + vdim);
 }
 
-int launch_window_attention(const WindowAttnArgs& a, bool f32, hipStream_t st) {
+static bool one_token_form(const WindowAttnArgs& a) { return a.kl.row <= 256 && a.vl.row <= 256 && a.M == 1 && a.parts && a.len_bound > 0; }
+
+bool window_takes_product(const WindowAttnArgs& a, bool f32) { return !f32 && one_token_form(a); }
+
+int launch_window_attention(const WindowAttnArgs& a, bool f32, hipStream_t st, const DenseArgs* beside) {
   AWQ_REQUIRE(a.proj && a.k_cache && a.v_cache && a.ctx && a.slope && a.M >= 1 && a.M <= 65535, "bad arguments");
   AWQ_REQUIRE(a.heads >= 1 && a.kv_heads >= 1 && a.heads % a.kv_heads == 0, "heads must be a multiple of kv_heads");
   AWQ_REQUIRE(a.dim >= 1 && a.dim <= 1024 && a.vdim >= 1 && a.vdim <= kMaxCols, "head sizes must be at most 1024");
   AWQ_REQUIRE(a.kl.slots > 0 && a.kl.slots % 64 == 0 && a.vl.slots == a.kl.slots && a.kl.row == window_row_padded(a.dim) &&
                   a.vl.row == window_row_padded(a.vdim) && a.ldp % 8 == 0 && a.ldc % 8 == 0,
               "bad cache layout");
-  const bool tiled = a.kl.row <= 256 && a.vl.row <= 256;
-  if (a.M == 1 && tiled && a.parts && a.len_bound > 0)
-    return f32 ? launch_decode<float>(a, st) : launch_decode<bf16_t>(a, st);
+  AWQ_REQUIRE(!beside || window_takes_product(a, f32), "no product beside this attention");
+  if (one_token_form(a)) return f32 ? launch_decode<float>(a, st, nullptr) : launch_decode<bf16_t>(a, st, beside);
   if (int rc = f32 ? launch_append<float>(a, st) : launch_append<bf16_t>(a, st)) return rc;
   if (f32) return launch_queries<float>(a, st);
-  if (!tiled || a.pos.dyn) return launch_queries<bf16_t>(a, st);
+  if (a.kl.row > 256 || a.vl.row > 256 || a.pos.dyn) return launch_queries<bf16_t>(a, st);
   if (a.kl.row == 64) launch_tiles<64>(a, st);
   else if (a.kl.row == 128) launch_tiles<128>(a, st);
   else launch_tiles<256>(a, st);

@@ -134,6 +134,29 @@ def test_greedy_generation(case):
     assert eng.generateResponse(prompt, 5) == out[:5]
 
 
+# rows of 32 inputs that a run of eight wavefronts leaves over, workgroups of 8 rows (up to 2,048 rows of more than 1,024 inputs) and
+# of 16, heads that share a kv head or have parts of a window to add, both mixers
+@pytest.mark.parametrize("width,ff,heads,kv_heads,dim,window", [(64, 1, 2, 2, 64, None), (96, 1030, 4, 2, 64, 70), (256, 2500, 8, 1, 32, 130),
+                                                                (2304, 1500, 3, 3, 128, 66), (320, 9000, 12, 3, 16, None)], ids=str)
+def test_single_tokens_with_the_second_matrix_beside_the_mixer(awq, torch_gpu, tmp_path, width, ff, heads, kv_heads, dim, window):
+    cfg = km.model(width, 64, [km.attention(heads, kv_heads, dim, dim, window, ff=ff), km.lightning(3, dim + 4, dim, [0.6, 0.9, 0.99], ff=ff)],
+                   groups=2, taps=4, loop=(0, 2, 2))
+    w = km.weights(cfg, width + ff)
+    km.write(str(tmp_path), cfg, w)
+    tokens = np.random.default_rng(3).integers(0, 64, 84).tolist()
+    taps = []
+    plain.forward(cfg, w, tokens, taps)
+    eng = awq.open_model(str(tmp_path), max_positions=300)
+    eng.set_layer_tap(True)
+    eng.forward(tokens[:72])
+    for t in range(72, 84):
+        eng.forward(tokens[t:t + 1])
+        got = eng.read_layer_tap().reshape(len(taps), width)
+        for i in range(len(taps)):
+            assert km.rms_error(got[i], taps[i][t]) < LIMIT["bfloat16"], "layer run %d, token %d" % (i, t)
+    eng.close()
+
+
 def test_long_sequence_in_wrapping_rings(awq, torch_gpu, tmp_path):
     """more positions than a ring holds: a window behind one pass of 2048"""
     cfg = km.model(32, 64, [km.attention(2, 1, 16, 8, 9, ff=32), km.lightning(1, 8, 8, [0.99])], groups=2, taps=2)
