@@ -119,20 +119,45 @@ __global__ __launch_bounds__(256) void dense_one_f32_kernel(DenseArgs a, std::co
 }
 
 // --- many tokens ---------------------------------------------------------------------------------------------
-// On v_mfma_f32_32x32x2_f32: a workgroup of four wavefronts takes 64 rows and 32 TW C tokens, steps of 32 inputs.  Two
-// wavefronts share the rows, TW the tokens (C accumulators each) and KW the inputs of a step, whose sums meet in LDS.
-// Weights and tokens go through LDS, 128 bytes per row and step, the eight 16-byte pieces of row r at positions c ^ (r & 7),
-// requested a step ahead into registers.  Lane (n, kh) reads piece 2 j + kh of row n of both operands, and instruction e
-// multiplies element e of the two: the inputs of a step are met in another order on both sides alike.
-// Up to about 50 tokens bound by the weights' bytes (2 operations per token and 4 bytes against 134 TFLOP/s and 5.1 TB/s),
-// beyond by the matrix cores.  Where the tiles do not fill the device, k is cut over `cuts` workgroups and a second launch
-// adds their sums, as in bfloat16.  333 tokens, sums added: 1,024 rows of 4,096 inputs 39 us, 7,168 of 1,024 57, 32,768 of 1,024
-// 212 (106 TFLOP/s); 4 x 4 sums per thread without matrix cores took 270, 135 and 482.  20 tokens on 1,024 x 4,096: 18, was 273.
-template <int TW, int KW, int C, int OUT, bool LISTED = false>
-__global__ __launch_bounds__(256) void dense_many_f32_kernel(DenseArgs a, int row_tiles, int tok_tiles, int cuts) {
-  static_assert(TW * KW == 2, "four wavefronts, two of them share the rows");
-  constexpr int TOK = 32 * TW * C, NL = (64 + TOK) / 32;  // pieces per thread and step
-  __shared__ __attribute__((aligned(16))) float tiles[2][(64 + TOK) * 32];
+// Four numbers as sums of three bfloat16 terms: the upper halves of the numbers, of what that leaves, and of what is left then.  Eight
+// bits of significand each, so the sum is the number itself (down to 2^-110, where the last term leaves the range).
+struct Split4 {
+  uint2 part[3];
+};
+__device__ __forceinline__ uint2 upper_halves(const f32x4_t v) {
+  return make_uint2(__builtin_amdgcn_perm(__float_as_uint(v[1]), __float_as_uint(v[0]), 0x07060302u),
+                    __builtin_amdgcn_perm(__float_as_uint(v[3]), __float_as_uint(v[2]), 0x07060302u));
+}
+__device__ __forceinline__ Split4 split4(f32x4_t v) {
+  Split4 s;
+#pragma unroll
+  for (int p = 0; p < 3; ++p) {
+    s.part[p] = upper_halves(v);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] -= __uint_as_float(__float_as_uint(v[e]) & 0xffff0000u);
+  }
+  return s;
+}
+
+// On v_mfma_f32_32x32x16_bf16, whose products are exact and which does 16 times the operations of v_mfma_f32_32x32x2_f32: both operands
+// as three terms each and the six products of two terms that are 2^-18 of the whole or more (the others 2^-24 at most, of either sign); where a step's weights are
+// bfloat16 numbers, as a checkpoint in bfloat16 has them, three are left and nothing is left out.  The first terms' products have a sum
+// of their own, which is rounded once per 16 inputs.  A workgroup of
+// four wavefronts takes 32 RW rows and 32 TW C tokens, steps of 32 inputs; KW wavefronts share the inputs of a step, whose
+// sums meet in LDS.  Weights and tokens are requested two steps ahead into registers, split once and go through LDS, a term's 64 bytes per row and
+// step, the four 16-byte pieces of row r at positions c ^ (r / 4 & 3).  Bound by the splitting (vector instructions) beside the matrix
+// cores, at few tokens by the weights' bytes.  Where the tiles do not fill the device, k is cut over `cuts` workgroups and a second
+// launch adds their sums, as in bfloat16.  333 tokens: 1,024 rows of 4,096 inputs 39.7 -> 27 us, 7,168 of 1,024 59 -> 35, 32,768 of
+// 1,024 211 -> 116 (v_mfma_f32_32x32x2_f32 before); with weights that are no bfloat16 numbers 35, 52 and 183, and up to 50 tokens, where weights' bytes
+// and trips to memory are the time, up to 6 % more than before.  Off from 64 bits by 0.8e-7 to 1.9e-7, before 1.6e-7 to 5.7e-7.
+// An infinity has no such terms (what it leaves is NaN): a wavefront that finds sums that are not finite forms them again, in binary32.
+template <int RW, int TW, int KW, int C, int OUT, bool LISTED = false>
+__global__ __launch_bounds__(256, 2) void dense_many_f32_kernel(DenseArgs a, int row_tiles, int tok_tiles, int cuts) {
+  static_assert(RW * TW * KW == 4 && (KW == 1 || (KW == 2 && C == 1)), "four wavefronts");
+  constexpr int ROWS = 32 * RW, TOK = 32 * TW * C, NW = ROWS / 32, NL = (ROWS + TOK) / 32;  // pieces per thread and step, NW of weights
+  constexpr int PLANE = (ROWS + TOK) * 32;
+  __shared__ __attribute__((aligned(16))) bf16_t planes[2][3][PLANE];
+  __shared__ __attribute__((aligned(16))) int wide[4];  // by wavefront that split them: some of the weights so far were no bfloat16 numbers
   const int total = row_tiles * tok_tiles * cuts;
   // workgroups whose indices agree modulo 8 share a die: each die walks its own run of row tiles
   const int per = (total + 7) >> 3;
@@ -152,65 +177,122 @@ __global__ __launch_bounds__(256) void dense_many_f32_kernel(DenseArgs a, int ro
   }
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, kh = lane >> 5;
-  const int rw = wave & 1, tw = TW == 2 ? wave >> 1 : 0, kw = KW == 2 ? wave >> 1 : 0;
-  const DenseSegment& s = segment_of(a, rt * 64);
-  if (rt * 64 >= a.seg[a.n_seg - 1].row0 + a.seg[a.n_seg - 1].rows) return;  // padding
+  const int rw = wave % RW, tw = TW > 1 ? wave / RW : 0, kw = KW > 1 ? wave / RW : 0;
+  const DenseSegment& s = segment_of(a, rt * ROWS);
+  if (rt * ROWS >= a.seg[a.n_seg - 1].row0 + a.seg[a.n_seg - 1].rows) return;  // padding
   const int all_steps = (int)(a.k >> 5);
   const int first_step = (int)((int64_t)all_steps * cut / cuts);
   const int steps = (int)((int64_t)all_steps * (cut + 1) / cuts) - first_step;
+  const float* const w_rows = reinterpret_cast<const float*>(a.w) + group * a.w_batch + (int64_t)rt * ROWS * a.k + first_step * 32;
+  const float* const x_rows = reinterpret_cast<const float*>(s.x) + blockIdx.y * a.x_batch + first_step * 32;
+  auto token = [&](int i) __attribute__((always_inline)) {
+    int64_t tok = min(tt0 + i, n_tok - 1);
+    if constexpr (LISTED) tok = list[tok] / a.list_div;
+    return tok;
+  };
 
-  // this thread's pieces of a step: place tid % 8 of rows tid / 8 + 32 i, the first two of them weights
+  // this thread's pieces of a step: place tid % 8 of rows tid / 8 + 32 i, the first NW of them weights
   const float* src[NL];
   const int lr = tid >> 3, at = (tid & 7) << 2;
 #pragma unroll
-  for (int i = 0; i < NL; ++i) {
-    if (i < 2) {
-      src[i] = reinterpret_cast<const float*>(a.w) + group * a.w_batch + (int64_t)(rt * 64 + lr + 32 * i) * a.k;
+  for (int i = 0; i < NL; ++i) src[i] = (i < NW ? w_rows + (int64_t)(lr + 32 * i) * a.k : x_rows + token(lr + 32 * (i - NW)) * s.ldx) + at;
+  const int place = lr * 32 + ((((tid & 7) >> 1) ^ ((lr >> 2) & 3)) << 3) + (tid & 1) * 4;
+  typedef f32x4_t Step[NL];
+  auto request = [&](Step& to, int step) __attribute__((always_inline)) {
+    step = min(step, steps - 1);
+#pragma unroll
+    for (int i = 0; i < NL; ++i) to[i] = *reinterpret_cast<const f32x4u_t*>(src[i] + step * 32);
+  };
+  int dirty = 3;  // buffers whose second and third terms of this wavefront's weights may be other than zero
+  auto keep = [&](const Step& from, int buf) __attribute__((always_inline)) {
+    bf16_t* const to = planes[buf][0] + place;
+    uint32_t below = 0;
+#pragma unroll
+    for (int i = 0; i < NW; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) below |= __float_as_uint(from[i][e]);
+    const bool any = __builtin_amdgcn_ballot_w64((below & 0xffffu) != 0) != 0;
+    if (any || (dirty >> buf & 1)) {
+#pragma unroll
+      for (int i = 0; i < NW; ++i) {
+        const Split4 w = split4(from[i]);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2*>(to + p * PLANE + i * 1024) = w.part[p];
+      }
+      if (lane == 0 && (any || dirty == 3)) wide[wave] = any ? 1 : 0;
+      dirty = any ? dirty | 1 << buf | 4 : dirty & ~(1 << buf);
     } else {
-      int64_t tok = min(tt0 + lr + 32 * (i - 2), n_tok - 1);
-      if constexpr (LISTED) tok = list[tok] / a.list_div;
-      src[i] = reinterpret_cast<const float*>(s.x) + blockIdx.y * a.x_batch + tok * s.ldx;
+#pragma unroll
+      for (int i = 0; i < NW; ++i) *reinterpret_cast<uint2*>(to + i * 1024) = upper_halves(from[i]);
     }
-    src[i] += first_step * 32 + at;
-  }
-  const int place = lr * 32 + (((tid & 7) ^ (lr & 7)) << 2);
-  f32x4_t next[NL];
-  auto request = [&](int step) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < NL; ++i) next[i] = *reinterpret_cast<const f32x4u_t*>(src[i] + step * 32);
-  };
-  auto keep = [&](float* to) __attribute__((always_inline)) {
+    for (int i = NW; i < NL; ++i) {
+      const Split4 x = split4(from[i]);
 #pragma unroll
-    for (int i = 0; i < NL; ++i) *reinterpret_cast<f32x4_t*>(to + i * 1024 + place) = next[i];
+      for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2*>(to + p * PLANE + i * 1024) = x.part[p];
+    }
   };
-  f32x16_t acc[C];
+  f32x16_t acc[C], low[C];
 #pragma unroll
   for (int t = 0; t < C; ++t)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) acc[t][i] = 0.0f;
-  request(0);
-  keep(tiles[0]);
-  __syncthreads();
-  for (int st = 0; st < steps; ++st) {
-    if (st + 1 < steps) request(st + 1);
-    const float* const now = tiles[st & 1];
+    for (int i = 0; i < 16; ++i) acc[t][i] = low[t][i] = 0.0f;
+  auto multiply = [&](int buf, bool all) __attribute__((always_inline)) {
 #pragma unroll
-    for (int jj = 0; jj < 4 / KW; ++jj) {
-      const int piece = ((2 * (jj + kw * 2) + kh) ^ (n & 7)) << 2;
-      const f32x4_t wv = *reinterpret_cast<const f32x4_t*>(now + (rw * 32 + n) * 32 + piece);
-      f32x4_t xv[C];
+    for (int jj = 0; jj < 2 / KW; ++jj) {
+      const int piece = ((2 * (jj + kw) + kh) ^ ((n >> 2) & 3)) << 3;
+      auto term = [&](int p, int row) __attribute__((always_inline)) {
+        return *reinterpret_cast<const bf16x8_t*>(planes[buf][p] + (row + n) * 32 + piece);
+      };
+      bf16x8_t xv[3][C];
 #pragma unroll
-      for (int t = 0; t < C; ++t) xv[t] = *reinterpret_cast<const f32x4_t*>(now + (64 + (tw * C + t) * 32 + n) * 32 + piece);
+      for (int p = 0; p < 3; ++p)
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
+        for (int t = 0; t < C; ++t) xv[p][t] = term(p, ROWS + (tw * C + t) * 32);
+      auto add = [&](f32x16_t (&to)[C], bf16x8_t wv, int p) __attribute__((always_inline)) {
 #pragma unroll
-        for (int t = 0; t < C; ++t) acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(wv[e], xv[t][e], acc[t], 0, 0, 0);
+        for (int t = 0; t < C; ++t) to[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv, xv[p][t], to[t], 0, 0, 0);
+      };
+      const bf16x8_t w0 = term(0, rw * 32);
+      if (all) {
+        const bf16x8_t w1 = term(1, rw * 32), w2 = term(2, rw * 32);
+        add(low, w2, 0);
+        add(low, w1, 1);
+        add(low, w1, 0);
+      }
+      add(low, w0, 2);
+      add(acc, w0, 0);
+      add(low, w0, 1);
     }
-    if (st + 1 < steps) keep(tiles[(st + 1) & 1]);  // its readers passed the barrier behind the step before
+  };
+  auto step = [&](Step& now, Step& after, int st) __attribute__((always_inline)) {
+    // `now` is in LDS already; `after` arrives for the step behind this one
     __syncthreads();
+    typedef int int4_t __attribute__((ext_vector_type(4)));
+    const int4_t some = *reinterpret_cast<const volatile int4_t*>(wide);
+    const bool all = __builtin_amdgcn_readfirstlane(some[0] | some[1] | some[2] | some[3]) != 0;
+    request(now, st + 2);
+    multiply(st & 1, all);
+    if (st + 1 < steps) keep(after, (st + 1) & 1);  // its readers passed the barrier
+  };
+  Step even, odd;
+  request(even, 0);
+  request(odd, 1);
+  keep(even, 0);
+  for (int st = 0;;) {
+    step(even, odd, st);
+    if (++st == steps) break;
+    step(odd, even, st);
+    if (++st == steps) break;
   }
+#pragma unroll
+  for (int t = 0; t < C; ++t)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[t][i] += low[t][i];
+  __syncthreads();
+  float* const turns = reinterpret_cast<float*>(&planes[0][0][0]);
   if constexpr (KW == 2) {
-    float* const other = tiles[0] + rw * 1024;
+    float* const other = turns + rw * 1024;
     if (kw == 1) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) other[i * 64 + lane] = acc[0][i];
@@ -221,7 +303,22 @@ __global__ __launch_bounds__(256) void dense_many_f32_kernel(DenseArgs a, int ro
     for (int i = 0; i < 16; ++i) acc[0][i] += other[i * 64 + lane];
     wave_sync();
   }
-  store_block_rows<float, OUT, LISTED>(a, tiles[0] + wave * 1024, acc, rt * 64 + rw * 32, tt0 + tw * C * 32, n_tok, list, row_tiles * 64,
+#pragma unroll
+  for (int t = 0; t < C; ++t) {
+    bool finite = true;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) finite = finite && __builtin_fabsf(acc[t][i]) < INFINITY;
+    if (__builtin_amdgcn_ballot_w64(!finite) == 0) continue;
+    f32x16_t again;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) again[i] = 0.0f;
+    const float *w = w_rows + (int64_t)(rw * 32 + n) * a.k + kh, *x = x_rows + token((tw * C + t) * 32 + n) * s.ldx + kh;
+    for (int i = 0; i < 32 * steps; i += 2) again = __builtin_amdgcn_mfma_f32_32x32x2f32(w[i], x[i], again, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      if (!(__builtin_fabsf(acc[t][i]) < INFINITY)) acc[t][i] = again[i];
+  }
+  store_block_rows<float, OUT, LISTED>(a, turns + wave * 1024, acc, rt * ROWS + rw * 32, tt0 + tw * C * 32, n_tok, list, row_tiles * ROWS,
                                        cut);
 }
 
@@ -241,31 +338,36 @@ int launch_one(const DenseArgs& a, int64_t rows, hipStream_t st) {
   return AWQ_OK;
 }
 
-// The time of a product of many tokens in us, but for what all forms of it share, for the choice between tiles of 32, 64 and 128
-// tokens and shares of k: a step of a workgroup that has its compute unit to itself, the steps of several on one, weights
-// at 4.6 TB/s, the shares' sums written and read at 6.8 TB/s.  Fitted to 1,190 timings (eight shapes from 256 x 1,536 to 32,768
-// x 1,024, 3 to 512 tokens, 1 to 16 shares; 5 % off in the mean square with 7.3 us added).  The form it picks takes 2.9 % longer
-// on average than the fastest timed; two workgroups per compute unit whatever the size, as it was, 7.4 %, up to 30 %.
-float many_time(const DenseArgs& a, int64_t rows, int tile, int64_t cuts) {
-  const float alone = tile == 32 ? 0.52f : tile == 64 ? 0.65f : 1.18f, beside = tile == 32 ? 0.32f : tile == 64 ? 0.56f : 1.05f;
+// The tiles of a product of many tokens: few rows and tokens make many workgroups, four, three and two of which a compute unit holds.
+struct Form {
+  int rows, tokens;
+  float alone, beside, end;  // a step of a workgroup that has its unit to itself, and of one of several; the end of a tile
+};
+constexpr int kForms = 3;
+constexpr Form kForm[kForms] = {{64, 32, 0.4714f, 0.2758f, 0.0706f}, {64, 64, 0.7176f, 0.3196f, 0.018f}, {128, 64, 0.7455f, 0.5484f, 0.0376f}};
+
+// The time of a product in us, but for what all forms of it share: what the choice of a form and of a number of shares of k needs.  Fitted
+// for the choice, not for the time, to 5,997 timings (20 shapes from 256 x 256 to 32,768 x 1,024, 2 to 512 tokens, 1 to 16 shares; weights that
+// are bfloat16 numbers).  The form it picks takes 0.8 % longer on average than the fastest timed, 11 % at the 99th of 100.
+float many_time(const DenseArgs& a, int64_t rows, const Form& f, int64_t cuts) {
   const float steps = (float)(((a.k >> 5) + cuts - 1) / cuts);
-  const float per_unit = ceilf((float)(rows / 64 * ((a.M + tile - 1) / tile) * cuts * a.batch) / 256.0f);
-  float t = std::max(steps * alone, (float)rows * (float)a.k * (float)a.batch * 4.0f / 4.6e6f);
-  if (per_unit > 1.0f) t = std::max(t, steps * beside * per_unit);
-  if (cuts > 1) t += 2.3f + (float)cuts * (float)a.M * (float)rows * 8.0f / 6.8e6f;
-  return t;
+  const float per_unit = ceilf((float)(rows / f.rows * ((a.M + f.tokens - 1) / f.tokens) * cuts * a.batch) / 256.0f);
+  float t = std::max(steps * f.alone, (float)rows * (float)a.k * (float)a.batch * 4.0f / 7.169e6f);
+  if (per_unit > 1.0f) t = std::max(t, steps * f.beside * per_unit);
+  if (cuts > 1) return t + 2.743f + (float)cuts * (0.3704f + (float)a.M * (float)rows * 8.0f / 4.476e6f);
+  return t + per_unit * f.end;
 }
 
 template <int OUT, bool LISTED>
-int launch_tiles(const DenseArgs& a, int64_t rows, int tile, int tok_tiles, int cuts, hipStream_t st) {
-  const int row_tiles = (int)(rows / 64);
+int launch_tiles(const DenseArgs& a, int64_t rows, int form, int tok_tiles, int cuts, hipStream_t st) {
+  const int row_tiles = (int)(rows / kForm[form].rows);
   const dim3 grid((unsigned)(((int64_t)row_tiles * tok_tiles * cuts + 7) / 8 * 8), (unsigned)a.batch);
-  if (tile == 32)
-    hipLaunchKernelGGL((dense_many_f32_kernel<1, 2, 1, OUT, LISTED>), grid, dim3(256), 0, st, a, row_tiles, tok_tiles, cuts);
-  else if (tile == 64)
-    hipLaunchKernelGGL((dense_many_f32_kernel<2, 1, 1, OUT, LISTED>), grid, dim3(256), 0, st, a, row_tiles, tok_tiles, cuts);
+  if (form == 0)
+    hipLaunchKernelGGL((dense_many_f32_kernel<2, 1, 2, 1, OUT, LISTED>), grid, dim3(256), 0, st, a, row_tiles, tok_tiles, cuts);
+  else if (form == 1)
+    hipLaunchKernelGGL((dense_many_f32_kernel<2, 2, 1, 1, OUT, LISTED>), grid, dim3(256), 0, st, a, row_tiles, tok_tiles, cuts);
   else
-    hipLaunchKernelGGL((dense_many_f32_kernel<2, 1, 2, OUT, LISTED>), grid, dim3(256), 0, st, a, row_tiles, tok_tiles, cuts);
+    hipLaunchKernelGGL((dense_many_f32_kernel<4, 1, 1, 2, OUT, LISTED>), grid, dim3(256), 0, st, a, row_tiles, tok_tiles, cuts);
   AWQ_HIP_TRY(hipGetLastError());
   return AWQ_OK;
 }
@@ -275,18 +377,18 @@ int launch_many(const DenseArgs& a, int64_t rows, hipStream_t st) {
   int64_t most = 1;  // shares of k: at least four steps each
   if (a.workspace && a.batch == 1 && a.M <= 65535)
     most = std::max<int64_t>(1, std::min(std::min<int64_t>(16, a.k >> 7), a.workspace_floats / (a.M * rows)));
-  int tile = 32;
+  int form = 0;
   int64_t cuts = 1;
   float best = HUGE_VALF;
-  for (int t = 32; t <= 128; t *= 2)
+  for (int f = 0; f < kForms; ++f)
     for (int64_t c = 1; c <= most; ++c) {
-      const float time = many_time(a, rows, t, c);
-      if (time < best) best = time, tile = t, cuts = c;
+      const float time = many_time(a, rows, kForm[f], c);
+      if (time < best) best = time, form = f, cuts = c;
     }
-  const int64_t tok_tiles = (a.M + tile - 1) / tile, tiles = rows / 64 * tok_tiles;
+  const int64_t tok_tiles = (a.M + kForm[form].tokens - 1) / kForm[form].tokens, tiles = rows / 64 * tok_tiles;
   AWQ_REQUIRE(tiles < (1ll << 26), "too large");
-  if (cuts == 1) return launch_tiles<OUT, false>(a, rows, tile, (int)tok_tiles, 1, st);
-  if (int rc = launch_tiles<DENSE_PART, false>(a, rows, tile, (int)tok_tiles, (int)cuts, st)) return rc;
+  if (cuts == 1) return launch_tiles<OUT, false>(a, rows, form, (int)tok_tiles, 1, st);
+  if (int rc = launch_tiles<DENSE_PART, false>(a, rows, form, (int)tok_tiles, (int)cuts, st)) return rc;
   hipLaunchKernelGGL((dense_parts_kernel<float, OUT>), dim3((unsigned)((rows / 4 + 255) / 256), (unsigned)a.M), dim3(256), 0, st, a,
                      (int)rows, (int)cuts);
   AWQ_HIP_TRY(hipGetLastError());
@@ -321,7 +423,7 @@ int launch_dense_one_joined_f32(const DenseArgs& a, const JoinArgs& j, int64_t r
 }
 
 int launch_dense_many_f32(const DenseArgs& a, int64_t rows, hipStream_t st) {
-  if (a.tiles) return launch_tiles<DENSE_STORE, true>(a, rows, a.tile_tokens <= 32 ? 32 : 64, a.max_tiles, 1, st);
+  if (a.tiles) return launch_tiles<DENSE_STORE, true>(a, rows, a.tile_tokens <= 32 ? 0 : 1, a.max_tiles, 1, st);
   switch (a.out) {
     case DENSE_STORE: return launch_many<DENSE_STORE>(a, rows, st);
     case DENSE_RESIDUAL: return launch_many<DENSE_RESIDUAL>(a, rows, st);

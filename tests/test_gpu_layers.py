@@ -129,6 +129,56 @@ def test_binary32_products_at_the_edges_of_tiles(awq, lib, dev, tokens, rows, k)
             assert np.abs(got - want).max() < 8 * k ** 0.5 * 2.0 ** -24
 
 
+# weights that are bfloat16 numbers, all of them, all but those of one step (the first, a middle one, the last) and none; sizes at
+# which no term of a product leaves binary32's range; tiles of 32 tokens with k shared by wavefronts, of 64, and of 128 rows
+@pytest.mark.parametrize("tokens,rows", [(5, 300), (70, 300), (300, 8200)])
+@pytest.mark.parametrize("wide", ["none", "first", "middle", "last", "one", "all"])
+@pytest.mark.parametrize("scale", [1.0, 2.0 ** -90, 2.0 ** 100])
+def test_binary32_products_of_weights_in_either_format(awq, lib, dev, tokens, rows, wide, scale):
+    print("binary32 weights", tokens, rows, wide, scale, flush=True)
+    k = 576
+    rng = np.random.default_rng(rows)
+    fine = (rng.standard_normal((rows, k)) / k ** 0.5).astype(np.float32)
+    w = km.bf16(fine)
+    steps = {"none": [], "first": [0], "middle": [7], "last": [17], "one": [7], "all": range(18)}[wide]
+    for i in steps:
+        w[:, 32 * i:32 * i + 32] = fine[:, 32 * i:32 * i + 32]
+    if wide == "one":
+        w = km.bf16(fine)
+        w[rows - 2, 230] = fine[rows - 2, 230]
+    block = dev.torch.zeros((rows + 255) // 256 * 256 * k, dtype=dev.torch.float32, device="cuda")
+    d = dev.f(w)
+    awq.check(lib.awq_dense_pack(d.data_ptr(), 1, rows, k, block.data_ptr(), k, 0, 0, 1, dev.stream))
+    x = (rng.standard_normal((tokens, k)) * scale).astype(np.float32)
+    for floats in (0, 1 << 22):
+        ws, y = dev.empty((1 << 22,), True), dev.empty((tokens, rows), True)
+
+        def run():
+            a = awq.AwqDenseArgs()
+            xd = dev.f(x)
+            a.w, a.k, a.tokens, a.n_segments, a.out = block.data_ptr(), k, tokens, 1, awq.DENSE_F32
+            a.segment[0] = awq.AwqDenseSegment(xd.data_ptr(), y.data_ptr(), k, rows, 0, rows, 0, 0, 0, 0)
+            a.workspace, a.workspace_floats = (ws.data_ptr() if floats else None), floats
+            awq.check(lib.awq_dense(ctypes.byref(a), 1, dev.stream))
+            return dev.host(y).astype(np.float64)
+        want = x.astype(np.float64) @ w.T.astype(np.float64)
+        # 36 sums of 16 products: 36 roundings of 2^-24 of partial sums, which are below 6 (2.5 million outputs of rms 1) and, in the
+        # mean square over all, sqrt(i / 36) behind the i-th: 2^-24 sqrt(18).  A term left out is 2^-17 of its product.
+        before = run()
+        assert np.abs(before - want).max() < 36 * 6 * 2.0 ** -24 * scale
+        assert np.sqrt(np.mean((before - want) ** 2)) < 18 ** 0.5 * 2.0 ** -24 * scale
+        # what is not finite stays with its token (the others have the bits they had), and is what products and sums of binary32 make of it
+        keep = x.copy()
+        x[1, 3], x[2, 100], x[2, 101], x[3, 575], x[4, 40] = np.inf, np.inf, -np.inf, np.nan, -np.inf
+        with np.errstate(invalid="ignore"):
+            want = x.astype(np.float64) @ w.T.astype(np.float64)
+        got = run()
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.sign(got[1]), np.sign(want[1])) and np.isinf(got[[1, 4]]).all()
+        rest = [t for t in range(tokens) if not 1 <= t <= 4]
+        assert np.array_equal(got[rest], before[rest])
+        x = keep
+
+
 @pytest.mark.parametrize("k", [64, 192, 320, 448, 1024, 1088, 1152, 1536, 1792, 2048, 2112, 2560, 3072, 3584, 4160, 8192, 8256, 12352])
 @pytest.mark.parametrize("rows", [1, 9, 1000, 2048, 2049])
 def test_products_of_one_token(awq, lib, dev, rows, k):
