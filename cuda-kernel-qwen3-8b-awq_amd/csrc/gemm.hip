@@ -1221,6 +1221,148 @@ __global__ __launch_bounds__(512) void gemm_shared32_kernel(GemmParams p) {
   }
 }
 
+constexpr int waitcnt_vm(int n) { return (n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14); }
+constexpr int kWaitLds = 15 | (7 << 4) | (3 << 14);  // lgkmcnt(0) alone
+// how many of a wavefront's requests are behind the ones of chunk c: `tokens` per chunk, `na` chunks ahead, ahead of `weights` per chunk, `wa` ahead
+constexpr int panel_behind(int c, int nc, int na, int wa, int tokens, int weights) {
+  int behind = 0, seen = 0;
+  const auto request = [&](int chunk, int n) {
+    if (chunk >= nc) return;
+    if (seen == 2) behind += n;
+    if (chunk == c) ++seen;
+  };
+  for (int i = 0; i < na || i < wa; ++i) {
+    if (i < na) request(i, tokens);
+    if (i < wa) request(i, weights);
+  }
+  for (int i = 0; i < c; ++i) {
+    request(i + na, tokens);
+    request(i + wa, weights);
+  }
+  return behind;
+}
+
+// 17..64 tokens: a stream of weights, beside which every workgroup reads all tokens' inputs of its k.  A workgroup of eight wavefronts takes RG
+// row groups and all of k or a share, a wavefront an eighth of that in NC chunks of 64 inputs.  A wavefront's weights and
+// the tokens' inputs that they meet are its own, so that nothing waits for another wavefront until the sums meet in LDS: the tokens
+// go straight into a ring of NS places of its own (global_load_lds, 128 bytes per token and chunk, the eight 16-byte pieces of row r at
+// positions c ^ (r / 2 & 7)), the weights into registers, requested in the order of their use NS and WA chunks ahead (up to 32 tokens two
+// and four chunks are enough, and more of them only delay the first; beyond, all weights at the start).  Lane (q, r) holds dwords
+// 2 (q % 2) and + 1 of row r of block q / 2 of the chunk (one 8-byte request) and reads the token pieces 2 q and 2 q + 1;
+// v_mfma_f32_16x16x32_f16 with the tokens as the first operand, so that 33 to 48 are three tiles and not four.  As many row groups as
+// leave one workgroup per compute unit.  Loads and nothing else take 85 to 90 % of its time.  17, 24, 40, 48, 64 tokens, us: 12,288 x 4,096 9.3, 9.5,
+// 12.0, 12.3, 14.0 (gemm_shared32_kernel, 192 workgroups: 11.0, 10.5, 14.1, 14.2, 14.4), 4,096 x 4,096 5.9, 6.1, 7.5, 7.8, 8.8
+// (gemm_shared_kernel 6.5, 6.4, 8.4, 8.5, 8.9), 4,096 x 12,288 with k over four workgroups and the launch that adds at 17, 24, 48 11.8, 12.3, 16.3 (12.9, 13.0, 16.6).
+constexpr int panel_places(int tt) { return tt == 3 ? 3 : 2; }
+template <int RG, int TT, int NC, bool ZINT>
+__global__ __launch_bounds__(512, 2) void gemm_panel_kernel(GemmParams p, int n_rg) {
+  typedef __attribute__((address_space(1))) const void* gptr_t;
+  typedef __attribute__((address_space(3))) void* lptr_t;
+  constexpr int NS = panel_places(TT), WA = TT == 2 && NC > 4 ? 4 : NC;
+  static_assert(NC >= NS, "a ring of whole chunks");
+  constexpr int kPlace = 16 * TT * 64;  // halves
+  extern __shared__ __attribute__((aligned(16))) unsigned char panel_lds[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int q = lane >> 4, r = lane & 15;
+  const int rg0 = blockIdx.x * RG;
+  half_t* const ring = reinterpret_cast<half_t*>(panel_lds) + wave * NS * kPlace;
+  const int blk0 = ((int)blockIdx.y * 8 + wave) * (2 * NC);  // of 32 inputs
+  const half_t* src[2 * TT];
+#pragma unroll
+  for (int i = 0; i < 2 * TT; ++i) {
+    const int row = 8 * i + (lane >> 3);
+    src[i] = p.x + (int64_t)min(row, p.M - 1) * p.k + blk0 * 32 + (((lane & 7) ^ ((row >> 1) & 7)) << 3);
+  }
+  auto tokens = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 2 * TT; ++i)
+      __builtin_amdgcn_global_load_lds((gptr_t)(src[i] + c * 64), (lptr_t)(ring + (c % NS) * kPlace + i * 512), 16, 0, 0);
+  };
+  half_t sc[RG], zz[RG];
+  const u32x2_t* wp[RG];
+#pragma unroll
+  for (int i = 0; i < RG; ++i) {
+    const int rg = min(rg0 + i, n_rg - 1);  // a workgroup past the last row group repeats it and stores nothing
+    const int gi = ((rg >> 3) % p.kg) % p.mg;
+    sc[i] = p.scale[gi];
+    zz[i] = p.zp[gi];
+    wp[i] = reinterpret_cast<const u32x2_t*>(p.wq + (((int64_t)rg * p.nblk + blk0 + (q >> 1)) * 16 + r) * 4 + 2 * (q & 1));
+  }
+  u32x2_t w[NC][RG];
+  auto weights = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < RG; ++i) w[c][i] = __builtin_nontemporal_load(wp[i] + c * 64);
+  };
+  float4_t acc[RG][TT];
+#pragma unroll
+  for (int i = 0; i < RG; ++i)
+#pragma unroll
+    for (int t = 0; t < TT; ++t) acc[i][t] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  static_for<(NS > WA ? NS : WA)>([&](auto C) __attribute__((always_inline)) {
+    constexpr int c = decltype(C)::value;
+    if constexpr (c < NS) tokens(c);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (c < WA) weights(c);
+    __builtin_amdgcn_sched_barrier(0);
+  });
+  static_for<NC>([&](auto C) __attribute__((always_inline)) {
+    constexpr int c = decltype(C)::value;
+    // Requests that may still be on their way when the chunk's tokens and weights are there.  (The wait has to cover the weights too:
+    // the compiler, which takes a request into LDS for one of any kind, would wait for all there are.)
+    constexpr int after = panel_behind(c, NC, NS, WA, 2 * TT, RG);
+    static_assert(after < 64, "the request counter has six bits");
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm(after));
+    asm volatile("" ::: "memory");
+    const half_t* const place = ring + (c % NS) * kPlace;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      half8_t x[TT];
+#pragma unroll
+      for (int t = 0; t < TT; ++t) x[t] = *reinterpret_cast<const half8_t*>(place + (16 * t + r) * 64 + (((2 * q + j) ^ ((r >> 1) & 7)) << 3));
+#pragma unroll
+      for (int i = 0; i < RG; ++i) {
+        const half8_t wop = dequant8<ZINT, false>(w[c][i][j], sc[i], zz[i]);
+#pragma unroll
+        for (int t = 0; t < TT; ++t) acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[t], wop, acc[i][t], 0, 0, 0);
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+    if constexpr (c + NS < NC) {
+      __builtin_amdgcn_s_waitcnt(kWaitLds);  // this place has been read
+      tokens(c + NS);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (c + WA < NC) weights(c + WA);
+    __builtin_amdgcn_sched_barrier(0);
+  });
+  __syncthreads();  // the sums take the place of the tokens
+  float* const red = reinterpret_cast<float*>(panel_lds);  // [8 wavefronts][RG][TT][64 lanes][4]
+#pragma unroll
+  for (int i = 0; i < RG; ++i)
+#pragma unroll
+    for (int t = 0; t < TT; ++t) *reinterpret_cast<float4_t*>(red + (((wave * RG + i) * TT + t) * 64 + lane) * 4) = acc[i][t];
+  __syncthreads();
+  // D[token 4 (lane / 16) + e][row lane % 16] sits in element e of the lane; a thread's rows fastest
+  with_epilogue(p, [&](auto E) {
+#pragma unroll
+    for (int idx = tid; idx < RG * TT * 256; idx += 512) {
+      const int i = (idx >> 4) % RG, row = idx & 15, token = idx / (16 * RG);
+      const int rg = rg0 + i;
+      const float* part = red + ((i * TT + (token >> 4)) * 64 + ((token >> 2) & 3) * 16 + row) * 4 + (token & 3);
+      float v = part[0];
+#pragma unroll
+      for (int wv = 1; wv < 8; ++wv) v += part[wv * (RG * TT * 256)];
+      if (token >= p.M || rg >= n_rg) continue;
+      const int gi = ((rg >> 3) % p.kg) % p.mg;
+      v *= (float)p.scale[gi];
+      if (p.kz > 1) p.part[((int64_t)blockIdx.y * p.M + token) * p.m + rg * 16 + row] = v;  // finished by launch_reduce
+      else store_out<decltype(E)::value, true>(p, token, rg * 16 + row, v);
+    }
+  });
+}
+
 // k cut over several workgroups: the chunks' FP32 partial sums are added in
 // chunk order (whatever order the workgroups ran in), then the epilogue
 __global__ __launch_bounds__(256) void reduce_parts_kernel(GemmParams p) {
@@ -1455,6 +1597,48 @@ int launch_shared32(const GemmParams& p, bool zint, hipStream_t st) {
   return AWQ_OK;
 }
 
+// 17..64 tokens where gemm_panel_kernel is the faster one (times there): row groups per workgroup, and workgroups that share k; 0: another
+// kernel takes the product.  16,384 x 4,096 where it has three tiles of tokens only (40 tokens: 14.1 us against 15.4; 64: 16.9 against
+// 15.7), 4,096 x 12,288 up to 48 tokens (64: 18.1 against 17.9).
+struct PanelForm {
+  int rg, kz;
+};
+static PanelForm panel_form(int64_t m, int64_t k, int64_t M, bool has_workspace) {
+  if (M < 17 || M > 64) return {0, 0};
+  if (k == 4096 && m == 4096) return {1, 1};
+  if (k == 4096 && m == 12288) return {3, 1};
+  if (k == 4096 && m == 16384 && M > 32 && M <= 48) return {4, 1};
+  if (k == 12288 && m == 4096 && M <= 48 && has_workspace) return {4, 4};
+  return {0, 0};
+}
+template <int RG, int TT, int NC>
+int launch_panel(const GemmParams& p, bool zint, hipStream_t st) {
+  auto kern = zint ? gemm_panel_kernel<RG, TT, NC, true> : gemm_panel_kernel<RG, TT, NC, false>;
+  constexpr int ring = 8 * panel_places(TT) * 16 * TT * 64 * 2, sums = 8 * RG * TT * 1024, lds = ring > sums ? ring : sums;
+  static_assert(lds <= 160 * 1024, "LDS of one compute unit");
+  if (lds > 65536) {
+    // more LDS than a launch gets by default: raise this kernel's limit, once per device
+    static std::atomic<uint64_t> raised[2];
+    int dev = 0;
+    AWQ_HIP_TRY(hipGetDevice(&dev));
+    const uint64_t bit = 1ull << (dev & 63);
+    if (!(raised[zint].load(std::memory_order_relaxed) & bit)) {
+      AWQ_HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+      raised[zint].fetch_or(bit, std::memory_order_relaxed);
+    }
+  }
+  const int n_rg = p.m / 16;
+  hipLaunchKernelGGL(kern, dim3((unsigned)((n_rg + RG - 1) / RG), (unsigned)p.kz), dim3(512), lds, st, p, n_rg);
+  if (p.kz > 1) launch_reduce(p, st);
+  return AWQ_OK;
+}
+template <int RG, int NC>
+int launch_panel_tokens(const GemmParams& p, bool zint, hipStream_t st) {
+  if (p.M <= 32) return launch_panel<RG, 2, NC>(p, zint, st);
+  if (p.M <= 48) return launch_panel<RG, 3, NC>(p, zint, st);
+  return launch_panel<RG, 4, NC>(p, zint, st);
+}
+
 // Which workgroup shape a many-token product takes (measured on the three matrix shapes of the
 // model, 128 to 4096 tokens):
 //   fewer than 80 tiles of 256 rows x 128 tokens          k split
@@ -1503,9 +1687,11 @@ int gemm_norm_shares(int64_t m, int64_t k, int64_t M) {
 // with a tile per workgroup, 3 rows split with 64 tokens per workgroup, 4 rows split with the work cut evenly,
 // 5 up to 16 tokens with several row groups per workgroup, 6 17..64 and 129..192 tokens on 4096 rows with the tokens shared
 // through LDS, 7 17..256 tokens on 10240..16384 rows the same way with 64 rows per workgroup, 8 the same with k
-// cut over four workgroups (4096 x 12288 at 128..320 tokens)
+// cut over four workgroups (4096 x 12288 at 128..320 tokens), 9 17..48 tokens on 4096 x 12288, a wavefront's
+// operands all its own and k cut over four workgroups.  Of 6 and 7 up to 64 tokens the kernel is that of 9 where panel_form says so
 int gemm_plan(int64_t m, int64_t k, int64_t M, int has_workspace) {
   if (M >= 2 && mid_row_groups(m, k, M)) return 5;
+  if (panel_form(m, k, M, has_workspace != 0).kz > 1) return 9;
   if (shared_takes(m, k, M)) return 6;
   if (shared32_takes(m, k, M)) return 7;
   if (has_workspace && shared32_kcut_takes(m, k, M)) return 8;
@@ -1563,6 +1749,18 @@ int launch_gemm(const void* wq, const half_t* scale, const half_t* zp, int64_t m
   p.sk_head = nullptr;
   p.sk_part = nullptr;
   p.norm = norm;
+  const bool panel_room = workspace && kSkHeaderBytes + 4 * M * m * 4 <= workspace_bytes;
+  if (const PanelForm f = panel_form(m, k, M, panel_room); f.rg) {
+    p.kz = f.kz;
+    if (f.kz > 1) p.part = (float*)((char*)workspace + kSkHeaderBytes);
+    int rc;
+    if (f.kz > 1) rc = M <= 32 ? launch_panel<4, 2, 6>(p, zp_integral, st) : launch_panel<4, 3, 6>(p, zp_integral, st);
+    else if (f.rg == 4) rc = launch_panel<4, 3, 8>(p, zp_integral, st);
+    else rc = f.rg == 3 ? launch_panel_tokens<3, 8>(p, zp_integral, st) : launch_panel_tokens<1, 8>(p, zp_integral, st);
+    if (rc) return rc;
+    AWQ_HIP_TRY(hipGetLastError());
+    return AWQ_OK;
+  }
   if (shared32_kcut_takes(m, k, M) && workspace && kSkHeaderBytes + 4 * M * m * 4 <= workspace_bytes) {
     p.kz = 4;
     p.part = (float*)((char*)workspace + kSkHeaderBytes);
@@ -1580,7 +1778,7 @@ int launch_gemm(const void* wq, const half_t* scale, const half_t* zp, int64_t m
   }
   if (shared_takes(m, k, M)) {
     int rc;
-    if (k == 4096) rc = M <= 32 ? launch_shared<2, 16>(p, zp_integral, st) : launch_shared<4, 16>(p, zp_integral, st);
+    if (k == 4096) rc = launch_shared<4, 16>(p, zp_integral, st);
     else rc = M <= 32 ? launch_shared<2, 8>(p, zp_integral, st) : launch_shared<4, 8>(p, zp_integral, st);
     if (rc) return rc;
     AWQ_HIP_TRY(hipGetLastError());

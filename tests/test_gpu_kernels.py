@@ -794,6 +794,35 @@ def test_gemm_matches_fp32_accumulate_reference(awq, lib, oracle, torch_gpu, m, 
     assert p99a <= 2.0 ** -10 and p99b <= 2.0 ** -10
 
 
+# one, two, three and four tiles of 16 tokens filled by one token and to the last, a third of a tile of rows past the last row group; k over
+# four workgroups with room for their sums and without
+@pytest.mark.parametrize("M", [17, 31, 32, 33, 47, 48, 49, 64])
+@pytest.mark.parametrize("m,k", [(4096, 4096), (12288, 4096), (16384, 4096), (4096, 12288)])
+def test_gemm_of_17_to_64_tokens(awq, lib, torch_gpu, m, k, M):
+    torch = torch_gpu
+    rng = np.random.default_rng(m + k + M)
+    zp_int = M % 2 == 0
+    packed, scale, zp = rand_awq(rng, m, k, zp_int=zp_int)
+    d_in, d_s, d_z = dev(torch, packed), dev(torch, scale), dev(torch, zp)
+    d_dq = torch.zeros(m * k, dtype=torch.float16, device="cuda")
+    awq.check(lib.awq_dequant(d_in.data_ptr(), d_s.data_ptr(), d_z.data_ptr(), d_dq.data_ptr(), m, k, m // 128, stream(torch)))
+    d_w = torch.zeros(m * k // 2, dtype=torch.uint8, device="cuda")
+    awq.check(lib.awq_linear_repack(d_in.data_ptr(), d_w.data_ptr(), m, k, stream(torch)))
+    d_x = torch.from_numpy(rng.standard_normal((M, k)).astype(np.float16)).cuda()
+    want = (d_x.float() @ d_dq.view(k, m).float()).double()
+    rms = float(want.square().mean().sqrt())
+    print("gemm", m, k, M, flush=True)
+    d_ws = torch.zeros(4096 + 16 * M * m, dtype=torch.uint8, device="cuda")
+    for ws in (None, d_ws.data_ptr()):
+        d_y = torch.full((M + 1, m), float("nan"), dtype=torch.float16, device="cuda")
+        awq.check(lib.awq_gemm(d_w.data_ptr(), d_s.data_ptr(), d_z.data_ptr(), m, k, d_x.data_ptr(), d_y.data_ptr(), M, int(zp_int), ws, stream(torch)))
+        got = d_y.double()
+        assert bool(torch.isnan(got[M]).all())
+        # a rounding of the output to binary16 (2^-11) and of every weight of the reference (2^-11 each, as many signs: of the rms)
+        assert bool(((got[:M] - want).abs() <= 2.0 ** -11 * want.abs() + 6 * 2.0 ** -11 * rms).all())
+        assert int(d_ws[:4096].to(torch.int32).sum().item()) == 0
+
+
 def _random_gemm_shapes(n, seed):
     """(m, k, M): multiples of 128 / 512 whose scale group does not depend on the input index"""
     rng = np.random.default_rng(seed)
