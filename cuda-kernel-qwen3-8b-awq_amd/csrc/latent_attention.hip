@@ -1,10 +1,12 @@
 // Attention over a shared latent (layers.hpp): keys and values of all heads are linear images of one cached vector per
 // position, beside a rotated key part that the heads share; softmax with a learned score that has no key.
+#include "lane_sums.hpp"
 #include "query_attention.hpp"
 
 namespace {
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef float q4u_t __attribute__((ext_vector_type(4), aligned(4)));
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef short short4_t __attribute__((ext_vector_type(4)));
 constexpr float kLog2e = 1.44269504088896340736f;
@@ -177,6 +179,188 @@ __global__ __launch_bounds__(256) void latent_query_kernel(LatentAttnArgs a, int
       });
   for (int i = 0; i < QN && t0 + i < M; ++i)  // what pads the value product's inputs
     for (int d = rank + tid; d < kv_in; d += 256) reinterpret_cast<T*>(a.ol)[((int64_t)(t0 + i) * a.heads + h) * kv_in + d] = (T)0.0f;
+}
+
+// --- in the latent space, one query in binary32 ------------------------------------------------------------------
+// The three launches of a token as in bfloat16.  Bound by the trips to memory one behind the other, so everything of a launch is requested at
+// once.  Tudasun of width 1,024 at 48 to 72 positions: queries, rotation, cache row 4.2 us, W_uk 4.4, all keys of a head in one workgroup 9.6
+// and W_uv 3.4; now 4.6,
+// 4.5 and 4.2 (keys in shares, each row read once).
+constexpr int kOneKeys = 16, kOneParts = 64;
+
+__host__ __device__ inline int one_blocks_per_part(int keys, int parts, int* blocks) {
+  *blocks = (keys + kOneKeys - 1) / kOneKeys;
+  return (*blocks + parts - 1) / parts;
+}
+
+// blockIdx.x: head, blockIdx.y: 64 of its latent entries, 16 a wavefront, two rows of W_uk at a time; rotation and cache row as in
+// latent_query_one_kernel.  `kq`: padded inputs of a row.
+__global__ __launch_bounds__(256) void latent_query_one_f32_kernel(LatentAttnArgs a, int kq, int64_t w_block, int chunks) {
+  extern __shared__ float turn[];
+  __shared__ float sums[4];
+  const int h = blockIdx.x, part = blockIdx.y, pos = a.pos.position();
+  if (part == chunks) {
+    if (h != 0) return;
+    turns_of(a, pos, turn);
+    append_row<float>(a, 0, pos, turn, sums);
+    return;
+  }
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int row0 = part * 64 + wave * 16 + (lane >> 5), rank = a.l.rank;
+  float* const q = reinterpret_cast<float*>(a.q) + (int64_t)h * (a.dim + a.l.rot);
+  float* const ql = reinterpret_cast<float*>(a.ql) + (int64_t)h * a.l.row();
+  const float* const w = reinterpret_cast<const float*>(a.w_uk) + h * w_block;
+  float acc[8] = {};
+  for (int at = 4 * (lane & 31); at < a.dim; at += 128) {  // (a multiple of 4)
+    f32x4_t wv[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) wv[i] = *reinterpret_cast<const f32x4_t*>(w + (int64_t)min(row0 + 2 * i, rank - 1) * kq + at);
+    const q4u_t x = *reinterpret_cast<const q4u_t*>(q + at);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[i] = __builtin_fmaf(wv[i][e], x[e], acc[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) acc[i] = lanes::sum<32>(acc[i]);
+#pragma unroll
+  for (int i = 0; i < 8; ++i)
+    if ((lane & 31) == i && row0 + 2 * i < rank) ql[row0 + 2 * i] = acc[i];
+  if (part == 0) {
+    turns_of(a, pos, turn);
+    rotate_queries<float, true>(a, q, ql, 1, turn);
+  }
+}
+
+// blockIdx.x: head, blockIdx.y: a share of its keys.  Sixteen lanes hold a key's row, NQ pieces of four values each, as key and as
+// value, and go on with every sixteenth key with a maximum and a sum of their own; the sixteen meet in LDS at the end.  A part is
+// [maximum, sum, -, -, columns].
+template <int NQ>
+__global__ __launch_bounds__(256) void latent_one_parts_kernel(LatentAttnArgs a) {
+  extern __shared__ __attribute__((aligned(16))) float held[];  // [16][rank padded]
+  __shared__ float gm[16], gl[16];
+  const int h = blockIdx.x, part = blockIdx.y, parts = gridDim.y, tid = threadIdx.x, sub = tid & 15, group = tid >> 4;
+  const int row = a.l.row(), rp = a.l.rank_padded(), keys = a.pos.position() + 1;
+  int blocks;
+  const int per = one_blocks_per_part(keys, parts, &blocks), first = part * per, last = min(first + per, blocks);
+  if (first >= last) return;
+  const float* const cache = reinterpret_cast<const float*>(a.cache);
+  const float* const ql = reinterpret_cast<const float*>(a.ql) + (int64_t)h * row;
+  f32x4_t q[NQ], acc[NQ];
+#pragma unroll
+  for (int i = 0; i < NQ; ++i) {
+    const int c = 4 * (sub + 16 * i);
+    q[i] = c < row ? *reinterpret_cast<const f32x4_t*>(ql + c) : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    acc[i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+  float m = -INFINITY, l = 0.0f;
+  for (int b = first; b < last; ++b) {
+    const int key = b * kOneKeys + group;
+    const float* const from = cache + (int64_t)min(key, keys - 1) * row;
+    f32x4_t k[NQ];
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+      const int c = 4 * (sub + 16 * i);
+      k[i] = c < row ? *reinterpret_cast<const f32x4_t*>(from + c) : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+    float dot = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NQ; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) dot = __builtin_fmaf(q[i][e], k[i][e], dot);
+    const float s = lanes::sum<16>(dot) * a.scale;
+    if (key >= keys) continue;
+    const float now = fmaxf(m, s);
+    const float p = s > -INFINITY || s != s ? expf(s - now) : 0.0f, alpha = m > -INFINITY ? expf(m - now) : 0.0f;
+#pragma unroll
+    for (int i = 0; i < NQ; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[i][e] = __builtin_fmaf(p, k[i][e], acc[i][e] * alpha);
+    l = __builtin_fmaf(l, alpha, p);
+    m = now;
+  }
+  if (sub == 0) gm[group] = m, gl[group] = l;
+  __syncthreads();
+  float all = gm[0], sum = 0.0f;
+#pragma unroll
+  for (int g = 1; g < 16; ++g) all = fmaxf(all, gm[g]);
+  const auto factor = [&](float x) { return x > -INFINITY ? expf(x - all) : 0.0f; };
+#pragma unroll
+  for (int g = 0; g < 16; ++g) sum = __builtin_fmaf(factor(gm[g]), gl[g], sum);
+  const float mine = factor(m);
+#pragma unroll
+  for (int i = 0; i < NQ; ++i) {
+    const int c = 4 * (sub + 16 * i);
+    if (c < rp) *reinterpret_cast<f32x4_t*>(held + group * rp + c) = acc[i] * mine;
+  }
+  __syncthreads();
+  float* const out = a.parts + ((int64_t)h * parts + part) * (rp + 4);
+  for (int c = 4 * tid; c < rp; c += 1024) {
+    f32x4_t v = *reinterpret_cast<const f32x4_t*>(held + c);
+#pragma unroll
+    for (int g = 1; g < 16; ++g) v = v + *reinterpret_cast<const f32x4_t*>(held + g * rp + c);
+    *reinterpret_cast<f32x4_t*>(out + 4 + c) = v;
+  }
+  if (tid == 0) out[0] = all, out[1] = sum;
+}
+
+// blockIdx.x: head, blockIdx.y: 16 of its values, four a wavefront; every workgroup combines the parts and the sink for itself while its weights
+// are on their way.  `kv_in`: padded inputs of a row of W_uv, at most 1,024.
+__global__ __launch_bounds__(256) void latent_value_one_f32_kernel(LatentAttnArgs a, int parts, int kv_in, int64_t w_block) {
+  __shared__ __attribute__((aligned(16))) float ol[kMaxCols];
+  __shared__ float scale[kOneParts];
+  const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int row0 = blockIdx.y * 16 + wave * 4, rank = a.l.rank, ps = a.l.rank_padded() + 4;
+  const float* const w = reinterpret_cast<const float*>(a.w_uv) + h * w_block;
+  f32x4_t wv[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int c = 4 * lane + 256 * u;
+      wv[i][u] = c < kv_in ? *reinterpret_cast<const f32x4_t*>(w + (int64_t)min(row0 + i, a.vdim - 1) * kv_in + c) : f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+  int blocks;
+  const int per = one_blocks_per_part(a.pos.position() + 1, parts, &blocks), used = (blocks + per - 1) / per;
+  const float* const p = a.parts + (int64_t)h * parts * ps;
+  const float sink = a.sink ? a.sink[h] : -INFINITY;
+  const float pm = lane < used ? p[(int64_t)lane * ps] : -INFINITY, pl = lane < used ? p[(int64_t)lane * ps + 1] : 0.0f;
+  const float m = fmaxf(sink, lanes::maximum(pm));
+  const float e = lane < used ? expf(pm - m) : 0.0f;
+  const float l = lanes::sum(e * pl) + (a.sink ? expf(sink - m) : 0.0f);
+  if (wave == 0) scale[lane] = e;
+  __syncthreads();
+  const int c = 4 * tid;
+  if (c < kv_in) {
+    f32x4_t v = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (c < rank) {
+#pragma unroll 8
+      for (int s = 0; s < used; ++s) {
+        const f32x4_t x = *reinterpret_cast<const f32x4_t*>(p + (int64_t)s * ps + 4 + c);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = __builtin_fmaf(scale[s], x[i], v[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = c + i < rank ? v[i] / l : 0.0f;
+    }
+    *reinterpret_cast<f32x4_t*>(ol + c) = v;
+  }
+  __syncthreads();
+  float acc[4] = {};
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    if (4 * lane + 256 * u >= kv_in) continue;
+    const f32x4_t x = *reinterpret_cast<const f32x4_t*>(ol + 4 * lane + 256 * u);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i] = __builtin_fmaf(wv[i][u][j], x[j], acc[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) acc[i] = lanes::sum(acc[i]);
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (lane == i && row0 + i < a.vdim) reinterpret_cast<float*>(a.ctx)[(int64_t)h * a.vdim + row0 + i] = acc[i];
 }
 
 // --- in the latent space, on the matrix cores ------------------------------------------------------------------
@@ -613,6 +797,12 @@ int64_t form_from(const LatentAttnArgs& a) {
   return std::max<int64_t>(32, (int64_t)a.l.rank * (a.dim + a.vdim) / saved);
 }
 
+// One query in binary32: rows of up to 768 values, and workgroups for two per compute unit
+bool one_in_parts(const LatentAttnArgs& a) { return a.l.row() <= 768 && a.dim % 4 == 0; }
+int one_parts_of(const LatentAttnArgs& a, int64_t keys) {
+  return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(512 / a.heads, (keys + kOneKeys - 1) / kOneKeys), kOneParts));
+}
+
 int parts_of(const LatentAttnArgs& a, int64_t M, int64_t keys) {
   const int64_t row_tiles = (M * a.heads + kRows - 1) / kRows, tiles = (keys + kKeys - 1) / kKeys;
   return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(512 / row_tiles, tiles), kMaxParts));
@@ -675,6 +865,23 @@ void launch_queries(const LatentAttnArgs& a, hipStream_t st) {
   }
 }
 
+int launch_one_f32(const LatentAttnArgs& a, hipStream_t st) {
+  const int chunks = (a.l.rank + 63) / 64, parts = one_parts_of(a, a.pos.dyn ? a.max_pos : a.pos.pos0 + 1), row = a.l.row();
+  hipLaunchKernelGGL(latent_query_one_f32_kernel, dim3((unsigned)a.heads, (unsigned)(chunks + (a.down ? 1 : 0))), dim3(256),
+                     (size_t)(a.l.rot + 2) * 4, st, a, (int)q_inputs(a), latent_uk_block(a), chunks);
+  AWQ_HIP_TRY(hipGetLastError());
+  const dim3 g((unsigned)a.heads, (unsigned)parts);
+  const size_t lds = (size_t)kOneKeys * a.l.rank_padded() * 4;  // (48 KB at most)
+  if (row <= 256) hipLaunchKernelGGL(latent_one_parts_kernel<4>, g, dim3(256), lds, st, a);
+  else if (row <= 576) hipLaunchKernelGGL(latent_one_parts_kernel<9>, g, dim3(256), lds, st, a);
+  else hipLaunchKernelGGL(latent_one_parts_kernel<12>, g, dim3(256), lds, st, a);
+  AWQ_HIP_TRY(hipGetLastError());
+  hipLaunchKernelGGL(latent_value_one_f32_kernel, dim3((unsigned)a.heads, (unsigned)((a.vdim + 15) / 16)), dim3(256), 0, st, a, parts,
+                     (int)v_inputs(a), latent_uv_block(a));
+  AWQ_HIP_TRY(hipGetLastError());
+  return AWQ_OK;
+}
+
 }  // namespace
 
 int64_t latent_uk_block(const LatentAttnArgs& a) { return round_up(a.l.rank, kDenseRowAlign) * q_inputs(a); }
@@ -694,6 +901,7 @@ LatentScratch latent_scratch(const LatentAttnArgs& a, int64_t max_tokens, bool f
   s.ql = M * a.heads * a.l.row() * unit;
   s.ol = M * a.heads * v_inputs(a) * unit;
   if (form) s.kv = a.max_pos * a.heads * (a.dim + a.vdim) * unit;
+  if (f32 && one_in_parts(a)) s.parts = (int64_t)a.heads * one_parts_of(a, a.max_pos) * (a.l.rank_padded() + 4) * 4;
   if (on_matrix_cores(a, f32)) s.parts = std::max<int64_t>(512 * kRows, M * a.heads) * (a.l.rank_padded() + 4) * 4;
   return s;
 }
@@ -750,6 +958,7 @@ int launch_latent_attention(const LatentAttnArgs& a, bool f32, hipStream_t st) {
     return AWQ_OK;
   }
   const bool cores = on_matrix_cores(a, f32);
+  if (f32 && a.M == 1 && a.parts && one_in_parts(a)) return launch_one_f32(a, st);
   if (a.M == 1 && cores && a.dim % kDenseKAlign == 0 && ((a.dim + a.l.rot) & 7) == 0 && ((uintptr_t)a.q & 15) == 0) {
     const int chunks = (a.l.rank + 63) / 64;
     hipLaunchKernelGGL(latent_query_one_kernel, dim3((unsigned)a.heads, (unsigned)(chunks + (a.down ? 1 : 0))), dim3(256),

@@ -536,6 +536,32 @@ def test_latent_attention(awq, lib, dev, f32, shape):
         assert km.rms_error(got, want) < (3e-5 if f32 else 0.03), sizes
 
 
+# one query in binary32: keys in shares of one and of several blocks (90 heads leave five shares), where there is no place for shares, and sizes
+# that have no such form (heads of 22, rows of more than 768)
+@pytest.mark.parametrize("shape,parts", [((90, 8, 6, 4, 40), True), ((600, 4, 2, 4, 8), True), ((3, 20, 6, 12, 37), False), ((3, 22, 6, 12, 37), True),
+                                         ((2, 20, 6, 12, 800), True)], ids=str)
+def test_single_queries_in_binary32(awq, lib, dev, shape, parts):
+    heads, dim, rot, vdim, rank = shape
+    print("latent attention, one query", shape, parts, flush=True)
+    rng = np.random.default_rng(rank)
+    T, eps, base, scale = 180, 1e-3, 300.0, 2.5 * (dim + rot) ** -0.5
+    q = km.bf16(rng.standard_normal((T, heads * (dim + rot))))
+    down = rng.standard_normal((T, rank + rot)).astype(np.float32)
+    norm, sink = 1 + 0.3 * rng.standard_normal(rank), 2 * rng.standard_normal(heads)
+    uk, uv = (km.bf16(rng.standard_normal((heads * n, rank)) / rank ** 0.5) for n in (dim, vdim))
+    c = plain.rms(down[:, :rank].astype(np.float64), eps) * norm.astype(np.float32)
+    qh = q.reshape(T, heads, dim + rot).astype(np.float64)
+    want = plain.latent_attention(qh[:, :, :dim], plain.rotate(qh[:, :, dim:], 0, base), c, plain.rotate(down[:, rank:].astype(np.float64), 0, base),
+                                  uk.reshape(heads, dim, rank), uv.reshape(heads, vdim, rank), scale, sink)
+    layer = Latent(awq, lib, dev, 1, heads, dim, rot, vdim, rank, uk, uv, norm, sink, scale, eps, base, T, T)
+    if not parts:
+        layer.a.parts = None
+    layer.run(q, down, 0)
+    for t in (0, 1, 15, 16, 17, 78, 79, 80, 81, 159, 160, 179):
+        got = layer.run(q[t:t + 1], down[t:t + 1], t)
+        assert km.rms_error(got, want[t:t + 1]) < 3e-5, t
+
+
 @pytest.mark.parametrize("shape", [(3, 20, 6, 12, 37), (5, 20, 6, 12, 37), (2, 64, 32, 64, 128), (9, 64, 32, 64, 128)], ids=str)
 def test_latents_that_a_query_does_not_see(awq, lib, dev, shape):
     """several queries share a reading of the rows in binary32; the rows behind a query's own may hold anything"""
