@@ -182,7 +182,7 @@ int ConfigModel::open(std::unique_ptr<ConfigModel> e, const Safetensors& file, c
   return AWQ_OK;
 }
 
-int ConfigModel::logits_of(const float* x, const int32_t* which, int64_t n, bool sample) {
+int ConfigModel::logits_of(const float* x, const int32_t* which, int64_t n, bool sample, bool formed) {
   NormConvArgs a;
   a.x = x;
   a.rows = which;
@@ -193,8 +193,8 @@ int ConfigModel::logits_of(const float* x, const int32_t* which, int64_t n, bool
   a.w1 = final_norm;
   a.out1 = head_in;
   a.ld = ld;
-  const bool fused = sample && dense_norm_fused(a, f32);
-  if (!fused)
+  const bool fused = !formed && sample && dense_norm_fused(a, f32);
+  if (!fused && !formed)
     if (int rc = launch_norm_conv(a, f32, stream)) return rc;
   DenseArgs d;
   d.w = head;
@@ -219,10 +219,13 @@ int ConfigModel::logits_of(const float* x, const int32_t* which, int64_t n, bool
 int ConfigModel::enqueue_step(StepKind kind, int64_t) {
   PassPos pos;
   pos.dyn = d_state;
-  if (kind != STEP_SAMPLE)
-    if (int rc = run_pass(true, nullptr, 1, pos)) return rc;
+  head_wanted = kind == STEP_GENERATE;
+  head_formed = false;
+  const int rc = kind != STEP_SAMPLE ? run_pass(true, nullptr, 1, pos) : AWQ_OK;
+  head_wanted = false;
+  if (rc) return rc;
   if (kind == STEP_PROMPT) return AWQ_OK;
-  if (int rc = logits_of(stream_of(true), nullptr, 1, true)) return rc;
+  if (int rc2 = logits_of(stream_of(true), nullptr, 1, true, head_formed)) return rc2;
   return launch_take_best(best, dense_candidates(vocab), d_token, d_out, d_state, kind == STEP_GENERATE ? 1 : 0, stream);
 }
 

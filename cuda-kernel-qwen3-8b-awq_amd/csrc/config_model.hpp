@@ -63,6 +63,9 @@ struct ConfigModel : awq_engine {
   float* tap = nullptr;
   int64_t tap_tokens = 0;
 
+  // a step that samples behind its pass: the pass may leave the norm of its stream in head_in, and then says so
+  bool head_wanted = false, head_formed = false;
+
   // --- the model's part
   virtual int load_layers(Loader& ld) = 0;
   virtual int make_buffers() = 0;  // activations, caches, recurrent state
@@ -94,7 +97,8 @@ struct ConfigModel : awq_engine {
   int zeroed(void** p, int64_t bytes);
   // a pass calls it behind layer run `run`; the pass's last call ends it
   int tap_layer(int64_t run, const float* x, int64_t M);
-  int logits_of(const float* x, const int32_t* which, int64_t n, bool sample);
+  // `formed`: the norm of x is in head_in already
+  int logits_of(const float* x, const int32_t* which, int64_t n, bool sample, bool formed = false);
   // weights, buffers and driver behind a checked folder; `e` stays the caller's when it fails
   static int open(std::unique_ptr<ConfigModel> e, const Safetensors& file, const awq_open_options& opt, awq_engine** out);
 };

@@ -350,8 +350,17 @@ int launch_route(const RouteArgs& a, hipStream_t st);
 // --- around a sublayer (sublayer_ops.hip) --------------------------------------------------------------------------
 // x[t] = table[token] (float), side[t] = side_table[token] (both tables in the activations' type); the one token of
 // pos.dyn as in launch_embed_sinusoid
+// norm (where embed_takes_norm): h[t] = RMS norm of x[t] times w, in the activations' type
+struct EmbedNorm {
+  const float* w = nullptr;  // [width]
+  float eps = 0.0f;
+  void* h = nullptr;  // [M][ldh]
+  int64_t ldh = 0;
+};
 int launch_embed_tokens(const void* table, const void* side_table, bool f32, const int32_t* tokens, const int32_t* last,
-                        PassPos pos, int64_t M, int64_t width, int64_t side_width, float* x, void* side, hipStream_t st);
+                        PassPos pos, int64_t M, int64_t width, int64_t side_width, float* x, void* side, hipStream_t st,
+                        const EmbedNorm* norm = nullptr);
+bool embed_takes_norm(int64_t width, int64_t side_width, const EmbedNorm& n);
 // What ends a sublayer: x += RMS norm(y * gate) * w_post, then out = RMS norm(x) * w_next.
 struct JoinArgs {
   float* x = nullptr;         // [M][width]

@@ -800,8 +800,11 @@ int TudasunEngine::token_input(int i, Buffers& b, int64_t M, JoinArgs* end) {
 int TudasunEngine::run_pass(bool one, const int32_t* ids, int64_t M, PassPos pos) {
   Buffers& b = one ? step : pass;
   const int n = (int)layers.size();
-  if (int rc = launch_embed_tokens(embed, side_embed, f32, ids, d_token, pos, M, width, side_width(), b.x, b.side, stream)) return rc;
-  {
+  const EmbedNorm first{layers[0].norm1, eps, b.h, ld};
+  const bool normed = embed_takes_norm(width, side_width(), first);
+  if (int rc = launch_embed_tokens(embed, side_embed, f32, ids, d_token, pos, M, width, side_width(), b.x, b.side, stream, normed ? &first : nullptr))
+    return rc;
+  if (!normed) {
     NormConvArgs a;
     a.x = b.x;
     a.M = M;
@@ -825,6 +828,11 @@ int TudasunEngine::run_pass(bool one, const int32_t* ids, int64_t M, PassPos pos
       return AWQ_OK;
     }
     e.x_out = last ? b.x : x;
+    if (last && head_wanted && !e.out) {  // the next token's logits read the norm of the stream
+      e.w_next = final_norm;
+      e.out = head_in;
+      head_formed = true;
+    }
     return launch_join(e, f32, stream);
   };
   is_waiting = false;
