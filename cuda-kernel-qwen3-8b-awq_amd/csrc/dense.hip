@@ -452,6 +452,10 @@ int launch_many(const DenseArgs& a, int64_t rows, hipStream_t st) {
   if (c.cuts > 1) {
     launch_form<DENSE_PART, false>(a, *form, rows, tok_tiles, c.cuts, st);
     AWQ_HIP_TRY(hipGetLastError());
+    if (OUT == DENSE_F32 && a.shares) {
+      *a.shares = c.cuts;
+      return AWQ_OK;
+    }
     hipLaunchKernelGGL((dense_parts_kernel<bf16_t, OUT>), dim3((unsigned)((rows / 4 + 255) / 256), (unsigned)a.M), dim3(256), 0, st, a,
                        (int)rows, (int)c.cuts);
   } else {
@@ -537,7 +541,7 @@ bool dense_norm_fused(const NormConvArgs& n, bool f32) {
 // and 6.76, 2,048 8.00, 7.98, 7.56 and 7.67, 2,816 10.4, 10.4, 10.3 and 10.9; 4,096, 64 after 128, 37.2, 37.2, 37.0 and 39.7; width
 // 1,024 in binary32 6.97, 7.08, 6.84 and 6.98.
 bool dense_join_fused(const JoinArgs& j, int64_t rows, bool f32) {
-  return j.M == 1 && j.out && j.x_out && j.x_out != j.x && (j.top == 0 || j.out != j.h) && j.top <= kJoinTop && j.width <= (f32 ? 2048 : 4096) &&
+  return j.M == 1 && j.y_shares == 1 && j.out && j.x_out && j.x_out != j.x && (j.top == 0 || j.out != j.h) && j.top <= kJoinTop && j.width <= (f32 ? 2048 : 4096) &&
          ((j.width | j.ldo | j.ldg | j.ldh) & 3) == 0 && j.ldo % kDenseKAlign == 0 && rows * j.width <= 16 << 20;
 }
 
@@ -598,6 +602,8 @@ int launch_dense(const DenseArgs& args, bool f32, hipStream_t st, const NormConv
     return f32 ? launch_dense_many_f32(a, rows, st) : launch_listed(a, rows, st);
   }
   AWQ_REQUIRE(a.out >= DENSE_STORE && a.out <= DENSE_ARGMAX, "unknown output");
+  AWQ_REQUIRE(!a.shares || (a.out == DENSE_F32 && a.n_seg == 1 && last.act == DENSE_NONE), "the shares of this product cannot be left");
+  if (a.shares) *a.shares = 1;
   AWQ_REQUIRE(a.out != DENSE_ARGMAX || (a.M == 1 && a.best), "sampling takes one token");
   if (norm) {
     AWQ_REQUIRE(dense_norm_fused(*norm, f32) && a.M == 1 && a.k == norm->ld && a.batch == 1 && !a.gate_o && a.n_seg <= (norm->w2 ? 2 : 1) &&

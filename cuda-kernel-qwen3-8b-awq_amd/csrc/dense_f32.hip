@@ -389,6 +389,10 @@ int launch_many(const DenseArgs& a, int64_t rows, hipStream_t st) {
   AWQ_REQUIRE(tiles < (1ll << 26), "too large");
   if (cuts == 1) return launch_tiles<OUT, false>(a, rows, form, (int)tok_tiles, 1, st);
   if (int rc = launch_tiles<DENSE_PART, false>(a, rows, form, (int)tok_tiles, (int)cuts, st)) return rc;
+  if (OUT == DENSE_F32 && a.shares) {
+    *a.shares = (int32_t)cuts;
+    return AWQ_OK;
+  }
   hipLaunchKernelGGL((dense_parts_kernel<float, OUT>), dim3((unsigned)((rows / 4 + 255) / 256), (unsigned)a.M), dim3(256), 0, st, a,
                      (int)rows, (int)cuts);
   AWQ_HIP_TRY(hipGetLastError());

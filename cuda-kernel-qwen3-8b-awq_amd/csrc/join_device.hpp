@@ -42,6 +42,28 @@ __device__ __forceinline__ float group_sum(float v, float* sums) {
   return lanes::sum<16>((lane & 15) < waves ? sums[lane & 15] : 0.0f);
 }
 
+// y of token t from column c on, its shares in order, four requested at a time
+template <int V>
+__device__ __forceinline__ void read_y(const JoinArgs& a, int64_t t, int c, float (&v)[V]) {
+  if (a.y_shares == 1) {
+    read<float, V>(a.y + t * a.width + c, v);
+    return;
+  }
+  const float* const y = a.y + t * a.ldy + c;
+  for (int s = 0; s < a.y_shares; s += 4) {
+    float u[4][V];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (s + i < a.y_shares) read<float, V>(y + (s + i) * a.y_share, u[i]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (s + i < a.y_shares) {
+#pragma unroll
+        for (int e = 0; e < V; ++e) v[e] = s + i == 0 ? u[i][e] : v[e] + u[i][e];
+      }
+  }
+}
+
 // Choices of a token that wait in registers.
 constexpr int kJoinTop = 8;
 
@@ -63,7 +85,7 @@ struct JoinRow {
 #pragma unroll
       for (int i = 0; i < V; ++i) v[q][i] = g[q][i] = r[q][i] = h[q][i] = 0.0f;
       if (c >= W) continue;
-      if (a.y) read<float, V>(a.y + t * W + c, v[q]);
+      if (a.y) read_y<V>(a, t, c, v[q]);
       if (a.gate) read<T, V>(reinterpret_cast<const T*>(a.gate) + t * a.ldg + c, g[q]);
       read<float, V>(a.x + t * W + c, r[q]);
       if (a.top > 0) read<T, V>(reinterpret_cast<const T*>(a.h) + t * a.ldh + c, h[q]);

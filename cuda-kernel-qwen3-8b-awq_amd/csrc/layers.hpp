@@ -97,6 +97,9 @@ struct DenseArgs {
   float gate_eps = 0.0f;
   float* workspace = nullptr;          // sums of products that are cut along k; may be null
   int64_t workspace_floats = 0;
+  // host, DENSE_F32 of one segment without activation: receives in how many shares k was cut; where more than one, their sums stay in the workspace,
+  // [share][token][rows padded], for a launch that adds them (JoinArgs), and y is not written
+  int32_t* shares = nullptr;
   // Several products in one launch (DENSE_STORE): product b has its weight block w_batch elements (rows padded times k)
   // behind the one ahead, its input x_batch and its output y_batch elements.  ids (device, one token only): product b
   // takes weight block ids[b], and is left out where that is not below n_groups.
@@ -368,6 +371,9 @@ struct JoinArgs {
   int64_t M = 0, width = 0;
   float eps = 0.0f;
   const float* y = nullptr;   // [M][width], or null
+  // more than one (where join_adds_shares): y is the sum of as many arrays, added in order, y_share floats apart, of rows of ldy
+  int32_t y_shares = 1;
+  int64_t y_share = 0, ldy = 0;
   // y is to be multiplied by sigmoid(y_gate[t]) (null: by 1), and the experts' outputs are added to it: sum over j < top
   // of weights[t][j] * (ids[t][j] < experts ? pairs[t * top + j] : h[t])
   const float* y_gate = nullptr;
@@ -385,5 +391,6 @@ struct JoinArgs {
   int64_t ldo = 0;
 };
 int launch_join(const JoinArgs& a, bool f32, hipStream_t st);
+bool join_adds_shares(const JoinArgs& a);
 // z <- a N(z) + b N(z^2) + c N(z^3) + e with N the division of a token's n values by their root mean square; [M][ld]
 int launch_polynorm(void* z, int64_t ld, int64_t n, int64_t M, const float* abce, float eps, bool f32, hipStream_t st);

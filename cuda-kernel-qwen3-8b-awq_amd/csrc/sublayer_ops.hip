@@ -224,6 +224,12 @@ void embed_tokens(const void* table, const void* side_table, const int32_t* toke
                        side_width, x, (T*)side);
 }
 
+// a row of a token is one turn of its workgroup's threads
+bool row_form(const JoinArgs& a) {
+  const int64_t threads = a.M < 512 ? 1024 : 256;
+  return ((a.width | a.ldo | a.ldg | a.ldh) & 3) == 0 && a.width / 4 <= threads && a.top <= kJoinTop;
+}
+
 template <typename T>
 int join(const JoinArgs& a, hipStream_t st) {
   const size_t lds = (size_t)a.width * 4;
@@ -232,7 +238,7 @@ int join(const JoinArgs& a, hipStream_t st) {
   const int64_t items = a.width / (quads ? 4 : 1);
   const dim3 b((unsigned)std::min<int64_t>(a.M < 512 ? 1024 : 256, round_up(items, 64)));
   // by measurement above wherever the registers hold a row; wider rows, more choices and odd widths keep the general form
-  if (quads && items <= (int64_t)b.x && a.top <= kJoinTop) hipLaunchKernelGGL((join_row_kernel<T, 4>), g, b, 0, st, a);
+  if (row_form(a)) hipLaunchKernelGGL((join_row_kernel<T, 4>), g, b, 0, st, a);
   else if (quads) hipLaunchKernelGGL((join_kernel<T, 4>), g, b, lds, st, a);
   else hipLaunchKernelGGL((join_kernel<T, 1>), g, b, lds, st, a);
   AWQ_HIP_TRY(hipGetLastError());
@@ -278,8 +284,13 @@ int launch_embed_tokens(const void* table, const void* side_table, bool f32, con
   return AWQ_OK;
 }
 
+// Where the row waits in registers.  Tudasun of width 2,048, 129 tokens: eight launches of 4.3 us less, 884 -> 843 us; at 1,024 tokens of width
+// 4,096, whose join makes three trips as it is, one product is cut, and its shares in the join cost what the launch had.
+bool join_adds_shares(const JoinArgs& a) { return row_form(a); }
+
 int launch_join(const JoinArgs& a, bool f32, hipStream_t st) {
   AWQ_REQUIRE(a.x && a.w_post && (a.y || a.top > 0) && a.M >= 1 && a.M < (1ll << 31), "bad arguments");
+  AWQ_REQUIRE(a.y_shares == 1 || (a.y_shares > 1 && a.y && join_adds_shares(a) && a.ldy >= a.width && ((a.ldy | a.y_share) & 3) == 0), "bad shares");
   AWQ_REQUIRE(a.width >= 1 && a.width <= 16000, "width must be at most 16000");  // a row in 64 KB of LDS, sums beside it
   AWQ_REQUIRE(a.top == 0 || (a.pairs && a.ids && a.weights && a.h && a.ldh >= a.width), "bad experts");
   AWQ_REQUIRE((!a.out || a.ldo >= a.width) && (!a.gate || a.ldg >= a.width), "bad shape");

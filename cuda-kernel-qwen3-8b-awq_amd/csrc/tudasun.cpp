@@ -309,7 +309,8 @@ struct TudasunEngine final : ConfigModel {
   // the parts of a layer
   DenseArgs product(const void* w, int64_t k, int64_t M) const;
   int mix(int i, Buffers& b, int64_t M, PassPos pos);
-  int dense_feed_forward(int i, Buffers& b, int64_t M);
+  int product_ahead_of(JoinArgs* end, DenseArgs* a, const void* x, int64_t ldx, float* y);
+  int dense_feed_forward(int i, Buffers& b, int64_t M, JoinArgs* end);
   int routed_feed_forward(int i, Buffers& b, int64_t M, JoinArgs* end);
   int token_input(int i, Buffers& b, int64_t M, JoinArgs* end);
 };
@@ -581,6 +582,24 @@ DenseSegment& segment(DenseArgs* a, const void* x, int64_t ldx, void* y, int64_t
   return s;
 }
 
+// a product whose binary32 output, y [tokens][width], only the end of the sublayer reads (all but its first operand is known): shares of k
+// are added there
+int TudasunEngine::product_ahead_of(JoinArgs* end, DenseArgs* a, const void* x, int64_t ldx, float* y) {
+  int32_t shares = 1;
+  a->out = DENSE_F32;
+  if (join_adds_shares(*end)) a->shares = &shares;
+  segment(a, x, ldx, y, width, 0, width);
+  if (int rc = launch_dense(*a, f32, stream)) return rc;
+  end->y = y;
+  if (shares > 1) {
+    end->y = dense_ws;
+    end->y_shares = shares;
+    end->ldy = round_up(width, kDenseRowAlign);
+    end->y_share = a->M * end->ldy;
+  }
+  return AWQ_OK;
+}
+
 int TudasunEngine::mix(int i, Buffers& b, int64_t M, PassPos pos) {
   const LayerSpec& s = spec.layers[i];
   const LayerDev& L = layers[i];
@@ -675,7 +694,7 @@ int TudasunEngine::mix(int i, Buffers& b, int64_t M, PassPos pos) {
   return launch_head_norm(b.o, gate, L.ldp, L.mix_norm, b.ctx, L.mixed_k, s.heads, s.vdim, M, eps, f32, stream);
 }
 
-int TudasunEngine::dense_feed_forward(int i, Buffers& b, int64_t M) {
+int TudasunEngine::dense_feed_forward(int i, Buffers& b, int64_t M, JoinArgs* end) {
   const LayerSpec& s = spec.layers[i];
   const LayerDev& L = layers[i];
   {
@@ -688,9 +707,7 @@ int TudasunEngine::dense_feed_forward(int i, Buffers& b, int64_t M) {
   }
   if (int rc = launch_polynorm(b.mid, L.ff_k, s.ff, M, L.act, eps, f32, stream)) return rc;
   DenseArgs a = product(L.w_down, L.ff_k, M);
-  a.out = DENSE_F32;
-  segment(&a, b.mid, L.ff_k, b.y, width, 0, width);
-  return launch_dense(a, f32, stream);
+  return product_ahead_of(end, &a, b.mid, L.ff_k, b.y);
 }
 
 int TudasunEngine::routed_feed_forward(int i, Buffers& b, int64_t M, JoinArgs* end) {
@@ -763,13 +780,6 @@ int TudasunEngine::routed_feed_forward(int i, Buffers& b, int64_t M, JoinArgs* e
     if (beside) down.batch += 1, down.fixed = 1;
     if (int rc = launch_dense(down, f32, stream)) return rc;
   }
-  if (s.shared_ff && !beside) {
-    DenseArgs a = product(L.w_shared_down, L.shared_k, M);
-    a.out = DENSE_F32;
-    segment(&a, b.shared_mid, L.shared_k, b.y, width, 0, width);
-    if (int rc = launch_dense(a, f32, stream)) return rc;
-  }
-  end->y = s.shared_ff ? shared_y : nullptr;
   end->y_gate = s.shared_ff ? b.shared_gate : nullptr;
   end->pairs = b.pairs;
   end->ids = b.ids;
@@ -778,6 +788,11 @@ int TudasunEngine::routed_feed_forward(int i, Buffers& b, int64_t M, JoinArgs* e
   end->experts = s.experts;
   end->h = b.h;
   end->ldh = ld;
+  end->y = s.shared_ff ? shared_y : nullptr;
+  if (s.shared_ff && !beside) {
+    DenseArgs a = product(L.w_shared_down, L.shared_k, M);
+    if (int rc = product_ahead_of(end, &a, b.shared_mid, L.shared_k, b.y)) return rc;
+  }
   return AWQ_OK;
 }
 
@@ -790,11 +805,8 @@ int TudasunEngine::token_input(int i, Buffers& b, int64_t M, JoinArgs* end) {
   g.ldmul = side_width();
   if (int rc = launch_dense(a, f32, stream, nullptr, take_waiting())) return rc;
   DenseArgs p = product(L.w_side_proj, side_k, M);
-  p.out = DENSE_F32;
-  segment(&p, b.side_mid, side_k, b.y, width, 0, width);
-  end->y = b.y;
   end->w_post = L.side_norm;
-  return launch_dense(p, f32, stream);
+  return product_ahead_of(end, &p, b.side_mid, side_k, b.y);
 }
 
 int TudasunEngine::run_pass(bool one, const int32_t* ids, int64_t M, PassPos pos) {
@@ -848,6 +860,7 @@ int TudasunEngine::run_pass(bool one, const int32_t* ids, int64_t M, PassPos pos
       e.width = width;
       e.eps = eps;
       e.ldo = ld;
+      e.ldg = ldg;
       return e;
     };
     // what the next sublayer reads: x itself for the token input, the next layer's first norm, nothing behind the last
@@ -863,13 +876,9 @@ int TudasunEngine::run_pass(bool one, const int32_t* ids, int64_t M, PassPos pos
     if (int rc = mix(i, b, M, pos)) return rc;
     {
       DenseArgs a = product(L.w_o, L.mixed_k, M);
-      a.out = DENSE_F32;
-      segment(&a, b.ctx, L.mixed_k, b.y, width, 0, width);
-      if (int rc = launch_dense(a, f32, stream)) return rc;
       JoinArgs e = ending();
-      e.y = b.y;
+      if (int rc = product_ahead_of(&e, &a, b.ctx, L.mixed_k, b.y)) return rc;
       e.gate = gate_now;
-      e.ldg = ldg;
       e.w_post = L.norm1b;
       int64_t next = L.mid.rows;
       if (s.mlp != MLP_NONE) {
@@ -882,10 +891,8 @@ int TudasunEngine::run_pass(bool one, const int32_t* ids, int64_t M, PassPos pos
     }
     if (s.mlp != MLP_NONE) {
       JoinArgs e = ending();
-      e.y = b.y;
-      if (int rc = s.mlp == MLP_DENSE ? dense_feed_forward(i, b, M) : routed_feed_forward(i, b, M, &e)) return rc;
+      if (int rc = s.mlp == MLP_DENSE ? dense_feed_forward(i, b, M, &e) : routed_feed_forward(i, b, M, &e)) return rc;
       e.gate = gate_now;
-      e.ldg = ldg;
       e.w_post = L.norm2b;
       const int64_t next = leaves(&e, spec.side > 0);
       if (int rc = end_sublayer(e, next, end && !spec.side)) return rc;
