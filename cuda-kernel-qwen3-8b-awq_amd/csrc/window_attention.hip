@@ -605,6 +605,196 @@ void launch_tiles(const WindowAttnArgs& a, hipStream_t st) {
   else hipLaunchKernelGGL((window_tile_kernel<DK, 256>), g, dim3(256), 0, st, a);
 }
 
+// Many tokens, binary32, on v_mfma_f32_16x16x4_f32: sixteen queries of one head per workgroup, whose wavefronts take every eighth tile of
+// sixteen keys with a maximum and a sum of their own and meet in LDS at the end.  Operands come straight from the cache, queries as
+// columns throughout, lane (r, c) = (lane % 16, lane / 16):
+//     S^T[key][query] = K Q^T         instruction (i, e) takes element 16 i + 4 c + e of key r and of query r
+//     O^T[col][query] += V^T P^T      instruction (b, j) takes column DV / 16 r + b of key 4 c + j, whose weight the lane has just formed
+// A value is not in the sums of a query that does not see it, and a query's bits are its own: they do not depend on the queries beside
+// it, nor, without a window, on where the pass begins.
+// Bound by the matrix cores' binary32 rate and, for few queries, by the trips to the cache.  8 heads of 128, the appending launch
+// included, us, and before a few queries at a time by vector instructions (window_query_kernel): 333 queries 24 (44), 512 30 (61), of 12 heads 46 (84), 333 of 32
+// heads of 64 29 (84), 333 behind 3,000 keys in a window of 1,024 43 (105), 2 queries there 37 (39); 4 queries alone 10.0 (8.8), 64 11.6 (10.9).
+template <int DK, int DV>
+__global__ __launch_bounds__(512) void window_tile_f32_kernel(WindowAttnArgs a) {
+  constexpr int KQ = DK / 16, VB = DV / 16, NW = 8;
+  constexpr int PARTS = 16;  // of a score: chains of four or eight products, which round no more than a lane's share and a tree
+  __shared__ float most[NW][16], sums[NW][16];
+  __shared__ __attribute__((aligned(16))) float held[NW - 1][16 * DV];
+  const int h = blockIdx.x, g = h / (a.heads / a.kv_heads), tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, c = lane >> 4;
+  const int M = (int)a.M, pos0 = a.pos.pos0, q0 = blockIdx.y * 16, qi = q0 + r, qc = min(qi, M - 1), pq = pos0 + qc;
+  auto oldest = [&](int p) { return a.window > 0 ? max(0, p - a.window + 1) : 0; };
+  const int first = pos0 + q0, last = pos0 + min(q0 + 15, M - 1), lo_q = oldest(pq);
+  const int k_begin = oldest(first) & ~15, k_end = last + 1;
+  const int busy = min(NW, (k_end - k_begin + 15) >> 4);  // wavefronts that have a tile; the others are not waited for
+  if (wave >= busy) return;
+  const float* const q = reinterpret_cast<const float*>(a.proj) + (int64_t)qc * a.ldp + (int64_t)h * a.dim;
+  f32x4_t qv[KQ];
+#pragma unroll
+  for (int i = 0; i < KQ; ++i) {
+    const int at = 16 * i + 4 * c;
+    if (a.dim == DK) {
+      qv[i] = *reinterpret_cast<const f32x4u_t*>(q + at);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) qv[i][e] = at + e < a.dim ? q[at + e] : 0.0f;
+    }
+  }
+  const float mul = a.scale * temperature(a, pq), slope = a.slope[h];
+  const float* const kc = reinterpret_cast<const float*>(a.k_cache);
+  const float* const vc = reinterpret_cast<const float*>(a.v_cache);
+  f32x4_t k[KQ], v[4][VB / 4], acc[VB];
+  float m = -INFINITY, l = 0.0f;
+#pragma unroll
+  for (int b = 0; b < VB; ++b) acc[b] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+  // (16 positions from a multiple of 16 on never wrap)
+  auto load_keys = [&](int k0) __attribute__((always_inline)) {
+    if (k0 >= k_end) return;
+    const int slot = k0 % a.kl.slots, over = k_end - 1 - k0;
+    const float* const row = kc + ring_row(a.kl, g, slot + min(r, over)) + 4 * c;
+#pragma unroll
+    for (int i = 0; i < KQ; ++i) k[i] = *reinterpret_cast<const f32x4_t*>(row + 16 * i);
+  };
+  auto load_values = [&](int k0) __attribute__((always_inline)) {
+    if (k0 >= k_end) return;
+    const int slot = k0 % a.vl.slots, over = k_end - 1 - k0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float* const val = vc + ring_row(a.vl, g, slot + min(4 * c + j, over)) + VB * r;
+#pragma unroll
+      for (int b = 0; b < VB / 4; ++b) v[j][b] = *reinterpret_cast<const f32x4_t*>(val + 4 * b);
+    }
+  };
+  load_keys(k_begin + 16 * wave);
+  load_values(k_begin + 16 * wave);
+  for (int k0 = k_begin + 16 * wave; k0 < k_end; k0 += 16 * NW) {
+    f32x4_t part[PARTS];
+#pragma unroll
+    for (int i = 0; i < PARTS; ++i) part[i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < KQ; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        f32x4_t& to = part[(4 * i + e) % PARTS];
+        to = __builtin_amdgcn_mfma_f32_16x16x4f32(k[i][e], qv[i][e], to, 0, 0, 0);
+      }
+    load_keys(k0 + 16 * NW);
+#pragma unroll
+    for (int half = PARTS / 2; half > 0; half /= 2)
+#pragma unroll
+      for (int i = 0; i < half; ++i) part[i] = part[i] + part[i + half];
+    const f32x4_t s = part[0];
+    float p[4], top = -INFINITY;
+    bool seen[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int key = k0 + 4 * c + j;
+      seen[j] = key <= pq && key >= lo_q;
+      p[j] = s[j] * mul - slope * (float)(pq - key);
+      top = fmaxf(top, seen[j] ? p[j] : -INFINITY);
+    }
+    top = fmaxf(top, __shfl_xor(top, 16, 64));
+    top = fmaxf(top, __shfl_xor(top, 32, 64));
+    const float now = fmaxf(m, top), alpha = m > -INFINITY ? expf(m - now) : 0.0f;
+    l *= alpha;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      p[j] = seen[j] && p[j] != -INFINITY ? expf(p[j] - now) : 0.0f;
+      l += p[j];
+    }
+    m = now;
+#pragma unroll
+    for (int b = 0; b < VB; ++b) acc[b] = acc[b] * alpha;
+    // where some query does not see some key: values that are not finite go alone, to the queries that see them
+    bool odd = false;
+    if (k0 + 15 > first || k0 < oldest(last)) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int b = 0; b < VB; ++b) odd = odd || !(__builtin_fabsf(v[j][b >> 2][b & 3]) < INFINITY);
+      odd = __builtin_amdgcn_ballot_w64(odd) != 0;
+      if (odd) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int b = 0; b < VB; ++b)
+            if (!(__builtin_fabsf(v[j][b >> 2][b & 3]) < INFINITY)) v[j][b >> 2][b & 3] = 0.0f;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int b = 0; b < VB; ++b) acc[b] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[j][b >> 2][b & 3], p[j], acc[b], 0, 0, 0);
+    if (odd) {
+      for (int at = 0; at < min(16, k_end - k0); ++at) {
+        const int key = k0 + at;
+        const float* const val = vc + ring_row(a.vl, g, key % a.vl.slots);
+        float w = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float o = __shfl(p[j], (at >> 2) * 16 + r, 64);
+          if ((at & 3) == j) w = o;
+        }
+        if (key > pq || key < lo_q) continue;
+#pragma unroll
+        for (int b = 0; b < VB; ++b)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float x = val[VB * (4 * c + j) + b];
+            if (!(__builtin_fabsf(x) < INFINITY)) acc[b][j] = __builtin_fmaf(w, x, acc[b][j]);
+          }
+      }
+    }
+    load_values(k0 + 16 * NW);
+  }
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (c == 0) most[wave][r] = m, sums[wave][r] = l;
+  __syncthreads();
+  float all = most[0][r];
+  for (int w = 1; w < busy; ++w) all = fmaxf(all, most[w][r]);
+  const auto factor = [&](float x) { return x > -INFINITY ? expf(x - all) : 0.0f; };
+  const float mine = factor(m);
+#pragma unroll
+  for (int b = 0; b < VB; ++b) {
+    acc[b] = acc[b] * mine;
+    if (wave > 0) *reinterpret_cast<f32x4_t*>(held[wave - 1] + (b * 64 + lane) * 4) = acc[b];
+  }
+  __syncthreads();
+  if (wave > 0 || qi >= M) return;
+  float total = 0.0f;
+  for (int w = 0; w < busy; ++w) total = __builtin_fmaf(factor(most[w][r]), sums[w][r], total);
+  float* const out = reinterpret_cast<float*>(a.ctx) + (int64_t)qi * a.ldc + (int64_t)h * a.vdim;
+  for (int w = 1; w < busy; ++w) {
+#pragma unroll
+    for (int b = 0; b < VB; ++b) acc[b] = acc[b] + *reinterpret_cast<const f32x4_t*>(held[w - 1] + (b * 64 + lane) * 4);
+  }
+#pragma unroll
+  for (int b = 0; b < VB; ++b) acc[b] = acc[b] / total;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const int col = VB * (4 * c + j);
+#pragma unroll
+    for (int b = 0; b < VB; b += 4) {
+      if (col + b + 3 < a.vdim) {
+        *reinterpret_cast<f32x4u_t*>(out + col + b) = f32x4_t{acc[b][j], acc[b + 1][j], acc[b + 2][j], acc[b + 3][j]};
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (col + b + e < a.vdim) out[col + b + e] = acc[b + e][j];
+      }
+    }
+  }
+}
+
+template <int DK>
+void launch_tiles_f32(const WindowAttnArgs& a, hipStream_t st) {
+  const dim3 g((unsigned)a.heads, (unsigned)((a.M + 15) / 16));
+  if (a.vl.row == 64) hipLaunchKernelGGL((window_tile_f32_kernel<DK, 64>), g, dim3(512), 0, st, a);
+  else hipLaunchKernelGGL((window_tile_f32_kernel<DK, 128>), g, dim3(512), 0, st, a);
+}
+
 template <typename T>
 int launch_append(const WindowAttnArgs& a, hipStream_t st) {
   const int row = std::max(a.kl.row, a.vl.row);
@@ -672,7 +862,13 @@ int launch_window_attention(const WindowAttnArgs& a, bool f32, hipStream_t st, c
   AWQ_REQUIRE(!beside || window_takes_product(a, f32), "no product beside this attention");
   if (one_token_form(a)) return f32 ? launch_decode<float>(a, st, nullptr) : launch_decode<bf16_t>(a, st, beside);
   if (int rc = f32 ? launch_append<float>(a, st) : launch_append<bf16_t>(a, st)) return rc;
-  if (f32) return launch_queries<float>(a, st);
+  if (f32) {
+    if (a.kl.row > 128 || a.vl.row > 128 || a.pos.dyn) return launch_queries<float>(a, st);
+    if (a.kl.row == 64) launch_tiles_f32<64>(a, st);
+    else launch_tiles_f32<128>(a, st);
+    AWQ_HIP_TRY(hipGetLastError());
+    return AWQ_OK;
+  }
   if (a.kl.row > 256 || a.vl.row > 256 || a.pos.dyn) return launch_queries<bf16_t>(a, st);
   if (a.kl.row == 64) launch_tiles<64>(a, st);
   else if (a.kl.row == 128) launch_tiles<128>(a, st);

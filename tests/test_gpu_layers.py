@@ -626,6 +626,28 @@ def test_values_that_a_query_does_not_see(awq, lib, dev, f32, shape, window):
             assert np.array_equal(got[~sees], want[~sees]) and not np.isfinite(got[sees]).any(), (at, sizes)
 
 
+@pytest.mark.parametrize("heads,kv,dim,vdim", [(4, 2, 64, 128), (6, 2, 100, 60), (2, 1, 130, 256)], ids=str)
+@pytest.mark.parametrize("sizes", [[2, 14, 1], [15, 17, 33], [127, 2, 16], [129, 3]], ids=str)
+@pytest.mark.parametrize("window", [0, 40])
+def test_roundings_of_window_attention(awq, lib, dev, heads, kv, dim, vdim, sizes, window):
+    """Portions that end beside the edges of tiles of 16 queries and 128 keys, on a ring that wraps.  A score of up to S rounds by
+    S x 2^-24 (its products' sum, its bias, their difference), which its weight takes over with expf's 2^-23; a mean of values rounds
+    by less: (S + 4) x 2^-24, and S is below 16 here."""
+    print("roundings, window attention", heads, kv, dim, vdim, sizes, window, flush=True)
+    rng = np.random.default_rng(dim + sizes[0])
+    T, eps, scale, n = 300, 1e-6, 3.0 / dim ** 0.5, heads * dim + kv * (dim + vdim)
+    proj, pv = dev.act(np.pad(rng.standard_normal((T, n)), ((0, 0), (0, -n % 8))), True)
+    q = plain.rms(pv[:, :heads * dim].reshape(T, heads, dim), eps)
+    k = plain.rms(pv[:, heads * dim:(heads + kv) * dim].reshape(T, kv, dim), eps)
+    want = plain.window_attention(q, k, pv[:, (heads + kv) * dim:n].reshape(T, kv, vdim), window or None, scale, (0.0, 1.0))
+    assert scale * np.abs(np.einsum("thd,shd->hts", q, np.repeat(k, heads // kv, 1))).max() < 16
+    slots = ((window or T) - 1 + max(sizes) + 63) // 64 * 64
+    got = attend(awq, lib, dev, True, proj, heads, kv, dim, vdim, window, scale, eps, (0.0, 1.0), sizes, T, slots, T)
+    off = np.linalg.norm(got - want) / np.linalg.norm(want)
+    print("error %.1e" % off, flush=True)
+    assert off < 20 * 2.0 ** -24
+
+
 @pytest.mark.parametrize("f32", FORMATS, ids=["bf16", "f32"])
 @pytest.mark.parametrize("window", [1, 2, 31, 32, 33, 64, 65, 96, 128, 160])
 def test_window_edges(awq, lib, dev, f32, window):
