@@ -522,9 +522,10 @@ __global__ __launch_bounds__(512) void gemm_shared_kernel(GemmParams p, int n_rg
 // of k goes through two instructions, slice j taking dwords j (kh = 0) and
 // j + 2 (kh = 1) of each row's 16 bytes, so that a lane's two weight dwords
 // (2kh, 2kh + 1) are adjacent in the weight stream.
-// Two workgroup shapes:
+// Workgroup shapes:
 //   rows split: 4 wavefronts x 64 rows = 256 rows, one shared
 //     token tile per step; for products with many tiles.
+//   halves: the same with 8 wavefronts, the second four on the second half of k; where a compute unit has one workgroup.
 //   k split: the 4 wavefronts share 64 rows and take a quarter
 //     of k each (a token tile of their own per step), partial sums meet in LDS;
 //     four times as many workgroups for products with few tiles.
@@ -572,20 +573,23 @@ __device__ __forceinline__ int sk_wg_of(int64_t q, int64_t W, int G) {
 
 constexpr int EPI_PART = -1;  // rows split: a share of k only, FP32 sums to the workspace
 
-enum WideMode { WIDE_ROWS = 0, WIDE_K = 1, WIDE_ROWS_CUT = 2 };  // rows split (a tile per workgroup), k split, rows split with work cut evenly
+// rows split (a tile per workgroup), k split, rows split with work cut evenly, rows split with a half of k for each half of the wavefronts
+enum WideMode { WIDE_ROWS = 0, WIDE_K = 1, WIDE_ROWS_CUT = 2, WIDE_HALVES = 3 };
 
 template <bool ZINT, int MODE, int EPI, int TT>
-__global__ __launch_bounds__(256, (MODE == WIDE_K && TT == 4) ? 1 : ((MODE == WIDE_ROWS && TT == 2) ? 3 : 2)) void gemm_wide_kernel(GemmParams p) {
+__global__ __launch_bounds__(MODE == WIDE_HALVES ? 512 : 256, (MODE == WIDE_K && TT == 4) ? 1 : ((MODE == WIDE_ROWS && TT == 2) ? 3 : 2)) void gemm_wide_kernel(GemmParams p) {
   constexpr bool KSPLIT = MODE == WIDE_K;
   constexpr bool CUT = MODE == WIDE_ROWS_CUT;
+  constexpr int HALVES = MODE == WIDE_HALVES ? 2 : 1;
   constexpr int kTokens = 32 * TT;                   // tokens per workgroup
   constexpr int kSlot = kTokens * kWideStride;       // halves per token tile in LDS
   extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
   half_t* xs = reinterpret_cast<half_t*>(smem_raw);  // [2][NKB][32 TT tokens][kWideStride]
   constexpr int NKB = KSPLIT ? 4 : 1;
   constexpr int NH = kWideNH;
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = threadIdx.x & 255, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = HALVES == 2 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) : 0;
   const int n = lane & 31, kh = lane >> 5;
   // a step is NH blocks of k; a tile (k split: this wavefront's quarter of this workgroup's chunk) has
   // an even number of them (checked by the launcher)
@@ -603,9 +607,13 @@ __global__ __launch_bounds__(256, (MODE == WIDE_K && TT == 4) ? 1 : ((MODE == WI
   do {
     // this piece: steps [s_lo, s_lo + steps) of the tile
     int s_lo = 0, steps = tile_steps;
-    if (MODE == WIDE_ROWS && EPI == EPI_PART) {  // share blockIdx.y of k
+    if (EPI == EPI_PART) {  // share blockIdx.y of k
       s_lo = tile_steps * (int)blockIdx.y / p.kz;
       steps = tile_steps * ((int)blockIdx.y + 1) / p.kz - s_lo;
+    }
+    if (HALVES == 2) {
+      s_lo += half * (steps / 2);
+      steps /= 2;
     }
     if (CUT) {
       const int64_t q0 = (int64_t)tile * S2;
@@ -672,7 +680,10 @@ __global__ __launch_bounds__(256, (MODE == WIDE_K && TT == 4) ? 1 : ((MODE == WI
 #pragma unroll
       for (int h = 0; h < NH; ++h)
 #pragma unroll
-        for (int a = 0; a < kWideRP; ++a) wd[a][f][h] = KSPLIT ? __builtin_nontemporal_load(wp[a] + (int64_t)(f * NH + h) * 32) : wp[a][(int64_t)(f * NH + h) * 32];
+        for (int a = 0; a < kWideRP; ++a) {
+          const int64_t at = (int64_t)((f < steps ? f : steps - 1) * NH + h) * 32;  // (a k of 128 has two steps)
+          wd[a][f][h] = KSPLIT ? __builtin_nontemporal_load(wp[a] + at) : wp[a][at];
+        }
 
     f32x16_t acc[kWideRP][TT];
 #pragma unroll
@@ -696,9 +707,10 @@ __global__ __launch_bounds__(256, (MODE == WIDE_K && TT == 4) ? 1 : ((MODE == WI
       typedef __attribute__((address_space(1))) const void* gptr_t;
       typedef __attribute__((address_space(3))) void* lptr_t;
       constexpr int kTile = kTokens * 64;  // halves
-      __shared__ __attribute__((aligned(16))) half_t tile_a[kTile];
-      __shared__ __attribute__((aligned(16))) half_t tile_b[kTile];
-      __shared__ __attribute__((aligned(16))) half_t tile_c[kTile];
+      __shared__ __attribute__((aligned(16))) half_t tiles_a[HALVES * kTile];
+      __shared__ __attribute__((aligned(16))) half_t tiles_b[HALVES * kTile];
+      __shared__ __attribute__((aligned(16))) half_t tiles_c[HALVES * kTile];
+      half_t *const tile_a = tiles_a + half * kTile, *const tile_b = tiles_b + half * kTile, *const tile_c = tiles_c + half * kTile;
       // requests: instruction i of this wavefront covers token rows (wave TT + i) 8 .. + 7
       const int piece = (lane & 7) ^ ((lane >> 3) & 7);  // piece of k this lane fetches for its row
       const half_t* src[TT];
@@ -797,6 +809,26 @@ __global__ __launch_bounds__(256, (MODE == WIDE_K && TT == 4) ? 1 : ((MODE == WI
         step(s0, I0{});
         if (s0 + 1 < steps) step(s0 + 1, I1{});
         if (s0 + 2 < steps) step(s0 + 2, I2{});
+      }
+      if constexpr (HALVES == 2) {
+        // the halves of a sum meet: the first half of the wavefronts finishes row pair 0 of each tile, the second pair 1, in turns of
+        // 32 tokens through the places of two tiles (a place holds 16 sums of 256 threads)
+        static_assert(HALVES * kTile * 2 >= 16 * 256 * 4, "the sums take the places of the tiles");
+        float* const to = reinterpret_cast<float*>(half ? tiles_a : tiles_b);
+        const float* const from = reinterpret_cast<const float*>(half ? tiles_b : tiles_a);
+#pragma unroll
+        for (int t = 0; t < TT; ++t) {
+          __builtin_amdgcn_s_waitcnt(0x0f70);  // the last requests, of no use, have landed
+          __syncthreads();
+#pragma unroll
+          for (int i = 0; i < 16; ++i) to[i * 256 + tid] = half ? acc[0][t][i] : acc[1][t][i];
+          __syncthreads();
+#pragma unroll
+          for (int i = 0; i < 16; ++i) {
+            const float other = from[i * 256 + tid];
+            acc[0][t][i] = half ? other + acc[1][t][i] : acc[0][t][i] + other;
+          }
+        }
       }
     } else {
       // k split: the same software pipeline over quarter steps.  A wavefront stages its own slot
@@ -979,8 +1011,8 @@ __global__ __launch_bounds__(256, (MODE == WIDE_K && TT == 4) ? 1 : ((MODE == WI
       }
       if (!rows_ok) continue;
 #pragma unroll
-      for (int a = 0; a < kWideRP; ++a) {
-        const int row = rg0 * 16 + a * 32 + n;
+      for (int a = 0; a < kWideRP / HALVES; ++a) {
+        const int row = rg0 * 16 + (HALVES == 2 ? half : a) * 32 + n;
 #pragma unroll
         for (int t = 0; t < TT; ++t) {
           // Residuals some at a time: y may be res, so that a load behind a store of the same instance waits for its own trip to
@@ -1483,16 +1515,30 @@ int launch_wide(const GemmParams& p, bool zint, int n_wgs, hipStream_t st) {
       raised[variant].fetch_or(bit, std::memory_order_relaxed);
     }
   }
-  hipLaunchKernelGGL(kern, grid, dim3(256), lds, st, p);
+  hipLaunchKernelGGL(kern, grid, dim3(MODE == WIDE_HALVES ? 512 : 256), lds, st, p);
   if (KSPLIT && p.kz > 1) launch_reduce(p, st);
   return AWQ_OK;
 }
 
+// Two wavefronts per SIMD, each with a half of the workgroup's part of k, where workgroups have a compute unit each to themselves: one
+// wavefront waits for its own tokens and conversions, two fill the matrix cores for each other.  4,096 x 4,096, us, before and with
+// halves: 641 tokens 37.5, 33.8; 768 35.6, 31.1; 1,000 37.3, 35.0 (in a prompt pass 53, 42); 1,300 58.3, 54.7; 2,048 59.9, 58.0; 4,096 x 12,288 at
+// 1,300 147, 130, at 2,048 164, 159; 12,288 x 4,096 at 257 45.9, 35.8, at 512 53.7, 50.6; 1,536 x 1,536 at 2,048 17.2, 16.0; the shares of
+// gemm_norm_shares at 700 tokens 2.9 % of a prompt pass.  Not where a unit has two or three workgroups (4,096 x 4,096 at 1,152 tokens 54.3, 60.6;
+// 12,288 x 4,096 at 1,000 91.5, 102.2, at 2,048 163.3, 171.3), nor where the halves are so short that their meeting shows (k of 512
+// and 1,024: 0 to 4 % slower).  `blocks`: 32-wide blocks of k of a workgroup; each half takes whole steps.
+static bool halves_pay(int64_t wgs, int64_t blocks) { return wgs <= kSkWgs && blocks >= 48 && blocks % (2 * kWideNH) == 0; }
+
 // rows split, a tile of 128 tokens and a share of k per workgroup
 int launch_wide_shares(const GemmParams& p, bool zint, hipStream_t st) {
   const dim3 grid((unsigned)p.n_tiles, (unsigned)p.kz);
-  if (zint) hipLaunchKernelGGL((gemm_wide_kernel<true, WIDE_ROWS, EPI_PART, kWideTT>), grid, dim3(256), 0, st, p);
-  else hipLaunchKernelGGL((gemm_wide_kernel<false, WIDE_ROWS, EPI_PART, kWideTT>), grid, dim3(256), 0, st, p);
+  if (p.nblk % p.kz == 0 && halves_pay((int64_t)p.n_tiles * p.kz, p.nblk / p.kz)) {
+    if (zint) hipLaunchKernelGGL((gemm_wide_kernel<true, WIDE_HALVES, EPI_PART, kWideTT>), grid, dim3(512), 0, st, p);
+    else hipLaunchKernelGGL((gemm_wide_kernel<false, WIDE_HALVES, EPI_PART, kWideTT>), grid, dim3(512), 0, st, p);
+  } else {
+    if (zint) hipLaunchKernelGGL((gemm_wide_kernel<true, WIDE_ROWS, EPI_PART, kWideTT>), grid, dim3(256), 0, st, p);
+    else hipLaunchKernelGGL((gemm_wide_kernel<false, WIDE_ROWS, EPI_PART, kWideTT>), grid, dim3(256), 0, st, p);
+  }
   launch_reduce(p, st);
   return AWQ_OK;
 }
@@ -1847,13 +1893,15 @@ int launch_gemm(const void* wq, const half_t* scale, const half_t* zp, int64_t m
       int rc;
       if (plan == PLAN_ROWS_64) {
         p.n_tiles = (int32_t)(nr * ((M + 63) / 64));
-        rc = launch_wide<WIDE_ROWS, 2>(p, zp_integral, p.n_tiles, st);
+        rc = halves_pay(p.n_tiles, p.nblk) ? launch_wide<WIDE_HALVES, 2>(p, zp_integral, p.n_tiles, st)
+                                           : launch_wide<WIDE_ROWS, 2>(p, zp_integral, p.n_tiles, st);
       } else if (plan == PLAN_ROWS_CUT) {
         p.sk_head = (int32_t*)workspace;
         p.sk_part = (float*)ws_part;
         rc = launch_wide<WIDE_ROWS_CUT, 4>(p, zp_integral, (int)(2 * tiles <= kSkWgs ? 2 * tiles : kSkWgs), st);
       } else {
-        rc = launch_wide<WIDE_ROWS, 4>(p, zp_integral, (int)tiles, st);
+        rc = halves_pay(tiles, p.nblk) ? launch_wide<WIDE_HALVES, 4>(p, zp_integral, (int)tiles, st)
+                                       : launch_wide<WIDE_ROWS, 4>(p, zp_integral, (int)tiles, st);
       }
       if (rc) return rc;
     } else {

@@ -614,7 +614,7 @@ void launch_tiles(const WindowAttnArgs& a, hipStream_t st) {
 // it, nor, without a window, on where the pass begins.
 // Bound by the matrix cores' binary32 rate and, for few queries, by the trips to the cache.  8 heads of 128, the appending launch
 // included, us, and before a few queries at a time by vector instructions (window_query_kernel): 333 queries 24 (44), 512 30 (61), of 12 heads 46 (84), 333 of 32
-// heads of 64 29 (84), 333 behind 3,000 keys in a window of 1,024 43 (105), 2 queries there 37 (39); 4 queries alone 10.0 (8.8), 64 11.6 (10.9).
+// heads of 64 33 (83), 333 behind 3,000 keys in a window of 1,024 43 (105), 2 queries there 37 (39); 4 queries alone 10.1 (8.8), 64 11.7 (10.9).
 template <int DK, int DV>
 __global__ __launch_bounds__(512) void window_tile_f32_kernel(WindowAttnArgs a) {
   constexpr int KQ = DK / 16, VB = DV / 16, NW = 8;

@@ -823,6 +823,32 @@ def test_gemm_of_17_to_64_tokens(awq, lib, torch_gpu, m, k, M):
         assert int(d_ws[:4096].to(torch.int32).sum().item()) == 0
 
 
+# a workgroup to itself on its compute unit, its wavefronts in two halves of k: rows and tokens over the edge, as many
+# workgroups as units and some more, tiles of 64 and of 128 tokens, the shortest k of halves and a shorter one
+@pytest.mark.parametrize("m,k,M", [(384, 1536, 5121), (4096, 2048, 1024), (4096, 2048, 1025), (4096, 4096, 1281), (12288, 4096, 257), (1536, 1536, 2048), (1024, 1024, 2600)])
+def test_gemm_of_one_workgroup_for_each_unit(awq, lib, torch_gpu, m, k, M):
+    torch = torch_gpu
+    rng = np.random.default_rng(m + k + M)
+    zp_int = M % 2 == 0
+    packed, scale, zp = rand_awq(rng, m, k, zp_int=zp_int)
+    d_in, d_s, d_z = dev(torch, packed), dev(torch, scale), dev(torch, zp)
+    d_dq = torch.zeros(m * k, dtype=torch.float16, device="cuda")
+    awq.check(lib.awq_dequant(d_in.data_ptr(), d_s.data_ptr(), d_z.data_ptr(), d_dq.data_ptr(), m, k, m // 128, stream(torch)))
+    d_w = torch.zeros(m * k // 2, dtype=torch.uint8, device="cuda")
+    awq.check(lib.awq_linear_repack(d_in.data_ptr(), d_w.data_ptr(), m, k, stream(torch)))
+    d_x = torch.from_numpy(rng.standard_normal((M, k)).astype(np.float16)).cuda()
+    want = (d_x.float() @ d_dq.view(k, m).float()).double()
+    rms = float(want.square().mean().sqrt())
+    print("gemm", m, k, M, lib.awq_gemm_plan(m, k, M, 0), flush=True)
+    assert lib.awq_gemm_plan(m, k, M, 0) in (2, 3)
+    d_y = torch.full((M + 1, m), float("nan"), dtype=torch.float16, device="cuda")
+    awq.check(lib.awq_gemm(d_w.data_ptr(), d_s.data_ptr(), d_z.data_ptr(), m, k, d_x.data_ptr(), d_y.data_ptr(), M, int(zp_int), None, stream(torch)))
+    got = d_y.double()
+    assert bool(torch.isnan(got[M]).all())
+    # a rounding of the output to binary16 (2^-11) and of every weight of the reference (2^-11 each, as many signs: of the rms)
+    assert bool(((got[:M] - want).abs() <= 2.0 ** -11 * want.abs() + 6 * 2.0 ** -11 * rms).all())
+
+
 def _random_gemm_shapes(n, seed):
     """(m, k, M): multiples of 128 / 512 whose scale group does not depend on the input index"""
     rng = np.random.default_rng(seed)
