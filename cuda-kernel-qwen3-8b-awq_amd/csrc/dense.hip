@@ -117,12 +117,14 @@ __global__ __launch_bounds__(NW * 64) void dense_few_kernel(DenseArgs a) {
 // a wait for everything on its way at each barrier, 474); at few by the trips to memory (33 tokens, 4,096 x 4,096: 17.8,
 // was 19.9).
 // LISTED: the tokens come from runs of a list, each with a weight block of its own.
-template <int TT, int RB, int OUT, bool LISTED = false>
-__global__ __launch_bounds__(256, 2) void dense_many_kernel(DenseArgs a, int row_tiles, int tok_tiles, int cuts) {
+// HALVES 2: four more wavefronts, which take the second half of k with tiles of their own (halves_pay).
+template <int TT, int RB, int OUT, bool LISTED = false, int HALVES = 1>
+__global__ __launch_bounds__(HALVES * 256, 2) void dense_many_kernel(DenseArgs a, int row_tiles, int tok_tiles, int cuts) {
   // three arrays, so that the compiler can tell which reads a request on its way may touch
-  __shared__ __attribute__((aligned(16))) bf16_t tile0[32 * TT * 64];
-  __shared__ __attribute__((aligned(16))) bf16_t tile1[32 * TT * 64];
-  __shared__ __attribute__((aligned(16))) bf16_t tile2[32 * TT * 64];
+  constexpr int kTile = 32 * TT * 64;
+  __shared__ __attribute__((aligned(16))) bf16_t tiles0[HALVES * kTile];
+  __shared__ __attribute__((aligned(16))) bf16_t tiles1[HALVES * kTile];
+  __shared__ __attribute__((aligned(16))) bf16_t tiles2[HALVES * kTile];
   const int total = row_tiles * tok_tiles * cuts;
   // workgroups whose indices agree modulo 8 share a die: each die walks its own run of row tiles
   const int per = (total + 7) >> 3;
@@ -140,12 +142,15 @@ __global__ __launch_bounds__(256, 2) void dense_many_kernel(DenseArgs a, int row
     n_tok = run.count;
     list = a.list + run.first;
   }
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = threadIdx.x & 255, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = HALVES == 2 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) : 0;
+  bf16_t *const tile0 = tiles0 + half * kTile, *const tile1 = tiles1 + half * kTile, *const tile2 = tiles2 + half * kTile;
   const int n = lane & 31, kh = lane >> 5;
   const DenseSegment& s = segment_of(a, rt * 128 * RB);
   const int all_steps = (int)(a.k >> 6);
-  const int first_step = (int)((int64_t)all_steps * cut / cuts);
-  const int steps = (int)((int64_t)all_steps * (cut + 1) / cuts) - first_step;
+  const int first_of_cut = (int)((int64_t)all_steps * cut / cuts);
+  const int steps = ((int)((int64_t)all_steps * (cut + 1) / cuts) - first_of_cut) / HALVES;
+  const int first_step = first_of_cut + half * steps;
   const int64_t k16 = a.k >> 4;
 
   // this lane's pieces of the token tile
@@ -264,12 +269,40 @@ __global__ __launch_bounds__(256, 2) void dense_many_kernel(DenseArgs a, int row
     }
   }
   const int row_w = (rt * 4 + wave) * 32 * RB;
-  float* const turn = reinterpret_cast<float*>(TT == 4 ? tile0 : (wave < 2 ? tile0 : tile1)) + (TT == 4 ? wave : wave & 1) * 1024;
   __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): no request is on its way into the tiles any more
   __syncthreads();                     // the last step's readers are done
+  if constexpr (HALVES == 2) {
+    // the halves of a sum meet: the first half of the wavefronts finishes the first half of the tokens
+    constexpr int TH = TT / 2;
+    float* const to = reinterpret_cast<float*>(half ? tiles0 : tiles1);
+    const float* const from = reinterpret_cast<const float*>(half ? tiles1 : tiles0);
+    f32x16_t mine[RB][TH];
 #pragma unroll
-  for (int b = 0; b < RB; ++b)
-    store_block_rows<bf16_t, OUT, LISTED>(a, turn, acc[b], row_w + 32 * b, tt0, n_tok, list, row_tiles * 128 * RB, cut);
+    for (int b = 0; b < RB; ++b) {
+#pragma unroll
+      for (int t = 0; t < TH; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) to[(t * 16 + i) * 256 + tid] = half ? acc[b][t][i] : acc[b][TH + t][i];
+      __syncthreads();
+#pragma unroll
+      for (int t = 0; t < TH; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          const float other = from[(t * 16 + i) * 256 + tid];
+          mine[b][t][i] = half ? other + acc[b][TH + t][i] : acc[b][t][i] + other;
+        }
+      __syncthreads();
+    }
+    float* const turn = reinterpret_cast<float*>(half ? tiles1 : tiles0) + wave * 1024;
+#pragma unroll
+    for (int b = 0; b < RB; ++b)
+      store_block_rows<bf16_t, OUT, LISTED>(a, turn, mine[b], row_w + 32 * b, tt0 + half * 32 * TH, n_tok, list, row_tiles * 128 * RB, cut);
+  } else {
+    float* const turn = reinterpret_cast<float*>(TT == 4 ? tile0 : (wave < 2 ? tile0 : tile1)) + (TT == 4 ? wave : wave & 1) * 1024;
+#pragma unroll
+    for (int b = 0; b < RB; ++b)
+      store_block_rows<bf16_t, OUT, LISTED>(a, turn, acc[b], row_w + 32 * b, tt0, n_tok, list, row_tiles * 128 * RB, cut);
+  }
 }
 
 template <typename S>
@@ -413,6 +446,13 @@ constexpr ManyForm kManyForms[4] = {{2, 2, 512, 0.5296f, 0.0068f, 0.4825f, 2.990
 float shares_time(const DenseArgs& a, int64_t rows, int64_t cuts) {
   return 2.71f + (float)cuts * (0.3703f + (float)a.M * (float)rows * 8.0f / 2.708e6f);
 }
+// Two wavefronts per SIMD, each with a half of k, where a tile of a product has a compute unit to itself (at most 256 of them): one
+// waits for its trips to memory and its tokens, two have products for each other.  us, with four wavefronts and with eight: 1,024 x 512 at 129 tokens
+// 8.1, 7.7; 2,048 x 1,024 at 333 10.3, 9.6; 2,048 x 2,048 at 512 14.2, 12.5; 6,144 x 2,048 at 200 18.9, 16.7; 4,096 x 4,096 at 512 32.6, 29.3, at 1,000
+// 41.6, 38.9; 12,288 x 2,048 at 129 23.9, 21.8.  Not for shares of k, which are short already (1,024 x 4,096 at 512 tokens in four 16.2, 17.1), nor for
+// tokens of a list, whose tiles are mostly without any (no gain).
+bool halves_pay(int64_t groups, int64_t steps, int64_t cuts) { return cuts == 1 && groups <= 256 && steps >= 8 && steps % 2 == 0; }
+
 // The time of a product in us, but for what all forms of it share: what the choice of a form and of a number of shares of k needs.
 // The numbers are fitted for the choice, not for the time, to 49,600 timings (2,153 products: 111 shapes from 256 x 64 to 32,768 x 1,024,
 // 28,672 x 8,192 and 4,096 x 16,384, 33 to 2,048 tokens, all forms, 1 to 16 shares, every kind of output, weights from memory).  The form
@@ -427,6 +467,8 @@ float many_time(const DenseArgs& a, int64_t rows, const ManyForm& f, int64_t cut
   const float wait = f.wait + f.root * sqrtf((float)std::min<int64_t>(256, row_tiles * cuts * a.batch));
   const float per_unit = ceilf(groups / 256.0f);
   float t = steps * wait * ceilf(groups / (float)f.resident);
+  // (what eight wavefronts give, where it was timed; sums that another launch adds anyway are cheaper in shares)
+  if (halves_pay((int64_t)groups, a.k >> 6, cuts) && a.k <= 4096 && !a.shares) t -= steps * (f.rb == 1 ? 0.05f : 0.02f);
   if (per_unit > 1.0f) t = std::max(t, steps * per_unit * f.step);
   t = std::max(t, (float)rows * (float)a.k * (float)a.batch * 2.0f / 9.12e6f);
   return cuts > 1 ? t + shares_time(a, rows, cuts) : t + per_unit * f.end * (a.out == DENSE_F32 ? 1.0f : 1.7f);
@@ -435,11 +477,19 @@ float many_time(const DenseArgs& a, int64_t rows, const ManyForm& f, int64_t cut
 template <int OUT, bool LISTED>
 void launch_form(const DenseArgs& a, const ManyForm& f, int64_t rows, int64_t tok_tiles, int64_t cuts, hipStream_t st) {
   const int row_tiles = (int)(rows / (128 * f.rb));
-  const dim3 grid((unsigned)((row_tiles * tok_tiles * cuts + 7) / 8 * 8), (unsigned)a.batch), b(256);
-  if (f.tt == 2 && f.rb == 2) hipLaunchKernelGGL((dense_many_kernel<2, 2, OUT, LISTED>), grid, b, 0, st, a, row_tiles, (int)tok_tiles, (int)cuts);
-  else if (f.tt == 2) hipLaunchKernelGGL((dense_many_kernel<2, 1, OUT, LISTED>), grid, b, 0, st, a, row_tiles, (int)tok_tiles, (int)cuts);
-  else if (f.rb == 2) hipLaunchKernelGGL((dense_many_kernel<4, 2, OUT, LISTED>), grid, b, 0, st, a, row_tiles, (int)tok_tiles, (int)cuts);
-  else hipLaunchKernelGGL((dense_many_kernel<4, 1, OUT, LISTED>), grid, b, 0, st, a, row_tiles, (int)tok_tiles, (int)cuts);
+  const dim3 grid((unsigned)((row_tiles * tok_tiles * cuts + 7) / 8 * 8), (unsigned)a.batch);
+  const auto launch = [&](auto halves) {
+    constexpr int H = decltype(halves)::value;
+    const dim3 b(H * 256);
+    if (f.tt == 2 && f.rb == 2) hipLaunchKernelGGL((dense_many_kernel<2, 2, OUT, LISTED, H>), grid, b, 0, st, a, row_tiles, (int)tok_tiles, (int)cuts);
+    else if (f.tt == 2) hipLaunchKernelGGL((dense_many_kernel<2, 1, OUT, LISTED, H>), grid, b, 0, st, a, row_tiles, (int)tok_tiles, (int)cuts);
+    else if (f.rb == 2) hipLaunchKernelGGL((dense_many_kernel<4, 2, OUT, LISTED, H>), grid, b, 0, st, a, row_tiles, (int)tok_tiles, (int)cuts);
+    else hipLaunchKernelGGL((dense_many_kernel<4, 1, OUT, LISTED, H>), grid, b, 0, st, a, row_tiles, (int)tok_tiles, (int)cuts);
+  };
+  if constexpr (!LISTED && OUT != DENSE_PART) {
+    if (halves_pay(row_tiles * tok_tiles * a.batch, a.k >> 6, cuts)) return launch(std::integral_constant<int, 2>{});
+  }
+  launch(std::integral_constant<int, 1>{});
 }
 
 template <int OUT>

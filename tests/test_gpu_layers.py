@@ -323,6 +323,31 @@ def test_products_of_many_tokens_in_every_form(awq, lib, dev, rows, k, tokens):
         assert (off <= exact + (2.0 ** -8 * np.abs(want) if out == awq.DENSE_STORE else 8 * 2.0 ** -24)).all()
 
 
+# tiles of every size with a compute unit to each and an even number of steps, which two halves of a workgroup share: as many as there
+# are units and some more, rows and tokens that end inside a tile, the fewest steps
+@pytest.mark.parametrize("rows,k,tokens", [(1000, 512, 129), (2048, 1024, 1000), (2048, 1024, 1100), (8200, 2176, 400), (12300, 2048, 129), (4100, 2048, 1025), (300, 640, 34)])
+def test_products_whose_k_two_halves_share(awq, lib, dev, rows, k, tokens):
+    print("halves", rows, k, tokens, flush=True)
+    rng = np.random.default_rng(rows + tokens)
+    block = dev.torch.zeros((rows + 255) // 256 * 256 * k, dtype=dev.torch.bfloat16, device="cuda")
+    w, wv = dev.act(rng.standard_normal((rows, k)) / k ** 0.5, False)
+    awq.check(lib.awq_dense_pack(w.data_ptr(), 0, rows, k, block.data_ptr(), k, 0, 0, 0, dev.stream))
+    x, xv = dev.act(rng.standard_normal((tokens, k)), False)
+    want = xv @ wv.T
+    for out in (awq.DENSE_F32, awq.DENSE_RESIDUAL, awq.DENSE_STORE):
+        y = dev.empty((tokens + 1, rows), out != awq.DENSE_STORE, fill=0.5)
+        y[tokens] = float("nan")
+        a = awq.AwqDenseArgs()
+        a.w, a.k, a.tokens, a.n_segments, a.out = block.data_ptr(), k, tokens, 1, out
+        a.segment[0] = awq.AwqDenseSegment(x.data_ptr(), y.data_ptr(), k, rows, 0, rows, 0, 0, 0, 0)
+        awq.check(lib.awq_dense(ctypes.byref(a), 0, dev.stream))
+        got = dev.host(y)
+        assert np.isnan(got[tokens]).all()
+        off = np.abs(got[:tokens] - want - (0.5 if out == awq.DENSE_RESIDUAL else 0.0))
+        # exact operands: about sqrt(k) roundings of 2^-24 of a sum's size; then as in the test above
+        assert (off <= 8 * k ** 0.5 * 2.0 ** -24 + (2.0 ** -8 * np.abs(want) if out == awq.DENSE_STORE else 8 * 2.0 ** -24)).all()
+
+
 @pytest.mark.parametrize("k", [64, 320, 512, 576])
 @pytest.mark.parametrize("rows,tokens", [(2000, 2001), (8200, 1030)])
 def test_products_of_few_inputs_and_many_tokens(awq, lib, dev, rows, tokens, k):
