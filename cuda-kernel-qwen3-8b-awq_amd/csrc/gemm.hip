@@ -1529,6 +1529,15 @@ int launch_wide(const GemmParams& p, bool zint, int n_wgs, hipStream_t st) {
 // and 1,024: 0 to 4 % slower).  `blocks`: 32-wide blocks of k of a workgroup; each half takes whole steps.
 static bool halves_pay(int64_t wgs, int64_t blocks) { return wgs <= kSkWgs && blocks >= 48 && blocks % (2 * kWideNH) == 0; }
 
+// rows split, a tile of 64 tokens and a share of k per workgroup, halves of it for its wavefronts
+int launch_wide_shares64(const GemmParams& p, bool zint, hipStream_t st) {
+  const dim3 grid((unsigned)p.n_tiles, (unsigned)p.kz);
+  if (zint) hipLaunchKernelGGL((gemm_wide_kernel<true, WIDE_HALVES, EPI_PART, 2>), grid, dim3(512), 0, st, p);
+  else hipLaunchKernelGGL((gemm_wide_kernel<false, WIDE_HALVES, EPI_PART, 2>), grid, dim3(512), 0, st, p);
+  launch_reduce(p, st);
+  return AWQ_OK;
+}
+
 // rows split, a tile of 128 tokens and a share of k per workgroup
 int launch_wide_shares(const GemmParams& p, bool zint, hipStream_t st) {
   const dim3 grid((unsigned)p.n_tiles, (unsigned)p.kz);
@@ -1728,6 +1737,18 @@ int gemm_norm_shares(int64_t m, int64_t k, int64_t M) {
   return tiles * 3 <= 2 * kSkWgs ? 3 : 0;
 }
 
+// The same with tiles of 64 tokens, where those of 128 are too few: shares that give 192 of the compute units a workgroup, of at most 4.  The
+// norm has its launch's trip in common with the sums, and a workgroup has eight wavefronts (halves_pay).  Prompts of 36 layers, ms, without and
+// with it for 4,096 x 4,096 and for 4,096 x 12,288: 192 tokens 5.62, 5.36 and 5.32; 250 6.89, 6.52 and 6.61; 300 6.87, 6.64 and 6.41; 400 8.43, 8.22
+// (the second has shares of tiles of 128); 512 8.82, 8.63.  128 workgroups: 70 tokens 3.99, 4.01 and 4.11, 128 4.26, 4.23 and 4.29.
+static int norm_shares64(int64_t m, int64_t k, int64_t M) {
+  const int64_t tiles = (m + 255) / 256 * ((M + 63) / 64), blocks = k / AWQ_BLOCK_K;
+  if (k < 4096 || m < 4096 || m > kNormRow || M < 65 || gemm_norm_shares(m, k, M)) return 0;
+  for (int kz : {4, 3, 2})
+    if (tiles * kz <= kSkWgs && blocks % (2 * kWideNH * kz) == 0) return tiles * kz >= 192 ? kz : 0;
+  return 0;
+}
+
 // room for a header and the partial sums of a product whose work is cut over workgroups (0: never cut)
 // the shape awq_gemm takes for a product (diagnostics and tests): 0 few tokens, 1 k split, 2 rows split
 // with a tile per workgroup, 3 rows split with 64 tokens per workgroup, 4 rows split with the work cut evenly,
@@ -1804,6 +1825,16 @@ int launch_gemm(const void* wq, const half_t* scale, const half_t* zp, int64_t m
     else if (f.rg == 4) rc = launch_panel<4, 3, 8>(p, zp_integral, st);
     else rc = f.rg == 3 ? launch_panel_tokens<3, 8>(p, zp_integral, st) : launch_panel_tokens<1, 8>(p, zp_integral, st);
     if (rc) return rc;
+    AWQ_HIP_TRY(hipGetLastError());
+    return AWQ_OK;
+  }
+  if (const int shares = norm && epilogue == EPI_RESIDUAL && workspace ? norm_shares64(m, k, M) : 0;
+      shares && kSkHeaderBytes + (int64_t)shares * M * m * 4 <= workspace_bytes) {
+    p.nr = (int32_t)((m + 255) / 256);
+    p.n_tiles = (int32_t)(p.nr * ((M + 63) / 64));
+    p.kz = shares;
+    p.part = (float*)((char*)workspace + kSkHeaderBytes);
+    if (int rc = launch_wide_shares64(p, zp_integral, st)) return rc;
     AWQ_HIP_TRY(hipGetLastError());
     return AWQ_OK;
   }

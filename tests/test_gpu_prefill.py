@@ -119,6 +119,24 @@ def test_sums_of_a_cut_product_normed_by_their_launch(awq, oracle, torch_gpu, hi
     oracle.awqo_model_destroy(model)
 
 
+@pytest.mark.parametrize("n", [129, 200, 320, 385, 512, 513])
+def test_prompts_whose_short_products_go_in_shares(awq, oracle, torch_gpu, n):
+    """k of Wo and W2 in four, three and two shares of tiles of 64 tokens, full and nearly empty, and the first count past them"""
+    cfg = awq.make_config(n_layers=2, hidden=4096, inter=12288, vocab=1024, max_pos=576)
+    model = make_oracle_model(oracle, cfg)   # only as the host buffer of the weights here
+    eng = awq.QWen3AWQInfer.empty(cfg)
+    fill_pair(awq, oracle, cfg, 80, engine=eng, model=model, profile=awq.SYNTH_BALANCED)
+    prompt = np.random.default_rng(n).integers(0, cfg.vocab, n).tolist()
+    eng.reset()
+    eng.prefill(prompt)
+    want = as_f32(eng.read_hidden()).copy()
+    eng.reset()
+    eng.prefill(prompt, batched=True)
+    assert close(as_f32(eng.read_hidden()), want), n
+    eng.close()
+    oracle.awqo_model_destroy(model)
+
+
 @pytest.mark.parametrize("n", [17, 32, 40, 48, 64])
 def test_prompts_of_17_to_64_tokens_at_the_model_width(awq, oracle, torch_gpu, n):
     """every product's end behind the kernel for so few: residual, GeLU, sums with the norm of the next layer"""
