@@ -1727,7 +1727,7 @@ static WidePlan plan_wide(int64_t m, int64_t k, int64_t M, bool has_workspace) {
 // each compute unit one workgroup, three where two units' worth are then less than full.  Rows then cost no launch for their
 // norm (5.7 us), and nothing waits for another workgroup's sums.  4,096 x 12,288 with the launch that adds, against the k-split
 // workgroups up to 512 tokens and the work cut evenly above: 384 tokens 54 us (61), 512 61 (66), 640 73 (103), 768 91 (106), 1,000
-// 104 (119), 1,152 126 (150), 1,280 132 (160); from 1,281 on (176 tiles) a tile per workgroup is faster (1,536: 166 against 152).  At
+// 104 (119; with eight wavefronts 100), 1,152 126 (150), 1,280 132 (160); from 1,281 on (176 tiles) a tile per workgroup is faster (1,536: 166 against 152).  At
 // k = 4,096 the sums' way through memory costs more than the tiles gain (1,000 tokens 48 us with two shares, 39 without).
 int gemm_norm_shares(int64_t m, int64_t k, int64_t M) {
   const int64_t tiles = (m + 255) / 256 * ((M + kWideTokens - 1) / kWideTokens);
