@@ -153,7 +153,7 @@ struct Qwen3Engine final : awq_engine {
   // workspaces
   void* attn_ws = nullptr;
   void* sample_ws = nullptr;  // best candidate and workgroup counts of the sampling launch
-  uint8_t* embed_rows = nullptr;  // the embedding transposed into token rows, for the sampling launch's gather
+  uint8_t* embed_rows = nullptr;  // the embedding transposed into token rows, for the gathers of the sampling launch and of prompt passes
   // activations of the batched prompt pass, [chunk][n] each; allocated at first use
   struct {
     half_t *hidden = nullptr, *norm = nullptr, *qkv = nullptr, *q = nullptr, *ctx = nullptr, *mid = nullptr;
@@ -964,9 +964,7 @@ int Qwen3Engine::enqueue_prompt_pass(const int32_t* tokens, int64_t pos0, int64_
   if (int rc = ensure_prefill_buffers(e)) return rc;
   const int64_t H = e->cfg.hidden;
   AWQ_HIP_TRY(hipMemcpyAsync(e->pb.tokens, tokens, (size_t)M * 4, hipMemcpyHostToDevice, e->stream));
-  if (int rc = launch_embed_batch(e->embed.packed, e->embed.scale, e->embed.zp, H, e->cfg.vocab, e->pb.tokens, M,
-                                  e->pb.hidden, e->stream))
-    return rc;
+  if (int rc = launch_embed_batch(e->embed_rows, e->embed.scale, e->embed.zp, H, e->pb.tokens, M, e->pb.hidden, e->stream)) return rc;
   bool normed = false;
   for (int l = 0; l < e->cfg.n_layers; ++l)
     if (int rc = enqueue_layer_batch(e, l, pos0, M, &normed)) return rc;
@@ -1046,8 +1044,7 @@ int Qwen3Engine::enqueue_exact_pass(const int32_t* tokens, int64_t pos0, int64_t
   Qwen3Engine* e = this;
   const int64_t H = e->cfg.hidden;
   AWQ_HIP_TRY(hipMemcpyAsync(e->pc.tokens, tokens, (size_t)M * 4, hipMemcpyHostToDevice, e->stream));
-  if (int rc = launch_embed_batch(e->embed.packed, e->embed.scale, e->embed.zp, H, e->cfg.vocab, e->pc.tokens, M, e->pc.hidden, e->stream))
-    return rc;
+  if (int rc = launch_embed_batch(e->embed_rows, e->embed.scale, e->embed.zp, H, e->pc.tokens, M, e->pc.hidden, e->stream)) return rc;
   if (int rc = enqueue_canon_layers(e, e->pc.hidden, pos0, M)) return rc;
   // the state the generation loop starts from (:1357): the last position's output
   return launch_copy(e->pc.hidden + (M - 1) * H, e->hidden, H * 2, e->stream);
