@@ -139,17 +139,20 @@ __device__ __forceinline__ Split4 split4(f32x4_t v) {
   return s;
 }
 
-// On v_mfma_f32_32x32x16_bf16, whose products are exact and which does 16 times the operations of v_mfma_f32_32x32x2_f32: both operands
-// as three terms each and the six products of two terms that are 2^-18 of the whole or more (the others 2^-24 at most, of either sign); where a step's weights are
-// bfloat16 numbers, as a checkpoint in bfloat16 has them, three are left and nothing is left out.  The first terms' products have a sum
-// of their own, which is rounded once per 16 inputs.  A workgroup of
-// four wavefronts takes 32 RW rows and 32 TW C tokens, steps of 32 inputs; KW wavefronts share the inputs of a step, whose
-// sums meet in LDS.  Weights and tokens are requested two steps ahead into registers, split once and go through LDS, a term's 64 bytes per row and
-// step, the four 16-byte pieces of row r at positions c ^ (r / 4 & 3).  Bound by the splitting (vector instructions) beside the matrix
-// cores, at few tokens by the weights' bytes.  Where the tiles do not fill the device, k is cut over `cuts` workgroups and a second
-// launch adds their sums, as in bfloat16.  333 tokens: 1,024 rows of 4,096 inputs 39.7 -> 27 us, 7,168 of 1,024 59 -> 35, 32,768 of
-// 1,024 211 -> 116 (v_mfma_f32_32x32x2_f32 before); with weights that are no bfloat16 numbers 35, 52 and 183, and up to 50 tokens, where weights' bytes
-// and trips to memory are the time, up to 6 % more than before.  Off from 64 bits by 0.8e-7 to 1.9e-7, before 1.6e-7 to 5.7e-7.
+// On v_mfma_f32_32x32x16_bf16, whose products are exact and which does 16 times the operations of v_mfma_f32_32x32x2_f32: both
+// operands as three terms each and all products of two terms but the one of the last two, which is 2^-30 of the whole at most.  (A
+// second and a third term's product is up to 2^-22 of the whole, and cut terms have the sign of their number: without these two a
+// product came out smaller by 0.7 x 2^-24 on average and 7.8 x 2^-24 at most.)  Where a step's weights are bfloat16 numbers, as a
+// checkpoint in bfloat16 has them, three products are left and nothing is left out.  The first terms' products have a sum of their
+// own, which is rounded once per 16 inputs.
+// A workgroup of four wavefronts takes 32 RW rows and 32 TW C tokens, steps of 32 inputs; KW wavefronts share the inputs of a step,
+// whose sums meet in LDS.  Weights and tokens are requested two steps ahead into registers, split once and go through LDS, a term's
+// 64 bytes per row and step, the four 16-byte pieces of row r at positions c ^ (r / 4 & 3).  Where the tiles do not fill the device, k
+// is cut over `cuts` workgroups and a second launch adds their sums, as in bfloat16.
+// Bound by the splitting (vector instructions) beside the matrix cores, at few tokens by the weights' bytes.  333 tokens, us, on
+// v_mfma_f32_32x32x2_f32 before, weights that are bfloat16 numbers, and weights that are not: 1,024 rows of 4,096 inputs 40, 27, 39;
+// 7,168 of 1,024 58, 34, 57; 32,768 of 1,024 220, 111, 207.  Up to 50 tokens weights that are not take up to 11 % more than before.
+// Off from 64 bits (norm) by 0.8e-7 to 1.8e-7 with 300 to 1,024 rows of 64 to 4,096 inputs, either way; before 1.1e-7 to 2.2e-7.
 // An infinity has no such terms (what it leaves is NaN): a wavefront that finds sums that are not finite forms them again, in binary32.
 template <int RW, int TW, int KW, int C, int OUT, bool LISTED = false>
 __global__ __launch_bounds__(256, 2) void dense_many_f32_kernel(DenseArgs a, int row_tiles, int tok_tiles, int cuts) {
@@ -256,6 +259,8 @@ __global__ __launch_bounds__(256, 2) void dense_many_f32_kernel(DenseArgs a, int
       const bf16x8_t w0 = term(0, rw * 32);
       if (all) {
         const bf16x8_t w1 = term(1, rw * 32), w2 = term(2, rw * 32);
+        add(low, w2, 1);
+        add(low, w1, 2);
         add(low, w2, 0);
         add(low, w1, 1);
         add(low, w1, 0);
@@ -303,12 +308,13 @@ __global__ __launch_bounds__(256, 2) void dense_many_f32_kernel(DenseArgs a, int
     for (int i = 0; i < 16; ++i) acc[0][i] += other[i * 64 + lane];
     wave_sync();
   }
+  const auto holds = [](float v) { return __builtin_fabsf(v) < INFINITY; };
 #pragma unroll
   for (int t = 0; t < C; ++t) {
-    bool finite = true;
+    bool all = true;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) finite = finite && __builtin_fabsf(acc[t][i]) < INFINITY;
-    if (__builtin_amdgcn_ballot_w64(!finite) == 0) continue;
+    for (int i = 0; i < 16; ++i) all = all && holds(acc[t][i]);
+    if (__builtin_amdgcn_ballot_w64(!all) == 0) continue;
     f32x16_t again;
 #pragma unroll
     for (int i = 0; i < 16; ++i) again[i] = 0.0f;
@@ -316,7 +322,7 @@ __global__ __launch_bounds__(256, 2) void dense_many_f32_kernel(DenseArgs a, int
     for (int i = 0; i < 32 * steps; i += 2) again = __builtin_amdgcn_mfma_f32_32x32x2f32(w[i], x[i], again, 0, 0, 0);
 #pragma unroll
     for (int i = 0; i < 16; ++i)
-      if (!(__builtin_fabsf(acc[t][i]) < INFINITY)) acc[t][i] = again[i];
+      if (!holds(acc[t][i])) acc[t][i] = again[i];
   }
   store_block_rows<float, OUT, LISTED>(a, turns + wave * 1024, acc, rt * ROWS + rw * 32, tt0 + tw * C * 32, n_tok, list, row_tiles * ROWS,
                                        cut);

@@ -163,7 +163,7 @@ def test_binary32_products_of_weights_in_either_format(awq, lib, dev, tokens, ro
             return dev.host(y).astype(np.float64)
         want = x.astype(np.float64) @ w.T.astype(np.float64)
         # 36 sums of 16 products: 36 roundings of 2^-24 of partial sums, which are below 6 (2.5 million outputs of rms 1) and, in the
-        # mean square over all, sqrt(i / 36) behind the i-th: 2^-24 sqrt(18).  A term left out is 2^-17 of its product.
+        # mean square over all, sqrt(i / 36) behind the i-th: 2^-24 sqrt(18).  What is left out of a product is 2^-30 of it.
         before = run()
         assert np.abs(before - want).max() < 36 * 6 * 2.0 ** -24 * scale
         assert np.sqrt(np.mean((before - want) ** 2)) < 18 ** 0.5 * 2.0 ** -24 * scale
@@ -177,6 +177,44 @@ def test_binary32_products_of_weights_in_either_format(awq, lib, dev, tokens, ro
         rest = [t for t in range(tokens) if not 1 <= t <= 4]
         assert np.array_equal(got[rest], before[rest])
         x = keep
+
+
+def binary32_product(awq, lib, dev, w, x, floats):
+    """x w^T by awq_dense in binary32, with a workspace of so many floats"""
+    (rows, k), tokens = w.shape, len(x)
+    block = dev.torch.zeros((rows + 255) // 256 * 256 * k, dtype=dev.torch.float32, device="cuda")
+    wd, xd, y, ws = dev.f(w), dev.f(x), dev.empty((tokens, rows), True), dev.empty((max(1, floats),), True)
+    awq.check(lib.awq_dense_pack(wd.data_ptr(), 1, rows, k, block.data_ptr(), k, 0, 0, 1, dev.stream))
+    a = awq.AwqDenseArgs()
+    a.w, a.k, a.tokens, a.n_segments, a.out = block.data_ptr(), k, tokens, 1, awq.DENSE_F32
+    a.segment[0] = awq.AwqDenseSegment(xd.data_ptr(), y.data_ptr(), k, rows, 0, rows, 0, 0, 0, 0)
+    a.workspace, a.workspace_floats = (ws.data_ptr() if floats else None), floats
+    awq.check(lib.awq_dense(ctypes.byref(a), 1, dev.stream))
+    return dev.host(y)
+
+
+# A product of two binary32 numbers rounds by 2^-24 of itself; their bfloat16 terms' sums by 2^-24 of what is 2^-6 of it, five times, and
+# what is left out is 2^-30: an eighth more.  Where all terms have one sign, what were left out of the products would add up: roundings
+# go either way, and the mean of many outputs' errors is far below one.  0x3f80ffff has the largest second and third terms.
+@pytest.mark.parametrize("tokens,rows", [(5, 300), (33, 300), (70, 300), (300, 8200)])
+@pytest.mark.parametrize("k", [64, 576])
+def test_no_bits_of_a_binary32_product_are_left_out(awq, lib, dev, tokens, rows, k):
+    print("binary32 bits", tokens, rows, k, flush=True)
+    rng = np.random.default_rng(rows + k)
+    worst = np.array([0x3f80ffff], np.uint32).view(np.float32)[0]
+    w, x = rng.standard_normal((rows, k)).astype(np.float32), rng.standard_normal((tokens, k)).astype(np.float32)
+    one = np.zeros_like(x)
+    at = rng.integers(0, k, tokens)
+    one[np.arange(tokens), at] = x[np.arange(tokens), at]
+    for floats in (0, 1 << 22):
+        for wv, xv in ((w, one), (np.full_like(w, worst), np.where(one != 0, worst, np.float32(0)))):
+            want = xv.astype(np.float64) @ wv.T.astype(np.float64)
+            assert (np.abs(binary32_product(awq, lib, dev, wv, xv, floats) - want) <= 1.125 * 2.0 ** -24 * np.abs(want)).all()
+        wv, xv = np.abs(w), np.abs(x)
+        want = xv.astype(np.float64) @ wv.T.astype(np.float64)
+        off = np.mean((binary32_product(awq, lib, dev, wv, xv, floats) - want) / want)
+        print("mean %.3f x 2^-24" % (off * 2 ** 24), flush=True)
+        assert abs(off) < 0.3 * 2.0 ** -24
 
 
 @pytest.mark.parametrize("k", [64, 192, 320, 448, 1024, 1088, 1152, 1536, 1792, 2048, 2112, 2560, 3072, 3584, 4160, 8192, 8256, 12352])
