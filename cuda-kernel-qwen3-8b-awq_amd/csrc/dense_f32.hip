@@ -120,7 +120,7 @@ __global__ __launch_bounds__(256) void dense_one_f32_kernel(DenseArgs a, std::co
 
 // --- many tokens ---------------------------------------------------------------------------------------------
 // Four numbers as sums of three bfloat16 terms: the upper halves of the numbers, of what that leaves, and of what is left then.  Eight
-// bits of significand each, so the sum is the number itself (down to 2^-110, where the last term leaves the range).
+// bits of significand each, so the sum is the number itself, down to 2^-110: there the last terms leave the range of bfloat16.
 struct Split4 {
   uint2 part[3];
 };
@@ -153,7 +153,9 @@ __device__ __forceinline__ Split4 split4(f32x4_t v) {
 // v_mfma_f32_32x32x2_f32 before, weights that are bfloat16 numbers, and weights that are not: 1,024 rows of 4,096 inputs 40, 27, 39;
 // 7,168 of 1,024 58, 34, 57; 32,768 of 1,024 220, 111, 207.  Up to 50 tokens weights that are not take up to 11 % more than before.
 // Off from 64 bits (norm) by 0.8e-7 to 1.8e-7 with 300 to 1,024 rows of 64 to 4,096 inputs, either way; before 1.1e-7 to 2.2e-7.
-// An infinity has no such terms (what it leaves is NaN): a wavefront that finds sums that are not finite forms them again, in binary32.
+// An infinity has no such terms (what it leaves is NaN), and numbers below 2^-110 not all of theirs: a wavefront that finds sums that
+// are not finite, or other than zero and below 2^-100, forms them again, in binary32.  (Inputs of 2^-115 were off by 37 x 2^-24 of the
+// result, of 2^-120 by 1,180, and still are beside operands so large that the sum is 2^-100 and more.)
 template <int RW, int TW, int KW, int C, int OUT, bool LISTED = false>
 __global__ __launch_bounds__(256, 2) void dense_many_f32_kernel(DenseArgs a, int row_tiles, int tok_tiles, int cuts) {
   static_assert(RW * TW * KW == 4 && (KW == 1 || (KW == 2 && C == 1)), "four wavefronts");
@@ -308,13 +310,16 @@ __global__ __launch_bounds__(256, 2) void dense_many_f32_kernel(DenseArgs a, int
     for (int i = 0; i < 16; ++i) acc[0][i] += other[i * 64 + lane];
     wave_sync();
   }
-  const auto holds = [](float v) { return __builtin_fabsf(v) < INFINITY; };
+  const auto holds = [](float v) __attribute__((always_inline)) {
+    const uint32_t size = __float_as_uint(v) & 0x7fffffffu, least = __float_as_uint(0x1p-100f);
+    return (int)(size - least < 0x7f800000u - least) | (int)(size == 0);
+  };
 #pragma unroll
   for (int t = 0; t < C; ++t) {
-    bool all = true;
+    int all = 1;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) all = all && holds(acc[t][i]);
-    if (__builtin_amdgcn_ballot_w64(!all) == 0) continue;
+    for (int i = 0; i < 16; ++i) all &= holds(acc[t][i]);
+    if (__builtin_amdgcn_ballot_w64(all == 0) == 0) continue;
     f32x16_t again;
 #pragma unroll
     for (int i = 0; i < 16; ++i) again[i] = 0.0f;

@@ -193,6 +193,21 @@ def binary32_product(awq, lib, dev, w, x, floats):
     return dev.host(y)
 
 
+# Operands whose last bits are below bfloat16's range, 2^-133.  288 instructions of two products, each rounding their sum and partial sums that are
+# sqrt(i / 288) of the result's rms in the mean square: sqrt(288) x 2^-24 at most.
+@pytest.mark.parametrize("tokens,rows", [(5, 300), (70, 300), (300, 1100)])
+@pytest.mark.parametrize("of_w,of_x", [(0, -110), (0, -118), (0, -124), (-120, 0), (-60, -60)])
+def test_binary32_products_of_tiny_operands(awq, lib, dev, tokens, rows, of_w, of_x):
+    print("tiny operands", tokens, rows, of_w, of_x, flush=True)
+    rng = np.random.default_rng(rows)
+    w = (rng.standard_normal((rows, 576)) * 2.0 ** of_w).astype(np.float32)
+    x = (rng.standard_normal((tokens, 576)) * 2.0 ** of_x).astype(np.float32)
+    want = x.astype(np.float64) @ w.T.astype(np.float64)
+    for floats in (0, 1 << 22):
+        off = binary32_product(awq, lib, dev, w, x, floats) - want
+        assert np.sqrt(np.mean(off ** 2)) < 288 ** 0.5 * 2.0 ** -24 * np.sqrt(np.mean(want ** 2))
+
+
 # A product of two binary32 numbers rounds by 2^-24 of itself; their bfloat16 terms' sums by 2^-24 of what is 2^-6 of it, five times, and
 # what is left out is 2^-30: an eighth more.  Where all terms have one sign, what were left out of the products would add up: roundings
 # go either way, and the mean of many outputs' errors is far below one.  0x3f80ffff has the largest second and third terms.
