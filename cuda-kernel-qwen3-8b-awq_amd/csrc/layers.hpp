@@ -226,6 +226,7 @@ int64_t window_parts_floats(int32_t heads, int32_t vdim, int64_t window, int64_t
 // beside (where window_takes_product): a product in the same launch.
 int launch_window_attention(const WindowAttnArgs& a, bool f32, hipStream_t st, const DenseArgs* beside = nullptr);
 bool window_takes_product(const WindowAttnArgs& a, bool f32);
+bool window_few_queries(const WindowAttnArgs& a);  // binary32, several tokens: on vector instructions
 
 // --- linear attention with a decaying state (linear_attention.hip) -------------------------------------------
 // per head S <- decay S + k v^T, o = S^T q; state [heads][vdim][round_up(dim, 64)] float (S transposed), zero ahead of

@@ -612,23 +612,29 @@ void launch_tiles(const WindowAttnArgs& a, hipStream_t st) {
 //     O^T[col][query] += V^T P^T      instruction (b, j) takes column DV / 16 r + b of key 4 c + j, whose weight the lane has just formed
 // A value is not in the sums of a query that does not see it, and a query's bits are its own: they do not depend on the queries beside
 // it, nor, without a window, on where the pass begins.
-// Bound by the matrix cores' binary32 rate and, for few queries, by the trips to the cache.  8 heads of 128, the appending launch
-// included, us, and before a few queries at a time by vector instructions (window_query_kernel): 333 queries 24 (44), 512 30 (61), of 12 heads 46 (84), 333 of 32
-// heads of 64 33 (83), 333 behind 3,000 keys in a window of 1,024 43 (105), 2 queries there 37 (39); 4 queries alone 10.1 (8.8), 64 11.7 (10.9).
+// Bound by the matrix cores' binary32 rate and, for few queries, by the trips to the cache.  All eight wavefronts add the parts up at
+// the end, four columns of a query a thread: by one of them, with 32 divisions a lane, 8 heads of 128 took 0.4 to 1.2 us more.
+// us, the appending launch included, beside a few queries at a time by vector instructions (window_query_kernel):
+//   8 heads of 128, from position 0    333 queries 22 (42)      512 queries 27 (59)
+//   12 heads of 128, from position 0   512 queries 43 (84)
+//   32 heads of 64, from position 0    333 queries 31 (80)
+//   8 heads of 128 behind 3,000 keys, window 1,024   333 queries 39 (106)   2 queries 34.5 (38.5)
+//   8 heads of 128, from position 0    4 queries 8.5 (8.0)      64 queries 10.6 (10.0)
+//   8 heads of 128 behind 150 keys     4 queries 13.5 (12.3)    32 queries 14.6 (12.7)      (window_few_queries)
 template <int DK, int DV>
 __global__ __launch_bounds__(512) void window_tile_f32_kernel(WindowAttnArgs a) {
   constexpr int KQ = DK / 16, VB = DV / 16, NW = 8;
   constexpr int PARTS = 16;  // of a score: chains of four or eight products, which round no more than a lane's share and a tree
   __shared__ float most[NW][16], sums[NW][16];
-  __shared__ __attribute__((aligned(16))) float held[NW - 1][16 * DV];
+  constexpr int STRIDE = DV + 4;
+  __shared__ __attribute__((aligned(16))) float held[NW][16 * STRIDE];
   const int h = blockIdx.x, g = h / (a.heads / a.kv_heads), tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, c = lane >> 4;
   const int M = (int)a.M, pos0 = a.pos.pos0, q0 = blockIdx.y * 16, qi = q0 + r, qc = min(qi, M - 1), pq = pos0 + qc;
   auto oldest = [&](int p) { return a.window > 0 ? max(0, p - a.window + 1) : 0; };
   const int first = pos0 + q0, last = pos0 + min(q0 + 15, M - 1), lo_q = oldest(pq);
   const int k_begin = oldest(first) & ~15, k_end = last + 1;
-  const int busy = min(NW, (k_end - k_begin + 15) >> 4);  // wavefronts that have a tile; the others are not waited for
-  if (wave >= busy) return;
+  const int busy = min(NW, (k_end - k_begin + 15) >> 4);  // wavefronts that have a tile
   const float* const q = reinterpret_cast<const float*>(a.proj) + (int64_t)qc * a.ldp + (int64_t)h * a.dim;
   f32x4_t qv[KQ];
 #pragma unroll
@@ -755,36 +761,35 @@ __global__ __launch_bounds__(512) void window_tile_f32_kernel(WindowAttnArgs a) 
   float all = most[0][r];
   for (int w = 1; w < busy; ++w) all = fmaxf(all, most[w][r]);
   const auto factor = [&](float x) { return x > -INFINITY ? expf(x - all) : 0.0f; };
-  const float mine = factor(m);
+  if (wave < busy) {
+    const float mine = factor(m);
+    float* const to = held[wave] + r * STRIDE + 4 * VB * c;
 #pragma unroll
-  for (int b = 0; b < VB; ++b) {
-    acc[b] = acc[b] * mine;
-    if (wave > 0) *reinterpret_cast<f32x4_t*>(held[wave - 1] + (b * 64 + lane) * 4) = acc[b];
+    for (int b = 0; b < VB; ++b) acc[b] = acc[b] * mine;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int b = 0; b < VB; b += 4) *reinterpret_cast<f32x4_t*>(to + VB * j + b) = f32x4_t{acc[b][j], acc[b + 1][j], acc[b + 2][j], acc[b + 3][j]};
   }
   __syncthreads();
-  if (wave > 0 || qi >= M) return;
-  float total = 0.0f;
-  for (int w = 0; w < busy; ++w) total = __builtin_fmaf(factor(most[w][r]), sums[w][r], total);
-  float* const out = reinterpret_cast<float*>(a.ctx) + (int64_t)qi * a.ldc + (int64_t)h * a.vdim;
-  for (int w = 1; w < busy; ++w) {
-#pragma unroll
-    for (int b = 0; b < VB; ++b) acc[b] = acc[b] + *reinterpret_cast<const f32x4_t*>(held[w - 1] + (b * 64 + lane) * 4);
+  // all wavefronts add the parts up, four columns of a query a thread
+  const int of = tid / (DV / 4), col = 4 * (tid % (DV / 4));
+  if (of >= 16 || q0 + of >= M) return;
+  float top = most[0][of], total = 0.0f;
+  for (int w = 1; w < busy; ++w) top = fmaxf(top, most[w][of]);
+  f32x4_t sum = *reinterpret_cast<const f32x4_t*>(held[0] + of * STRIDE + col);
+  for (int w = 0; w < busy; ++w) {
+    total = __builtin_fmaf(most[w][of] > -INFINITY ? expf(most[w][of] - top) : 0.0f, sums[w][of], total);
+    if (w > 0) sum = sum + *reinterpret_cast<const f32x4_t*>(held[w] + of * STRIDE + col);
   }
+  sum = sum / total;
+  float* const out = reinterpret_cast<float*>(a.ctx) + (int64_t)(q0 + of) * a.ldc + (int64_t)h * a.vdim;
+  if (col + 3 < a.vdim) {
+    *reinterpret_cast<f32x4u_t*>(out + col) = sum;
+  } else {
 #pragma unroll
-  for (int b = 0; b < VB; ++b) acc[b] = acc[b] / total;
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int col = VB * (4 * c + j);
-#pragma unroll
-    for (int b = 0; b < VB; b += 4) {
-      if (col + b + 3 < a.vdim) {
-        *reinterpret_cast<f32x4u_t*>(out + col + b) = f32x4_t{acc[b][j], acc[b + 1][j], acc[b + 2][j], acc[b + 3][j]};
-      } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (col + b + e < a.vdim) out[col + b + e] = acc[b + e][j];
-      }
-    }
+    for (int e = 0; e < 4; ++e)
+      if (col + e < a.vdim) out[col + e] = sum[e];
   }
 }
 
@@ -850,6 +855,15 @@ int64_t window_parts_floats(int32_t heads, int32_t vdim, int64_t window, int64_t
 
 static bool one_token_form(const WindowAttnArgs& a) { return a.kl.row <= 256 && a.vl.row <= 256 && a.M == 1 && a.parts && a.len_bound > 0; }
 
+// Few queries on few keys in binary32: a tile of sixteen queries keeps a compute unit's matrix cores busy for all of them, vector
+// instructions form what there is.  Up to 384 rows (query, head) and 320 keys of heads of 65 to 128 values they take 0 to 15 % less
+// (5 % more at worst: 12 heads, 32 queries from position 0); above, 8 heads, 64 queries and 64 keys 10.0 us against 10.6, 100 and 148
+// 15.4 against 14.6.  Heads of up to 64 are half the tile's work: 32 of them, 4 queries, 7.7 us against 6.8.  Not without a window:
+// there a query's bits do not depend on the pass that it comes in.
+bool window_few_queries(const WindowAttnArgs& a) {
+  return a.window > 0 && a.kl.row == 128 && a.vl.row == 128 && a.heads * a.M <= 384 && std::min<int64_t>(a.pos.pos0, a.window - 1) + a.M <= 320;
+}
+
 bool window_takes_product(const WindowAttnArgs& a, bool f32) { return !f32 && one_token_form(a); }
 
 int launch_window_attention(const WindowAttnArgs& a, bool f32, hipStream_t st, const DenseArgs* beside) {
@@ -863,7 +877,7 @@ int launch_window_attention(const WindowAttnArgs& a, bool f32, hipStream_t st, c
   if (one_token_form(a)) return f32 ? launch_decode<float>(a, st, nullptr) : launch_decode<bf16_t>(a, st, beside);
   if (int rc = f32 ? launch_append<float>(a, st) : launch_append<bf16_t>(a, st)) return rc;
   if (f32) {
-    if (a.kl.row > 128 || a.vl.row > 128 || a.pos.dyn) return launch_queries<float>(a, st);
+    if (a.kl.row > 128 || a.vl.row > 128 || a.pos.dyn || window_few_queries(a)) return launch_queries<float>(a, st);
     if (a.kl.row == 64) launch_tiles_f32<64>(a, st);
     else launch_tiles_f32<128>(a, st);
     AWQ_HIP_TRY(hipGetLastError());

@@ -726,6 +726,13 @@ def test_roundings_of_window_attention(awq, lib, dev, heads, kv, dim, vdim, size
     assert off < 20 * 2.0 ** -24
 
 
+@pytest.mark.parametrize("sizes", [[2, 47], [48, 49, 3], [50, 1, 48]], ids=str)
+@pytest.mark.parametrize("window", [40, 270, 280, 300])
+def test_few_queries_of_a_window_and_more(awq, lib, dev, sizes, window):
+    """portions beside the line between the two forms, 384 rows and 320 keys; the bound is that of the test above"""
+    test_roundings_of_window_attention(awq, lib, dev, 8, 2, 128, 100, sizes, window)
+
+
 @pytest.mark.parametrize("f32", FORMATS, ids=["bf16", "f32"])
 @pytest.mark.parametrize("window", [1, 2, 31, 32, 33, 64, 65, 96, 128, 160])
 def test_window_edges(awq, lib, dev, f32, window):
