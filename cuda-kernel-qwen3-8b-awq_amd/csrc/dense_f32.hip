@@ -151,7 +151,8 @@ __device__ __forceinline__ Split4 split4(f32x4_t v) {
 // is cut over `cuts` workgroups and a second launch adds their sums, as in bfloat16.
 // Bound by the splitting (vector instructions) beside the matrix cores, at few tokens by the weights' bytes.  333 tokens, us, on
 // v_mfma_f32_32x32x2_f32 before, weights that are bfloat16 numbers, and weights that are not: 1,024 rows of 4,096 inputs 40, 27, 39;
-// 7,168 of 1,024 58, 34, 57; 32,768 of 1,024 220, 111, 207.  Up to 50 tokens weights that are not take up to 11 % more than before.
+// 7,168 of 1,024 58, 34, 57; 32,768 of 1,024 220, 111, 207.  Up to 64 tokens weights that are not take more than before,
+// up to 15 % with 256 inputs and 11 % with more, weights that are mostly less (1,024 x 4,096, 33 tokens: 18.0, 17.3 and 18.2 us).
 // Off from 64 bits (norm) by 0.8e-7 to 1.8e-7 with 300 to 1,024 rows of 64 to 4,096 inputs, either way; before 1.1e-7 to 2.2e-7.
 // An infinity has no such terms (what it leaves is NaN), and numbers below 2^-110 not all of theirs: a wavefront that finds sums that
 // are not finite, or other than zero and below 2^-100, forms them again, in binary32.  (Inputs of 2^-115 were off by 37 x 2^-24 of the
@@ -359,13 +360,15 @@ constexpr Form kForm[kForms] = {{64, 32, 0.4714f, 0.2758f, 0.0706f}, {64, 64, 0.
 
 // The time of a product in us, but for what all forms of it share: what the choice of a form and of a number of shares of k needs.  Fitted
 // for the choice, not for the time, to 5,997 timings (20 shapes from 256 x 256 to 32,768 x 1,024, 2 to 512 tokens, 1 to 16 shares; weights that
-// are bfloat16 numbers).  The form it picks takes 0.8 % longer on average than the fastest timed, 11 % at the 99th of 100.
+// are bfloat16 numbers).  The 0.25 us of a share is fitted apart, to 700 products (50 shapes, 8 to 333 tokens, weights of either kind, all
+// forms timed): with 0.37, as the fit of all gave it, 1,024 x 4,096 at 33 to 64 tokens went in 8 shares instead of 16 and took 6 to 9 %
+// longer.  The form it picks takes 0.8 % longer on average than the fastest timed, 11 % at the 99th of 100.
 float many_time(const DenseArgs& a, int64_t rows, const Form& f, int64_t cuts) {
   const float steps = (float)(((a.k >> 5) + cuts - 1) / cuts);
   const float per_unit = ceilf((float)(rows / f.rows * ((a.M + f.tokens - 1) / f.tokens) * cuts * a.batch) / 256.0f);
   float t = std::max(steps * f.alone, (float)rows * (float)a.k * (float)a.batch * 4.0f / 7.169e6f);
   if (per_unit > 1.0f) t = std::max(t, steps * f.beside * per_unit);
-  if (cuts > 1) return t + 2.743f + (float)cuts * (0.3704f + (float)a.M * (float)rows * 8.0f / 4.476e6f);
+  if (cuts > 1) return t + 2.743f + (float)cuts * (0.25f + (float)a.M * (float)rows * 8.0f / 4.476e6f);
   return t + per_unit * f.end;
 }
 
@@ -383,19 +386,27 @@ int launch_tiles(const DenseArgs& a, int64_t rows, int form, int tok_tiles, int 
   return AWQ_OK;
 }
 
-template <int OUT>
-int launch_many(const DenseArgs& a, int64_t rows, hipStream_t st) {
+struct Choice {
+  int form = 0;
+  int64_t cuts = 1;
+};
+Choice choose(const DenseArgs& a, int64_t rows) {
   int64_t most = 1;  // shares of k: at least four steps each
   if (a.workspace && a.batch == 1 && a.M <= 65535)
     most = std::max<int64_t>(1, std::min(std::min<int64_t>(16, a.k >> 7), a.workspace_floats / (a.M * rows)));
-  int form = 0;
-  int64_t cuts = 1;
+  Choice best_of;
   float best = HUGE_VALF;
   for (int f = 0; f < kForms; ++f)
     for (int64_t c = 1; c <= most; ++c) {
       const float time = many_time(a, rows, kForm[f], c);
-      if (time < best) best = time, form = f, cuts = c;
+      if (time < best) best = time, best_of = Choice{f, c};
     }
+  return best_of;
+}
+
+template <int OUT>
+int launch_many(const DenseArgs& a, int64_t rows, hipStream_t st) {
+  const auto [form, cuts] = choose(a, rows);
   const int64_t tok_tiles = (a.M + kForm[form].tokens - 1) / kForm[form].tokens, tiles = rows / 64 * tok_tiles;
   AWQ_REQUIRE(tiles < (1ll << 26), "too large");
   if (cuts == 1) return launch_tiles<OUT, false>(a, rows, form, (int)tok_tiles, 1, st);
@@ -435,6 +446,11 @@ int launch_dense_one_joined_f32(const DenseArgs& a, const JoinArgs& j, int64_t r
   else launch(std::integral_constant<int, 2>{});
   AWQ_HIP_TRY(hipGetLastError());
   return AWQ_OK;
+}
+
+DenseForm dense_form_f32(const DenseArgs& a, int64_t rows) {
+  const Choice c = choose(a, rows);
+  return DenseForm{kForm[c.form].tokens / 32, kForm[c.form].rows / 64, (int32_t)c.cuts};
 }
 
 int launch_dense_many_f32(const DenseArgs& a, int64_t rows, hipStream_t st) {

@@ -147,6 +147,7 @@ struct DenseForm {
   int32_t tt = 0, rb = 0, cuts = 1;
 };
 DenseForm dense_form(const DenseArgs& a, int64_t rows);
+DenseForm dense_form_f32(const DenseArgs& a, int64_t rows);  // binary32, rb in 64 rows
 bool dense_norm_fused(const NormConvArgs& n, bool f32);
 bool dense_gate_fused(int64_t n, int64_t k_padded, int64_t M, bool f32);
 

@@ -153,3 +153,12 @@ def test_forms_that_are_near_the_fastest(lib, tmp_path):
             (4096, 512, 1500): [(2, 1)]}
     for shape, form in zip(near, forms_of(tmp_path, near)):
         assert form[:2] in near[shape], shape
+
+
+def test_shares_of_binary32_products(lib, tmp_path):
+    """timed within 5 % of the fastest form, weights of either kind; 8 shares instead of the first three's, or none, were 6 to 13 % behind it"""
+    shapes = {(1024, 4096, 33): 16, (1024, 4096, 64): 16, (2048, 4096, 8): 13, (4096, 512, 48): 4, (7168, 512, 32): 4}
+    calls = "".join("{ DenseArgs a; a.k = %d; a.M = %d; a.out = DENSE_F32; a.workspace = (float*)16; a.workspace_floats = 1 << 25;"
+                    " const DenseForm f = dense_form_f32(a, %d); printf(\"%%d %%d %%d\\n\", f.tt, f.rb, f.cuts); }" % (k, m, r) for r, k, m in shapes)
+    got = host_program(tmp_path, "#include <stdio.h>\n#include \"layers.hpp\"\nint main() { %s }" % calls.replace("\n", "\\n"))
+    assert got == [v for cuts in shapes.values() for v in (1, 1, cuts)]
