@@ -384,8 +384,8 @@ int KugilixEngine::run_pass(bool one, const int32_t* ids, int64_t M, PassPos pos
       }
       if (int rc = launch_dense(a, f32, stream, norm_fused ? &norm : nullptr)) return rc;
     }
-    // A single token's W_down does not wait for the mixer: it is part of the mixer's launch, which leaves most of the device idle, and
-    // W_o alone follows.  With [W_o | W_down] behind the mixer and so: width 1,024, 16 tokens after 9, 2,648 and 2,566 us, 2,048, 32 after
+    // A single token's W_down does not wait for the mixer: it is part of the mixer's launch, where that leaves the device room, and W_o
+    // alone follows.  With [W_o | W_down] behind the mixer and so: width 1,024, 16 tokens after 9, 2,648 and 2,566 us, 2,048, 32 after
     // 100, 9,355 and 9,032, 4,096 20,380 and 19,825.
     DenseArgs down;
     down.w = (const char*)L.w_out + L.mixed_k * 32 * unit();  // (blocks of 32 rows)
@@ -426,7 +426,7 @@ int KugilixEngine::run_pass(bool one, const int32_t* ids, int64_t M, PassPos pos
       a.parts = attn_parts;
       a.done = attn_done;
       a.len_bound = (int32_t)max_pos;
-      beside = s.ff && window_takes_product(a, f32);
+      beside = s.ff && window_takes_product(a, f32, down.k * W);
       if (int rc = launch_window_attention(a, f32, stream, beside ? &down : nullptr)) return rc;
     } else {
       LinearAttnArgs a;

@@ -226,7 +226,7 @@ int64_t window_parts_floats(int32_t heads, int32_t vdim, int64_t window, int64_t
 // not so in bfloat16 tiles of 64 queries (heads of up to 256), where a value meets queries of its tile with weight zero.
 // beside (where window_takes_product): a product in the same launch.
 int launch_window_attention(const WindowAttnArgs& a, bool f32, hipStream_t st, const DenseArgs* beside = nullptr);
-bool window_takes_product(const WindowAttnArgs& a, bool f32);
+bool window_takes_product(const WindowAttnArgs& a, bool f32, int64_t weights);
 bool window_few_queries(const WindowAttnArgs& a);  // binary32, several tokens: on vector instructions
 
 // --- linear attention with a decaying state (linear_attention.hip) -------------------------------------------

@@ -383,6 +383,9 @@ int launch_decode_beside(const WindowAttnArgs& a, int chunks, int parts, size_t 
   return AWQ_OK;
 }
 
+// query heads of a workgroup
+int decode_heads(int per_group) { return per_group <= 2 ? per_group : per_group <= 4 ? 4 : 8; }
+
 template <typename T, int R, bool SAME>
 int launch_decode_parts(const WindowAttnArgs& a, int parts, const DenseArgs* beside, hipStream_t st) {
   const int chunks = (a.heads / a.kv_heads + R - 1) / R;
@@ -406,11 +409,11 @@ template <typename T>
 int launch_decode(const WindowAttnArgs& a, hipStream_t st, const DenseArgs* beside) {
   const int parts = window_parts(a.window, a.len_bound);
   AWQ_REQUIRE(parts >= 1 && parts <= 65535, "too many keys");
-  const int per = a.heads / a.kv_heads;
+  const int at_once = decode_heads(a.heads / a.kv_heads);
   const bool same = a.done && window_counted_parts(a.heads, a.kv_heads, a.window, a.len_bound);
   const auto launch = same ? launch_decode_parts<T, 1, true>
-                           : per == 1 ? launch_decode_parts<T, 1, false>
-                                      : per == 2 ? launch_decode_parts<T, 2, false> : per <= 4 ? launch_decode_parts<T, 4, false> : launch_decode_parts<T, 8, false>;
+                           : at_once == 1 ? launch_decode_parts<T, 1, false>
+                                          : at_once == 2 ? launch_decode_parts<T, 2, false> : at_once == 4 ? launch_decode_parts<T, 4, false> : launch_decode_parts<T, 8, false>;
   if (int rc = launch(a, parts, beside, st)) return rc;
   AWQ_HIP_TRY(hipGetLastError());
   if (parts > 1 && !same) {
@@ -864,7 +867,17 @@ bool window_few_queries(const WindowAttnArgs& a) {
   return a.window > 0 && a.kl.row == 128 && a.vl.row == 128 && a.heads * a.M <= 384 && std::min<int64_t>(a.pos.pos0, a.window - 1) + a.M <= 320;
 }
 
-bool window_takes_product(const WindowAttnArgs& a, bool f32) { return !f32 && one_token_form(a); }
+// Where few workgroups attend: there is one for each part of what the sequence may hold, so most of a long one's without a window
+// find nothing to do, and the product's stand behind all of them.  Kugilix, 32 tokens behind 9, us, with [W_o | W_down] behind the
+// mixer and with W_down in its launch: width 4,096 (50 M weights), window 1,024 (512 attend) 19,851 and 19,154; no window, 2,048 positions
+// (1,024) 19,862 and 20,414, 32,768 (16,384) 19,937 and 21,519.  Width 2,048 (13 M): 2,048 positions (512) 9,156 and 8,816, 4,096 (1,024)
+// 9,099 and 8,834 (behind 3,500 10,115 and 10,164), 32,768 (8,192) 9,100 and 9,458.  With the product's workgroups ahead: 19,386 with the window.
+bool window_takes_product(const WindowAttnArgs& a, bool f32, int64_t weights) {
+  if (f32 || !one_token_form(a)) return false;
+  const int per = a.heads / a.kv_heads, at_once = decode_heads(per);
+  const int64_t attend = (int64_t)a.kv_heads * ((per + at_once - 1) / at_once) * window_parts(a.window, a.len_bound);
+  return attend <= 512 || (attend <= 1024 && weights <= 16 << 20);
+}
 
 int launch_window_attention(const WindowAttnArgs& a, bool f32, hipStream_t st, const DenseArgs* beside) {
   AWQ_REQUIRE(a.proj && a.k_cache && a.v_cache && a.ctx && a.slope && a.M >= 1 && a.M <= 65535, "bad arguments");
@@ -873,7 +886,7 @@ int launch_window_attention(const WindowAttnArgs& a, bool f32, hipStream_t st, c
   AWQ_REQUIRE(a.kl.slots > 0 && a.kl.slots % 64 == 0 && a.vl.slots == a.kl.slots && a.kl.row == window_row_padded(a.dim) &&
                   a.vl.row == window_row_padded(a.vdim) && a.ldp % 8 == 0 && a.ldc % 8 == 0,
               "bad cache layout");
-  AWQ_REQUIRE(!beside || window_takes_product(a, f32), "no product beside this attention");
+  AWQ_REQUIRE(!beside || window_takes_product(a, f32, beside->k * beside->seg[0].rows), "no product beside this attention");
   if (one_token_form(a)) return f32 ? launch_decode<float>(a, st, nullptr) : launch_decode<bf16_t>(a, st, beside);
   if (int rc = f32 ? launch_append<float>(a, st) : launch_append<bf16_t>(a, st)) return rc;
   if (f32) {

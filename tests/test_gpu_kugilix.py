@@ -157,6 +157,26 @@ def test_single_tokens_with_the_second_matrix_beside_the_mixer(awq, torch_gpu, t
     eng.close()
 
 
+# 512, 1,024 and 1,088 workgroups attend: the second matrix in their launch, and behind it with W_o
+@pytest.mark.parametrize("max_positions", [2048, 4096, 4160])
+def test_single_tokens_of_sequences_that_may_grow_long(awq, torch_gpu, tmp_path, max_positions):
+    cfg = km.model(96, 64, [km.attention(16, 16, 16, 16, None, ff=300)], groups=2, taps=4, loop=(0, 1, 2))
+    w = km.weights(cfg, 396)
+    km.write(str(tmp_path), cfg, w)
+    tokens = np.random.default_rng(4).integers(0, 64, 70).tolist()
+    taps = []
+    plain.forward(cfg, w, tokens, taps)
+    eng = awq.open_model(str(tmp_path), max_positions=max_positions)
+    eng.set_layer_tap(True)
+    eng.forward(tokens[:62])
+    for t in range(62, 70):
+        eng.forward(tokens[t:t + 1])
+        got = eng.read_layer_tap().reshape(len(taps), 96)
+        for i in range(len(taps)):
+            assert km.rms_error(got[i], taps[i][t]) < LIMIT["bfloat16"], "layer run %d, token %d" % (i, t)
+    eng.close()
+
+
 def test_long_sequence_in_wrapping_rings(awq, torch_gpu, tmp_path):
     """more positions than a ring holds: a window behind one pass of 2048"""
     cfg = km.model(32, 64, [km.attention(2, 1, 16, 8, 9, ff=32), km.lightning(1, 8, 8, [0.99])], groups=2, taps=2)
