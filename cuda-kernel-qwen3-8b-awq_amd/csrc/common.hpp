@@ -147,6 +147,8 @@ int64_t gemv_workspace_bytes(int64_t m, int64_t k);
 int launch_gemv(const LinearArgs& a, hipStream_t st);
 int64_t gemm_workspace_bytes(int64_t m, int64_t k, int64_t M);
 int gemm_plan(int64_t m, int64_t k, int64_t M, int has_workspace);
+int gemm_panel_rows(int64_t m, int64_t k, int64_t M, int has_workspace);  // 17..64 tokens: rows per workgroup of gemm_panel_kernel; 0: not by it
+int gemm_norm_shares64(int64_t m, int64_t k, int64_t M);  // where gemm_norm_shares has none: of tiles of 64 tokens
 int gemm_norm_shares(int64_t m, int64_t k, int64_t M);  // shares of k where the norm of the rows is asked for too; 0: as gemm_plan
 // The RMS norm of the product's rows, for the launch that follows: where a launch adds partial sums it is done there (`done`),
 // else it is left to the caller.

@@ -1274,17 +1274,19 @@ constexpr int panel_behind(int c, int nc, int na, int wa, int tokens, int weight
   return behind;
 }
 
-// 17..64 tokens: a stream of weights, beside which every workgroup reads all tokens' inputs of its k.  A workgroup of eight wavefronts takes RG
-// row groups and all of k or a share, a wavefront an eighth of that in NC chunks of 64 inputs.  A wavefront's weights and
-// the tokens' inputs that they meet are its own, so that nothing waits for another wavefront until the sums meet in LDS: the tokens
-// go straight into a ring of NS places of its own (global_load_lds, 128 bytes per token and chunk, the eight 16-byte pieces of row r at
-// positions c ^ (r / 2 & 7)), the weights into registers, requested in the order of their use NS and WA chunks ahead (up to 32 tokens two
-// and four chunks are enough, and more of them only delay the first; beyond, all weights at the start).  Lane (q, r) holds dwords
-// 2 (q % 2) and + 1 of row r of block q / 2 of the chunk (one 8-byte request) and reads the token pieces 2 q and 2 q + 1;
-// v_mfma_f32_16x16x32_f16 with the tokens as the first operand, so that 33 to 48 are three tiles and not four.  As many row groups as
-// leave one workgroup per compute unit.  Loads and nothing else take 85 to 90 % of its time.  17, 24, 40, 48, 64 tokens, us: 12,288 x 4,096 9.3, 9.5,
-// 12.0, 12.3, 14.0 (gemm_shared32_kernel, 192 workgroups: 11.0, 10.5, 14.1, 14.2, 14.4), 4,096 x 4,096 5.9, 6.1, 7.5, 7.8, 8.8
-// (gemm_shared_kernel 6.5, 6.4, 8.4, 8.5, 8.9), 4,096 x 12,288 with k over four workgroups and the launch that adds at 17, 24, 48 11.8, 12.3, 16.3 (12.9, 13.0, 16.6).
+// 17..64 tokens: a stream of weights, beside which every workgroup reads all tokens' inputs of its k.  A workgroup of eight
+// wavefronts takes RG row groups and all of k or a share, a wavefront an eighth of that in NC chunks of 64 inputs.  A wavefront's
+// weights and the tokens' inputs that they meet are its own, so that nothing waits for another wavefront until the sums meet in LDS.
+// The tokens go straight into a ring of NS places of its own (global_load_lds, 128 bytes per token and chunk, the eight 16-byte
+// pieces of row r at positions c ^ (r / 2 & 7)), the weights into registers, requested in the order of their use NS and WA chunks
+// ahead.  (Up to 32 tokens two and four chunks are enough, and more of them only delay the first; beyond, all weights at the start.)
+// Lane (q, r) holds dwords 2 (q % 2) and + 1 of row r of block q / 2 of the chunk, one 8-byte request, and reads the token pieces 2 q
+// and 2 q + 1; v_mfma_f32_16x16x32_f16 with the tokens as the first operand, so that 33 to 48 are three tiles and not four.  As many
+// row groups as leave one workgroup per compute unit (panel_form).  Loads and nothing else take 85 to 90 % of its time.
+// us, and by the kernel that took the product before:  17            24            40            48            64 tokens
+//   12,288 x 4,096 (gemm_shared32_kernel)             9.3  11.0     9.5  10.5    12.0  14.1    12.3  14.2    14.0  14.4
+//   4,096 x 4,096 (gemm_shared_kernel)                5.9   6.5     6.1   6.4     7.5   8.4     7.8   8.5     8.8   8.9
+//   4,096 x 12,288, the launch that adds included    11.8  12.9    12.3  13.0    15.7  16.7    16.3  16.6
 constexpr int panel_places(int tt) { return tt == 3 ? 3 : 2; }
 template <int RG, int TT, int NC, bool ZINT>
 __global__ __launch_bounds__(512, 2) void gemm_panel_kernel(GemmParams p, int n_rg) {
@@ -1652,19 +1654,33 @@ int launch_shared32(const GemmParams& p, bool zint, hipStream_t st) {
   return AWQ_OK;
 }
 
-// 17..64 tokens where gemm_panel_kernel is the faster one (times there): row groups per workgroup, and workgroups that share k; 0: another
-// kernel takes the product.  16,384 x 4,096 where it has three tiles of tokens only (40 tokens: 14.1 us against 15.4; 64: 16.9 against
-// 15.7), 4,096 x 12,288 up to 48 tokens (64: 18.1 against 17.9).
+// 17..64 tokens by gemm_panel_kernel: row groups per workgroup, and workgroups that share k; 0: another kernel takes the product.  A
+// workgroup for each compute unit: as many row groups as leave 256 of them, up to the four whose sums a wavefront holds.  k of 2,048 and
+// 4,096 in one workgroup, as gemm_shared_kernel and gemm_shared32_kernel have it, and of 12,288 over four, as gemm_shared32_kernel has it
+// from 128 tokens on; there is no instance for another k.  Up to 48 tokens it is the fastest wherever it was timed (128 to 16,384 rows),
+// but for 17 to 32 tokens of 10,240 rows and more of 2,048 inputs, whose weights are there before the tokens: 14,336 rows, 32 tokens 7.3 us
+// by gemm_shared32_kernel, 7.8.  The fourth tile of 16 tokens pays on fewer shapes.  us, other kernel and this one:
+//                         17            32            48            64 tokens
+//   2,048 x 4,096     7.8   5.7     8.6   6.7     8.6   7.6     8.9   8.8     (1,024 rows  8.3  8.6: not taken)
+//   8,192 x 4,096    10.8   8.5    11.0   9.1    14.5  10.2    15.6  11.5
+//   16,384 x 4,096   13.2  12.3    12.5  12.5    16.7  15.6    17.1  18.1: not taken
+//   2,048 x 2,048     6.7   4.1     7.2   4.4     7.5   5.4     7.8   6.2     (6,144 rows  7.2  7.6: not taken)
+//   2,048 x 12,288   11.9   9.6    12.4  10.5    15.5  12.0    16.3  13.3     (4,096 rows 18.5 18.9: not taken)
 struct PanelForm {
   int rg, kz;
 };
 static PanelForm panel_form(int64_t m, int64_t k, int64_t M, bool has_workspace) {
-  if (M < 17 || M > 64) return {0, 0};
-  if (k == 4096 && m == 4096) return {1, 1};
-  if (k == 4096 && m == 12288) return {3, 1};
-  if (k == 4096 && m == 16384 && M > 32 && M <= 48) return {4, 1};
-  if (k == 12288 && m == 4096 && M <= 48 && has_workspace) return {4, 4};
-  return {0, 0};
+  const bool cut = k == 12288;
+  if (M < 17 || M > 64 || (k != 2048 && k != 4096 && !(cut && has_workspace))) return {0, 0};
+  const int kz = cut ? 4 : 1;
+  const int64_t rg = (m / 16 * kz + 255) / 256;
+  bool takes = rg <= 4;
+  if (M <= 32 && k == 2048) takes = rg <= 2;
+  if (M > 48) takes = cut ? rg <= 3 : k == 4096 ? m >= 2048 && rg <= 3 : m <= 2048;
+  return takes ? PanelForm{(int)rg, kz} : PanelForm{0, 0};
+}
+int gemm_panel_rows(int64_t m, int64_t k, int64_t M, int has_workspace) {
+  return mid_row_groups(m, k, M) ? 0 : 16 * panel_form(m, k, M, has_workspace != 0).rg;
 }
 template <int RG, int TT, int NC>
 int launch_panel(const GemmParams& p, bool zint, hipStream_t st) {
@@ -1691,7 +1707,15 @@ template <int RG, int NC>
 int launch_panel_tokens(const GemmParams& p, bool zint, hipStream_t st) {
   if (p.M <= 32) return launch_panel<RG, 2, NC>(p, zint, st);
   if (p.M <= 48) return launch_panel<RG, 3, NC>(p, zint, st);
-  return launch_panel<RG, 4, NC>(p, zint, st);
+  if constexpr (RG <= 3) return launch_panel<RG, 4, NC>(p, zint, st);
+  AWQ_REQUIRE(false, "no such panel");
+}
+template <int NC>
+int launch_panel_rows(const GemmParams& p, int rg, bool zint, hipStream_t st) {
+  if (rg == 1) return launch_panel_tokens<1, NC>(p, zint, st);
+  if (rg == 2) return launch_panel_tokens<2, NC>(p, zint, st);
+  if (rg == 3) return launch_panel_tokens<3, NC>(p, zint, st);
+  return launch_panel_tokens<4, NC>(p, zint, st);
 }
 
 // Which workgroup shape a many-token product takes (measured on the three matrix shapes of the
@@ -1737,11 +1761,14 @@ int gemm_norm_shares(int64_t m, int64_t k, int64_t M) {
   return tiles * 3 <= 2 * kSkWgs ? 3 : 0;
 }
 
-// The same with tiles of 64 tokens, where those of 128 are too few: shares that give 192 of the compute units a workgroup, of at most 4.  The
-// norm has its launch's trip in common with the sums, and a workgroup has eight wavefronts (halves_pay).  Prompts of 36 layers, ms, without and
-// with it for 4,096 x 4,096 and for 4,096 x 12,288: 192 tokens 5.62, 5.36 and 5.32; 250 6.89, 6.52 and 6.61; 300 6.87, 6.64 and 6.41; 400 8.43, 8.22
-// (the second has shares of tiles of 128); 512 8.82, 8.63.  128 workgroups: 70 tokens 3.99, 4.01 and 4.11, 128 4.26, 4.23 and 4.29.
-static int norm_shares64(int64_t m, int64_t k, int64_t M) {
+// The same with tiles of 64 tokens, where those of 128 are too few: shares that give 192 of the compute units a workgroup, of at most
+// 4.  The norm has its launch's trip in common with the sums, and a workgroup has eight wavefronts (halves_pay).  Prompts of 36
+// layers, ms:                              192 tokens    250    400    512
+//   neither in such shares                    5.62       6.89   8.43   8.82
+//   4,096 x 4,096                             5.36       6.52   8.22   8.63
+//   4,096 x 12,288 (above: tiles of 128)      5.32       6.61
+// With 128 workgroups no more: 70 tokens 3.99, 4.01 and 4.11, 128 4.26, 4.23 and 4.29.
+int gemm_norm_shares64(int64_t m, int64_t k, int64_t M) {
   const int64_t tiles = (m + 255) / 256 * ((M + 63) / 64), blocks = k / AWQ_BLOCK_K;
   if (k < 4096 || m < 4096 || m > kNormRow || M < 65 || gemm_norm_shares(m, k, M)) return 0;
   for (int kz : {4, 3, 2})
@@ -1754,8 +1781,9 @@ static int norm_shares64(int64_t m, int64_t k, int64_t M) {
 // with a tile per workgroup, 3 rows split with 64 tokens per workgroup, 4 rows split with the work cut evenly,
 // 5 up to 16 tokens with several row groups per workgroup, 6 17..64 and 129..192 tokens on 4096 rows with the tokens shared
 // through LDS, 7 17..256 tokens on 10240..16384 rows the same way with 64 rows per workgroup, 8 the same with k
-// cut over four workgroups (4096 x 12288 at 128..320 tokens), 9 17..48 tokens on 4096 x 12288, a wavefront's
-// operands all its own and k cut over four workgroups.  Of 6 and 7 up to 64 tokens the kernel is that of 9 where panel_form says so
+// cut over four workgroups (4096 x 12288 at 128..320 tokens), 9 17..64 tokens on a k of 12288, a wavefront's
+// operands all its own and k cut over four workgroups.  Of 1, 6 and 7 up to 64 tokens the kernel is that of 9, without the cut, where
+// gemm_panel_rows says so: its rows per workgroup (0: it does not take the product)
 int gemm_plan(int64_t m, int64_t k, int64_t M, int has_workspace) {
   if (M >= 2 && mid_row_groups(m, k, M)) return 5;
   if (panel_form(m, k, M, has_workspace != 0).kz > 1) return 9;
@@ -1817,18 +1845,18 @@ int launch_gemm(const void* wq, const half_t* scale, const half_t* zp, int64_t m
   p.sk_part = nullptr;
   p.norm = norm;
   const bool panel_room = workspace && kSkHeaderBytes + 4 * M * m * 4 <= workspace_bytes;
-  if (const PanelForm f = panel_form(m, k, M, panel_room); f.rg) {
+  // (a norm of these rows comes with the sums of the k-split workgroups, which it costs less than a launch of its own)
+  const bool sums_normed = norm && epilogue == EPI_RESIDUAL && !shared_takes(m, k, M) && !shared32_takes(m, k, M);
+  if (const PanelForm f = panel_form(m, k, M, panel_room); f.rg && (f.kz > 1 || !sums_normed)) {
     p.kz = f.kz;
     if (f.kz > 1) p.part = (float*)((char*)workspace + kSkHeaderBytes);
-    int rc;
-    if (f.kz > 1) rc = M <= 32 ? launch_panel<4, 2, 6>(p, zp_integral, st) : launch_panel<4, 3, 6>(p, zp_integral, st);
-    else if (f.rg == 4) rc = launch_panel<4, 3, 8>(p, zp_integral, st);
-    else rc = f.rg == 3 ? launch_panel_tokens<3, 8>(p, zp_integral, st) : launch_panel_tokens<1, 8>(p, zp_integral, st);
-    if (rc) return rc;
+    if (int rc = f.kz > 1 ? launch_panel_rows<6>(p, f.rg, zp_integral, st)
+                          : k == 4096 ? launch_panel_rows<8>(p, f.rg, zp_integral, st) : launch_panel_rows<4>(p, f.rg, zp_integral, st))
+      return rc;
     AWQ_HIP_TRY(hipGetLastError());
     return AWQ_OK;
   }
-  if (const int shares = norm && epilogue == EPI_RESIDUAL && workspace ? norm_shares64(m, k, M) : 0;
+  if (const int shares = norm && epilogue == EPI_RESIDUAL && workspace ? gemm_norm_shares64(m, k, M) : 0;
       shares && kSkHeaderBytes + (int64_t)shares * M * m * 4 <= workspace_bytes) {
     p.nr = (int32_t)((m + 255) / 256);
     p.n_tiles = (int32_t)(p.nr * ((M + 63) / 64));

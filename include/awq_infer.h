@@ -343,9 +343,9 @@ int64_t awq_gemm_workspace_bytes(int64_t m, int64_t k, int64_t M);
  * streamed through LDS, 7 17 to 256 tokens on 10240 to 16384 rows the same way: 64 rows per
  * workgroup on the 32 x 32 x 16 matrix instruction, 64 tokens after the other against weights
  * that stay in registers, 8 the same with k cut over four workgroups and a second launch that adds
- * their FP32 sums (4096 x 12288 at 128 to 320 tokens; needs the workspace), 9 17 to 48 tokens on 4096 x 12288: k cut over
- * four workgroups and there over eight wavefronts, each with weights and tokens of its own (needs the workspace); 6 and 7 on
- * a k of 4096 take 17 to 64 tokens the same way, without the cut, 16 or 48 rows per workgroup. */
+ * their FP32 sums (4096 x 12288 at 128 to 320 tokens; needs the workspace), 9 17 to 64 tokens on a k of 12288: k cut over
+ * four workgroups and there over eight wavefronts, each with weights and tokens of its own (needs the workspace); 1, 6 and 7 on
+ * a k of 2048 or 4096 mostly take 17 to 64 tokens the same way, without the cut, 16 to 64 rows per workgroup. */
 int awq_gemm_plan(int64_t m, int64_t k, int64_t M, int has_workspace);
 int awq_gemm(const void* repacked, const void* scale, const void* zp, int64_t m, int64_t k, const void* x, void* y,
              int64_t M, int32_t zp_integral, void* workspace, void* stream);

@@ -823,6 +823,14 @@ def test_gemm_of_17_to_64_tokens(awq, lib, torch_gpu, m, k, M):
         assert int(d_ws[:4096].to(torch.int32).sum().item()) == 0
 
 
+# the same on other rows and other k: one to four row groups in a workgroup, 8 to 256 workgroups
+@pytest.mark.parametrize("M", [17, 33, 48, 49, 64])
+@pytest.mark.parametrize("m,k", [(128, 4096), (2048, 4096), (8192, 4096), (128, 2048), (2048, 2048), (6144, 2048), (12288, 2048), (16384, 2048), (384, 12288),
+                                 (1536, 12288), (3072, 12288)])
+def test_gemm_of_17_to_64_tokens_of_other_shapes(awq, lib, torch_gpu, m, k, M):
+    test_gemm_of_17_to_64_tokens(awq, lib, torch_gpu, m, k, M)
+
+
 # a workgroup to itself on its compute unit, its wavefronts in two halves of k: rows and tokens over the edge, as many
 # workgroups as units and some more, tiles of 64 and of 128 tokens, the shortest k of halves and a shorter one
 @pytest.mark.parametrize("m,k,M", [(384, 1536, 5121), (4096, 2048, 1024), (4096, 2048, 1025), (4096, 4096, 1281), (12288, 4096, 257), (1536, 1536, 2048), (1024, 1024, 2600)])

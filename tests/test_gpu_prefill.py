@@ -121,7 +121,8 @@ def test_sums_of_a_cut_product_normed_by_their_launch(awq, oracle, torch_gpu, hi
 
 @pytest.mark.parametrize("n", [129, 200, 320, 385, 512, 513])
 def test_prompts_whose_short_products_go_in_shares(awq, oracle, torch_gpu, n):
-    """k of Wo and W2 in four, three and two shares of tiles of 64 tokens, full and nearly empty, and the first count past them"""
+    """k of Wo in four and two shares of tiles of 64 tokens, of W2 in four, full and nearly empty, and counts between and past them
+    (which count goes how: test_shares_of_tiles_of_64_tokens)"""
     cfg = awq.make_config(n_layers=2, hidden=4096, inter=12288, vocab=1024, max_pos=576)
     model = make_oracle_model(oracle, cfg)   # only as the host buffer of the weights here
     eng = awq.QWen3AWQInfer.empty(cfg)

@@ -129,6 +129,29 @@ def test_shares_of_the_second_matrix(lib, tmp_path):
     assert got == list(SHARES.values()) + [0] * 4
 
 
+def test_products_of_17_to_64_tokens_with_operands_of_a_wavefronts_own(lib, tmp_path):
+    """rows per workgroup, 0: another kernel; m, k, tokens, whether there is room for the sums of a cut k"""
+    rows = {(4096, 4096): (16, 16, 16, 16, 16), (8192, 4096): (32,) * 5, (12288, 4096): (48,) * 5, (16384, 4096): (64, 64, 64, 64, 0),
+            (2048, 4096): (16,) * 5, (1024, 4096): (16, 16, 16, 16, 0), (4096, 2048): (16, 16, 16, 16, 0), (2048, 2048): (16,) * 5,
+            (8192, 2048): (32, 32, 32, 32, 0), (10240, 2048): (0, 0, 48, 48, 0), (20480, 2048): (0,) * 5, (4096, 12288): (64, 64, 64, 64, 0),
+            (3072, 12288): (48,) * 5, (128, 12288): (16,) * 5, (6144, 12288): (0,) * 5, (4096, 8192): (0,) * 5}
+    tokens = (17, 32, 33, 48, 49)
+    calls = [(*shape, t, 1) for shape in rows for t in tokens] + [(4096, 4096, 16, 1), (4096, 4096, 65, 1), (4096, 4096, 64, 0), (4096, 12288, 17, 0)]
+    lines = "".join('printf("%%d\\n", gemm_panel_rows(%d, %d, %d, %d));' % c for c in calls)
+    got = host_program(tmp_path, '#include <stdio.h>\n#include "common.hpp"\nint main() { %s }' % lines)
+    assert got == [r for five in rows.values() for r in five] + [0, 0, 16, 0]
+    plans = [(4096, 12288, 17, 1), (4096, 12288, 48, 1), (2048, 12288, 64, 1), (4096, 12288, 49, 1), (4096, 12288, 48, 0)]
+    assert [lib.awq_gemm_plan(*p) for p in plans] == [9, 9, 9, 1, 1]
+
+
+def test_shares_of_tiles_of_64_tokens(lib, tmp_path):
+    """of Wo and W2 behind prompts of 129 to 512 tokens; the other kernels have the rest"""
+    calls = [(4096, k, n) for k in (4096, 12288) for n in (128, 129, 192, 193, 200, 256, 257, 320, 321, 385, 512, 513)]
+    lines = "".join('printf("%%d\\n", gemm_norm_shares64(%d, %d, %d));' % c for c in calls)
+    got = host_program(tmp_path, '#include <stdio.h>\n#include "common.hpp"\nint main() { %s }' % lines)
+    assert got == [0, 4, 4, 4, 4, 4, 0, 0, 2, 2, 2, 0] + [0, 4, 4, 4, 4, 4, 0, 0, 0, 0, 0, 0]
+
+
 def forms_of(tmp_path, shapes):
     program = """
 #include <stdio.h>
