@@ -447,10 +447,14 @@ float shares_time(const DenseArgs& a, int64_t rows, int64_t cuts) {
   return 2.71f + (float)cuts * (0.3703f + (float)a.M * (float)rows * 8.0f / 2.708e6f);
 }
 // Two wavefronts per SIMD, each with a half of k, where a tile of a product has a compute unit to itself (at most 256 of them): one
-// waits for its trips to memory and its tokens, two have products for each other.  us, with four wavefronts and with eight: 1,024 x 512 at 129 tokens
-// 8.1, 7.7; 2,048 x 1,024 at 333 10.3, 9.6; 2,048 x 2,048 at 512 14.2, 12.5; 6,144 x 2,048 at 200 18.9, 16.7; 4,096 x 4,096 at 512 32.6, 29.3, at 1,000
-// 41.6, 38.9; 12,288 x 2,048 at 129 23.9, 21.8.  Not for shares of k, which are short already (1,024 x 4,096 at 512 tokens in four 16.2, 17.1), nor for
-// tokens of a list, whose tiles are mostly without any (no gain).
+// waits for its trips to memory and its tokens, two have products for each other.  us, with four wavefronts and with eight:
+//   1,024 x 512    129 tokens    8.1   7.7       4,096 x 4,096     512 tokens   32.6   29.3
+//   2,048 x 1,024  333 tokens   10.3   9.6       4,096 x 4,096   1,000 tokens   41.6   38.9
+//   2,048 x 2,048  512 tokens   14.2  12.5       8,192 x 8,192     512 tokens   86.3   76.9
+//   6,144 x 2,048  200 tokens   18.9  16.7       2,048 x 8,192   2,048 tokens   84.4   75.6
+//   12,288 x 2,048 129 tokens   23.9  21.8       4,096 x 16,384  2,048 tokens    250    241
+// Not for shares of k, which are short already (1,024 x 4,096 at 512 tokens in four 16.2, 17.1), nor for tokens of a list, whose tiles
+// are mostly without any (no gain).
 bool halves_pay(int64_t groups, int64_t steps, int64_t cuts) { return cuts == 1 && groups <= 256 && steps >= 8 && steps % 2 == 0; }
 
 // The time of a product in us, but for what all forms of it share: what the choice of a form and of a number of shares of k needs.
@@ -467,7 +471,8 @@ float many_time(const DenseArgs& a, int64_t rows, const ManyForm& f, int64_t cut
   const float wait = f.wait + f.root * sqrtf((float)std::min<int64_t>(256, row_tiles * cuts * a.batch));
   const float per_unit = ceilf(groups / 256.0f);
   float t = steps * wait * ceilf(groups / (float)f.resident);
-  // (what eight wavefronts give, where it was timed; sums that another launch adds anyway are cheaper in shares)
+  // What eight wavefronts give, where that was timed for the choice.  (Beyond 4,096 inputs the choice is the one without, and they only
+  // make it faster; sums that another launch adds anyway are cheaper in shares.)
   if (halves_pay((int64_t)groups, a.k >> 6, cuts) && a.k <= 4096 && !a.shares) t -= steps * (f.rb == 1 ? 0.05f : 0.02f);
   if (per_unit > 1.0f) t = std::max(t, steps * per_unit * f.step);
   t = std::max(t, (float)rows * (float)a.k * (float)a.batch * 2.0f / 9.12e6f);

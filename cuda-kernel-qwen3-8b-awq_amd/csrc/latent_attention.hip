@@ -182,10 +182,10 @@ __global__ __launch_bounds__(256) void latent_query_kernel(LatentAttnArgs a, int
 }
 
 // --- in the latent space, one query in binary32 ------------------------------------------------------------------
-// The three launches of a token as in bfloat16.  Bound by the trips to memory one behind the other, so everything of a launch is requested at
-// once.  Tudasun of width 1,024 at 48 to 72 positions: queries, rotation, cache row 4.2 us, W_uk 4.4, all keys of a head in one workgroup 9.6
-// and W_uv 3.4; now 4.6,
-// 4.5 and 4.2 (keys in shares, each row read once).
+// The three launches of a token as in bfloat16.  Bound by the trips to memory one behind the other, so everything of a launch is
+// requested at once; keys go in shares, each row read once.  Tudasun of width 1,024 at 48 to 72 positions, us: queries with W_uk,
+// rotation and cache row 4.4, the keys 4.9, the parts with W_uv 4.4; as four launches queries, rotation and cache row 4.2, W_uk 4.4,
+// all keys of a head in one workgroup 9.6, W_uv 3.4.
 constexpr int kOneKeys = 16, kOneParts = 64;
 
 __host__ __device__ inline int one_blocks_per_part(int keys, int parts, int* blocks) {

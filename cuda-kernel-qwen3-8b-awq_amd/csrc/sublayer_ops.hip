@@ -284,8 +284,10 @@ int launch_embed_tokens(const void* table, const void* side_table, bool f32, con
   return AWQ_OK;
 }
 
-// Where the row waits in registers.  Tudasun of width 2,048, 129 tokens: eight launches of 4.3 us less, 884 -> 843 us; at 1,024 tokens of width
-// 4,096, whose join makes three trips as it is, one product is cut, and its shares in the join cost what the launch had.
+// Where the row waits in registers.  Tudasun of width 2,048, 129 tokens: eight launches of 4.3 us less, 884 -> 843 us.  From 512 tokens
+// on that is up to a width of 1,024 (row_form): 512 tokens of width 768 751 -> 733 us, of 1,024 801 -> 795, in binary32 1,294 -> 1,267;
+// 2,048 tokens the same within 1 %.  Wider rows make three trips to memory in their join as it is: at 1,024 tokens of width 4,096 one
+// product is cut, and its shares in the join cost what the launch had.
 bool join_adds_shares(const JoinArgs& a) { return row_form(a); }
 
 int launch_join(const JoinArgs& a, bool f32, hipStream_t st) {
