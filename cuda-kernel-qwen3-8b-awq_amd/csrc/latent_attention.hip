@@ -384,8 +384,7 @@ __device__ __forceinline__ int tiles_per_part(int row0, int rows, int heads, int
 }
 
 template <int NT>
-__global__ __launch_bounds__(256) void latent_rows_kernel(LatentAttnArgs a) {
-  extern __shared__ __attribute__((aligned(16))) char raw[];
+__device__ __forceinline__ void attend_rows(const LatentAttnArgs& a, char* raw, int parts) {
   const int row = a.l.row(), rp = a.l.rank_padded(), KS = row + 8;
   bf16_t* const kt = reinterpret_cast<bf16_t*>(raw);                // [64][KS]
   bf16_t* const qt = kt + kKeys * KS;                               // [32][KS]
@@ -394,7 +393,7 @@ __global__ __launch_bounds__(256) void latent_rows_kernel(LatentAttnArgs a) {
   bf16_t* const pl = ph + kRows * kWeightStride;
   float* const fade = reinterpret_cast<float*>(pl + kRows * kWeightStride);  // [32]
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int rows = (int)a.M * a.heads, row0 = blockIdx.x * kRows, parts = gridDim.y, part = blockIdx.y;
+  const int rows = (int)a.M * a.heads, row0 = blockIdx.x * kRows, part = blockIdx.y;
   const int pos0 = a.pos.position();
   int tiles;
   const int per = tiles_per_part(row0, rows, a.heads, pos0, parts, &tiles);
@@ -535,33 +534,150 @@ __global__ __launch_bounds__(256) void latent_rows_kernel(LatentAttnArgs a) {
   }
 }
 
-// The parts of query row r and the sink: `scale` receives every part's factor; returns what the weighted parts are divided by
-__device__ __forceinline__ float combine_factors(const LatentAttnArgs& a, int r, int parts, float* scale, int* used_parts) {
-  const int tid = threadIdx.x, lane = tid & 63, ps = a.l.rank_padded() + 4;
+template <int NT>
+__global__ __launch_bounds__(256) void latent_rows_kernel(LatentAttnArgs a) {
+  extern __shared__ __attribute__((aligned(16))) char raw[];
+  attend_rows<NT>(a, raw, gridDim.y);
+}
+
+// One token of few keys: tiles of 64 keys leave a handful of workgroups at work, each a chain of trips and 64 KB of stores in pieces of 16 bytes.
+// Up to kBlocks blocks of 16 keys (as many as there are parts) go to a workgroup for each 128 columns: keys and queries
+// as operands straight into registers (a wavefront takes 16 queries and every second slice of a row), the columns once more for LDS, where
+// they are values, everything requested at once.  32 heads, rank 512, 128 to 150 positions: 9.7 us (tiles of 64) -> 5.7, 12 heads 8.3 -> 4.9;
+// all columns of a block in one workgroup 7.5.  From 33 blocks on tiles of 64: every part is read again by every workgroup of the
+// value launch.
+constexpr int kBlockKeys = 16, kBlocks = 32, kBlockCols = 128, kBlockScores = kBlockKeys + 4, kBlockWeights = kBlockKeys + 8;
+__host__ __device__ inline int blocks_room(int parts) { return parts < kBlocks ? parts : kBlocks; }
+__device__ __forceinline__ bool in_blocks(int pos, int parts) { return pos / kBlockKeys < blocks_room(parts); }
+
+template <int NT>
+__global__ __launch_bounds__(256) void latent_rows_one_kernel(LatentAttnArgs a, int parts) {
+  extern __shared__ __attribute__((aligned(16))) char raw[];
+  const int pos = a.pos.position();
+  if (!in_blocks(pos, parts)) {
+    if ((int)blockIdx.y < parts) attend_rows<NT>(a, raw, parts);
+    return;
+  }
+  const int part = blockIdx.y % blocks_room(parts), quarter = blockIdx.y / blocks_room(parts), key0 = part * kBlockKeys;
+  if (quarter >= NT || key0 > pos) return;
+  constexpr int KS = kBlockCols + 8;
+  // (less than the tiles of 64 keys take at the shortest row)
+  bf16_t* const kt = reinterpret_cast<bf16_t*>(raw);                            // [16][KS]
+  float* const sc = reinterpret_cast<float*>(kt + kBlockKeys * KS);             // [2][32][kBlockScores]
+  bf16_t* const ph = reinterpret_cast<bf16_t*>(sc + 2 * kRows * kBlockScores);  // [32][kBlockWeights], twice
+  bf16_t* const pl = ph + kRows * kBlockWeights;
+  const int row = a.l.row(), rp = a.l.rank_padded();
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int row0 = blockIdx.x * kRows;
+  const bf16_t* const cache = reinterpret_cast<const bf16_t*>(a.cache) + (int64_t)key0 * row;  // (the cache is whole tiles)
+  const bf16_t* const ql = reinterpret_cast<const bf16_t*>(a.ql);
+  const int n16 = lane & 15, c16 = lane >> 4, n32 = lane & 31, kh = lane >> 5;
+  const int qb = wave & 1, turn = wave >> 1, slices = row >> 5;
+  constexpr int kSlices = kMaxRow / 64;
+  bf16x8_t ko[kSlices], qo[kSlices];
+  const bf16_t* const qrow = ql + (int64_t)min(row0 + 16 * qb + n16, a.heads - 1) * row + 8 * c16;
+  const bf16_t* const krow = cache + n16 * row + 8 * c16;
+#pragma unroll
+  for (int i = 0; i < kSlices; ++i) {  // (past the row its last piece again: a condition would have each request waited for)
+    const int slice = min(2 * i + turn, slices - 1);
+    qo[i] = *reinterpret_cast<const bf16x8_t*>(qrow + 32 * slice);
+    ko[i] = *reinterpret_cast<const bf16x8_t*>(krow + 32 * slice);
+  }
+  const int kr = tid >> 4, kf = (tid & 15) * 8;
+  bf16x8_t kx = *reinterpret_cast<const bf16x8_t*>(cache + kr * row + min(quarter * kBlockCols + kf, row - 8));
+  f32x4_t s = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+  for (int i = 0; i < kSlices; ++i)
+    if (2 * i + turn < slices) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ko[i], qo[i], s, 0, 0, 0);
+  *reinterpret_cast<f32x4_t*>(sc + (turn * kRows + 16 * qb + n16) * kBlockScores + 4 * c16) = s;
+  if (key0 + kr > pos)  // not of this sequence: weight zero, but not as a factor of an infinity
+#pragma unroll
+    for (int e = 0; e < 8; ++e) kx[e] = (bf16_t)0.0f;
+  *reinterpret_cast<bf16x8_t*>(kt + kr * KS + kf) = kx;
+  __syncthreads();
+  // the softmax: eight threads per row, two keys each
+  const int sr = tid >> 3, sk = (tid & 7) * 2;
+  float m, l;
+  {
+    const float mul = a.scale * kLog2e;
+    float x[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const float sum = sc[sr * kBlockScores + sk + e] + sc[(kRows + sr) * kBlockScores + sk + e];
+      x[e] = key0 + sk + e <= pos ? sum * mul : -INFINITY;
+    }
+    m = lanes::maximum<8>(fmaxf(x[0], x[1]));
+    const float base = m == -INFINITY ? 0.0f : m, p0 = exp2f(x[0] - base), p1 = exp2f(x[1] - base);
+    l = lanes::sum<8>(p0 + p1);
+    typedef bf16_t bf16x2_t __attribute__((ext_vector_type(2)));
+    const bf16x2_t hi = {(bf16_t)p0, (bf16_t)p1};
+    *reinterpret_cast<bf16x2_t*>(ph + sr * kBlockWeights + sk) = hi;
+    *reinterpret_cast<bf16x2_t*>(pl + sr * kBlockWeights + sk) = bf16x2_t{(bf16_t)(p0 - (float)hi[0]), (bf16_t)(p1 - (float)hi[1])};
+  }
+  __syncthreads();
+  const int L16 = lane & 15, at = n32 * kBlockWeights + 4 * kh;
+  const bf16_t* const vlane = kt + (4 * kh + (L16 >> 2)) * KS + 16 * ((lane >> 4) & 1) + 4 * (L16 & 3);
+  const bf16x4_t h0 = *reinterpret_cast<const bf16x4_t*>(ph + at), h1 = *reinterpret_cast<const bf16x4_t*>(ph + at + 8);
+  const bf16x4_t l0 = *reinterpret_cast<const bf16x4_t*>(pl + at), l1 = *reinterpret_cast<const bf16x4_t*>(pl + at + 8);
+  const bf16x8_t whi = {h0[0], h0[1], h0[2], h0[3], h1[0], h1[1], h1[2], h1[3]};
+  const bf16x8_t wlo = {l0[0], l0[1], l0[2], l0[3], l1[0], l1[1], l1[2], l1[3]};
+  const int ps = rp + 4, col = quarter * kBlockCols + 32 * wave;
+  if (col < rp) {
+    const short4_t lo4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((short4_t __attribute__((address_space(3)))*)(vlane + 32 * wave));
+    const short4_t up4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((short4_t __attribute__((address_space(3)))*)(vlane + 8 * KS + 32 * wave));
+    const bf16x4_t l4 = __builtin_bit_cast(bf16x4_t, lo4), u4 = __builtin_bit_cast(bf16x4_t, up4);
+    const bf16x8_t vv = {l4[0], l4[1], l4[2], l4[3], u4[0], u4[1], u4[2], u4[3]};
+    f32x16_t o;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) o[e] = 0.0f;
+    o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vv, whi, o, 0, 0, 0);
+    o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vv, wlo, o, 0, 0, 0);
+    float* const mine = a.parts + ((int64_t)(row0 + n32) * parts + part) * ps + 4 + col;
+    if (row0 + n32 < a.heads)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) *reinterpret_cast<f32x4_t*>(mine + 8 * u + 4 * kh) = f32x4_t{o[4 * u], o[4 * u + 1], o[4 * u + 2], o[4 * u + 3]};
+  }
+  if (quarter == 0 && sk == 0 && row0 + sr < a.heads) {
+    float* const to = a.parts + ((int64_t)(row0 + sr) * parts + part) * ps;
+    to[0] = m;
+    to[1] = l;
+  }
+}
+
+// The parts that query row r has
+__device__ __forceinline__ int used_parts(const LatentAttnArgs& a, int r, int parts) {
+  const int pos = a.pos.position();
+  if (a.M == 1 && in_blocks(pos, parts)) return pos / kBlockKeys + 1;
   int tiles;
-  const int per = tiles_per_part(r / kRows * kRows, (int)a.M * a.heads, a.heads, a.pos.position(), parts, &tiles);
-  const int used = (tiles + per - 1) / per;
+  const int per = tiles_per_part(r / kRows * kRows, (int)a.M * a.heads, a.heads, pos, parts, &tiles);
+  return (tiles + per - 1) / per;
+}
+// ... and the sink: `scale` receives every part's factor; returns what the weighted parts are divided by
+__device__ __forceinline__ float combine_factors(const LatentAttnArgs& a, int r, int head, int parts, int used, float* scale) {
+  const int tid = threadIdx.x, lane = tid & 63, ps = a.l.rank_padded() + 4;
   const float* const p = a.parts + (int64_t)r * parts * ps;
-  const float sink = a.sink ? a.sink[r % a.heads] * kLog2e : -INFINITY;
+  const float sink = a.sink ? a.sink[head] * kLog2e : -INFINITY;
   float pm[kMaxParts / 64], pl[kMaxParts / 64], m = sink, l = 0.0f;
 #pragma unroll
   for (int i = 0; i < kMaxParts / 64; ++i) {
-    const int s = lane + 64 * i;
-    pm[i] = s < used ? p[(int64_t)s * ps] : -INFINITY;
-    pl[i] = s < used ? p[(int64_t)s * ps + 1] : 0.0f;
-    m = fmaxf(m, pm[i]);
+    const int64_t at = (int64_t)min(lane + 64 * i, used - 1) * ps;
+    pm[i] = p[at];
+    pl[i] = p[at + 1];
   }
 #pragma unroll
-  for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+  for (int i = 0; i < kMaxParts / 64; ++i) {
+    if (lane + 64 * i >= used) pm[i] = -INFINITY, pl[i] = 0.0f;
+    m = fmaxf(m, pm[i]);
+  }
+  m = lanes::maximum(m);
 #pragma unroll
   for (int i = 0; i < kMaxParts / 64; ++i) {
     const float e = exp2f(pm[i] - m);
     l = __builtin_fmaf(e, pl[i], l);
     if (tid < 64) scale[lane + 64 * i] = e;
   }
-  l = wave_sum(l) + exp2f(sink - m);
+  l = lanes::sum(l) + exp2f(sink - m);
   __syncthreads();
-  *used_parts = used;
   return l;
 }
 __device__ __forceinline__ float combine_column(const LatentAttnArgs& a, int r, int parts, const float* scale, int used, int c) {
@@ -576,45 +692,61 @@ __device__ __forceinline__ float combine_column(const LatentAttnArgs& a, int r, 
 // a workgroup per query row
 __global__ __launch_bounds__(256) void latent_combine_kernel(LatentAttnArgs a, int parts, int kv_in) {
   __shared__ float scale[kMaxParts];
-  const int r = blockIdx.x;
-  int used;
-  const float inv = 1.0f / combine_factors(a, r, parts, scale, &used);
+  const int r = blockIdx.x, used = used_parts(a, r, parts);
+  const float inv = 1.0f / combine_factors(a, r, r % a.heads, parts, used, scale);
   bf16_t* const out = reinterpret_cast<bf16_t*>(a.ol) + (int64_t)r * kv_in;
   for (int c = threadIdx.x; c < kv_in; c += 256) out[c] = (bf16_t)(c < a.l.rank ? combine_column(a, r, parts, scale, used, c) * inv : 0.0f);
 }
 
-// One token: the same and the product with W_uv in one launch.  blockIdx.x: head, blockIdx.y: 64 of its values, 16 a
-// wavefront; every workgroup combines for itself while its weights are on their way.
+// One token: the same and the product with W_uv in one launch.  blockIdx.x: head, blockIdx.y: 16 of its values, a quarter of the inputs
+// each wavefront; every workgroup combines for itself, two columns a thread, while its weights are on their way, the first parts
+// requested ahead of the factors.  32 heads, rank 512: 64 values a workgroup and its weights waited for ahead of the parts 6.4 us, now 4.8.
+constexpr int kOneValues = 16, kOneInputs = 512;  // (rank_padded of the rows kernels)
 __global__ __launch_bounds__(256) void latent_value_one_kernel(LatentAttnArgs a, int parts, int kv_in, int64_t w_block) {
-  extern __shared__ __attribute__((aligned(16))) bf16_t ol[];  // [kv_in]
-  __shared__ float scale[kMaxParts];
-  constexpr int U = 16;
+  __shared__ __attribute__((aligned(16))) bf16_t ol[kOneInputs];
+  __shared__ float scale[kMaxParts], sums[4][kOneValues];
+  constexpr int U = kOneInputs / 128, F = 16;
   const int h = blockIdx.x, tid = threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, c = lane >> 4;
-  const int row0 = blockIdx.y * 64 + wave * 16, steps = kv_in >> 5;
-  const bool mine = row0 < a.vdim;
+  const int row0 = blockIdx.y * kOneValues, steps = kv_in >> 5, rank = a.l.rank, rp = a.l.rank_padded(), ps = rp + 4;
   const bf16x8_t* w = reinterpret_cast<const bf16x8_t*>(reinterpret_cast<const bf16_t*>(a.w_uv) + h * w_block) +
                       ((int64_t)(row0 >> 5) * (kv_in >> 4) + (c >> 1)) * 64 + 32 * (c & 1) + (row0 & 16) + r;
   bf16x8_t wv[U];
 #pragma unroll
-  for (int i = 0; i < U; ++i)
-    if (mine && i < steps) wv[i] = w[(int64_t)i * 128];
-  int used;
-  const float inv = 1.0f / combine_factors(a, h, parts, scale, &used);
-  for (int col = tid; col < kv_in; col += 256) ol[col] = (bf16_t)(col < a.l.rank ? combine_column(a, h, parts, scale, used, col) * inv : 0.0f);
+  for (int i = 0; i < U; ++i) wv[i] = w[(int64_t)min(wave + 4 * i, steps - 1) * 128];
+  const int used = used_parts(a, h, parts), col = 2 * tid;
+  typedef float f32x2_t __attribute__((ext_vector_type(2)));
+  const float* const p = a.parts + (int64_t)h * parts * ps + 4 + min(col, rp - 2);
+  f32x2_t first[F];
+#pragma unroll
+  for (int s = 0; s < F; ++s) first[s] = *reinterpret_cast<const f32x2_t*>(p + (int64_t)min(s, used - 1) * ps);
+  const float inv = 1.0f / combine_factors(a, h, h, parts, used, scale);
+  f32x2_t v = {0.0f, 0.0f};
+#pragma unroll
+  for (int s = 0; s < F; ++s)
+    if (s < used)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) v[e] = __builtin_fmaf(scale[s], first[s][e], v[e]);
+#pragma unroll 8
+  for (int s = F; s < used; ++s) {
+    const f32x2_t x = *reinterpret_cast<const f32x2_t*>(p + (int64_t)s * ps);
+#pragma unroll
+    for (int e = 0; e < 2; ++e) v[e] = __builtin_fmaf(scale[s], x[e], v[e]);
+  }
+#pragma unroll
+  for (int e = 0; e < 2; ++e)
+    if (col + e < kv_in) ol[col + e] = (bf16_t)(col + e < rank ? v[e] * inv : 0.0f);
   __syncthreads();
-  if (!mine) return;
   const bf16x8_t* x = reinterpret_cast<const bf16x8_t*>(ol) + c;
   f32x4_t acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
   for (int i = 0; i < U; ++i)
-    if (i < steps) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[i], x[i * 4], acc, 0, 0, 0);
-  for (int i = U; i < steps; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[(int64_t)i * 128], x[i * 4], acc, 0, 0, 0);
-  if (r != 0) return;
-  bf16_t* const out = reinterpret_cast<bf16_t*>(a.ctx) + (int64_t)h * a.vdim + row0;
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-    if (row0 + 4 * c + j < a.vdim) out[4 * c + j] = (bf16_t)acc[j];
+    if (wave + 4 * i < steps) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wv[i], x[(wave + 4 * i) * 4], acc, 0, 0, 0);
+  if (r == 0) *reinterpret_cast<f32x4_t*>(&sums[wave][4 * c]) = acc;
+  __syncthreads();
+  if (tid < kOneValues && row0 + tid < a.vdim)
+    reinterpret_cast<bf16_t*>(a.ctx)[(int64_t)h * a.vdim + row0 + tid] =
+        (bf16_t)((sums[0][tid] + sums[1][tid]) + (sums[2][tid] + sums[3][tid]));
 }
 
 // --- with keys and values formed first -------------------------------------------------------------------------
@@ -804,7 +936,9 @@ int one_parts_of(const LatentAttnArgs& a, int64_t keys) {
 }
 
 int parts_of(const LatentAttnArgs& a, int64_t M, int64_t keys) {
-  const int64_t row_tiles = (M * a.heads + kRows - 1) / kRows, tiles = (keys + kKeys - 1) / kKeys;
+  const int64_t row_tiles = (M * a.heads + kRows - 1) / kRows;
+  int64_t tiles = (keys + kKeys - 1) / kKeys;
+  if (M == 1) tiles = std::max(tiles, std::min<int64_t>((keys + kBlockKeys - 1) / kBlockKeys, kBlocks));
   return (int)std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(512 / row_tiles, tiles), kMaxParts));
 }
 
@@ -819,15 +953,22 @@ int launch_prepare(const LatentAttnArgs& a, hipStream_t st) {
 
 static_assert((size_t)(kKeys + kRows) * (kMaxRow + 8) * 2 + kRows * kScoreStride * 4 + 4 * kRows * kWeightStride + kRows * 4 <= 160 * 1024,
               "more LDS than a compute unit has");
+static_assert(kBlockKeys * (kBlockCols + 8) * 2 + 2 * kRows * kBlockScores * 4 + 4 * kRows * kBlockWeights <= (kKeys + kRows) * (64 + 8) * 2 + kRows * kScoreStride * 4 + 4 * kRows * kWeightStride,
+              "blocks take more LDS than tiles of the shortest rows");
 template <int NT>
 int launch_rows(const LatentAttnArgs& a, int parts, hipStream_t st) {
   static bool raised = false;  // more LDS than the default limit of a launch
   if (!raised) {
     AWQ_HIP_TRY(hipFuncSetAttribute((const void*)latent_rows_kernel<NT>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+    AWQ_HIP_TRY(hipFuncSetAttribute((const void*)latent_rows_one_kernel<NT>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     raised = true;
   }
-  hipLaunchKernelGGL(latent_rows_kernel<NT>, dim3((unsigned)((a.M * a.heads + kRows - 1) / kRows), (unsigned)parts), dim3(256),
-                     rows_lds(a.l.row()), st, a);
+  const unsigned tiles = (unsigned)((a.M * a.heads + kRows - 1) / kRows);
+  if (a.M == 1)
+    hipLaunchKernelGGL(latent_rows_one_kernel<NT>, dim3(tiles, (unsigned)std::max(parts, blocks_room(parts) * NT)), dim3(256),
+                       rows_lds(a.l.row()), st, a, parts);
+  else
+    hipLaunchKernelGGL(latent_rows_kernel<NT>, dim3(tiles, (unsigned)parts), dim3(256), rows_lds(a.l.row()), st, a);
   AWQ_HIP_TRY(hipGetLastError());
   return AWQ_OK;
 }
@@ -977,8 +1118,8 @@ int launch_latent_attention(const LatentAttnArgs& a, bool f32, hipStream_t st) {
     if (int rc = rp <= 128 ? launch_rows<1>(a, parts, st) : rp <= 256 ? launch_rows<2>(a, parts, st) : launch_rows<4>(a, parts, st))
       return rc;
     if (a.M == 1) {
-      hipLaunchKernelGGL(latent_value_one_kernel, dim3((unsigned)a.heads, (unsigned)((a.vdim + 63) / 64)), dim3(256),
-                         (size_t)v_inputs(a) * 2, st, a, parts, (int)v_inputs(a), latent_uv_block(a));
+      hipLaunchKernelGGL(latent_value_one_kernel, dim3((unsigned)a.heads, (unsigned)((a.vdim + kOneValues - 1) / kOneValues)), dim3(256), 0,
+                         st, a, parts, (int)v_inputs(a), latent_uv_block(a));
       AWQ_HIP_TRY(hipGetLastError());
       return AWQ_OK;
     }

@@ -536,6 +536,35 @@ def test_latent_attention(awq, lib, dev, f32, shape):
         assert km.rms_error(got, want) < (3e-5 if f32 else 0.03), sizes
 
 
+# one query in bfloat16: blocks of 16 keys up to as many as there are parts (at most 32), tiles of 64 from there on; row tiles of heads that are
+# not whole, and so many heads that two parts are left
+@pytest.mark.parametrize("shape", [(33, 32, 32, 24, 128), (2, 128, 64, 40, 512), (3, 64, 6, 12, 37), (8000, 8, 2, 4, 32)], ids=str)
+def test_single_queries_in_bfloat16(awq, lib, dev, shape):
+    heads, dim, rot, vdim, rank = shape
+    print("latent attention, one query", shape, flush=True)
+    rng = np.random.default_rng(rank)
+    T, eps, base, scale = 560 if heads < 100 else 48, 1e-3, 300.0, 2.5 * (dim + rot) ** -0.5
+    q = km.bf16(rng.standard_normal((T, heads * (dim + rot))))
+    down = rng.standard_normal((T, rank + rot)).astype(np.float32)
+    norm, sink = 1 + 0.3 * rng.standard_normal(rank), 2 * rng.standard_normal(heads)
+    uk, uv = (km.bf16(rng.standard_normal((heads * n, rank)) / rank ** 0.5) for n in (dim, vdim))
+    c = plain.rms(down[:, :rank].astype(np.float64), eps) * norm.astype(np.float32)
+    kr = plain.rotate(down[:, rank:].astype(np.float64), 0, base)
+    layer = Latent(awq, lib, dev, 0, heads, dim, rot, vdim, rank, uk, uv, norm, sink, scale, eps, base, T, T)
+    there = 0
+    for t in (0, 1, 14, 15, 16, 31, 32, 33, 47, 63, 64, 255, 510, 511, 512, 513, 559):
+        if t >= T:
+            break
+        if there < t:
+            layer.run(q[there:t], down[there:t], there)
+        there = t + 1
+        qh = q[t:t + 1].reshape(1, heads, dim + rot).astype(np.float64)
+        want = plain.latent_attention(qh[:, :, :dim], plain.rotate(qh[:, :, dim:], t, base), c[:t + 1], kr[:t + 1], uk.reshape(heads, dim, rank),
+                                      uv.reshape(heads, vdim, rank), scale, sink, t)
+        got = layer.run(q[t:t + 1], down[t:t + 1], t)
+        assert km.rms_error(got, want) < 0.03, t
+
+
 # one query in binary32: keys in shares of one and of several blocks (90 heads leave five shares), where there is no place for shares, and sizes
 # that have no such form (heads of 22, rows of more than 768)
 @pytest.mark.parametrize("shape,parts", [((90, 8, 6, 4, 40), True), ((600, 4, 2, 4, 8), True), ((3, 20, 6, 12, 37), False), ((3, 22, 6, 12, 37), True),
