@@ -207,6 +207,7 @@ SIGNATURES.update({
     "awq_window_attention": (ctypes.c_int, [ctypes.POINTER(AwqWindowArgs), _i32, _vp]),
     "awq_dense_pack_form": (ctypes.c_int, [_vp, _i32, _i64, _i64, _vp, _i64, _i64, _i64, _i32, _i32, _vp]),
     "awq_gated_state": (ctypes.c_int, [ctypes.POINTER(AwqGatedStateArgs), _i32, _vp]),
+    "awq_gated_state_segments": (ctypes.c_int, [ctypes.POINTER(AwqGatedStateArgs), _i32, _vp, _i64, _vp]),
     "awq_head_norm": (ctypes.c_int, [_vp, _vp, _i64, _vp, _vp, _i64, _i32, _i32, _i64, _f32, _i32, _vp]),
     "awq_latent_row": (_i32, [_i32, _i32]),
     "awq_latent_sizes": (ctypes.c_int, [ctypes.POINTER(AwqLatentArgs), _i64, _i32, ctypes.POINTER(AwqLatentBytes)]),
@@ -217,6 +218,7 @@ SIGNATURES.update({
     "awq_join": (ctypes.c_int, [ctypes.POINTER(AwqJoinArgs), _i32, _vp]),
     "awq_polynorm": (ctypes.c_int, [_vp, _i64, _i64, _i64, _vp, _f32, _i32, _vp]),
     "awq_linear_attention": (ctypes.c_int, [_vp, _i64, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _vp]),
+    "awq_linear_attention_segments": (ctypes.c_int, [_vp, _i64, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _vp, _i64, _vp]),
 })
 
 _lib = None

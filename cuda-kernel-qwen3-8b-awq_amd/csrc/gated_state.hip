@@ -344,8 +344,14 @@ constexpr int chunk_lds() {
   return 2 * (2 * C * (D + 4) + C * kValueStride + B * D + 4 * B * 256) * 4;
 }
 
-// EVEN: dim is even, two channels make one load; keys: there are keys beside the decays
-template <typename T, int D, bool EVEN, bool keys, bool HEAD>
+// EVEN: dim is even, two channels make one load; keys: there are keys beside the decays.
+// Where heads and columns leave compute units without a workgroup, a pass is cut into segments (a.seg_tokens, blockIdx.z) that go side by
+// side, in two launches.  AHEAD: for every segment but the last the state that it adds to an empty one and what it leaves of
+// a row of the state ahead of it; the first starts from the state itself and keeps a copy.  Then the outputs, every segment starting from
+// those sums, and the last one's state.  The workspace holds
+//     [segments][heads][vdim][dimp]: the state ahead of the pass, then what the segments but the last add,
+//     [segments - 1][heads][dimp]: what is left of a row (not HEAD).
+template <typename T, int D, bool EVEN, bool keys, bool HEAD, bool AHEAD>
 __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
   static_assert(keys || !HEAD, "a head's decay leaves no keys");
   constexpr int B = chunk_blocks<D>(), C = B * kBlock, S4 = D + 4, VS = kValueStride;
@@ -360,11 +366,14 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
   __shared__ int unsafe[3][B];                // of the running chunk, the one being formed, and one to be cleared
   const int head = blockIdx.x, c0 = blockIdx.y * 16;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int M = (int)a.M, nv = min(16, a.vdim - c0), chunks = (M + C - 1) / C;
-  const T* const q = reinterpret_cast<const T*>(a.q) + (int64_t)head * a.dim;
-  const T* const k = keys ? reinterpret_cast<const T*>(a.k) + (int64_t)head * a.dim : q;
-  const T* const v = reinterpret_cast<const T*>(a.v) + (int64_t)head * a.vdim + c0;
-  const float* const g = HEAD ? a.head_decay : a.g + (int64_t)head * a.dim;
+  const int segment = blockIdx.z;
+  const int64_t tok0 = (int64_t)segment * a.seg_tokens;
+  const int M = (int)(a.seg_tokens ? min((int64_t)a.seg_tokens, a.M - tok0) : a.M);  // tokens of this segment, counted from tok0
+  const int nv = min(16, a.vdim - c0), chunks = (M + C - 1) / C;
+  const T* const q = reinterpret_cast<const T*>(a.q) + tok0 * a.ldp + (int64_t)head * a.dim;
+  const T* const k = keys ? reinterpret_cast<const T*>(a.k) + tok0 * a.ldp + (int64_t)head * a.dim : q;
+  const T* const v = reinterpret_cast<const T*>(a.v) + tok0 * a.ldp + (int64_t)head * a.vdim + c0;
+  const float* const g = HEAD ? a.head_decay : a.g + tok0 * a.ldg + (int64_t)head * a.dim;
   const float of_head = HEAD ? a.head_decay[head] : 0.0f;
   __shared__ float power[HEAD ? kBlock + 1 : 1], power_rest[HEAD ? kBlock + 1 : 1];  // of the decay: their sum is the n-th
   if constexpr (HEAD) {
@@ -398,7 +407,7 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
       for (int t = 0; t < kHalf; ++t) {
         const int64_t tok = min(at + t0 + t, M - 1);
         if constexpr (!HEAD) gr[t] = two(g + tok * a.ldg + dc);
-        qr[t] = two(q + tok * a.ldp + dc);
+        if constexpr (!AHEAD) qr[t] = two(q + tok * a.ldp + dc);
         if constexpr (keys) kr[t] = two(k + tok * a.ldp + dc);
       }
 #pragma unroll
@@ -423,10 +432,10 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
 #pragma unroll
           for (int e = 0; e < 2; ++e) {
             const bool there = has[e] && at + t < M;
-            qv[e] = there ? (float)qr[t][e] * a.q_scale : 0.0f;
+            if constexpr (!AHEAD) qv[e] = there ? (float)qr[t][e] * a.q_scale : 0.0f;
             kv[e] = there ? (float)kr[t][e] : 0.0f;
           }
-          *reinterpret_cast<f32x2_t*>(qs + t * S4) = qv;
+          if constexpr (!AHEAD) *reinterpret_cast<f32x2_t*>(qs + t * S4) = qv;
           *reinterpret_cast<f32x2_t*>(ks + t * S4) = kv;
         }
         values();
@@ -459,10 +468,10 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
         for (int e = 0; e < 2; ++e) {
           const bool there = has[e] && at + t < M;
           const float x = L[t][e] + ahead[e] - mid[e];
-          qv[e] = (there ? (float)qr[t][e] * a.q_scale : 0.0f) * __builtin_amdgcn_exp2f(x);
+          if constexpr (!AHEAD) qv[e] = (there ? (float)qr[t][e] * a.q_scale : 0.0f) * __builtin_amdgcn_exp2f(x);
           kv[e] = (keys ? (there ? (float)kr[t][e] : 0.0f) : gr[t][e]) * __builtin_amdgcn_exp2f(-x);
         }
-        *reinterpret_cast<f32x2_t*>(qs + t * S4) = qv;
+        if constexpr (!AHEAD) *reinterpret_cast<f32x2_t*>(qs + t * S4) = qv;
         *reinterpret_cast<f32x2_t*>(ks + t * S4) = kv;
       }
       if (half == 0)
@@ -478,7 +487,7 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
 #pragma unroll
       for (int w = 1; w < 4; ++w) sum = sum + *reinterpret_cast<const f32x4_t*>(red + w * B * 256);
       if (chunk * C + t >= M) return;
-      float* const out = a.o + ((int64_t)(chunk * C + t) * a.heads + head) * a.vdim + c0 + c;
+      float* const out = a.o + ((tok0 + chunk * C + t) * a.heads + head) * a.vdim + c0 + c;
       if (c + 3 < nv && (a.vdim & 3) == 0) {
         *reinterpret_cast<f32x4_t*>(out) = sum;
       } else {
@@ -495,24 +504,54 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
       if (p < B) unsafe[(i + 2) % 3][p] = 0;
       if (i + 1 < chunks) form(i + 1);
       if (i + 2 < chunks) load(i + 2);
-      if (i > 0) store(i - 1);
+      if (!AHEAD && i > 0) store(i - 1);
       __syncthreads();
     }
-    store(chunks - 1);
+    if constexpr (!AHEAD) store(chunks - 1);
     return;
   }
 
   const int n = lane & 15, j4 = (lane >> 4) * 4;
   const int dimp = (a.dim + 63) & ~63;
   const int row0 = wave * (D / 4);        // this wavefront's rows of the state
-  float* const state = a.state + ((int64_t)head * a.vdim + c0 + n) * dimp;
+  const int64_t column = ((int64_t)head * a.vdim + c0 + n) * dimp, states = (int64_t)a.heads * a.vdim * dimp;
+  float* const state = a.state + column;
   f32x4_t s[NT];                          // s[i]: rows row0 + 16 i + j4 .. + 3 of column n
+  f32x4_t left[NT];                       // AHEAD, not HEAD: the product of the decays
+  float over = 0.0f, over_rest = 0.0f;    // HEAD: the decay's power over a segment
+  if (HEAD && !AHEAD && segment > 1) {
+    double x = 1.0, y = (double)of_head;
+    for (int e = a.seg_tokens; e; e >>= 1, y *= y)
+      if (e & 1) x *= y;
+    over = (float)x;
+    over_rest = (float)(x - (double)over);
+  }
   const bool fresh = a.pos.position() == 0;
 #pragma unroll
   for (int i = 0; i < NT; ++i) {
     const int d = row0 + 16 * i + j4;
+    const bool there = d < dimp && n < nv;
     s[i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    if (!fresh && d < dimp && n < nv) s[i] = *reinterpret_cast<const f32x4_t*>(state + d);
+    left[i] = f32x4_t{1.0f, 1.0f, 1.0f, 1.0f};
+    if (AHEAD || !a.seg_tokens) {
+      if (!fresh && there && segment == 0) s[i] = *reinterpret_cast<const f32x4_t*>(state + d);
+      if (AHEAD && segment == 0 && there) *reinterpret_cast<f32x4_t*>(a.workspace + column + d) = s[i];
+    } else if (there) {
+      const float* const from = a.workspace + column + d;
+      s[i] = *reinterpret_cast<const f32x4_t*>(from + (segment == 0 ? 0 : states));
+      for (int j = 2; j <= segment; ++j) {
+        const f32x4_t add = *reinterpret_cast<const f32x4_t*>(from + j * states);
+        if constexpr (HEAD) {  // the power as a sum of two numbers, as that of a block
+#pragma unroll
+          for (int e = 0; e < 4; ++e) s[i][e] = __builtin_fmaf(s[i][e], over, __builtin_fmaf(s[i][e], over_rest, add[e]));
+          continue;
+        }
+        const f32x4_t f =
+            *reinterpret_cast<const f32x4_t*>(a.workspace + (int64_t)gridDim.z * states + ((int64_t)(j - 1) * a.heads + head) * dimp + d);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[i][e] = s[i][e] != 0.0f ? __builtin_fmaf(s[i][e], f[e], add[e]) : add[e];  // (no 0 x infinity)
+      }
+    }
   }
   // HEAD: a power that is no number, or leaves the range where a product with it is as exact as others, is not used; nor is any
   // for a state that is not finite (the power's second number may be 0)
@@ -557,7 +596,7 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
               const f32x4_t qv = *reinterpret_cast<const f32x4_t*>(qs + (b * kBlock + n) * S4 + row0 + 16 * i + j4);
               const f32x4_t kv = *reinterpret_cast<const f32x4_t*>(ks + (b * kBlock + n) * S4 + row0 + 16 * i + j4);
 #pragma unroll
-              for (int e = 0; e < 4; ++e) {
+              for (int e = 0; e < 4 && !AHEAD; ++e) {
                 const int j = 2 * i + (e & 1);
                 w[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[e], qv[e], w[j], 0, 0, 0);
                 ot[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(s[i][e], qv[e], ot[j], 0, 0, 0);
@@ -580,15 +619,17 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
               for (int e = 0; e < 4; ++e)
                 s[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(ks[(b * kBlock + j4 + e) * S4 + row0 + 16 * i + n], later[e], s[i], 0, 0, 0);
             }
+            if constexpr (!AHEAD) {
 #pragma unroll
-            for (int half = NT; half > 0; half >>= 1)
+              for (int half = NT; half > 0; half >>= 1)
 #pragma unroll
-              for (int i = 0; i < half; ++i) w[i] = w[i] + w[i + half], ot[i] = ot[i] + ot[i + half];
-            // w[0][i]: key token j4 + i, query token n
+                for (int i = 0; i < half; ++i) w[i] = w[i] + w[i + half], ot[i] = ot[i] + ot[i + half];
+              // w[0][i]: key token j4 + i, query token n
 #pragma unroll
-            for (int i = 0; i < 4; ++i) o[i] = __builtin_fmaf(ot[0][i], out_power, ot[0][i] * out_power_rest);
+              for (int i = 0; i < 4; ++i) o[i] = __builtin_fmaf(ot[0][i], out_power, ot[0][i] * out_power_rest);
 #pragma unroll
-            for (int i = 0; i < 4; ++i) o = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[i], j4 + i <= n ? w[0][i] * back[i] : 0.0f, o, 0, 0, 0);
+              for (int i = 0; i < 4; ++i) o = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[i], j4 + i <= n ? w[0][i] * back[i] : 0.0f, o, 0, 0, 0);
+            }
           }
         } else {
           f32x4_t w = {0.0f, 0.0f, 0.0f, 0.0f}, f[NT];
@@ -597,6 +638,11 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
             f[i] = *reinterpret_cast<const f32x4_t*>(ts + b * D + row0 + 16 * i + j4);
 #pragma unroll
             for (int e = 0; e < 4; ++e) s[i][e] *= f[i][e];
+            if constexpr (AHEAD) {
+#pragma unroll
+              for (int e = 0; e < 4; ++e) left[i][e] *= f[i][e] * f[i][e];
+              continue;
+            }
             const f32x4_t qv = *reinterpret_cast<const f32x4_t*>(qs + (b * kBlock + n) * S4 + row0 + 16 * i + j4);
             const f32x4_t kv = *reinterpret_cast<const f32x4_t*>(ks + (b * kBlock + n) * S4 + row0 + 16 * i + j4);
 #pragma unroll
@@ -615,7 +661,7 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
           }
           // w[i]: key token j4 + i, query token n
 #pragma unroll
-          for (int i = 0; i < 4; ++i) o = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[i], j4 + i <= n ? w[i] : 0.0f, o, 0, 0, 0);
+          for (int i = 0; i < 4 && !AHEAD; ++i) o = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[i], j4 + i <= n ? w[i] : 0.0f, o, 0, 0, 0);
         }
       } else {
         if constexpr (HEAD) whole = false;
@@ -633,6 +679,7 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
               if constexpr (HEAD) key = (float)k[tok * a.ldp + r];
               else decay_and_key(g[tok * a.ldg + r], keys, keys ? (float)k[tok * a.ldp + r] : 0.0f, decay, key);
               s[i][e] = __builtin_fmaf(key, value, decay * s[i][e]);
+              left[i][e] *= decay;
               out = __builtin_fmaf(s[i][e], (float)q[tok * a.ldp + r] * a.q_scale, out);
             }
           out += __shfl_xor(out, 16, 64);
@@ -644,28 +691,67 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
           }
         }
       }
-      *reinterpret_cast<f32x4_t*>(red + (wave * B + b) * 256 + n * 16 + j4) = o;
+      if constexpr (!AHEAD) *reinterpret_cast<f32x4_t*>(red + (wave * B + b) * 256 + n * 16 + j4) = o;
     }
     __syncthreads();
   }
+  if (!AHEAD && a.seg_tokens && segment != (int)gridDim.z - 1) return;
   if (n < nv)
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
       const int d = row0 + 16 * i + j4;
-      if (d < dimp) *reinterpret_cast<f32x4_t*>(state + d) = s[i];
+      if (d < dimp) *reinterpret_cast<f32x4_t*>(AHEAD ? a.workspace + (segment + 1) * states + column + d : state + d) = s[i];
+    }
+  if (AHEAD && !HEAD && n == 0 && c0 == 0)
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+      const int d = row0 + 16 * i + j4;
+      if (d < dimp)
+        *reinterpret_cast<f32x4_t*>(a.workspace + (int64_t)(gridDim.z + 1) * states + ((int64_t)segment * a.heads + head) * dimp + d) = left[i];
     }
 }
 
+// Segments of a pass: as many as have a compute unit for each workgroup (a workgroup's LDS leaves no place for a second), where they pay: a
+// chunk of the launch ahead takes about 0.8 of one of outputs, and a launch more with the states between as long as three.
+// Heads of 128: 10 heads, 1,800 tokens (57 chunks, 3 segments) 144 -> 32 + 54 us; 16 heads, 700 tokens (22 chunks, 2 segments)
+// as long as in one.
+constexpr int kMaxSegments = 16;
+int segment_tokens(const GatedStateArgs& a, int chunk) {
+  const int64_t blocks = (int64_t)a.heads * ((a.vdim + 15) / 16), chunks = (a.M + chunk - 1) / chunk;
+  int64_t n = std::min<int64_t>(std::min<int64_t>(256 / blocks, kMaxSegments), chunks);
+  const int64_t floats = (int64_t)a.heads * (a.vdim + 1) * round_up(a.dim, 64);  // of a segment
+  if (a.workspace) n = std::min(n, a.workspace_floats / floats);
+  if (!a.workspace || n < 2) return 0;
+  const int64_t of_one = (chunks + n - 1) / n;
+  return 10 * chunks > 18 * of_one + 30 ? (int)of_one * chunk : 0;
+}
+
 template <typename T, int D, bool EVEN, bool KEYS, bool HEAD = false>
-int launch_chunk_form(const GatedStateArgs& a, hipStream_t st) {
+int launch_chunk_form(const GatedStateArgs& u, hipStream_t st) {
+  const dim3 g((unsigned)u.heads, (unsigned)((u.vdim + 15) / 16));
+  GatedStateArgs a = u;
+  if constexpr (EVEN) {
+    static bool raised_ahead = false;
+    a.seg_tokens = segment_tokens(a, chunk_blocks<D>() * kBlock);
+    if (a.seg_tokens) {
+      if (!raised_ahead) {
+        AWQ_HIP_TRY(hipFuncSetAttribute((const void*)gated_chunk_kernel<T, D, EVEN, KEYS, HEAD, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                        chunk_lds<D>()));
+        raised_ahead = true;
+      }
+      const dim3 ahead(g.x, g.y, (unsigned)((a.M - 1) / a.seg_tokens));
+      hipLaunchKernelGGL((gated_chunk_kernel<T, D, EVEN, KEYS, HEAD, true>), ahead, dim3(512), chunk_lds<D>(), st, a);
+      AWQ_HIP_TRY(hipGetLastError());
+    }
+  }
   static bool raised = false;  // more LDS than the default limit of a launch
   if (!raised) {
-    AWQ_HIP_TRY(hipFuncSetAttribute((const void*)gated_chunk_kernel<T, D, EVEN, KEYS, HEAD>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    AWQ_HIP_TRY(hipFuncSetAttribute((const void*)gated_chunk_kernel<T, D, EVEN, KEYS, HEAD, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     chunk_lds<D>()));
     raised = true;
   }
-  hipLaunchKernelGGL((gated_chunk_kernel<T, D, EVEN, KEYS, HEAD>), dim3((unsigned)a.heads, (unsigned)((a.vdim + 15) / 16)), dim3(512),
-                     chunk_lds<D>(), st, a);
+  const dim3 all(g.x, g.y, a.seg_tokens ? (unsigned)((a.M + a.seg_tokens - 1) / a.seg_tokens) : 1u);
+  hipLaunchKernelGGL((gated_chunk_kernel<T, D, EVEN, KEYS, HEAD, false>), all, dim3(512), chunk_lds<D>(), st, a);
   AWQ_HIP_TRY(hipGetLastError());
   return AWQ_OK;
 }
@@ -738,6 +824,8 @@ GatedStateArgs of_linear(const LinearAttnArgs& u) {
   a.o = u.o;
   a.M = u.M;
   a.pos = u.pos;
+  a.workspace = u.workspace;
+  a.workspace_floats = u.workspace_floats;
   return a;
 }
 

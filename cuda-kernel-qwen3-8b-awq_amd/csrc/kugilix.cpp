@@ -441,6 +441,8 @@ int KugilixEngine::run_pass(bool one, const int32_t* ids, int64_t M, PassPos pos
       a.o = b.o;
       a.M = M;
       a.pos = pos;
+      a.workspace = dense_ws;
+      a.workspace_floats = dense_ws_floats;
       beside = s.ff && linear_takes_product(a, f32);
       if (int rc = launch_linear_attention(a, f32, stream, beside ? &down : nullptr)) return rc;
       gate = (const char*)b.proj + (int64_t)s.heads * (2 * s.dim + s.vdim) * unit();

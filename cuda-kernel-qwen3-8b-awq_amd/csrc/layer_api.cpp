@@ -147,9 +147,8 @@ extern "C" int awq_window_attention(const awq_window_args* u, int32_t f32, void*
   return launch_window_attention(a, f32 != 0, (hipStream_t)stream);
 }
 
-extern "C" int awq_linear_attention(const void* proj, int64_t ldp, int32_t heads, int32_t dim, int32_t vdim,
-                                    const float* decay, const float* log2_decay, float* state, float* o, int64_t n_tokens,
-                                    int64_t pos0, int32_t f32, void* stream) {
+static LinearAttnArgs linear_of(const void* proj, int64_t ldp, int32_t heads, int32_t dim, int32_t vdim, const float* decay,
+                                const float* log2_decay, float* state, float* o, int64_t n_tokens, int64_t pos0) {
   LinearAttnArgs a;
   a.proj = proj;
   a.ldp = ldp;
@@ -162,12 +161,30 @@ extern "C" int awq_linear_attention(const void* proj, int64_t ldp, int32_t heads
   a.o = o;
   a.M = n_tokens;
   a.pos = at_position(pos0);
+  return a;
+}
+
+extern "C" int awq_linear_attention(const void* proj, int64_t ldp, int32_t heads, int32_t dim, int32_t vdim,
+                                    const float* decay, const float* log2_decay, float* state, float* o, int64_t n_tokens,
+                                    int64_t pos0, int32_t f32, void* stream) {
+  return launch_linear_attention(linear_of(proj, ldp, heads, dim, vdim, decay, log2_decay, state, o, n_tokens, pos0), f32 != 0,
+                                 (hipStream_t)stream);
+}
+
+extern "C" int awq_linear_attention_segments(const void* proj, int64_t ldp, int32_t heads, int32_t dim, int32_t vdim,
+                                             const float* decay, const float* log2_decay, float* state, float* o, int64_t n_tokens,
+                                             int64_t pos0, int32_t f32, float* workspace, int64_t workspace_floats, void* stream) {
+  LinearAttnArgs a = linear_of(proj, ldp, heads, dim, vdim, decay, log2_decay, state, o, n_tokens, pos0);
+  a.workspace = workspace;
+  a.workspace_floats = workspace_floats;
   return launch_linear_attention(a, f32 != 0, (hipStream_t)stream);
 }
 
-extern "C" int awq_gated_state(const awq_gated_state_args* u, int32_t f32, void* stream) {
+extern "C" int awq_gated_state_segments(const awq_gated_state_args* u, int32_t f32, float* workspace, int64_t workspace_floats, void* stream) {
   AWQ_REQUIRE(u != nullptr, "args is NULL");
   GatedStateArgs a;
+  a.workspace = workspace;
+  a.workspace_floats = workspace_floats;
   a.q = u->q;
   a.k = u->k;
   a.v = u->v;
@@ -187,6 +204,10 @@ extern "C" int awq_gated_state(const awq_gated_state_args* u, int32_t f32, void*
   a.ctx = u->ctx;
   a.eps = u->eps;
   return launch_gated_state(a, f32 != 0, (hipStream_t)stream);
+}
+
+extern "C" int awq_gated_state(const awq_gated_state_args* u, int32_t f32, void* stream) {
+  return awq_gated_state_segments(u, f32, nullptr, 0, stream);
 }
 
 extern "C" int awq_head_norm(const float* o, const void* gate, int64_t ldg, const float* w, void* ctx, int64_t ldc, int32_t heads,

@@ -243,6 +243,9 @@ struct LinearAttnArgs {
   float* o = nullptr;  // [M][heads * vdim]
   int64_t M = 0;
   PassPos pos;
+  float* workspace = nullptr;  // states between segments of a pass that go side by side; may be null
+  int64_t workspace_floats = 0;
+  int32_t seg_tokens = 0;      // of a segment (the launch sets it), 0: one after the other
 };
 int64_t linear_state_floats(int32_t heads, int32_t dim, int32_t vdim);
 // beside (where linear_takes_product): a product in the same launch
@@ -269,6 +272,9 @@ struct GatedStateArgs {
   float* o = nullptr;  // [M][heads * vdim]
   int64_t M = 0;
   PassPos pos;
+  float* workspace = nullptr;    // states between segments of a pass that go side by side; may be null
+  int64_t workspace_floats = 0;
+  int32_t seg_tokens = 0;        // of a segment (the launch sets it), 0: one after the other
   // one token: ctx = the heads' norm below instead of o, in the same launch; null: none
   const float* norm = nullptr;
   const void* gate = nullptr;

@@ -102,8 +102,12 @@ constexpr int linear_chunk_lds() {
   return (kChunk * (D + 16) + 4 * 32 * kVStride + 3 * 32 * (D + 8)) * 2;
 }
 
-// WHOLE: rows of q, k and v are 16-byte pieces
-template <int D, bool WHOLE>
+// WHOLE: rows of q, k and v are 16-byte pieces.
+// Where heads and columns leave compute units without a workgroup, a pass is cut into segments (a.seg_tokens, blockIdx.z) that go side by
+// side, in two launches.  AHEAD: for every segment but the last the state that it adds to an empty one; the first starts from the
+// state itself and keeps a copy.  Then the outputs, every segment starting from the sum of those ahead of it, decayed, and the last one's
+// state.  The workspace holds [segments][heads][vdim][dimp]: the state ahead of the pass, then what the segments but the last add.
+template <int D, bool WHOLE, bool AHEAD>
 __global__ __launch_bounds__(512) void linear_chunk_kernel(LinearAttnArgs a) {
   extern __shared__ __attribute__((aligned(16))) char lds_raw[];
   constexpr int KS = D + 16, SS = D + 8, NT = D / 32;  // NT tiles of 32 state rows, over four wavefronts
@@ -117,15 +121,18 @@ __global__ __launch_bounds__(512) void linear_chunk_kernel(LinearAttnArgs a) {
   const int wave = wave8 & 3;
   const bool outputs = wave8 < 4;
   const int n = lane & 31, kh = lane >> 5;
-  const int M = (int)a.M;
-  const bf16_t* const p = reinterpret_cast<const bf16_t*>(a.proj);
+  const int segment = blockIdx.z;
+  const int64_t tok0 = (int64_t)segment * a.seg_tokens;
+  const int M = (int)(a.seg_tokens ? min((int64_t)a.seg_tokens, a.M - tok0) : a.M);  // tokens of this segment, counted from tok0
+  const bf16_t* const p = reinterpret_cast<const bf16_t*>(a.proj) + tok0 * a.ldp;
   const bf16_t* const q = p + (int64_t)head * a.dim;
   const bf16_t* const k = p + (int64_t)(a.heads + head) * a.dim;
   const bf16_t* const v = p + (int64_t)2 * a.heads * a.dim + (int64_t)head * a.vdim + v0;
   const int nv = min(32, a.vdim - v0);
   const float lg = a.log2_decay[head];
   const int dimp = (a.dim + 63) & ~63;
-  float* const state = a.state + ((int64_t)head * a.vdim + v0 + n) * dimp;
+  const int64_t column = ((int64_t)head * a.vdim + v0 + n) * dimp, states = (int64_t)a.heads * a.vdim * dimp;
+  float* const state = a.state + column;
 
   auto piece = [&](const bf16_t* row, int at, int len) __attribute__((always_inline)) {
     bf16x8_t r;
@@ -140,6 +147,14 @@ __global__ __launch_bounds__(512) void linear_chunk_kernel(LinearAttnArgs a) {
     return r;
   };
 
+  float over = 0.0f, over_rest = 0.0f;  // the decay's power over a segment, a sum of two numbers (with one the states' errors grew by a half)
+  if (!AHEAD && segment > 1) {
+    double x = 1.0, y = (double)a.decay[head];
+    for (int e = a.seg_tokens; e; e >>= 1, y *= y)
+      if (e & 1) x *= y;
+    over = (float)x;
+    over_rest = (float)(x - (double)over);
+  }
   // the state: rows 32 (wave + 4 i) + 8 g + 4 kh + j of column n in s[i][4 g + j]
   f32x16_t s[TPW];
   const bool holds = !outputs && wave < NT;
@@ -150,7 +165,19 @@ __global__ __launch_bounds__(512) void linear_chunk_kernel(LinearAttnArgs a) {
     for (int g = 0; g < 4; ++g) {
       const int d = 32 * (wave + 4 * i) + 8 * g + 4 * kh;
       f32x4_t x = {0.0f, 0.0f, 0.0f, 0.0f};
-      if (!fresh && holds && d < dimp && n < nv) x = *reinterpret_cast<const f32x4_t*>(state + d);
+      const bool there = holds && d < dimp && n < nv;
+      if (AHEAD || !a.seg_tokens) {
+        if (!fresh && there && segment == 0) x = *reinterpret_cast<const f32x4_t*>(state + d);
+        if (AHEAD && segment == 0 && there) *reinterpret_cast<f32x4_t*>(a.workspace + column + d) = x;
+      } else if (there) {
+        const float* const from = a.workspace + column + d;
+        x = *reinterpret_cast<const f32x4_t*>(from + (segment == 0 ? 0 : states));
+        for (int j = 2; j <= segment; ++j) {
+          const f32x4_t add = *reinterpret_cast<const f32x4_t*>(from + j * states);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[e] = __builtin_fmaf(x[e], over, __builtin_fmaf(x[e], over_rest, add[e]));
+        }
+      }
 #pragma unroll
       for (int j = 0; j < 4; ++j) s[i][4 * g + j] = x[j];
     }
@@ -179,7 +206,7 @@ __global__ __launch_bounds__(512) void linear_chunk_kernel(LinearAttnArgs a) {
 #pragma unroll
   for (int i = 0; i < 16; ++i) wr[i] = __builtin_amdgcn_exp2f((float)(31 - (8 * (i >> 2) + 4 * kh + (i & 3))) * lg);
   load(0);
-  if (outputs) load_q(0);
+  if (!AHEAD && outputs) load_q(0);
   for (int c0 = 0; c0 < M; c0 += kChunk) {
     const int len = min(kChunk, M - c0);
     __syncthreads();  // the previous chunk's readers are done
@@ -238,7 +265,7 @@ __global__ __launch_bounds__(512) void linear_chunk_kernel(LinearAttnArgs a) {
     __syncthreads();
     if (c0 + kChunk < M) load(c0 + kChunk);
 
-    if (outputs && 32 * wave < len) {
+    if (!AHEAD && outputs && 32 * wave < len) {
       // one accumulator per term of the state: three independent chains of matrix instructions
       f32x16_t om[3];
 #pragma unroll
@@ -300,7 +327,7 @@ __global__ __launch_bounds__(512) void linear_chunk_kernel(LinearAttnArgs a) {
       for (int i = 0; i < 16; ++i) o[i] += o2[i];
       if (c0 + kChunk < M) load_q(c0 + kChunk);
       if (tq < len) {
-        float* out = a.o + (int64_t)(c0 + tq) * a.heads * a.vdim + (int64_t)head * a.vdim + v0;
+        float* out = a.o + (tok0 + c0 + tq) * a.heads * a.vdim + (int64_t)head * a.vdim + v0;
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
           const int c = 8 * g + 4 * kh;
@@ -351,6 +378,7 @@ __global__ __launch_bounds__(512) void linear_chunk_kernel(LinearAttnArgs a) {
         for (int j = 0; j < 16; ++j) s[i][j] += sl[i][j];
     }
   }
+  if (!AHEAD && a.seg_tokens && segment != (int)gridDim.z - 1) return;
   if (holds && n < nv)
 #pragma unroll
     for (int i = 0; i < TPW; ++i)
@@ -358,20 +386,47 @@ __global__ __launch_bounds__(512) void linear_chunk_kernel(LinearAttnArgs a) {
       for (int g = 0; g < 4; ++g) {
         const int d = 32 * (wave + 4 * i) + 8 * g + 4 * kh;
         if (d < dimp)
-          *reinterpret_cast<f32x4_t*>(state + d) = f32x4_t{s[i][4 * g], s[i][4 * g + 1], s[i][4 * g + 2], s[i][4 * g + 3]};
+          *reinterpret_cast<f32x4_t*>(AHEAD ? a.workspace + (segment + 1) * states + column + d : state + d) = f32x4_t{s[i][4 * g], s[i][4 * g + 1], s[i][4 * g + 2], s[i][4 * g + 3]};
       }
 }
 
+// Segments of a pass: as many as have a compute unit for each workgroup (a workgroup's LDS leaves no place for a second), where they pay: a
+// chunk of the launch ahead takes about 0.7 of one of outputs, and a launch more with the states between as long as three.  Width 1,024
+// (8 heads), 3,000 tokens in two passes of 12 chunks: the whole prompt 2,330 -> 2,130 us, 900 tokens 913 -> 860, 15 heads and 1,500 tokens 1,995 ->
+// 1,920; where the rule says no, 24 heads and 2,000 tokens 4,305 -> 4,312, 20 heads and 600 tokens 1,483 -> 1,512, 10 and 400 697 -> 718.
+constexpr int kMaxSegments = 16;
+int segment_tokens(const LinearAttnArgs& a) {
+  const int64_t blocks = (int64_t)a.heads * ((a.vdim + 31) / 32), chunks = (a.M + kChunk - 1) / kChunk;
+  int64_t n = std::min<int64_t>(std::min<int64_t>(256 / blocks, kMaxSegments), chunks);
+  if (a.workspace) n = std::min(n, a.workspace_floats / linear_state_floats(a.heads, a.dim, a.vdim));
+  if (!a.workspace || n < 2) return 0;
+  const int64_t of_one = (chunks + n - 1) / n;
+  return 10 * chunks > 17 * of_one + 30 ? (int)of_one * kChunk : 0;
+}
+
 template <int D, bool WHOLE>
-int launch_chunks(const LinearAttnArgs& a, hipStream_t st) {
+int launch_chunks(const LinearAttnArgs& u, hipStream_t st) {
   static bool raised = false;  // more LDS than the default limit of a launch
   if (!raised) {
-    AWQ_HIP_TRY(hipFuncSetAttribute((const void*)linear_chunk_kernel<D, WHOLE>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    AWQ_HIP_TRY(hipFuncSetAttribute((const void*)linear_chunk_kernel<D, WHOLE, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     linear_chunk_lds<D>()));
+    if constexpr (WHOLE)
+      AWQ_HIP_TRY(hipFuncSetAttribute((const void*)linear_chunk_kernel<D, WHOLE, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                      linear_chunk_lds<D>()));
     raised = true;
   }
-  hipLaunchKernelGGL((linear_chunk_kernel<D, WHOLE>), dim3((unsigned)a.heads, (unsigned)((a.vdim + 31) / 32)), dim3(512),
-                     linear_chunk_lds<D>(), st, a);
+  LinearAttnArgs a = u;
+  dim3 g((unsigned)a.heads, (unsigned)((a.vdim + 31) / 32));
+  if constexpr (WHOLE) {
+    a.seg_tokens = segment_tokens(a);
+    if (a.seg_tokens) {
+      g.z = (unsigned)((a.M - 1) / a.seg_tokens);
+      hipLaunchKernelGGL((linear_chunk_kernel<D, WHOLE, true>), g, dim3(512), linear_chunk_lds<D>(), st, a);
+      AWQ_HIP_TRY(hipGetLastError());
+      ++g.z;
+    }
+  }
+  hipLaunchKernelGGL((linear_chunk_kernel<D, WHOLE, false>), g, dim3(512), linear_chunk_lds<D>(), st, a);
   AWQ_HIP_TRY(hipGetLastError());
   return AWQ_OK;
 }

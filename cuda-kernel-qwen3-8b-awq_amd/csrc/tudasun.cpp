@@ -682,6 +682,8 @@ int TudasunEngine::mix(int i, Buffers& b, int64_t M, PassPos pos) {
   a.o = b.o;
   a.M = M;
   a.pos = pos;
+  a.workspace = dense_ws;
+  a.workspace_floats = dense_ws_floats;
   const void* gate = s.type == MIX_GLA ? proj(2 * keys + mixed) : nullptr;
   if (M == 1) {
     a.norm = L.mix_norm;

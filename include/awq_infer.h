@@ -572,6 +572,12 @@ int awq_window_attention(const awq_window_args* args, int32_t f32, void* stream)
 int awq_linear_attention(const void* proj, int64_t ldp, int32_t heads, int32_t dim, int32_t vdim, const float* decay,
                          const float* log2_decay, float* state, float* o, int64_t n_tokens, int64_t pos0, int32_t f32,
                          void* stream);
+/* The same with room for the states between segments of a pass, which then go side by
+ * side where heads and columns are few: workspace_floats floats, 16-byte aligned, at
+ * least heads * vdim * round_up(dim, 64) for each of two segments or more. */
+int awq_linear_attention_segments(const void* proj, int64_t ldp, int32_t heads, int32_t dim, int32_t vdim, const float* decay,
+                                  const float* log2_decay, float* state, float* o, int64_t n_tokens, int64_t pos0, int32_t f32,
+                                  float* workspace, int64_t workspace_floats, void* stream);
 
 /* Linear attention whose state decays per channel: per head
  * S <- diag(decay) S + k v^T, o = S^T (q_scale q); state as above.  q, v
@@ -593,6 +599,8 @@ typedef struct awq_gated_state_args {
   float eps, reserved;
 } awq_gated_state_args;
 int awq_gated_state(const awq_gated_state_args* args, int32_t f32, void* stream);
+/* the same with room for segments, heads * (vdim + 1) * round_up(dim, 64) floats each */
+int awq_gated_state_segments(const awq_gated_state_args* args, int32_t f32, float* workspace, int64_t workspace_floats, void* stream);
 /* ctx[t][h][c] = RMS norm over each head's vdim values of o, times w [vdim], times silu(gate) (gate NULL: 1) */
 int awq_head_norm(const float* o, const void* gate, int64_t ldg, const float* w, void* ctx, int64_t ldc, int32_t heads,
                   int32_t vdim, int64_t n_tokens, float eps, int32_t f32, void* stream);

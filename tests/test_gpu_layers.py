@@ -632,6 +632,43 @@ def test_roundings_of_linear_attention(awq, lib, dev, f32, T, sizes, heads, dim,
     assert worst[0] < 4 * 2.0 ** -25 and worst[1] < min(T, 256) ** 0.5 * 2.0 ** -25
 
 
+@pytest.mark.parametrize("f32", FORMATS, ids=["bf16", "f32"])
+@pytest.mark.parametrize("heads,dim,vdim", [(3, 24, 16), (2, 128, 96), (1, 256, 40), (2, 100, 36), (4, 64, 8), (80, 16, 8)])
+def test_segments_of_linear_attention(awq, lib, dev, f32, heads, dim, vdim):
+    """segments side by side, by room for none, two, three and all of them: whole and ragged last ones, behind a state.  In bfloat16 rows that are not
+    whole pieces have none; 80 heads leave three.  Bound: as in test_linear_attention"""
+    print("segments of linear attention", heads, dim, vdim, f32, flush=True)
+    rng = np.random.default_rng(dim)
+    T, n = 1700, heads * (2 * dim + vdim)
+    ldp = (n + 7) // 8 * 8
+    proj, pv = dev.act(np.pad(rng.standard_normal((T, n)) * 0.5 + 0.2, ((0, 0), (0, ldp - n))), f32)
+    q, k = (pv[:, i * heads * dim:(i + 1) * heads * dim].reshape(T, heads, dim) for i in (0, 1))
+    v = pv[:, 2 * heads * dim:n].reshape(T, heads, vdim)
+    decay = np.array(([0.999, 0.3, 0.9, 1e-6] * heads)[:heads], np.float32)
+    want, S = plain.linear_attention(q, k, v, decay.astype(np.float64))
+    d_decay, d_lg = dev.f(decay), dev.f(np.log2(decay.astype(np.float64)))
+    dimp = (dim + 63) // 64 * 64
+    room = heads * (vdim + 1) * dimp
+    # A weight's two terms of 8 bits are 2^-17 off, and a head of 16 inputs that forgets at once cancels up to 4.2 to 1 in an output: 3.2e-5, one chunk
+    # after the other.  Beside that a segment adds two roundings of binary32 to the states: 2e-7.
+    for sizes, rooms in (([T], (0, 16, 3, 2, 1)), ([1, 1100, 599], (0, 16)), ([1152, 548], (0, 16))):
+        for segments in rooms:
+            ws, state, o = dev.empty((max(4, segments * room),), True), dev.empty((heads, vdim, dimp), True), dev.empty((T, heads * vdim), True)
+            at = i = 0
+            while at < T:
+                m = min(sizes[i % len(sizes)], T - at)
+                awq.check(lib.awq_linear_attention_segments(proj[at:].data_ptr(), ldp, heads, dim, vdim, d_decay.data_ptr(), d_lg.data_ptr(),
+                                                            state.data_ptr(), o[at:].data_ptr(), m, at, f32, ws.data_ptr(), segments * room, dev.stream))
+                at, i = at + m, i + 1
+            got, s = dev.host(o).reshape(T, heads, vdim), dev.host(state)[:, :, :dim].transpose(0, 2, 1)
+            off = [km.rms_error(got[:, h], want[:, h]) for h in range(heads)]
+            alone = off if segments == 0 else alone
+            assert max(off) < (3e-5 if dim > 16 else 3.3e-5), (sizes, segments)
+            for h in range(heads):
+                assert off[h] < alone[h] + 2e-7, (sizes, segments, h)
+                assert np.abs(s[h] - S[h]).max() <= 3e-5 * np.abs(S[h]).max(), (sizes, segments, h)
+
+
 def attend(awq, lib, dev, f32, proj, heads, kv, dim, vdim, window, scale, eps, temp, sizes, T, slots, max_pos):
     """the attention of T tokens in portions; proj: the tensor with all tokens' projections (kept as it is)"""
     kr, vr = lib.awq_window_row(dim), lib.awq_window_row(vdim)

@@ -390,6 +390,51 @@ def test_several_tokens_of_a_state_are_those_of_single_ones(awq, lib, dev, f32, 
 
 
 @pytest.mark.parametrize("f32", FORMATS, ids=["bf16", "f32"])
+@pytest.mark.parametrize("keys", [True, False], ids=["keys", "no keys"])
+@pytest.mark.parametrize("heads,dim,vdim", [(3, 20, 12), (4, 64, 40), (2, 128, 96), (2, 256, 40), (3, 101, 35), (70, 16, 16)])
+def test_segments_of_a_state(awq, lib, dev, f32, keys, heads, dim, vdim):
+    """segments side by side, by room for none, two, three and all of them: whole and ragged last ones, behind a state, with blocks that go token by
+    token and a value that is infinite.  Odd dims have none; 70 heads leave three.  Bound: as in test_gated_state"""
+    print("segments of a state", heads, dim, vdim, f32, keys, flush=True)
+    rng = np.random.default_rng(dim)
+    T, hd = 801, heads * dim
+    q, k, v, rate = state_inputs(rng, T, heads, dim, vdim, keys)
+    parts = [q.reshape(T, -1)] + ([k.reshape(T, -1)] if keys else []) + [v.reshape(T, -1)]
+    n = sum(p.shape[1] for p in parts)
+    ldp = up(n, 8)
+    x = np.pad(np.concatenate(parts, axis=1), ((0, 0), (0, ldp - n)))
+    g = (-rate if keys else 1.0 - 2.0 ** -rate).astype(np.float32)
+    decay = 2.0 ** g.astype(np.float64) if keys else 1.0 - g.astype(np.float64)
+    d_g, room = dev.f(g.reshape(T, hd)), heads * (vdim + 1) * up(dim, 64)
+
+    def run(proj, sizes, segments):
+        ws = dev.empty((max(4, segments * room),), True)
+        state, o = dev.empty((heads, vdim, up(dim, 64)), True), dev.empty((T, heads * vdim), True)
+        for t, m in portions(T, sizes):
+            base, unit = proj[t:].data_ptr(), proj.element_size()
+            a = awq.AwqGatedStateArgs(base, base + hd * unit if keys else None, base + (n - heads * vdim) * unit, d_g[t:].data_ptr(), ldp, hd,
+                                      heads, dim, vdim, 0.3, state.data_ptr(), o[t:].data_ptr(), m, t)
+            awq.check(lib.awq_gated_state_segments(ctypes.byref(a), f32, ws.data_ptr(), segments * room, dev.stream))
+        return dev.host(o).reshape(T, heads, vdim), dev.host(state)[:, :, :dim]
+
+    proj, pv = dev.act(x, f32)
+    kv = pv[:, hd:2 * hd].reshape(T, heads, dim) if keys else g.astype(np.float64)
+    want, S = plain.gated_state(pv[:, :hd].reshape(T, heads, dim) * 0.3, kv, pv[:, n - heads * vdim:n].reshape(T, heads, vdim), decay)
+    for sizes, segments in (([T], 16), ([T], 2), ([T], 3), ([T], 1), ([1, 500, 300], 16), ([256, 545], 16)):
+        got, s = run(proj, sizes, segments)
+        for h in range(heads):
+            assert km.rms_error(got[:, h], want[:, h]) < 5e-5, (sizes, segments, h)
+            assert np.abs(s[h].T - S[h]).max() <= 5e-5 * np.abs(S[h]).max(), (sizes, segments, h)
+    x[300, n - heads * vdim + 1] = np.inf  # column 1 of the first head
+    proj, _ = dev.act(x, f32)
+    alone, beside = run(proj, [T], 0), run(proj, [T], 16)
+    for a, b in zip(alone, beside):
+        fine = np.isfinite(a)
+        assert not fine.all() and np.array_equal(fine, np.isfinite(b))
+        assert np.abs(a[fine] - b[fine]).max() < 2e-5 * np.abs(a[fine]).max()
+
+
+@pytest.mark.parametrize("f32", FORMATS, ids=["bf16", "f32"])
 def test_a_key_far_back_in_a_state(awq, lib, dev, f32):
     """one token writes a marked row, hundreds of tokens later a query reads just that row"""
     T, dim, vdim, far = 420, 64, 32, 37
