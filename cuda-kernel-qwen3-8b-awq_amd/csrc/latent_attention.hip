@@ -2,6 +2,7 @@
 // position, beside a rotated key part that the heads share; softmax with a learned score that has no key.
 #include "lane_sums.hpp"
 #include "query_attention.hpp"
+#include "tile_halves.hpp"
 
 namespace {
 
@@ -753,14 +754,18 @@ __global__ __launch_bounds__(256) void latent_value_one_kernel(LatentAttnArgs a,
 // 128 queries of one head per workgroup, 32 per wavefront, keys and values of 32 positions at a time through LDS; the
 // operands as in window_attention.hip.  The sink is the state that a query's running maximum and sum start from.
 constexpr int kTileQueries = 128, kTileKeys = 32;
+constexpr float kSlack = 8.0f;
 
-template <int DK, int DV>
-__global__ __launch_bounds__(256, (DK + DV > 256) ? 1 : 2) void latent_tile_kernel(LatentAttnArgs a) {
+template <int DK, int DV, int HALVES>
+__global__ __launch_bounds__(256 * HALVES, (DK + DV > 256) ? 1 : 2) void latent_tile_kernel(LatentAttnArgs a) {
   constexpr int KS = DK + 8, VS = DV + 16;
   constexpr int KP = DK / 64, VP = DV / 64;  // 16-byte pieces of a tile per thread
-  __shared__ __attribute__((aligned(16))) bf16_t ks2[2 * kTileKeys * KS];
-  __shared__ __attribute__((aligned(16))) bf16_t vs2[2 * kTileKeys * VS];
-  const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  constexpr int kTiles = 2 * kTileKeys * (KS + VS);
+  __shared__ __attribute__((aligned(16))) bf16_t tiles[HALVES * kTiles];
+  __shared__ float ml[HALVES == 2 ? 1024 : 1];
+  const int half = HALVES == 2 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) : 0;
+  bf16_t *const ks2 = tiles + half * kTiles, *const vs2 = ks2 + 2 * kTileKeys * KS;
+  const int h = blockIdx.x, tid = threadIdx.x & 255, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, kh = lane >> 5;
   const int M = (int)a.M, pos0 = a.pos.pos0;
   const int q_first = (gridDim.y - 1 - blockIdx.y) * kTileQueries;  // the longest rows first
@@ -787,7 +792,8 @@ __global__ __launch_bounds__(256, (DK + DV > 256) ? 1 : 2) void latent_tile_kern
   for (int d = 0; d < DV / 32; ++d)
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[d][i] = 0.0f;
-  float m_run = a.sink ? a.sink[h] * kLog2e : -1e30f, l_run = a.sink ? 1.0f : 0.0f;
+  const bool sink = a.sink && half == 0;
+  float m_run = sink ? a.sink[h] * kLog2e : -1e30f, l_run = sink ? 1.0f : 0.0f;
   const float mul = a.scale * kLog2e;
   struct TileRegs {
     bf16x8_t k[KP], v[VP];
@@ -797,15 +803,15 @@ __global__ __launch_bounds__(256, (DK + DV > 256) ? 1 : 2) void latent_tile_kern
     if (k0 >= k_end) return;
 #pragma unroll
     for (int i = 0; i < KP; ++i) {
-      const int pc = tid + i * 256, key = min(k0 + pc / (DK / 8), k_end - 1), at = (pc % (DK / 8)) * 8;
-      r.k[i] = at < a.dim ? *reinterpret_cast<const bf16x8_t*>(kx + key * ldkv + at)
-               : at < qk  ? *reinterpret_cast<const bf16x8_t*>(cache + (int64_t)key * row + at - a.dim)
-                          : zero;
+      // (past a row's end its last piece, which meets zeros of the query: a condition around a request has the ones ahead of it waited for)
+      const int pc = tid + i * 256, key = min(k0 + pc / (DK / 8), k_end - 1), at = min((pc % (DK / 8)) * 8, qk - 8);
+      const bf16_t* const from = at < a.dim ? kx + key * ldkv + at : cache + (int64_t)key * row + at - a.dim;
+      r.k[i] = *reinterpret_cast<const bf16x8_t*>(from);
     }
 #pragma unroll
     for (int i = 0; i < VP; ++i) {
-      const int pc = tid + i * 256, key = min(k0 + pc / (DV / 8), k_end - 1), at = (pc % (DV / 8)) * 8;
-      r.v[i] = at < a.vdim ? *reinterpret_cast<const bf16x8_t*>(vx + key * ldkv + at) : zero;
+      const int pc = tid + i * 256, key = min(k0 + pc / (DV / 8), k_end - 1), at = min((pc % (DV / 8)) * 8, a.vdim - 8);
+      r.v[i] = *reinterpret_cast<const bf16x8_t*>(vx + key * ldkv + at);
     }
   };
   auto store_tile = [&](int half, const TileRegs& r) __attribute__((always_inline)) {
@@ -820,17 +826,37 @@ __global__ __launch_bounds__(256, (DK + DV > 256) ? 1 : 2) void latent_tile_kern
       *reinterpret_cast<bf16x8_t*>(vs2 + (half * kTileKeys + key) * VS + at) = r.v[i];
     }
   };
-  auto step = [&](int k0, int half) __attribute__((always_inline)) {
+  // Bound by the chain of a wavefront that has a SIMD nearly to itself, so operands are read four products ahead and the first values
+  // ahead of the softmax.  (Two tiles to a softmax: no registers for it with halves, without them no faster.)
+  auto step = [&](int k0, int at) __attribute__((always_inline)) {
     if (k0 > w_last) return;  // no query of this wavefront sees a key of the tile
-    const bf16_t* ks = ks2 + half * kTileKeys * KS;
-    const bf16_t* vs = vs2 + half * kTileKeys * VS;
+    const bf16_t* const klane = ks2 + (at * kTileKeys + n) * KS + 8 * kh;
+    const int L16 = lane & 15;
+    const bf16_t* const vlane = vs2 + (at * kTileKeys + 4 * kh + (L16 >> 2)) * VS + 16 * ((lane >> 4) & 1) + 4 * (L16 & 3);
+    auto values = [&](int j, int d) __attribute__((always_inline)) {
+      const bf16_t* vp = vlane + 16 * j * VS + d * 32;
+      const short4_t l = __builtin_amdgcn_ds_read_tr16_b64_v4i16((short4_t __attribute__((address_space(3)))*)vp);
+      const short4_t u = __builtin_amdgcn_ds_read_tr16_b64_v4i16((short4_t __attribute__((address_space(3)))*)(vp + 8 * VS));
+      const bf16x4_t l4 = __builtin_bit_cast(bf16x4_t, l), u4 = __builtin_bit_cast(bf16x4_t, u);
+      return bf16x8_t{l4[0], l4[1], l4[2], l4[3], u4[0], u4[1], u4[2], u4[3]};
+    };
     f32x16_t s;
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = 0.0f;
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int d = 0; d < DK / 16; ++d)
-      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8_t*>(ks + n * KS + 16 * d + 8 * kh), qop[d], s,
-                                                  0, 0, 0);
+      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8_t*>(klane + 16 * d), qop[d], s, 0, 0, 0);
+    bf16x8_t vv[DV / 32];  // (of the first slice)
+#pragma unroll
+    for (int d = 0; d < DV / 32; ++d) vv[d] = values(0, d);
+    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+    for (int d = 0; d < DK / 16; ++d) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
     // s[i]: key k0 + 8 (i / 4) + 4 kh + i % 4 for this lane's query
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] *= mul;
@@ -841,75 +867,99 @@ __global__ __launch_bounds__(256, (DK + DV > 256) ? 1 : 2) void latent_tile_kern
     float mx = s[0];
 #pragma unroll
     for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float m_new = fmaxf(m_run, mx);
-    const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-    float rs = 0.0f;
-    bf16x8_t hi[2], lo[2];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const float p = __builtin_amdgcn_exp2f(s[i] - m_new);
-      rs += p;
-      hi[i >> 3][i & 7] = (bf16_t)p;
-      lo[i >> 3][i & 7] = (bf16_t)(p - (float)hi[i >> 3][i & 7]);
-    }
-    rs += __shfl_xor(rs, 32, 64);
-    l_run = l_run * alpha + rs;
-    m_run = m_new;
-    if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
+    const HalfPair best = half_pair(mx);
+    mx = fmaxf(best.low, best.high);
+    // the maximum that weights are relative to moves only once it is 2^kSlack behind: sums grow by as much and no more
+    if (__builtin_amdgcn_ballot_w64(!(mx <= m_run + kSlack)) != 0) {
+      const float m_new = fmaxf(m_run, mx), alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+      l_run *= alpha;
+      m_run = m_new;
 #pragma unroll
       for (int d = 0; d < DV / 32; ++d)
 #pragma unroll
         for (int i = 0; i < 16; ++i) o[d][i] *= alpha;
     }
-    const int L16 = lane & 15;
-    const bf16_t* vlane = vs + (4 * kh + (L16 >> 2)) * VS + 16 * ((lane >> 4) & 1) + 4 * (L16 & 3);
+    float rs = 0.0f;
+    bf16x8_t hi[2], lo[2];
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int i = 0; i < 16; ++i) {
+      const float p = __builtin_amdgcn_exp2f(s[i] - m_run);
+      rs += p;
+      hi[i >> 3][i & 7] = (bf16_t)p;
+      lo[i >> 3][i & 7] = (bf16_t)(p - (float)hi[i >> 3][i & 7]);
+    }
+    const HalfPair sums = half_pair(rs);
+    l_run += sums.low + sums.high;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+#pragma unroll
+      for (int d = 0; d < DV / 32; ++d) o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vv[d], hi[j], o[d], 0, 0, 0);
 #pragma unroll
       for (int d = 0; d < DV / 32; ++d) {
-        const bf16_t* vp = vlane + 16 * j * VS + d * 32;
-        const short4_t l = __builtin_amdgcn_ds_read_tr16_b64_v4i16((short4_t __attribute__((address_space(3)))*)vp);
-        const short4_t u = __builtin_amdgcn_ds_read_tr16_b64_v4i16((short4_t __attribute__((address_space(3)))*)(vp + 8 * VS));
-        const bf16x4_t l4 = __builtin_bit_cast(bf16x4_t, l), u4 = __builtin_bit_cast(bf16x4_t, u);
-        const bf16x8_t vv = {l4[0], l4[1], l4[2], l4[3], u4[0], u4[1], u4[2], u4[3]};
-        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vv, hi[j], o[d], 0, 0, 0);
-        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vv, lo[j], o[d], 0, 0, 0);
+        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vv[d], lo[j], o[d], 0, 0, 0);
+        if (j + 1 < 2) vv[d] = values(j + 1, d);
       }
+    }
   };
-  load_tile(0, ra);
-  load_tile(kTileKeys, rb);
-  for (int k0 = 0; k0 < k_end; k0 += 2 * kTileKeys) {
+  const int first = 2 * kTileKeys * half;
+  load_tile(first, ra);
+  load_tile(first + kTileKeys, rb);
+  // The first products wait for the queries here: inside the loop, where the number of requests on their way is not known, that wait would be one for
+  // everything, the next tiles with it.
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+  for (int k0 = first; k0 - 2 * kTileKeys * half < k_end; k0 += 2 * HALVES * kTileKeys) {
     __syncthreads();  // the previous tiles' readers are done
-    store_tile(0, ra);
+    if (k0 < k_end) store_tile(0, ra);
     if (k0 + kTileKeys < k_end) store_tile(1, rb);
     __syncthreads();
-    load_tile(k0 + 2 * kTileKeys, ra);
-    load_tile(k0 + 3 * kTileKeys, rb);
-    step(k0, 0);
+    load_tile(k0 + 2 * HALVES * kTileKeys, ra);
+    load_tile(k0 + (2 * HALVES + 1) * kTileKeys, rb);
+    if (k0 < k_end) step(k0, 0);
     if (k0 + kTileKeys < k_end) step(k0 + kTileKeys, 1);
   }
+  constexpr int kOut = DV / 32 / HALVES;  // blocks that this wavefront ends
+  f32x16_t ended[kOut];
+  if constexpr (HALVES == 2) {
+    merge_halves<DV>(o, m_run, l_run, reinterpret_cast<float*>(ks2), reinterpret_cast<const float*>(tiles + (half ^ 1) * kTiles), ml, tid, half, ended);
+  } else {
+#pragma unroll
+    for (int d = 0; d < kOut; ++d) ended[d] = o[d];
+  }
   if (qi >= M) return;
-  // o[d][i]: column 32 d + 8 (i / 4) + 4 kh + i % 4
+  // ended[d][i]: column 32 (kOut half + d) + 8 (i / 4) + 4 kh + i % 4
   const float inv = 1.0f / l_run;
   bf16_t* out = reinterpret_cast<bf16_t*>(a.ctx) + (int64_t)qi * a.ldc + (int64_t)h * a.vdim;
 #pragma unroll
-  for (int d = 0; d < DV / 32; ++d)
+  for (int d = 0; d < kOut; ++d)
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const int c = 32 * d + 8 * u + 4 * kh;
+      const int c = 32 * (kOut * half + d) + 8 * u + 4 * kh;
       if (c < a.vdim)  // vdim is a multiple of 8
-        *reinterpret_cast<bf16x4_t*>(out + c) = bf16x4_t{(bf16_t)(o[d][4 * u] * inv), (bf16_t)(o[d][4 * u + 1] * inv),
-                                                         (bf16_t)(o[d][4 * u + 2] * inv), (bf16_t)(o[d][4 * u + 3] * inv)};
+        *reinterpret_cast<bf16x4_t*>(out + c) = bf16x4_t{(bf16_t)(ended[d][4 * u] * inv), (bf16_t)(ended[d][4 * u + 1] * inv),
+                                                         (bf16_t)(ended[d][4 * u + 2] * inv), (bf16_t)(ended[d][4 * u + 3] * inv)};
     }
+}
+
+// Halves of the keys where the longest run of keys is more than a turn of both: 32 heads of 128 + 64 and 128, 1,024 tokens 62 -> 45 us,
+// 2,048 tokens (two workgroups to a compute unit, one after the other) 125 -> 93, 10 heads, 1,800 tokens 93 -> 62.  Wider rows
+// leave no registers for two wavefronts.
+template <int DK, int DV>
+void launch_tile(const LatentAttnArgs& a, hipStream_t st) {
+  const dim3 g((unsigned)a.heads, (unsigned)((a.M + kTileQueries - 1) / kTileQueries));
+  if constexpr (DK + DV <= 320 && DV <= 128) {
+    if (a.pos.pos0 + a.M > 4 * kTileKeys) {
+      hipLaunchKernelGGL((latent_tile_kernel<DK, DV, 2>), g, dim3(512), 0, st, a);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((latent_tile_kernel<DK, DV, 1>), g, dim3(256), 0, st, a);
 }
 
 template <int DK>
 void launch_tiles(const LatentAttnArgs& a, hipStream_t st) {
-  const dim3 g((unsigned)a.heads, (unsigned)((a.M + kTileQueries - 1) / kTileQueries));
-  if (a.vdim <= 64) hipLaunchKernelGGL((latent_tile_kernel<DK, 64>), g, dim3(256), 0, st, a);
-  else if (a.vdim <= 128) hipLaunchKernelGGL((latent_tile_kernel<DK, 128>), g, dim3(256), 0, st, a);
-  else hipLaunchKernelGGL((latent_tile_kernel<DK, 256>), g, dim3(256), 0, st, a);
+  if (a.vdim <= 64) launch_tile<DK, 64>(a, st);
+  else if (a.vdim <= 128) launch_tile<DK, 128>(a, st);
+  else launch_tile<DK, 256>(a, st);
 }
 
 int64_t q_inputs(const LatentAttnArgs& a) { return round_up(a.dim, kDenseKAlign); }

@@ -1,0 +1,46 @@
+// Tiles of queries whose keys two sets of four wavefronts share: what their halves of a softmax come to (window_attention.hip,
+// latent_attention.hip).
+#pragma once
+#include "common.hpp"
+
+namespace {
+
+// the values of lane % 32 and lane % 32 + 32
+struct HalfPair {
+  float low, high;
+};
+__device__ __forceinline__ HalfPair half_pair(float x) {
+  typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
+  const u32x2_t p = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return {__uint_as_float(p[0]), __uint_as_float(p[1])};
+}
+
+// A wavefront's o[d][i] are sums of weights and values for one query a lane (two lanes share a query), m its maximum (binary logarithm), l the sum of
+// the weights.  Behind this a wavefront of half h has the sums of both halves of the blocks from h DV / 64 on, and l is the whole sum.
+// `mine` and `other`: 16 KB of the halves' tiles, ml [2][2][256].
+template <int DV, typename V>
+__device__ __forceinline__ void merge_halves(const V (&o)[DV / 32], float m, float& l, float* mine, const float* other, float* ml, int tid, int half,
+                                             V (&out)[DV / 64]) {
+  constexpr int H = DV / 64;
+  float f = 0.0f, f_other = 0.0f;
+  __syncthreads();  // the last tiles' readers are done
+  ml[half * 512 + tid] = m;
+  ml[half * 512 + 256 + tid] = l;
+#pragma unroll
+  for (int d = 0; d < H; ++d) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) mine[i * 256 + tid] = half ? o[d][i] : o[H + d][i];
+    __syncthreads();
+    if (d == 0) {
+      const float m_other = ml[(half ^ 1) * 512 + tid], l_other = ml[(half ^ 1) * 512 + 256 + tid], both = fmaxf(m, m_other);
+      f = __builtin_amdgcn_exp2f(m - both);
+      f_other = __builtin_amdgcn_exp2f(m_other - both);
+      l = l * f + l_other * f_other;
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) out[d][i] = (half ? o[H + d][i] : o[d][i]) * f + other[i * 256 + tid] * f_other;
+    if (d + 1 < H) __syncthreads();
+  }
+}
+
+}  // namespace

@@ -1,6 +1,7 @@
 // Attention over a sliding window with a distance bias (layers.hpp).
 #include "dense_one_device.hpp"
 #include "query_attention.hpp"
+#include "tile_halves.hpp"
 
 namespace {
 
@@ -432,15 +433,19 @@ int launch_decode(const WindowAttnArgs& a, hipStream_t st, const DenseArgs* besi
 // LDS read).  Scores and weights are binary32; a weight enters the product as the sum of two bfloat16 terms.
 typedef short short4_t __attribute__((ext_vector_type(4)));
 constexpr int kTileQueries = 128, kTileKeys = 32;
+constexpr float kSlack = 8.0f;
 
-template <int DK, int DV>
-__global__ __launch_bounds__(256, (DK + DV > 256) ? 1 : 2) void window_tile_kernel(WindowAttnArgs a) {
+template <int DK, int DV, int HALVES>
+__global__ __launch_bounds__(256 * HALVES, (DK + DV > 256) ? 1 : 2) void window_tile_kernel(WindowAttnArgs a) {
   constexpr int KS = DK + 8, VS = DV + 16;
   constexpr int KP = DK / 64, VP = DV / 64;  // 16-byte pieces of a tile per thread
-  __shared__ __attribute__((aligned(16))) bf16_t ks2[2 * kTileKeys * KS];
-  __shared__ __attribute__((aligned(16))) bf16_t vs2[2 * kTileKeys * VS];
+  constexpr int kTiles = 2 * kTileKeys * (KS + VS);
+  __shared__ __attribute__((aligned(16))) bf16_t tiles[HALVES * kTiles];
+  __shared__ float ml[HALVES == 2 ? 1024 : 1];
+  const int half = HALVES == 2 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) : 0;
+  bf16_t *const ks2 = tiles + half * kTiles, *const vs2 = ks2 + 2 * kTileKeys * KS;
   const int h = blockIdx.x, g = h / (a.heads / a.kv_heads);
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = threadIdx.x & 255, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, kh = lane >> 5;
   const int M = (int)a.M, pos0 = a.pos.pos0;
   const int q_first = blockIdx.y * kTileQueries;
@@ -505,21 +510,41 @@ __global__ __launch_bounds__(256, (DK + DV > 256) ? 1 : 2) void window_tile_kern
       *reinterpret_cast<bf16x8_t*>(vs2 + (half * kTileKeys + key) * VS + at) = r.v[i];
     }
   };
-  auto step = [&](int k0, int half) __attribute__((always_inline)) {
+  // Bound by the chain of a wavefront that has a SIMD nearly to itself, so operands are read four products ahead and the first values
+  // ahead of the softmax.  (Two tiles to a softmax: no registers for it with halves, without them no faster.)
+  auto step = [&](int k0, int at) __attribute__((always_inline)) {
     if (k0 > w_last || k0 + kTileKeys <= lo_wave) return;  // no query of this wavefront sees a key of the tile
-    const bf16_t* ks = ks2 + half * kTileKeys * KS;
-    const bf16_t* vs = vs2 + half * kTileKeys * VS;
+    const bf16_t* const klane = ks2 + (at * kTileKeys + n) * KS + 8 * kh;
+    const int L16 = lane & 15;
+    const bf16_t* const vlane = vs2 + (at * kTileKeys + 4 * kh + (L16 >> 2)) * VS + 16 * ((lane >> 4) & 1) + 4 * (L16 & 3);
+    auto values = [&](int j, int d) __attribute__((always_inline)) {
+      const bf16_t* vp = vlane + 16 * j * VS + d * 32;
+      const short4_t l = __builtin_amdgcn_ds_read_tr16_b64_v4i16((short4_t __attribute__((address_space(3)))*)vp);
+      const short4_t u = __builtin_amdgcn_ds_read_tr16_b64_v4i16((short4_t __attribute__((address_space(3)))*)(vp + 8 * VS));
+      const bf16x4_t l4 = __builtin_bit_cast(bf16x4_t, l), u4 = __builtin_bit_cast(bf16x4_t, u);
+      return bf16x8_t{l4[0], l4[1], l4[2], l4[3], u4[0], u4[1], u4[2], u4[3]};
+    };
     f32x16_t s;
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = 0.0f;
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int d = 0; d < DK / 16; ++d)
-      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8_t*>(ks + n * KS + 16 * d + 8 * kh), qop[d], s,
-                                                  0, 0, 0);
-    // s[i]: key k0 + 8 (i / 4) + 4 kh + i % 4 for this lane's query
-    const int base = k0 + 4 * kh - pq;
+      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8_t*>(klane + 16 * d), qop[d], s, 0, 0, 0);
+    bf16x8_t vv[DV / 32];  // (of the first slice)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) s[i] = __builtin_fmaf(s[i], mul, slope * (float)(base + 8 * (i >> 2) + (i & 3)));
+    for (int d = 0; d < DV / 32; ++d) vv[d] = values(0, d);
+    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+    for (int d = 0; d < DK / 16; ++d) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    // s[i]: key k0 + 8 (i / 4) + 4 kh + i % 4 for this lane's query
+    const float base = (float)(k0 + 4 * kh - pq);  // (sums of whole numbers below 2^24)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] = __builtin_fmaf(s[i], mul, slope * (base + (float)(8 * (i >> 2) + (i & 3))));
     if (k0 + kTileKeys - 1 > w_first || k0 < lo_full) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
@@ -530,82 +555,107 @@ __global__ __launch_bounds__(256, (DK + DV > 256) ? 1 : 2) void window_tile_kern
     float mx = s[0];
 #pragma unroll
     for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float m_new = fmaxf(m_run, mx);
-    const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-    float rs = 0.0f;
-    bf16x8_t hi[2], lo[2];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const float p = __builtin_amdgcn_exp2f(s[i] - m_new);
-      rs += p;
-      hi[i >> 3][i & 7] = (bf16_t)p;
-      lo[i >> 3][i & 7] = (bf16_t)(p - (float)hi[i >> 3][i & 7]);
-    }
-    rs += __shfl_xor(rs, 32, 64);
-    l_run = l_run * alpha + rs;
-    m_run = m_new;
-    if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
+    const HalfPair best = half_pair(mx);
+    mx = fmaxf(best.low, best.high);
+    // the maximum that weights are relative to moves only once it is 2^kSlack behind: sums grow by as much and no more
+    if (__builtin_amdgcn_ballot_w64(!(mx <= m_run + kSlack)) != 0) {
+      const float m_new = fmaxf(m_run, mx), alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+      l_run *= alpha;
+      m_run = m_new;
 #pragma unroll
       for (int d = 0; d < DV / 32; ++d)
 #pragma unroll
         for (int i = 0; i < 16; ++i) o[d][i] *= alpha;
     }
-    const int L16 = lane & 15;
-    const bf16_t* vlane = vs + (4 * kh + (L16 >> 2)) * VS + 16 * ((lane >> 4) & 1) + 4 * (L16 & 3);
+    float rs = 0.0f;
+    bf16x8_t hi[2], lo[2];
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int i = 0; i < 16; ++i) {
+      const float p = __builtin_amdgcn_exp2f(s[i] - m_run);
+      rs += p;
+      hi[i >> 3][i & 7] = (bf16_t)p;
+      lo[i >> 3][i & 7] = (bf16_t)(p - (float)hi[i >> 3][i & 7]);
+    }
+    const HalfPair sums = half_pair(rs);
+    l_run += sums.low + sums.high;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+#pragma unroll
+      for (int d = 0; d < DV / 32; ++d) o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vv[d], hi[j], o[d], 0, 0, 0);
 #pragma unroll
       for (int d = 0; d < DV / 32; ++d) {
-        const bf16_t* vp = vlane + 16 * j * VS + d * 32;
-        const short4_t l = __builtin_amdgcn_ds_read_tr16_b64_v4i16((short4_t __attribute__((address_space(3)))*)vp);
-        const short4_t u = __builtin_amdgcn_ds_read_tr16_b64_v4i16((short4_t __attribute__((address_space(3)))*)(vp + 8 * VS));
-        const bf16x4_t l4 = __builtin_bit_cast(bf16x4_t, l), u4 = __builtin_bit_cast(bf16x4_t, u);
-        const bf16x8_t vv = {l4[0], l4[1], l4[2], l4[3], u4[0], u4[1], u4[2], u4[3]};
-        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vv, hi[j], o[d], 0, 0, 0);
-        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vv, lo[j], o[d], 0, 0, 0);
+        o[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vv[d], lo[j], o[d], 0, 0, 0);
+        if (j + 1 < 2) vv[d] = values(j + 1, d);
       }
+    }
   };
-  load_tile(k_begin, ra);
-  load_tile(k_begin + kTileKeys, rb);
-  for (int k0 = k_begin; k0 < k_end; k0 += 2 * kTileKeys) {
+  const int first = k_begin + 2 * kTileKeys * half;
+  load_tile(first, ra);
+  load_tile(first + kTileKeys, rb);
+  // The first products wait for the queries here: inside the loop, where the number of requests on their way is not known, that wait would be one for
+  // everything, the next tiles with it.
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+  for (int k0 = first; k0 - 2 * kTileKeys * half < k_end; k0 += 2 * HALVES * kTileKeys) {
     __syncthreads();  // the previous tiles' readers are done
-    store_tile(0, ra);
+    if (k0 < k_end) store_tile(0, ra);
     if (k0 + kTileKeys < k_end) store_tile(1, rb);
     __syncthreads();
-    load_tile(k0 + 2 * kTileKeys, ra);
-    load_tile(k0 + 3 * kTileKeys, rb);
-    step(k0, 0);
+    load_tile(k0 + 2 * HALVES * kTileKeys, ra);
+    load_tile(k0 + (2 * HALVES + 1) * kTileKeys, rb);
+    if (k0 < k_end) step(k0, 0);
     if (k0 + kTileKeys < k_end) step(k0 + kTileKeys, 1);
   }
+  constexpr int kOut = DV / 32 / HALVES;  // blocks that this wavefront ends
+  f32x16_t ended[kOut];
+  if constexpr (HALVES == 2) {
+    merge_halves<DV>(o, m_run, l_run, reinterpret_cast<float*>(ks2), reinterpret_cast<const float*>(tiles + (half ^ 1) * kTiles), ml, tid, half, ended);
+  } else {
+#pragma unroll
+    for (int d = 0; d < kOut; ++d) ended[d] = o[d];
+  }
   if (qi >= M) return;
-  // o[d][i]: column 32 d + 8 (i / 4) + 4 kh + i % 4
+  // ended[d][i]: column 32 (kOut half + d) + 8 (i / 4) + 4 kh + i % 4
   const float inv = 1.0f / l_run;
   bf16_t* out = reinterpret_cast<bf16_t*>(a.ctx) + (int64_t)qi * a.ldc + (int64_t)h * a.vdim;
 #pragma unroll
-  for (int d = 0; d < DV / 32; ++d)
+  for (int d = 0; d < kOut; ++d)
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const int c = 32 * d + 8 * u + 4 * kh;
+      const int c = 32 * (kOut * half + d) + 8 * u + 4 * kh;
       if (c + 3 < a.vdim && (a.vdim & 3) == 0) {
         bf16x4_t v;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = (bf16_t)(o[d][4 * u + j] * inv);
+        for (int j = 0; j < 4; ++j) v[j] = (bf16_t)(ended[d][4 * u + j] * inv);
         *reinterpret_cast<bf16x4_t*>(out + c) = v;
       } else {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-          if (c + j < a.vdim) out[c + j] = (bf16_t)(o[d][4 * u + j] * inv);
+          if (c + j < a.vdim) out[c + j] = (bf16_t)(ended[d][4 * u + j] * inv);
       }
     }
 }
 
+// Halves of the keys where a compute unit has a workgroup at most and the longest run of keys is more than a turn of both: 8 heads of
+// 128 in a window of 1,024, 2,000 tokens 50 -> 42 us, 16 heads 58 -> 49, 400 tokens of 8 heads 21 -> 18; 90 tokens of 16 heads 8.5 -> 9.7, 32 heads
+// and 2,000 tokens (two workgroups a unit) 90 -> 93.  Wider rows leave no registers for two wavefronts.
+template <int DK, int DV>
+void launch_tile(const WindowAttnArgs& a, hipStream_t st) {
+  const dim3 g((unsigned)a.heads, (unsigned)((a.M + kTileQueries - 1) / kTileQueries));
+  const int64_t keys = a.window > 0 ? std::min<int64_t>(a.pos.pos0 + a.M, (int64_t)a.window + kTileQueries - 1) : a.pos.pos0 + a.M;
+  if constexpr (DK + DV <= 256) {
+    if ((int64_t)g.x * g.y <= 256 && keys > 4 * kTileKeys) {
+      hipLaunchKernelGGL((window_tile_kernel<DK, DV, 2>), g, dim3(512), 0, st, a);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((window_tile_kernel<DK, DV, 1>), g, dim3(256), 0, st, a);
+}
+
 template <int DK>
 void launch_tiles(const WindowAttnArgs& a, hipStream_t st) {
-  const dim3 g((unsigned)a.heads, (unsigned)((a.M + kTileQueries - 1) / kTileQueries));
-  if (a.vl.row == 64) hipLaunchKernelGGL((window_tile_kernel<DK, 64>), g, dim3(256), 0, st, a);
-  else if (a.vl.row == 128) hipLaunchKernelGGL((window_tile_kernel<DK, 128>), g, dim3(256), 0, st, a);
-  else hipLaunchKernelGGL((window_tile_kernel<DK, 256>), g, dim3(256), 0, st, a);
+  if (a.vl.row == 64) launch_tile<DK, 64>(a, st);
+  else if (a.vl.row == 128) launch_tile<DK, 128>(a, st);
+  else launch_tile<DK, 256>(a, st);
 }
 
 // Many tokens, binary32, on v_mfma_f32_16x16x4_f32: sixteen queries of one head per workgroup, whose wavefronts take every eighth tile of
