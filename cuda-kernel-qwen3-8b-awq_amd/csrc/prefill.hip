@@ -8,6 +8,7 @@
 // what the reference's column-per-token cublasGemmEx operands (ldb = k,
 // ldc = m) look like in memory.
 #include "common.hpp"
+#include "tile_halves.hpp"
 
 namespace {
 
@@ -144,16 +145,22 @@ constexpr int kFaKStride = 136;   // halves per key row of the K tile (128 + 8 o
 constexpr int kFaVStride = 144;   // halves per key row of the V tile (128 + 16: four consecutive rows start 8 banks apart)
 typedef short short4_t __attribute__((ext_vector_type(4)));
 
-__global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const half_t* __restrict__ q,
+// HALVES 2: two sets of four wavefronts take turns of 64 keys each and meet in LDS, where a wavefront would have a SIMD to itself and wait for
+// its own chain; for the same reason operands are read four products ahead and the first values ahead of the softmax.
+template <int HALVES>
+__global__ __launch_bounds__(256 * HALVES, HALVES == 2 ? 1 : 2) void prefill_attention_kernel(const half_t* __restrict__ q,
                                                                 const half_t* __restrict__ kc,
                                                                 const half_t* __restrict__ vc,
                                                                 half_t* __restrict__ ctx, KvLayout kv, int pos0,
                                                                 int M, int use_len_hi) {
-  __shared__ __attribute__((aligned(16))) half_t ks2[2 * kFaKeys * kFaKStride];
-  __shared__ __attribute__((aligned(16))) half_t vs2[2 * kFaKeys * kFaVStride];
+  constexpr int kTiles = 2 * kFaKeys * (kFaKStride + kFaVStride);
+  __shared__ __attribute__((aligned(16))) half_t tiles[HALVES * kTiles];
+  __shared__ float ml[HALVES == 2 ? 1024 : 1];
+  const int share = HALVES == 2 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) : 0;
+  half_t *const ks2 = tiles + share * kTiles, *const vs2 = ks2 + 2 * kFaKeys * kFaKStride;
   const int head = blockIdx.x, n_heads = gridDim.x;
   const int H = n_heads * AWQ_HEAD_DIM;
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = threadIdx.x & 255, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = lane & 31, kh = lane >> 5;
   const half_t* kh_ptr = kc;
@@ -218,22 +225,46 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const half_t*
     }
     __syncthreads();
     // the next two tiles travel while these are multiplied
-    load_tile(k0 + 2 * kFaKeys, ra);
-    load_tile(k0 + 3 * kFaKeys, rb);
+    load_tile(k0 + 2 * HALVES * kFaKeys, ra);
+    load_tile(k0 + (2 * HALVES + 1) * kFaKeys, rb);
   };
   auto step = [&](int k0, int half) __attribute__((always_inline)) {
     if (k0 >= L_wave) return;  // nothing of this tile is attended by this wavefront's queries
     const half_t* ks = ks2 + half * kFaKeys * kFaKStride;
     const half_t* vs = vs2 + half * kFaKeys * kFaVStride;
 
+    // V transposed, the first operand of the second product: component 32 dt + n of four consecutive keys per 8-byte half.  The
+    // transposing LDS read delivers exactly that from the tile as it came from memory: within 16 lanes, lane i receives
+    // element i % 4 of the 8-byte pieces that lanes i / 4, i / 4 + 4, i / 4 + 8, i / 4 + 12 point at -- so lane L points at the row
+    // of key L / 4 of the four, components 4 (L % 4) .. + 3 of the group's sixteen.
+    const int L16 = lane & 15;
+    const half_t* vlane = vs + (4 * kh + (L16 >> 2)) * kFaVStride + 16 * ((lane >> 4) & 1) + 4 * (L16 & 3);
+    auto values = [&](int j, int dt) __attribute__((always_inline)) {
+      const half_t* vp = vlane + 16 * j * kFaVStride + dt * 32;
+      const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((short4_t __attribute__((address_space(3)))*)vp);
+      const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((short4_t __attribute__((address_space(3)))*)(vp + 8 * kFaVStride));
+      const half4_t lh = __builtin_bit_cast(half4_t, lo), hh = __builtin_bit_cast(half4_t, hi);
+      return half8_t{lh[0], lh[1], lh[2], lh[3], hh[0], hh[1], hh[2], hh[3]};
+    };
     f32x16_t sacc;
 #pragma unroll
     for (int i = 0; i < 16; ++i) sacc[i] = 0.0f;
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int s = 0; s < 8; ++s) {
       const half8_t kop = *reinterpret_cast<const half8_t*>(ks + n * kFaKStride + 16 * s + 8 * kh);
       sacc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kop, qop[s], sacc, 0, 0, 0);
     }
+    half8_t vop[4];
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt) vop[dt] = values(0, dt);
+    __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
     // sacc[i] is the score of key k0 + 8 (i / 4) + 4 kh + i % 4 for this lane's query.  A tile that
     // lies wholly inside the attended range of every query of the wavefront (nearly all tiles of a
     // long prompt) needs no masks; the scale goes into the exponent's multiply-add.
@@ -243,72 +274,71 @@ __global__ __launch_bounds__(256, 2) void prefill_attention_kernel(const half_t*
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const int key = k0 + 8 * (i >> 2) + 4 * kh + (i & 3);
-        sacc[i] = key < Lq ? sacc[i] : -1e30f;  // 2^(scale * -1e30 - m) is 0
+        sacc[i] = key < Lq ? sacc[i] : -INFINITY;  // (also where none of a half's keys has been seen, and the maximum is -1e30)
       }
     }
 #pragma unroll
     for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sacc[i]);
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    // (a tile in which none of this query's keys is attended leaves the maximum where it was)
-    const float m_new = fmaxf(m_run, mx > -1e29f ? mx * scale2 : -1e30f);
-    const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-    float rs = 0.0f;
-    half8_t pop[2];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const float pe = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[i], scale2, -m_new));
-      rs += pe;
-      pop[i >> 3][i & 7] = (half_t)pe;
-    }
-    rs += __shfl_xor(rs, 32, 64);
-    l_run = l_run * alpha + rs;
-    m_run = m_new;
-    // once the running maxima have settled (most tiles), alpha is 1 in every lane
-    if (__builtin_amdgcn_ballot_w64(alpha != 1.0f) != 0) {
+    const HalfPair best = half_pair(mx);
+    mx = fmaxf(best.low, best.high);
+    // (a tile in which none of this query's keys is attended leaves the maximum where it was; so does one that is less than 2^8 ahead
+    // of it: sums grow by as much and no more)
+    const float m_tile = mx > -1e29f ? mx * scale2 : -1e30f;
+    if (__builtin_amdgcn_ballot_w64(!(m_tile <= m_run + 8.0f)) != 0) {
+      const float m_new = fmaxf(m_run, m_tile), alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+      l_run *= alpha;
+      m_run = m_new;
 #pragma unroll
       for (int dt = 0; dt < 4; ++dt)
 #pragma unroll
         for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
     }
-    // second product: slice j takes keys 16 j + 8 (e / 4) + 4 kh + e % 4, e = 0..7, which are this
-    // lane's probabilities 8 j .. 8 j + 7.  Its first operand is V transposed: component 32 dt + n of
-    // four consecutive keys per 8-byte half.  The transposing LDS read delivers exactly that from the
-    // tile as it came from memory: within 16 lanes, lane i receives element i % 4 of the 8-byte pieces
-    // that lanes i / 4, i / 4 + 4, i / 4 + 8, i / 4 + 12 point at -- so lane L points at the row of key
-    // L / 4 of the four, components 4 (L % 4) .. + 3 of the group's sixteen.
-    const int L16 = lane & 15;
-    const half_t* vlane = vs + (4 * kh + (L16 >> 2)) * kFaVStride + 16 * ((lane >> 4) & 1) + 4 * (L16 & 3);
+    float rs = 0.0f;
+    half8_t pop[2];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
+    for (int i = 0; i < 16; ++i) {
+      const float pe = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[i], scale2, -m_run));
+      rs += pe;
+      pop[i >> 3][i & 7] = (half_t)pe;
+    }
+    const HalfPair sums = half_pair(rs);
+    l_run += sums.low + sums.high;
+    // second product: slice j takes keys 16 j + 8 (e / 4) + 4 kh + e % 4, e = 0..7, which are this lane's probabilities 8 j .. 8 j + 7
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
 #pragma unroll
       for (int dt = 0; dt < 4; ++dt) {
-        const half_t* vp = vlane + 16 * j * kFaVStride + dt * 32;
-        const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((short4_t __attribute__((address_space(3)))*)vp);
-        const short4_t hi =
-            __builtin_amdgcn_ds_read_tr16_b64_v4i16((short4_t __attribute__((address_space(3)))*)(vp + 8 * kFaVStride));
-        const half4_t lh = __builtin_bit_cast(half4_t, lo), hh = __builtin_bit_cast(half4_t, hi);
-        const half8_t vop = half8_t{lh[0], lh[1], lh[2], lh[3], hh[0], hh[1], hh[2], hh[3]};
-        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vop, pop[j], o[dt], 0, 0, 0);
+        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vop[dt], pop[j], o[dt], 0, 0, 0);
+        if (j == 0) vop[dt] = values(1, dt);
       }
-    }
   };
-  load_tile(0, ra);
-  load_tile(kFaKeys, rb);
-  for (int k0 = 0; k0 < L_wg; k0 += 2 * kFaKeys) {
+  const int first = 2 * kFaKeys * share;
+  load_tile(first, ra);
+  load_tile(first + kFaKeys, rb);
+  for (int k0 = first; k0 - first < L_wg; k0 += 2 * HALVES * kFaKeys) {
     stage(k0);
     step(k0, 0);
     if (k0 + kFaKeys < L_wg) step(k0 + kFaKeys, 1);
   }
-  // o[dt][i] is component 32 dt + 8 (i / 4) + 4 kh + i % 4 of this lane's query
+  constexpr int kOut = 4 / HALVES;  // blocks of 32 components that this wavefront ends
+  f32x16_t ended[kOut];
+  if constexpr (HALVES == 2) {
+    merge_halves<AWQ_HEAD_DIM>(o, m_run, l_run, reinterpret_cast<float*>(ks2), reinterpret_cast<const float*>(tiles + (share ^ 1) * kTiles), ml, tid,
+                               share, ended);
+  } else {
+#pragma unroll
+    for (int dt = 0; dt < kOut; ++dt) ended[dt] = o[dt];
+  }
+  // ended[dt][i] is component 32 (kOut share + dt) + 8 (i / 4) + 4 kh + i % 4 of this lane's query
   if (qi < M) {
     const float inv = 1.0f / l_run;
-    half_t* out = ctx + (int64_t)qi * H + head * AWQ_HEAD_DIM;
+    half_t* out = ctx + (int64_t)qi * H + head * AWQ_HEAD_DIM + 32 * kOut * share;
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
+    for (int dt = 0; dt < kOut; ++dt)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const half4_t v = half4_t{(half_t)(o[dt][4 * g] * inv), (half_t)(o[dt][4 * g + 1] * inv),
-                                  (half_t)(o[dt][4 * g + 2] * inv), (half_t)(o[dt][4 * g + 3] * inv)};
+        const half4_t v = half4_t{(half_t)(ended[dt][4 * g] * inv), (half_t)(ended[dt][4 * g + 1] * inv),
+                                  (half_t)(ended[dt][4 * g + 2] * inv), (half_t)(ended[dt][4 * g + 3] * inv)};
         *reinterpret_cast<half4_t*>(out + dt * 32 + 8 * g + 4 * kh) = v;
       }
   }
@@ -351,8 +381,13 @@ int launch_prefill_attention(const half_t* q, const half_t* kc, const half_t* vc
                              int64_t max_pos, KvLayout kv, int64_t pos0, int64_t M, int use_len_hi, hipStream_t st) {
   AWQ_REQUIRE(n_heads > 0 && max_pos > 0, "n_heads and max_pos must be positive");
   AWQ_REQUIRE(M >= 1 && M <= 65535 * kFaQueries && pos0 >= 0 && pos0 + M <= max_pos, "positions out of range");
-  hipLaunchKernelGGL(prefill_attention_kernel, dim3((unsigned)n_heads, (unsigned)((M + kFaQueries - 1) / kFaQueries)),
-                     dim3(256), 0, st, q, kc, vc, ctx, kv, (int)pos0, (int)M, use_len_hi);
+  const dim3 g((unsigned)n_heads, (unsigned)((M + kFaQueries - 1) / kFaQueries));
+  // Halves of the keys from two turns of each on: 32 heads at 1,000 tokens 38 -> 25 us (prompt of 36 layers 13.03 -> 12.75 ms), 2,048
+  // tokens 27.0 -> 26.1 ms, 300 as before; 140 tokens 4.77 ms without and 4.82 with.
+  if (pos0 + M > 8 * kFaKeys)
+    hipLaunchKernelGGL(prefill_attention_kernel<2>, g, dim3(512), 0, st, q, kc, vc, ctx, kv, (int)pos0, (int)M, use_len_hi);
+  else
+    hipLaunchKernelGGL(prefill_attention_kernel<1>, g, dim3(256), 0, st, q, kc, vc, ctx, kv, (int)pos0, (int)M, use_len_hi);
   AWQ_HIP_TRY(hipGetLastError());
   return AWQ_OK;
 }
