@@ -940,8 +940,8 @@ __global__ __launch_bounds__(256 * HALVES, (DK + DV > 256) ? 1 : 2) void latent_
     }
 }
 
-// Halves of the keys where the longest run of keys is more than a turn of both: 32 heads of 128 + 64 and 128, 1,024 tokens 62 -> 45 us,
-// 2,048 tokens (two workgroups to a compute unit, one after the other) 125 -> 93, 10 heads, 1,800 tokens 93 -> 62.  Wider rows
+// Halves of the keys where the longest run of keys is more than a turn of both: 32 heads of 128 + 64 and 128, 1,024 tokens 62 -> 42 us,
+// 2,048 tokens (two workgroups to a compute unit, one after the other) 125 -> 87, 10 heads, 1,800 tokens 93 -> 57.  Wider rows
 // leave no registers for two wavefronts.
 template <int DK, int DV>
 void launch_tile(const LatentAttnArgs& a, hipStream_t st) {

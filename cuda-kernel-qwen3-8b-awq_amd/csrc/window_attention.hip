@@ -635,15 +635,16 @@ __global__ __launch_bounds__(256 * HALVES, (DK + DV > 256) ? 1 : 2) void window_
     }
 }
 
-// Halves of the keys where a compute unit has a workgroup at most and the longest run of keys is more than a turn of both: 8 heads of
-// 128 in a window of 1,024, 2,000 tokens 50 -> 42 us, 16 heads 58 -> 49, 400 tokens of 8 heads 21 -> 18; 90 tokens of 16 heads 8.5 -> 9.7, 32 heads
-// and 2,000 tokens (two workgroups a unit) 90 -> 93.  Wider rows leave no registers for two wavefronts.
+// Halves of the keys where a compute unit has a workgroup at most and the longest run of keys is more than two turns of both: 8 heads of
+// 128 in a window of 1,024, 2,000 tokens 52 -> 39 us, 16 heads 58 -> 47, 400 tokens of 8 heads 21 -> 17; 90 tokens of 16 heads 7.9 -> 9.7, a
+// prompt of 150 tokens of 8 heads 445 -> 460, 32 heads and 2,000 tokens (two workgroups a unit) 84 -> 93.  Wider rows leave no registers
+// for two wavefronts.
 template <int DK, int DV>
 void launch_tile(const WindowAttnArgs& a, hipStream_t st) {
   const dim3 g((unsigned)a.heads, (unsigned)((a.M + kTileQueries - 1) / kTileQueries));
   const int64_t keys = a.window > 0 ? std::min<int64_t>(a.pos.pos0 + a.M, (int64_t)a.window + kTileQueries - 1) : a.pos.pos0 + a.M;
   if constexpr (DK + DV <= 256) {
-    if ((int64_t)g.x * g.y <= 256 && keys > 4 * kTileKeys) {
+    if ((int64_t)g.x * g.y <= 256 && keys > 8 * kTileKeys) {
       hipLaunchKernelGGL((window_tile_kernel<DK, DV, 2>), g, dim3(512), 0, st, a);
       return;
     }
