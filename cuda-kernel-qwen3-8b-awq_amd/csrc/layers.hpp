@@ -237,6 +237,7 @@ struct LinearAttnArgs {
   const void* proj = nullptr;  // [M][ldp]: heads * dim of q, heads * dim of k, heads * vdim of v
   int64_t ldp = 0;
   int32_t heads = 0, dim = 0, vdim = 0;
+  int32_t seg_tokens = 0;      // of a segment (the launch sets it), 0: one after the other; here among the preloaded arguments
   const float* decay = nullptr;       // [heads]
   const float* log2_decay = nullptr;  // [heads], null unless every decay is positive: many tokens then go in chunks
   float* state = nullptr;
@@ -245,7 +246,6 @@ struct LinearAttnArgs {
   PassPos pos;
   float* workspace = nullptr;  // states between segments of a pass that go side by side; may be null
   int64_t workspace_floats = 0;
-  int32_t seg_tokens = 0;      // of a segment (the launch sets it), 0: one after the other
 };
 int64_t linear_state_floats(int32_t heads, int32_t dim, int32_t vdim);
 // beside (where linear_takes_product): a product in the same launch
