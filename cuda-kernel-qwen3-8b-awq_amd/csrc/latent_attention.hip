@@ -754,7 +754,6 @@ __global__ __launch_bounds__(256) void latent_value_one_kernel(LatentAttnArgs a,
 // 128 queries of one head per workgroup, 32 per wavefront, keys and values of 32 positions at a time through LDS; the
 // operands as in window_attention.hip.  The sink is the state that a query's running maximum and sum start from.
 constexpr int kTileQueries = 128, kTileKeys = 32;
-constexpr float kSlack = 8.0f;
 
 template <int DK, int DV, int HALVES>
 __global__ __launch_bounds__(256 * HALVES, (DK + DV > 256) ? 1 : 2) void latent_tile_kernel(LatentAttnArgs a) {
@@ -869,16 +868,7 @@ __global__ __launch_bounds__(256 * HALVES, (DK + DV > 256) ? 1 : 2) void latent_
     for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
     const HalfPair best = half_pair(mx);
     mx = fmaxf(best.low, best.high);
-    // the maximum that weights are relative to moves only once it is 2^kSlack behind: sums grow by as much and no more
-    if (__builtin_amdgcn_ballot_w64(!(mx <= m_run + kSlack)) != 0) {
-      const float m_new = fmaxf(m_run, mx), alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-      l_run *= alpha;
-      m_run = m_new;
-#pragma unroll
-      for (int d = 0; d < DV / 32; ++d)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) o[d][i] *= alpha;
-    }
+    move_maximum(mx, m_run, l_run, o);
     float rs = 0.0f;
     bf16x8_t hi[2], lo[2];
 #pragma unroll

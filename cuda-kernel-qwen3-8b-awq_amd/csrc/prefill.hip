@@ -281,18 +281,8 @@ __global__ __launch_bounds__(256 * HALVES, HALVES == 2 ? 1 : 2) void prefill_att
     for (int i = 0; i < 16; ++i) mx = fmaxf(mx, sacc[i]);
     const HalfPair best = half_pair(mx);
     mx = fmaxf(best.low, best.high);
-    // (a tile in which none of this query's keys is attended leaves the maximum where it was; so does one that is less than 2^8 ahead
-    // of it: sums grow by as much and no more)
-    const float m_tile = mx > -1e29f ? mx * scale2 : -1e30f;
-    if (__builtin_amdgcn_ballot_w64(!(m_tile <= m_run + 8.0f)) != 0) {
-      const float m_new = fmaxf(m_run, m_tile), alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-      l_run *= alpha;
-      m_run = m_new;
-#pragma unroll
-      for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) o[dt][i] *= alpha;
-    }
+    // (a tile in which none of this query's keys is attended leaves the maximum where it was)
+    move_maximum(mx > -1e29f ? mx * scale2 : -1e30f, m_run, l_run, o);
     float rs = 0.0f;
     half8_t pop[2];
 #pragma unroll

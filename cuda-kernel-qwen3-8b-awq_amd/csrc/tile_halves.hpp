@@ -1,5 +1,5 @@
-// Tiles of queries whose keys two sets of four wavefronts share: what their halves of a softmax come to (window_attention.hip,
-// latent_attention.hip).
+// Tiles of queries whose keys two sets of four wavefronts share: a maximum that moves when it must, and what their halves of a softmax come to
+// (window_attention.hip, latent_attention.hip, prefill.hip).
 #pragma once
 #include "common.hpp"
 
@@ -13,6 +13,23 @@ __device__ __forceinline__ HalfPair half_pair(float x) {
   typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
   const u32x2_t p = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   return {__uint_as_float(p[0]), __uint_as_float(p[1])};
+}
+
+// The maximum m that a query's weights are relative to moves to mx, the largest score of a tile, only once it is 2^kSlack behind it: sums grow by
+// as much and no more (the conditional rescaling of FlashAttention-4).  Every query decides for itself, so that its bits do not
+// depend on those that share its wavefront; what the wavefront decides is whether any has to.
+constexpr float kSlack = 8.0f;
+template <int BLOCKS, typename V>
+__device__ __forceinline__ void move_maximum(float mx, float& m, float& l, V (&o)[BLOCKS]) {
+  const bool moves = mx > m + kSlack;
+  if (__builtin_amdgcn_ballot_w64(moves) == 0) return;
+  const float to = moves ? mx : m, alpha = moves ? __builtin_amdgcn_exp2f(m - to) : 1.0f;
+  l *= alpha;
+  m = to;
+#pragma unroll
+  for (int d = 0; d < BLOCKS; ++d)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[d][i] *= alpha;
 }
 
 // A wavefront's o[d][i] are sums of weights and values for one query a lane (two lanes share a query), m its maximum (binary logarithm), l the sum of

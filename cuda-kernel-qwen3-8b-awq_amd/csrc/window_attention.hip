@@ -433,7 +433,6 @@ int launch_decode(const WindowAttnArgs& a, hipStream_t st, const DenseArgs* besi
 // LDS read).  Scores and weights are binary32; a weight enters the product as the sum of two bfloat16 terms.
 typedef short short4_t __attribute__((ext_vector_type(4)));
 constexpr int kTileQueries = 128, kTileKeys = 32;
-constexpr float kSlack = 8.0f;
 
 template <int DK, int DV, int HALVES>
 __global__ __launch_bounds__(256 * HALVES, (DK + DV > 256) ? 1 : 2) void window_tile_kernel(WindowAttnArgs a) {
@@ -557,16 +556,7 @@ __global__ __launch_bounds__(256 * HALVES, (DK + DV > 256) ? 1 : 2) void window_
     for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
     const HalfPair best = half_pair(mx);
     mx = fmaxf(best.low, best.high);
-    // the maximum that weights are relative to moves only once it is 2^kSlack behind: sums grow by as much and no more
-    if (__builtin_amdgcn_ballot_w64(!(mx <= m_run + kSlack)) != 0) {
-      const float m_new = fmaxf(m_run, mx), alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-      l_run *= alpha;
-      m_run = m_new;
-#pragma unroll
-      for (int d = 0; d < DV / 32; ++d)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) o[d][i] *= alpha;
-    }
+    move_maximum(mx, m_run, l_run, o);
     float rs = 0.0f;
     bf16x8_t hi[2], lo[2];
 #pragma unroll

@@ -407,6 +407,27 @@ def test_prefill_attention_matches_the_one_query_path(awq, lib, oracle, torch_gp
                                      0, stream(torch)) != 0     # runs past max_pos
 
 
+@pytest.mark.parametrize("pos0,M", [(0, 64), (70, 130), (300, 64), (0, 300)])
+def test_prefill_attention_of_a_query_is_its_own(awq, lib, torch_gpu, pos0, M):
+    """32 queries share a wavefront; those behind the twentieth of each 32 get scores that jump from tile to tile, which the bits of the others do
+    not notice"""
+    torch = torch_gpu
+    nh, mp = 2, 512
+    rng = np.random.default_rng(M + pos0)
+    kv = [dev(torch, rng.standard_normal((nh, mp, 128)).astype(np.float16)) for _ in range(2)]
+    q = rng.standard_normal((M, nh * 128)).astype(np.float16)
+    own = np.arange(M) % 32 < 20
+    print("prefill attention, queries of their own", pos0, M, flush=True)
+    out = []
+    for factor in (1, 24):
+        d_q = dev(torch, np.where(own[:, None], q, factor * q).astype(np.float16))
+        d_o = torch.zeros((M, nh * 128), dtype=torch.float16, device="cuda")
+        awq.check(lib.awq_prefill_attention(d_q.data_ptr(), kv[0].data_ptr(), kv[1].data_ptr(), d_o.data_ptr(), nh, mp, pos0, M, 1, stream(torch)))
+        torch.cuda.synchronize()
+        out.append(d_o.cpu().numpy().view(np.uint16))
+    assert np.array_equal(out[0][own], out[1][own]) and not np.array_equal(out[0][~own], out[1][~own])
+
+
 def test_gelu_all_fp16_values_and_residual(awq, lib, oracle, torch_gpu):
     torch = torch_gpu
     allh = np.arange(65536, dtype=np.uint16).view(np.float16)

@@ -717,6 +717,28 @@ def test_window_attention(awq, lib, dev, f32, shape, window):
         assert km.rms_error(got, want) < (3e-5 if f32 else 0.01), sizes
 
 
+@pytest.mark.parametrize("T", [96, 400])
+@pytest.mark.parametrize("window", [0, 90])
+def test_a_query_among_others(awq, lib, dev, window, T):
+    """bfloat16, 32 queries to a wavefront: those behind the twentieth of each 32 meet one key in every tile that they nearly equal, at scores that
+    grow, and the bits of the others do not notice"""
+    heads, dim = 3, 128
+    print("a query among others", window, T, flush=True)
+    rng = np.random.default_rng(T + window)
+    q, k, v = (rng.standard_normal((T, heads, dim)) for _ in range(3))
+    own = np.arange(T) % 32 < 20
+    to = rng.standard_normal((heads, dim))
+    others = np.where(own[:, None, None], q, to)
+    for t in range(7, T, 32):
+        k[t] = to + (T - t) / 100 * k[t]
+    out = []
+    for x in (q, others):
+        proj, _ = dev.act(np.concatenate([y.reshape(T, -1) for y in (x, k, v)], axis=1), False)
+        out.append(attend(awq, lib, dev, 0, proj, heads, heads, dim, dim, window, 2.0 * dim ** -0.5, 1e-6, (0.0, 1.0), [T], T,
+                          ((window or T) + T + 63) // 64 * 64, T))
+    assert np.array_equal(out[0][own], out[1][own]) and not np.array_equal(out[0][~own], out[1][~own])
+
+
 @pytest.mark.parametrize("f32,shape", [(1, (4, 2, 64, 64)), (1, (6, 1, 20, 12)), (1, (2, 1, 300, 72)), (0, (2, 1, 300, 72)),
                                        (1, (10, 2, 64, 36)), (0, (10, 1, 300, 72)), (0, (6, 1, 300, 72))], ids=str)
 @pytest.mark.parametrize("window", [0, 1, 2, 5, 250])

@@ -581,6 +581,23 @@ def test_latent_attention(awq, lib, dev, f32, shape):
         assert km.rms_error(got, want) < (3e-5 if f32 else 0.03), sizes
 
 
+@pytest.mark.parametrize("T", [96, 400])
+def test_a_query_of_the_tiles_among_others(awq, lib, dev, T):
+    """bfloat16 with keys and values formed, 32 queries to a wavefront: those behind the twentieth of each 32 get scores that jump from tile to
+    tile, and the bits of the others do not notice"""
+    heads, dim, rot, vdim, rank = 3, 40, 16, 48, 256
+    print("a query of the tiles among others", T, flush=True)
+    rng = np.random.default_rng(T)
+    q = rng.standard_normal((T, heads * (dim + rot)))
+    down = rng.standard_normal((T, rank + rot)).astype(np.float32)
+    uk, uv = (km.bf16(rng.standard_normal((heads * n, rank)) / rank ** 0.5) for n in (dim, vdim))
+    own = np.arange(T) % 32 < 20
+    layer = Latent(awq, lib, dev, 0, heads, dim, rot, vdim, rank, uk, uv, np.ones(rank), None, (dim + rot) ** -0.5, 1e-6, 300.0, T, T)
+    assert layer.forms
+    out = [layer.run(np.where(own[:, None], q, f * q), down, 0) for f in (1, 24)]
+    assert np.array_equal(out[0][own], out[1][own]) and not np.array_equal(out[0][~own], out[1][~own])
+
+
 # one query in bfloat16: blocks of 16 keys up to as many as there are parts (at most 32), tiles of 64 from there on; row tiles of heads that are
 # not whole, and so many heads that two parts are left.  Bound: 0.03 of the largest of some 800 outputs as in the tests above; of n outputs with errors like
 # normal numbers the largest grows with the root of 2 ln n
