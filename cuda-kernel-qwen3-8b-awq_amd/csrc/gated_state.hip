@@ -1,6 +1,7 @@
 // Linear attention whose state decays per channel (layers.hpp): per head S <- diag(decay_t) S + k_t v_t^T, o_t = S^T q_t.
 #include "lane_sums.hpp"
 #include "layers.hpp"
+#include "segment_join.hpp"
 
 #include <type_traits>
 
@@ -518,14 +519,7 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
   float* const state = a.state + column;
   f32x4_t s[NT];                          // s[i]: rows row0 + 16 i + j4 .. + 3 of column n
   f32x4_t left[NT];                       // AHEAD, not HEAD: the product of the decays
-  float over = 0.0f, over_rest = 0.0f;    // HEAD: the decay's power over a segment
-  if (HEAD && !AHEAD && segment > 1) {
-    double x = 1.0, y = (double)of_head;
-    for (int e = a.seg_tokens; e; e >>= 1, y *= y)
-      if (e & 1) x *= y;
-    over = (float)x;
-    over_rest = (float)(x - (double)over);
-  }
+  const double over = HEAD && !AHEAD && segment > 1 ? segment_power(of_head, a.seg_tokens) : 0.0;
   const bool fresh = a.pos.position() == 0;
 #pragma unroll
   for (int i = 0; i < NT; ++i) {
@@ -541,9 +535,9 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
       s[i] = *reinterpret_cast<const f32x4_t*>(from + (segment == 0 ? 0 : states));
       for (int j = 2; j <= segment; ++j) {
         const f32x4_t add = *reinterpret_cast<const f32x4_t*>(from + j * states);
-        if constexpr (HEAD) {  // the power as a sum of two numbers, as that of a block
+        if constexpr (HEAD) {
 #pragma unroll
-          for (int e = 0; e < 4; ++e) s[i][e] = __builtin_fmaf(s[i][e], over, __builtin_fmaf(s[i][e], over_rest, add[e]));
+          for (int e = 0; e < 4; ++e) s[i][e] = behind_segment(s[i][e], over, add[e]);
           continue;
         }
         const f32x4_t f =

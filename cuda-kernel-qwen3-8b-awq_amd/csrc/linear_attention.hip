@@ -1,5 +1,6 @@
 // Linear attention with a decaying state (layers.hpp): per head S <- decay S + k v^T, o = S^T q.
 #include "dense_one_device.hpp"
+#include "segment_join.hpp"
 
 namespace {
 
@@ -149,14 +150,7 @@ __global__ __launch_bounds__(512) void linear_chunk_kernel(LinearAttnArgs a) {
     return r;
   };
 
-  float over = 0.0f, over_rest = 0.0f;  // the decay's power over a segment, a sum of two numbers (with one the states' errors grew by a half)
-  if (MODE == 2 && segment > 1) {
-    double x = 1.0, y = (double)a.decay[head];
-    for (int e = a.seg_tokens; e; e >>= 1, y *= y)
-      if (e & 1) x *= y;
-    over = (float)x;
-    over_rest = (float)(x - (double)over);
-  }
+  const double over = MODE == 2 && segment > 1 ? segment_power(a.decay[head], a.seg_tokens) : 0.0;
   // the state: rows 32 (wave + 4 i) + 8 g + 4 kh + j of column n in s[i][4 g + j]
   f32x16_t s[TPW];
   const bool holds = !outputs && wave < NT;
@@ -177,7 +171,7 @@ __global__ __launch_bounds__(512) void linear_chunk_kernel(LinearAttnArgs a) {
         for (int j = 2; j <= segment; ++j) {
           const f32x4_t add = *reinterpret_cast<const f32x4_t*>(from + j * states);
 #pragma unroll
-          for (int e = 0; e < 4; ++e) x[e] = __builtin_fmaf(x[e], over, __builtin_fmaf(x[e], over_rest, add[e]));
+          for (int e = 0; e < 4; ++e) x[e] = behind_segment(x[e], over, add[e]);
         }
       }
 #pragma unroll

@@ -669,6 +669,47 @@ def test_segments_of_linear_attention(awq, lib, dev, f32, heads, dim, vdim):
                 assert np.abs(s[h] - S[h]).max() <= 3e-5 * np.abs(S[h]).max(), (sizes, segments, h)
 
 
+@pytest.mark.parametrize("f32", FORMATS, ids=["bf16", "f32"])
+@pytest.mark.parametrize("segments", [16, 3])
+def test_segments_behind_a_state_that_is_not_finite(awq, lib, dev, f32, segments):
+    """Infinities and NaN are where one piece has them, whichever decay brings them along: powers that binary32 holds exactly, that it does not hold
+    (0.3, and 1.5 over a state of zero), and one that leaves of 1e36 what only 64 bits have a factor for.  Bound: as in test_linear_attention"""
+    print("segments behind infinities", segments, f32, flush=True)
+    rng = np.random.default_rng(segments)
+    decay = np.array([0.5, 0.75, 0.9995, 0.3, 1.5, 0.86, 0.9], np.float32)
+    heads, dim, vdim, T, pos0 = len(decay), 64, 16, 1700, 64
+    n = heads * (2 * dim + vdim)
+    x = rng.standard_normal((T, n)) * 0.5 + 0.2
+    k = x[:, heads * dim:2 * heads * dim].reshape(T, heads, dim).copy()
+    k[:, 4:6] = 0.0
+    x[:, heads * dim:2 * heads * dim] = k.reshape(T, -1)
+    for t in range(500, 570, 10):  # (of the first of three segments)
+        x[t, heads * dim + 5 * dim:heads * dim + 6 * dim] = 1e18 * rng.standard_normal(dim)
+        x[t, 2 * heads * dim + 5 * vdim:2 * heads * dim + 6 * vdim] = 1e18 * rng.standard_normal(vdim)
+    proj, pv = dev.act(x, f32)
+    first = rng.standard_normal((heads, vdim, dim))
+    first[:4, 1, 3], first[:4, 2, 7], first[:4, 2, 9], first[4:6] = np.inf, -np.inf, np.inf, 0.0
+    d_decay, d_lg = dev.f(decay), dev.f(np.log2(decay.astype(np.float64)))
+    room, out = heads * (vdim + 1) * dim, []
+    for r in (0, segments):
+        ws, state, o = dev.empty((max(4, r * room),), True), dev.f(first), dev.empty((T, heads * vdim), True)
+        awq.check(lib.awq_linear_attention_segments(proj.data_ptr(), n, heads, dim, vdim, d_decay.data_ptr(), d_lg.data_ptr(), state.data_ptr(),
+                                                    o.data_ptr(), T, pos0, f32, ws.data_ptr(), r * room, dev.stream))
+        out.append((dev.host(o).reshape(T, heads, vdim).transpose(1, 2, 0), dev.host(state)))
+    for one, beside in zip(*out):
+        for is_so in (np.isnan, np.isposinf, np.isneginf):
+            assert np.array_equal(is_so(one), is_so(beside)), is_so.__name__
+        assert np.isposinf(out[0][1][1:3, 1, 3]).all() and not np.isfinite(one[:3, 1:3]).all()
+        for h in range(heads):
+            fine = np.isfinite(one[h])
+            assert fine.any() and np.abs(one[h][fine] - beside[h][fine]).max() <= 3e-5 * np.abs(one[h][fine]).max(), h
+    q, k, v = (pv[:, at:at + m].reshape(T, heads, -1)[:, 5:6] for at, m in
+               ((0, heads * dim), (heads * dim, heads * dim), (2 * heads * dim, heads * vdim)))
+    want = plain.linear_attention(q, k, v, decay[5:6].astype(np.float64))[0][1280:1300, 0].T  # (tokens of the third segment)
+    for o, _ in out:
+        assert np.abs(o[5][:, 1280:1300] - want).max() <= 3e-5 * np.abs(want).max()
+
+
 def attend(awq, lib, dev, f32, proj, heads, kv, dim, vdim, window, scale, eps, temp, sizes, T, slots, max_pos):
     """the attention of T tokens in portions; proj: the tensor with all tokens' projections (kept as it is)"""
     kr, vr = lib.awq_window_row(dim), lib.awq_window_row(vdim)
