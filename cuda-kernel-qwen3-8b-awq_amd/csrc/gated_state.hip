@@ -351,7 +351,7 @@ constexpr int chunk_lds() {
 // a row of the state ahead of it; the first starts from the state itself and keeps a copy.  Then the outputs, every segment starting from
 // those sums, and the last one's state.  The workspace holds
 //     [segments][heads][vdim][dimp]: the state ahead of the pass, then what the segments but the last add,
-//     [segments - 1][heads][dimp]: what is left of a row (not HEAD).
+//     [segments - 1][heads][dimp]: the root of what is left of a row (not HEAD).
 template <typename T, int D, bool EVEN, bool keys, bool HEAD, bool AHEAD>
 __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
   static_assert(keys || !HEAD, "a head's decay leaves no keys");
@@ -518,7 +518,7 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
   const int64_t column = ((int64_t)head * a.vdim + c0 + n) * dimp, states = (int64_t)a.heads * a.vdim * dimp;
   float* const state = a.state + column;
   f32x4_t s[NT];                          // s[i]: rows row0 + 16 i + j4 .. + 3 of column n
-  f32x4_t left[NT];                       // AHEAD, not HEAD: the product of the decays
+  f32x4_t left[NT];                       // AHEAD, not HEAD: the root of the product of the decays
   const double over = HEAD && !AHEAD && segment > 1 ? segment_power(of_head, a.seg_tokens) : 0.0;
   const bool fresh = a.pos.position() == 0;
 #pragma unroll
@@ -543,7 +543,7 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
         const f32x4_t f =
             *reinterpret_cast<const f32x4_t*>(a.workspace + (int64_t)gridDim.z * states + ((int64_t)(j - 1) * a.heads + head) * dimp + d);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s[i][e] = s[i][e] != 0.0f ? __builtin_fmaf(s[i][e], f[e], add[e]) : add[e];  // (no 0 x infinity)
+        for (int e = 0; e < 4; ++e) s[i][e] = behind_segment(s[i][e], of_root(f[e]), add[e]);
       }
     }
   }
@@ -634,7 +634,7 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
             for (int e = 0; e < 4; ++e) s[i][e] *= f[i][e];
             if constexpr (AHEAD) {
 #pragma unroll
-              for (int e = 0; e < 4; ++e) left[i][e] *= f[i][e] * f[i][e];
+              for (int e = 0; e < 4; ++e) left[i][e] = times_decay(left[i][e], f[i][e], 0x1p-126f);
               continue;
             }
             const f32x4_t qv = *reinterpret_cast<const f32x4_t*>(qs + (b * kBlock + n) * S4 + row0 + 16 * i + j4);
@@ -659,6 +659,11 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
         }
       } else {
         if constexpr (HEAD) whole = false;
+        constexpr bool kLeft = AHEAD && !HEAD;
+        double product[kLeft ? 4 * NT : 1];  // of the block's decays
+        if constexpr (kLeft)
+#pragma unroll
+          for (int i = 0; i < 4 * NT; ++i) product[i] = 1.0;
         for (int t = 0; t < kBlock && chunk * C + b * kBlock + t < M; ++t) {
           const int64_t tok = chunk * C + b * kBlock + t;
           const float value = vs[(b * kBlock + t) * VS + n];
@@ -673,7 +678,7 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
               if constexpr (HEAD) key = (float)k[tok * a.ldp + r];
               else decay_and_key(g[tok * a.ldg + r], keys, keys ? (float)k[tok * a.ldp + r] : 0.0f, decay, key);
               s[i][e] = __builtin_fmaf(key, value, decay * s[i][e]);
-              left[i][e] *= decay;
+              if constexpr (kLeft) product[4 * i + e] = times_decay(product[4 * i + e], (double)decay, 0x1p-252);
               out = __builtin_fmaf(s[i][e], (float)q[tok * a.ldp + r] * a.q_scale, out);
             }
           out += __shfl_xor(out, 16, 64);
@@ -684,6 +689,14 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
             if (n == t) o[i] = x;
           }
         }
+        if constexpr (kLeft)
+#pragma unroll
+          for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const double x = product[4 * i + e];
+              left[i][e] = times_decay(left[i][e], (float)__builtin_copysign(sqrt(__builtin_fabs(x)), x), 0x1p-126f);
+            }
       }
       if constexpr (!AHEAD) *reinterpret_cast<f32x4_t*>(red + (wave * B + b) * 256 + n * 16 + j4) = o;
     }

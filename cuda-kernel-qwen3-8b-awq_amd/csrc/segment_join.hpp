@@ -18,4 +18,13 @@ __device__ __forceinline__ float behind_segment(float ahead, double power, float
   return ahead != 0.0f ? (float)__builtin_fma((double)ahead, power, (double)add) : add;
 }
 
+// Where every channel has a decay of its own a segment leaves a product of them, kept as its root (with the product's sign): the smallest root,
+// 2^-126, is that of a factor that brings nothing finite with it, and products stay above it as powers do.
+template <typename R>
+__device__ __forceinline__ R times_decay(R left, R by, R smallest) {
+  const R x = left * by;
+  return __builtin_elementwise_abs(x) < smallest && left != (R)0 && by != (R)0 ? __builtin_elementwise_copysign(smallest, x) : x;
+}
+__device__ __forceinline__ double of_root(float r) { return (double)r * __builtin_fabs((double)r); }
+
 }  // namespace

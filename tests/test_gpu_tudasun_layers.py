@@ -435,6 +435,44 @@ def test_segments_of_a_state(awq, lib, dev, f32, keys, heads, dim, vdim):
 
 
 @pytest.mark.parametrize("f32", FORMATS, ids=["bf16", "f32"])
+@pytest.mark.parametrize("keys", [True, False], ids=["keys", "no keys"])
+@pytest.mark.parametrize("dim", [64, 256])
+def test_segments_behind_values_that_are_not_finite(awq, lib, dev, f32, keys, dim):
+    """Infinities and NaN are where one piece has them, although the product of a segment's decays is 2^-250 or less, token by token
+    in some blocks, and in one channel zero.  Bound: as in test_gated_state"""
+    print("segments behind infinities", dim, f32, keys, flush=True)
+    rng = np.random.default_rng(dim)
+    heads, vdim, T, pos0 = 2, 16, 801, 64
+    hd, n = heads * dim, (2 + keys) * heads * dim - heads * (dim - vdim)
+    x = rng.standard_normal((T, n))
+    x[100, n - heads * vdim + 1], x[100, n - heads * vdim + 2], x[130, n - 2] = np.inf, -np.inf, np.inf
+    rate = 0.9 + 0.2 * rng.random((T, heads, dim))
+    rate[:, :, 3], rate[300:310, :, 8:12] = 1e-3, 30.0
+    rate[400:402, :, 5] = 1000.0  # decays of zero (one alone leaves 2^-150)
+    g = (-rate if keys else 1.0 - 2.0 ** -rate).astype(np.float32)
+    proj, _ = dev.act(x, f32)
+    d_g, first = dev.f(g.reshape(T, hd)), rng.standard_normal((heads, vdim, dim))
+    first[:, 4, 7], first[:, 5, 5] = np.inf, -np.inf
+    base, unit, room = proj.data_ptr(), proj.element_size(), heads * (vdim + 1) * dim
+
+    def run(segments):
+        ws, state, o = dev.empty((max(4, segments * room),), True), dev.f(first), dev.empty((T, heads * vdim), True)
+        a = awq.AwqGatedStateArgs(base, base + hd * unit if keys else None, base + (n - heads * vdim) * unit, d_g.data_ptr(), n, hd, heads, dim,
+                                  vdim, 0.3, state.data_ptr(), o.data_ptr(), T, pos0)
+        awq.check(lib.awq_gated_state_segments(ctypes.byref(a), f32, ws.data_ptr(), segments * room, dev.stream))
+        return dev.host(o), dev.host(state)
+
+    alone = run(0)
+    assert np.isposinf(alone[1][:, 4, 7]).all() and np.isnan(alone[1][:, 5, 5]).all() and np.isposinf(alone[1][0, 1]).any()
+    for segments in (16, 3):
+        for one, beside in zip(alone, run(segments)):
+            for is_so in (np.isnan, np.isposinf, np.isneginf):
+                assert np.array_equal(is_so(one), is_so(beside)), (segments, is_so.__name__)
+            fine = np.isfinite(one)
+            assert fine.any() and np.abs(one[fine] - beside[fine]).max() < 5e-5 * np.abs(one[fine]).max(), segments
+
+
+@pytest.mark.parametrize("f32", FORMATS, ids=["bf16", "f32"])
 def test_a_key_far_back_in_a_state(awq, lib, dev, f32):
     """one token writes a marked row, hundreds of tokens later a query reads just that row"""
     T, dim, vdim, far = 420, 64, 32, 37
