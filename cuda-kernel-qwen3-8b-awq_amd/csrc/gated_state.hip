@@ -352,8 +352,11 @@ constexpr int chunk_lds() {
 // those sums, and the last one's state.  The workspace holds
 //     [segments][heads][vdim][dimp]: the state ahead of the pass, then what the segments but the last add,
 //     [segments - 1][heads][dimp]: the root of what is left of a row (not HEAD).
-template <typename T, int D, bool EVEN, bool keys, bool HEAD, bool AHEAD>
+// (MODE 0: a pass in one piece, 1: AHEAD, 2: outputs of segments.  One piece without the segments' arguments in the way: 16 tokens, 8 heads of 128
+// 4.88 us, with them 5.10, 4 heads of 256 4.94 and 5.19.)
+template <typename T, int D, bool EVEN, bool keys, bool HEAD, int MODE>
 __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
+  constexpr bool AHEAD = MODE == 1, SEGMENTS = MODE != 0;
   static_assert(keys || !HEAD, "a head's decay leaves no keys");
   constexpr int B = chunk_blocks<D>(), C = B * kBlock, S4 = D + 4, VS = kValueStride;
   constexpr int NT = D / 64;                  // tiles of 16 state rows per wavefront
@@ -367,9 +370,9 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
   __shared__ int unsafe[3][B];                // of the running chunk, the one being formed, and one to be cleared
   const int head = blockIdx.x, c0 = blockIdx.y * 16;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int segment = blockIdx.z;
-  const int64_t tok0 = (int64_t)segment * a.seg_tokens;
-  const int M = (int)(a.seg_tokens ? min((int64_t)a.seg_tokens, a.M - tok0) : a.M);  // tokens of this segment, counted from tok0
+  const int segment = SEGMENTS ? blockIdx.z : 0;
+  const int64_t tok0 = SEGMENTS ? (int64_t)segment * a.seg_tokens : 0;
+  const int M = (int)(SEGMENTS ? min((int64_t)a.seg_tokens, a.M - tok0) : a.M);  // tokens of this segment, counted from tok0
   const int nv = min(16, a.vdim - c0), chunks = (M + C - 1) / C;
   const T* const q = reinterpret_cast<const T*>(a.q) + tok0 * a.ldp + (int64_t)head * a.dim;
   const T* const k = keys ? reinterpret_cast<const T*>(a.k) + tok0 * a.ldp + (int64_t)head * a.dim : q;
@@ -519,7 +522,7 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
   float* const state = a.state + column;
   f32x4_t s[NT];                          // s[i]: rows row0 + 16 i + j4 .. + 3 of column n
   f32x4_t left[NT];                       // AHEAD, not HEAD: the root of the product of the decays
-  const double over = HEAD && !AHEAD && segment > 1 ? segment_power(of_head, a.seg_tokens) : 0.0;
+  const double over = HEAD && MODE == 2 && segment > 1 ? segment_power(of_head, a.seg_tokens) : 0.0;
   const bool fresh = a.pos.position() == 0;
 #pragma unroll
   for (int i = 0; i < NT; ++i) {
@@ -527,7 +530,7 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
     const bool there = d < dimp && n < nv;
     s[i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     left[i] = f32x4_t{1.0f, 1.0f, 1.0f, 1.0f};
-    if (AHEAD || !a.seg_tokens) {
+    if constexpr (MODE != 2) {
       if (!fresh && there && segment == 0) s[i] = *reinterpret_cast<const f32x4_t*>(state + d);
       if (AHEAD && segment == 0 && there) *reinterpret_cast<f32x4_t*>(a.workspace + column + d) = s[i];
     } else if (there) {
@@ -702,7 +705,7 @@ __global__ __launch_bounds__(512) void gated_chunk_kernel(GatedStateArgs a) {
     }
     __syncthreads();
   }
-  if (!AHEAD && a.seg_tokens && segment != (int)gridDim.z - 1) return;
+  if (MODE == 2 && segment != (int)gridDim.z - 1) return;
   if (n < nv)
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
@@ -733,34 +736,32 @@ int segment_tokens(const GatedStateArgs& a, int chunk) {
   return 10 * chunks > 18 * of_one + 30 ? (int)of_one * chunk : 0;
 }
 
-template <typename T, int D, bool EVEN, bool KEYS, bool HEAD = false>
-int launch_chunk_form(const GatedStateArgs& u, hipStream_t st) {
-  const dim3 g((unsigned)u.heads, (unsigned)((u.vdim + 15) / 16));
-  GatedStateArgs a = u;
-  if constexpr (EVEN) {
-    static bool raised_ahead = false;
-    a.seg_tokens = segment_tokens(a, chunk_blocks<D>() * kBlock);
-    if (a.seg_tokens) {
-      if (!raised_ahead) {
-        AWQ_HIP_TRY(hipFuncSetAttribute((const void*)gated_chunk_kernel<T, D, EVEN, KEYS, HEAD, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                        chunk_lds<D>()));
-        raised_ahead = true;
-      }
-      const dim3 ahead(g.x, g.y, (unsigned)((a.M - 1) / a.seg_tokens));
-      hipLaunchKernelGGL((gated_chunk_kernel<T, D, EVEN, KEYS, HEAD, true>), ahead, dim3(512), chunk_lds<D>(), st, a);
-      AWQ_HIP_TRY(hipGetLastError());
-    }
-  }
+template <typename T, int D, bool EVEN, bool KEYS, bool HEAD, int MODE>
+int launch_chunk_kernel(const GatedStateArgs& a, unsigned segments, hipStream_t st) {
   static bool raised = false;  // more LDS than the default limit of a launch
   if (!raised) {
-    AWQ_HIP_TRY(hipFuncSetAttribute((const void*)gated_chunk_kernel<T, D, EVEN, KEYS, HEAD, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    AWQ_HIP_TRY(hipFuncSetAttribute((const void*)gated_chunk_kernel<T, D, EVEN, KEYS, HEAD, MODE>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     chunk_lds<D>()));
     raised = true;
   }
-  const dim3 all(g.x, g.y, a.seg_tokens ? (unsigned)((a.M + a.seg_tokens - 1) / a.seg_tokens) : 1u);
-  hipLaunchKernelGGL((gated_chunk_kernel<T, D, EVEN, KEYS, HEAD, false>), all, dim3(512), chunk_lds<D>(), st, a);
+  const dim3 g((unsigned)a.heads, (unsigned)((a.vdim + 15) / 16), segments);
+  hipLaunchKernelGGL((gated_chunk_kernel<T, D, EVEN, KEYS, HEAD, MODE>), g, dim3(512), chunk_lds<D>(), st, a);
   AWQ_HIP_TRY(hipGetLastError());
   return AWQ_OK;
+}
+
+template <typename T, int D, bool EVEN, bool KEYS, bool HEAD = false>
+int launch_chunk_form(const GatedStateArgs& u, hipStream_t st) {
+  if constexpr (EVEN) {
+    GatedStateArgs a = u;
+    a.seg_tokens = segment_tokens(a, chunk_blocks<D>() * kBlock);
+    if (a.seg_tokens) {
+      const unsigned ahead = (unsigned)((a.M - 1) / a.seg_tokens);
+      if (int rc = launch_chunk_kernel<T, D, EVEN, KEYS, HEAD, 1>(a, ahead, st)) return rc;
+      return launch_chunk_kernel<T, D, EVEN, KEYS, HEAD, 2>(a, ahead + 1, st);
+    }
+  }
+  return launch_chunk_kernel<T, D, EVEN, KEYS, HEAD, 0>(u, 1, st);
 }
 template <typename T, int D>
 int launch_chunks(const GatedStateArgs& a, hipStream_t st) {
