@@ -802,7 +802,7 @@ __global__ __launch_bounds__(256 * HALVES, (DK + DV > 256) ? 1 : 2) void latent_
     if (k0 >= k_end) return;
 #pragma unroll
     for (int i = 0; i < KP; ++i) {
-      // (past a row's end its last piece, which meets zeros of the query: a condition around a request has the ones ahead of it waited for)
+      // (past a row's end its last piece: a condition around a request has the ones ahead of it waited for)
       const int pc = tid + i * 256, key = min(k0 + pc / (DK / 8), k_end - 1), at = min((pc % (DK / 8)) * 8, qk - 8);
       const bf16_t* const from = at < a.dim ? kx + key * ldkv + at : cache + (int64_t)key * row + at - a.dim;
       r.k[i] = *reinterpret_cast<const bf16x8_t*>(from);
@@ -817,7 +817,7 @@ __global__ __launch_bounds__(256 * HALVES, (DK + DV > 256) ? 1 : 2) void latent_
 #pragma unroll
     for (int i = 0; i < KP; ++i) {
       const int pc = tid + i * 256, key = pc / (DK / 8), at = (pc % (DK / 8)) * 8;
-      *reinterpret_cast<bf16x8_t*>(ks2 + (half * kTileKeys + key) * KS + at) = r.k[i];
+      *reinterpret_cast<bf16x8_t*>(ks2 + (half * kTileKeys + key) * KS + at) = at < qk ? r.k[i] : zero;  // (the query's zeros there meet no infinity)
     }
 #pragma unroll
     for (int i = 0; i < VP; ++i) {

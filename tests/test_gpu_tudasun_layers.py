@@ -636,6 +636,26 @@ def test_a_query_of_the_tiles_among_others(awq, lib, dev, T):
     assert np.array_equal(out[0][own], out[1][own]) and not np.array_equal(out[0][~own], out[1][~own])
 
 
+def test_an_infinite_key_that_weighs_nothing(awq, lib, dev):
+    """bfloat16 with keys and values formed, rows of 56 in tiles of 64: at a score of minus infinity as at one that is merely very low"""
+    heads, dim, rot, vdim, rank, T = 2, 40, 16, 48, 256, 96
+    print("an infinite key", flush=True)
+    rng = np.random.default_rng(1)
+    q = rng.standard_normal((T, heads, dim + rot))
+    q[:, :, dim + 12:dim + 14] = -1.0, 0.0  # (turned by less than a quarter: negative)
+    uk, uv = (km.bf16(rng.standard_normal((heads * n, rank)) / rank ** 0.5) for n in (dim, vdim))
+    layer = Latent(awq, lib, dev, 0, heads, dim, rot, vdim, rank, uk, uv, np.ones(rank), None, (dim + rot) ** -0.5, 1e-6, 300.0, T, T)
+    assert layer.forms
+    rows = dev.torch.from_numpy(rng.standard_normal((T, layer.row)).astype(np.float32)).cuda().to(dev.torch.bfloat16)
+    out = []
+    for low in (1e30, np.inf):
+        layer.cache[:T] = rows
+        for t in (20, 33, 70):
+            layer.cache[t, rank + 12] = low
+        out.append(layer.run(q.reshape(T, -1), None, 0))
+    assert np.isfinite(out[0]).all() and np.array_equal(*out)
+
+
 # one query in bfloat16: blocks of 16 keys up to as many as there are parts (at most 32), tiles of 64 from there on; row tiles of heads that are
 # not whole, and so many heads that two parts are left.  Bound: 0.03 of the largest of some 800 outputs as in the tests above; of n outputs with errors like
 # normal numbers the largest grows with the root of 2 ln n
