@@ -970,11 +970,13 @@ int64_t form_from(const LatentAttnArgs& a) {
 }
 
 // A pass whose keys are mostly its own forms them with fewer queries: a key of its own costs what its latent query costs otherwise, and keys ahead
-// of the pass are paid for by what the pass saves on all of them; two launches fewer besides.  Prompts of Tudasun 2048, 129 tokens 815 -> 777 us, 40
+// of the pass are paid for by what the pass saves on all of them; two launches fewer besides.  Only for a caller that says so (a.own_keys): q is
+// turned in place and kv written, which a pass of so few leaves alone otherwise.  Prompts of Tudasun 2048, 129 tokens 815 -> 777 us, 40
 // tokens 685 -> 662, 3 tokens 457 -> 438; 1024, 24 tokens 446 -> 416; 4096, 70 tokens 1,490 -> 1,445.
 bool forms_few(const LatentAttnArgs& a) {
   const double saved = 2.0 * a.l.rank - a.dim - a.vdim, keys = (double)(a.pos.pos0 + a.M);
-  return a.M > 1 && a.w_kv && a.kv && ((a.ldq | a.ldc) & 7) == 0 && (double)a.M * keys * saved >= (double)a.pos.pos0 * a.l.rank * (a.dim + a.vdim);
+  return a.own_keys && a.M > 1 && a.w_kv && a.kv && ((a.ldq | a.ldc) & 7) == 0 && (((uintptr_t)a.q | (uintptr_t)a.ctx) & 15) == 0 &&
+         (double)a.M * keys * saved >= (double)a.pos.pos0 * a.l.rank * (a.dim + a.vdim);
 }
 
 // One query in binary32: rows of up to 768 values, and workgroups for two per compute unit

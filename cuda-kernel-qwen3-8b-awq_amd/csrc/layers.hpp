@@ -320,6 +320,7 @@ struct LatentAttnArgs {
   float* parts = nullptr;
   float* dense_ws = nullptr;
   int64_t dense_ws_floats = 0;
+  bool own_keys = false;  // a pass of a few tokens may take the second form too
 };
 struct LatentScratch {
   int64_t qa = 0, ql = 0, ol = 0, kv = 0, parts = 0;  // bytes

@@ -656,6 +656,7 @@ int TudasunEngine::mix(int i, Buffers& b, int64_t M, PassPos pos) {
     a.parts = (float*)s_parts;
     a.dense_ws = dense_ws;
     a.dense_ws_floats = dense_ws_floats;
+    a.own_keys = true;
     return launch_latent_attention(a, f32, stream);
   }
   if (s.type == MIX_GLA) {

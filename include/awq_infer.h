@@ -609,7 +609,8 @@ int awq_head_norm(const float* o, const void* gate, int64_t ldg, const float* w,
  * query head h with a position is (q . W_uk[h] c + q_rot . k_rot) * scale, the
  * value W_uv[h] c, softmax with exp(sink[h]) in the denominator (sink NULL: not).
  * q [n_tokens][ldq]: heads of dim unrotated, then rot rotated values (pairs 2 i, 2 i + 1
- * by position * freq[i], freq binary64; changed in place by passes of many tokens).  down [n_tokens][ldd] float:
+ * by position * freq[i], freq binary64; changed in place by the passes that form keys and values: bfloat16, w_kv and kv
+ * there, from max(32, rank (dim + vdim) / (2 rank - dim - vdim)) tokens on).  down [n_tokens][ldd] float:
  * latent (normalised with `norm` before it is cached) and key part; NULL: the cache
  * already has these positions.  cache: rows of awq_latent_row(rank, rot) elements, max_pos
  * of them rounded up to 64.  Weights packed by awq_latent_pack into the three blocks of

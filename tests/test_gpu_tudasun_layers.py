@@ -636,6 +636,29 @@ def test_a_query_of_the_tiles_among_others(awq, lib, dev, T):
     assert np.array_equal(out[0][own], out[1][own]) and not np.array_equal(out[0][~own], out[1][~own])
 
 
+@pytest.mark.parametrize("n,at", [(2, 0), (24, 0), (52, 0), (30, 10)])
+def test_a_short_pass_leaves_its_queries_alone(awq, lib, dev, n, at):
+    """where keys and values are formed from 53 tokens on: q, which a second layer may read again, and kv"""
+    heads, dim, rot, vdim, rank = 3, 40, 16, 48, 256
+    print("a short pass over latents", n, at, flush=True)
+    rng = np.random.default_rng(n)
+    uk, uv = (km.bf16(rng.standard_normal((heads * m, rank)) / rank ** 0.5) for m in (dim, vdim))
+    layer = Latent(awq, lib, dev, 0, heads, dim, rot, vdim, rank, uk, uv, np.ones(rank), None, 0.2, 1e-6, 300.0, 128, 128)
+    assert layer.forms
+    a, torch = layer.a, dev.torch
+    layer.cache[:] = torch.from_numpy(rng.standard_normal(tuple(layer.cache.shape)).astype(np.float32)).cuda().to(torch.bfloat16)
+    layer.keep["kv"][:] = 77
+    q, _ = dev.act(rng.standard_normal((n, heads * (dim + rot))), False)
+    before, out = q.clone(), []
+    for _ in range(2):
+        ctx = dev.empty((n, heads * vdim), False)
+        a.q, a.ldq, a.down, a.ctx, a.ldc, a.n_tokens, a.pos0 = q.data_ptr(), q.shape[1], None, ctx.data_ptr(), heads * vdim, n, at
+        awq.check(lib.awq_latent_attention(ctypes.byref(a), 0, dev.stream))
+        out.append(dev.host(ctx))
+    assert torch.equal(q, before) and bool((layer.keep["kv"] == 77).all())
+    assert np.isfinite(out[0]).all() and np.array_equal(*out)
+
+
 def test_an_infinite_key_that_weighs_nothing(awq, lib, dev):
     """bfloat16 with keys and values formed, rows of 56 in tiles of 64: at a score of minus infinity as at one that is merely very low"""
     heads, dim, rot, vdim, rank, T = 2, 40, 16, 48, 256, 96
