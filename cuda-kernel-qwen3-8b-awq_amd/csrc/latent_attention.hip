@@ -971,12 +971,15 @@ int64_t form_from(const LatentAttnArgs& a) {
 
 // A pass whose keys are mostly its own forms them with fewer queries: a key of its own costs what its latent query costs otherwise, and keys ahead
 // of the pass are paid for by what the pass saves on all of them; two launches fewer besides.  Only for a caller that says so (a.own_keys): q is
-// turned in place and kv written, which a pass of so few leaves alone otherwise.  Prompts of Tudasun 2048, 129 tokens 815 -> 777 us, 40
+// turned in place and kv written, which a pass of so few leaves alone otherwise.  Nor behind a long context with few heads: a workgroup goes
+// through all keys of its 128 queries alone, 25 ns each (128 + 64 wide), where the latent space has parts.  Rank 512, 8 heads, 160
+// tokens at 1,000: 49 us here, 56 there, at 2,000 80 and 66; 2 heads at 380 31 and 34, at 800 41 and 38; 32 heads at 2,000 94 and 149; rank 256,
+// dim 64, 16 heads, 84 tokens at 800 32 and 37, at 1,600 50 and 41.  Prompts of Tudasun 2048, 129 tokens 815 -> 777 us, 40
 // tokens 685 -> 662, 3 tokens 457 -> 438; 1024, 24 tokens 446 -> 416; 4096, 70 tokens 1,490 -> 1,445.
 bool forms_few(const LatentAttnArgs& a) {
   const double saved = 2.0 * a.l.rank - a.dim - a.vdim, keys = (double)(a.pos.pos0 + a.M);
   return a.own_keys && a.M > 1 && a.w_kv && a.kv && ((a.ldq | a.ldc) & 7) == 0 && (((uintptr_t)a.q | (uintptr_t)a.ctx) & 15) == 0 &&
-         (double)a.M * keys * saved >= (double)a.pos.pos0 * a.l.rank * (a.dim + a.vdim);
+         keys <= 448.0 + 0.5625 * (double)a.M * a.heads && (double)a.M * keys * saved >= (double)a.pos.pos0 * a.l.rank * (a.dim + a.vdim);
 }
 
 // One query in binary32: rows of up to 768 values, and workgroups for two per compute unit
