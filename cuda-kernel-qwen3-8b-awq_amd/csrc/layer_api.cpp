@@ -174,6 +174,7 @@ extern "C" int awq_linear_attention(const void* proj, int64_t ldp, int32_t heads
 extern "C" int awq_linear_attention_segments(const void* proj, int64_t ldp, int32_t heads, int32_t dim, int32_t vdim,
                                              const float* decay, const float* log2_decay, float* state, float* o, int64_t n_tokens,
                                              int64_t pos0, int32_t f32, float* workspace, int64_t workspace_floats, void* stream) {
+  AWQ_REQUIRE(((uintptr_t)workspace & 15) == 0 && workspace_floats >= 0, "the workspace is 16-byte aligned");
   LinearAttnArgs a = linear_of(proj, ldp, heads, dim, vdim, decay, log2_decay, state, o, n_tokens, pos0);
   a.workspace = workspace;
   a.workspace_floats = workspace_floats;
@@ -182,6 +183,7 @@ extern "C" int awq_linear_attention_segments(const void* proj, int64_t ldp, int3
 
 extern "C" int awq_gated_state_segments(const awq_gated_state_args* u, int32_t f32, float* workspace, int64_t workspace_floats, void* stream) {
   AWQ_REQUIRE(u != nullptr, "args is NULL");
+  AWQ_REQUIRE(((uintptr_t)workspace & 15) == 0 && workspace_floats >= 0, "the workspace is 16-byte aligned");
   GatedStateArgs a;
   a.workspace = workspace;
   a.workspace_floats = workspace_floats;

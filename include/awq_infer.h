@@ -599,7 +599,7 @@ typedef struct awq_gated_state_args {
   float eps, reserved;
 } awq_gated_state_args;
 int awq_gated_state(const awq_gated_state_args* args, int32_t f32, void* stream);
-/* the same with room for segments, heads * (vdim + 1) * round_up(dim, 64) floats each */
+/* the same with room for segments as above, heads * (vdim + 1) * round_up(dim, 64) floats each, 16-byte aligned */
 int awq_gated_state_segments(const awq_gated_state_args* args, int32_t f32, float* workspace, int64_t workspace_floats, void* stream);
 /* ctx[t][h][c] = RMS norm over each head's vdim values of o, times w [vdim], times silu(gate) (gate NULL: 1) */
 int awq_head_norm(const float* o, const void* gate, int64_t ldg, const float* w, void* ctx, int64_t ldc, int32_t heads,

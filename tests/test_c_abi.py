@@ -95,6 +95,17 @@ def test_gemm_rejects_bad_arguments_before_any_gpu_call(lib):
     assert call(base, base, 6144, 4096, 40) == 1 and b"scale group" in lib.awq_last_error()
 
 
+@pytest.mark.parametrize("address,floats", [(0x10008, 1 << 20), (0x10001, 1 << 20), (0x10000, -1)])
+def test_segments_reject_a_bad_workspace_before_any_gpu_call(awq, lib, address, floats):
+    """the kernels read and write it in pieces of 16 bytes; the addresses here are no memory"""
+    p = 0x100000
+    rc = lib.awq_linear_attention_segments(p, 24 * 64, 8, 64, 64, p, p, p, p, 1000, 0, 0, address, floats, None)
+    assert rc == 1 and b"aligned" in lib.awq_last_error()
+    a = awq.AwqGatedStateArgs(p, p, p, p, 24 * 64, 8 * 64, 8, 64, 64, 0.3, p, p, 1000, 0)
+    rc = lib.awq_gated_state_segments(ctypes.byref(a), 0, address, floats, None)
+    assert rc == 1 and b"aligned" in lib.awq_last_error()
+
+
 def test_cli_usage_error():
     exe = os.path.join(ROOT, "cuda-kernel-qwen3-8b-awq_amd", "qwen3_awq_infer")
     res = subprocess.run([exe], capture_output=True, text=True)
