@@ -407,6 +407,33 @@ def test_prefill_attention_matches_the_one_query_path(awq, lib, oracle, torch_gp
                                      0, stream(torch)) != 0     # runs past max_pos
 
 
+@pytest.mark.parametrize("steep", [1, 16])
+@pytest.mark.parametrize("first_layer", [0, 1])
+@pytest.mark.parametrize("pos0,M", [(0, 257), (0, 300), (100, 289), (250, 7), (256, 130)])
+def test_prefill_attention_with_the_keys_in_halves(awq, lib, torch_gpu, pos0, M, first_layer, steep):
+    """More than 256 positions: ragged ends in either half, queries that see keys of one half only, and scores that rise by more than 2^8 from tile to
+    tile.  Weights and outputs are rounded to 11 bits, 2^-11 of the largest value each; scores of up to 16 x 6 in binary32 add 2^-17."""
+    torch = torch_gpu
+    nh, mp = 3, 512
+    rng = np.random.default_rng(pos0 * 1000 + M)
+    q = (steep * rng.standard_normal((M, nh, 128))).astype(np.float16)
+    k, v = (rng.standard_normal((nh, mp, 128)).astype(np.float16) for _ in range(2))
+    s = np.einsum("thd,hpd->htp", q.astype(np.float64), k.astype(np.float64)) / 128 ** 0.5
+    at = pos0 + np.arange(M)
+    seen = np.maximum(at, 1) if first_layer else at + 1
+    s = np.where(np.arange(mp) < seen[:, None], s, -np.inf)
+    w = np.exp(s - s.max(-1, keepdims=True))
+    want = np.einsum("htp,hpd->thd", w / w.sum(-1, keepdims=True), v.astype(np.float64)).reshape(M, nh * 128)
+    d_q, d_k, d_v = dev(torch, q.reshape(M, -1)), dev(torch, k), dev(torch, v)
+    d_o = torch.full((M, nh * 128), float("nan"), dtype=torch.float16, device="cuda")
+    print("prefill attention in halves", pos0, M, first_layer, steep, flush=True)
+    awq.check(lib.awq_prefill_attention(d_q.data_ptr(), d_k.data_ptr(), d_v.data_ptr(), d_o.data_ptr(), nh, mp, pos0, M, first_layer,
+                                        stream(torch)))
+    torch.cuda.synchronize()
+    got = d_o.cpu().numpy().astype(np.float64)
+    assert np.abs(got - want).max() <= 1.5 * 2.0 ** -10 * np.abs(v.astype(np.float64)).max()
+
+
 @pytest.mark.parametrize("pos0,M", [(0, 64), (70, 130), (300, 64), (0, 300)])
 def test_prefill_attention_of_a_query_is_its_own(awq, lib, torch_gpu, pos0, M):
     """32 queries share a wavefront; those behind the twentieth of each 32 get scores that jump from tile to tile, which the bits of the others do

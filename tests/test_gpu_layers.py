@@ -758,6 +758,32 @@ def test_window_attention(awq, lib, dev, f32, shape, window):
         assert km.rms_error(got, want) < (3e-5 if f32 else 0.01), sizes
 
 
+@pytest.mark.parametrize("steep", [3.0, 16.0])
+@pytest.mark.parametrize("shape", [(3, 3, 128, 128), (4, 2, 64, 128), (10, 2, 64, 36), (2, 1, 100, 60)], ids=str)
+@pytest.mark.parametrize("window", [0, 160, 257])
+def test_window_attention_with_the_keys_in_halves(awq, lib, dev, shape, window, steep):
+    """bfloat16, more than 256 keys: every instance with halves, ragged ends, queries that see keys of one half only and, where scores are steep, maxima
+    that move by more than 2^8 in either half.  Beside the output's rounding (2^-9) a component of q or k that the norm leaves
+    at the edge of a rounding may fall on the other side: up to steep / sqrt(dim) x 2^-8 x 3^2 of a score, 5 % of a weight at worst, a few of them in
+    a row whose other weights hold"""
+    heads, kv, dim, vdim = shape
+    print("window attention in halves", shape, window, steep, flush=True)
+    rng = np.random.default_rng(dim + window)
+    T, eps, scale = 400, 1e-3, steep / dim ** 0.5
+    n = heads * dim + kv * (dim + vdim)
+    proj, pv = dev.act(np.pad(2 * rng.standard_normal((T, n)), ((0, 0), (0, -n % 8))), False)
+    q = km.bf16(plain.rms(pv[:, :heads * dim].reshape(T, heads, dim), eps)).astype(np.float64)
+    k = km.bf16(plain.rms(pv[:, heads * dim:(heads + kv) * dim].reshape(T, kv, dim), eps)).astype(np.float64)
+    v = pv[:, (heads + kv) * dim:n].reshape(T, kv, vdim)
+    want = plain.window_attention(q, k, v, window or None, scale, (0.0, 1.0))
+    for sizes in ([400], [300, 100], [7, 280, 113]):
+        slots = ((window or T) - 1 + max(sizes) + 63) // 64 * 64
+        got = attend(awq, lib, dev, 0, proj, heads, kv, dim, vdim, window, scale, eps, (0.0, 1.0), sizes, T, slots, T)
+        off = km.rms_error(got, want)
+        print("error %.1e" % off, flush=True)
+        assert off < (0.01 if steep < 4 else 0.03), sizes
+
+
 @pytest.mark.parametrize("T", [96, 400])
 @pytest.mark.parametrize("window", [0, 90])
 def test_a_query_among_others(awq, lib, dev, window, T):

@@ -619,6 +619,48 @@ def test_latent_attention(awq, lib, dev, f32, shape):
         assert km.rms_error(got, want) < (3e-5 if f32 else 0.03), sizes
 
 
+# a shape for each width of the tiles (queries 64 .. 256, values 64 .. 256), with halves of the keys and without
+TILES = [(40, 16, 16, 24, 64), (2, 40, 16, 104, 256), (2, 72, 24, 48, 256), (3, 80, 16, 120, 256), (2, 136, 24, 40, 320), (2, 128, 64, 128, 384),
+         (2, 200, 40, 56, 448), (1, 200, 56, 128, 512), (1, 24, 8, 200, 320), (1, 96, 32, 256, 512)]
+
+
+@pytest.mark.parametrize("steep", [2.5, 12.0])
+@pytest.mark.parametrize("shape", TILES, ids=str)
+def test_latent_attention_with_formed_keys(awq, lib, dev, shape, steep):
+    """bfloat16: portions that form keys and values in every instance of the tiles, ragged ends in either half of the keys, queries that see keys of
+    one half only, and maxima that move by more than 2^8 in either.  The statement rounds rows, queries, keys and values as the kernels do;
+    beside the output's rounding (2^-9) one that falls on the other side of an edge changes a score by steep / sqrt(dim) x 2^-8 x 3^2"""
+    heads, dim, rot, vdim, rank = shape
+    print("latent attention, formed keys", shape, steep, flush=True)
+    rng = np.random.default_rng(rank + vdim)
+    T, eps, base, scale = 400, 1e-3, 300.0, steep * (dim + rot) ** -0.5
+    r = lambda x: km.bf16(x).astype(np.float64)
+    q = km.bf16(rng.standard_normal((T, heads * (dim + rot))))
+    down = rng.standard_normal((T, rank + rot)).astype(np.float32)
+    sink = 2 * rng.standard_normal(heads)
+    uk, uv = (km.bf16(rng.standard_normal((heads * n, rank)) / rank ** 0.5) for n in (dim, vdim))
+    layer = Latent(awq, lib, dev, 0, heads, dim, rot, vdim, rank, uk, uv, np.ones(rank), sink, scale, eps, base, T, T)
+    first = max(32, rank * (dim + vdim) // (2 * rank - dim - vdim))
+    assert layer.forms and first <= 270
+    c, kr = r(plain.rms(down[:, :rank].astype(np.float64), eps)), r(plain.rotate(down[:, rank:].astype(np.float64), 0, base))
+    qh = q.reshape(T, heads, dim + rot).astype(np.float64)
+    qr, want = r(plain.rotate(qh[:, :, dim:], 0, base)), np.zeros((T, heads, vdim))
+    seen = np.arange(T)[None, :] <= np.arange(T)[:, None]
+    for h in range(heads):
+        k, v = r(c @ uk[h * dim:(h + 1) * dim].T.astype(np.float64)), r(c @ uv[h * vdim:(h + 1) * vdim].T.astype(np.float64))
+        s = np.where(seen, (qh[:, h, :dim] @ k.T + qr[:, h] @ kr.T) * scale, -np.inf)
+        m = np.maximum(s.max(1), sink[h])[:, None]
+        w = np.exp(s - m)
+        want[:, h] = w @ v / (w.sum(1, keepdims=True) + np.exp(sink[h] - m))
+    for sizes in ([T], [130, 270], [200, 200]):
+        if min(sizes) < first:
+            continue
+        got = np.concatenate([layer.run(q[at:at + n], down[at:at + n], at) for at, n in portions(T, sizes)])
+        off = km.rms_error(got, want)
+        print("error %.1e" % off, flush=True)
+        assert off < (0.01 if steep < 4 else 0.03), sizes
+
+
 @pytest.mark.parametrize("T", [96, 400])
 def test_a_query_of_the_tiles_among_others(awq, lib, dev, T):
     """bfloat16 with keys and values formed, 32 queries to a wavefront: those behind the twentieth of each 32 get scores that jump from tile to
