@@ -372,8 +372,9 @@ int launch_prefill_attention(const half_t* q, const half_t* kc, const half_t* vc
   AWQ_REQUIRE(n_heads > 0 && max_pos > 0, "n_heads and max_pos must be positive");
   AWQ_REQUIRE(M >= 1 && M <= 65535 * kFaQueries && pos0 >= 0 && pos0 + M <= max_pos, "positions out of range");
   const dim3 g((unsigned)n_heads, (unsigned)((M + kFaQueries - 1) / kFaQueries));
-  // Halves of the keys from two turns of each on: 32 heads at 1,000 tokens 38 -> 25 us (prompt of 36 layers 13.03 -> 12.75 ms), 2,048
-  // tokens 27.0 -> 26.1 ms, 300 as before; 140 tokens 4.77 ms without and 4.82 with.
+  // Halves of the keys from two turns of each on: 32 heads at 1,000 tokens 33 -> 24 us (prompt of 36 layers 13.49 -> 13.22 ms), 2,048
+  // tokens 28.0 -> 27.2 ms, 257 to 275 0.2 to 0.4 us a layer more and 300 as much less; prompt of 140 tokens 4.77 ms without and 4.82 with.
+  // A query sums its keys in one order in either form, whatever the pass, and in another order in the other.
   if (pos0 + M > 8 * kFaKeys)
     hipLaunchKernelGGL(prefill_attention_kernel<2>, g, dim3(512), 0, st, q, kc, vc, ctx, kv, (int)pos0, (int)M, use_len_hi);
   else
