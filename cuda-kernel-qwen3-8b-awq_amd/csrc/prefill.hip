@@ -282,7 +282,7 @@ __global__ __launch_bounds__(256 * HALVES, HALVES == 2 ? 1 : 2) void prefill_att
     const HalfPair best = half_pair(mx);
     mx = fmaxf(best.low, best.high);
     // (a tile in which none of this query's keys is attended leaves the maximum where it was)
-    move_maximum(mx > -1e29f ? mx * scale2 : -1e30f, m_run, l_run, o);
+    move_maximum<HALVES == 2>(mx > -1e29f ? mx * scale2 : -1e30f, m_run, l_run, o);
     float rs = 0.0f;
     half8_t pop[2];
 #pragma unroll

@@ -15,13 +15,14 @@ __device__ __forceinline__ HalfPair half_pair(float x) {
   return {__uint_as_float(p[0]), __uint_as_float(p[1])};
 }
 
-// The maximum m that a query's weights are relative to moves to mx, the largest score of a tile, only once it is 2^kSlack behind it: sums grow by
-// as much and no more (the conditional rescaling of FlashAttention-4).  Every query decides for itself, so that its bits do not
-// depend on those that share its wavefront; what the wavefront decides is whether any has to.
+// The maximum m that a query's weights are relative to moves to mx, the largest score of a tile: always, or (LAGS) only once it is 2^kSlack behind
+// it: sums grow by as much and no more (the conditional rescaling of FlashAttention-4).  Every query decides for itself, so that its
+// bits do not depend on those that share its wavefront; what the wavefront decides is whether any has to.
+// A maximum that lags saves the rescaling of most tiles: latents of 192 + 64, 1,024 tokens of 16 heads 98 -> 84 us, int4 256 tokens 9.8 -> 9.2; windows 0 to 1 %.
 constexpr float kSlack = 8.0f;
-template <int BLOCKS, typename V>
+template <bool LAGS, int BLOCKS, typename V>
 __device__ __forceinline__ void move_maximum(float mx, float& m, float& l, V (&o)[BLOCKS]) {
-  const bool moves = mx > m + kSlack;
+  const bool moves = mx > (LAGS ? m + kSlack : m);
   if (__builtin_amdgcn_ballot_w64(moves) == 0) return;
   const float to = moves ? mx : m, alpha = moves ? __builtin_amdgcn_exp2f(m - to) : 1.0f;
   l *= alpha;

@@ -556,7 +556,7 @@ __global__ __launch_bounds__(256 * HALVES, (DK + DV > 256) ? 1 : 2) void window_
     for (int i = 1; i < 16; ++i) mx = fmaxf(mx, s[i]);
     const HalfPair best = half_pair(mx);
     mx = fmaxf(best.low, best.high);
-    move_maximum(mx, m_run, l_run, o);
+    move_maximum<HALVES == 2>(mx, m_run, l_run, o);
     float rs = 0.0f;
     bf16x8_t hi[2], lo[2];
 #pragma unroll
